@@ -4,7 +4,7 @@ There is no CPU fallback: if the library cannot be loaded the package raises.
 """
 
 import ctypes
-import os
+import importlib.util
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_void_p, POINTER
 
 import torch
@@ -145,6 +145,21 @@ def lib():
   return _lib
 
 
+_native = None
+
+
+def native():
+  """The layers' host path (csrc/host.cpp), loaded once, after the library it calls."""
+  global _native
+  if _native is None:
+    lib()
+    spec = importlib.util.spec_from_file_location('ocnn_host', _build.HOST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    _native = module
+  return _native
+
+
 class OcnnHipError(RuntimeError):
   pass
 
@@ -163,11 +178,15 @@ DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 WGRAD_PLAIN, WGRAD_DENSE_RW, WGRAD_SPARSE, WGRAD_PLANNED, WGRAD_ZERO_PADDED = range(5)
 
 
-def dtype_code(t):
+def dtype_code_of(dtype):
   try:
-    return DTYPE_CODE[t.dtype]
+    return DTYPE_CODE[dtype]
   except KeyError:
-    raise TypeError('unsupported feature dtype {}; use float32, float16 or bfloat16'.format(t.dtype))
+    raise TypeError('unsupported feature dtype {}; use float32, float16 or bfloat16'.format(dtype))
+
+
+def dtype_code(t):
+  return dtype_code_of(t.dtype)
 
 
 def require_gpu(*tensors):

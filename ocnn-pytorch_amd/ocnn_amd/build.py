@@ -1,8 +1,10 @@
-"""Builds libocnn_hip.so (gfx950) from csrc/ with hipcc, in-tree."""
+"""Builds, in-tree, libocnn_hip.so (gfx950) from csrc/*.hip with hipcc, and ocnn_host.so, the layers'
+host path on torch's C++ API (csrc/host.cpp), with the host compiler."""
 
 import hashlib
 import os
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -10,6 +12,7 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 CSRC = os.path.join(HERE, 'csrc')
 LIB_DIR = os.path.join(HERE, 'lib')
 LIB_PATH = os.path.join(LIB_DIR, 'libocnn_hip.so')
+HOST_PATH = os.path.join(LIB_DIR, 'ocnn_host.so')
 INCLUDE = os.path.join(ROOT, 'include')
 
 # file -> extra flags.  The key/build kernels must round every fp32 operation
@@ -38,6 +41,22 @@ COMMON = ['-O3', '--offload-arch=gfx950', '-fPIC', '-std=c++17', '-I', INCLUDE, 
           '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops']
 
 
+def _host_commands():
+  """Compiler and linker command of ocnn_host.so: torch's headers and libraries, and the HIP library
+  beside it.  (torch's ROCm headers ask for the platform to be named.)"""
+  import torch
+  base = os.path.dirname(torch.__file__)
+  obj = os.path.join(LIB_DIR, 'obj', 'host.o')
+  system = [os.path.join(base, 'include'), os.path.join(base, 'include', 'torch', 'csrc', 'api', 'include'),
+            os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include'), sysconfig.get_paths()['include']]
+  compile_ = ['g++', '-O2', '-std=c++17', '-fPIC', '-fvisibility=hidden', '-Wall', '-D__HIP_PLATFORM_AMD__=1',
+              '-DUSE_ROCM=1', '-I', INCLUDE] + ['-isystem' + d for d in system] + [
+                  '-c', os.path.join(CSRC, 'host.cpp'), '-o', obj]
+  link = ['g++', '-shared', '-o', HOST_PATH, obj, '-L', os.path.join(base, 'lib'), '-ltorch_python', '-ltorch',
+          '-ltorch_cpu', '-lc10', '-lc10_hip', '-L', LIB_DIR, '-locnn_hip', '-Wl,-rpath,$ORIGIN']
+  return compile_, link
+
+
 STAMP_PATH = os.path.join(LIB_DIR, 'sources.sha256')
 
 
@@ -51,6 +70,8 @@ def source_hash():
       with open(path, 'rb') as f:
         h.update(f.read())
   h.update(repr((COMMON[:4] + COMMON[8:], sorted(SOURCES.items()))).encode())
+  import torch
+  h.update(torch.__version__.encode())               # (the host part is built against its C++ API)
   return h.hexdigest()
 
 
@@ -61,7 +82,7 @@ def is_current():
       stamp = f.read().strip()
   except OSError:
     return False
-  return os.path.exists(LIB_PATH) and stamp == source_hash()
+  return os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH) and stamp == source_hash()
 
 
 def _hipcc():
@@ -91,13 +112,17 @@ def build_library(verbose=False):
     _run([hipcc] + COMMON + extra + ['-c', os.path.join(CSRC, name), '-o', obj])
     return obj
 
-  with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+  host_compile, host_link = _host_commands()
+  with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as pool:
+    host = pool.submit(_run, host_compile)
     objs = list(pool.map(compile_one, SOURCES.items()))
+    host.result()
   _run([hipcc, '--offload-arch=gfx950', '-shared', '-fPIC', '-o', LIB_PATH] + objs)
+  _run(host_link)
   with open(STAMP_PATH, 'w') as f:
     f.write(source_hash() + '\n')
   if verbose:
-    print('built', LIB_PATH)
+    print('built', LIB_PATH, HOST_PATH)
   return LIB_PATH
 
 

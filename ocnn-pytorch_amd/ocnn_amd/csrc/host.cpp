@@ -1,0 +1,498 @@
+// Host path of the layers: what runs between a module's forward() and the launches of the C ABI,
+// natively.  A small layer's kernels take a few dozen microseconds; the same calls made from Python
+// (argument lists through ctypes, a Python autograd node, the interpreter lock in the backward
+// thread) took 100 - 150.
+//
+// A GatherOp / WgradOp is one pass of a layer with everything that depends on the shapes and the
+// table only - which kernel, the plan's arrays and figures, the workspace size - decided when it is
+// made (nn/octree_conv.py); run() allocates the result and a workspace and calls the library.  A
+// ConvLayer holds the up to three passes of a layer on an octree; conv() is its autograd node.
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <memory>
+#include <optional>
+#include <vector>
+
+#include "ocnn_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+void check(int rc) { TORCH_CHECK(rc == 0, "libocnn_hip: ", ocnn_last_error(), " (code ", rc, ")"); }
+
+void* hip_stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+int code_of(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return OCNN_F32;
+    case at::kHalf: return OCNN_F16;
+    case at::kBFloat16: return OCNN_BF16;
+    default: TORCH_CHECK_TYPE(false, "unsupported feature dtype ", t, "; use float32, float16 or bfloat16");
+  }
+}
+
+void require_gpu(const Tensor& t) {
+  TORCH_CHECK(t.is_cuda(), "ocnn_amd kernels need tensors on a HIP device, got a tensor on ", t.device());
+}
+
+const void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+const void* ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
+template <typename T> T* typed(const Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
+
+Tensor workspace(int64_t bytes, const Tensor& like) {
+  return at::empty({std::max<int64_t>(bytes, 256)}, like.options().dtype(at::kByte));
+}
+
+// The arrays and figures of a tile plan and, where a kernel walks pairs, of its pair plan.
+struct PlanArrays {
+  Tensor loc, uptr, urows;
+  int umax = 0;
+  int64_t total = 0;
+  double occupancy = 1.0;
+  Tensor cptr, ent, lists;                    // pair plan
+  int64_t n_blocks = 0;
+  int max_blocks = 0, n_lists = 0;
+  std::vector<int32_t> lists_host, group_bounds;
+  std::vector<int64_t> list_count;
+};
+
+// codes on top of the library's OCNN_GATHER_* / OCNN_WGRAD_*
+constexpr int kWgradSparseInverse = 5;        // the pair plan of the inverse table, operands exchanged
+
+struct GatherOp {
+  int kernel = OCNN_GATHER_PLAIN, K = 0, cin = 0, cout = 0;
+  int64_t rows_in = 0, rows = 0, ws_bytes = 0;
+  bool transposed = false, reverse = false;
+  std::shared_ptr<PlanArrays> plan;
+  // dense one-slot form: rows read / written through an index of the non-empty nodes
+  Tensor in_index, out_index, children;
+  int64_t rows_all = 0;                       // rows of the padded result
+  // the rows of tiles that are too dense for the plan: table, places in the result, their own pass
+  Tensor overflow_table, overflow_rows;
+  int bias_repeat = 1, view_cols = 0;         // dense form: bias once per child; result seen with this many columns
+  std::shared_ptr<GatherOp> overflow, padded; // padded: this pass with channels in whole multiples (zero-padded)
+
+  Tensor run(Tensor data, Tensor table, Tensor W, OptTensor bias) const {
+    require_gpu(data);
+    require_gpu(W);
+    const int code = code_of(data.scalar_type());
+    data = data.contiguous();
+    W = W.contiguous();
+    TORCH_CHECK(W.scalar_type() == data.scalar_type() && W.numel() == (int64_t)K * cin * cout,
+                "weights do not match the table and channels");
+    if (bias.has_value()) {
+      bias = bias->to(data.scalar_type()).contiguous();
+      if (bias_repeat > 1) bias = bias->repeat({bias_repeat});
+    }
+    if (padded) return run_padded(data, table, W, bias);
+    void* st = hip_stream();
+    const bool wide_out = kernel == OCNN_GATHER_DENSE_RW && out_index.defined();
+    Tensor out = at::empty({wide_out ? rows_all : rows, cout}, data.options());
+    Tensor ws = workspace(ws_bytes, data);
+    const PlanArrays* p = plan.get();
+    switch (kernel) {
+      case OCNN_GATHER_DENSE_RW: {
+        const int64_t in_rows = data.numel() / cin;
+        check(ocnn_conv_dense_rw_indexed(code, ptr(data), in_rows, typed<int32_t>(in_index), rows, ptr(W), cin, cout,
+                                         transposed, ptr(bias), out.data_ptr(), out.size(0), typed<int32_t>(out_index),
+                                         ws.data_ptr(), ws.numel(), st));
+        if (out_index.defined())              // zeros for the empty nodes
+          check(ocnn_pad(code, nullptr, typed<int32_t>(children), rows_all, cout, 0.f, out.data_ptr(), st));
+        break;
+      }
+      case OCNN_GATHER_DENSE:
+        check(ocnn_conv_dense(code, ptr(data), rows, ptr(W), cin, cout, transposed, ptr(bias), out.data_ptr(),
+                              ws.data_ptr(), ws.numel(), st));
+        break;
+      case OCNN_GATHER_RW:
+        check(ocnn_conv_gather_rw(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
+                                  typed<int32_t>(p->urows), p->umax, p->total, rows, K, ptr(W), cin, cout, transposed,
+                                  reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        break;
+      case OCNN_GATHER_WIDE:
+        check(ocnn_conv_gather_wide(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
+                                    typed<int32_t>(p->urows), p->umax, p->total, p->occupancy, rows, K, ptr(W), cin,
+                                    cout, transposed, reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(),
+                                    st));
+        break;
+      case OCNN_GATHER_SPARSE:
+        check(ocnn_conv_gather_sparse(code, ptr(data), rows_in, typed<int32_t>(p->uptr), typed<int32_t>(p->urows),
+                                      p->umax, p->total, typed<int32_t>(p->cptr), typed<uint32_t>(p->ent), p->n_blocks,
+                                      p->max_blocks, typed<int32_t>(p->lists), p->n_lists, p->group_bounds.data(),
+                                      rows, K, ptr(W), cin, cout, transposed, reverse, ptr(bias), out.data_ptr(),
+                                      ws.data_ptr(), ws.numel(), st));
+        break;
+      case OCNN_GATHER_PLANNED:
+        check(ocnn_conv_gather_planned(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
+                                       typed<int32_t>(p->urows), rows, K, ptr(W), cin, cout, transposed, reverse,
+                                       ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        break;
+      default:
+        TORCH_CHECK(table.defined(), "this pass needs the neighbour table");
+        require_gpu(table);
+        TORCH_CHECK(table.scalar_type() == at::kInt && table.is_contiguous() && table.numel() == rows * K,
+                    "conv_gather: the table does not match");
+        check(ocnn_conv_gather(code, ptr(data), rows_in, typed<int32_t>(table), rows, K, ptr(W), cin, cout, transposed,
+                               reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
+    }
+    if (overflow) out.index_copy_(0, overflow_rows, overflow->run(data, overflow_table, W, bias));
+    return view_cols ? out.view({-1, view_cols}) : out;
+  }
+
+ private:
+  Tensor run_padded(const Tensor& data, const Tensor& table, const Tensor& W, const OptTensor& bias) const {
+    const int pi = padded->cin - cin, po = padded->cout - cout;
+    Tensor Wk = transposed ? W.view({K, cout, cin}) : W.view({K, cin, cout});
+    Wk = transposed ? at::constant_pad_nd(Wk, {0, pi, 0, po}) : at::constant_pad_nd(Wk, {0, po, 0, pi});
+    OptTensor b;
+    if (bias.has_value()) b = at::constant_pad_nd(*bias, {0, po});
+    // (the dense form may come as the rows of the children: eight rows of a table row's channels)
+    const Tensor rows_in_view = data.view({-1, cin});
+    Tensor out = padded->run(pi ? at::constant_pad_nd(rows_in_view, {0, pi}) : rows_in_view, table, Wk, b);
+    return po ? out.slice(1, 0, cout).contiguous() : out;
+  }
+};
+
+struct WgradOp {
+  int kernel = OCNN_WGRAD_PLAIN, K = 0, ca = 0, cb = 0;
+  int64_t rows_x = 0, rows = 0, ws_bytes = 0;
+  bool out_transposed = false;
+  std::shared_ptr<PlanArrays> plan;
+  Tensor g_index;                             // dense one-slot form: row i of the sum takes row g_index[i] of g
+  std::vector<int64_t> shape;                 // shape the result is seen with, if not (K, ca, cb)
+  Tensor overflow_table, overflow_rows;
+  std::shared_ptr<WgradOp> overflow, padded;
+
+  Tensor run(Tensor x, Tensor g, Tensor table) const {
+    require_gpu(x);
+    require_gpu(g);
+    const int code = code_of(x.scalar_type());
+    TORCH_CHECK(x.scalar_type() == g.scalar_type(), "conv_wgrad: operands of different types");
+    x = x.contiguous();
+    g = g.contiguous();
+    if (padded) {
+      x = x.view({-1, ca});
+      const int pa = padded->ca - ca, pb = padded->cb - cb;
+      Tensor gw = padded->run(pa ? at::constant_pad_nd(x, {0, pa}) : x, pb ? at::constant_pad_nd(g, {0, pb}) : g, table);
+      gw = out_transposed ? gw.slice(1, 0, cb).slice(2, 0, ca) : gw.slice(1, 0, ca).slice(2, 0, cb);
+      gw = gw.contiguous();
+      return shape.empty() ? gw : gw.view(shape);
+    }
+    void* st = hip_stream();
+    Tensor gw = at::empty({K, out_transposed ? cb : ca, out_transposed ? ca : cb}, x.options());
+    Tensor ws = workspace(ws_bytes, x);
+    const PlanArrays* p = plan.get();
+    switch (kernel) {
+      case OCNN_WGRAD_DENSE_RW:
+        check(ocnn_conv_dense_wgrad_rw_indexed(code, ptr(x), x.numel() / ca, nullptr, ptr(g), g.size(0),
+                                               typed<int32_t>(g_index), rows, ca, cb, out_transposed, gw.data_ptr(),
+                                               ws.data_ptr(), ws.numel(), st));
+        break;
+      case OCNN_WGRAD_SPARSE:
+        check(ocnn_conv_wgrad_sparse(code, ptr(x), rows_x, ca, ptr(g), rows, cb, typed<int32_t>(p->uptr),
+                                     typed<int32_t>(p->urows), p->umax, p->total, typed<int32_t>(p->cptr),
+                                     typed<uint32_t>(p->ent), p->n_blocks, p->lists_host.data(), p->list_count.data(),
+                                     p->n_lists, K, !out_transposed, gw.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        break;
+      case kWgradSparseInverse:               // rows: those of x, which are the rows of the inverse table
+        check(ocnn_conv_wgrad_sparse(code, ptr(g), rows_x, cb, ptr(x), rows, ca, typed<int32_t>(p->uptr),
+                                     typed<int32_t>(p->urows), p->umax, p->total, typed<int32_t>(p->cptr),
+                                     typed<uint32_t>(p->ent), p->n_blocks, p->lists_host.data(), p->list_count.data(),
+                                     p->n_lists, K, out_transposed, gw.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        if (overflow) gw.add_(overflow->run(g, x.index_select(0, overflow_rows), overflow_table));
+        return gw;
+      case OCNN_WGRAD_PLANNED:
+        check(ocnn_conv_wgrad_planned(code, ptr(x), rows_x, ptr(g), typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
+                                      typed<int32_t>(p->urows), p->umax, p->total, rows, K, ca, cb, out_transposed,
+                                      gw.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        break;
+      default:
+        TORCH_CHECK(table.defined(), "this pass needs the neighbour table");
+        require_gpu(table);
+        TORCH_CHECK(table.scalar_type() == at::kInt && table.is_contiguous() && table.numel() == rows * K,
+                    "conv_wgrad: the table does not match");
+        check(ocnn_conv_wgrad(code, ptr(x), rows_x, ptr(g), typed<int32_t>(table), rows, K, ca, cb, out_transposed,
+                              gw.data_ptr(), ws.data_ptr(), ws.numel(), st));
+    }
+    if (overflow) gw.add_(overflow->run(x, g.index_select(0, overflow_rows), overflow_table));
+    return shape.empty() ? gw : gw.view(shape);
+  }
+};
+
+Tensor column_sum(Tensor g) {
+  require_gpu(g);
+  g = g.contiguous();
+  Tensor out = at::empty({g.size(1)}, g.options());
+  Tensor ws = workspace(ocnn_colsum_workspace_bytes(g.size(0), (int)g.size(1)), g);
+  check(ocnn_colsum(code_of(g.scalar_type()), ptr(g), g.size(0), (int)g.size(1), out.data_ptr(), ws.data_ptr(),
+                    ws.numel(), hip_stream()));
+  return out;
+}
+
+// The passes of one layer on one octree, in one data type.  fwd: data -> out; dgrad: grad -> data
+// gradient; wgrad over (data, grad), for a deconvolution over (grad, data).  The backward passes are
+// made when a call first needs them.
+struct ConvLayer {
+  std::shared_ptr<GatherOp> fwd, dgrad;
+  std::shared_ptr<WgradOp> wgrad;
+  Tensor fwd_table, dgrad_table, wgrad_table;
+  bool wgrad_of_grad = false;                 // deconvolution: x = grad (the fine side), g = data
+};
+
+// ---- autograd nodes ---------------------------------------------------------------------------
+
+// The node behind `out` when a gradient can be asked for: its edges lead to `inputs`.
+template <typename N> std::shared_ptr<N> make_node(const variable_list& inputs) {
+  auto node = std::shared_ptr<N>(new N(), torch::autograd::deleteNode);
+  node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+  return node;
+}
+
+bool any_requires_grad(const variable_list& v) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor& t : v)
+    if (t.defined() && t.requires_grad()) return true;
+  return false;
+}
+
+struct ConvBackward : public Node {
+  SavedVariable data, weights;
+  std::shared_ptr<ConvLayer> layer;
+
+  variable_list apply(variable_list&& grads) override {
+    variable_list out(3);
+    if (!grads[0].defined()) return out;
+    Tensor grad = grads[0].contiguous(), x = data.unpack(), w = weights.unpack();
+    at::AutoDispatchBelowADInplaceOrView below;
+    if (task_should_compute_output(0)) out[0] = layer->dgrad->run(grad, layer->dgrad_table, w, std::nullopt);
+    if (task_should_compute_output(1))
+      out[1] = layer->wgrad_of_grad ? layer->wgrad->run(grad, x, layer->wgrad_table)
+                                    : layer->wgrad->run(x, grad, layer->wgrad_table);
+    if (task_should_compute_output(2)) out[2] = column_sum(grad);
+    return out;
+  }
+  void release_variables() override {
+    data.reset_data();
+    weights.reset_data();
+  }
+  std::string name() const override { return "OctreeConvBackward"; }
+};
+
+Tensor conv(const std::shared_ptr<ConvLayer>& layer, const Tensor& data_in, const Tensor& weights, const OptTensor& bias) {
+  const variable_list inputs{data_in, weights, bias.has_value() ? *bias : Tensor()};
+  const bool track = any_requires_grad(inputs);
+  Tensor data, w, out;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    data = data_in.contiguous();
+    w = weights.to(data.scalar_type()).contiguous();
+    out = layer->fwd->run(data, layer->fwd_table, w, bias);
+  }
+  if (track) {
+    auto node = make_node<ConvBackward>(inputs);
+    node->data = SavedVariable(data, false);
+    node->weights = SavedVariable(w, false);
+    node->layer = layer;
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+// ---- batch norm (nn/batchnorm.py) -------------------------------------------------------------
+
+// A per-channel parameter as the kernels read it (f32 / f16 / bf16, contiguous).
+Tensor as_param(const Tensor& t) {
+  if (!t.defined()) return t;
+  const auto k = t.scalar_type();
+  return (k == at::kFloat || k == at::kHalf || k == at::kBFloat16 ? t : t.to(at::kFloat)).contiguous();
+}
+
+int param_code(const Tensor& gamma, const Tensor& beta) {
+  const Tensor& t = gamma.defined() ? gamma : beta;
+  return t.defined() ? code_of(t.scalar_type()) : OCNN_F32;
+}
+
+struct BatchNormBackward : public Node {
+  SavedVariable x, mean, invstd, gamma, beta, y;
+  bool relu = false, training = false, has_residual = false, keeps_y = false;
+  at::ScalarType wdtype = at::kFloat, bdtype = at::kFloat;
+
+  variable_list apply(variable_list&& grads) override {
+    variable_list out(4);
+    if (!grads[0].defined()) return out;
+    Tensor dy = grads[0].contiguous(), xs = x.unpack(), mu = mean.unpack(), is = invstd.unpack();
+    Tensor ga = gamma.unpack(), be = beta.unpack(), ys;
+    if (keeps_y) ys = y.unpack(shared_from_this());
+    at::AutoDispatchBelowADInplaceOrView below;
+    const int64_t rows = xs.size(0), c = xs.size(1);
+    const auto f32 = xs.options().dtype(at::kFloat);
+    Tensor sums = at::empty({2, c}, f32);                     // dgamma, dbeta
+    const bool want_res = has_residual && task_should_compute_output(3);
+    Tensor dx, dres, gw, gb;
+    if (task_should_compute_output(0) || want_res) dx = at::empty_like(xs);
+    if (want_res) dres = at::empty_like(xs);
+    // the parameter gradients come out in the parameters' dtype where the kernels hold it
+    const bool want_w = ga.defined() && task_should_compute_output(1), want_b = be.defined() && task_should_compute_output(2);
+    if (want_w && wdtype == ga.scalar_type()) gw = at::empty({c}, ga.options());
+    if (want_b && bdtype == be.scalar_type() && (!ga.defined() || be.scalar_type() == ga.scalar_type()))
+      gb = at::empty({c}, be.options());
+    Tensor ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), xs);
+    float* s = (float*)sums.data_ptr();
+    check(ocnn_batch_norm_backward(code_of(xs.scalar_type()), ptr(xs), ptr(dy), rows, (int)c, (const float*)ptr(mu),
+                                   (const float*)ptr(is), ptr(ga), ptr(be), param_code(ga, be), relu, training, ptr(ys),
+                                   typed<void>(dx), typed<void>(dres), s, s + c, typed<void>(gw), typed<void>(gb),
+                                   ws.data_ptr(), ws.numel(), hip_stream()));
+    if (want_w && !gw.defined()) gw = sums[0].to(wdtype);
+    if (want_b && !gb.defined()) gb = sums[1].to(bdtype);
+    if (task_should_compute_output(0)) out[0] = dx;
+    out[1] = gw;
+    out[2] = gb;
+    out[3] = dres;
+    return out;
+  }
+  void release_variables() override {
+    for (SavedVariable* v : {&x, &mean, &invstd, &gamma, &beta, &y}) v->reset_data();
+  }
+  std::string name() const override { return "BatchNormReluBackward"; }
+};
+
+// batch_stats: statistics of this batch (and, with track, the running ones moved by `factor`);
+// otherwise the running statistics.  count: num_batches_tracked, incremented with the statistics.
+Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, const Tensor& running_mean,
+                  const Tensor& running_var, const Tensor& count, bool batch_stats, bool track, double factor, double eps,
+                  bool relu, const Tensor& residual_in) {
+  const variable_list inputs{x_in, weight, bias, residual_in};
+  const bool grad = any_requires_grad(inputs);
+  Tensor x, mean, invstd, gamma, beta, y;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    x = x_in.contiguous();
+    const int64_t rows = x.size(0), c = x.size(1);
+    const int code = code_of(x.scalar_type());
+    void* st = hip_stream();
+    gamma = as_param(weight);
+    beta = as_param(bias);
+    if (gamma.defined() && beta.defined() && beta.scalar_type() != gamma.scalar_type()) beta = beta.to(gamma.scalar_type());
+    if (batch_stats) {
+      Tensor stats = at::empty({3, c}, x.options().dtype(at::kFloat));
+      mean = stats[0];
+      invstd = stats[2];
+      Tensor var = stats[1], ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), x);
+      const auto known = [](const Tensor& t) {
+        return t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16;
+      };
+      const bool moves = track && running_mean.defined();
+      const bool in_place = moves && known(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
+                            running_mean.is_contiguous() && running_var.is_contiguous();
+      check(ocnn_batch_norm_stats(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
+                                  (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
+                                  in_place ? running_var.data_ptr() : nullptr,
+                                  in_place ? code_of(running_mean.scalar_type()) : 0, in_place ? (float)factor : 0.f,
+                                  typed<int64_t>(count), ws.data_ptr(), ws.numel(), st));
+      if (moves && !in_place) {
+        Tensor unbiased = var * ((double)rows / (double)std::max<int64_t>(rows - 1, 1));
+        running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
+        running_var.mul_(1 - factor).add_(unbiased.to(running_var.scalar_type()), factor);
+      }
+    } else {
+      mean = running_mean.to(at::kFloat).contiguous();
+      invstd = at::rsqrt(running_var.to(at::kFloat) + eps);
+    }
+    y = at::empty_like(x);
+    Tensor residual;
+    if (residual_in.defined()) {
+      residual = residual_in.contiguous();
+      TORCH_CHECK(residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type(),
+                  "batch_norm: the residual does not match the input");
+    }
+    check(ocnn_batch_norm_apply(code, ptr(x), rows, (int)c, (const float*)mean.data_ptr(), (const float*)invstd.data_ptr(),
+                                ptr(gamma), ptr(beta), param_code(gamma, beta), relu, ptr(residual), y.data_ptr(), st));
+  }
+  if (grad) {
+    auto node = make_node<BatchNormBackward>(inputs);
+    node->relu = relu;
+    node->training = batch_stats;
+    node->has_residual = residual_in.defined();
+    node->keeps_y = node->has_residual && relu;   // with a residual the ReLU's mask is not a function of x alone
+    if (weight.defined()) node->wdtype = weight.scalar_type();
+    if (bias.defined()) node->bdtype = bias.scalar_type();
+    node->x = SavedVariable(x, false);
+    node->mean = SavedVariable(mean, false);
+    node->invstd = SavedVariable(invstd, false);
+    if (gamma.defined()) node->gamma = SavedVariable(gamma, false);
+    if (beta.defined()) node->beta = SavedVariable(beta, false);
+    torch::autograd::set_history(y, node);
+    if (node->keeps_y) node->y = SavedVariable(y, true);
+  }
+  return y;
+}
+
+Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+}  // namespace
+
+PYBIND11_MODULE(ocnn_host, m) {
+  namespace py = pybind11;
+  py::class_<PlanArrays, std::shared_ptr<PlanArrays>>(m, "PlanArrays")
+      .def(py::init<>())
+#define FIELD(name) .def_readwrite(#name, &PlanArrays::name)
+      FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(umax) FIELD(total) FIELD(occupancy) FIELD(cptr) FIELD(ent) FIELD(lists)
+          FIELD(n_blocks) FIELD(max_blocks) FIELD(n_lists) FIELD(lists_host) FIELD(group_bounds) FIELD(list_count);
+#undef FIELD
+  py::class_<GatherOp, std::shared_ptr<GatherOp>>(m, "GatherOp")
+      .def(py::init<>())
+#define FIELD(name) .def_readwrite(#name, &GatherOp::name)
+      FIELD(kernel) FIELD(K) FIELD(cin) FIELD(cout) FIELD(rows_in) FIELD(rows) FIELD(ws_bytes) FIELD(transposed)
+          FIELD(reverse) FIELD(plan) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
+              FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded) FIELD(bias_repeat) FIELD(view_cols)
+#undef FIELD
+      .def("copy", [](const GatherOp& op) { return std::make_shared<GatherOp>(op); })
+      .def("run", [](const GatherOp& op, const Tensor& data, const OptTensor& table, const Tensor& W, const OptTensor& bias) {
+        pybind11::gil_scoped_release free;
+        at::AutoDispatchBelowADInplaceOrView below;
+        return op.run(data, or_undefined(table), W, bias);
+      });
+  py::class_<WgradOp, std::shared_ptr<WgradOp>>(m, "WgradOp")
+      .def(py::init<>())
+#define FIELD(name) .def_readwrite(#name, &WgradOp::name)
+      FIELD(kernel) FIELD(K) FIELD(ca) FIELD(cb) FIELD(rows_x) FIELD(rows) FIELD(ws_bytes) FIELD(out_transposed) FIELD(plan)
+          FIELD(g_index) FIELD(shape) FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded)
+#undef FIELD
+      .def("copy", [](const WgradOp& op) { return std::make_shared<WgradOp>(op); })
+      .def("seen_as", [](const WgradOp& op, std::vector<int64_t> shape) {
+        auto copy = std::make_shared<WgradOp>(op);
+        copy->shape = std::move(shape);
+        return copy;
+      })
+      .def("run", [](const WgradOp& op, const Tensor& x, const Tensor& g, const OptTensor& table) {
+        pybind11::gil_scoped_release free;
+        at::AutoDispatchBelowADInplaceOrView below;
+        return op.run(x, g, or_undefined(table));
+      });
+  py::class_<ConvLayer, std::shared_ptr<ConvLayer>>(m, "ConvLayer")
+      .def(py::init<>())
+#define FIELD(name) .def_readwrite(#name, &ConvLayer::name)
+      FIELD(fwd) FIELD(dgrad) FIELD(wgrad) FIELD(fwd_table) FIELD(dgrad_table) FIELD(wgrad_table) FIELD(wgrad_of_grad);
+#undef FIELD
+  m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;
+  m.def("conv", &conv, py::call_guard<py::gil_scoped_release>());
+  m.def("column_sum", &column_sum, py::call_guard<py::gil_scoped_release>());
+  m.def(
+      "batch_norm",
+      [](const Tensor& x, const OptTensor& w, const OptTensor& b, const OptTensor& rm, const OptTensor& rv,
+         const OptTensor& count, bool batch_stats, bool track, double factor, double eps, bool relu, const OptTensor& res) {
+        return batch_norm(x, or_undefined(w), or_undefined(b), or_undefined(rm), or_undefined(rv), or_undefined(count),
+                          batch_stats, track, factor, eps, relu, or_undefined(res));
+      },
+      py::call_guard<py::gil_scoped_release>());
+}

@@ -9,8 +9,9 @@ import torch
 import torch.nn
 import torch.nn.functional as F
 
+from . import _lib
 from .nn import OctreeConv, OctreeDeconv
-from .nn.octree_conv import conv_gather, conv_wgrad, column_sum
+from .nn.octree_conv import _gather_op, _wgrad_op, conv_wgrad, column_sum
 from .nn.batchnorm import BatchNormRelu1d
 
 
@@ -69,36 +70,24 @@ def _identity_table(rows, device):
   return _IDENTITY[key]
 
 
-class _RowsLinear(torch.autograd.Function):
+_LINEAR = {}
+
+
+def _rows_linear(x, weight, bias):
   """y = x W^T + b on many rows through the one-slot form of the convolution kernels
   (weights (out, in) as torch.nn.Linear holds them)."""
-
-  @staticmethod
-  def forward(ctx, x, weight, bias):
-    x = x.contiguous()
-    w = weight.to(x.dtype).contiguous()
-    ctx.save_for_backward(x, w)
-    ctx.has_bias = bias is not None
-    ctx.wdtype = weight.dtype
-    rows = x.shape[0]
-    return conv_gather(x, rows, _identity_table(rows, x.device), w.view(1, w.shape[0], w.shape[1]),
-                       w.shape[0], True, False, None if bias is None else bias.to(x.dtype), None, dense=True)
-
-  @staticmethod
-  def backward(ctx, grad):
-    x, w = ctx.saved_tensors
-    grad = grad.contiguous()
-    rows = x.shape[0]
-    table = _identity_table(rows, x.device)
-    gx = gw = gb = None
-    if ctx.needs_input_grad[0]:
-      gx = conv_gather(grad, rows, table, w.view(1, w.shape[0], w.shape[1]), w.shape[1], False, False,
-                       None, None, dense=True)
-    if ctx.needs_input_grad[1]:
-      gw = conv_wgrad(x, grad, table, True, None, dense=True).view(w.shape).to(ctx.wdtype)
-    if ctx.has_bias and ctx.needs_input_grad[2]:
-      gb = column_sum(grad)
-    return gx, gw, gb
+  rows, cin, cout = x.shape[0], weight.shape[1], weight.shape[0]
+  key = (rows, cin, cout, x.dtype, x.device)
+  layer = _LINEAR.get(key)
+  if layer is None:
+    if len(_LINEAR) > 64:
+      _LINEAR.clear()
+    layer = _LINEAR[key] = _lib.native().ConvLayer()
+    layer.fwd = _gather_op(x.dtype, rows, rows, 1, cin, cout, True, False, None, True)
+    layer.dgrad = _gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True)
+    layer.wgrad = _wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin])
+    layer.fwd_table = layer.dgrad_table = layer.wgrad_table = _identity_table(rows, x.device)
+  return _lib.native().conv(layer, x, weight, bias)
 
 
 class _RowsLinearNarrow(torch.autograd.Function):
@@ -142,7 +131,7 @@ class Conv1x1(torch.nn.Module):
     lin = self.linear
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 4096 and lin.in_features % 32 == 0 and lin.out_features % 16 == 0):
-      return _RowsLinear.apply(data, lin.weight, lin.bias)
+      return _rows_linear(data, lin.weight, lin.bias)
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 65536 and lin.in_features % 32 == 0 and lin.out_features < 16):
       return _RowsLinearNarrow.apply(data, lin.weight, lin.bias)

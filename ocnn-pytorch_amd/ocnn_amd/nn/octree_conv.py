@@ -11,7 +11,6 @@ table is centrally symmetric (stride 1, every kernel but 2x2x2) and through
 the inverse table otherwise, so no atomics are involved anywhere.
 """
 
-import ctypes
 from typing import List
 
 import torch
@@ -21,6 +20,7 @@ from torch.autograd import Function
 
 from .. import _lib
 from ..octree.contract import tables_of
+from ..octree.octree import Octree
 from ..utils import list2str, resize_with_last_val, xavier_uniform_
 from .octree2col import col2octree, octree2col
 from .octree_pad import _depad_raw, _pad_raw, octree_depad, octree_pad
@@ -30,7 +30,7 @@ from .octree_pad import _depad_raw, _pad_raw, octree_depad, octree_pad
 # the layer level needs: when odd channel counts run zero-padded, and from how many rows on the
 # pair-plan kernels pay for loading their weights)
 PAD_MIN_ROWS = 16384
-_CHOICES = {}            # kernel choices of the calls without a plan, by shape (see _conv_gather)
+_OPS = {}                # passes without a plan, by shape (see _gather_op)
 SPARSE_MAX_OCCUPANCY = 0.3
 SPARSE_MIN_ROWS = 32768
 
@@ -67,6 +67,89 @@ def _block_map(kernel, device):
 
 
 
+def _plan_args(plan):
+  """(has_plan, max distinct rows, entries of the row lists, occupancy, reuse) for the
+  selection functions of the library."""
+  if plan is None:
+    return 0, 0, 0, 1.0, 0.0
+  return 1, plan.umax, plan.total, float(plan.occupancy), float(plan.reuse)
+
+
+def _plan_arrays(plan, pairs):
+  """The native view of a tile plan, with its pair plan when `pairs`; kept with the plan."""
+  name = '_native_pairs' if pairs else '_native'
+  arrays = plan.__dict__.get(name)
+  if arrays is None:
+    arrays = _lib.native().PlanArrays()
+    arrays.loc, arrays.uptr, arrays.urows = plan.loc, plan.uptr, plan.urows
+    arrays.umax, arrays.total, arrays.occupancy = plan.umax, plan.total, float(plan.occupancy)
+    if pairs:
+      pp = plan.pairs()
+      arrays.cptr, arrays.ent, arrays.lists = pp.cptr, pp.ent, pp.lists
+      arrays.n_blocks, arrays.max_blocks, arrays.n_lists = pp.n_blocks, pp.max_blocks, pp.n_lists
+      arrays.lists_host, arrays.list_count = list(pp.lists_host), list(pp.list_count_host)
+      arrays.group_bounds = list(pp.group_bounds_host)
+    plan.__dict__[name] = arrays
+  return arrays
+
+
+def _memo(plan):
+  """Where the passes made for a plan are kept: with it; those without a plan by shape."""
+  memo = _OPS if plan is None else plan.__dict__.setdefault('_ops', {})
+  if len(memo) > 256:
+    memo.clear()
+  return memo
+
+
+def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=None, dense=False):
+  """The gather-GEMM of a shape as a native pass (csrc/host.cpp).  The library picks the kernel
+  (ocnn_conv_gather_choose); the choice depends on the shapes and the plan only, so the pass is
+  made once per plan.  The few tiles that are too dense for a plan get a pass of their own on the
+  plan-free kernel, its rows put in place afterwards."""
+  memo, key = _memo(plan), ('g', dtype, rows_in, rows, K, cin, cout, transposed, reverse, dense)
+  op = memo.get(key)
+  if op is not None:
+    return op
+  L, code = _lib.lib(), _lib.dtype_code_of(dtype)
+  op = _lib.native().GatherOp()
+  op.rows_in, op.rows, op.K, op.cin, op.cout, op.transposed, op.reverse = rows_in, rows, K, cin, cout, transposed, reverse
+  op.kernel = L.ocnn_conv_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan))
+  if op.kernel == _lib.GATHER_ZERO_PADDED:
+    op.padded = _gather_op(dtype, rows_in, rows, K, -(-cin // 32) * 32, -(-cout // 16) * 16, transposed, reverse, plan)
+  else:
+    sparse = op.kernel == _lib.GATHER_SPARSE
+    op.ws_bytes = (L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout) if sparse
+                   else L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
+    if op.kernel in (_lib.GATHER_RW, _lib.GATHER_WIDE, _lib.GATHER_PLANNED, _lib.GATHER_SPARSE):
+      op.plan = _plan_arrays(plan, sparse)
+      if plan.overflow_rows is not None:
+        op.overflow_rows, op.overflow_table = plan.overflow_rows, plan.overflow_table
+        op.overflow = _gather_op(dtype, rows_in, plan.overflow_table.shape[0], K, cin, cout, transposed, reverse)
+  memo[key] = op
+  return op
+
+
+def _indexed_gather_op(dtype, rows, data_rows, cin, cout, transposed, in_index=None, pad_to=None):
+  """The dense one-slot pass that reads its rows through `in_index` (int32) and / or writes them
+  through the index of the non-empty nodes (pad_to = (octree, depth)).  None when the kernel does
+  not take the shape: the indexed form also addresses the tensors over all nodes with 32-bit
+  offsets."""
+  L = _lib.lib()
+  base = _gather_op(dtype, rows, rows, 1, cin, cout, transposed, False, None, True)
+  n_out = rows if pad_to is None else int(pad_to[0].nnum[pad_to[1]])
+  if base.kernel != _lib.GATHER_DENSE_RW or \
+      not L.ocnn_conv_dense_rw_supported(_lib.dtype_code_of(dtype), max(data_rows, n_out), cin, cout):
+    return None
+  op = base.copy()
+  if in_index is not None:
+    op.in_index = in_index
+  if pad_to is not None:
+    octree, depth = pad_to
+    op.out_index, op.children, op.rows_all = octree._nempty_index32(depth), octree.children[depth], n_out
+    assert op.out_index.numel() == rows, 'conv_gather: one result row per non-empty node'
+  return op
+
+
 def conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias=None, plan=None, dense=False,
                 in_index=None, pad_to=None):
   """out (rows, cout) = gather-GEMM over `table` (int32, (rows, K)).  With a
@@ -77,121 +160,61 @@ def conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias=None, p
   all nodes without a depad pass).
   pad_to = (octree, depth) (with dense only): the result comes back as octree_pad would make it,
   a row for every node of `depth`, zeros for the empty ones: the kernel writes its rows there."""
-  if pad_to is not None:
-    if not dense:
-      return _pad_raw(conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias, plan, dense, in_index),
-                      *pad_to)
-    return _conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias, None, dense, in_index, pad_to)[0]
-  out, planned = _conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias, plan, dense, in_index)
-  if planned and plan is not None and plan.overflow_rows is not None:
-    # the few tiles that are too dense for the plan: plan-free kernel, results put in place
-    sub, _ = _conv_gather(data, rows_in, plan.overflow_table, W, cout, transposed, reverse, bias, None, False)
-    out.index_copy_(0, plan.overflow_rows, sub)
-  return out
-
-
-def _plan_args(plan):
-  """(has_plan, max distinct rows, entries of the row lists, occupancy, reuse) for the
-  selection functions of the library."""
-  if plan is None:
-    return 0, 0, 0, 1.0, 0.0
-  return 1, plan.umax, plan.total, float(plan.occupancy), float(plan.reuse)
-
-
-def _conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias, plan, dense, in_index=None, pad_to=None):
-  """conv_gather without the overflow rows of the plan; also returns whether a kernel on
-  the plan ran.  The library picks the kernel (ocnn_conv_gather_choose)."""
   _lib.require_gpu(data, table, W)
-  L = _lib.lib()
-  data, W, table = data.contiguous(), W.contiguous(), table.contiguous()
+  table = table.contiguous()
   rows, K = table.shape
-  cin = data.shape[1]
-  assert W.dtype == data.dtype and table.dtype == torch.int32
+  cin, dtype = data.shape[1], data.dtype
+  assert W.dtype == dtype and table.dtype == torch.int32
   assert W.numel() == K * cin * cout, 'weights do not match the table and channels'
-  if bias is not None:
-    bias = bias.to(data.dtype).contiguous()
-  code = _lib.dtype_code(data)
-  # (the choice and the workspace size depend on the shapes and the plan only: asked once per plan)
-  memo = _CHOICES if plan is None else plan.__dict__.setdefault('_choices', {})
-  key = ('g', code, rows_in, rows, K, cin, cout, bool(dense))
-  picked = memo.get(key)
-  if picked is None:
-    if len(memo) > 256:
-      memo.clear()
-    picked = memo[key] = (L.ocnn_conv_gather_choose(code, rows_in, rows, K, cin, cout, int(bool(dense)),
-                                                     *_plan_args(plan)),
-                          L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
-  kernel, ws_bytes = picked
-  if kernel == _lib.GATHER_DENSE_RW and (in_index is not None or pad_to is not None):
-    # the indexed form also addresses the tensors over all nodes with 32-bit offsets: past that
-    # range the rows are copied out (depad) / in (pad) around the kernel on the compact rows
-    n_all = max(data.shape[0], rows if pad_to is None else int(pad_to[0].nnum[pad_to[1]]))
-    if not L.ocnn_conv_dense_rw_supported(code, n_all, cin, cout):
-      if in_index is not None:
-        data, in_index = data.index_select(0, in_index.long()), None
-      out, planned = _conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias, plan, dense)
-      return (out if pad_to is None else _pad_raw(out, *pad_to)), planned
-  if in_index is not None and kernel != _lib.GATHER_DENSE_RW:
-    data, in_index = data.index_select(0, in_index.long()), None       # the other kernels take compact rows
-  if pad_to is not None and kernel != _lib.GATHER_DENSE_RW:          # the other kernels write compact rows
-    out, planned = _conv_gather(data, rows_in, table, W, cout, transposed, reverse, bias, plan, dense, in_index)
-    return _pad_raw(out, *pad_to), planned
-  if kernel == _lib.GATHER_ZERO_PADDED:
-    cin_p, cout_p = -(-cin // 32) * 32, -(-cout // 16) * 16
-    Wk = W.view(K, cout, cin) if transposed else W.view(K, cin, cout)
-    pad_w = (0, cin_p - cin, 0, cout_p - cout) if transposed else (0, cout_p - cout, 0, cin_p - cin)
-    out = conv_gather(F.pad(data, (0, cin_p - cin)), rows_in, table, F.pad(Wk, pad_w), cout_p,
-                      transposed, reverse, None if bias is None else F.pad(bias, (0, cout_p - cout)), plan)
-    return out[:, :cout].contiguous(), False
-  ws = _lib.workspace(ws_bytes, data.device)
-  if kernel == _lib.GATHER_DENSE_RW:
-    out_index, n_out = None, rows
-    if pad_to is not None:
-      octree, depth = pad_to
-      out_index, n_out = octree._nempty_index32(depth), int(octree.nnum[depth])
-      assert out_index.numel() == rows, 'conv_gather: one result row per non-empty node'
-    out = torch.empty((n_out, cout), dtype=data.dtype, device=data.device)
-    _lib.check(L.ocnn_conv_dense_rw_indexed(code, _lib.ptr(data), data.shape[0], _lib.ptr(in_index), rows,
-                                            _lib.ptr(W), cin, cout, int(transposed), _lib.ptr(bias), _lib.ptr(out),
-                                            n_out, _lib.ptr(out_index), _lib.ptr(ws), ws.numel(), _lib.stream()))
-    if pad_to is not None:                                            # zeros for the empty nodes
-      _lib.check(L.ocnn_pad(code, None, _lib.ptr(octree.children[depth]), n_out, cout, 0.0, _lib.ptr(out),
-                            _lib.stream()))
-    return out, False
-  out = torch.empty((rows, cout), dtype=data.dtype, device=data.device)
-  tail = (_lib.ptr(bias), _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream())
-  if kernel == _lib.GATHER_DENSE:
-    _lib.check(L.ocnn_conv_dense(code, _lib.ptr(data), rows, _lib.ptr(W), cin, cout, int(transposed), *tail))
-    return out, False
-  if kernel == _lib.GATHER_RW:
-    _lib.check(L.ocnn_conv_gather_rw(
-        code, _lib.ptr(data), rows_in, _lib.ptr(plan.loc), _lib.ptr(plan.uptr), _lib.ptr(plan.urows),
-        plan.umax, plan.total, rows, K, _lib.ptr(W), cin, cout, int(transposed), int(reverse), *tail))
-    return out, True
-  if kernel == _lib.GATHER_WIDE:
-    _lib.check(L.ocnn_conv_gather_wide(
-        code, _lib.ptr(data), rows_in, _lib.ptr(plan.loc), _lib.ptr(plan.uptr), _lib.ptr(plan.urows),
-        plan.umax, plan.total, float(plan.occupancy), rows, K, _lib.ptr(W), cin, cout, int(transposed),
-        int(reverse), *tail))
-    return out, True
-  if kernel == _lib.GATHER_SPARSE:
-    pp = plan.pairs()
-    ws = _lib.workspace(L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout), data.device)
-    _lib.check(L.ocnn_conv_gather_sparse(
-        code, _lib.ptr(data), rows_in, _lib.ptr(plan.uptr), _lib.ptr(plan.urows), plan.umax, plan.total,
-        _lib.ptr(pp.cptr), _lib.ptr(pp.ent), pp.n_blocks, pp.max_blocks, _lib.ptr(pp.lists), pp.n_lists,
-        ctypes.addressof(pp.group_bounds_host), rows, K, _lib.ptr(W), cin, cout, int(transposed), int(reverse),
-        _lib.ptr(bias), _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream()))
-    return out, True
-  if kernel == _lib.GATHER_PLANNED:
-    _lib.check(L.ocnn_conv_gather_planned(
-        code, _lib.ptr(data), rows_in, _lib.ptr(plan.loc), _lib.ptr(plan.uptr),
-        _lib.ptr(plan.urows), rows, K, _lib.ptr(W), cin, cout, int(transposed), int(reverse), *tail))
-    return out, True
-  _lib.check(L.ocnn_conv_gather(
-      code, _lib.ptr(data), rows_in, _lib.ptr(table), rows, K, _lib.ptr(W),
-      cin, cout, int(transposed), int(reverse), *tail))
-  return out, False
+  if dense and (in_index is not None or pad_to is not None):
+    op = _indexed_gather_op(dtype, rows, data.shape[0], cin, cout, bool(transposed), in_index, pad_to)
+    if op is not None:
+      return op.run(data, table, W, bias)
+  if in_index is not None:                                          # the other kernels take compact rows
+    data = data.index_select(0, in_index.long())
+  out = _gather_op(dtype, rows_in, rows, K, cin, cout, bool(transposed), bool(reverse), plan,
+                   bool(dense)).run(data, table, W, bias)
+  return out if pad_to is None else _pad_raw(out, *pad_to)           # .. and write compact rows
+
+
+def _wgrad_op(dtype, rows_x, rows, K, ca, cb, out_transposed, plan=None, dense=False):
+  """The weight gradient of a shape as a native pass; see _gather_op."""
+  memo, key = _memo(plan), ('w', dtype, rows_x, rows, K, ca, cb, out_transposed, dense)
+  op = memo.get(key)
+  if op is not None:
+    return op
+  L, code = _lib.lib(), _lib.dtype_code_of(dtype)
+  op = _lib.native().WgradOp()
+  op.rows_x, op.rows, op.K, op.ca, op.cb, op.out_transposed = rows_x, rows, K, ca, cb, out_transposed
+  op.kernel = L.ocnn_conv_wgrad_choose(code, rows_x, rows, K, ca, cb, int(dense), *_plan_args(plan)[:4])
+  if op.kernel == _lib.WGRAD_ZERO_PADDED:
+    op.padded = _wgrad_op(dtype, rows_x, rows, K, -(-ca // 32) * 32, -(-cb // 32) * 32, out_transposed, plan)
+  elif op.kernel == _lib.WGRAD_DENSE_RW:
+    op.ws_bytes = L.ocnn_conv_dense_wgrad_rw_workspace_bytes(ca, cb)
+  elif op.kernel == _lib.WGRAD_SPARSE:
+    op.ws_bytes = L.ocnn_conv_wgrad_sparse_workspace_bytes(rows, ca, cb)
+  elif op.kernel == _lib.WGRAD_PLANNED:
+    op.ws_bytes = L.ocnn_conv_wgrad_planned_workspace_bytes_for(code, rows_x, rows, K, ca, cb)
+  else:
+    op.ws_bytes = L.ocnn_conv_wgrad_workspace_bytes_for(code, rows_x, rows, K, ca, cb)
+  if op.kernel in (_lib.WGRAD_SPARSE, _lib.WGRAD_PLANNED):
+    op.plan = _plan_arrays(plan, op.kernel == _lib.WGRAD_SPARSE)
+    if plan.overflow_rows is not None:                   # (their share of the sums is added)
+      op.overflow_rows, op.overflow_table = plan.overflow_rows, plan.overflow_table
+      op.overflow = _wgrad_op(dtype, rows_x, plan.overflow_table.shape[0], K, ca, cb, out_transposed)
+  memo[key] = op
+  return op
+
+
+def _indexed_wgrad_op(dtype, rows, g_rows, ca, cb, g_index):
+  """The dense one-slot sums with row g_index[i] of g for row i, or None (see _indexed_gather_op)."""
+  base = _wgrad_op(dtype, rows, rows, 1, ca, cb, False, None, True)
+  if base.kernel != _lib.WGRAD_DENSE_RW or \
+      not _lib.lib().ocnn_conv_dense_wgrad_rw_supported(_lib.dtype_code_of(dtype), max(rows, g_rows), ca, cb):
+    return None
+  op = base.copy()
+  op.g_index = g_index
+  return op
 
 
 def conv_wgrad(x, g, table, out_transposed=False, plan=None, dense=False, g_index=None):
@@ -200,113 +223,49 @@ def conv_wgrad(x, g, table, out_transposed=False, plan=None, dense=False, g_inde
   dense: the table is the one-slot identity (row i reads row i).
   g_index (int32, with dense only): row i of the sum takes row g_index[i] of `g`, which may then
   have more rows than the table (see conv_gather)."""
-  gw, planned = _conv_wgrad(x, g, table, out_transposed, plan, dense, g_index)
-  if planned and plan is not None and plan.overflow_rows is not None:
-    # the few tiles that are too dense for the plan: their share of the sums, plan-free kernel
-    more, _ = _conv_wgrad(x, g.index_select(0, plan.overflow_rows), plan.overflow_table, out_transposed, None,
-                          False)
-    gw += more
-  return gw
-
-
-def _conv_wgrad(x, g, table, out_transposed, plan, dense, g_index=None):
-  """conv_wgrad without the overflow rows of the plan; also returns whether a kernel on the
-  plan ran.  The library picks the kernel (ocnn_conv_wgrad_choose)."""
   _lib.require_gpu(x, g, table)
-  L = _lib.lib()
-  x, g, table = x.contiguous(), g.contiguous(), table.contiguous()
+  table = table.contiguous()
   rows, K = table.shape
-  ca, cb = x.shape[1], g.shape[1]
-  code = _lib.dtype_code(x)
-  memo = _CHOICES if plan is None else plan.__dict__.setdefault('_choices', {})
-  key = ('w', code, x.shape[0], rows, K, ca, cb, bool(dense))
-  kernel = memo.get(key)
-  if kernel is None:
-    if len(memo) > 256:
-      memo.clear()
-    kernel = memo[key] = L.ocnn_conv_wgrad_choose(code, x.shape[0], rows, K, ca, cb, int(bool(dense)),
-                                                  *_plan_args(plan)[:4])
-  if g_index is not None and (kernel != _lib.WGRAD_DENSE_RW or
-                              not L.ocnn_conv_dense_wgrad_rw_supported(code, max(rows, g.shape[0]), ca, cb)):
-    # (the other kernels take compact rows, and so does the dense one past its 32-bit offset range)
-    g, g_index = g.index_select(0, g_index.long()), None
-  assert (g_index is not None or g.shape[0] == rows) and x.dtype == g.dtype and table.dtype == torch.int32
-  if kernel == _lib.WGRAD_ZERO_PADDED:
-    ca_p, cb_p = -(-ca // 32) * 32, -(-cb // 32) * 32
-    gw = conv_wgrad(F.pad(x, (0, ca_p - ca)), F.pad(g, (0, cb_p - cb)), table, out_transposed, plan)
-    return (gw[:, :cb, :ca] if out_transposed else gw[:, :ca, :cb]).contiguous(), False
-  shape = (K, cb, ca) if out_transposed else (K, ca, cb)
-  gw = torch.empty(shape, dtype=x.dtype, device=x.device)
-  if kernel == _lib.WGRAD_DENSE_RW:
-    ws = _lib.workspace(L.ocnn_conv_dense_wgrad_rw_workspace_bytes(ca, cb), x.device)
-    _lib.check(L.ocnn_conv_dense_wgrad_rw_indexed(code, _lib.ptr(x), x.shape[0], None, _lib.ptr(g), g.shape[0],
-                                                  _lib.ptr(g_index), rows, ca, cb, int(out_transposed),
-                                                  _lib.ptr(gw), _lib.ptr(ws), ws.numel(), _lib.stream()))
-    return gw, False
-  if kernel == _lib.WGRAD_SPARSE:
-    pp = plan.pairs()
-    ws = _lib.workspace(L.ocnn_conv_wgrad_sparse_workspace_bytes(rows, ca, cb), x.device)
-    _lib.check(L.ocnn_conv_wgrad_sparse(
-        code, _lib.ptr(x), x.shape[0], ca, _lib.ptr(g), rows, cb, _lib.ptr(plan.uptr), _lib.ptr(plan.urows),
-        plan.umax, plan.total, _lib.ptr(pp.cptr), _lib.ptr(pp.ent), pp.n_blocks,
-        ctypes.addressof(pp.lists_host), ctypes.addressof(pp.list_count_host), pp.n_lists, K,
-        int(not out_transposed), _lib.ptr(gw), _lib.ptr(ws), ws.numel(), _lib.stream()))
-    return gw, True
-  if kernel == _lib.WGRAD_PLANNED:
-    ws = _lib.workspace(L.ocnn_conv_wgrad_planned_workspace_bytes_for(code, x.shape[0], rows, K, ca, cb), x.device)
-    _lib.check(L.ocnn_conv_wgrad_planned(
-        code, _lib.ptr(x), x.shape[0], _lib.ptr(g), _lib.ptr(plan.loc), _lib.ptr(plan.uptr),
-        _lib.ptr(plan.urows), plan.umax, plan.total, rows, K, ca, cb, int(out_transposed),
-        _lib.ptr(gw), _lib.ptr(ws), ws.numel(), _lib.stream()))
-    return gw, True
-  ws = _lib.workspace(L.ocnn_conv_wgrad_workspace_bytes_for(code, x.shape[0], rows, K, ca, cb), x.device)
-  _lib.check(L.ocnn_conv_wgrad(
-      code, _lib.ptr(x), x.shape[0], _lib.ptr(g), _lib.ptr(table), rows, K, ca, cb,
-      int(out_transposed), _lib.ptr(gw), _lib.ptr(ws), ws.numel(), _lib.stream()))
-  return gw, False
+  ca, cb, dtype = x.shape[1], g.shape[1], x.dtype
+  assert dtype == g.dtype and table.dtype == torch.int32
+  if g_index is not None:
+    op = _indexed_wgrad_op(dtype, rows, g.shape[0], ca, cb, g_index) if dense and not out_transposed else None
+    if op is not None:
+      return op.run(x, g, table)
+    g = g.index_select(0, g_index.long())
+  assert g.shape[0] == rows
+  return _wgrad_op(dtype, x.shape[0], rows, K, ca, cb, bool(out_transposed), plan, bool(dense)).run(x, g, table)
 
 
-def conv_wgrad_inverse(x, g, plan_t, out_transposed=False):
+def _wgrad_inverse_op(dtype, rows_x, rows_g, cx, cg, out_transposed, plan_t):
   """The same sums as conv_wgrad, taken over the INVERSE table (row j, slot k -> the row i
   with table[i][k] == j; plan_t is its tile plan): gW[k] = sum_j x[j]^T (x) g[Tt[j,k]].  For
   tables in which every row is pointed at from one slot only (2x2x2 stride 2: a node has one
   parent) the inverse has 1 / K of its entries set and tiles of few distinct rows, which is
   what the pair-plan kernel is made for.  None when the kernel does not take the shape."""
-  _lib.require_gpu(x, g)
-  L = _lib.lib()
-  x, g = x.contiguous(), g.contiguous()
-  K = plan_t.K
-  cx, cg = x.shape[1], g.shape[1]
-  code = _lib.DTYPE_CODE.get(x.dtype, -1)
-  if not (plan_t.rows == x.shape[0] and plan_t.rows >= SPARSE_MIN_ROWS and
-          plan_t.occupancy <= SPARSE_MAX_OCCUPANCY and x.dtype == g.dtype and
-          L.ocnn_conv_wgrad_sparse_supported(code, g.shape[0], x.shape[0], K, cg, cx, plan_t.umax)):
+  L, K, code = _lib.lib(), plan_t.K, _lib.DTYPE_CODE.get(dtype, -1)
+  if not (plan_t.rows == rows_x and plan_t.rows >= SPARSE_MIN_ROWS and plan_t.occupancy <= SPARSE_MAX_OCCUPANCY and
+          L.ocnn_conv_wgrad_sparse_supported(code, rows_g, rows_x, K, cg, cx, plan_t.umax)):
     return None
-  pp = plan_t.pairs()
-  gw = torch.empty((K, cg, cx) if out_transposed else (K, cx, cg), dtype=x.dtype, device=x.device)
-  ws = _lib.workspace(L.ocnn_conv_wgrad_sparse_workspace_bytes(x.shape[0], cg, cx), x.device)
-  _lib.check(L.ocnn_conv_wgrad_sparse(
-      code, _lib.ptr(g), g.shape[0], cg, _lib.ptr(x), x.shape[0], cx, _lib.ptr(plan_t.uptr),
-      _lib.ptr(plan_t.urows), plan_t.umax, plan_t.total, _lib.ptr(pp.cptr), _lib.ptr(pp.ent), pp.n_blocks,
-      ctypes.addressof(pp.lists_host), ctypes.addressof(pp.list_count_host), pp.n_lists, K, int(out_transposed),
-      _lib.ptr(gw), _lib.ptr(ws), ws.numel(), _lib.stream()))
-  if plan_t.overflow_rows is not None:                     # (tiles too dense for the plan)
-    more, _ = _conv_wgrad(g, x.index_select(0, plan_t.overflow_rows), plan_t.overflow_table, not out_transposed,
-                          None, False)
-    gw += more
-  return gw
+  memo, key = _memo(plan_t), ('i', dtype, rows_x, rows_g, cx, cg, out_transposed)
+  op = memo.get(key)
+  if op is None:
+    native = _lib.native()
+    op = native.WgradOp()
+    op.kernel, op.K, op.ca, op.cb, op.out_transposed = native.WGRAD_SPARSE_INVERSE, K, cx, cg, out_transposed
+    op.rows_x, op.rows = rows_g, rows_x                    # rows the inverse table points at; its own rows
+    op.ws_bytes = L.ocnn_conv_wgrad_sparse_workspace_bytes(rows_x, cg, cx)
+    op.plan = _plan_arrays(plan_t, True)
+    if plan_t.overflow_rows is not None:                   # (tiles too dense for the plan)
+      op.overflow_rows, op.overflow_table = plan_t.overflow_rows, plan_t.overflow_table
+      op.overflow = _wgrad_op(dtype, rows_g, plan_t.overflow_table.shape[0], K, cg, cx, not out_transposed)
+    memo[key] = op
+  return op
 
 
 def column_sum(g):
   """g.sum(0) with a fixed reduction order."""
-  _lib.require_gpu(g)
-  L = _lib.lib()
-  g = g.contiguous()
-  out = torch.empty(g.shape[1], dtype=g.dtype, device=g.device)
-  ws = _lib.workspace(L.ocnn_colsum_workspace_bytes(g.shape[0], g.shape[1]), g.device)
-  _lib.check(L.ocnn_colsum(_lib.dtype_code(g), _lib.ptr(g), g.shape[0], g.shape[1],
-                           _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream()))
-  return out
+  return _lib.native().column_sum(g)
 
 
 class OctreeConvBase:
@@ -379,20 +338,9 @@ class OctreeConvBase:
     return self.octree._table_t(self.neigh_depth, self.kernel, self.stride, self.nempty,
                                 self.fine_h)
 
-  def _plan(self, data, cin, cout, inverse=False):
-    """Tile plan for the staged kernel, when the shape can use it."""
-    L, code = _lib.lib(), _lib.DTYPE_CODE.get(data.dtype, -1)
-    rows = data.shape[0]
-    # (asked by every pass of every step: the answer is kept with the table it belongs to and
-    # goes when the octree drops that table)
-    memo = self.neigh.__dict__.setdefault('_plan_memo', {}) if hasattr(self.neigh, '__dict__') else None
-    key = (code, rows, cin, cout, bool(inverse), self.fine_h)
-    octree = self.octree
-    ck = ((self.neigh_depth, self.kernel, self.stride, bool(self.nempty)), bool(inverse))
-    if memo is not None and key in memo:
-      plan = memo[key]
-      if plan is None or octree._plans.get(ck) is plan:
-        return plan
+  def _plan(self, dtype, rows, cin, cout, inverse=False):
+    """Tile plan of the table (or its inverse), when a kernel on it takes the shape."""
+    L, code = _lib.lib(), _lib.DTYPE_CODE.get(dtype, -1)
     if self.neigh.shape[0] >= PAD_MIN_ROWS:               # odd channel counts run zero-padded
       cin, cout = -(-cin // 32) * 32, -(-cout // 32) * 32
     if not (L.ocnn_conv_gather_planned_supported(code, rows, cin, cout) or
@@ -400,12 +348,8 @@ class OctreeConvBase:
             L.ocnn_conv_gather_wide_supported(code, rows, self.kdim, cin, cout, 0) or
             L.ocnn_conv_gather_sparse_supported(code, rows, self.kdim, cin, cout, 0) or
             L.ocnn_conv_wgrad_planned_supported(code, rows, rows, self.kdim, cin, cout, 0)):
-      plan = None
-    else:
-      plan = octree._plan(self.neigh_depth, self.kernel, self.stride, self.nempty, inverse, self.fine_h)
-    if memo is not None:
-      memo[key] = plan
-    return plan
+      return None
+    return self.octree._plan(self.neigh_depth, self.kernel, self.stride, self.nempty, inverse, self.fine_h)
 
   def _identity(self, rows, device):
     """(rows, 1) table [0, 1, ..]: the one-slot 'gather' of the dense form."""
@@ -415,44 +359,97 @@ class OctreeConvBase:
       cache[key] = torch.arange(rows, dtype=torch.int32, device=device).view(rows, 1)
     return cache[key]
 
+  # The three passes as (native pass, table).  None: not one pass; the *_gemm methods put it together.
+  def forward_op(self, dtype, pad_to=None):
+    """(fine rows, in_conv) -> (table rows, out_conv); see forward_gemm."""
+    if self.dense_children:
+      P, cin = self.neigh.shape[0], 8 * self.in_conv
+      op = (_gather_op(dtype, P, P, 1, cin, self.out_conv, False, False, None, True) if pad_to is None
+            else _indexed_gather_op(dtype, P, P, cin, self.out_conv, False, None, pad_to))
+      return op and (op, self._identity(P, self.neigh.device))
+    if pad_to is not None:
+      return None
+    rows, K = self.neigh.shape
+    plan = self._plan(dtype, self.fine_h, self.in_conv, self.out_conv)
+    return _gather_op(dtype, self.fine_h, rows, K, self.in_conv, self.out_conv, False, False, plan), self.neigh
+
+  def backward_op(self, dtype, coarse_index=None, coarse_rows=0):
+    """(table rows, out_conv) -> (fine rows, in_conv); see backward_gemm."""
+    rows, K = self.neigh.shape
+    if self.dense_children:
+      cout = 8 * self.in_conv
+      index = None if coarse_index is None else coarse_index
+      op = _indexed_gather_op(dtype, rows, max(rows, coarse_rows), self.out_conv, cout, True, index)
+      if op is None:
+        return None
+      op.bias_repeat, op.view_cols = 8, self.in_conv
+      return op, self._identity(rows, self.neigh.device)
+    if coarse_index is not None or self.block_children:
+      return None
+    if self.symmetric:
+      plan = self._plan(dtype, rows, self.out_conv, self.in_conv)
+      return _gather_op(dtype, rows, rows, K, self.out_conv, self.in_conv, True, True, plan), self.neigh
+    plan = self._plan(dtype, rows, self.out_conv, self.in_conv, inverse=True)
+    return (_gather_op(dtype, rows, self.fine_h, K, self.out_conv, self.in_conv, True, False, plan),
+            self._inverse_table())
+
+  def weight_op(self, dtype, out_transposed=False, coarse_index=None, coarse_rows=0):
+    """data (fine rows), grad (table rows) -> (K, in_conv, out_conv); see weight_gemm."""
+    rows, K = self.neigh.shape
+    if self.dense_children:
+      ca = 8 * self.in_conv
+      if out_transposed:
+        return None
+      op = _indexed_wgrad_op(dtype, rows, max(rows, coarse_rows), ca, self.out_conv, coarse_index) \
+          if coarse_index is not None else None
+      if op is None:
+        return None
+      op = op.seen_as([8, self.in_conv, self.out_conv])
+      return op, self._identity(rows, self.neigh.device)
+    if coarse_index is not None or (self.block_children and self.kernel == '333'):
+      return None
+    # (3x3x3 over all nodes: 20 of the 27 slots of a table row are set, and the plan-free kernel
+    # over the table is faster than the pairs of the inverse)
+    if self.stride == 2 and (self.kernel == '222' or (self.kernel == '333' and self.nempty)) and \
+        rows >= SPARSE_MIN_ROWS // 8 and \
+        _lib.lib().ocnn_conv_wgrad_sparse_supported(_lib.DTYPE_CODE.get(dtype, -1), rows, self.fine_h, self.kdim,
+                                                    self.out_conv, self.in_conv, 0):
+      plan_t = self.octree._plan(self.neigh_depth, self.kernel, self.stride, self.nempty, True, self.fine_h)
+      op = _wgrad_inverse_op(dtype, self.fine_h, rows, self.in_conv, self.out_conv, out_transposed, plan_t)
+      if op is not None:
+        return op, self.neigh
+    plan = self._plan(dtype, self.fine_h, self.in_conv, self.out_conv)
+    return _wgrad_op(dtype, self.fine_h, rows, K, self.in_conv, self.out_conv, out_transposed, plan), self.neigh
+
   def forward_gemm(self, data, weights, bias=None, pad_to=None):
     """(fine rows, in_conv) -> (table rows, out_conv).  pad_to = (octree, depth): the result
     padded to all nodes of `depth` (octree_pad of the table rows)."""
-    if self.dense_children:
-      P = self.neigh.shape[0]
-      return conv_gather(data.view(P, 8 * self.in_conv), P, self._identity(P, data.device),
-                         weights.view(1, 8 * self.in_conv, self.out_conv), self.out_conv, False,
-                         False, bias, None, dense=True, pad_to=pad_to)
-    plan = self._plan(data, self.in_conv, self.out_conv)
-    out = conv_gather(data, self.fine_h, self.neigh, weights, self.out_conv, False, False, bias,
-                      plan)
-    return out if pad_to is None else _pad_raw(out, *pad_to)
+    made = self.forward_op(data.dtype, pad_to)
+    if made is not None:
+      return made[0].run(data, made[1], weights, bias)
+    return _pad_raw(self.forward_gemm(data, weights, bias), *pad_to)
 
   def backward_gemm(self, grad, weights, bias=None, coarse_index=None):
     """(table rows, out_conv) -> (fine rows, in_conv).  coarse_index (int32): `grad` holds the
     table's rows at these rows of a larger tensor (all nodes of the depth, not only the
     non-empty ones the table has rows for)."""
+    made = self.backward_op(grad.dtype, coarse_index, grad.shape[0])
+    if made is not None:
+      return made[0].run(grad, made[1], weights, bias)
+    if coarse_index is not None:
+      grad = grad.index_select(0, coarse_index.long())
     if self.dense_children:
       # gin.view(P, 8 * in_conv) = grad @ W'^T with W' = weights.view(8 * in_conv, out_conv)
       P = self.neigh.shape[0]
-      b8 = None if bias is None else bias.repeat(8)
-      out = conv_gather(grad, P, self._identity(P, grad.device),
-                        weights.view(1, 8 * self.in_conv, self.out_conv), 8 * self.in_conv, True,
-                        False, b8, None, dense=True, in_index=coarse_index)
+      out = conv_gather(grad, P, self._identity(P, grad.device), weights.view(1, 8 * self.in_conv, self.out_conv),
+                        8 * self.in_conv, True, False, None if bias is None else bias.repeat(8), None, dense=True)
       return out.view(8 * P, self.in_conv)
-    if coarse_index is not None:
-      grad = grad.index_select(0, coarse_index.long())
     if self.block_children:
       out = self._backward_blocks(grad, weights, bias)
       if out is not None:
         return out
-    if self.symmetric:
-      plan = self._plan(grad, self.out_conv, self.in_conv)
-      return conv_gather(grad, grad.shape[0], self.neigh, weights, self.in_conv, True, True, bias,
-                         plan)
-    plan = self._plan(grad, self.out_conv, self.in_conv, inverse=True)
-    return conv_gather(grad, grad.shape[0], self._inverse_table(), weights, self.in_conv, True,
-                       False, bias, plan)
+    plan = self._plan(grad.dtype, grad.shape[0], self.out_conv, self.in_conv, inverse=True)
+    return conv_gather(grad, grad.shape[0], self._inverse_table(), weights, self.in_conv, True, False, bias, plan)
 
   def _backward_blocks(self, grad, weights, bias):
     """backward_gemm of a stride-2 layer over all nodes as a 2x2x2 stride-1 gather over the
@@ -503,6 +500,9 @@ class OctreeConvBase:
   def weight_gemm(self, data, grad, out_transposed=False, coarse_index=None):
     """data: fine rows; grad: table rows -> (K, in_conv, out_conv).  coarse_index: as in
     backward_gemm."""
+    made = self.weight_op(data.dtype, out_transposed, coarse_index, grad.shape[0])
+    if made is not None:
+      return made[0].run(data, grad, made[1])
     if self.dense_children:
       P = self.neigh.shape[0]
       gw = conv_wgrad(data.view(P, 8 * self.in_conv), grad, self._identity(P, data.device), False,
@@ -510,21 +510,11 @@ class OctreeConvBase:
       return gw.transpose(1, 2).contiguous() if out_transposed else gw
     if coarse_index is not None:
       grad = grad.index_select(0, coarse_index.long())
-    if self.block_children and self.kernel == '333':      # (8 x 8 blocks issued: a loss for 3 or 9 slots)
-      gw = self._weight_blocks(data, grad, out_transposed)
-      if gw is not None:
-        return gw
-    # (3x3x3 over all nodes: 20 of the 27 slots of a table row are set, and the plan-free kernel
-    # over the table is faster than the pairs of the inverse)
-    if self.stride == 2 and (self.kernel == '222' or (self.kernel == '333' and self.nempty)) and \
-        self.neigh.shape[0] >= SPARSE_MIN_ROWS // 8 and \
-        _lib.lib().ocnn_conv_wgrad_sparse_supported(_lib.DTYPE_CODE.get(data.dtype, -1), grad.shape[0],
-                                                    data.shape[0], self.kdim, grad.shape[1], data.shape[1], 0):
-      plan_t = self.octree._plan(self.neigh_depth, self.kernel, self.stride, self.nempty, True, self.fine_h)
-      gw = conv_wgrad_inverse(data, grad, plan_t, out_transposed)
-      if gw is not None:
-        return gw
-    plan = self._plan(data, self.in_conv, self.out_conv)
+      return self.weight_gemm(data, grad, out_transposed)
+    gw = self._weight_blocks(data, grad, out_transposed)  # (8 x 8 blocks issued: a loss for 3 or 9 slots)
+    if gw is not None:
+      return gw
+    plan = self._plan(data.dtype, data.shape[0], self.in_conv, self.out_conv)
     return conv_wgrad(data, grad, self.neigh, out_transposed, plan)
 
 
@@ -624,13 +614,93 @@ class OctreeDeconvFunction(Function):
     return (grad_out, grad_w) + (None,) * 8 + (grad_b, None)
 
 
+class _Layer:
+  """A layer on an octree in one data type: its native passes and the shape of its input.  (Kept by
+  the octree, and therefore without a reference to it.)"""
+
+  def __init__(self, eng, dtype, padded):
+    self.dtype, self.padded = dtype, padded    # padded: stride 2 over all nodes, octree_pad / octree_depad folded in
+    self.conv = eng.is_conv_layer()
+    self.pad_depth = (eng.out_depth if self.conv else eng.in_depth) if padded else None
+    self.shape = eng.in_shape if self.conv or not padded else (int(eng.octree.nnum[eng.in_depth]), eng.in_channels)
+    self.native = _lib.native().ConvLayer()
+    self.native.wgrad_of_grad = not self.conv
+    made = self._pass(eng, True)
+    self.ok = made is not None                 # the forward pass is one native pass
+    if self.ok:
+      self.native.fwd, self.native.fwd_table = made
+    # the backward passes are made when a call first needs them: None = not yet, False = not one pass
+    self.dgrad = self.wgrad = None
+
+  def _coarse(self, octree):
+    """(index, rows) of the padded side: what the passes read the coarse rows through."""
+    if not self.padded:
+      return None, 0
+    return octree._nempty_index32(self.pad_depth), int(octree.nnum[self.pad_depth])
+
+  def _pass(self, eng, forward):
+    if forward == self.conv:
+      return eng.forward_op(self.dtype, (eng.octree, self.pad_depth) if self.padded else None)
+    return eng.backward_op(self.dtype, *self._coarse(eng.octree))
+
+  def make_dgrad(self, eng):
+    made = self._pass(eng, False)
+    self.dgrad = made is not None
+    if made is not None:
+      self.native.dgrad, self.native.dgrad_table = made
+
+  def make_wgrad(self, eng):
+    made = eng.weight_op(self.dtype, False, *self._coarse(eng.octree))
+    self.wgrad = made is not None
+    if made is not None:
+      self.native.wgrad, self.native.wgrad_table = made
+
+
+def _apply(engine, function, data, weights, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
+           max_buffer, bias, padded):
+  """The layer through the native node where each of its passes is one (kept with the octree),
+  through `function` otherwise."""
+  if isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE:
+    key = (engine, depth, tuple(kernel_size), stride, nempty, in_channels, out_channels, data.dtype, padded,
+           SPARSE_MIN_ROWS)
+    layer = octree._layers.get(key)
+
+    def made_engine():
+      eng = engine(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
+      eng.setup(octree, depth)
+      return eng
+
+    if layer is None:
+      layer = octree._layers[key] = _Layer(made_engine(), data.dtype, padded)
+    if layer.ok:
+      assert data.shape == layer.shape, \
+          'The shape of input data is wrong: expected {}, got {}.'.format(layer.shape, tuple(data.shape))
+      ok = True
+      if torch.is_grad_enabled():
+        # (the rows of a padded gradient are summed over the non-empty nodes only: the other route)
+        if padded and layer.conv and bias is not None and bias.requires_grad:
+          ok = False
+        if ok and data.requires_grad:
+          if layer.dgrad is None:
+            layer.make_dgrad(made_engine())
+          ok = layer.dgrad
+        if ok and weights.requires_grad:
+          if layer.wgrad is None:
+            layer.make_wgrad(made_engine())
+          ok = layer.wgrad
+      if ok:
+        return _lib.native().conv(layer.native, data, weights, bias)
+  return function.apply(data, weights, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
+                        max_buffer, bias, padded)
+
+
 def octree_conv(data, weights, octree, depth: int, in_channels: int, out_channels: int,
                 kernel_size: List[int] = [3, 3, 3], stride: int = 1, nempty: bool = False,
                 max_buffer: int = int(2e8), bias=None, padded: bool = False):
   """Functional form (ocnn/nn/octree_conv.py:296), with an optional bias that the kernel adds
   and, for stride 2 over all nodes, the octree_pad of the result folded in (`padded`)."""
-  return OctreeConvFunction.apply(data, weights, octree, depth, in_channels, out_channels, kernel_size, stride,
-                                  nempty, max_buffer, bias, padded)
+  return _apply(_OctreeConv, OctreeConvFunction, data, weights, octree, depth, in_channels, out_channels, kernel_size,
+                stride, nempty, max_buffer, bias, padded)
 
 
 def octree_deconv(data, weights, octree, depth: int, in_channels: int, out_channels: int,
@@ -638,8 +708,8 @@ def octree_deconv(data, weights, octree, depth: int, in_channels: int, out_chann
                   max_buffer: int = int(2e8), bias=None, padded: bool = False):
   """Functional form (ocnn/nn/octree_conv.py:297), with an optional bias that the kernel adds
   and, for stride 2 over all nodes, the octree_depad of the input folded in (`padded`)."""
-  return OctreeDeconvFunction.apply(data, weights, octree, depth, in_channels, out_channels, kernel_size, stride,
-                                    nempty, max_buffer, bias, padded)
+  return _apply(_OctreeDeconv, OctreeDeconvFunction, data, weights, octree, depth, in_channels, out_channels,
+                kernel_size, stride, nempty, max_buffer, bias, padded)
 
 
 class OctreeConv(OctreeConvBase, torch.nn.Module):

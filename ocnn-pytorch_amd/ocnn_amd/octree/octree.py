@@ -218,6 +218,13 @@ class TilePlan:
     self.total, self.umax, self.nnz = total, umax, nnz
     self._table = self._ucount = self._stats = self._lists = None
 
+  def __getstate__(self):
+    """(copies leave out the layers' native passes, which are made again when asked for)"""
+    return {k: v for k, v in vars(self).items() if k not in ('_ops', '_native', '_native_pairs', '_on_pairs')}
+
+  def __setstate__(self, state):
+    vars(self).update(state, _on_pairs=None)
+
   @property
   def occupancy(self):
     """Share of the table's entries that hold a row."""
@@ -364,6 +371,7 @@ class Octree:
     self._tables = {}        # (depth, kernel, stride, nempty) -> int32 table
     self._tables_t = {}      # same key -> inverse table
     self._plans = {}         # (key, inverse) -> TilePlan
+    self._layers = {}        # the layers' passes on this octree (nn/octree_conv.py)
     self._plans_prebuilt = False
 
     self.nnum = torch.zeros(num, dtype=torch.long)
@@ -380,8 +388,12 @@ class Octree:
     self.lut_child = ((grid % 2) * torch.tensor([4, 2, 1], device=dev)).sum(2)
     self.lut_kernel = {k: torch.tensor(v, device=dev) for k, v in LUT_KERNEL.items()}
 
+  def __getstate__(self):
+    return dict(vars(self), _layers={})        # (native passes are made again when asked for)
+
   # ---- cache bookkeeping ---------------------------------------------------
   def _drop_tables(self, depth, nempty_only=False):
+    self._layers.clear()
     for cache in (self._tables, self._tables_t):
       for key in [k for k in cache if k[0] == depth and (k[3] or not nempty_only)]:
         del cache[key]
@@ -548,7 +560,7 @@ class Octree:
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
     self._nempty_indices32 = [None] * num
-    self._tables, self._tables_t, self._plans = {}, {}, {}
+    self._tables, self._tables_t, self._plans, self._layers = {}, {}, {}, {}
     self._plans_prebuilt = False
     return idx
 
@@ -940,7 +952,7 @@ class Octree:
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
     self._nempty_indices32 = [None] * num
-    self._tables, self._tables_t, self._plans = {}, {}, {}
+    self._tables, self._tables_t, self._plans, self._layers = {}, {}, {}, {}
     low48 = (1 << 48) - 1
     for d in range(num):
       self.keys[d] = torch.cat([(o.keys[d] & low48) | (i << 48)
