@@ -123,6 +123,14 @@ SIGNATURES = {
     'ocnn_colsum': (_i, [_i, _p, _l, _i, _p, _p, _l, _p]),
 }
 
+# the library's entry points for this package alone (csrc/host_api.hpp)
+INTERNAL_SIGNATURES = {
+    'ocnnx_gather_choose': (_i, [_i, _l, _l, _i, _i, _i, _i, _i, _i, _l, _d, _d]),
+    'ocnnx_gather_tile_supported': (_i, [_i, _l, _i, _i, _i, _i]),
+    'ocnnx_gather_tile_workspace_bytes': (_l, [_i, _l, _i, _i, _i]),
+    'ocnnx_gather_tile': (_i, [_i, _p, _l, _p, _p, _p, _i, _l, _d, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _l, _i, _i, _p]),
+}
+
 _lib = None
 
 
@@ -137,7 +145,7 @@ def lib():
   if not _build.is_current():
     _build.build_library()
   handle = ctypes.CDLL(path)
-  for name, (res, args) in SIGNATURES.items():
+  for name, (res, args) in list(SIGNATURES.items()) + list(INTERNAL_SIGNATURES.items()):
     fn = getattr(handle, name)      # AttributeError if the symbol is missing
     fn.restype = res
     fn.argtypes = args
@@ -172,9 +180,10 @@ def check(rc):
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
-# codes of ocnn_conv_gather_choose / ocnn_conv_wgrad_choose (include/ocnn_hip.h)
+# codes of ocnn_conv_gather_choose / ocnn_conv_wgrad_choose (include/ocnn_hip.h); TILE: of
+# ocnnx_gather_choose only
 (GATHER_PLAIN, GATHER_DENSE_RW, GATHER_DENSE, GATHER_RW, GATHER_SPARSE, GATHER_WIDE, GATHER_PLANNED,
- GATHER_ZERO_PADDED) = range(8)
+ GATHER_ZERO_PADDED, GATHER_TILE) = range(9)
 WGRAD_PLAIN, WGRAD_DENSE_RW, WGRAD_SPARSE, WGRAD_PLANNED, WGRAD_ZERO_PADDED = range(5)
 
 

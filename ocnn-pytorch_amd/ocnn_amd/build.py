@@ -24,7 +24,8 @@ SOURCES = {
     'conv.hip': [],
     'conv_staged.hip': [],
     'conv_rw.hip': [],
-    'conv_wide.hip': [],
+    'conv_tile.hip': [],
+    'conv_dense.hip': [],
     'conv_sparse.hip': [],
     'wgrad_sparse.hip': [],
     'dense_rw.hip': [],
@@ -50,7 +51,7 @@ def _host_commands():
   system = [os.path.join(base, 'include'), os.path.join(base, 'include', 'torch', 'csrc', 'api', 'include'),
             os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include'), sysconfig.get_paths()['include']]
   compile_ = ['g++', '-O2', '-std=c++17', '-fPIC', '-fvisibility=hidden', '-Wall', '-D__HIP_PLATFORM_AMD__=1',
-              '-DUSE_ROCM=1', '-I', INCLUDE] + ['-isystem' + d for d in system] + [
+              '-DUSE_ROCM=1', '-I', INCLUDE, '-I', CSRC] + ['-isystem' + d for d in system] + [
                   '-c', os.path.join(CSRC, 'host.cpp'), '-o', obj]
   link = ['g++', '-shared', '-o', HOST_PATH, obj, '-L', os.path.join(base, 'lib'), '-ltorch_python', '-ltorch',
           '-ltorch_cpu', '-lc10', '-lc10_hip', '-L', LIB_DIR, '-locnn_hip', '-Wl,-rpath,$ORIGIN']

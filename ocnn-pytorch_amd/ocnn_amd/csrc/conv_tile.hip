@@ -1,0 +1,553 @@
+// Gather-GEMM on the tile plan of the neighbour table, with the weights streamed from L2: every
+// layer whose weights do not stay in registers (conv_rw.hip) and, in fp32, every planned layer.
+//
+// A workgroup takes one tile of 128 table rows and 32 .. 256 output channels.  The distinct input
+// rows of the tile are staged in LDS 128 bytes at a time (64 channels of f16 / bf16, 32 of fp32);
+// the weights stream straight into registers, already in the layout of the MFMA A operand (no LDS
+// round trip).  M = output channels, N = rows, v_mfma_f32_32x32x16.  The four waves split the
+// output channels (WR = 1), or, where a layer has fewer than 96 of them, the rows as well (WR = 2:
+// 64 output channels, WR = 4: 32): a wave owns 32 MB channels x 128 / WR rows.  Two workgroups
+// share a CU: while one waits for its next chunk of channels the other computes.
+//
+// fp32: x = hi + lo in bf16 pieces, accumulated in fp32 as hi hi + hi lo + lo hi (about 1e-5
+// relative).  The rows are read as fp32 and split on their way into LDS, so that a row's 128 bytes
+// there are [hi | lo] of 32 channels, and the same pair of LDS reads and of weight loads feeds three
+// MFMAs: a third of the reads per MFMA that the layer takes as a bf16 layer of three times the
+// channels ([hi | hi | lo] x [hi; lo; hi]), and no passes that write and read the pieces.
+//
+// Few tiles (the coarse levels of a network, small clouds): 128 rows x 128 channels of 256 -> 256 are
+// 50 us of one workgroup's time however many CUs are idle.  The launch then also splits the
+// reduction, over chunks of input channels first (a chunk's rows are staged by one workgroup
+// either way) and over the slots; each part writes fp32 sums of its own, and a second kernel adds
+// them in the order of the parts.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+#include "host_api.hpp"
+#include "mma.hpp"
+
+namespace ocnn {
+
+constexpr int kTgRows = 128;   // rows per tile (the plan's tile size)
+constexpr int kTgCap = 416;    // staged rows; plans with a larger tile use another kernel
+constexpr int kTgRowsAlloc = (kTgCap + 8) / 8 * 8;   // LDS rows 0..kTgCap in whole 8-row groups
+// share of a table's entries that are set up to which the kernel tests for empty (32-row block,
+// slot) units: at 32 - 38 % (the non-empty nodes of depths 7 and 6 of a depth-9 octree) a quarter
+// to a half of the units are empty and the launches are 3 - 14 % faster, at 41 - 50 % 0 - 7 % slower
+constexpr double kTgSkipMaxOccupancy = 0.40;
+
+// (Not in the kernel template: the arguments of the global->LDS load builtin must not be
+// type-dependent expressions.)
+static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char* dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, off, 0, 0, 0);
+}
+
+// Packed weights: [input-channel chunk cc][slot k][32 output channels cg][step s][lane][8].
+// v_mfma_f32_32x32x16 A operand: lane l holds A[l % 32][8 * (l / 32) + j];
+// D: lane l, register r holds D[8 * (r / 4) + 4 * (l / 32) + r % 4][l % 32].
+//   output channel = 32 cg + perm(lane % 32), perm(8a + 4q + b) = 16 q + 4 a + b,
+// so that a lane ends with 16 consecutive output channels per M tile.
+//   16-bit: input channel = 64 cc + 16 s + 8 (lane / 32) + j
+//   fp32:   input channel = 32 cc + 16 (s / 2) + 8 (lane / 32) + j, s % 2 = 0: high piece, 1: low
+// Input channels are padded to whole chunks with zero weights.  A thread packs the eight values of
+// a lane (both pieces of them): 16-byte writes.
+template <typename I, typename T>
+__global__ __launch_bounds__(256) void pack_weights_tile_kernel(const I* __restrict__ w, T* __restrict__ out, int K,
+                                                                int cin, int cout, int transposed, int reverse) {
+  constexpr bool F32 = std::is_same<I, float>::value;
+  constexpr int CH = F32 ? 32 : 64, STEPS = F32 ? 2 : 4;
+  int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int ncc = (cin + CH - 1) / CH, ncg = cout >> 5;
+  if (e >= (int64_t)ncc * K * ncg * STEPS * 64) return;
+  const int lane = (int)(e & 63), s = (int)((e >> 6) % STEPS);
+  int64_t unit = (e >> 6) / STEPS;                           // (cc K + k) ncg + cg
+  const int64_t base = unit;
+  const int cg = (int)(unit % ncg);
+  unit /= ncg;
+  const int k = (int)(unit % K), cc = (int)(unit / K);
+  const int q = lane >> 5, m = lane & 31;
+  const int chan = CH * cc + 16 * s + 8 * q;
+  const int co = 32 * cg + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
+  const int kk = reverse ? K - 1 - k : k;
+  I v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    v[j] = chan + j >= cin ? (I)0.f
+                           : (transposed ? w[((int64_t)kk * cout + co) * cin + chan + j]
+                                         : w[((int64_t)kk * cin + chan + j) * cout + co]);
+  typedef __attribute__((ext_vector_type(8))) T t8;
+  t8 hi;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) hi[j] = (T)v[j];
+  T* dst = out + base * 2048 + lane * 8;
+  if constexpr (F32) {
+    t8 lo;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) lo[j] = (T)(v[j] - (float)hi[j]);
+    *(t8*)(dst + (2 * s) * 512) = hi;
+    *(t8*)(dst + (2 * s + 1) * 512) = lo;
+  } else {
+    *(t8*)(dst + s * 512) = hi;
+  }
+}
+
+// SKIP: per slot and 32-row block of the tile a wave asks whether any row has an entry there (a
+// ballot over the positions it reads anyway) and leaves the block's MFMAs out otherwise.  The
+// kernel is bound by the power its MFMAs draw (also those on zero rows), and the branches cost
+// 2 - 7 % where nothing is empty: it pays from about a quarter of the (block, slot) units empty -
+// the non-empty nodes of coarse levels -, which the launch decides from the table's occupancy.
+//
+// blockIdx.z = part of the reduction: chunks c0 .. c1 - 1 of input channels, slots k0 .. k1 - 1.
+template <typename T, bool F32, int MB, int WR, bool SKIP>
+__global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
+    const void* __restrict__ in, uint32_t in_bytes, const uint16_t* __restrict__ loc,
+    const int32_t* __restrict__ uptr, const int32_t* __restrict__ urows, const T* __restrict__ wpk,
+    const void* __restrict__ bias_, void* __restrict__ out_, float* __restrict__ partial, int64_t rows_out, int K,
+    int cin, int cout, int64_t tiles, int64_t tiles_per_xcd, int sc, int sk) {
+  typedef typename std::conditional<F32, float, T>::type O;
+  constexpr int RB = 4 / WR, WC = 4 / WR, CH = F32 ? 32 : 64;
+  __shared__ __attribute__((aligned(16))) char s_rows[kTgRowsAlloc * 128];
+  __shared__ __attribute__((aligned(16))) uint16_t s_loc[27 * kTgRows];
+  __shared__ int32_t s_u[kTgRowsAlloc];
+
+  const int64_t tile = tiles_per_xcd > 0 ? xcd_tile(blockIdx.x, tiles_per_xcd) : (int64_t)blockIdx.x;
+  if (tile >= tiles) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wc = wave % WC, wr = wave / WC;
+  const int q = lane >> 5, r32 = lane & 31;
+  const int ncc = (cin + CH - 1) / CH;
+  const int ncg = cout >> 5;
+  const int cg0 = ((int)blockIdx.y * WC + wc) * MB;         // first 32-channel group of this wave
+  const uint32_t pitch = (uint32_t)cin * (F32 ? 4u : 2u);
+  const int zc = (int)blockIdx.z / sk, zk = (int)blockIdx.z - zc * sk;
+  const int c0 = ncc * zc / sc, c1 = ncc * (zc + 1) / sc;
+  const int k0 = K * zk / sk, k1 = K * (zk + 1) / sk;
+
+  // ---- the tile's list of distinct rows and its table positions -> LDS ----
+  const int32_t p0 = uptr[tile];
+  const int U = uptr[tile + 1] - p0;
+  for (int i = tid; i < kTgRowsAlloc; i += 256)
+    s_u[i] = (i >= 1 && i <= U) ? urows[p0 + i - 1] : -1;  // LDS row p holds list entry p - 1; row 0 = zeros
+  {
+    const u32x4* src = (const u32x4*)(loc + (tile * K + k0) * (int64_t)kTgRows);
+    for (int i = tid; i < (k1 - k0) * 16; i += 256) ((u32x4*)s_loc)[i] = src[i];
+  }
+  const int groups = (U + 8) >> 3;                          // 8-row groups of LDS rows 0..U
+
+  const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(in, in_bytes);
+  // piece i of a wave: the 8 LDS rows from 8 wave + 32 i on, a lane 16 bytes of one of them.
+  // 16-byte chunk c of LDS row p sits at chunk c ^ ((p >> 1) & 7) (bank swizzle)
+  const int st_p = 8 * wave + (lane >> 3);                  // LDS row of piece 0; piece i: + 32 i
+  const uint32_t st_x = (uint32_t)(((lane >> 4) + 4 * wave) & 7);
+  const uint32_t st_c = (uint32_t)(((lane & 7) ^ st_x) * 16);
+  const bool half_oob = !F32 && (cin & 63) != 0 && st_c >= 64;      // this lane's piece of a half chunk at the end
+  constexpr int kRowPieces = (kTgCap + 1 + 31) / 32;
+
+  f32x16 acc[RB][MB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[rb][mb][r] = 0.f;
+
+  // ---- operands ----
+  // A: weights of (chunk, slot), step s; one 16-byte load per lane and M tile
+  const int64_t kstride = (int64_t)ncg * 2048;               // elements between consecutive (chunk, slot)
+  const T* wbase = wpk + lane * 8;
+  const bool active = cg0 < ncg;                             // (wave-uniform)
+  u32x4 A[4][MB];                                            // ring over the steps
+  auto load_a = [&](int kk, int s, u32x4 (&a)[MB]) {
+    const T* p = wbase + (int64_t)kk * kstride + s * 512;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) a[mb] = *(const u32x4*)(p + (int64_t)min(cg0 + mb, ncg - 1) * 2048);
+  };
+  // the (chunk, slot) after (cc, k) of this part (after the last one: itself, unused)
+  auto next_kk = [&](int cc, int k) {
+    return k + 1 < k1 ? cc * K + k + 1 : (cc + 1 < c1 ? (cc + 1) * K + k0 : cc * K + k);
+  };
+  // B: a lane reads 16 bytes (8 input channels, or their high or low pieces) of the neighbour row of
+  // row 32 rb + r32.  pv = byte address of the row in s_rows with the swizzle of step 0 folded in.
+  const uint16_t* lcw = s_loc + 32 * RB * wr + r32;
+  uint32_t pvc[RB], pvn[RB];
+  // (SKIP) which 32-row blocks of the tile have an entry in the slot at all, wave-uniform
+  bool nzc[RB], nzn[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) nzc[rb] = nzn[rb] = true;
+  auto load_pos = [&](int k, uint32_t (&pv)[RB], bool (&nz)[RB]) {
+    const uint16_t* p = lcw + (k - k0) * kTgRows;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const uint32_t l = p[32 * rb];                         // 0 = empty = the zero row
+      pv[rb] = (l << 7) | (((l << 3) & 0x70u) ^ ((uint32_t)q << 4));
+      if constexpr (SKIP) nz[rb] = __builtin_amdgcn_ballot_w64(l != 0u) != 0ull;
+    }
+  };
+  auto read_b = [&](const uint32_t (&pv)[RB], int s, u32x4 (&b)[RB]) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) b[rb] = *(const u32x4*)(s_rows + (pv[rb] ^ ((uint32_t)s << 5)));
+  };
+  auto multiply = [&](const u32x4 (&a)[MB], const u32x4 (&b)[RB]) {
+    if (active) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+        if (!SKIP || nzc[rb]) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) acc[rb][mb] = Mma32<T>::run(a[mb], b[rb], acc[rb][mb]);
+        }
+    }
+  };
+  auto advance = [&]() {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      pvc[rb] = pvn[rb];
+      if constexpr (SKIP) nzc[rb] = nzn[rb];
+    }
+  };
+
+  // the distinct rows' channels of chunk cc -> LDS
+  // the list entries of this lane's pieces, read once for all chunks (one LDS wait, not one per piece)
+  __syncthreads();
+  int32_t ids[kRowPieces];
+#pragma unroll
+  for (int i = 0; i < kRowPieces; ++i) ids[i] = s_u[min(st_p + 32 * i, kTgRowsAlloc - 1)];   // -1: out of range, loads zeros
+  auto stage_chunk = [&](int cc) {
+    if constexpr (F32) {
+      // fp32 rows through registers, split into their bf16 pieces on the way: a lane's four channels
+      // 4 (lane % 8) .. are half a 16-byte chunk of either piece
+      f32x4 v[kRowPieces];
+#pragma unroll
+      for (int i = 0; i < kRowPieces; ++i)
+        if (wave + 4 * i < groups)
+          v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rs_in, (uint32_t)ids[i] * pitch + (uint32_t)cc * 128u + (uint32_t)(lane & 7) * 16u, 0, 0));
+      __syncthreads();                                       // every wave is done with the chunk before
+      const uint32_t half = (uint32_t)(lane & 1) * 8u, ch = (uint32_t)(lane & 7) >> 1;
+#pragma unroll
+      for (int i = 0; i < kRowPieces; ++i)
+        if (wave + 4 * i < groups) {
+          typedef __attribute__((ext_vector_type(4))) T t4;
+          t4 hi, lo;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            hi[j] = (T)v[i][j];
+            lo[j] = (T)(v[i][j] - (float)hi[j]);
+          }
+          char* row = s_rows + (st_p + 32 * i) * 128;
+          *(t4*)(row + (ch ^ st_x) * 16u + half) = hi;
+          *(t4*)(row + ((ch | 4u) ^ st_x) * 16u + half) = lo;
+        }
+      __syncthreads();
+    } else {
+      __syncthreads();                                       // every wave is done with the chunk before
+#pragma unroll
+      for (int i = 0; i < kRowPieces; ++i) {
+        const int g = wave + 4 * i;
+        if (g < groups) {
+          uint32_t off = (uint32_t)ids[i] * pitch + ((uint32_t)cc * 128u + st_c);
+          if (cc == ncc - 1 && half_oob) off = 0xffffff00u;  // past the row's channels: zeros, not the next row
+          tg_dma16(rs_in, s_rows + g * 1024, off);
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+  };
+
+  if constexpr (F32) {
+    // weights in pairs (high, low piece of a k-step), fetched one k-step ahead
+    u32x4 Bh[2][RB], Bl[2][RB];
+    auto load_pair = [&](int kk, int j) {
+      load_a(kk, 2 * j, A[2 * j]);
+      load_a(kk, 2 * j + 1, A[2 * j + 1]);
+    };
+    load_pair(c0 * K + k0, 0);
+    for (int cc = c0; cc < c1; ++cc) {
+      stage_chunk(cc);
+      load_pos(k0, pvc, nzc);
+      read_b(pvc, 0, Bh[0]);
+      read_b(pvc, 2, Bl[0]);
+      for (int k = k0; k < k1; ++k) {
+        load_pos(k + 1 < k1 ? k + 1 : k0, pvn, nzn);
+        load_pair(cc * K + k, 1);
+        read_b(pvc, 1, Bh[1]);
+        read_b(pvc, 3, Bl[1]);
+        multiply(A[0], Bh[0]);
+        multiply(A[0], Bl[0]);
+        multiply(A[1], Bh[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_pair(next_kk(cc, k), 0);
+        read_b(pvn, 0, Bh[0]);                               // (past the last slot: unused)
+        read_b(pvn, 2, Bl[0]);
+        multiply(A[2], Bh[1]);
+        multiply(A[2], Bl[1]);
+        multiply(A[3], Bh[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        advance();
+      }
+    }
+  } else {
+    u32x4 Bb[2][RB];
+    const int nfull = min(c1, cin >> 6);                     // whole 64-channel chunks up to here
+    load_a(c0 * K + k0, 0, A[0]);
+    load_a(c0 * K + k0, 1, A[1]);
+    for (int cc = c0; cc < nfull; ++cc) {
+      stage_chunk(cc);
+      load_pos(k0, pvc, nzc);
+      read_b(pvc, 0, Bb[0]);
+      for (int k = k0; k < k1; ++k) {
+        const int kk = cc * K + k, kn = next_kk(cc, k);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          // fetches: positions of the next slot, weights two k-steps ahead, rows one k-step ahead
+          if (s == 0) load_pos(k + 1 < k1 ? k + 1 : k0, pvn, nzn);
+          load_a(s >= 2 ? kn : kk, (s + 2) & 3, A[(s + 2) & 3]);
+          if (s < 3) read_b(pvc, s + 1, Bb[(s + 1) & 1]);
+          else read_b(pvn, 0, Bb[0]);                        // (past the last slot: unused)
+          multiply(A[s], Bb[s & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        advance();
+      }
+    }
+    if (nfull < c1) {
+      // Half a chunk at the end (cin % 64 == 32): two k-steps per slot instead of four.  The
+      // weights of a slot sit in one pair of the ring while the next slot's go into the other,
+      // so the slots are taken two at a time (the chunk before left the first pair filled).
+      const int cc = nfull;
+      stage_chunk(cc);
+      load_pos(k0, pvc, nzc);
+      read_b(pvc, 0, Bb[0]);
+      auto half_slot = [&](int k, auto ring) {
+        constexpr int r = decltype(ring)::value;             // this slot's pair of the ring: 0 or 2
+        const int kn = next_kk(cc, k);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if (s == 0) load_pos(k + 1 < k1 ? k + 1 : k0, pvn, nzn);
+          load_a(kn, s, A[(r ^ 2) + s]);
+          if (s == 0) read_b(pvc, 1, Bb[1]);
+          else read_b(pvn, 0, Bb[0]);                        // (past the last slot: unused)
+          multiply(A[r + s], Bb[s]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        advance();
+      };
+      for (int k = k0; k < k1; k += 2) {
+        half_slot(k, std::integral_constant<int, 0>{});
+        if (k + 1 < k1) half_slot(k + 1, std::integral_constant<int, 2>{});
+      }
+    }
+  }
+
+  // ---- epilogue: a lane holds 16 consecutive output channels of a row per M tile ----
+  const O* bias = (const O*)bias_;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    if (cg0 + mb >= ncg) continue;
+    const int co = 32 * (cg0 + mb) + 16 * q;
+    float bv[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bv[r] = bias && !partial ? to_f32(bias[co + r]) : 0.f;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
+      if (row >= rows_out) continue;
+      if (F32 || partial) {
+        float* dst = (partial ? partial + (int64_t)blockIdx.z * rows_out * cout : (float*)out_) + row * cout + co;
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          *(f32x4*)(dst + r) = f32x4{acc[rb][mb][r] + bv[r], acc[rb][mb][r + 1] + bv[r + 1],
+                                     acc[rb][mb][r + 2] + bv[r + 2], acc[rb][mb][r + 3] + bv[r + 3]};
+      } else {
+        unsigned pk[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) pk[r] = pack2<T>(acc[rb][mb][2 * r] + bv[2 * r], acc[rb][mb][2 * r + 1] + bv[2 * r + 1]);
+        T* dst = (T*)out_ + row * cout + co;
+        *(u32x4*)(dst) = u32x4{pk[0], pk[1], pk[2], pk[3]};
+        *(u32x4*)(dst + 8) = u32x4{pk[4], pk[5], pk[6], pk[7]};
+      }
+    }
+  }
+}
+
+// out = sum of the parts, in their order, (+ bias); four consecutive values a thread
+template <typename O>
+__global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict__ partial, int parts, int64_t n, int cout,
+                                                         const O* __restrict__ bias, O* __restrict__ out) {
+  const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (e >= n) return;
+  f32x4 acc = *(const f32x4*)(partial + e);
+  int s = 1;
+  for (; s + 4 <= parts; s += 4) {                           // four loads in flight
+    f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = *(const f32x4*)(partial + (s + u) * n + e);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc += v[u];
+  }
+  for (; s < parts; ++s) acc += *(const f32x4*)(partial + s * n + e);
+  const int c = (int)(e % cout);
+  if (bias)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += to_f32(bias[c + i]);
+  typedef __attribute__((ext_vector_type(4))) O o4;
+  o4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = from_f32<O>(acc[i]);
+  *(o4*)(out + e) = o;
+}
+
+struct TileLaunch {
+  int mb, wr;                  // shape of a wave (see above)
+  int gy;                      // blocks of output channels
+  int sc, sk;                  // parts of the reduction: chunks x slots
+};
+
+// How a launch is cut up.  WR by the output channels (96 or more keep three of the four waves busy
+// along them); 256 channels a workgroup halve the LDS reads per MFMA where there are tiles enough.
+//
+// The reduction is split while the launch stays within the workgroups that run at once: one a CU for
+// short ones, whose time is latency (up to 64 (chunk, slot) units of 16 MFMAs a wave; an fp32 unit
+// counts half as much again), two for longer ones, and rounds of them from 200 units on, where
+// the last, half-empty round costs more than the parts' sums.  A part keeps at least kTgMinUnits units:
+// below that staging the rows is all it does.  Measured (us, 3x3x3, 17 - 22 % occupied, one part -> split): fp16
+// 256 -> 256 on 1 / 30 / 100 tiles 72 -> 18, 72 -> 37, 74 -> 65, 128 -> 128 on 1 / 30 / 64 tiles 38 -> 15, 37 -> 25,
+// 37 -> 31 and no gain from 150 on; fp32 256 -> 256 on 30 / 150 / 300 tiles 170 -> 52, 230 -> 171, 379 -> 310.
+constexpr int kTgMinUnits = 6;
+
+static TileLaunch tile_launch(bool f32, int64_t tiles, int K, int cin, int cout) {
+  TileLaunch t{1, 1, 1, 1, 1};
+  t.wr = cout <= 32 ? 4 : (cout <= 64 ? 2 : 1);
+  if (!f32 && cout % 256 == 0 && tiles * (cout / 256) > 256) t.mb = 2;
+  t.gy = (int)cdiv(cout, 128 / t.wr * t.mb);
+  const int64_t blocks = tiles * t.gy;
+  const int ncc = (int)cdiv(cin, f32 ? 32 : 64);
+  const int units = ncc * K * (f32 ? 3 : 2) / 2;
+  const int64_t target = units <= 64 ? 256 : (units < 200 ? 512 : 1200);
+  if (blocks > 0 && blocks * 2 <= target) {
+    const int want = (int)std::min<int64_t>(target / blocks, std::max(1, ncc * K / kTgMinUnits));
+    t.sc = std::max(1, std::min(ncc, want));
+    t.sk = std::max(1, std::min(K, want / t.sc));
+  }
+  return t;
+}
+
+}  // namespace ocnn
+
+using namespace ocnn;
+
+static int64_t tile_packed_bytes(int dtype, int K, int cin, int cout) {
+  return align_up(dtype == OCNN_F32 ? (int64_t)K * align_up(cin, 32) * cout * 4 : (int64_t)K * align_up(cin, 64) * cout * 2,
+                  256);
+}
+
+extern "C" int ocnnx_gather_tile_supported(int dtype, int64_t rows_in, int K, int cin, int cout, int plan_max_distinct) {
+  if (dtype < 0 || dtype > 2) return 0;
+  if (cin < 32 || cin % 32 != 0 || cout < 32 || cout % 32 != 0 || cin > 2048 || cout > 2048) return 0;
+  if (K < 1 || K > 27) return 0;
+  if (plan_max_distinct < 0 || plan_max_distinct > kTgCap) return 0;
+  if (rows_in < 0 || rows_in * cin * dtype_size(dtype) > 0xfff00000ll) return 0;
+  return 1;
+}
+
+extern "C" int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out, int K, int cin, int cout) {
+  const TileLaunch t = tile_launch(dtype == OCNN_F32, cdiv(rows_out, kTgRows), K, cin, cout);
+  const int64_t parts = t.sc * t.sk;
+  return tile_packed_bytes(dtype, K, cin, cout) + (parts > 1 ? parts * rows_out * cout * 4 : 0);
+}
+
+template <typename T, bool F32>
+static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr, const int32_t* urows,
+                    int64_t rows_out, int K, int cin, int cout, const void* w, int w_transposed, int reverse,
+                    const void* bias, void* out, void* ws, int64_t ws_bytes, bool skip, int split_c, int split_k,
+                    hipStream_t st) {
+  typedef typename std::conditional<F32, float, T>::type O;
+  const int dtype = F32 ? OCNN_F32 : OCNN_F16;
+  const int64_t lanes = cdiv(cin, F32 ? 32 : 64) * (int64_t)K * (cout / 32) * (F32 ? 2 : 4) * 64;
+  hipLaunchKernelGGL((pack_weights_tile_kernel<O, T>), dim3((unsigned)cdiv(lanes, 256)), dim3(256), 0, st, (const O*)w,
+                     (T*)ws, K, cin, cout, w_transposed, reverse);
+  const int64_t tiles = cdiv(rows_out, kTgRows);
+  TileLaunch t = tile_launch(F32, tiles, K, cin, cout);
+  if (split_c > 0 && split_k > 0) {
+    t.sc = std::min<int>(split_c, (int)cdiv(cin, F32 ? 32 : 64));
+    t.sk = std::min(split_k, K);
+  }
+  const int64_t packed = tile_packed_bytes(dtype, K, cin, cout);
+  if (packed + (int64_t)t.sc * t.sk * rows_out * cout * 4 > ws_bytes) t.sc = t.sk = 1;   // (no room for the parts)
+  const int parts = t.sc * t.sk;
+  float* partial = parts > 1 ? (float*)((char*)ws + packed) : nullptr;
+  // few tiles: in launch order, so that they spread over the XCDs
+  const int64_t per_xcd = parts > 1 ? 0 : cdiv(tiles, 8);
+  const dim3 grid((unsigned)(per_xcd > 0 ? per_xcd * 8 : tiles), (unsigned)t.gy, (unsigned)parts);
+  const uint32_t in_bytes = (uint32_t)(rows_in * cin * sizeof(O));
+#define OCNN_TILE_LAUNCH(MB_, WR_, SKIP_)                                                                           \
+  hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WR_, SKIP_>), grid, dim3(256), 0, st, in, in_bytes, loc, \
+                     uptr, urows, (const T*)ws, bias, out, partial, rows_out, K, cin, cout, tiles, per_xcd, t.sc, t.sk)
+#define OCNN_TILE_CASE(MB_, WR_)           \
+  if (t.mb == MB_ && t.wr == WR_) {        \
+    if (skip) OCNN_TILE_LAUNCH(MB_, WR_, true); \
+    else OCNN_TILE_LAUNCH(MB_, WR_, false);     \
+  }
+  OCNN_TILE_CASE(1, 1) OCNN_TILE_CASE(1, 2) OCNN_TILE_CASE(1, 4)
+  if constexpr (!F32) {
+    OCNN_TILE_CASE(2, 1)
+  }
+#undef OCNN_TILE_CASE
+#undef OCNN_TILE_LAUNCH
+  if (partial)
+    hipLaunchKernelGGL(tile_parts_kernel<O>, dim3((unsigned)cdiv(rows_out * cout / 4, 256)), dim3(256), 0, st, partial,
+                       parts, rows_out * cout, cout, (const O*)bias, (O*)out);
+  return check_launch("conv_gather_tile");
+}
+
+extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
+                                 const int32_t* urows, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
+                                 int64_t rows_out, int K, const void* w, int cin, int cout, int w_transposed,
+                                 int reverse_slots, const void* bias, void* out, void* workspace, int64_t workspace_bytes,
+                                 int split_c, int split_k, void* stream) {
+  OCNN_REQUIRE(ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct),
+               "conv_gather_tile: shape not supported");
+  OCNN_REQUIRE(rows_out >= 0 && rows_out < (1ll << 31) && plan_total >= 0 && plan_total < (1ll << 29),
+               "conv_gather_tile: rows out of range");
+  if (rows_out == 0) return OCNN_OK;
+  OCNN_REQUIRE_PTRS("conv_gather_tile", loc, uptr, urows, w, out, workspace);
+  OCNN_REQUIRE(rows_in == 0 || in, "conv_gather_tile: in is NULL");
+  if (workspace_bytes < (dtype == OCNN_F32 ? (int64_t)K * cin * cout * 4 : (int64_t)K * align_up(cin, 64) * cout * 2)) {
+    set_error("conv_gather_tile: workspace too small");
+    return OCNN_ERR_WORKSPACE;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
+  const bool skip = K != 8 && plan_occupancy >= 0.0 && plan_occupancy <= kTgSkipMaxOccupancy;
+  if (dtype == OCNN_F32)
+    return run_tile<bf16, true>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
+                                bias, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+  if (dtype == OCNN_F16)
+    return run_tile<f16, false>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
+                                bias, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+  return run_tile<bf16, false>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
+                               bias, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+}
+
+// The public entry point: 16-bit wide layers, with whatever room for parts the workspace has.
+extern "C" int ocnn_conv_gather_wide_supported(int dtype, int64_t rows_in, int K, int cin, int cout,
+                                               int plan_max_distinct) {
+  if (dtype != OCNN_F16 && dtype != OCNN_BF16) return 0;
+  if (cin < 64 || cout < 96) return 0;
+  return ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct);
+}
+
+extern "C" int ocnn_conv_gather_wide(int dtype, const void* in, int64_t rows_in, const uint16_t* loc,
+                                     const int32_t* uptr, const int32_t* urows, int plan_max_distinct,
+                                     int64_t plan_total, double plan_occupancy, int64_t rows_out, int K,
+                                     const void* w, int cin, int cout, int w_transposed, int reverse_slots,
+                                     const void* bias, void* out, void* workspace, int64_t workspace_bytes,
+                                     void* stream) {
+  OCNN_REQUIRE(ocnn_conv_gather_wide_supported(dtype, rows_in, K, cin, cout, plan_max_distinct),
+               "conv_gather_wide: shape not supported");
+  return ocnnx_gather_tile(dtype, in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out,
+                           K, w, cin, cout, w_transposed, reverse_slots, bias, out, workspace, workspace_bytes, 0, 0,
+                           stream);
+}

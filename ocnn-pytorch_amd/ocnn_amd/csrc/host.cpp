@@ -18,7 +18,7 @@
 #include <optional>
 #include <vector>
 
-#include "ocnn_hip.h"
+#include "host_api.hpp"
 
 namespace {
 
@@ -119,11 +119,10 @@ struct GatherOp {
                                   typed<int32_t>(p->urows), p->umax, p->total, rows, K, ptr(W), cin, cout, transposed,
                                   reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
         break;
-      case OCNN_GATHER_WIDE:
-        check(ocnn_conv_gather_wide(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
-                                    typed<int32_t>(p->urows), p->umax, p->total, p->occupancy, rows, K, ptr(W), cin,
-                                    cout, transposed, reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(),
-                                    st));
+      case OCNNX_GATHER_TILE:
+        check(ocnnx_gather_tile(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
+                                typed<int32_t>(p->urows), p->umax, p->total, p->occupancy, rows, K, ptr(W), cin, cout,
+                                transposed, reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), 0, 0, st));
         break;
       case OCNN_GATHER_SPARSE:
         check(ocnn_conv_gather_sparse(code, ptr(data), rows_in, typed<int32_t>(p->uptr), typed<int32_t>(p->urows),
@@ -132,7 +131,7 @@ struct GatherOp {
                                       rows, K, ptr(W), cin, cout, transposed, reverse, ptr(bias), out.data_ptr(),
                                       ws.data_ptr(), ws.numel(), st));
         break;
-      case OCNN_GATHER_PLANNED:
+      case OCNN_GATHER_PLANNED:               // (tiles of more rows than the other kernels stage)
         check(ocnn_conv_gather_planned(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
                                        typed<int32_t>(p->urows), rows, K, ptr(W), cin, cout, transposed, reverse,
                                        ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));

@@ -6,6 +6,7 @@
 // its entry point checks on top (32-bit buffer offsets of the output, of the table, of the
 // plan) are repeated here, so a choice is always one that the chosen entry point accepts.
 #include "common.hpp"
+#include "host_api.hpp"
 
 using namespace ocnn;
 
@@ -54,6 +55,22 @@ extern "C" int ocnn_conv_gather_choose(int dtype, int64_t rows_in, int64_t rows_
       return OCNN_GATHER_PLANNED;
   }
   return OCNN_GATHER_PLAIN;
+}
+
+// The same for this package's own host path, which also has the kernel of conv_tile.hip in its full
+// range: it takes what would run plan-free or multi-pass on a table with a plan (every fp32 layer;
+// 16-bit layers of 32 or 64 output channels that are not square), and the wide layers, which it
+// splits where there are few tiles.
+extern "C" int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout,
+                                   int identity_table, int has_plan, int plan_max_distinct, int64_t plan_total,
+                                   double plan_occupancy, double plan_reuse) {
+  const int pick = ocnn_conv_gather_choose(dtype, rows_in, rows_out, K, cin, cout, identity_table, has_plan,
+                                           plan_max_distinct, plan_total, plan_occupancy, plan_reuse);
+  if (has_plan && rows_ok(rows_out, plan_total) &&
+      (pick == OCNN_GATHER_PLAIN || pick == OCNN_GATHER_PLANNED || pick == OCNN_GATHER_WIDE) &&
+      ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct))
+    return OCNNX_GATHER_TILE;
+  return pick;
 }
 
 extern "C" int ocnn_conv_wgrad_choose(int dtype, int64_t rows_x, int64_t rows, int K, int ca, int cb,

@@ -103,7 +103,7 @@ def _memo(plan):
 
 def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=None, dense=False):
   """The gather-GEMM of a shape as a native pass (csrc/host.cpp).  The library picks the kernel
-  (ocnn_conv_gather_choose); the choice depends on the shapes and the plan only, so the pass is
+  (ocnnx_gather_choose); the choice depends on the shapes and the plan only, so the pass is
   made once per plan.  The few tiles that are too dense for a plan get a pass of their own on the
   plan-free kernel, its rows put in place afterwards."""
   memo, key = _memo(plan), ('g', dtype, rows_in, rows, K, cin, cout, transposed, reverse, dense)
@@ -113,14 +113,15 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
   L, code = _lib.lib(), _lib.dtype_code_of(dtype)
   op = _lib.native().GatherOp()
   op.rows_in, op.rows, op.K, op.cin, op.cout, op.transposed, op.reverse = rows_in, rows, K, cin, cout, transposed, reverse
-  op.kernel = L.ocnn_conv_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan))
+  op.kernel = L.ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan))
   if op.kernel == _lib.GATHER_ZERO_PADDED:
     op.padded = _gather_op(dtype, rows_in, rows, K, -(-cin // 32) * 32, -(-cout // 16) * 16, transposed, reverse, plan)
   else:
     sparse = op.kernel == _lib.GATHER_SPARSE
-    op.ws_bytes = (L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout) if sparse
-                   else L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
-    if op.kernel in (_lib.GATHER_RW, _lib.GATHER_WIDE, _lib.GATHER_PLANNED, _lib.GATHER_SPARSE):
+    op.ws_bytes = (L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout) if sparse else
+                   L.ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout) if op.kernel == _lib.GATHER_TILE else
+                   L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
+    if op.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE, _lib.GATHER_SPARSE, _lib.GATHER_PLANNED):
       op.plan = _plan_arrays(plan, sparse)
       if plan.overflow_rows is not None:
         op.overflow_rows, op.overflow_table = plan.overflow_rows, plan.overflow_table
@@ -343,9 +344,9 @@ class OctreeConvBase:
     L, code = _lib.lib(), _lib.DTYPE_CODE.get(dtype, -1)
     if self.neigh.shape[0] >= PAD_MIN_ROWS:               # odd channel counts run zero-padded
       cin, cout = -(-cin // 32) * 32, -(-cout // 32) * 32
-    if not (L.ocnn_conv_gather_planned_supported(code, rows, cin, cout) or
+    if not (L.ocnnx_gather_tile_supported(code, rows, self.kdim, cin, cout, 0) or
             L.ocnn_conv_gather_rw_supported(code, rows, self.kdim, cin, cout, 0) or
-            L.ocnn_conv_gather_wide_supported(code, rows, self.kdim, cin, cout, 0) or
+            L.ocnn_conv_gather_planned_supported(code, rows, cin, cout) or
             L.ocnn_conv_gather_sparse_supported(code, rows, self.kdim, cin, cout, 0) or
             L.ocnn_conv_wgrad_planned_supported(code, rows, rows, self.kdim, cin, cout, 0)):
       return None

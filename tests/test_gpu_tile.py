@@ -1,0 +1,53 @@
+"""The gather-GEMM of csrc/conv_tile.hip at the edges of its ranges: rows around a tile, every
+division of the waves, halves of a 64-channel chunk, and the reduction in one and several parts."""
+
+import numpy as np
+import pytest
+import torch
+
+from ocnn_amd import _lib
+from ocnn_amd.octree.octree import TilePlan
+from oracle import conv_ref as C
+
+pytestmark = pytest.mark.gpu
+TOL = {torch.float32: 2e-5, torch.float16: 2e-3, torch.bfloat16: 1e-2}
+
+
+def _gather(x, plan, w, cout, transposed, reverse, b, parts, occupancy):
+  L, P, K = _lib.lib(), _lib.ptr, plan.K
+  code, cin = _lib.dtype_code(x), x.shape[1]
+  assert L.ocnnx_gather_tile_supported(code, x.shape[0], K, cin, cout, plan.umax)
+  out = torch.full((plan.rows, cout), float('nan'), dtype=x.dtype, device='cuda')
+  size = L.ocnnx_gather_tile_workspace_bytes(code, plan.rows, K, cin, cout)
+  if parts != (0, 0):
+    size = 8 * K * cin * cout + 1024 + parts[0] * parts[1] * plan.rows * cout * 4
+  ws = torch.empty(size, dtype=torch.uint8, device='cuda')
+  _lib.check(L.ocnnx_gather_tile(code, P(x), x.shape[0], P(plan.loc), P(plan.uptr), P(plan.urows), plan.umax, plan.total,
+                                 occupancy, plan.rows, K, P(w), cin, cout, int(transposed), int(reverse), P(b), P(out),
+                                 P(ws), size, *parts, _lib.stream()))
+  return out
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,cout', [(32, 32), (96, 64), (64, 96), (160, 160), (128, 256)])
+def test_tile_kernel(dtype, cin, cout):
+  for rows, K in ((1, 27), (127, 9), (129, 27), (2000, 8)):
+    print('tile kernel', dtype, cin, cout, 'rows', rows, 'K', K, flush=True)
+    g = torch.Generator().manual_seed(rows + cin)
+    t = (torch.arange(rows)[:, None] + torch.randint(-40, 41, (rows, K), generator=g)).clamp_(0, rows - 1).int()
+    t[torch.rand(rows, K, generator=g) < 0.4] = -1
+    plan = TilePlan(t.cuda())
+    x = torch.randn(rows, cin, generator=g).to(dtype)
+    w = (torch.randn(K, cin, cout, generator=g) / (K * cin) ** 0.5).to(dtype)
+    b = torch.randn(cout, generator=g).to(dtype)
+    t64, f64 = t.numpy().astype(np.int64), lambda v: v.double().numpy()
+    want = C.forward_gemm(f64(x), f64(w), t64) + f64(b)
+    wt = w.flip(0).transpose(1, 2).contiguous()          # read transposed and mirrored: the same layer
+    for parts in ((0, 0), (1, 1), (2, 1), (3, 4), (64, 27)):
+      for occupancy in (1.0, 0.3):                       # without and with the test for empty blocks
+        for ww, tr, rev in ((w, False, False), (wt, True, True)):
+          got = _gather(x.cuda(), plan, ww.cuda(), cout, tr, rev, b.cuda(), parts, occupancy)
+          err = np.abs(got.double().cpu().numpy() - want).max() / np.abs(want).max()
+          assert err < TOL[dtype], (parts, occupancy, tr, err)
+          again = _gather(x.cuda(), plan, ww.cuda(), cout, tr, rev, b.cuda(), parts, occupancy)
+          assert torch.equal(got, again)
