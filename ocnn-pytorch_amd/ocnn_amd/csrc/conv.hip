@@ -691,10 +691,7 @@ static int run_wgrad_f32_split(const void* x, int64_t rows_x, const void* g, con
   bf16* gh = (bf16*)((char*)ws + 2 * xb);
   bf16* gl = (bf16*)((char*)ws + 2 * xb + gb);
   float* partial = (float*)((char*)ws + 2 * xb + 2 * gb);
-  hipLaunchKernelGGL(split2_kernel, dim3((unsigned)cdiv(rows_x * ca, 256)), dim3(256), 0, st,
-                     (const float*)x, rows_x * ca, xh, xl);
-  hipLaunchKernelGGL(split2_kernel, dim3((unsigned)cdiv(rows * cb, 256)), dim3(256), 0, st,
-                     (const float*)g, rows * cb, gh, gl);
+  launch_split2(x, rows_x * ca, xh, xl, g, rows * cb, gh, gl, st);
   constexpr int KG = kWgradSlots;
   dim3 grid(p.splits, (unsigned)(cdiv(K, KG) * (ca / p.TILE)), (unsigned)(cb / p.TILE));
   const uint32_t xbytes = (uint32_t)(rows_x * ca * 2), gbytes = (uint32_t)(rows * cb * 2);

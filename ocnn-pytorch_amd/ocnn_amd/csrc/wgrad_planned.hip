@@ -61,7 +61,12 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
     const uint16_t* __restrict__ loc, uint32_t loc_bytes, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ urows, uint32_t urows_bytes, int64_t tiles,
-    int64_t tiles_per_split, int nsplit, int ca, int cb, float* __restrict__ partial) {
+    int64_t tiles_per_split, int nsplit, int ca, int cb, float* __restrict__ partial, const T* __restrict__ x_lo,
+    const T* __restrict__ g_lo, int64_t set) {
+  // fp32 data as bf16 pieces: hi hi, hi lo, lo hi, each with sums of its own
+  if (blockIdx.z == 1) g = g_lo;
+  if (blockIdx.z == 2) x = x_lo;
+  partial += blockIdx.z * set;
   constexpr int H = C / 32;                   // 32-channel halves of a row
   constexpr int NU = H * NFULL + NHALF;       // 32 x C accumulator units per wave
   constexpr int NS = NFULL + NHALF;           // distinct slots per wave
@@ -379,8 +384,10 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 using namespace ocnn;
 
 
-static int wp_splits(int K, int ca, int cb, int n_cu) {
-  const int groups = (K == 27 && ca >= 64) ? 2 : 1;
+// ranges of tiles: as many as keep a workgroup on every CU (the LDS holds one), with the slot groups, the
+// blocks of channel pairs and, in fp32, the three products of bf16 pieces as further workgroups
+static int wp_splits(int K, int ca, int cb, int n_cu, int products) {
+  const int groups = ((K == 27 && ca >= 64) ? 2 : 1) * products;
   const int blocks = ca >= 64 ? ((ca + 63) / 64) * ((cb + 63) / 64) : 1;
   int s = std::max(8, n_cu / (groups * blocks) / 8 * 8);      // a multiple of 8: ranges are dealt to the XCDs
   return std::min(s, 256);
@@ -411,7 +418,7 @@ extern "C" int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int6
 
 extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes(int K, int ca, int cb) {
   const int n_cu = wp_cu_count();
-  const int64_t splits = n_cu > 0 ? wp_splits(K, ca, cb, n_cu) : 256;
+  const int64_t splits = n_cu > 0 ? wp_splits(K, ca, cb, n_cu, 1) : 256;
   return align_up(splits * K * ca * cb * 4, 256);
 }
 
@@ -424,46 +431,54 @@ extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes_for(int dtype, int64_
   return 2 * align_up(rows_x * ca * 2, 256) + 2 * align_up(rows * cb * 2, 256) + 3 * sums;
 }
 
+struct WpArgs {
+  const void *x, *g, *x_lo, *g_lo;            // x_lo, g_lo: the low bf16 pieces of fp32 data (products = 3)
+  int products;
+  int64_t rows_x, rows, set, per, plan_total;
+  const uint16_t* loc;
+  const int32_t *uptr, *urows;
+  int K, ca, cb, nsplit;
+  float* partial;
+};
+
 template <typename T, int C, int KK, int NFULL, int NHALF, int GROUPS>
-static void launch_wp(const void* x, int64_t rows_x, const void* g, const uint16_t* loc, const int32_t* uptr,
-                      const int32_t* urows, int64_t plan_total, int64_t rows, int ca, int cb, int nsplit,
-                      int64_t per, float* partial, hipStream_t st) {
-  const int64_t tiles = cdiv(rows, kWpRows);
-  const uint32_t xb = (uint32_t)(rows_x * ca * 2), gb = (uint32_t)(rows * cb * 2);
-  const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(plan_total * 4);
-  if (ca == C && cb == C)
-    hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, C, KK, NFULL, NHALF, GROUPS, false>), dim3(nsplit * GROUPS),
-                       dim3(256), 0, st, (const T*)x, xb, (const T*)g, gb, loc, lb, uptr, urows, ub, tiles, per,
-                       nsplit, ca, cb, partial);
+static void launch_wp(const WpArgs& a, hipStream_t st) {
+  const int64_t tiles = cdiv(a.rows, kWpRows);
+  const uint32_t xb = (uint32_t)(a.rows_x * a.ca * 2), gb = (uint32_t)(a.rows * a.cb * 2);
+  const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(a.plan_total * 4);
+#define OCNN_WP_KERNEL(BLK_, GY_)                                                                                        \
+  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, C, KK, NFULL, NHALF, GROUPS, BLK_>),                                  \
+                     dim3(a.nsplit * GROUPS, GY_, a.products), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g, gb,   \
+                     a.loc, lb, a.uptr, a.urows, ub, tiles, a.per, a.nsplit, a.ca, a.cb, a.partial, (const T*)a.x_lo,    \
+                     (const T*)a.g_lo, a.set)
+  if (a.ca == C && a.cb == C)
+    OCNN_WP_KERNEL(false, 1);
   else if constexpr (C == 64)
-    hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, C, KK, NFULL, NHALF, GROUPS, true>),
-                       dim3(nsplit * GROUPS, ((ca + C - 1) / C) * ((cb + C - 1) / C)), dim3(256), 0, st, (const T*)x, xb, (const T*)g,
-                       gb, loc, lb, uptr, urows, ub, tiles, per, nsplit, ca, cb, partial);
+    OCNN_WP_KERNEL(true, ((a.ca + C - 1) / C) * ((a.cb + C - 1) / C));
+#undef OCNN_WP_KERNEL
 }
 
-// the launches of one pass over the plan: per-range sums of x^T g into `partial`
+// per-range sums of x^T g into `partial`
 template <typename T>
-static void launch_wp_pass(const void* x, int64_t rows_x, const void* g, const uint16_t* loc, const int32_t* uptr,
-                           const int32_t* urows, int64_t plan_total, int64_t rows, int K, int ca, int cb,
-                           int nsplit, int64_t per, float* partial, hipStream_t st) {
-#define OCNN_WP_LAUNCH(CC, KK, NF, NH, GR) \
-  launch_wp<T, CC, KK, NF, NH, GR>(x, rows_x, g, loc, uptr, urows, plan_total, rows, ca, cb, nsplit, per, partial, st)
-  if (ca >= 64) {
-    if (K == 27) OCNN_WP_LAUNCH(64, 27, 3, 1, 2);
-    else if (K == 9) OCNN_WP_LAUNCH(64, 9, 2, 1, 1);
-    else if (K == 8) OCNN_WP_LAUNCH(64, 8, 2, 0, 1);
+static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
+#define OCNN_WP_LAUNCH(CC, KK, NF, NH, GR) launch_wp<T, CC, KK, NF, NH, GR>(a, st)
+  if (a.ca >= 64) {
+    if (a.K == 27) OCNN_WP_LAUNCH(64, 27, 3, 1, 2);
+    else if (a.K == 9) OCNN_WP_LAUNCH(64, 9, 2, 1, 1);
+    else if (a.K == 8) OCNN_WP_LAUNCH(64, 8, 2, 0, 1);
     else OCNN_WP_LAUNCH(64, 3, 1, 0, 1);
   } else {
-    if (K == 27) OCNN_WP_LAUNCH(32, 27, 7, 0, 1);
-    else if (K == 9) OCNN_WP_LAUNCH(32, 9, 3, 0, 1);
-    else if (K == 8) OCNN_WP_LAUNCH(32, 8, 2, 0, 1);
+    if (a.K == 27) OCNN_WP_LAUNCH(32, 27, 7, 0, 1);
+    else if (a.K == 9) OCNN_WP_LAUNCH(32, 9, 3, 0, 1);
+    else if (a.K == 8) OCNN_WP_LAUNCH(32, 8, 2, 0, 1);
     else OCNN_WP_LAUNCH(32, 3, 1, 0, 1);
   }
 #undef OCNN_WP_LAUNCH
 }
 
-// T: the type of x, g and gw (float: x and g go through the kernels as two bf16 pieces each,
-// three passes into three sets of sums, one reduction over all of them)
+// T: the type of x, g and gw.  float: x and g go through the kernel as two bf16 pieces each, the three
+// products as workgroups of one launch with sums of their own (a third of the ranges each: a third
+// of the sums to add up, and one launch where a small layer waited for three), one reduction over all of them
 template <typename T>
 static int run_wp(const void* x, int64_t rows_x, const void* g, const uint16_t* loc, const int32_t* uptr,
                   const int32_t* urows, int64_t plan_total, int64_t rows, int K, int ca, int cb,
@@ -474,40 +489,30 @@ static int run_wp(const void* x, int64_t rows_x, const void* g, const uint16_t* 
     set_error("conv_wgrad_planned: cannot query the device");
     return OCNN_ERR_HIP;
   }
-  const int nsplit = wp_splits(K, ca, cb, n_cu);
+  WpArgs a{x, g, nullptr, nullptr, kPieces ? 3 : 1, rows_x, rows, 0, 0, plan_total, loc, uptr, urows, K, ca, cb, 0, nullptr};
+  a.nsplit = wp_splits(K, ca, cb, n_cu, a.products);
   const int64_t tiles = cdiv(rows, kWpRows);
-  const int64_t per = std::max<int64_t>(1, cdiv(tiles, nsplit));
-  const int used = (int)cdiv(tiles, per);                 // ranges that hold tiles
-  const int64_t set = (int64_t)used * K * ca * cb;         // floats of one set of sums
+  a.per = std::max<int64_t>(1, cdiv(tiles, a.nsplit));
+  const int used = (int)cdiv(tiles, a.per);               // ranges that hold tiles
+  a.set = (int64_t)used * K * ca * cb;                     // floats of one set of sums
   const int64_t xb = kPieces ? align_up(rows_x * ca * 2, 256) : 0, gb = kPieces ? align_up(rows * cb * 2, 256) : 0;
-  if (ws_bytes < 2 * xb + 2 * gb + (kPieces ? 3 : 1) * set * 4) {
+  if (ws_bytes < 2 * xb + 2 * gb + a.products * a.set * 4) {
     set_error("conv_wgrad_planned: workspace too small");
     return OCNN_ERR_WORKSPACE;
   }
-  float* partial = (float*)((char*)ws + 2 * xb + 2 * gb);
-  if constexpr (kPieces) {
-    if (rows > 0) {
-      bf16* xh = (bf16*)ws;
-      bf16* xl = (bf16*)((char*)ws + xb);
-      bf16* gh = (bf16*)((char*)ws + 2 * xb);
-      bf16* gl = (bf16*)((char*)ws + 2 * xb + gb);
-      if (rows_x > 0)
-        hipLaunchKernelGGL(split2_kernel, dim3((unsigned)cdiv(rows_x * ca, 256)), dim3(256), 0, st, (const float*)x,
-                           rows_x * ca, xh, xl);
-      hipLaunchKernelGGL(split2_kernel, dim3((unsigned)cdiv(rows * cb, 256)), dim3(256), 0, st, (const float*)g,
-                         rows * cb, gh, gl);
-      const bf16* xs[3] = {xh, xh, xl};
-      const bf16* gs[3] = {gh, gl, gh};
-      for (int i = 0; i < 3; ++i)
-        launch_wp_pass<bf16>(xs[i], rows_x, gs[i], loc, uptr, urows, plan_total, rows, K, ca, cb, nsplit, per,
-                             partial + i * set, st);
+  a.partial = (float*)((char*)ws + 2 * xb + 2 * gb);
+  if (rows > 0) {
+    if constexpr (kPieces) {
+      bf16 *xh = (bf16*)ws, *xl = (bf16*)((char*)ws + xb);
+      bf16 *gh = (bf16*)((char*)ws + 2 * xb), *gl = (bf16*)((char*)ws + 2 * xb + gb);
+      launch_split2(x, rows_x * ca, xh, xl, g, rows * cb, gh, gl, st);
+      a.x = xh, a.x_lo = xl, a.g = gh, a.g_lo = gl;
+      launch_wp_sums<bf16>(a, st);
+    } else {
+      launch_wp_sums<T>(a, st);
     }
-    launch_wgrad_reduce<float>(partial, rows > 0 ? 3 * used : 0, K, ca, cb, out_transposed, (float*)gw, st);
-  } else {
-    if (rows > 0)
-      launch_wp_pass<T>(x, rows_x, g, loc, uptr, urows, plan_total, rows, K, ca, cb, nsplit, per, partial, st);
-    launch_wgrad_reduce<T>(partial, rows > 0 ? used : 0, K, ca, cb, out_transposed, (T*)gw, st);
   }
+  launch_wgrad_reduce<T>(a.partial, rows > 0 ? a.products * used : 0, K, ca, cb, out_transposed, (T*)gw, st);
   return check_launch("conv_wgrad_planned");
 }
 
