@@ -365,6 +365,10 @@ struct BatchNormBackward : public Node {
   std::string name() const override { return "BatchNormReluBackward"; }
 };
 
+bool known_type(const Tensor& t) {
+  return t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16;
+}
+
 // batch_stats: statistics of this batch (and, with track, the running ones moved by `factor`);
 // otherwise the running statistics.  count: num_batches_tracked, incremented with the statistics.
 Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, const Tensor& running_mean,
@@ -387,11 +391,8 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
       mean = stats[0];
       invstd = stats[2];
       Tensor var = stats[1], ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), x);
-      const auto known = [](const Tensor& t) {
-        return t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16;
-      };
       const bool moves = track && running_mean.defined();
-      const bool in_place = moves && known(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
+      const bool in_place = moves && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
                             running_mean.is_contiguous() && running_var.is_contiguous();
       check(ocnn_batch_norm_stats(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
                                   (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
@@ -403,9 +404,6 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
         running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
         running_var.mul_(1 - factor).add_(unbiased.to(running_var.scalar_type()), factor);
       }
-    } else {
-      mean = running_mean.to(at::kFloat).contiguous();
-      invstd = at::rsqrt(running_var.to(at::kFloat) + eps);
     }
     y = at::empty_like(x);
     Tensor residual;
@@ -414,8 +412,20 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
       TORCH_CHECK(residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type(),
                   "batch_norm: the residual does not match the input");
     }
+    const int pcode = param_code(gamma, beta);
+    if (!batch_stats && !grad && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
+        running_mean.is_contiguous() && running_var.is_contiguous()) {
+      check(ocnnx_batch_norm_running(code, ptr(x), rows, (int)c, running_mean.data_ptr(), running_var.data_ptr(),
+                                     code_of(running_mean.scalar_type()), (float)eps, ptr(gamma), ptr(beta), pcode, relu,
+                                     ptr(residual), y.data_ptr(), st));
+      return y;
+    }
+    if (!batch_stats) {                               // (the backward pass reads mean and invstd)
+      mean = running_mean.to(at::kFloat).contiguous();
+      invstd = at::rsqrt(running_var.to(at::kFloat) + eps);
+    }
     check(ocnn_batch_norm_apply(code, ptr(x), rows, (int)c, (const float*)mean.data_ptr(), (const float*)invstd.data_ptr(),
-                                ptr(gamma), ptr(beta), param_code(gamma, beta), relu, ptr(residual), y.data_ptr(), st));
+                                ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(), st));
   }
   if (grad) {
     auto node = make_node<BatchNormBackward>(inputs);

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "host_api.hpp"
 
 namespace ocnn {
 
@@ -188,7 +189,9 @@ __global__ void bn_stats_finish_kernel(const float* __restrict__ partial, int nb
 
 // y = (x - mean) * (invstd * gamma) + beta (+ res), then max(., 0) when relu.  A thread keeps the
 // constants of its VEC channels in registers and walks every rpp-th row of the workgroup's
-// range, four rows in flight.
+// range, four rows in flight.  run_mean, run_var (dtype rdtype), when given, take the place of mean
+// and invstd: a module's running statistics as it holds them, the reciprocal formed here (made into
+// mean and invstd by passes of their own they were four of the five launches of a layer in evaluation).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, int64_t rows, int C,
                                                        int64_t rows_per_blk,
@@ -196,16 +199,28 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
                                                        const float* __restrict__ invstd,
                                                        const void* __restrict__ gamma,
                                                        const void* __restrict__ beta, int pdtype, int relu,
-                                                       const T* __restrict__ res, T* __restrict__ y) {
+                                                       const T* __restrict__ res, T* __restrict__ y,
+                                                       const void* __restrict__ run_mean,
+                                                       const void* __restrict__ run_var, int rdtype, float eps) {
   typedef BnVec<T, VEC> V;
   const int lpr = C / VEC, rpp = 256 / lpr;
   const int tid = threadIdx.x, rl = tid / lpr, cl = tid - rl * lpr;
   if (rl >= rpp) return;
   float m[VEC], sc[VEC], be[VEC];
+  if (run_var) {
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) {
-    m[v] = mean[cl * VEC + v];
-    sc[v] = invstd[cl * VEC + v];
+    for (int v = 0; v < VEC; ++v) {
+      m[v] = bn_param(run_mean, rdtype, cl * VEC + v, 0.f);
+      sc[v] = bn_param(run_var, rdtype, cl * VEC + v, 0.f);
+    }
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) sc[v] = 1.f / sqrtf(sc[v] + eps);
+  } else {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      m[v] = mean[cl * VEC + v];
+      sc[v] = invstd[cl * VEC + v];
+    }
   }
   {
     float ga[VEC];
@@ -467,21 +482,38 @@ extern "C" int ocnn_batch_norm_stats(int dtype, const void* x, int64_t rows, int
   return check_launch("batch_norm_stats");
 }
 
-extern "C" int ocnn_batch_norm_apply(int dtype, const void* x, int64_t rows, int channels, const float* mean,
-                                     const float* invstd, const void* gamma, const void* beta, int param_dtype,
-                                     int relu, const void* residual, void* y, void* stream) {
-  OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_apply: shape not supported");
-  OCNN_REQUIRE_PTRS("batch_norm_apply", x, mean, invstd, y);
-  hipStream_t st = (hipStream_t)stream;
+static int bn_apply(int dtype, const void* x, int64_t rows, int channels, const float* mean, const float* invstd,
+                    const void* gamma, const void* beta, int param_dtype, int relu, const void* residual, void* y,
+                    const void* run_mean, const void* run_var, int run_dtype, float eps, hipStream_t st) {
   int64_t per;
   int nblk;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
     bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_apply_kernel<T, VEC>), &per, &nblk);
     hipLaunchKernelGGL((bn_apply_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, per,
-                       mean, invstd, gamma, beta, param_dtype, relu, (const T*)residual, (T*)y);
+                       mean, invstd, gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var,
+                       run_dtype, eps);
   });
   return check_launch("batch_norm_apply");
+}
+
+extern "C" int ocnn_batch_norm_apply(int dtype, const void* x, int64_t rows, int channels, const float* mean,
+                                     const float* invstd, const void* gamma, const void* beta, int param_dtype,
+                                     int relu, const void* residual, void* y, void* stream) {
+  OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_apply: shape not supported");
+  OCNN_REQUIRE_PTRS("batch_norm_apply", x, mean, invstd, y);
+  return bn_apply(dtype, x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, residual, y, nullptr, nullptr, 0,
+                  0.f, (hipStream_t)stream);
+}
+
+extern "C" int ocnnx_batch_norm_running(int dtype, const void* x, int64_t rows, int channels, const void* running_mean,
+                                        const void* running_var, int running_dtype, float eps, const void* gamma,
+                                        const void* beta, int param_dtype, int relu, const void* residual, void* y,
+                                        void* stream) {
+  OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_running: shape not supported");
+  OCNN_REQUIRE_PTRS("batch_norm_running", x, running_mean, running_var, y);
+  return bn_apply(dtype, x, rows, channels, nullptr, nullptr, gamma, beta, param_dtype, relu, residual, y, running_mean,
+                  running_var, running_dtype, eps, (hipStream_t)stream);
 }
 
 extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy, int64_t rows, int channels,
