@@ -1,11 +1,14 @@
 // Octree construction: the sort of the point keys, the numbering of every layer's nodes in one
 // pass over the sorted points, keys and children of all layers, the per-leaf signal averages, and
 // the regrowing of an octree from split decisions.
+#include <algorithm>
 #include <cstring>
 
 #include <rocprim/rocprim.hpp>
 
 #include "common.hpp"
+#include "host_api.hpp"
+#include "morton.hpp"
 
 namespace ocnn {
 
@@ -183,21 +186,33 @@ struct BuildTree {
   int64_t* keys[kBuildMaxDepth + 1];
   int32_t* children[kBuildMaxDepth + 1];
   int64_t begin[kBuildMaxDepth + 2];   // running total of the node counts, by depth
+  int32_t* index[kBuildMaxDepth + 1];  // (optional) the non-empty nodes of the layers from the deepest full one on
 };
 
-// full layers, and -1 in the children of every other layer
+// Full layers, and -1 in the children of every other layer.  Four nodes a thread (the layers below the
+// full ones are whole groups of eight, and so are the full ones from layer 1 on).
 __global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= t.begin[depth + 1]) return;
-  int d = 0;
-  while (i >= t.begin[d + 1]) ++d;
-  const int64_t j = i - t.begin[d];
-  if (d <= full_depth) {
-    t.keys[d][j] = (j & ((1ll << (3 * d)) - 1)) | ((j >> (3 * d)) << 48);
-    t.children[d][j] = d < full_depth ? (int32_t)j : -1;
-  } else {
-    t.children[d][j] = -1;
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (i >= t.begin[depth + 1] - t.begin[1] + 4 * ((t.begin[1] + 3) / 4)) return;
+  const int64_t root = 4 * ((t.begin[1] + 3) / 4);            // layer 0 (a node per octree) padded to groups of four
+  if (i < root) {
+    for (int64_t j = i; j < i + 4 && j < t.begin[1]; ++j) {
+      t.keys[0][j] = j << 48;
+      t.children[0][j] = full_depth > 0 ? (int32_t)j : -1;
+    }
+    return;
   }
+  const int64_t at = i - root + t.begin[1];
+  int d = 1;
+  while (at >= t.begin[d + 1]) ++d;
+  const int64_t j = at - t.begin[d];
+  int4 c = make_int4(-1, -1, -1, -1);
+  if (d <= full_depth) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) t.keys[d][j + u] = ((j + u) & ((1ll << (3 * d)) - 1)) | (((j + u) >> (3 * d)) << 48);
+    if (d < full_depth) c = make_int4((int)j, (int)j + 1, (int)j + 2, (int)j + 3);
+  }
+  *(int4*)(t.children[d] + j) = c;
 }
 
 // Numbers every point's nodes (its span's offsets + the starts before it inside the span, counted
@@ -263,6 +278,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
         const int64_t kl = m >> (3 * l);
         const int64_t p = (int64_t)s[l + 1 < N ? l + 1 : l] - 1;
         t.children[d][(p << 3) | (kl & 7)] = (int32_t)s[l] - 1;
+        if (t.index[d]) t.index[d][s[l] - 1] = (int32_t)((p << 3) | (kl & 7));
         if (l + 1 <= lv[it]) {
           const int64_t first = (b << 48) | ((kl >> 3) << 3);
           int64_t* dst = t.keys[d] + (p << 3);
@@ -273,8 +289,10 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     }
     if (lv[it] >= levels) {
       const int64_t at = (b << (3 * full_depth)) | (m >> (3 * levels));
-      if (at < t.begin[full_depth + 1] - t.begin[full_depth])      // a batch id beyond batch_size has no node
+      if (at < t.begin[full_depth + 1] - t.begin[full_depth]) {    // a batch id beyond batch_size has no node
         t.children[full_depth][at] = (int32_t)top - 1;
+        if (t.index[full_depth]) t.index[full_depth][top - 1] = (int32_t)at;
+      }
     }
   }
 }
@@ -343,7 +361,7 @@ static int build_fill_t(const char* ws, int64_t n, int key_bits, int depth, int 
   if (build_layout_t<K, N>(n, &L) != OCNN_OK) { set_error("octree_build_fill: rocprim size query failed"); return OCNN_ERR_HIP; }
   const K* csorted = (const K*)(ws + L.csorted);
   const uint32_t* offs = (const uint32_t*)(ws + L.offs);
-  hipLaunchKernelGGL(build_init_kernel, dim3((unsigned)cdiv(t.begin[depth + 1], 256)), dim3(256), 0, st, t, depth,
+  hipLaunchKernelGGL(build_init_kernel, dim3((unsigned)cdiv(t.begin[depth + 1] + 4, 1024)), dim3(256), 0, st, t, depth,
                      full_depth);
   hipLaunchKernelGGL((build_scatter_kernel<K, N>), dim3((unsigned)L.spans), dim3(kBuildThreads), 0, st, csorted, offs,
                      perm, n, key_bits, depth, full_depth, t, inverse, seg_start);
@@ -504,10 +522,9 @@ extern "C" int ocnn_octree_build_scan(const int64_t* key, int64_t n, int depth, 
 #undef OCNN_BUILD_SCAN
 }
 
-extern "C" int ocnn_octree_build_fill(const void* workspace, int64_t n, int depth, int full_depth, int batch_size,
-                                      int batch_bits, const int64_t* h_sizes, const int32_t* perm,
-                                      int64_t* const* h_keys, int32_t* const* h_children, int64_t* inverse,
-                                      int32_t* seg_start, void* stream) {
+static int build_fill(const void* workspace, int64_t n, int depth, int full_depth, int batch_size, int batch_bits,
+                      const int64_t* h_sizes, const int32_t* perm, int64_t* const* h_keys, int32_t* const* h_children,
+                      int32_t* const* h_index, int64_t* inverse, int32_t* seg_start, void* stream) {
   if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
   OCNN_REQUIRE(batch_size >= 1 && batch_size <= (1 << batch_bits) && ((int64_t)batch_size << (3 * full_depth)) < (1ll << 31),
                "octree_build_fill: batch_size=%d does not fit batch_bits=%d / full_depth=%d", batch_size, batch_bits,
@@ -522,6 +539,7 @@ extern "C" int ocnn_octree_build_fill(const void* workspace, int64_t n, int dept
                  "octree_build_fill: depth %d: %lld nodes or a missing array", d, (long long)nnum);
     t.keys[d] = h_keys[d];
     t.children[d] = h_children[d];
+    t.index[d] = h_index ? h_index[d] : nullptr;
     t.begin[d + 1] = t.begin[d] + nnum;
   }
   OCNN_REQUIRE(h_sizes[levels] <= ((int64_t)batch_size << (3 * full_depth)),
@@ -531,4 +549,301 @@ extern "C" int ocnn_octree_build_fill(const void* workspace, int64_t n, int dept
   build_fill_t<K, N>((const char*)workspace, n, key_bits, depth, full_depth, t, perm, inverse, seg_start, (hipStream_t)stream)
   OCNN_BUILD_DISPATCH(OCNN_BUILD_FILL);
 #undef OCNN_BUILD_FILL
+}
+
+extern "C" int ocnn_octree_build_fill(const void* workspace, int64_t n, int depth, int full_depth, int batch_size,
+                                      int batch_bits, const int64_t* h_sizes, const int32_t* perm,
+                                      int64_t* const* h_keys, int32_t* const* h_children, int64_t* inverse,
+                                      int32_t* seg_start, void* stream) {
+  return build_fill(workspace, n, depth, full_depth, batch_size, batch_bits, h_sizes, perm, h_keys, h_children, nullptr,
+                    inverse, seg_start, stream);
+}
+
+extern "C" int ocnnx_tree_fill(const void* workspace, int64_t n, int depth, int full_depth, int batch_size, int batch_bits,
+                               const int64_t* h_sizes, const int32_t* perm, int64_t* const* h_keys,
+                               int32_t* const* h_children, int32_t* const* h_index, int64_t* inverse, int32_t* seg_start,
+                               void* stream) {
+  OCNN_REQUIRE_PTRS("tree_fill", h_index);
+  return build_fill(workspace, n, depth, full_depth, batch_size, batch_bits, h_sizes, perm, h_keys, h_children, h_index,
+                    inverse, seg_start, stream);
+}
+
+// ---- keys and sort ----------------------------------------------------------------------------
+// The library's radix sort takes 95 us for 20 000 points (five kernels of 15 us, most of it the chains
+// of its decoupled look-back, and seven fills), four times what its bytes cost.  Here a
+// cloud is a number of spans of kSortSpan points and a pass is counts of the digit by span, then one stable
+// scatter.  Up to kSortInlineSpans spans every workgroup of the scatter reads the counts of all spans
+// itself; more of them are scanned by a launch in between.  Digits have up to 11 bits: a depth-6
+// octree takes two passes, depth 9 with eight clouds three.
+constexpr int kSortSpan = 2048;
+constexpr int kSortThreads = 256, kSortItems = kSortSpan / kSortThreads;
+constexpr int kSortMaxBits = 11;
+constexpr int kSortInlineSpans = 64;
+constexpr int64_t kSortMaxPoints = 1 << 22;
+constexpr int64_t kSortAtomicMax = 32768;   // up to here a pass counts the next digit with atomics instead of a launch
+
+struct SortPlan {
+  int passes, bits;                          // digits of `bits` bits
+  int spans;
+  int64_t key[2], val[2], hist[2], totals, total;   // workspace offsets: ping-pong keys and values, counts [span][digit]
+};
+
+static SortPlan sort_plan(int64_t n, int total_bits) {
+  SortPlan s;
+  s.passes = std::max(1, (int)cdiv(total_bits, kSortMaxBits));
+  s.bits = std::max(1, (int)cdiv(total_bits, s.passes));
+  s.spans = (int)cdiv(n, kSortSpan);
+  int64_t off = 0;
+  for (int i = 0; i < 2; ++i) { s.key[i] = off; off += align_up(n * 4, 256); }
+  for (int i = 0; i < 2; ++i) { s.val[i] = off; off += align_up(n * 4, 256); }
+  for (int i = 0; i < 2; ++i) { s.hist[i] = off; off += align_up(((int64_t)s.spans << s.bits) * 4, 256); }
+  s.totals = off; off += align_up(4ll << s.bits, 256);
+  s.total = off;
+  return s;
+}
+
+// Normalised points and their sort keys (batch id right above the Morton bits), the counts of the
+// first digit by span, and zeros for the counts of the second.
+__global__ __launch_bounds__(kSortThreads) void tree_keys_kernel(
+    const float* __restrict__ pts, int64_t n, float bx, float by, float bz, float factor, const void* __restrict__ batch,
+    int batch_is_float, int depth, float* __restrict__ pts_out, uint32_t* __restrict__ key, int bits,
+    uint32_t* __restrict__ hist, uint32_t* __restrict__ hist_next) {
+  __shared__ uint32_t s_hist[1 << kSortMaxBits];
+  const int bins = 1 << bits;
+  for (int i = threadIdx.x; i < bins; i += kSortThreads) s_hist[i] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kSortItems; ++it) {
+    const int64_t i = (int64_t)blockIdx.x * kSortSpan + it * kSortThreads + threadIdx.x;
+    if (i >= n) continue;
+    // (p - bbmin) * factor: a subtraction then a multiplication, each rounded
+    const float px = (pts[3 * i + 0] - bx) * factor;
+    const float py = (pts[3 * i + 1] - by) * factor;
+    const float pz = (pts[3 * i + 2] - bz) * factor;
+    pts_out[3 * i + 0] = px;
+    pts_out[3 * i + 1] = py;
+    pts_out[3 * i + 2] = pz;
+    uint64_t k = (uint64_t)encode((int64_t)px, (int64_t)py, (int64_t)pz, depth);      // trunc toward 0
+    if (batch) {
+      const int64_t b = batch_is_float ? (int64_t)((const float*)batch)[i] : ((const int64_t*)batch)[i];
+      k |= ((uint64_t)b & 0xffffull) << (3 * depth);
+    }
+    key[i] = (uint32_t)k;
+    atomicAdd(&s_hist[(uint32_t)k & (uint32_t)(bins - 1)], 1u);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < bins; i += kSortThreads) {
+    hist[(int64_t)blockIdx.x * bins + i] = s_hist[i];
+    hist_next[(int64_t)blockIdx.x * bins + i] = 0u;
+  }
+}
+
+__global__ __launch_bounds__(kSortThreads) void tree_digits_kernel(const uint32_t* __restrict__ key, int64_t n, int shift,
+                                                                   int bits, uint32_t* __restrict__ hist) {
+  __shared__ uint32_t s_hist[1 << kSortMaxBits];
+  const int bins = 1 << bits;
+  for (int i = threadIdx.x; i < bins; i += kSortThreads) s_hist[i] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kSortItems; ++it) {
+    const int64_t i = (int64_t)blockIdx.x * kSortSpan + it * kSortThreads + threadIdx.x;
+    if (i < n) atomicAdd(&s_hist[(key[i] >> shift) & (uint32_t)(bins - 1)], 1u);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < bins; i += kSortThreads) hist[(int64_t)blockIdx.x * bins + i] = s_hist[i];
+}
+
+// hist[span][digit] -> points of the digit in the spans before; totals[digit].  A workgroup takes 16
+// digits, 64 threads each a run of spans.
+__global__ __launch_bounds__(1024) void tree_spans_kernel(uint32_t* __restrict__ hist, int spans, int bins,
+                                                          uint32_t* __restrict__ totals) {
+  __shared__ uint32_t s_run[64][17];
+  const int b = blockIdx.x * 16 + (threadIdx.x & 15), c = threadIdx.x >> 4;
+  const int per = (spans + 63) / 64, lo = min(spans, c * per), hi = min(spans, lo + per);
+  uint32_t sum = 0u;
+  if (b < bins) {
+#pragma unroll 8
+    for (int sp = lo; sp < hi; ++sp) sum += hist[(int64_t)sp * bins + b];
+  }
+  s_run[c][threadIdx.x & 15] = sum;
+  __syncthreads();
+  uint32_t run = 0u;
+  for (int i = 0; i < c; ++i) run += s_run[i][threadIdx.x & 15];
+  if (b >= bins) return;
+  if (c == 63) totals[b] = run + sum;
+  for (int sp = lo; sp < hi; ++sp) {
+    const uint32_t v = hist[(int64_t)sp * bins + b];
+    hist[(int64_t)sp * bins + b] = run;
+    run += v;
+  }
+}
+
+// One stable pass.  A wave takes 128 consecutive points, 64 at a time: the lanes with the same digit
+// find each other with one ballot per bit, their rank among the wave's points is kept in registers;
+// the counts of the waves and of the spans before turn it into a place.  hist_next (or null): the
+// counts of the digit above, by the span that is written to.  totals: hist has been scanned.  (Sixteen waves a span and not four:
+// the ballots of a wave are a serial chain, 23 -> 9 us for 20 000 points.)
+constexpr int kPassThreads = 1024;
+__global__ __launch_bounds__(kPassThreads) void tree_sort_kernel(
+    const uint32_t* __restrict__ key, const uint32_t* __restrict__ val, int64_t n, int shift, int bits, int spans,
+    const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals, uint32_t* __restrict__ hist_next,
+    uint32_t* __restrict__ key_out, uint32_t* __restrict__ val_out) {
+  constexpr int kWaves = kPassThreads / 64, kMaxBins = 1 << kSortMaxBits, kPer = kMaxBins / kPassThreads;
+  constexpr int kItems = kSortSpan / kPassThreads;
+  __shared__ uint16_t s_cnt[kWaves][kMaxBins];               // points of a digit: in the wave, then in the waves before
+  __shared__ uint32_t s_base[kMaxBins];                      // first place of this span's points of a digit
+  __shared__ uint32_t s_wave[kWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int bins = 1 << bits;
+  const int64_t first = (int64_t)blockIdx.x * kSortSpan + wave * (kSortSpan / kWaves) + lane;
+  uint32_t k[kItems], v[kItems], rank[kItems];
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const int64_t i = first + it * 64;
+    k[it] = i < n ? key[i] : 0u;
+    v[it] = val == nullptr ? (uint32_t)i : (i < n ? val[i] : 0u);
+  }
+  // digit counts of all spans: thread t on the bins 2 t, 2 t + 1
+  uint32_t all[kPer], before[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int b = tid * kPer + u;
+    all[u] = before[u] = 0u;
+    if (b < bins && totals) {
+      all[u] = totals[b];
+      before[u] = hist[(int64_t)blockIdx.x * bins + b];
+    } else if (b < bins) {
+#pragma unroll 8
+      for (int sp = 0; sp < spans; ++sp) {
+        const uint32_t c = hist[(int64_t)sp * bins + b];
+        all[u] += c;
+        before[u] += sp < (int)blockIdx.x ? c : 0u;
+      }
+    }
+  }
+  for (int i = tid; i < bins; i += kPassThreads)
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s_cnt[w][i] = 0;
+  uint32_t own = 0u;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) own += all[u];
+  uint32_t incl = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t up = __shfl_up(incl, o);
+    if (lane >= o) incl += up;
+  }
+  if (lane == 63) s_wave[wave] = incl;
+  __syncthreads();
+  uint32_t at = incl - own;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) at += w < wave ? s_wave[w] : 0u;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int b = tid * kPer + u;
+    if (b < bins) s_base[b] = at + before[u];
+    at += all[u];
+  }
+  // ranks within the wave
+  volatile uint16_t* cnt = s_cnt[wave];
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const bool ok = first + it * 64 < n;
+    const uint32_t d = (k[it] >> shift) & (uint32_t)(bins - 1);
+    unsigned long long same = __ballot(ok);
+    for (int b = 0; b < bits; ++b) {
+      const unsigned long long ones = __ballot((d >> b) & 1u);
+      same &= (d >> b) & 1u ? ones : ~ones;
+    }
+    const uint32_t seen = cnt[d], r = lanes_below(same);
+    rank[it] = seen + r;
+    if (ok && r == 0u) cnt[d] = (uint16_t)(seen + (uint32_t)__popcll(same));
+  }
+  __syncthreads();
+  for (int b = tid; b < bins; b += kPassThreads) {
+    uint32_t run = 0u;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const uint32_t c = s_cnt[w][b];
+      s_cnt[w][b] = (uint16_t)run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    if (first + it * 64 >= n) continue;
+    const uint32_t d = (k[it] >> shift) & (uint32_t)(bins - 1);
+    const uint32_t to = s_base[d] + s_cnt[wave][d] + rank[it];
+    key_out[to] = k[it];
+    val_out[to] = v[it];
+    if (hist_next)
+      atomicAdd(&hist_next[(int64_t)(to / kSortSpan) * bins + ((k[it] >> (shift + bits)) & (uint32_t)(bins - 1))], 1u);
+  }
+}
+
+static int tree_key_bits(int depth, int batch_bits) { return 3 * depth + batch_bits; }
+static bool tree_own_sort(int64_t n, int depth, int batch_bits) {
+  return n <= kSortMaxPoints && tree_key_bits(depth, batch_bits) <= 32;
+}
+
+extern "C" int64_t ocnnx_tree_workspace_bytes(int64_t n, int depth, int full_depth, int batch_bits) {
+  const int64_t base = ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits);
+  if (base < 0) return base;
+  return base + (tree_own_sort(n, depth, batch_bits) ? sort_plan(n, tree_key_bits(depth, batch_bits)).total
+                                                   : align_up(n * 8, 256));
+}
+
+extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
+                               int batch_is_float, int depth, int full_depth, int batch_bits, float* pts_out,
+                               void* workspace, int64_t workspace_bytes, int32_t* perm, int64_t* sizes, void* stream) {
+  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
+  OCNN_REQUIRE_PTRS("tree_scan", pts, h_bbmin, pts_out, workspace, perm, sizes);
+  if (workspace_bytes < ocnnx_tree_workspace_bytes(n, depth, full_depth, batch_bits)) {
+    set_error("tree_scan: workspace too small");
+    return OCNN_ERR_WORKSPACE;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int key_bits = 3 * depth, levels = depth - full_depth;
+  const int64_t base = ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits);
+  char* more = (char*)workspace + base;
+  if (!tree_own_sort(n, depth, batch_bits)) {
+    int64_t* key = (int64_t*)more;
+    if (int rc = ocnn_points2key(pts, n, h_bbmin, factor, batch, batch_is_float, depth, pts_out, key, stream)) return rc;
+    return ocnn_octree_build_scan(key, n, depth, full_depth, batch_bits, workspace, base, perm, sizes, stream);
+  }
+  const SortPlan s = sort_plan(n, tree_key_bits(depth, batch_bits));
+  uint32_t* keys[2] = {(uint32_t*)(more + s.key[0]), (uint32_t*)(more + s.key[1])};
+  uint32_t* vals[2] = {(uint32_t*)(more + s.val[0]), (uint32_t*)(more + s.val[1])};
+  uint32_t* hist[2] = {(uint32_t*)(more + s.hist[0]), (uint32_t*)(more + s.hist[1])};
+  const bool atomics = n <= kSortAtomicMax && s.passes <= 2;   // (a third pass would need its counts cleared)
+  uint32_t* totals = s.spans > kSortInlineSpans ? (uint32_t*)(more + s.totals) : nullptr;
+  BuildLayout L;
+  if (build_layout_t<uint32_t, 8>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
+  if (levels + 1 > 8 && build_layout_t<uint32_t, 16>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
+  uint32_t* csorted = (uint32_t*)((char*)workspace + L.csorted);
+  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
+  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
+  const dim3 grid((unsigned)s.spans), block(kSortThreads);
+  hipLaunchKernelGGL(tree_keys_kernel, grid, block, 0, st, pts, n, h_bbmin[0], h_bbmin[1], h_bbmin[2], factor, batch,
+                     batch_is_float, depth, pts_out, keys[0], s.bits, hist[0], hist[1]);
+  for (int p = 0; p < s.passes; ++p) {
+    const bool last = p + 1 == s.passes;
+    if (p > 0 && !atomics)
+      hipLaunchKernelGGL(tree_digits_kernel, grid, block, 0, st, keys[p & 1], n, p * s.bits, s.bits, hist[p & 1]);
+    if (totals)
+      hipLaunchKernelGGL(tree_spans_kernel, dim3((unsigned)cdiv(1 << s.bits, 16)), dim3(1024), 0, st, hist[p & 1], s.spans,
+                         1 << s.bits, totals);
+    hipLaunchKernelGGL(tree_sort_kernel, grid, dim3(kPassThreads), 0, st, keys[p & 1], p == 0 ? nullptr : vals[p & 1], n, p * s.bits,
+                       s.bits, s.spans, hist[p & 1], totals, atomics && !last ? hist[(p + 1) & 1] : nullptr,
+                       last ? csorted : keys[(p + 1) & 1], last ? (uint32_t*)perm : vals[(p + 1) & 1]);
+  }
+#define OCNN_TREE_COUNT(N)                                                                                              \
+  hipLaunchKernelGGL((build_count_kernel<uint32_t, N>), dim3((unsigned)L.spans), dim3(kBuildThreads), 0, st, csorted, n, \
+                     key_bits, levels, sums);                                                                            \
+  hipLaunchKernelGGL(build_offsets_kernel<N>, dim3(1), dim3(1024), 0, st, sums, L.spans, levels, offs, sizes)
+  if (levels + 1 <= 8) { OCNN_TREE_COUNT(8); }
+  else { OCNN_TREE_COUNT(16); }
+#undef OCNN_TREE_COUNT
+  return check_launch("tree_scan");
 }

@@ -446,6 +446,111 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
   return y;
 }
 
+// ---- octree (octree/octree.py) ----------------------------------------------------------------
+
+struct Tree {
+  std::vector<Tensor> keys, children;
+  std::vector<OptTensor> index;               // of the non-empty nodes, from the deepest full layer on
+  std::vector<int64_t> nnum, nnum_nempty;
+  Tensor idx, points, perm, seg_start;
+  OptTensor normals;
+};
+
+// Build from the points: one sort, one numbering of all layers, one wait for the layers' sizes.
+Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<float> bbmin, double factor, int depth,
+                  int full_depth, int batch_size) {
+  require_gpu(pts);
+  pts = pts.to(at::kFloat).contiguous();
+  const int64_t n = pts.size(0);
+  bool batch_is_float = false;
+  if (batch.has_value()) {
+    batch_is_float = batch->is_floating_point();
+    batch = batch->reshape({-1}).to(batch_is_float ? at::kFloat : at::kLong).contiguous();
+  }
+  const auto i32 = pts.options().dtype(at::kInt), i64 = pts.options().dtype(at::kLong);
+  int batch_bits = 0;
+  while ((1 << batch_bits) < batch_size) ++batch_bits;
+  const int levels = depth - full_depth;
+  const int64_t ws_bytes = ocnnx_tree_workspace_bytes(n, depth, full_depth, batch_bits);
+  Tensor pts_norm = at::empty_like(pts), ws = workspace(ws_bytes, pts);
+  Tree t;
+  t.perm = at::empty({n}, i32);
+  // (written by the kernel straight into host memory: no copy to wait for on top of the kernel)
+  Tensor sizes = at::empty({levels + 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  const auto st = c10::hip::getCurrentHIPStream();
+  check(ocnnx_tree_scan((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
+                        full_depth, batch_bits, (float*)pts_norm.data_ptr(), ws.data_ptr(), ws_bytes,
+                        (int32_t*)t.perm.data_ptr(), (int64_t*)sizes.data_ptr(), st.stream()));
+  // what does not wait for the sizes is allocated while the sort runs
+  for (int d = 0; d <= full_depth; ++d) {
+    t.nnum.push_back((int64_t)batch_size << (3 * d));
+    t.keys.push_back(at::empty({t.nnum[d]}, i64));
+    t.children.push_back(at::empty({t.nnum[d]}, i32));
+  }
+  t.idx = at::empty({n}, i64);
+  t.seg_start = at::empty({n + 1}, i32);
+  if (normals.has_value()) normals = normals->to(at::kFloat).contiguous();
+  st.synchronize();
+  const std::vector<int64_t> size((int64_t*)sizes.data_ptr(), (int64_t*)sizes.data_ptr() + levels + 1);
+  for (int d = full_depth + 1; d <= depth; ++d) {
+    t.nnum.push_back(8 * size[depth - d + 1]);
+    t.keys.push_back(at::empty({t.nnum[d]}, i64));
+    t.children.push_back(at::empty({t.nnum[d]}, i32));
+  }
+  std::vector<int64_t*> keys;
+  std::vector<int32_t*> children, index;
+  for (int d = 0; d <= depth; ++d) {
+    t.nnum_nempty.push_back(d < full_depth ? t.nnum[d] : size[depth - d]);
+    t.index.push_back(d < full_depth ? OptTensor() : at::empty({t.nnum_nempty[d]}, i32));
+    keys.push_back((int64_t*)t.keys[d].data_ptr());
+    children.push_back((int32_t*)t.children[d].data_ptr());
+    index.push_back(d < full_depth ? nullptr : (int32_t*)t.index[d]->data_ptr());
+  }
+  check(ocnnx_tree_fill(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, size.data(),
+                        (const int32_t*)t.perm.data_ptr(), keys.data(), children.data(), index.data(),
+                        (int64_t*)t.idx.data_ptr(), (int32_t*)t.seg_start.data_ptr(), st.stream()));
+  t.points = at::empty({size[0], 3}, pts.options());
+  if (normals.has_value()) {
+    t.normals = at::empty({size[0], 3}, pts.options());
+    check(ocnn_leaf_points_normals((const float*)pts_norm.data_ptr(), (const float*)normals->data_ptr(),
+                                   (const int32_t*)t.perm.data_ptr(), (const int32_t*)t.seg_start.data_ptr(), size[0],
+                                   (float*)t.points.data_ptr(), (float*)t.normals->data_ptr(), st.stream()));
+  } else {
+    check(ocnn_leaf_average((const float*)pts_norm.data_ptr(), 3, (const int32_t*)t.perm.data_ptr(),
+                            (const int32_t*)t.seg_start.data_ptr(), size[0], 0, (float*)t.points.data_ptr(), st.stream()));
+  }
+  return t;
+}
+
+// The neighbour tables of layers 1 .. depth (entry 0 is left out).
+std::vector<Tensor> all_neigh(const std::vector<Tensor>& keys, const std::vector<Tensor>& children,
+                              const std::vector<OptTensor>& index, const std::vector<int64_t>& nnum,
+                              const std::vector<int64_t>& nnum_nempty, int full_depth, int batch_size) {
+  const int depth = (int)keys.size() - 1;
+  std::vector<Tensor> out;
+  std::vector<const int64_t*> k;
+  std::vector<const int32_t*> c, i;
+  std::vector<int32_t*> o{nullptr};
+  for (int d = 0; d <= depth; ++d) {
+    require_gpu(children[d]);
+    TORCH_CHECK(keys[d].is_contiguous() && children[d].is_contiguous() && keys[d].numel() == nnum[d] &&
+                    children[d].numel() == nnum[d] && keys[d].scalar_type() == at::kLong &&
+                    children[d].scalar_type() == at::kInt &&
+                    (!index[d].has_value() || (index[d]->numel() == nnum_nempty[d] && index[d]->is_contiguous())),
+                "octree layer ", d, " is inconsistent");
+    k.push_back((const int64_t*)keys[d].data_ptr());
+    c.push_back((const int32_t*)children[d].data_ptr());
+    i.push_back((const int32_t*)ptr(index[d]));
+    if (d > 0) {
+      out.push_back(at::empty({nnum[d], 27}, children[d].options()));
+      o.push_back((int32_t*)out.back().data_ptr());
+    }
+  }
+  check(ocnnx_neigh_all(depth, full_depth, batch_size, nnum.data(), nnum_nempty.data(), k.data(), c.data(), i.data(),
+                        o.data(), hip_stream()));
+  return out;
+}
+
 Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 
 }  // namespace
@@ -493,6 +598,13 @@ PYBIND11_MODULE(ocnn_host, m) {
 #define FIELD(name) .def_readwrite(#name, &ConvLayer::name)
       FIELD(fwd) FIELD(dgrad) FIELD(wgrad) FIELD(fwd_table) FIELD(dgrad_table) FIELD(wgrad_table) FIELD(wgrad_of_grad);
 #undef FIELD
+  py::class_<Tree>(m, "Tree")
+#define FIELD(name) .def_readonly(#name, &Tree::name)
+      FIELD(keys) FIELD(children) FIELD(index) FIELD(nnum) FIELD(nnum_nempty) FIELD(idx) FIELD(points) FIELD(normals)
+          FIELD(perm) FIELD(seg_start);
+#undef FIELD
+  m.def("build_octree", &build_octree, py::call_guard<py::gil_scoped_release>());
+  m.def("all_neigh", &all_neigh, py::call_guard<py::gil_scoped_release>());
   m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;
   m.def("conv", &conv, py::call_guard<py::gil_scoped_release>());
   m.def("column_sum", &column_sum, py::call_guard<py::gil_scoped_release>());

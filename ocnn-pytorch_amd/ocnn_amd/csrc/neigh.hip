@@ -2,6 +2,7 @@
 // (from the parent level's table), non-empty index lists, the table variants
 // get_neigh hands out, and the inverse table used by the gather-form backward.
 #include "common.hpp"
+#include "host_api.hpp"
 #include "morton.hpp"
 
 namespace ocnn {
@@ -39,7 +40,9 @@ constexpr int kParentsPerBlock = 32;
 
 // The 8 x 27 entries below one parent repeat the same (parent slot, child number) pattern, so
 // the pattern sits in LDS once a workgroup, and a thread writes four entries at a time: they
-// never straddle two parents (216 = 4 * 54).
+// never straddle two parents (216 = 4 * 54).  NT: stores that pass the caches by, for tables that
+// would not stay in them (530 MB: 128 -> 102 us).
+template <bool NT>
 __global__ __launch_bounds__(256) void neigh_from_parent_kernel(
     const int32_t* __restrict__ child_p, const int32_t* __restrict__ neigh_p,
     const int32_t* __restrict__ nempty_p, int64_t n_ne, int64_t* __restrict__ out64,
@@ -52,15 +55,29 @@ __global__ __launch_bounds__(256) void neigh_from_parent_kernel(
     child_slot_lut(threadIdx.x / 27, threadIdx.x % 27, &lp, &lc);
     lut[threadIdx.x] = (uint16_t)(lp | (lc << 8));
   }
-  for (int e = threadIdx.x; e < kParentsPerBlock * 27; e += 256) {
-    int p = e / 27, s = e % 27;
-    int32_t v = -1;
-    if (c0 + p < n_ne) {
-      int32_t q = nempty_p[c0 + p];
-      int32_t np = neigh_p[(int64_t)q * 27 + s];
-      if (np >= 0) v = child_p[np];        // test before dereferencing
+  // parents' node, its neighbour in the slot, that node's ordinal: three dependent loads, the
+  // entries of a thread side by side so that a workgroup waits three times and not twelve
+  // (4.9 M rows: 215 -> 125 us, the rate of a plain fill is 80)
+  {
+    constexpr int kPer = (kParentsPerBlock * 27 + 255) / 256;
+    int32_t q[kPer], np[kPer], v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int e = threadIdx.x + 256 * i, p = e / 27;
+      q[i] = e < kParentsPerBlock * 27 && c0 + p < n_ne ? nempty_p[c0 + p] : -1;
     }
-    cp[e] = v;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int e = threadIdx.x + 256 * i;
+      np[i] = q[i] >= 0 ? neigh_p[(int64_t)q[i] * 27 + e % 27] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = np[i] >= 0 ? child_p[np[i]] : -1;      // test before dereferencing
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int e = threadIdx.x + 256 * i;
+      if (e < kParentsPerBlock * 27) cp[e] = v[i];
+    }
   }
   __syncthreads();
   const int64_t base = c0 * 216;
@@ -75,13 +92,98 @@ __global__ __launch_bounds__(256) void neigh_from_parent_kernel(
       r[e] = v < 0 ? -1 : v * 8 + (l >> 8);
     }
     const int64_t o = base + 4 * (int64_t)c;
-    if (out32) *reinterpret_cast<int4*>(out32 + o) = make_int4(r[0], r[1], r[2], r[3]);
+    typedef __attribute__((ext_vector_type(4))) int i32x4;
+    if (out32) {
+      const i32x4 v = {r[0], r[1], r[2], r[3]};
+      if (NT) __builtin_nontemporal_store(v, (i32x4*)(out32 + o));
+      else *(i32x4*)(out32 + o) = v;
+    }
     if (out64) {
       *reinterpret_cast<longlong2*>(out64 + o) = make_longlong2((int64_t)r[0], (int64_t)r[1]);
       *reinterpret_cast<longlong2*>(out64 + o + 2) = make_longlong2((int64_t)r[2], (int64_t)r[3]);
     }
   }
 }
+
+// Tables of the full layers and of the layers with few nodes, all in one launch.  A layer's table is made
+// from its parents' table, so that a kernel a layer is a chain of launches, 5 - 6 us each however few the nodes;
+// here a (parent, slot) finds the neighbouring parent by walking down the tree from the deepest
+// full layer instead, and no layer waits for another.  A workgroup: 256 entries of a full layer, or
+// the 8 x 27 entries below each of 32 parents.
+struct WalkTree {
+  const int64_t* keys[17];
+  const int32_t* children[17];
+  const int32_t* index[17];
+  int32_t* neigh[17];
+  int64_t n_ne[17];           // non-empty nodes, by depth
+  int64_t block0[18];         // first workgroup of a layer's table; block0[last + 1] = all of them
+  int last, full_depth, batch;
+};
+
+__global__ __launch_bounds__(256) void neigh_walk_kernel(WalkTree t) {
+  __shared__ int32_t cp[kParentsPerBlock * 27];
+  int d = 1;
+  while ((int64_t)blockIdx.x >= t.block0[d + 1]) ++d;
+  const int64_t blk = (int64_t)blockIdx.x - t.block0[d];
+  if (d <= t.full_depth) {
+    const int64_t per = 1ll << (3 * d), total = (int64_t)t.batch * per, e = blk * 256 + threadIdx.x;
+    if (e >= total * 27) return;
+    const int64_t node = e / 27;
+    const int k = (int)(e - node * 27);
+    const uint64_t local = (uint64_t)(node & (per - 1));
+    const int64_t x = (int64_t)compact3(local >> 2) + (k / 9 - 1);
+    const int64_t y = (int64_t)compact3(local >> 1) + ((k / 3) % 3 - 1);
+    const int64_t z = (int64_t)compact3(local) + (k % 3 - 1);
+    const int64_t bound = 1ll << d;
+    int64_t v = -1;
+    if (x >= 0 && y >= 0 && z >= 0 && x < bound && y < bound && z < bound) v = encode(x, y, z, d) + (node - (int64_t)local);
+    t.neigh[d][e] = (int32_t)v;
+    return;
+  }
+  const int64_t c0 = blk * kParentsPerBlock, n_ne = t.n_ne[d - 1];
+  const int fd = t.full_depth, up = d - 1;                   // parents live in layer d - 1
+  for (int e = threadIdx.x; e < kParentsPerBlock * 27; e += 256) {
+    const int p = e / 27, s = e - p * 27;
+    int32_t v = -1;
+    if (c0 + p < n_ne) {
+      const uint64_t key = (uint64_t)t.keys[up][t.index[up][c0 + p]];
+      const int64_t b = (int64_t)(key >> 48), bound = 1ll << up;
+      const uint64_t m = key & ((1ull << 48) - 1);
+      const int64_t x = (int64_t)compact3(m >> 2) + (s / 9 - 1);
+      const int64_t y = (int64_t)compact3(m >> 1) + ((s / 3) % 3 - 1);
+      const int64_t z = (int64_t)compact3(m) + (s % 3 - 1);
+      // (a batch id beyond the batch has nodes but no place in the full layer)
+      if (b < t.batch && x >= 0 && y >= 0 && z >= 0 && x < bound && y < bound && z < bound) {
+        const uint64_t to = (uint64_t)encode(x, y, z, up);
+        int64_t node = (b << (3 * fd)) + (int64_t)(to >> (3 * (up - fd)));
+        v = t.children[fd][node];                             // ordinal of the node among the non-empty ones of its layer
+        for (int l = fd + 1; l <= up && v >= 0; ++l)
+          v = t.children[l][(int64_t)v * 8 + (int64_t)((to >> (3 * (up - l))) & 7u)];
+      }
+    }
+    cp[e] = v;
+  }
+  __syncthreads();
+  const int parents = (int)(n_ne - c0 < kParentsPerBlock ? n_ne - c0 : kParentsPerBlock);
+  int32_t* out = t.neigh[d] + c0 * 216;
+  for (int c = threadIdx.x; c < parents * 54; c += 256) {
+    const int p = c / 54, w = (c - p * 54) * 4;
+    int32_t r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = (w + e) / 27, k = (w + e) - j * 27;
+      int lp, lc;
+      child_slot_lut(j, k, &lp, &lc);
+      const int32_t v = cp[p * 27 + lp];
+      r[e] = v < 0 ? -1 : v * 8 + lc;
+    }
+    *reinterpret_cast<int4*>(out + 4 * (int64_t)c) = make_int4(r[0], r[1], r[2], r[3]);
+  }
+}
+
+// layers with up to this many parents are found by walking (27 walks of a few dependent loads each); in
+// larger ones the two loads an entry takes from the parents' table are what counts
+constexpr int64_t kWalkMaxParents = 16384;
 
 __global__ void nempty_index_kernel(const int32_t* children, int64_t n, int32_t* i32,
                                     int64_t* i64) {
@@ -153,13 +255,23 @@ extern "C" int ocnn_neigh_full(int depth, int batch, int64_t* out64, int32_t* ou
   return check_launch("neigh_full");
 }
 
+constexpr int64_t kStreamBytes = 128ll << 20;
+
+static void launch_from_parent(const int32_t* child_p, const int32_t* neigh_p, const int32_t* nempty_p, int64_t n_ne,
+                               int64_t* out64, int32_t* out32, hipStream_t st) {
+  const dim3 grid((unsigned)cdiv(n_ne, kParentsPerBlock));
+  if (n_ne * 216 * 4 >= kStreamBytes)
+    hipLaunchKernelGGL(neigh_from_parent_kernel<true>, grid, dim3(256), 0, st, child_p, neigh_p, nempty_p, n_ne, out64, out32);
+  else
+    hipLaunchKernelGGL(neigh_from_parent_kernel<false>, grid, dim3(256), 0, st, child_p, neigh_p, nempty_p, n_ne, out64, out32);
+}
+
 extern "C" int ocnn_neigh_from_parent(const int32_t* child_p, const int32_t* neigh_p,
                                       const int32_t* nempty_p, int64_t n_ne, int64_t* out64,
                                       int32_t* out32, void* stream) {
   OCNN_REQUIRE(n_ne > 0 && n_ne * 8 < (1ll << 31), "neigh_from_parent: n_ne=%lld", (long long)n_ne);
   OCNN_REQUIRE(child_p && neigh_p && nempty_p && (out64 || out32), "neigh_from_parent: a null array");
-  hipLaunchKernelGGL(neigh_from_parent_kernel, dim3(cdiv(n_ne, kParentsPerBlock)), dim3(256), 0,
-                     (hipStream_t)stream, child_p, neigh_p, nempty_p, n_ne, out64, out32);
+  launch_from_parent(child_p, neigh_p, nempty_p, n_ne, out64, out32, (hipStream_t)stream);
   return check_launch("neigh_from_parent");
 }
 
@@ -191,9 +303,46 @@ extern "C" int ocnn_neigh_all(int depth, int full_depth, int batch, const int64_
                  "neigh_all: layers %d and %d are inconsistent", d - 1, d);
     hipLaunchKernelGGL(nempty_index_kernel, dim3((unsigned)cdiv(h_nnum[d - 1], 256)), dim3(256), 0, st,
                        h_children[d - 1], h_nnum[d - 1], h_nempty_index[d - 1], (int64_t*)nullptr);
-    hipLaunchKernelGGL(neigh_from_parent_kernel, dim3((unsigned)cdiv(n_ne, kParentsPerBlock)), dim3(256), 0, st,
-                       h_children[d - 1], h_neigh[d - 1], h_nempty_index[d - 1], n_ne, (int64_t*)nullptr, h_neigh[d]);
+    launch_from_parent(h_children[d - 1], h_neigh[d - 1], h_nempty_index[d - 1], n_ne, nullptr, h_neigh[d], st);
   }
+  return check_launch("neigh_all");
+}
+
+// The same from arrays that already hold the indices of the non-empty nodes (ocnnx_tree_fill).
+extern "C" int ocnnx_neigh_all(int depth, int full_depth, int batch, const int64_t* h_nnum, const int64_t* h_nnum_nempty,
+                               const int64_t* const* h_keys, const int32_t* const* h_children,
+                               const int32_t* const* h_nempty_index, int32_t* const* h_neigh, void* stream) {
+  OCNN_REQUIRE(depth >= 1 && depth <= 16 && full_depth >= 1 && full_depth <= depth && full_depth <= 7 && batch >= 1,
+               "neigh_all: depth=%d full_depth=%d batch=%d out of range", depth, full_depth, batch);
+  OCNN_REQUIRE_PTRS("neigh_all", h_nnum, h_nnum_nempty, h_keys, h_children, h_nempty_index, h_neigh);
+  hipStream_t st = (hipStream_t)stream;
+  WalkTree t;
+  t.full_depth = full_depth;
+  t.batch = batch;
+  t.last = full_depth;
+  for (int d = 0; d <= depth; ++d) {
+    if (d >= 1)
+      OCNN_REQUIRE(h_neigh[d] != nullptr && h_nnum[d] > 0 && h_nnum[d] * 27 < (1ll << 31),
+                   "neigh_all: layer %d: no table, or no nodes, or 2^31 table entries and more", d);
+    if (d <= full_depth)
+      OCNN_REQUIRE(h_nnum[d] == ((int64_t)batch << (3 * d)), "neigh_all: layer %d is not full", d);
+    if (d > full_depth)
+      OCNN_REQUIRE(h_nnum_nempty[d - 1] > 0 && 8 * h_nnum_nempty[d - 1] == h_nnum[d] && h_children[d - 1] && h_keys[d - 1] &&
+                       h_nempty_index[d - 1] && (d == 1 || h_neigh[d - 1]),
+                   "neigh_all: layers %d and %d are inconsistent", d - 1, d);
+    t.keys[d] = h_keys[d];
+    t.children[d] = h_children[d];
+    t.index[d] = h_nempty_index[d];
+    t.neigh[d] = h_neigh[d];
+    t.n_ne[d] = h_nnum_nempty[d];
+    if (d > full_depth && t.last == d - 1 && h_nnum_nempty[d - 1] <= kWalkMaxParents) t.last = d;
+  }
+  t.block0[0] = t.block0[1] = 0;
+  for (int d = 1; d <= t.last; ++d)
+    t.block0[d + 1] = t.block0[d] + (d <= full_depth ? cdiv(h_nnum[d] * 27, 256) : cdiv(h_nnum_nempty[d - 1], kParentsPerBlock));
+  hipLaunchKernelGGL(neigh_walk_kernel, dim3((unsigned)t.block0[t.last + 1]), dim3(256), 0, st, t);
+  for (int d = t.last + 1; d <= depth; ++d)
+    launch_from_parent(h_children[d - 1], h_neigh[d - 1], h_nempty_index[d - 1], h_nnum_nempty[d - 1], nullptr, h_neigh[d], st);
   return check_launch("neigh_all");
 }
 

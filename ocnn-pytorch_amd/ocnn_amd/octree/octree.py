@@ -380,20 +380,33 @@ class Octree:
     self.batch_nnum = torch.zeros(num, bs, dtype=torch.long)
     self.batch_nnum_nempty = torch.zeros(num, bs, dtype=torch.long)
 
-    # the reference's public lookup tables (ocnn/octree/octree.py:85-106); the
-    # kernels compute the first two arithmetically
-    dev = self.device
-    grid = range_grid(2, 3, dev).unsqueeze(1) + range_grid(-1, 1, dev)
-    self.lut_parent = (trunc_div(grid, 2) * torch.tensor([9, 3, 1], device=dev)).sum(2)
-    self.lut_child = ((grid % 2) * torch.tensor([4, 2, 1], device=dev)).sum(2)
-    self.lut_kernel = {k: torch.tensor(v, device=dev) for k, v in LUT_KERNEL.items()}
+    self._luts = None
+
+  # the reference's public lookup tables (ocnn/octree/octree.py:85-106), made when asked for: the
+  # kernels compute the first two arithmetically
+  def _lut(self, which):
+    if self._luts is None:
+      dev = self.device
+      grid = range_grid(2, 3, dev).unsqueeze(1) + range_grid(-1, 1, dev)
+      self._luts = ((trunc_div(grid, 2) * torch.tensor([9, 3, 1], device=dev)).sum(2),
+                    ((grid % 2) * torch.tensor([4, 2, 1], device=dev)).sum(2),
+                    {k: torch.tensor(v, device=dev) for k, v in LUT_KERNEL.items()})
+    return self._luts[which]
+
+  lut_parent = property(lambda self: self._lut(0))
+  lut_child = property(lambda self: self._lut(1))
+  lut_kernel = property(lambda self: self._lut(2))
 
   def __getstate__(self):
     return dict(vars(self), _layers={})        # (native passes are made again when asked for)
 
   # ---- cache bookkeeping ---------------------------------------------------
   def _drop_tables(self, depth, nempty_only=False):
+    """Forgets what was derived from the tables of a layer (None: of every layer)."""
     self._layers.clear()
+    if depth is None:
+      self._tables, self._tables_t, self._plans = {}, {}, {}
+      return
     for cache in (self._tables, self._tables_t):
       for key in [k for k in cache if k[0] == depth and (k[3] or not nempty_only)]:
         del cache[key]
@@ -470,9 +483,7 @@ class Octree:
     assert point_cloud.batch_size == self.batch_size, 'Inconsistent batch_size'
     pts = point_cloud.points
     _lib.require_gpu(pts)
-    L = _lib.lib()
-    dev = pts.device
-    depth = self.depth
+    dev, depth = pts.device, self.depth
 
     # normalisation constants exactly as Points.normalize forms them
     box = bbmax - bbmin
@@ -485,84 +496,25 @@ class Octree:
       lo = lo * 3 if len(lo) == 1 else lo
     else:
       lo = [float(bbmin)] * 3
-    h_lo = (ctypes.c_float * 3)(*lo)
-
-    pts = pts.float().contiguous()
-    npt = pts.shape[0]
-    batch, batch_is_float = None, 0
-    if self.batch_size > 1:
-      batch = point_cloud.batch_id.view(-1)
-      if batch.is_floating_point():
-        batch, batch_is_float = batch.float().contiguous(), 1
-      else:
-        batch = batch.long().contiguous()
-    pts_norm = torch.empty_like(pts)
-    key = torch.empty(npt, dtype=torch.long, device=dev)
-    st = _lib.stream()
-    _lib.check(L.ocnn_points2key(_lib.ptr(pts), npt, h_lo, factor, _lib.ptr(batch),
-                                 batch_is_float, depth, _lib.ptr(pts_norm), _lib.ptr(key), st))
-
-    # sort, then every layer's node numbering in one scan: one read-back for the whole build
-    full_depth = self.full_depth
-    levels = depth - full_depth
-    batch_bits = max(0, (self.batch_size - 1).bit_length())
-    ws = _lib.workspace(L.ocnn_octree_build_workspace_bytes(npt, depth, full_depth, batch_bits), dev)
-    perm = torch.empty(npt, dtype=torch.int32, device=dev)
-    sizes = torch.empty(levels + 1, dtype=torch.long, device=dev)
-    _lib.check(L.ocnn_octree_build_scan(_lib.ptr(key), npt, depth, full_depth, batch_bits,
-                                        _lib.ptr(ws), ws.numel(), _lib.ptr(perm), _lib.ptr(sizes),
-                                        st))
-    # what does not wait for the sizes is allocated while the sort runs
-    full = [self.batch_size << (3 * d) for d in range(full_depth + 1)]
-    for d in range(full_depth + 1):
-      self.keys[d] = torch.empty(full[d], dtype=torch.long, device=dev)
-      self.children[d] = torch.empty(full[d], dtype=torch.int32, device=dev)
-    idx = torch.empty(npt, dtype=torch.long, device=dev)
-    seg_start = torch.empty(npt + 1, dtype=torch.int32, device=dev)
-    sizes = sizes.tolist()
-    nleaf = sizes[0]
-
-    nnum = full + [8 * sizes[depth - d + 1] for d in range(full_depth + 1, depth + 1)]
-    for d in range(full_depth + 1, depth + 1):
-      self.keys[d] = torch.empty(nnum[d], dtype=torch.long, device=dev)
-      self.children[d] = torch.empty(nnum[d], dtype=torch.int32, device=dev)
-    h_sizes = (ctypes.c_int64 * (levels + 1))(*sizes)
-    h_keys = (ctypes.c_void_p * (depth + 1))(*[t.data_ptr() for t in self.keys[:depth + 1]])
-    h_children = (ctypes.c_void_p * (depth + 1))(*[t.data_ptr() for t in self.children[:depth + 1]])
-    _lib.check(L.ocnn_octree_build_fill(_lib.ptr(ws), npt, depth, full_depth, self.batch_size,
-                                        batch_bits, h_sizes, _lib.ptr(perm), h_keys, h_children,
-                                        _lib.ptr(idx), _lib.ptr(seg_start), st))
-
-    # per-leaf signals
-    def leaf(src, mode):
-      src = src.float().contiguous()
-      out = torch.empty(nleaf, src.shape[1], dtype=torch.float32, device=dev)
-      _lib.check(L.ocnn_leaf_average(_lib.ptr(src), src.shape[1], _lib.ptr(perm),
-                                     _lib.ptr(seg_start), nleaf, mode, _lib.ptr(out), st))
-      return out
-
-    self.nnum[:depth + 1] = torch.tensor(nnum, dtype=torch.long)
-    self.nnum_nempty[:depth + 1] = torch.tensor(
-        full[:-1] + [sizes[depth - d] for d in range(full_depth, depth + 1)], dtype=torch.long)
-    if point_cloud.normals is not None:
-      nrm = point_cloud.normals.float().contiguous()
-      self.points[depth] = torch.empty(nleaf, 3, dtype=torch.float32, device=dev)
-      self.normals[depth] = torch.empty(nleaf, 3, dtype=torch.float32, device=dev)
-      _lib.check(L.ocnn_leaf_points_normals(_lib.ptr(pts_norm), _lib.ptr(nrm), _lib.ptr(perm), _lib.ptr(seg_start),
-                                            nleaf, _lib.ptr(self.points[depth]), _lib.ptr(self.normals[depth]), st))
-    else:
-      self.points[depth] = leaf(pts_norm, 0)
-    if point_cloud.features is not None:
-      self.features[depth] = leaf(point_cloud.features, 0)
-
+    tree = _lib.native().build_octree(pts, point_cloud.normals, point_cloud.batch_id if self.batch_size > 1 else None,
+                                      lo, factor, depth, self.full_depth, self.batch_size)
     num = depth + 1
+    self.keys, self.children = tree.keys, tree.children
+    self.nnum, self.nnum_nempty = torch.tensor(tree.nnum), torch.tensor(tree.nnum_nempty)
+    self.points[depth], self.normals[depth] = tree.points, tree.normals
+    if point_cloud.features is not None:               # per-leaf averages
+      src = point_cloud.features.float().contiguous()
+      leaves = tree.points.shape[0]
+      self.features[depth] = torch.empty(leaves, src.shape[1], dtype=torch.float32, device=dev)
+      _lib.check(_lib.lib().ocnn_leaf_average(_lib.ptr(src), src.shape[1], _lib.ptr(tree.perm), _lib.ptr(tree.seg_start),
+                                              leaves, 0, _lib.ptr(self.features[depth]), _lib.stream()))
     self.nempty_masks = [None] * num
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
-    self._nempty_indices32 = [None] * num
+    self._nempty_indices32 = tree.index
     self._tables, self._tables_t, self._plans, self._layers = {}, {}, {}, {}
     self._plans_prebuilt = False
-    return idx
+    return tree.idx
 
   def _grow_full(self, depth: int, with_children: bool = True):
     num = self.batch_size << (3 * depth)
@@ -671,29 +623,22 @@ class Octree:
     depth = self.depth
     nnum = [int(v) for v in self.nnum[:depth + 1].tolist()]
     nempty = [int(v) for v in self.nnum_nempty[:depth + 1].tolist()]
-    if dev.type != 'cuda' or self.full_depth < 1 or any(c is None for c in self.children[:depth + 1]) or \
+    if dev.type != 'cuda' or self.full_depth < 1 or \
+        any(c is None for c in self.children[:depth + 1] + self.keys[:depth + 1]) or \
         min(nnum[1:] + nempty) <= 0 or \
         any(nnum[d] != (self.batch_size << (3 * d) if d <= self.full_depth else 8 * nempty[d - 1])
             for d in range(1, depth + 1)):
       for d in range(1, depth + 1):                       # the layer-by-layer route says what is wrong
         self.construct_neigh(d)
       return
-    neigh = [None] + [torch.empty(nnum[d], 27, dtype=torch.int32, device=dev) for d in range(1, depth + 1)]
-    index = [torch.empty(nempty[d], dtype=torch.int32, device=dev) if self.full_depth <= d < depth else None
-             for d in range(depth + 1)]
-    ptrs = lambda ts: (ctypes.c_void_p * (depth + 1))(*[None if t is None else t.data_ptr() for t in ts])
+    index = [self._nempty_index32(d) if self.full_depth <= d < depth else None for d in range(depth + 1)]
     with torch.cuda.device(dev):
-      _lib.check(_lib.lib().ocnn_neigh_all(depth, self.full_depth, self.batch_size,
-                                           (ctypes.c_int64 * (depth + 1))(*nnum),
-                                           (ctypes.c_int64 * (depth + 1))(*nempty), ptrs(self.children[:depth + 1]),
-                                           ptrs(index), ptrs(neigh), _lib.stream()))
-    for d in range(1, depth + 1):
-      self.neighs[d] = neigh[d]
+      tables = _lib.native().all_neigh(self.keys[:depth + 1], self.children[:depth + 1], index, nnum, nempty,
+                                       self.full_depth, self.batch_size)
+    for d, table in enumerate(tables, 1):
+      self.neighs[d] = table
       self.nempty_neighs[d] = None
-      self._drop_tables(d)
-    for d in range(self.full_depth, depth):
-      self._nempty_indices32[d] = index[d]
-      self.nempty_indices[d] = None
+    self._drop_tables(None)
 
   # ---- search (ocnn/octree/octree.py:448-488) -------------------------------
   def search_xyzb(self, query: torch.Tensor, depth: int, nempty: bool = False):

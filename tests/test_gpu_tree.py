@@ -1,0 +1,46 @@
+"""Octree builds at the edges of the sort's ranges: points around a span, one to three digits, counts read
+in place or scanned, keys of more than 32 bits; and the tables of octrees whose layers are found by
+walking and from their parents."""
+
+import numpy as np
+import pytest
+import torch
+
+from ocnn_amd.octree import Octree, Points
+from oracle import octree_ref as R
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('n,depth,full_depth,batch', [(1, 3, 1, 1), (2047, 3, 2, 1), (2049, 6, 2, 3), (32768, 7, 2, 1),
+                                                      (32769, 6, 3, 5), (131072, 9, 2, 8), (131073, 8, 2, 1), (5000, 11, 2, 2),
+                                                      (300001, 8, 2, 4)])
+def test_build_and_tables(n, depth, full_depth, batch):
+  print('octree', n, depth, full_depth, batch, flush=True)
+  g = torch.Generator().manual_seed(n)
+  pts = torch.rand(n, 3, generator=g) * 1.98 - 0.99
+  pts[:, 2] = 0.3 * pts[:, 0] * pts[:, 1]                 # a surface
+  nrm = torch.randn(n, 3, generator=g)
+  bid = torch.randint(0, batch, (n, 1), generator=g).float()
+  bid[0], bid[-1] = 0, batch - 1
+  o = Octree(depth, full_depth, batch_size=batch)
+  idx = o.build_octree(Points(pts.cuda(), nrm.cuda(), batch_id=bid.cuda() if batch > 1 else None, batch_size=batch))
+  o.construct_all_neigh()
+  ref, want_idx = R.build_octree(pts.numpy(), nrm.numpy(), batch_id=bid.numpy() if batch > 1 else None, depth=depth,
+                                 full_depth=full_depth, batch_size=batch)
+  assert np.array_equal(idx.cpu().numpy(), want_idx)
+  for d in range(depth + 1):
+    assert np.array_equal(o.keys[d].cpu().numpy(), ref.keys[d]), d
+    assert np.array_equal(o.children[d].cpu().numpy(), ref.children[d]), d
+    assert int(o.nnum[d]) == ref.keys[d].shape[0]
+    if d >= full_depth:
+      assert np.array_equal(o._nempty_index32(d).cpu().numpy(), np.nonzero(ref.children[d] >= 0)[0]), d
+  assert np.abs(o.points[depth].cpu().numpy() - ref.points[depth]).max() < 1e-4 * 2 ** depth
+  again = Octree(depth, full_depth, batch_size=batch)
+  again.build_octree(Points(pts.cuda(), nrm.cuda(), batch_id=bid.cuda() if batch > 1 else None, batch_size=batch))
+  assert torch.equal(again.points[depth], o.points[depth]) and torch.equal(again.normals[depth], o.normals[depth])
+  layer = Octree(depth, full_depth, batch_size=batch)       # the tables layer by layer, from the parents' alone
+  layer.build_octree(Points(pts.cuda(), nrm.cuda(), batch_id=bid.cuda() if batch > 1 else None, batch_size=batch))
+  for d in range(1, depth + 1):
+    layer.construct_neigh(d)
+    assert torch.equal(layer.neighs.get32(d), o.neighs.get32(d)), d
