@@ -92,6 +92,55 @@ __global__ __launch_bounds__(256) void pack_weights_tile_kernel(const I* __restr
   }
 }
 
+// N consecutive values of a per-channel array (f32 / f16 / bf16; null: dflt), N a multiple of 4
+template <int N>
+__device__ __forceinline__ void load_channels(const void* p, int dtype, int c0, float dflt, float (&v)[N]) {
+  if (!p) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = dflt;
+  } else if (dtype == OCNN_F32) {
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+      const f32x4 q = *(const f32x4*)((const float*)p + c0 + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[i + j] = q[j];
+    }
+  } else {
+    unsigned short r[N];
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+      const u32x2 q = *(const u32x2*)((const unsigned short*)p + c0 + i);
+      r[i] = (unsigned short)q[0], r[i + 1] = (unsigned short)(q[0] >> 16);
+      r[i + 2] = (unsigned short)q[1], r[i + 3] = (unsigned short)(q[1] >> 16);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      v[i] = dtype == OCNN_F16 ? to_f32(__builtin_bit_cast(f16, r[i])) : __uint_as_float((uint32_t)r[i] << 16);
+  }
+}
+
+// What is added to N channels of a row's sums and what they are multiplied with: bias alone, or the batch
+// norm behind the layer with its running statistics, ((sum + bias) - mean) * sc + beta = sum * sc + sh.
+template <typename O, int N>
+__device__ __forceinline__ void layer_tail(const O* bias, const ocnnx_bn& bn, int c0, float (&sc)[N], float (&sh)[N]) {
+  load_channels<N>(bias, std::is_same<O, float>::value ? OCNN_F32 : (std::is_same<O, f16>::value ? OCNN_F16 : OCNN_BF16), c0,
+                   0.f, sh);
+#pragma unroll
+  for (int i = 0; i < N; ++i) sc[i] = 1.f;
+  if (bn.mean) {
+    float m[N], be[N], ga[N];
+    load_channels<N>(bn.var, bn.stat_dtype, c0, 1.f, sc);
+    load_channels<N>(bn.mean, bn.stat_dtype, c0, 0.f, m);
+    load_channels<N>(bn.gamma, bn.param_dtype, c0, 1.f, ga);
+    load_channels<N>(bn.beta, bn.param_dtype, c0, 0.f, be);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      sc[i] = ga[i] / sqrtf(sc[i] + bn.eps);
+      sh[i] = (sh[i] - m[i]) * sc[i] + be[i];
+    }
+  }
+}
+
 // SKIP: per slot and 32-row block of the tile a wave asks whether any row has an entry there (a
 // ballot over the positions it reads anyway) and leaves the block's MFMAs out otherwise.  The
 // kernel is bound by the power its MFMAs draw (also those on zero rows), and the branches cost
@@ -103,8 +152,8 @@ template <typename T, bool F32, int MB, int WR, bool SKIP>
 __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
     const void* __restrict__ in, uint32_t in_bytes, const uint16_t* __restrict__ loc,
     const int32_t* __restrict__ uptr, const int32_t* __restrict__ urows, const T* __restrict__ wpk,
-    const void* __restrict__ bias_, void* __restrict__ out_, float* __restrict__ partial, int64_t rows_out, int K,
-    int cin, int cout, int64_t tiles, int64_t tiles_per_xcd, int sc, int sk) {
+    const void* __restrict__ bias_, ocnnx_bn bn, void* __restrict__ out_, float* __restrict__ partial,
+    int64_t rows_out, int K, int cin, int cout, int64_t tiles, int64_t tiles_per_xcd, int sc, int sk) {
   typedef typename std::conditional<F32, float, T>::type O;
   constexpr int RB = 4 / WR, WC = 4 / WR, CH = F32 ? 32 : 64;
   __shared__ __attribute__((aligned(16))) char s_rows[kTgRowsAlloc * 128];
@@ -342,28 +391,48 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
   }
 
   // ---- epilogue: a lane holds 16 consecutive output channels of a row per M tile ----
-  const O* bias = (const O*)bias_;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     if (cg0 + mb >= ncg) continue;
     const int co = 32 * (cg0 + mb) + 16 * q;
-    float bv[16];
+    if (partial) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) bv[r] = bias && !partial ? to_f32(bias[co + r]) : 0.f;
+      for (int rb = 0; rb < RB; ++rb) {
+        const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
+        if (row >= rows_out) continue;
+        float* dst = partial + ((int64_t)blockIdx.z * rows_out + row) * cout + co;
+#pragma unroll
+        for (int r = 0; r < 16; r += 4)
+          *(f32x4*)(dst + r) = f32x4{acc[rb][mb][r], acc[rb][mb][r + 1], acc[rb][mb][r + 2], acc[rb][mb][r + 3]};
+      }
+      continue;
+    }
+    float mul[16], add[16];
+    layer_tail<O, 16>((const O*)bias_, bn, co, mul, add);
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
       if (row >= rows_out) continue;
-      if (F32 || partial) {
-        float* dst = (partial ? partial + (int64_t)blockIdx.z * rows_out * cout : (float*)out_) + row * cout + co;
+      float v[16];
 #pragma unroll
-        for (int r = 0; r < 16; r += 4)
-          *(f32x4*)(dst + r) = f32x4{acc[rb][mb][r] + bv[r], acc[rb][mb][r + 1] + bv[r + 1],
-                                     acc[rb][mb][r + 2] + bv[r + 2], acc[rb][mb][r + 3] + bv[r + 3]};
+      for (int r = 0; r < 16; ++r) v[r] = acc[rb][mb][r] * mul[r] + add[r];
+      if (bn.residual) {
+        const O* res = (const O*)bn.residual + row * cout + co;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] += to_f32(res[r]);
+      }
+      if (bn.relu) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = fmaxf(v[r], 0.f);
+      }
+      if constexpr (F32) {
+        float* dst = (float*)out_ + row * cout + co;
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) *(f32x4*)(dst + r) = f32x4{v[r], v[r + 1], v[r + 2], v[r + 3]};
       } else {
         unsigned pk[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) pk[r] = pack2<T>(acc[rb][mb][2 * r] + bv[2 * r], acc[rb][mb][2 * r + 1] + bv[2 * r + 1]);
+        for (int r = 0; r < 8; ++r) pk[r] = pack2<T>(v[2 * r], v[2 * r + 1]);
         T* dst = (T*)out_ + row * cout + co;
         *(u32x4*)(dst) = u32x4{pk[0], pk[1], pk[2], pk[3]};
         *(u32x4*)(dst + 8) = u32x4{pk[4], pk[5], pk[6], pk[7]};
@@ -372,10 +441,10 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
   }
 }
 
-// out = sum of the parts, in their order, (+ bias); four consecutive values a thread
+// out = sum of the parts, in their order, and what follows (layer_tail); four consecutive values a thread
 template <typename O>
 __global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict__ partial, int parts, int64_t n, int cout,
-                                                         const O* __restrict__ bias, O* __restrict__ out) {
+                                                         const O* __restrict__ bias, ocnnx_bn bn, O* __restrict__ out) {
   const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (e >= n) return;
   f32x4 acc = *(const f32x4*)(partial + e);
@@ -388,10 +457,14 @@ __global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict
     for (int u = 0; u < 4; ++u) acc += v[u];
   }
   for (; s < parts; ++s) acc += *(const f32x4*)(partial + s * n + e);
-  const int c = (int)(e % cout);
-  if (bias)
+  float mul[4], add[4];
+  layer_tail<O, 4>(bias, bn, (int)(e % cout), mul, add);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] += to_f32(bias[c + i]);
+  for (int i = 0; i < 4; ++i) {
+    acc[i] = acc[i] * mul[i] + add[i];
+    if (bn.residual) acc[i] += to_f32(((const O*)bn.residual)[e + i]);
+    if (bn.relu) acc[i] = fmaxf(acc[i], 0.f);
+  }
   typedef __attribute__((ext_vector_type(4))) O o4;
   o4 o;
 #pragma unroll
@@ -461,8 +534,8 @@ extern "C" int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out
 template <typename T, bool F32>
 static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr, const int32_t* urows,
                     int64_t rows_out, int K, int cin, int cout, const void* w, int w_transposed, int reverse,
-                    const void* bias, void* out, void* ws, int64_t ws_bytes, bool skip, int split_c, int split_k,
-                    hipStream_t st) {
+                    const void* bias, const ocnnx_bn& bn, void* out, void* ws, int64_t ws_bytes, bool skip, int split_c,
+                    int split_k, hipStream_t st) {
   typedef typename std::conditional<F32, float, T>::type O;
   const int dtype = F32 ? OCNN_F32 : OCNN_F16;
   const int64_t lanes = cdiv(cin, F32 ? 32 : 64) * (int64_t)K * (cout / 32) * (F32 ? 2 : 4) * 64;
@@ -484,7 +557,7 @@ static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const 
   const uint32_t in_bytes = (uint32_t)(rows_in * cin * sizeof(O));
 #define OCNN_TILE_LAUNCH(MB_, WR_, SKIP_)                                                                           \
   hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WR_, SKIP_>), grid, dim3(256), 0, st, in, in_bytes, loc, \
-                     uptr, urows, (const T*)ws, bias, out, partial, rows_out, K, cin, cout, tiles, per_xcd, t.sc, t.sk)
+                     uptr, urows, (const T*)ws, bias, bn, out, partial, rows_out, K, cin, cout, tiles, per_xcd, t.sc, t.sk)
 #define OCNN_TILE_CASE(MB_, WR_)           \
   if (t.mb == MB_ && t.wr == WR_) {        \
     if (skip) OCNN_TILE_LAUNCH(MB_, WR_, true); \
@@ -498,15 +571,15 @@ static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const 
 #undef OCNN_TILE_LAUNCH
   if (partial)
     hipLaunchKernelGGL(tile_parts_kernel<O>, dim3((unsigned)cdiv(rows_out * cout / 4, 256)), dim3(256), 0, st, partial,
-                       parts, rows_out * cout, cout, (const O*)bias, (O*)out);
+                       parts, rows_out * cout, cout, (const O*)bias, bn, (O*)out);
   return check_launch("conv_gather_tile");
 }
 
 extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
                                  const int32_t* urows, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
                                  int64_t rows_out, int K, const void* w, int cin, int cout, int w_transposed,
-                                 int reverse_slots, const void* bias, void* out, void* workspace, int64_t workspace_bytes,
-                                 int split_c, int split_k, void* stream) {
+                                 int reverse_slots, const void* bias, const ocnnx_bn* bn_or_null, void* out,
+                                 void* workspace, int64_t workspace_bytes, int split_c, int split_k, void* stream) {
   OCNN_REQUIRE(ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct),
                "conv_gather_tile: shape not supported");
   OCNN_REQUIRE(rows_out >= 0 && rows_out < (1ll << 31) && plan_total >= 0 && plan_total < (1ll << 29),
@@ -519,16 +592,18 @@ extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, con
     return OCNN_ERR_WORKSPACE;
   }
   hipStream_t st = (hipStream_t)stream;
+  ocnnx_bn bn = {};
+  if (bn_or_null) bn = *bn_or_null;
   // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
   const bool skip = K != 8 && plan_occupancy >= 0.0 && plan_occupancy <= kTgSkipMaxOccupancy;
   if (dtype == OCNN_F32)
     return run_tile<bf16, true>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
-                                bias, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+                                bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
   if (dtype == OCNN_F16)
     return run_tile<f16, false>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
-                                bias, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+                                bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
   return run_tile<bf16, false>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
-                               bias, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+                               bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
 }
 
 // The public entry point: 16-bit wide layers, with whatever room for parts the workspace has.
@@ -548,6 +623,6 @@ extern "C" int ocnn_conv_gather_wide(int dtype, const void* in, int64_t rows_in,
   OCNN_REQUIRE(ocnn_conv_gather_wide_supported(dtype, rows_in, K, cin, cout, plan_max_distinct),
                "conv_gather_wide: shape not supported");
   return ocnnx_gather_tile(dtype, in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out,
-                           K, w, cin, cout, w_transposed, reverse_slots, bias, out, workspace, workspace_bytes, 0, 0,
+                           K, w, cin, cout, w_transposed, reverse_slots, bias, nullptr, out, workspace, workspace_bytes, 0, 0,
                            stream);
 }

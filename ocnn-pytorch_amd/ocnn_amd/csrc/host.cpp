@@ -82,7 +82,9 @@ struct GatherOp {
   int bias_repeat = 1, view_cols = 0;         // dense form: bias once per child; result seen with this many columns
   std::shared_ptr<GatherOp> overflow, padded; // padded: this pass with channels in whole multiples (zero-padded)
 
-  Tensor run(Tensor data, Tensor table, Tensor W, OptTensor bias) const {
+  // bn: a batch norm with running statistics that follows the layer; in the same pass where the kernel
+  // has room for it, in place after it otherwise
+  Tensor run(Tensor data, Tensor table, Tensor W, OptTensor bias, const ocnnx_bn* bn = nullptr) const {
     require_gpu(data);
     require_gpu(W);
     const int code = code_of(data.scalar_type());
@@ -94,7 +96,7 @@ struct GatherOp {
       bias = bias->to(data.scalar_type()).contiguous();
       if (bias_repeat > 1) bias = bias->repeat({bias_repeat});
     }
-    if (padded) return run_padded(data, table, W, bias);
+    if (padded) return followed(run_padded(data, table, W, bias), bn);
     void* st = hip_stream();
     const bool wide_out = kernel == OCNN_GATHER_DENSE_RW && out_index.defined();
     Tensor out = at::empty({wide_out ? rows_all : rows, cout}, data.options());
@@ -122,7 +124,9 @@ struct GatherOp {
       case OCNNX_GATHER_TILE:
         check(ocnnx_gather_tile(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
                                 typed<int32_t>(p->urows), p->umax, p->total, p->occupancy, rows, K, ptr(W), cin, cout,
-                                transposed, reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), 0, 0, st));
+                                transposed, reverse, ptr(bias), overflow ? nullptr : bn, out.data_ptr(), ws.data_ptr(),
+                                ws.numel(), 0, 0, st));
+        if (!overflow) bn = nullptr;
         break;
       case OCNN_GATHER_SPARSE:
         check(ocnn_conv_gather_sparse(code, ptr(data), rows_in, typed<int32_t>(p->uptr), typed<int32_t>(p->urows),
@@ -145,10 +149,17 @@ struct GatherOp {
                                reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
     }
     if (overflow) out.index_copy_(0, overflow_rows, overflow->run(data, overflow_table, W, bias));
-    return view_cols ? out.view({-1, view_cols}) : out;
+    return followed(view_cols ? out.view({-1, view_cols}) : out, bn);
   }
 
  private:
+  static Tensor followed(const Tensor& out, const ocnnx_bn* bn) {
+    if (bn && out.size(0))
+      check(ocnnx_batch_norm_running(code_of(out.scalar_type()), out.data_ptr(), out.size(0), (int)out.size(1), bn->mean,
+                                     bn->var, bn->stat_dtype, bn->eps, bn->gamma, bn->beta, bn->param_dtype, bn->relu,
+                                     bn->residual, out.data_ptr(), hip_stream()));
+    return out;
+  }
   Tensor run_padded(const Tensor& data, const Tensor& table, const Tensor& W, const OptTensor& bias) const {
     const int pi = padded->cin - cin, po = padded->cout - cout;
     Tensor Wk = transposed ? W.view({K, cout, cin}) : W.view({K, cin, cout});
@@ -446,6 +457,37 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
   return y;
 }
 
+// A layer and the batch norm (+ residual, + ReLU) behind it, in evaluation and without gradients: the
+// normalisation rides on the convolution's own pass over its result where the kernel takes it.
+Tensor conv_bn(const std::shared_ptr<ConvLayer>& layer, const Tensor& data_in, const Tensor& weights, const OptTensor& bias,
+               const Tensor& running_mean, const Tensor& running_var, double eps, const OptTensor& gamma_in,
+               const OptTensor& beta_in, bool relu, const OptTensor& residual_in) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor data = data_in.contiguous(), w = weights.to(data.scalar_type()).contiguous();
+  const int cols = layer->fwd->view_cols ? layer->fwd->view_cols : layer->fwd->cout;
+  TORCH_CHECK(running_mean.numel() == cols && running_var.numel() == cols,
+              "running statistics of ", running_mean.numel(), " channels for a layer of ", cols);
+  Tensor mean = running_mean, var = running_var;
+  if (!known_type(mean) || mean.scalar_type() != var.scalar_type()) {
+    mean = mean.to(at::kFloat);
+    var = var.to(at::kFloat);
+  }
+  mean = mean.contiguous();
+  var = var.contiguous();
+  Tensor gamma = as_param(gamma_in.has_value() ? *gamma_in : Tensor()), beta = as_param(beta_in.has_value() ? *beta_in : Tensor());
+  if (gamma.defined() && beta.defined() && beta.scalar_type() != gamma.scalar_type()) beta = beta.to(gamma.scalar_type());
+  Tensor residual;
+  if (residual_in.has_value()) {
+    residual = residual_in->contiguous();
+    TORCH_CHECK(residual.scalar_type() == data.scalar_type() && residual.dim() == 2 &&
+                    residual.size(0) == layer->fwd->rows && residual.size(1) == running_mean.numel(),
+                "conv_bn: the residual does not match the layer");
+  }
+  const ocnnx_bn bn{mean.data_ptr(), var.data_ptr(), code_of(mean.scalar_type()), (float)eps,
+                    ptr(gamma), ptr(beta), param_code(gamma, beta), relu, ptr(residual)};
+  return layer->fwd->run(data, layer->fwd_table, w, bias, &bn);
+}
+
 // ---- octree (octree/octree.py) ----------------------------------------------------------------
 
 struct Tree {
@@ -607,6 +649,7 @@ PYBIND11_MODULE(ocnn_host, m) {
   m.def("all_neigh", &all_neigh, py::call_guard<py::gil_scoped_release>());
   m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;
   m.def("conv", &conv, py::call_guard<py::gil_scoped_release>());
+  m.def("conv_bn", &conv_bn, py::call_guard<py::gil_scoped_release>());
   m.def("column_sum", &column_sum, py::call_guard<py::gil_scoped_release>());
   m.def(
       "batch_norm",

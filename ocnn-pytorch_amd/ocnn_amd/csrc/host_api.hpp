@@ -9,6 +9,18 @@
 extern "C" {
 #endif
 
+// What follows a layer in evaluation, taken in the same pass: y = (x - mean) / sqrt(var + eps) * gamma + beta
+// (+ residual), then max(., 0) with relu.  mean null: nothing follows.  Statistics and parameters in
+// f32 / f16 / bf16 (gamma, beta, residual may be null).
+typedef struct {
+  const void *mean, *var;
+  int stat_dtype;
+  float eps;
+  const void *gamma, *beta;
+  int param_dtype, relu;
+  const void* residual;
+} ocnnx_bn;
+
 // Gather-GEMM on the tile plan, any of the three data types, channels in multiples of 32
 // (conv_tile.hip).  The workspace holds the packed weights and, where a launch of few tiles splits
 // its reduction, the parts' sums; with less room than ..._workspace_bytes() (but the packed
@@ -19,8 +31,8 @@ int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out, int K, in
 int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
                       const int32_t* urows, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
                       int64_t rows_out, int K, const void* w, int cin, int cout, int w_transposed, int reverse_slots,
-                      const void* bias, void* out, void* workspace, int64_t workspace_bytes, int split_c, int split_k,
-                      void* stream);
+                      const void* bias, const ocnnx_bn* bn, void* out, void* workspace, int64_t workspace_bytes,
+                      int split_c, int split_k, void* stream);
 
 // ocnn_conv_gather_choose with that kernel among the choices.
 #define OCNNX_GATHER_TILE 8

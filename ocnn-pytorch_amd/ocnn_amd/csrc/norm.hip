@@ -208,11 +208,7 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
   if (rl >= rpp) return;
   float m[VEC], sc[VEC], be[VEC];
   if (run_var) {
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) {
-      m[v] = bn_param(run_mean, rdtype, cl * VEC + v, 0.f);
-      sc[v] = bn_param(run_var, rdtype, cl * VEC + v, 0.f);
-    }
+    bn_params<VEC>(run_var, run_mean, rdtype, cl * VEC, sc, m);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) sc[v] = 1.f / sqrtf(sc[v] + eps);
   } else {

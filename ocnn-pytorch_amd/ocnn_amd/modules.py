@@ -27,7 +27,29 @@ class _LayerBn(torch.nn.Module):
       self.relu = torch.nn.ReLU(inplace=True)               # (kept for the module tree; applied by bn)
 
   def forward(self, data, *args):
-    return self.bn(getattr(self, self._name)(data, *args))
+    return layer_bn(getattr(self, self._name), self.bn, data, *args)
+
+
+def _hooked(*modules):
+  return (torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks or
+          any(m._forward_hooks or m._forward_pre_hooks for m in modules))
+
+
+def layer_bn(layer, bn, data, *args, residual=None, relu=None):
+  """bn(layer(data, *args), residual, relu).  In evaluation without gradients, with the layer and the
+  batch norm of this package as they are, one native call: the normalisation then rides on the
+  convolution's own pass over its result instead of reading and writing it once more."""
+  if (not torch.is_grad_enabled() and type(bn) is BatchNormRelu1d and not bn.training and
+      bn.running_mean is not None and type(layer) in (OctreeConv, OctreeDeconv, Conv1x1) and not _hooked(layer, bn)):
+    native = layer.native_layer(data, *args)
+    if native is not None and _lib.lib().ocnn_batch_norm_supported(_lib.DTYPE_CODE[data.dtype], 2, bn.num_features):
+      linear = layer.linear if type(layer) is Conv1x1 else None
+      return _lib.native().conv_bn(native, data, layer.weights if linear is None else linear.weight,
+                                   layer.bias if linear is None else linear.bias, bn.running_mean, bn.running_var, bn.eps,
+                                   bn.weight, bn.bias, bn.fused_relu if relu is None else relu, residual)
+  if residual is None and relu is None:
+    return bn(layer(data, *args))
+  return bn(layer(data, *args), residual=residual, relu=relu)
 
 
 class OctreeConvBn(_LayerBn):
@@ -73,10 +95,10 @@ def _identity_table(rows, device):
 _LINEAR = {}
 
 
-def _rows_linear(x, weight, bias):
-  """y = x W^T + b on many rows through the one-slot form of the convolution kernels
-  (weights (out, in) as torch.nn.Linear holds them)."""
-  rows, cin, cout = x.shape[0], weight.shape[1], weight.shape[0]
+def _rows_linear_layer(x, cin, cout):
+  """y = x W^T on many rows as the one-slot form of the convolution kernels (weights (out, in) as
+  torch.nn.Linear holds them)."""
+  rows = x.shape[0]
   key = (rows, cin, cout, x.dtype, x.device)
   layer = _LINEAR.get(key)
   if layer is None:
@@ -87,7 +109,7 @@ def _rows_linear(x, weight, bias):
     layer.dgrad = _gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True)
     layer.wgrad = _wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin])
     layer.fwd_table = layer.dgrad_table = layer.wgrad_table = _identity_table(rows, x.device)
-  return _lib.native().conv(layer, x, weight, bias)
+  return layer
 
 
 class _RowsLinearNarrow(torch.autograd.Function):
@@ -127,11 +149,19 @@ class Conv1x1(torch.nn.Module):
     super().__init__()
     self.linear = torch.nn.Linear(in_channels, out_channels, use_bias)
 
-  def forward(self, data: torch.Tensor):
+  def native_layer(self, data: torch.Tensor):
+    """The passes on this package's kernels, or None for the library's."""
     lin = self.linear
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 4096 and lin.in_features % 32 == 0 and lin.out_features % 16 == 0):
-      return _rows_linear(data, lin.weight, lin.bias)
+      return _rows_linear_layer(data, lin.in_features, lin.out_features)
+    return None
+
+  def forward(self, data: torch.Tensor):
+    lin = self.linear
+    native = self.native_layer(data)
+    if native is not None:
+      return _lib.native().conv(native, data, lin.weight, lin.bias)
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 65536 and lin.in_features % 32 == 0 and lin.out_features < 16):
       return _RowsLinearNarrow.apply(data, lin.weight, lin.bias)
@@ -168,11 +198,11 @@ class OctreeResBlock2(torch.nn.Module):
     self.relu = torch.nn.ReLU(inplace=True)
 
   def forward(self, data: torch.Tensor, octree, depth: int):
-    out = self.conv3x3b.conv(self.conv3x3a(data, octree, depth), octree, depth)
+    out = self.conv3x3a(data, octree, depth)
     if self.in_channels != self.out_channels:
       data = self.conv1x1(data)
-    # relu(bn(out) + data): the sum and the ReLU ride on the batch norm's pass over `out`
-    return self.conv3x3b.bn(out, residual=data, relu=True)
+    # relu(bn(conv(out)) + data): the sum and the ReLU ride on the batch norm's pass
+    return layer_bn(self.conv3x3b.conv, self.conv3x3b.bn, out, octree, depth, residual=data, relu=True)
 
 
 class OctreeResBlocks(torch.nn.Module):

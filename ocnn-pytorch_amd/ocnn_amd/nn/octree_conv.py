@@ -657,40 +657,50 @@ class _Layer:
       self.native.wgrad, self.native.wgrad_table = made
 
 
+def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
+  """The layer's native passes, made at its first call on this octree and kept with it: (layer or
+  None where the forward pass is not one native pass, function that makes its engine)."""
+  if not (isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE):
+    return None, None
+  key = (engine, depth, tuple(kernel_size), stride, nempty, in_channels, out_channels, data.dtype, padded,
+         SPARSE_MIN_ROWS)
+  layer = octree._layers.get(key)
+
+  def made_engine():
+    eng = engine(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
+    eng.setup(octree, depth)
+    return eng
+
+  if layer is None:
+    layer = octree._layers[key] = _Layer(made_engine(), data.dtype, padded)
+  if not layer.ok:
+    return None, None
+  assert data.shape == layer.shape, \
+      'The shape of input data is wrong: expected {}, got {}.'.format(layer.shape, tuple(data.shape))
+  return layer, made_engine
+
+
 def _apply(engine, function, data, weights, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
            max_buffer, bias, padded):
-  """The layer through the native node where each of its passes is one (kept with the octree),
-  through `function` otherwise."""
-  if isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE:
-    key = (engine, depth, tuple(kernel_size), stride, nempty, in_channels, out_channels, data.dtype, padded,
-           SPARSE_MIN_ROWS)
-    layer = octree._layers.get(key)
-
-    def made_engine():
-      eng = engine(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
-      eng.setup(octree, depth)
-      return eng
-
-    if layer is None:
-      layer = octree._layers[key] = _Layer(made_engine(), data.dtype, padded)
-    if layer.ok:
-      assert data.shape == layer.shape, \
-          'The shape of input data is wrong: expected {}, got {}.'.format(layer.shape, tuple(data.shape))
-      ok = True
-      if torch.is_grad_enabled():
-        # (the rows of a padded gradient are summed over the non-empty nodes only: the other route)
-        if padded and layer.conv and bias is not None and bias.requires_grad:
-          ok = False
-        if ok and data.requires_grad:
-          if layer.dgrad is None:
-            layer.make_dgrad(made_engine())
-          ok = layer.dgrad
-        if ok and weights.requires_grad:
-          if layer.wgrad is None:
-            layer.make_wgrad(made_engine())
-          ok = layer.wgrad
-      if ok:
-        return _lib.native().conv(layer.native, data, weights, bias)
+  """The layer through the native node where each of its passes is one, through `function` otherwise."""
+  layer, made_engine = _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
+                                 max_buffer, padded)
+  if layer is not None:
+    ok = True
+    if torch.is_grad_enabled():
+      # (the rows of a padded gradient are summed over the non-empty nodes only: the other route)
+      if padded and layer.conv and bias is not None and bias.requires_grad:
+        ok = False
+      if ok and data.requires_grad:
+        if layer.dgrad is None:
+          layer.make_dgrad(made_engine())
+        ok = layer.dgrad
+      if ok and weights.requires_grad:
+        if layer.wgrad is None:
+          layer.make_wgrad(made_engine())
+        ok = layer.wgrad
+    if ok:
+      return _lib.native().conv(layer.native, data, weights, bias)
   return function.apply(data, weights, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
                         max_buffer, bias, padded)
 
@@ -763,6 +773,15 @@ class OctreeConv(OctreeConvBase, torch.nn.Module):
     if pad:
       out = octree_pad(out, octree, depth - 1)
     return out
+
+  def native_layer(self, data: torch.Tensor, octree, depth: int):
+    """The native passes of this layer on `octree`, or None where it takes another route."""
+    if self.method != 'hip':
+      return None
+    layer, _ = _layer_of(_OctreeConv if self.is_conv_layer() else _OctreeDeconv, data, octree, depth, self.in_channels,
+                         self.out_channels, self.kernel_size, self.stride, self.nempty, self.max_buffer,
+                         self.stride == 2 and not self.nempty)
+    return None if layer is None else layer.native
 
   def extra_repr(self) -> str:
     return ('in_channels={}, out_channels={}, kernel_size={}, stride={}, '

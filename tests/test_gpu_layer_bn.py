@@ -1,0 +1,72 @@
+"""A layer and the batch norm behind it as one call in evaluation, against the two calls that run when
+gradients are on: every kernel that may take the layer, with and without bias, residual and ReLU."""
+
+import pytest
+import torch
+
+from ocnn_amd import synthetic
+from ocnn_amd.modules import Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
+from ocnn_amd.octree import Octree, Points
+
+pytestmark = pytest.mark.gpu
+TOL = {torch.float32: 1e-5, torch.float16: 4e-3, torch.bfloat16: 3e-2}
+
+
+def _octree(n=3000, depth=5):
+  points, normals = synthetic.sphere_cloud(n)
+  octree = Octree(depth, 2, device='cuda')
+  octree.build_octree(Points(points, normals).cuda())
+  octree.construct_all_neigh()
+  return octree
+
+
+def _randomise(module, dtype):
+  g = torch.Generator().manual_seed(5)
+  for m in module.modules():
+    if isinstance(m, torch.nn.BatchNorm1d):
+      for t, lo in ((m.running_var, 0.5), (m.weight.data, 0.5), (m.running_mean, -0.5), (m.bias.data, -0.5)):
+        t.copy_(torch.rand(t.shape, generator=g) + lo)
+  return module.to('cuda', dtype).eval()
+
+
+def _both(module, *args):
+  with torch.no_grad():
+    one = module(*args)
+  with torch.enable_grad():
+    two = module(*args).detach()
+  assert one.shape == two.shape and one.dtype == two.dtype
+  return (one.double() - two.double()).abs().max().item() / two.double().abs().max().item()
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('nempty', [False, True])
+def test_layer_bn(dtype, nempty):
+  octree, depth = _octree(), 5
+  for cls, cin, cout, kernel, stride, at in ((OctreeConvBnRelu, 32, 32, [3], 1, depth), (OctreeConvBnRelu, 64, 96, [3], 1, 4),
+                                             (OctreeConvBnRelu, 4, 32, [3], 1, depth), (OctreeConvBnRelu, 24, 40, [3], 1, depth),
+                                             (OctreeConvBnRelu, 32, 64, [2], 2, depth), (OctreeConvBnRelu, 256, 256, [3], 1, 3),
+                                             (OctreeDeconvBnRelu, 64, 32, [2], 2, depth - 1)):
+    print(cls.__name__, dtype, nempty, cin, cout, kernel, stride, at, flush=True)
+    layer = _randomise(cls(cin, cout, kernel, stride, nempty), dtype)
+    rows = int((octree.nnum_nempty if nempty else octree.nnum)[at])
+    x = torch.randn(rows, cin, generator=torch.Generator().manual_seed(cin)).to('cuda', dtype)
+    assert _both(layer, x, octree, at) < TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,cout', [(32, 32), (64, 32), (96, 128)])
+def test_residual_block(dtype, cin, cout):
+  octree = _octree(20000, 6)
+  rows = int(octree.nnum[6])
+  print('block', dtype, cin, cout, rows, flush=True)
+  x = torch.randn(rows, cin, generator=torch.Generator().manual_seed(cin)).to('cuda', dtype)
+  block = _randomise(OctreeResBlock2(cin, cout), dtype)
+  assert _both(block, x, octree, 6) < 2 * TOL[dtype]
+  shortcut = _randomise(Conv1x1Bn(cin, cout), dtype)
+  assert _both(shortcut, x) < TOL[dtype]
+  seen = []                                              # hooks of the parts are still called
+  handle = block.conv3x3b.conv.register_forward_hook(lambda *a: seen.append(1))
+  with torch.no_grad():
+    block(x, octree, 6)
+  handle.remove()
+  assert seen == [1]

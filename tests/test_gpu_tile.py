@@ -23,7 +23,7 @@ def _gather(x, plan, w, cout, transposed, reverse, b, parts, occupancy):
     size = 8 * K * cin * cout + 1024 + parts[0] * parts[1] * plan.rows * cout * 4
   ws = torch.empty(size, dtype=torch.uint8, device='cuda')
   _lib.check(L.ocnnx_gather_tile(code, P(x), x.shape[0], P(plan.loc), P(plan.uptr), P(plan.urows), plan.umax, plan.total,
-                                 occupancy, plan.rows, K, P(w), cin, cout, int(transposed), int(reverse), P(b), P(out),
+                                 occupancy, plan.rows, K, P(w), cin, cout, int(transposed), int(reverse), P(b), None, P(out),
                                  P(ws), size, *parts, _lib.stream()))
   return out
 
