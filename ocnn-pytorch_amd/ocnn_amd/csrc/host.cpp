@@ -564,6 +564,56 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   return t;
 }
 
+// ---- tile plans (octree/octree.py) ----------------------------------------
+
+struct BuiltPlan {
+  Tensor loc, uptr, urows, ucount;            // urows undefined: more than `pad` rows in a tile, or given up on
+  std::vector<int64_t> stats;
+};
+
+// The one-pass plans of several tables, one wait for the sizes of all of them.
+std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, int pad) {
+  const int n = (int)tables.size();
+  std::vector<BuiltPlan> out(n);
+  if (n == 0) return out;
+  std::vector<ocnnx_plan_item> items(n);
+  const auto i32 = tables[0].options(), i64 = i32.dtype(at::kLong), i16 = i32.dtype(at::kShort);
+  const int64_t tile_rows = ocnn_tile_plan_rows();
+  int64_t tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    const Tensor& t = tables[i];
+    require_gpu(t);
+    TORCH_CHECK(t.scalar_type() == at::kInt && t.dim() == 2 && t.is_contiguous() && t.device() == tables[0].device(),
+                "tile_plans: contiguous int32 tables of one device");
+    const int64_t own = (t.size(0) + tile_rows - 1) / tile_rows;
+    out[i].loc = at::empty({own, t.size(1), tile_rows}, i16);
+    out[i].uptr = at::empty({own + 1}, i32);
+    items[i] = {typed<int32_t>(t), typed<uint16_t>(out[i].loc), typed<int32_t>(out[i].uptr), nullptr, t.size(0), tiles,
+                (int)t.size(1)};
+    tiles += own;
+  }
+  Tensor counts = at::empty({2, std::max<int64_t>(tiles, 1)}, i32), lists = at::empty({std::max<int64_t>(tiles, 1) * pad}, i32);
+  Tensor stats = at::empty({n, 6}, i64), host = at::empty({n, 6}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  const auto st = c10::hip::getCurrentHIPStream();
+  int32_t* ucount = typed<int32_t>(counts);
+  check(ocnnx_plan_build(items.data(), n, cap, pad, ucount, ucount + counts.size(1), typed<int32_t>(lists),
+                         typed<int64_t>(stats), typed<int64_t>(host), st.stream()));
+  st.synchronize();
+  bool any = false;
+  for (int i = 0; i < n; ++i) {
+    const int64_t* v = typed<int64_t>(host) + 6 * i;
+    out[i].stats.assign(v, v + 6);
+    out[i].ucount = counts[0].slice(0, items[i].tile0, items[i].tile0 + out[i].uptr.size(0) - 1);
+    if (v[5] != 0 || v[3] > pad) continue;
+    out[i].urows = at::empty({std::max<int64_t>(v[2], 1)}, i32);
+    items[i].urows = typed<int32_t>(out[i].urows);
+    any = true;
+  }
+  if (any)
+    check(ocnnx_plan_compact(items.data(), n, cap, pad, ucount, typed<int64_t>(stats), typed<int32_t>(lists), st.stream()));
+  return out;
+}
+
 // The neighbour tables of layers 1 .. depth (entry 0 is left out).
 std::vector<Tensor> all_neigh(const std::vector<Tensor>& keys, const std::vector<Tensor>& children,
                               const std::vector<OptTensor>& index, const std::vector<int64_t>& nnum,
@@ -645,6 +695,11 @@ PYBIND11_MODULE(ocnn_host, m) {
       FIELD(keys) FIELD(children) FIELD(index) FIELD(nnum) FIELD(nnum_nempty) FIELD(idx) FIELD(points) FIELD(normals)
           FIELD(perm) FIELD(seg_start);
 #undef FIELD
+#define FIELD(name) .def_readonly(#name, &BuiltPlan::name)
+  py::class_<BuiltPlan>(m, "BuiltPlan")
+      FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(ucount) FIELD(stats);
+#undef FIELD
+  m.def("tile_plans", &tile_plans, py::call_guard<py::gil_scoped_release>());
   m.def("build_octree", &build_octree, py::call_guard<py::gil_scoped_release>());
   m.def("all_neigh", &all_neigh, py::call_guard<py::gil_scoped_release>());
   m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;

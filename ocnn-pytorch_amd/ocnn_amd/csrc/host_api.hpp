@@ -45,6 +45,22 @@ int ocnnx_batch_norm_running(int dtype, const void* x, int64_t rows, int channel
                              const void* running_var, int running_dtype, float eps, const void* gamma, const void* beta,
                              int param_dtype, int relu, const void* residual, void* y, void* stream);
 
+// Tile plans of n tables in one pass each over all of them (tile0: the tables' tiles numbered one behind the
+// other): counts, positions (loc) and, in `pad` entries a tile, the lists of distinct rows; then the
+// offsets uptr and the six sizes of ocnn_tile_plan_offsets per table, on the device and in host memory
+// that the device writes.  ocnnx_plan_compact moves the lists to urows (null: not of this table).
+typedef struct {
+  const int32_t* table;
+  uint16_t* loc;
+  int32_t *uptr, *urows;
+  int64_t rows, tile0;
+  int K;
+} ocnnx_plan_item;
+int ocnnx_plan_build(const ocnnx_plan_item* items, int n, int cap, int pad, int32_t* ucount, int32_t* tile_nnz,
+                     int32_t* lists, int64_t* stats, int64_t* host_stats, void* stream);
+int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, int pad, const int32_t* ucount, const int64_t* stats,
+                       const int32_t* lists, void* stream);
+
 // The octree build from the points on: normalised points, keys, sort and node counts (sizes: device,
 // levels + 1, as ocnn_octree_build_scan); then keys, children and the indices of the non-empty nodes of
 // the layers from the deepest full one on (h_index[d], d >= full_depth); then every neighbour table.

@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "host_api.hpp"
 #include "mma.hpp"
 
 namespace ocnn {
@@ -42,8 +43,8 @@ __device__ __forceinline__ int plan_hash(int32_t v) {
 // HASH = kPlanHashQuick (mode 2 only): a tile whose blocks do not fit gives up, ucount[tile] =
 // kPlanOverflow; the caller then plans the table in two passes with HASH = kPlanHash.
 template <int HASH>
-__global__ __launch_bounds__(kPlanThreads) void tile_plan_kernel(
-    const int32_t* __restrict__ table, int64_t rows, int K, int mode,
+__device__ __forceinline__ void plan_tile(
+    const int64_t tile, const int32_t* __restrict__ table, int64_t rows, int K, int mode,
     int32_t* __restrict__ ucount, const int32_t* __restrict__ uptr, int32_t* __restrict__ urows,
     uint16_t* __restrict__ loc, int32_t* __restrict__ tile_nnz, int pad) {
   constexpr int kList = HASH == kPlanHash ? kPlanMaxEntries : (HASH + 16 > kPlanPosWords ? HASH + 16 : kPlanPosWords);
@@ -55,7 +56,6 @@ __global__ __launch_bounds__(kPlanThreads) void tile_plan_kernel(
   __shared__ int32_t s_scan[2][kPlanThreads / 64];
   __shared__ int32_t s_nnz, s_over;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t tile = blockIdx.x;
   const int64_t e0 = tile * kPlanRows * K;
   const int64_t lim = rows * (int64_t)K;
   const int n = kPlanRows * K;
@@ -295,6 +295,39 @@ __global__ __launch_bounds__(kPlanThreads) void tile_plan_kernel(
     dst[i] = *(const u32x4*)(s_pos + (i >> 4) * kPitch + (i & 15) * 8);
 }
 
+__global__ __launch_bounds__(kPlanThreads) void tile_plan_kernel(
+    const int32_t* __restrict__ table, int64_t rows, int K, int mode, int32_t* __restrict__ ucount,
+    const int32_t* __restrict__ uptr, int32_t* __restrict__ urows, uint16_t* __restrict__ loc,
+    int32_t* __restrict__ tile_nnz) {
+  plan_tile<kPlanHash>(blockIdx.x, table, rows, K, mode, ucount, uptr, urows, loc, tile_nnz, 0);
+}
+
+// The one-pass build over the tiles of several tables: a network asks a fresh octree for a dozen plans,
+// most of them of a few tiles, and a launch each left the chip idle (13 x 8 us of build, 13 x 5 us of
+// offsets and 10 x 3.5 us of compaction for the U-Net on 40 k points; 30 us together in three launches).
+// Counts, lists and set entries of all tables stand one behind the other, by the tiles' common numbering.
+constexpr int kPlanItems = 24;          // tables a launch; their description travels as a kernel argument
+struct PlanItems {
+  int n;
+  ocnnx_plan_item it[kPlanItems];
+};
+
+__device__ __forceinline__ int plan_item_of(const PlanItems& p, int64_t tile) {
+  int i = 0;
+  while (i + 1 < p.n && tile >= p.it[i + 1].tile0) ++i;
+  return i;
+}
+
+__global__ __launch_bounds__(kPlanThreads) void tile_plan_build_kernel(PlanItems p, int64_t first, int32_t* __restrict__ ucount,
+                                                                       int32_t* __restrict__ lists,
+                                                                       int32_t* __restrict__ tile_nnz, int pad) {
+  const int64_t tile = first + blockIdx.x;
+  const ocnnx_plan_item& it = p.it[plan_item_of(p, tile)];
+  const int64_t t0 = it.tile0;
+  plan_tile<kPlanHashQuick>(tile - t0, it.table, it.rows, it.K, 2, ucount + t0, nullptr, lists + t0 * pad, it.loc,
+                            tile_nnz ? tile_nnz + t0 : nullptr, pad);
+}
+
 // Pair plan of a table, on top of its tile plan: per tile and LIST the rows that have a
 // neighbour, in blocks of 16 entries (position of the neighbour in the tile's list of rows
 // | row of the tile << 16).  A list is a slot, or
@@ -334,9 +367,9 @@ __global__ void pair_plan_kernel(const uint16_t* __restrict__ loc, int64_t tiles
 // tiles.  stats: [tiles over cap, dropped (0 | 1), total, largest count, entries set, tiles the
 // quick one-pass build gave up on (then nothing else here means anything)], the third to fifth
 // without the dropped tiles.
-__global__ __launch_bounds__(1024) void tile_plan_offsets_kernel(
+__device__ __forceinline__ void plan_offsets(
     const int32_t* __restrict__ ucount, const int32_t* __restrict__ tile_nnz, int64_t tiles, int cap,
-    int32_t* __restrict__ uptr, int64_t* __restrict__ stats) {
+    int32_t* __restrict__ uptr, int64_t* __restrict__ stats, int64_t* __restrict__ host_stats) {
   // the tiles in rounds of 4096, thread t on the four tiles from 4096 r + 4 t (consecutive
   // 16-byte loads, two rounds in flight); a round's counts fit 32 bits, the running offset is
   // carried from round to round by every thread
@@ -444,25 +477,37 @@ __global__ __launch_bounds__(1024) void tile_plan_offsets_kernel(
       max_all = max(max_all, s_wmax[w]);
     }
     uptr[tiles] = (int32_t)base;
-    stats[0] = n_big;
-    stats[1] = drop ? 1 : 0;
-    stats[2] = base;
-    stats[3] = max_all;
-    stats[4] = nnz_all;
-    stats[5] = n_over;
+    const int64_t v[6] = {n_big, drop ? 1 : 0, base, max_all, nnz_all, n_over};
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      stats[i] = v[i];
+      if (host_stats) host_stats[i] = v[i];               // (host memory: no copy to wait for on top of the kernel)
+    }
   }
+}
+
+__global__ __launch_bounds__(1024) void tile_plan_offsets_kernel(
+    const int32_t* __restrict__ ucount, const int32_t* __restrict__ tile_nnz, int64_t tiles, int cap,
+    int32_t* __restrict__ uptr, int64_t* __restrict__ stats) {
+  plan_offsets(ucount, tile_nnz, tiles, cap, uptr, stats, nullptr);
+}
+
+// workgroup i: table i
+__global__ __launch_bounds__(1024) void tile_plan_offsets_many_kernel(
+    PlanItems p, const int32_t* __restrict__ ucount, const int32_t* __restrict__ tile_nnz, int cap,
+    int64_t* __restrict__ stats, int64_t* __restrict__ host_stats) {
+  const ocnnx_plan_item& it = p.it[blockIdx.x];
+  plan_offsets(ucount + it.tile0, tile_nnz + it.tile0, (it.rows + kPlanRows - 1) / kPlanRows, cap, it.uptr,
+               stats + 6 * blockIdx.x, host_stats + 6 * blockIdx.x);
 }
 
 // After a one-pass build (mode 2 above): a wave per tile moves the tile's list from its fixed
 // place to its offset; a tile that the offsets dropped (more than `cap` distinct rows, few such
 // tiles) becomes empty: its positions are cleared.
-__global__ __launch_bounds__(256) void tile_plan_compact_kernel(
-    const int32_t* __restrict__ ucount, const int32_t* __restrict__ uptr, const int64_t* __restrict__ stats,
-    int cap, int pad, const int32_t* __restrict__ ulist, int32_t* __restrict__ urows, uint16_t* __restrict__ loc,
-    int K, int64_t tiles) {
+__device__ __forceinline__ void plan_compact(
+    int64_t tile, const int32_t* __restrict__ ucount, const int32_t* __restrict__ uptr, const int64_t* __restrict__ stats,
+    int cap, int pad, const int32_t* __restrict__ ulist, int32_t* __restrict__ urows, uint16_t* __restrict__ loc, int K) {
   const int lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tile >= tiles) return;
   const int U = ucount[tile];
   if (stats[1] != 0 && U > cap) {
     u32x4* p = (u32x4*)(loc + tile * (int64_t)(K * kPlanRows));
@@ -473,6 +518,27 @@ __global__ __launch_bounds__(256) void tile_plan_compact_kernel(
   const int32_t* src = ulist + tile * (int64_t)pad;
   int32_t* dst = urows + uptr[tile];
   for (int i = lane; i < U; i += 64) dst[i] = src[i];
+}
+
+__global__ __launch_bounds__(256) void tile_plan_compact_kernel(
+    const int32_t* __restrict__ ucount, const int32_t* __restrict__ uptr, const int64_t* __restrict__ stats,
+    int cap, int pad, const int32_t* __restrict__ ulist, int32_t* __restrict__ urows, uint16_t* __restrict__ loc,
+    int K, int64_t tiles) {
+  const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile < tiles) plan_compact(tile, ucount, uptr, stats, cap, pad, ulist, urows, loc, K);
+}
+
+// (urows null: a table that is filled in two passes)
+__global__ __launch_bounds__(256) void tile_plan_compact_many_kernel(
+    PlanItems p, int64_t first, int64_t last, const int32_t* __restrict__ ucount, const int64_t* __restrict__ stats, int cap,
+    int pad, const int32_t* __restrict__ lists) {
+  const int64_t tile = first + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile >= last) return;
+  const int i = plan_item_of(p, tile);
+  const ocnnx_plan_item& it = p.it[i];
+  const int64_t t0 = it.tile0;
+  if (it.urows)
+    plan_compact(tile - t0, ucount + t0, it.uptr, stats + 6 * i, cap, pad, lists + t0 * pad, it.urows, it.loc, it.K);
 }
 
 __global__ void pair_plan_zero_kernel(unsigned long long* __restrict__ slot_count, int K) {
@@ -510,27 +576,84 @@ using namespace ocnn;
 extern "C" int ocnn_tile_plan_rows(void) { return kPlanRows; }
 
 static int plan_launch(const int32_t* table, int64_t rows, int K, int mode, int32_t* ucount,
-                       const int32_t* uptr, int32_t* urows, uint16_t* loc, int32_t* tile_nnz, int pad,
-                       void* stream) {
+                       const int32_t* uptr, int32_t* urows, uint16_t* loc, int32_t* tile_nnz, void* stream) {
   OCNN_REQUIRE(K >= 1 && K <= 27 && rows >= 0 && rows < (1ll << 31), "tile_plan: bad shape");
   if (rows == 0) return OCNN_OK;
-  // count: the table and the counts; fill: the offsets, the lists and the positions; build: all but the offsets
-  OCNN_REQUIRE(table && (mode == 1 ? (uptr && urows && loc) : ucount != nullptr) && (mode != 2 || (urows && loc)),
-               "tile_plan: a required pointer is NULL");
-  int64_t tiles = cdiv(rows, kPlanRows);
-  if (mode == 2)
-    hipLaunchKernelGGL(tile_plan_kernel<kPlanHashQuick>, dim3((unsigned)tiles), dim3(kPlanThreads), 0,
-                       (hipStream_t)stream, table, rows, K, mode, ucount, uptr, urows, loc, tile_nnz, pad);
-  else
-    hipLaunchKernelGGL(tile_plan_kernel<kPlanHash>, dim3((unsigned)tiles), dim3(kPlanThreads), 0,
-                       (hipStream_t)stream, table, rows, K, mode, ucount, uptr, urows, loc, tile_nnz, pad);
+  // count: the table and the counts; fill: the offsets, the lists and the positions
+  OCNN_REQUIRE(table && (mode == 1 ? (uptr && urows && loc) : ucount != nullptr), "tile_plan: a required pointer is NULL");
+  hipLaunchKernelGGL(tile_plan_kernel, dim3((unsigned)cdiv(rows, kPlanRows)), dim3(kPlanThreads), 0, (hipStream_t)stream,
+                     table, rows, K, mode, ucount, uptr, urows, loc, tile_nnz);
   return check_launch("tile_plan");
+}
+
+// Calls f(items, first tile, tiles, number of the first item) for every kPlanItems of them.
+template <typename F>
+static void plan_groups(const ocnnx_plan_item* items, int n, F f) {
+  for (int g = 0; g < n; g += kPlanItems) {
+    PlanItems p;
+    p.n = std::min(kPlanItems, n - g);
+    int64_t tiles = 0;
+    for (int i = 0; i < p.n; ++i) {
+      p.it[i] = items[g + i];
+      tiles += cdiv(p.it[i].rows, kPlanRows);
+    }
+    f(p, items[g].tile0, tiles, g);
+  }
+}
+
+static int plan_items_check(const ocnnx_plan_item* items, int n) {
+  int64_t at = 0;
+  for (int i = 0; i < n; ++i) {
+    const ocnnx_plan_item& it = items[i];
+    OCNN_REQUIRE(it.K >= 1 && it.K <= 27 && it.rows >= 0 && it.rows < (1ll << 31) && it.tile0 == at,
+                 "tile_plan: bad shape");
+    OCNN_REQUIRE(it.uptr && (it.rows == 0 || (it.table && it.loc)), "tile_plan: a required pointer is NULL");
+    at += cdiv(it.rows, kPlanRows);
+  }
+  return OCNN_OK;
+}
+
+extern "C" int ocnnx_plan_build(const ocnnx_plan_item* items, int n, int cap, int pad, int32_t* ucount, int32_t* tile_nnz,
+                                int32_t* lists, int64_t* stats, int64_t* host_stats, void* stream) {
+  OCNN_REQUIRE(n >= 1 && pad >= 1 && pad <= 4096 && cap >= 0 && cap <= pad, "plan_build: bad sizes");
+  OCNN_REQUIRE_PTRS("plan_build", items, ucount, tile_nnz, lists, stats, host_stats);
+  if (const int rc = plan_items_check(items, n)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  plan_groups(items, n, [&](const PlanItems& p, int64_t first, int64_t tiles, int g) {
+    if (tiles > 0)
+      hipLaunchKernelGGL(tile_plan_build_kernel, dim3((unsigned)tiles), dim3(kPlanThreads), 0, st, p, first, ucount, lists,
+                         tile_nnz, pad);
+    hipLaunchKernelGGL(tile_plan_offsets_many_kernel, dim3((unsigned)p.n), dim3(1024), 0, st, p, ucount, tile_nnz, cap,
+                       stats + 6 * g, host_stats + 6 * g);
+  });
+  return check_launch("plan_build");
+}
+
+extern "C" int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, int pad, const int32_t* ucount,
+                                  const int64_t* stats, const int32_t* lists, void* stream) {
+  OCNN_REQUIRE(n >= 1 && pad >= 1 && cap >= 0 && cap <= pad, "plan_compact: bad sizes");
+  OCNN_REQUIRE_PTRS("plan_compact", items, ucount, stats, lists);
+  if (const int rc = plan_items_check(items, n)) return rc;
+  plan_groups(items, n, [&](const PlanItems& p, int64_t first, int64_t tiles, int g) {
+    if (tiles > 0)
+      hipLaunchKernelGGL(tile_plan_compact_many_kernel, dim3((unsigned)cdiv(tiles, 4)), dim3(256), 0, (hipStream_t)stream, p,
+                         first, first + tiles, ucount, stats + 6 * g, cap, pad, lists);
+  });
+  return check_launch("plan_compact");
 }
 
 extern "C" int ocnn_tile_plan_build(const int32_t* table, int64_t rows, int K, int pad, int32_t* ucount,
                                     int32_t* tile_nnz, int32_t* ulist, uint16_t* loc, void* stream) {
   OCNN_REQUIRE(pad >= 1 && pad <= 4096, "tile_plan_build: bad list size");
-  return plan_launch(table, rows, K, 2, ucount, nullptr, ulist, loc, tile_nnz, pad, stream);
+  OCNN_REQUIRE(K >= 1 && K <= 27 && rows >= 0 && rows < (1ll << 31), "tile_plan: bad shape");
+  if (rows == 0) return OCNN_OK;
+  OCNN_REQUIRE(table && ucount && ulist && loc, "tile_plan: a required pointer is NULL");
+  PlanItems p;
+  p.n = 1;
+  p.it[0] = {table, loc, nullptr, nullptr, rows, 0, K};
+  hipLaunchKernelGGL(tile_plan_build_kernel, dim3((unsigned)cdiv(rows, kPlanRows)), dim3(kPlanThreads), 0,
+                     (hipStream_t)stream, p, (int64_t)0, ucount, ulist, tile_nnz, pad);
+  return check_launch("tile_plan");
 }
 
 extern "C" int ocnn_tile_plan_compact(const int32_t* ucount, const int32_t* uptr, const int64_t* stats, int cap,
@@ -547,7 +670,7 @@ extern "C" int ocnn_tile_plan_compact(const int32_t* ucount, const int32_t* uptr
 
 extern "C" int ocnn_tile_plan_count(const int32_t* table, int64_t rows, int K, int32_t* ucount,
                                     int32_t* tile_nnz, void* stream) {
-  return plan_launch(table, rows, K, 0, ucount, nullptr, nullptr, nullptr, tile_nnz, 0, stream);
+  return plan_launch(table, rows, K, 0, ucount, nullptr, nullptr, nullptr, tile_nnz, stream);
 }
 
 extern "C" int ocnn_tile_plan_offsets(const int32_t* ucount, const int32_t* tile_nnz, int64_t tiles, int cap,
@@ -562,7 +685,7 @@ extern "C" int ocnn_tile_plan_offsets(const int32_t* ucount, const int32_t* tile
 
 extern "C" int ocnn_tile_plan_fill(const int32_t* table, int64_t rows, int K, const int32_t* uptr,
                                    int32_t* urows, uint16_t* loc, void* stream) {
-  return plan_launch(table, rows, K, 1, nullptr, uptr, urows, loc, nullptr, 0, stream);
+  return plan_launch(table, rows, K, 1, nullptr, uptr, urows, loc, nullptr, stream);
 }
 
 extern "C" int ocnn_pair_plan_slot_counts(const uint16_t* loc, int64_t tiles, int K, int64_t* slot_count,

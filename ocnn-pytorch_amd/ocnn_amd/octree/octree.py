@@ -128,95 +128,76 @@ class TilePlan:
   LIST_PAD = 416  # rows a tile's list may have in the one-pass build
 
   def __init__(self, table: torch.Tensor, cap: int = None):
-    self._count(table, cap)
-    self._finish(self._host_stats(self._stats.tolist(), table, cap))
-
-  def _host_stats(self, stats, table, cap):
-    """The sizes on the host; a table the one-pass build gave up on (tiles with more distinct
-    blocks of rows than its set holds: no locality) is counted again the long way first."""
-    if stats[5]:
-      self._count(table, cap, one_pass=False)
-      stats = self._stats.tolist()
-    return [int(v) for v in stats]
+    table = table.contiguous()
+    cap = self.CAP if cap is None else cap
+    self._set(table, cap, *self._one_pass([table], cap))
 
   @classmethod
   def build_many(cls, tables, cap: int = None):
-    """Plans of several tables with one device -> host read-back."""
-    plans = [cls.__new__(cls) for _ in tables]
-    for p, t in zip(plans, tables):
-      p._count(t, cap)
-    host = torch.stack([p._stats for p in plans]).tolist() if plans else []
-    for p, t, st in zip(plans, tables, host):
-      p._finish(p._host_stats(st, t, cap))
+    """Plans of several tables, in one launch of each kernel and with one wait for their sizes."""
+    plans, tables = [cls.__new__(cls) for _ in tables], [t.contiguous() for t in tables]
+    cap = cls.CAP if cap is None else cap
+    for p, t, built in zip(plans, tables, cls._one_pass(tables, cap)):
+      p._set(t, cap, built)
     return plans
 
-  def _count(self, table, cap, one_pass=True):
-    """First half: distinct rows per tile, their offsets, and the sizes the second half
-    needs on the host as one device vector."""
-    _lib.require_gpu(table)
-    L = _lib.lib()
-    table = table.contiguous()
-    rows, K = table.shape
-    self._tile_rows = L.ocnn_tile_plan_rows()
-    tiles = (rows + self._tile_rows - 1) // self._tile_rows
-    self._cap = self.CAP if cap is None else cap
-    self._table = table
-    self.rows, self.K = rows, K
+  @classmethod
+  def _one_pass(cls, tables, cap):
+    """Counts, positions and lists in one pass over the tables, the lists at fixed places (LIST_PAD
+    rows a tile) first.  (A limit above LIST_PAD takes the two passes of count and fill.)"""
+    if cap > cls.LIST_PAD or not tables:
+      return [None] * len(tables)
+    _lib.require_gpu(*tables)
+    with torch.cuda.device(tables[0].device):
+      return _lib.native().tile_plans(tables, cap, cls.LIST_PAD)
+
+  def _set(self, table, cap, built):
+    self.rows, self.K = table.shape
     self.overflow_rows = self.overflow_table = None
     self._pairs = None
     self._on_pairs = None          # called when the pair plan is first asked for
-    dev, st = table.device, _lib.stream()
-    self._ucount = torch.empty(tiles, dtype=torch.int32, device=dev)
-    tile_nnz = torch.empty(tiles, dtype=torch.int32, device=dev)
-    self.uptr = torch.empty(tiles + 1, dtype=torch.int32, device=dev)
-    self._stats = torch.empty(6, dtype=torch.int64, device=dev)
-    # One pass over the table: counts, positions and the lists at fixed places (LIST_PAD rows a
-    # tile); the second half only moves the lists to their offsets.  (A limit above LIST_PAD, or
-    # a table whose tiles do not fit it, takes the two passes of count and fill.)
-    self._lists = None
-    if one_pass and self._cap <= self.LIST_PAD:
-      self._lists = torch.empty(max(tiles, 1) * self.LIST_PAD, dtype=torch.int32, device=dev)
-      # uint16 payload, [tile][slot][row in tile]: whole tiles, the tail reads "empty"
-      self.loc = torch.empty((tiles, K, self._tile_rows), dtype=torch.int16, device=dev)
-      _lib.check(L.ocnn_tile_plan_build(_lib.ptr(table), rows, K, self.LIST_PAD, _lib.ptr(self._ucount),
-                                        _lib.ptr(tile_nnz), _lib.ptr(self._lists), _lib.ptr(self.loc), st))
+    if built is not None and not built.stats[5]:
+      self.uptr, self.urows, self.loc, ucount, stats = built.uptr, built.urows, built.loc, built.ucount, built.stats
     else:
-      _lib.check(L.ocnn_tile_plan_count(_lib.ptr(table), rows, K, _lib.ptr(self._ucount), _lib.ptr(tile_nnz), st))
-    _lib.check(L.ocnn_tile_plan_offsets(_lib.ptr(self._ucount), _lib.ptr(tile_nnz), tiles, self._cap,
-                                        _lib.ptr(self.uptr), _lib.ptr(self._stats), st))
-
-  def _finish(self, stats):
-    """Second half, with the sizes on the host: row lists and positions."""
-    L = _lib.lib()
-    table, tile_rows = self._table, self._tile_rows
-    rows, K = self.rows, self.K
-    tiles = self._ucount.numel()
-    dev = table.device
-    _, dropped, total, umax, nnz = stats[:5]
-    one_pass = self._lists is not None and umax <= self.LIST_PAD
+      # (tiles with more distinct blocks of rows than the one pass holds: no locality)
+      ucount, stats = self._count(table, cap)
+      self.urows = None
+    _, dropped, self.total, self.umax, self.nnz = stats[:5]
+    # how often a staged row is used by its tile: near 1 there is nothing to gain from staging
+    self.reuse = self.nnz / max(self.total, 1)
     if dropped:
-      big = self._ucount > self._cap
-      idx = (big.nonzero().view(-1, 1) * tile_rows + torch.arange(tile_rows, device=dev).view(1, -1)).view(-1)
-      idx = idx[idx < rows]
-      self.overflow_rows = idx
+      tile_rows = _lib.lib().ocnn_tile_plan_rows()
+      idx = ((ucount > cap).nonzero().view(-1, 1) * tile_rows +
+             torch.arange(tile_rows, device=table.device).view(1, -1)).view(-1)
+      self.overflow_rows = idx = idx[idx < self.rows]
       self.overflow_table = table.index_select(0, idx).contiguous()
-      if not one_pass:
+    if self.urows is None:
+      if dropped:
         table = table.clone()
         table[idx] = -1
-    # how often a staged row is used by its tile: near 1 there is nothing to gain from staging
-    self.reuse = nnz / max(total, 1)
-    self.urows = torch.empty(max(total, 1), dtype=torch.int32, device=dev)
-    if one_pass:
-      _lib.check(L.ocnn_tile_plan_compact(_lib.ptr(self._ucount), _lib.ptr(self.uptr), _lib.ptr(self._stats),
-                                          self._cap, self.LIST_PAD, _lib.ptr(self._lists), _lib.ptr(self.urows),
-                                          _lib.ptr(self.loc), K, tiles, _lib.stream()))
-    else:
-      # uint16 payload, [tile][slot][row in tile]: whole tiles, the tail reads "empty"
-      self.loc = torch.empty((tiles, K, tile_rows), dtype=torch.int16, device=dev)
-      _lib.check(L.ocnn_tile_plan_fill(_lib.ptr(table), rows, K, _lib.ptr(self.uptr),
-                                       _lib.ptr(self.urows), _lib.ptr(self.loc), _lib.stream()))
-    self.total, self.umax, self.nnz = total, umax, nnz
-    self._table = self._ucount = self._stats = self._lists = None
+      self._fill(table)
+
+  def _count(self, table, cap):
+    """First of two passes: distinct rows per tile, their offsets, and the sizes on the host."""
+    _lib.require_gpu(table)
+    L, P, st, dev = _lib.lib(), _lib.ptr, _lib.stream(), table.device
+    tiles = -(-self.rows // L.ocnn_tile_plan_rows())
+    ucount = torch.empty(tiles, dtype=torch.int32, device=dev)
+    tile_nnz = torch.empty(tiles, dtype=torch.int32, device=dev)
+    self.uptr = torch.empty(tiles + 1, dtype=torch.int32, device=dev)
+    stats = torch.empty(6, dtype=torch.int64, device=dev)
+    _lib.check(L.ocnn_tile_plan_count(P(table), self.rows, self.K, P(ucount), P(tile_nnz), st))
+    _lib.check(L.ocnn_tile_plan_offsets(P(ucount), P(tile_nnz), tiles, cap, P(self.uptr), P(stats), st))
+    return ucount, stats.tolist()
+
+  def _fill(self, table):
+    """Second pass: row lists and positions."""
+    L, P, dev = _lib.lib(), _lib.ptr, table.device
+    tile_rows = L.ocnn_tile_plan_rows()
+    self.urows = torch.empty(max(self.total, 1), dtype=torch.int32, device=dev)
+    # uint16 payload, [tile][slot][row in tile]: whole tiles, the tail reads "empty"
+    self.loc = torch.empty((-(-self.rows // tile_rows), self.K, tile_rows), dtype=torch.int16, device=dev)
+    _lib.check(L.ocnn_tile_plan_fill(P(table), self.rows, self.K, P(self.uptr), P(self.urows), P(self.loc), _lib.stream()))
 
   def __getstate__(self):
     """(copies leave out the layers' native passes, which are made again when asked for)"""
