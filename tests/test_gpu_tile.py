@@ -51,3 +51,21 @@ def test_tile_kernel(dtype, cin, cout):
           assert err < TOL[dtype], (parts, occupancy, tr, err)
           again = _gather(x.cuda(), plan, ww.cuda(), cout, tr, rev, b.cuda(), parts, occupancy)
           assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+def test_tile_kernel_weights_off_alignment(dtype):
+  """Weights that start one element past a 16-byte boundary give the bits of aligned ones."""
+  g = torch.Generator().manual_seed(5)
+  rows, K, cin, cout = 300, 27, 96, 64
+  t = torch.randint(-1, rows, (rows, K), generator=g).int()
+  t[torch.rand(rows, K, generator=g) < 0.9] = -1
+  plan = TilePlan(t.cuda())
+  x = torch.randn(rows, cin, generator=g).to(dtype).cuda()
+  b = torch.zeros(cout, dtype=dtype).cuda()
+  for shape, tr in (((K, cin, cout), False), ((K, cout, cin), True)):
+    w = torch.randn(shape, generator=g).to(dtype).cuda()
+    off = torch.empty(w.numel() + 1, dtype=dtype, device='cuda')[1:].view(shape)
+    off.copy_(w)
+    assert w.data_ptr() % 16 == 0 and off.data_ptr() % 16 != 0
+    assert torch.equal(_gather(x, plan, w, cout, tr, tr, b, (0, 0), 1.0), _gather(x, plan, off, cout, tr, tr, b, (0, 0), 1.0))
