@@ -47,10 +47,12 @@ struct WpStage {
   char* sl;
 };
 
-// A workgroup sums a C x C block (C = 64 or 32) of the channel pairs; blockIdx.y picks
-// the block when the layer has more channels (BLK; C = 64).  NFULL slots per wave with all
+// A workgroup sums a C x C block (C = 64 or 32) of the channel pairs of one range of tiles, one
+// of them when the layer has more channels (BLK; C = 64).  NFULL slots per wave with all
 // C x channels, NHALF (0/1, C = 64 only) slot shared by two waves (one x-channel half each);
-// GROUPS workgroups split the K slots.
+// GROUPS workgroups split the K slots.  The workgroups of a range (slot groups, blocks) are neighbours in
+// the numbering, and each XCD takes an eighth of all of them in a row: they stage the same rows, and every
+// XCD has the same number however few ranges there are.
 //
 // LDS layout: the two 32-channel halves of the staged rows live in separate arrays
 // of 64-byte rows.  A transposing read of a 16-lane group touches 4 rows x 32 B, a
@@ -61,12 +63,21 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
     const uint16_t* __restrict__ loc, uint32_t loc_bytes, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ urows, uint32_t urows_bytes, int64_t tiles,
-    int64_t tiles_per_split, int nsplit, int ca, int cb, float* __restrict__ partial, const T* __restrict__ x_lo,
-    const T* __restrict__ g_lo, int64_t set) {
-  // fp32 data as bf16 pieces: hi hi, hi lo, lo hi, each with sums of its own
-  if (blockIdx.z == 1) g = g_lo;
-  if (blockIdx.z == 2) x = x_lo;
-  partial += blockIdx.z * set;
+    int64_t tiles_per_split, int workgroups, int ca, int cb, float* __restrict__ partial,
+    const T* __restrict__ x_lo, const T* __restrict__ g_lo, int64_t set) {
+  int number = (int)xcd_tile(blockIdx.x, gridDim.x >> 3);
+  if (number >= workgroups) return;
+  const int grp = number % GROUPS;
+  number /= GROUPS;
+  // a block of a wider layer (channel counts are multiples of 32: the last block may be half)
+  const int nbb = BLK ? (cb + C - 1) / C : 1, nblocks = BLK ? nbb * ((ca + C - 1) / C) : 1;
+  const int block = __builtin_amdgcn_readfirstlane(number % nblocks);
+  const int split = __builtin_amdgcn_readfirstlane(number / nblocks);
+  // fp32 data as bf16 pieces: hi hi, hi lo, lo hi, each with sums of its own.  (A product's number is a grid
+  // index of its own: out of a division it made the pointers, and every staging load, vectors.)
+  if (blockIdx.y == 1) g = g_lo;
+  if (blockIdx.y == 2) x = x_lo;
+  partial += blockIdx.y * set;
   constexpr int H = C / 32;                   // 32-channel halves of a row
   constexpr int NU = H * NFULL + NHALF;       // 32 x C accumulator units per wave
   constexpr int NS = NFULL + NHALF;           // distinct slots per wave
@@ -96,11 +107,6 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // workgroups of one tile range sit on the same XCD (they stage the same rows)
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7, idx = bid >> 3;
-  const int grp = idx % GROUPS;
-  const int split = xcd * (nsplit >> 3) + idx / GROUPS;
   const int64_t t_begin = (int64_t)split * tiles_per_split;
   const int64_t t_end = min(tiles, t_begin + tiles_per_split);
   if (t_begin >= t_end) return;
@@ -155,8 +161,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   static_assert(kPieces <= 20 && (kWpCap + 1) % 16 == 0, "five steps of four pieces stage a tile");
   constexpr int RSH = 5 + H;                               // log2 of the bytes of a C-channel row
   // a block of a wider layer: rows of ca (cb) channels, this block's 64 start at xb (gb)
-  const int nbb = BLK ? (cb + C - 1) / C : 1;             // (channel counts are multiples of 32: the last block may be half)
-  const int blk_a = BLK ? (int)blockIdx.y / nbb : 0, blk_b = BLK ? (int)blockIdx.y % nbb : 0;
+  const int blk_a = __builtin_amdgcn_readfirstlane(block / nbb), blk_b = block - blk_a * nbb;
   const uint32_t x_pitch = BLK ? (uint32_t)ca * 2u : (1u << RSH), g_pitch = BLK ? (uint32_t)cb * 2u : (1u << RSH);
   const uint32_t xb = (uint32_t)blk_a << RSH, gb = (uint32_t)blk_b << RSH;
   const int st_half = H == 2 ? (wave & 1) : 0, st_g16 = H == 2 ? (wave >> 1) : wave;
@@ -384,13 +389,37 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 using namespace ocnn;
 
 
-// ranges of tiles: as many as keep a workgroup on every CU (the LDS holds one), with the slot groups, the
-// blocks of channel pairs and, in fp32, the three products of bf16 pieces as further workgroups
+// workgroups of one range of tiles (and one product of bf16 pieces): the slot groups, the blocks of channel pairs
+static int wp_range_workgroups(int K, int ca, int cb) {
+  const int groups = (K == 27 && ca >= 64) ? 2 : 1;
+  return groups * (ca >= 64 ? ((ca + 63) / 64) * ((cb + 63) / 64) : 1);
+}
+
+// ranges of tiles at most: as many as keep a workgroup on every CU (the LDS holds one)
 static int wp_splits(int K, int ca, int cb, int n_cu, int products) {
-  const int groups = ((K == 27 && ca >= 64) ? 2 : 1) * products;
-  const int blocks = ca >= 64 ? ((ca + 63) / 64) * ((cb + 63) / 64) : 1;
-  int s = std::max(8, n_cu / (groups * blocks) / 8 * 8);      // a multiple of 8: ranges are dealt to the XCDs
-  return std::min(s, 256);
+  return std::min(256, std::max(8, n_cu / (wp_range_workgroups(K, ca, cb) * products)));
+}
+
+// Tiles of a range, for the least time of
+//   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
+//   the first tile, writing the sums) + the sums of all ranges written and read back, in units of one tile's time.
+// Measured (fp16, 64 x 64 blocks of 27 slots): 2.45 us a tile and 8 us besides on 33 - 157 tiles a range; the sums
+// move at about 3.5 TB/s.  Rounds are counted on an XCD's CUs (64 -> 64 in fp32 with 42 ranges is 33
+// workgroups on 32 CUs: 245 us where 40 ranges take 143), the sums where there are few tiles (256 -> 256 in fp32: 21 MB a range).
+constexpr double kWpFixed = 3.3, kWpSumCost = 2.3e-7;        // tiles; tiles a byte of sums
+static int64_t wp_tiles_per_range(int64_t tiles, int K, int ca, int cb, int n_cu, int products) {
+  const int wgs = wp_range_workgroups(K, ca, cb), cu_xcd = std::max(1, n_cu / 8);
+  const double sums = (double)K * ca * cb * 4 * products * kWpSumCost;      // of one range
+  int64_t best = std::max<int64_t>(tiles, 1);
+  double least = 1e30;
+  for (int s = 1, most = wp_splits(K, ca, cb, n_cu, products); s <= most; ++s) {
+    const int64_t per = std::max<int64_t>(1, cdiv(tiles, s));
+    const int64_t used = cdiv(tiles, per);
+    if (used < s) continue;                                  // (the same ranges as fewer)
+    const double cost = (double)cdiv(cdiv(used * wgs, 8) * products, cu_xcd) * ((double)per + kWpFixed) + (double)used * sums;
+    if (cost < least) least = cost, best = per;
+  }
+  return best;
 }
 
 static int wp_cu_count() {
@@ -437,7 +466,7 @@ struct WpArgs {
   int64_t rows_x, rows, set, per, plan_total;
   const uint16_t* loc;
   const int32_t *uptr, *urows;
-  int K, ca, cb, nsplit;
+  int K, ca, cb, used;                        // used: ranges of tiles
   float* partial;
 };
 
@@ -445,16 +474,17 @@ template <typename T, int C, int KK, int NFULL, int NHALF, int GROUPS>
 static void launch_wp(const WpArgs& a, hipStream_t st) {
   const int64_t tiles = cdiv(a.rows, kWpRows);
   const uint32_t xb = (uint32_t)(a.rows_x * a.ca * 2), gb = (uint32_t)(a.rows * a.cb * 2);
+  const int wgs = a.used * wp_range_workgroups(a.K, a.ca, a.cb);
   const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(a.plan_total * 4);
-#define OCNN_WP_KERNEL(BLK_, GY_)                                                                                        \
+#define OCNN_WP_KERNEL(BLK_)                                                                                        \
   hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, C, KK, NFULL, NHALF, GROUPS, BLK_>),                                  \
-                     dim3(a.nsplit * GROUPS, GY_, a.products), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g, gb,   \
-                     a.loc, lb, a.uptr, a.urows, ub, tiles, a.per, a.nsplit, a.ca, a.cb, a.partial, (const T*)a.x_lo,    \
+                     dim3(8 * (unsigned)cdiv(wgs, 8), a.products), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g,    \
+                     gb, a.loc, lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial, (const T*)a.x_lo,     \
                      (const T*)a.g_lo, a.set)
   if (a.ca == C && a.cb == C)
-    OCNN_WP_KERNEL(false, 1);
+    OCNN_WP_KERNEL(false);
   else if constexpr (C == 64)
-    OCNN_WP_KERNEL(true, ((a.ca + C - 1) / C) * ((a.cb + C - 1) / C));
+    OCNN_WP_KERNEL(true);
 #undef OCNN_WP_KERNEL
 }
 
@@ -490,11 +520,10 @@ static int run_wp(const void* x, int64_t rows_x, const void* g, const uint16_t* 
     return OCNN_ERR_HIP;
   }
   WpArgs a{x, g, nullptr, nullptr, kPieces ? 3 : 1, rows_x, rows, 0, 0, plan_total, loc, uptr, urows, K, ca, cb, 0, nullptr};
-  a.nsplit = wp_splits(K, ca, cb, n_cu, a.products);
   const int64_t tiles = cdiv(rows, kWpRows);
-  a.per = std::max<int64_t>(1, cdiv(tiles, a.nsplit));
-  const int used = (int)cdiv(tiles, a.per);               // ranges that hold tiles
-  a.set = (int64_t)used * K * ca * cb;                     // floats of one set of sums
+  a.per = wp_tiles_per_range(tiles, K, ca, cb, n_cu, a.products);
+  a.used = (int)cdiv(tiles, a.per);
+  a.set = (int64_t)a.used * K * ca * cb;                     // floats of one set of sums
   const int64_t xb = kPieces ? align_up(rows_x * ca * 2, 256) : 0, gb = kPieces ? align_up(rows * cb * 2, 256) : 0;
   if (ws_bytes < 2 * xb + 2 * gb + a.products * a.set * 4) {
     set_error("conv_wgrad_planned: workspace too small");
@@ -512,7 +541,7 @@ static int run_wp(const void* x, int64_t rows_x, const void* g, const uint16_t* 
       launch_wp_sums<T>(a, st);
     }
   }
-  launch_wgrad_reduce<T>(a.partial, rows > 0 ? a.products * used : 0, K, ca, cb, out_transposed, (T*)gw, st);
+  launch_wgrad_reduce<T>(a.partial, rows > 0 ? a.products * a.used : 0, K, ca, cb, out_transposed, (T*)gw, st);
   return check_launch("conv_wgrad_planned");
 }
 

@@ -69,3 +69,33 @@ def test_tile_kernel_weights_off_alignment(dtype):
     off.copy_(w)
     assert w.data_ptr() % 16 == 0 and off.data_ptr() % 16 != 0
     assert torch.equal(_gather(x, plan, w, cout, tr, tr, b, (0, 0), 1.0), _gather(x, plan, off, cout, tr, tr, b, (0, 0), 1.0))
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('ca,cb', [(32, 32), (64, 64), (96, 160), (192, 192), (256, 256), (512, 320)])
+def test_planned_weight_gradient_ranges(dtype, ca, cb):
+  """The planned weight gradient at the edges of its division into ranges: one tile, fewer tiles than XCDs,
+  ranges that do not divide the tiles, more workgroups a range than CUs."""
+  L, P = _lib.lib(), _lib.ptr
+  code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype]
+  for rows, K in ((1, 27), (128, 9), (129, 3), (3 * 128, 27), (11 * 128 + 5, 27), (37 * 128 + 127, 8)):
+    print('planned weight gradient', dtype, ca, cb, 'rows', rows, 'K', K, flush=True)
+    g = torch.Generator().manual_seed(rows + ca)
+    t = (torch.arange(rows)[:, None] + torch.randint(-40, 41, (rows, K), generator=g)).clamp_(0, rows - 1).int()
+    t[torch.rand(rows, K, generator=g) < 0.4] = -1
+    plan = TilePlan(t.cuda())
+    x, grad = torch.randn(rows, ca, generator=g).to(dtype), torch.randn(rows, cb, generator=g).to(dtype)
+    assert _lib.dtype_code(x) == code and L.ocnn_conv_wgrad_planned_supported(code, rows, rows, K, ca, cb, plan.umax)
+    zero = torch.cat([x.double(), torch.zeros(1, ca, dtype=torch.float64)])
+    want = torch.stack([zero[t[:, k].long()].T @ grad.double() for k in range(K)])
+    size = L.ocnn_conv_wgrad_planned_workspace_bytes_for(code, rows, rows, K, ca, cb)
+    ws = torch.empty(size, dtype=torch.uint8, device='cuda')
+    xd, gd = x.cuda(), grad.cuda()
+    for transposed in (0, 1):
+      gw = torch.full((K, cb, ca) if transposed else (K, ca, cb), float('nan'), dtype=dtype, device='cuda')
+      _lib.check(L.ocnn_conv_wgrad_planned(code, P(xd), rows, P(gd), P(plan.loc), P(plan.uptr), P(plan.urows), plan.umax,
+                                           plan.total, rows, K, ca, cb, transposed, P(gw), P(ws), size, _lib.stream()))
+      got = gw.double().cpu()
+      if transposed:
+        got = got.transpose(1, 2)
+      assert (got - want).abs().max() / want.abs().max() < TOL[dtype], (rows, K, transposed)
