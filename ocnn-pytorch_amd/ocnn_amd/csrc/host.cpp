@@ -397,25 +397,6 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
     gamma = as_param(weight);
     beta = as_param(bias);
     if (gamma.defined() && beta.defined() && beta.scalar_type() != gamma.scalar_type()) beta = beta.to(gamma.scalar_type());
-    if (batch_stats) {
-      Tensor stats = at::empty({3, c}, x.options().dtype(at::kFloat));
-      mean = stats[0];
-      invstd = stats[2];
-      Tensor var = stats[1], ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), x);
-      const bool moves = track && running_mean.defined();
-      const bool in_place = moves && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
-                            running_mean.is_contiguous() && running_var.is_contiguous();
-      check(ocnn_batch_norm_stats(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
-                                  (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
-                                  in_place ? running_var.data_ptr() : nullptr,
-                                  in_place ? code_of(running_mean.scalar_type()) : 0, in_place ? (float)factor : 0.f,
-                                  typed<int64_t>(count), ws.data_ptr(), ws.numel(), st));
-      if (moves && !in_place) {
-        Tensor unbiased = var * ((double)rows / (double)std::max<int64_t>(rows - 1, 1));
-        running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
-        running_var.mul_(1 - factor).add_(unbiased.to(running_var.scalar_type()), factor);
-      }
-    }
     y = at::empty_like(x);
     Tensor residual;
     if (residual_in.defined()) {
@@ -424,6 +405,26 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
                   "batch_norm: the residual does not match the input");
     }
     const int pcode = param_code(gamma, beta);
+    if (batch_stats) {
+      Tensor stats = at::empty({3, c}, x.options().dtype(at::kFloat));
+      mean = stats[0];
+      invstd = stats[2];
+      Tensor var = stats[1], ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), x);
+      const bool moves = track && running_mean.defined();
+      const bool in_place = moves && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
+                            running_mean.is_contiguous() && running_var.is_contiguous();
+      check(ocnnx_batch_norm_training(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
+                                      (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
+                                      in_place ? running_var.data_ptr() : nullptr,
+                                      in_place ? code_of(running_mean.scalar_type()) : 0, in_place ? (float)factor : 0.f,
+                                      typed<int64_t>(count), ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(),
+                                      ws.data_ptr(), ws.numel(), st));
+      if (moves && !in_place) {
+        Tensor unbiased = var * ((double)rows / (double)std::max<int64_t>(rows - 1, 1));
+        running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
+        running_var.mul_(1 - factor).add_(unbiased.to(running_var.scalar_type()), factor);
+      }
+    }
     if (!batch_stats && !grad && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
         running_mean.is_contiguous() && running_var.is_contiguous()) {
       check(ocnnx_batch_norm_running(code, ptr(x), rows, (int)c, running_mean.data_ptr(), running_var.data_ptr(),
@@ -434,9 +435,10 @@ Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, 
     if (!batch_stats) {                               // (the backward pass reads mean and invstd)
       mean = running_mean.to(at::kFloat).contiguous();
       invstd = at::rsqrt(running_var.to(at::kFloat) + eps);
+      check(ocnn_batch_norm_apply(code, ptr(x), rows, (int)c, (const float*)mean.data_ptr(),
+                                  (const float*)invstd.data_ptr(), ptr(gamma), ptr(beta), pcode, relu, ptr(residual),
+                                  y.data_ptr(), st));
     }
-    check(ocnn_batch_norm_apply(code, ptr(x), rows, (int)c, (const float*)mean.data_ptr(), (const float*)invstd.data_ptr(),
-                                ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(), st));
   }
   if (grad) {
     auto node = make_node<BatchNormBackward>(inputs);

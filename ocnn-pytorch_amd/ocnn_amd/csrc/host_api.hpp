@@ -40,6 +40,12 @@ int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int
                         int has_plan, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
                         double plan_reuse);
 
+// ocnn_batch_norm_stats and ocnn_batch_norm_apply after each other: one launch where there are few rows.
+int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows, int channels, float eps, float* mean, float* var,
+                              float* invstd, void* running_mean, void* running_var, int running_dtype, float factor,
+                              int64_t* batches_tracked, const void* gamma, const void* beta, int param_dtype, int relu,
+                              const void* residual, void* y, void* workspace, int64_t workspace_bytes, void* stream);
+
 // ocnn_batch_norm_apply with a module's running statistics as it holds them (f32 / f16 / bf16).
 int ocnnx_batch_norm_running(int dtype, const void* x, int64_t rows, int channels, const void* running_mean,
                              const void* running_var, int running_dtype, float eps, const void* gamma, const void* beta,

@@ -403,6 +403,234 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
   }
 }
 
+// ---- few rows: the whole batch norm in one launch ----
+//
+// At a thousand rows (the coarse levels of a network, small clouds) a pass is launch latency, and a training
+// step's forward and backward pass have three launches each (sums, their sum, the elementwise pass).  Here a workgroup of
+// 1024 threads has 64 bytes of every row (kBnSmallLanes threads) to itself: sums, statistics and the
+// elementwise pass follow each other in the workgroup, the rows come from L2 the second time.  Measured, forward +
+// backward (us, three launches each -> one): fp32 337 x 256 21.5 -> 11.6, 1425 x 256 23.3 -> 17.0, 2048 x 256 23.8 -> 20.0,
+// fp16 337 x 256 28.5 -> 15.6, 2048 x 256 29.6 -> 27.1.  On more rows a workgroup reads too much by itself (with 32 bytes
+// of a row 4096 x 128 22.9 -> 29.5), so that is where the line lies.
+constexpr int kBnSmallThreads = 1024, kBnSmallLanes = 4;
+constexpr int64_t kBnSmallRows = 2048;
+
+// sums over the workgroup of the 2 VEC values of each thread, per thread of a row: s_out[kind][channel of the
+// workgroup], in a fixed order: 2 VEC threads' values in fp64, then those sums one after the other.
+template <int VEC>
+__device__ __forceinline__ void bn_small_sums(const float (&s1)[VEC], const float (&s2)[VEC], float* s_f, double* s_d,
+                                              double* s_out) {
+  constexpr int lpr = kBnSmallLanes;
+  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
+  constexpr int pitch = kBnSmallThreads / lpr + 1, sums = 2 * lpr * VEC, segments = kBnSmallThreads / sums;
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) {
+    s_f[(cl * VEC + v) * pitch + rl] = s1[v];
+    s_f[((lpr + cl) * VEC + v) * pitch + rl] = s2[v];
+  }
+  __syncthreads();
+  {
+    const float* p = s_f + (tid % sums) * pitch + tid / sums * (2 * VEC);
+    double a = 0.0;
+#pragma unroll
+    for (int i = 0; i < 2 * VEC; ++i) a += (double)p[i];
+    s_d[tid] = a;
+  }
+  __syncthreads();
+  if (tid < sums) {
+    double a = 0.0;
+#pragma unroll 8
+    for (int i = 0; i < segments; ++i) a += s_d[i * sums + tid];
+    s_out[tid] = a;
+  }
+  __syncthreads();
+}
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(kBnSmallThreads) void bn_small_kernel(
+    const T* __restrict__ x, int rows, int C, float eps, float* __restrict__ mean, float* __restrict__ var,
+    float* __restrict__ invstd, void* running_mean, void* running_var, int rdtype, float factor,
+    long long* batches_tracked, const void* __restrict__ gamma, const void* __restrict__ beta, int pdtype, int relu,
+    const T* __restrict__ res, T* __restrict__ y) {
+  typedef BnVec<T, VEC> V;
+  constexpr int lpr = kBnSmallLanes, rpp = kBnSmallThreads / lpr;
+  __shared__ float s_f[2 * VEC * (kBnSmallThreads + lpr)];
+  __shared__ double s_d[kBnSmallThreads], s_sum[2 * lpr * VEC];
+  __shared__ float s_mean[lpr * VEC], s_is[lpr * VEC];
+  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
+  const int c0 = ((int)blockIdx.x * lpr + cl) * VEC;         // first channel of the thread
+  const bool ok = c0 < C;
+  if (batches_tracked != nullptr && blockIdx.x == 0 && tid == 0) *batches_tracked += 1;
+  float s1[VEC], s2[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
+  if (ok) {
+    const V k = *(const V*)(x + c0);
+    for (int r = rl; r < rows; r += 4 * rpp) {               // (rows past the end repeat row 0, as in bn_stats_kernel)
+      V a[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a[u] = *(const V*)(x + (r + u * rpp < rows ? (int64_t)(r + u * rpp) * C : 0) + c0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) {
+          const float d = to_f32(a[u].v[v]) - to_f32(k.v[v]);
+          s1[v] += d;
+          s2[v] += d * d;
+        }
+    }
+  }
+  bn_small_sums<VEC>(s1, s2, s_f, s_d, s_sum);
+  if (tid < lpr * VEC) {
+    const int c = (int)blockIdx.x * lpr * VEC + tid;
+    if (c < C) {
+      const double m = s_sum[tid] / (double)rows;
+      const double va = fmax(s_sum[lpr * VEC + tid] / (double)rows - m * m, 0.0);
+      const float mf = (float)((double)to_f32(x[c]) + m), isf = (float)(1.0 / sqrt(va + (double)eps));
+      s_mean[tid] = mean[c] = mf;
+      s_is[tid] = invstd[c] = isf;
+      var[c] = (float)va;
+      if (running_mean) {
+        const float unbiased = (float)(va * ((double)rows / (double)max(rows - 1, 1)));
+        bn_store(running_mean, rdtype, c, (1.f - factor) * bn_param(running_mean, rdtype, c, 0.f) + factor * mf);
+        bn_store(running_var, rdtype, c, (1.f - factor) * bn_param(running_var, rdtype, c, 0.f) + factor * unbiased);
+      }
+    }
+  }
+  __syncthreads();
+  if (!ok) return;
+  float m[VEC], sc[VEC], be[VEC];
+  bn_params<VEC>(gamma, beta, pdtype, c0, sc, be);
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) {
+    m[v] = s_mean[cl * VEC + v];
+    sc[v] = s_is[cl * VEC + v] * sc[v];
+  }
+  for (int r = rl; r < rows; r += 4 * rpp) {
+    V a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t at = (int64_t)(r + u * rpp) * C + c0;
+      if (r + u * rpp < rows) {
+        a[u] = *(const V*)(x + at);
+        if (res) b[u] = *(const V*)(res + at);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (r + u * rpp >= rows) continue;
+      V o;
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        float t = (to_f32(a[u].v[v]) - m[v]) * sc[v] + be[v];
+        if (res) t = to_f32(from_f32<T>(t)) + to_f32(b[u].v[v]);
+        if (relu) t = fmaxf(t, 0.f);
+        o.v[v] = from_f32<T>(t);
+      }
+      *(V*)(y + (int64_t)(r + u * rpp) * C + c0) = o;
+    }
+  }
+}
+
+// the gradient, as bn_bwd_stats_kernel, bn_bwd_finish_kernel and bn_bwd_apply_kernel after each other
+template <typename T, int VEC>
+__global__ __launch_bounds__(kBnSmallThreads) void bn_bwd_small_kernel(
+    const T* __restrict__ x, const T* __restrict__ dy, int rows, int C, const float* __restrict__ mean,
+    const float* __restrict__ invstd, const void* __restrict__ gamma, const void* __restrict__ beta, int pdtype, int relu,
+    int training, const T* __restrict__ ymask, float* __restrict__ dbeta, float* __restrict__ dgamma, void* gw, void* gb,
+    T* __restrict__ dres, T* __restrict__ dx) {
+  typedef BnVec<T, VEC> V;
+  constexpr int lpr = kBnSmallLanes, rpp = kBnSmallThreads / lpr;
+  __shared__ float s_f[2 * VEC * (kBnSmallThreads + lpr)];
+  __shared__ double s_d[kBnSmallThreads], s_sum[2 * lpr * VEC];
+  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
+  const int c0 = ((int)blockIdx.x * lpr + cl) * VEC;
+  const bool ok = c0 < C;
+  float s1[VEC], s2[VEC], m[VEC], is[VEC], ga[VEC], be[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
+  if (ok) {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      m[v] = mean[c0 + v];
+      is[v] = invstd[c0 + v];
+    }
+    bn_params<VEC>(gamma, beta, pdtype, c0, ga, be);
+    for (int r = rl; r < rows; r += 2 * rpp) {
+      V a[2], g[2], ym[2];
+      bool in[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        in[u] = r + u * rpp < rows;
+        const int64_t at = (in[u] ? (int64_t)(r + u * rpp) * C : 0) + c0;
+        a[u] = *(const V*)(x + at);
+        g[u] = *(const V*)(dy + at);
+        if (ymask) ym[u] = *(const V*)(ymask + at);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) {
+          const float xc = to_f32(a[u].v[v]) - m[v];
+          const float xh = xc * is[v];
+          float d = in[u] ? to_f32(g[u].v[v]) : 0.f;
+          if (relu && !(ymask ? to_f32(ym[u].v[v]) > 0.f : xc * (is[v] * ga[v]) + be[v] > 0.f)) d = 0.f;
+          s1[v] += d;
+          s2[v] += d * xh;
+        }
+    }
+  }
+  bn_small_sums<VEC>(s1, s2, s_f, s_d, s_sum);
+  if (tid < lpr * VEC) {
+    const int c = (int)blockIdx.x * lpr * VEC + tid;
+    if (c < C) {
+      const float a = (float)s_sum[tid], b = (float)s_sum[lpr * VEC + tid];
+      dbeta[c] = a;
+      dgamma[c] = b;
+      if (gw) bn_store(gw, pdtype, c, b);
+      if (gb) bn_store(gb, pdtype, c, a);
+    }
+  }
+  if (!ok) return;
+  const float inv_n = 1.0f / (float)rows;
+  float db[VEC], dg[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) {
+    db[v] = training ? (float)s_sum[cl * VEC + v] * inv_n : 0.f;
+    dg[v] = training ? (float)s_sum[(lpr + cl) * VEC + v] * inv_n : 0.f;
+    ga[v] *= is[v];
+  }
+  for (int r = rl; r < rows; r += 2 * rpp) {
+    V a[2], g[2], ym[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t at = (int64_t)(r + u * rpp) * C + c0;
+      if (r + u * rpp < rows) {
+        a[u] = *(const V*)(x + at);
+        g[u] = *(const V*)(dy + at);
+        if (ymask) ym[u] = *(const V*)(ymask + at);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (r + u * rpp >= rows) continue;
+      const int64_t at = (int64_t)(r + u * rpp) * C + c0;
+      V o, gr;
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        const float xc = to_f32(a[u].v[v]) - m[v];
+        float d = to_f32(g[u].v[v]);
+        if (relu && !(ymask ? to_f32(ym[u].v[v]) > 0.f : xc * ga[v] + be[v] > 0.f)) d = 0.f;
+        gr.v[v] = from_f32<T>(d);
+        if (training) d = d - db[v] - (xc * is[v]) * dg[v];
+        o.v[v] = from_f32<T>(d * ga[v]);
+      }
+      *(V*)(dx + at) = o;
+      if (dres) *(V*)(dres + at) = gr;
+    }
+  }
+}
+
 }  // namespace ocnn
 
 using namespace ocnn;
@@ -502,6 +730,31 @@ extern "C" int ocnn_batch_norm_apply(int dtype, const void* x, int64_t rows, int
                   0.f, (hipStream_t)stream);
 }
 
+// Training: statistics of the batch (with the running ones moved) and the normalise pass behind them.
+extern "C" int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows, int channels, float eps, float* mean,
+                                         float* var, float* invstd, void* running_mean, void* running_var,
+                                         int running_dtype, float factor, int64_t* batches_tracked, const void* gamma,
+                                         const void* beta, int param_dtype, int relu, const void* residual, void* y,
+                                         void* workspace, int64_t workspace_bytes, void* stream) {
+  OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_training: shape not supported");
+  OCNN_REQUIRE_PTRS("batch_norm_training", x, mean, var, invstd, y, workspace);
+  if (rows > kBnSmallRows) {
+    const int status = ocnn_batch_norm_stats(dtype, x, rows, channels, eps, mean, var, invstd, running_mean, running_var,
+                                             running_dtype, factor, batches_tracked, workspace, workspace_bytes, stream);
+    if (status != OCNN_OK) return status;
+    return bn_apply(dtype, x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, residual, y, nullptr, nullptr,
+                    0, 0.f, (hipStream_t)stream);
+  }
+  OCNN_DISPATCH_DTYPE(dtype, {
+    constexpr int VEC = 16 / sizeof(T);
+    hipLaunchKernelGGL((bn_small_kernel<T, VEC>), dim3((unsigned)cdiv(channels, kBnSmallLanes * VEC)), dim3(kBnSmallThreads), 0,
+                       (hipStream_t)stream, (const T*)x, (int)rows, channels, eps, mean, var, invstd, running_mean,
+                       running_var, running_dtype, factor, (long long*)batches_tracked, gamma, beta, param_dtype, relu,
+                       (const T*)residual, (T*)y);
+  });
+  return check_launch("batch_norm_training");
+}
+
 extern "C" int ocnnx_batch_norm_running(int dtype, const void* x, int64_t rows, int channels, const void* running_mean,
                                         const void* running_var, int running_dtype, float eps, const void* gamma,
                                         const void* beta, int param_dtype, int relu, const void* residual, void* y,
@@ -528,6 +781,16 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
   int nblk;
   int64_t per_a;
   int nblk_a;
+  if (dx && rows <= kBnSmallRows) {
+    OCNN_DISPATCH_DTYPE(dtype, {
+      constexpr int VEC = 16 / sizeof(T);
+      hipLaunchKernelGGL((bn_bwd_small_kernel<T, VEC>), dim3((unsigned)cdiv(channels, kBnSmallLanes * VEC)), dim3(kBnSmallThreads),
+                         0, st, (const T*)x, (const T*)dy, (int)rows, channels, mean, invstd, gamma, beta,
+                         param_dtype, relu, training, (const T*)y, dbeta, dgamma, grad_gamma, grad_beta, (T*)d_residual,
+                         (T*)dx);
+    });
+    return check_launch("batch_norm_backward");
+  }
   bn_blocks(dtype, rows, channels, kBnMaxBlocks, &per, &nblk);
   float* partial = (float*)workspace;
   OCNN_DISPATCH_DTYPE(dtype, {

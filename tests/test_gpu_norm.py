@@ -353,3 +353,40 @@ def test_random_batch_norms_vs_torch():
     assert float((xg.grad.double().cpu() - xd.grad).abs().max()) <= 6 * tol * sc(xd.grad), case
     assert float((bn.weight.grad.double().cpu() - bn64.weight.grad).abs().max()) <= 16 * tol * sc(bn64.weight.grad), case
     assert float((bn.bias.grad.double().cpu() - bn64.bias.grad).abs().max()) <= 6 * tol * sc(bn64.bias.grad), case
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+def test_batch_norm_few_rows(dtype):
+  """The one-launch kernels at the edges of their range (up to 2048 rows; channels that fill no whole
+  workgroup) and the passes of their own just above it, against fp64."""
+  for rows, c in [(33, 8), (64, 32), (255, 40), (256, 1024), (1023, 24), (2048, 96), (2049, 96)]:
+    say('batch norm, few rows', dtype, rows, c)
+    g = torch.Generator().manual_seed(rows)
+    x = (torch.randn(rows, c, generator=g) + 3.0).to(dtype)
+    res, dy = torch.randn(rows, c, generator=g).to(dtype), torch.randn(rows, c, generator=g).to(dtype)
+    bn = BatchNormRelu1d(c, relu=False).to(DEV).to(dtype)
+    with torch.no_grad():
+      bn.weight.copy_(torch.rand(c, generator=g) + 0.5)
+      bn.bias.copy_(torch.randn(c, generator=g) * 0.3)
+    w, b = bn.weight.detach().double().cpu(), bn.bias.detach().double().cpu()
+    for residual in (False, True):
+      xg, rg = x.to(DEV).requires_grad_(), res.to(DEV).requires_grad_()
+      bn.zero_grad()
+      y = bn(xg, residual=rg if residual else None, relu=True)
+      y.backward(dy.to(DEV))
+      mu, var = x.double().mean(0), x.double().var(0, unbiased=False)
+      xhat = (x.double() - mu) / (var + bn.eps).sqrt()
+      z = xhat * w + b + (res.double() if residual else 0)
+      scale = lambda t: max(1.0, float(t.abs().max()))
+      assert float((y.detach().double().cpu() - z.clamp_min(0)).abs().max()) <= 2 * TOL[dtype] * scale(z)
+      # the kernel's own mask: an element at the kink may fall either way
+      d = dy.double() * (y.detach().cpu() > 0)
+      db, dg = d.sum(0), (d * xhat).sum(0)
+      dx = w / (var + bn.eps).sqrt() * (d - db / rows - xhat * dg / rows)
+      assert float((bn.bias.grad.double().cpu() - db).abs().max()) <= 4 * TOL[dtype] * scale(db)
+      assert float((bn.weight.grad.double().cpu() - dg).abs().max()) <= 4 * TOL[dtype] * scale(dg)
+      assert float((xg.grad.double().cpu() - dx).abs().max()) <= 4 * TOL[dtype] * scale(dx)
+      if residual:
+        assert torch.equal(rg.grad.cpu(), d.to(dtype))
+      again = bn(x.to(DEV), residual=res.to(DEV) if residual else None, relu=True)
+      assert torch.equal(again, y)
