@@ -226,11 +226,27 @@ __global__ void pad16_kernel(const u32x4* __restrict__ data, const int32_t* __re
   int64_t q = t / chunks;
   int c = (int)(t % chunks);
   int32_t ch = children[q];
-  if (data == nullptr) {                                   // only the rows of the empty nodes
-    if (ch < 0) out[t] = fill;
-    return;
-  }
   out[t] = ch >= 0 ? data[(int64_t)ch * chunks + c] : fill;
+}
+
+// Only the rows of the empty nodes, in place behind a kernel that wrote the others: a wave looks at 64 nodes (one
+// read of their children), lists the empty ones and writes their rows, 2^shift threads side by side on one.
+// Before, a thread per 16 bytes of every row, set or not, found its node by a 64-bit division: the
+// empty half of 128 channels at depth 7 of eight clouds 32 -> 19 us.
+__global__ __launch_bounds__(256) void pad16_empty_kernel(const int32_t* __restrict__ children, int64_t n, int chunks,
+                                                          int shift, u32x4 fill, u32x4* __restrict__ out) {
+  __shared__ uint8_t s_list[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t first = ((int64_t)blockIdx.x * 4 + wave) * 64;
+  const bool is_empty = first + lane < n && children[first + lane] < 0;
+  const uint64_t empty = __ballot(is_empty);
+  if (is_empty) s_list[wave][__popcll(empty & ((1ull << lane) - 1))] = (uint8_t)lane;
+  __syncthreads();
+  const int count = __popcll(empty), c0 = lane & ((1 << shift) - 1);
+  for (int i = lane >> shift; i < count; i += 64 >> shift) {
+    u32x4* row = out + (first + s_list[wave][i]) * chunks;
+    for (int c = c0; c < chunks; c += 1 << shift) row[c] = fill;
+  }
 }
 
 __global__ void depad16_kernel(const u32x4* __restrict__ data, const int32_t* __restrict__ children,
@@ -534,6 +550,13 @@ extern "C" int ocnn_pad(int dtype, const void* data, const int32_t* children, in
       else { bf16 v = (bf16)val; h = __builtin_bit_cast(unsigned short, v); }
       const unsigned b = (unsigned)h | ((unsigned)h << 16);
       fill = u32x4{b, b, b, b};
+    }
+    if (data == nullptr) {
+      int shift = 0;                                         // threads on a row: enough for it, a wave at most
+      while (shift < 6 && (1 << shift) < chunks) ++shift;
+      hipLaunchKernelGGL(pad16_empty_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, children, n, chunks, shift,
+                         fill, (u32x4*)out);
+      return check_launch("pad");
     }
     hipLaunchKernelGGL(pad16_kernel, dim3(cdiv(n * chunks, 256)), dim3(256), 0, st, (const u32x4*)data,
                        children, n, chunks, fill, (u32x4*)out);

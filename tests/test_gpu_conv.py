@@ -1944,3 +1944,22 @@ def test_the_documented_call_sequence_of_the_abi():
   ws3 = torch.empty(L.ocnn_conv_wgrad_workspace_bytes_for(code, rows_in, rows, K, 96, 96), dtype=torch.uint8, device=DEV)
   _lib.check(L.ocnn_conv_wgrad(code, P(x), rows_in, P(gr), P(table), rows, K, 96, 96, 0, P(want), P(ws3), ws3.numel(), st))
   assert rel_err(gw, f64(want)) < 1e-2
+
+
+@pytest.mark.parametrize('dtype,channels', [(torch.float16, 8), (torch.float16, 24), (torch.float32, 64), (torch.bfloat16, 128),
+                                            (torch.float32, 260), (torch.float32, 600)])
+def test_pad_empty_rows_only(dtype, channels):
+  """ocnn_pad without data writes the rows of the empty nodes and nothing else."""
+  L, P = _lib.lib(), _lib.ptr
+  code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype]
+  for n in (1, 63, 64, 65, 255, 257, 5000):
+    for share in (0.0, 0.5, 1.0):
+      g = torch.Generator().manual_seed(n)
+      empty = torch.rand(n, generator=g) < share
+      children = torch.where(empty, -1, torch.arange(n)).int().cuda()
+      out = torch.randn(n + 2, channels, generator=g).to(dtype)
+      want = out.clone()
+      want[1:-1][empty] = 1.5
+      out = out.cuda()
+      _lib.check(L.ocnn_pad(code, None, P(children), n, channels, 1.5, P(out[1:]), _lib.stream()))
+      assert torch.equal(out.cpu(), want), (n, share)
