@@ -4,6 +4,7 @@ There is no CPU fallback: if the library cannot be loaded the package raises.
 """
 
 import ctypes
+import functools
 import importlib.util
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_void_p, POINTER
 
@@ -166,6 +167,30 @@ def native():
     spec.loader.exec_module(module)
     _native = module
   return _native
+
+
+def recorded():
+  """True where a call has to be an autograd.Function because something looks on: torch.jit.trace records
+  a Function as one Python operation, but of a native call (native().conv, ...) only the torch operations
+  inside, that is an empty tensor."""
+  return torch.jit.is_tracing()
+
+
+def unrecorded(make):
+  """For what a layer's first call makes and keeps (tables, plans, passes): no part of a trace, which
+  would hand out values of its own in place of sizes."""
+  @functools.wraps(make)
+  def call(*args, **kwargs):
+    if not torch.jit.is_tracing():
+      return make(*args, **kwargs)
+    state = torch._C._get_tracing_state()
+    torch._C._set_tracing_state(None)
+    try:
+      return make(*args, **kwargs)
+    finally:
+      torch._C._set_tracing_state(state)
+
+  return call
 
 
 class OcnnHipError(RuntimeError):

@@ -14,6 +14,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <array>
 #include <memory>
 #include <optional>
 #include <vector>
@@ -148,7 +149,10 @@ struct GatherOp {
         check(ocnn_conv_gather(code, ptr(data), rows_in, typed<int32_t>(table), rows, K, ptr(W), cin, cout, transposed,
                                reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
     }
-    if (overflow) out.index_copy_(0, overflow_rows, overflow->run(data, overflow_table, W, bias));
+    if (overflow) {
+      at::tracer::impl::NoTracerDispatchMode quiet;          // (a trace must not own the plan's tensors)
+      out.index_copy_(0, overflow_rows, overflow->run(data, overflow_table, W, bias));
+    }
     return followed(view_cols ? out.view({-1, view_cols}) : out, bn);
   }
 
@@ -332,42 +336,59 @@ int param_code(const Tensor& gamma, const Tensor& beta) {
   return t.defined() ? code_of(t.scalar_type()) : OCNN_F32;
 }
 
+// What the backward pass reads, and how the forward pass was taken.
+struct BatchNormCall {
+  Tensor x, mean, invstd, gamma, beta, y;     // (y: only where the ReLU's mask is not a function of x alone)
+  bool relu = false, training = false, has_residual = false;
+  at::ScalarType wdtype = at::kFloat, bdtype = at::kFloat;
+};
+
+// Gradients of x, weight, bias and residual, those of them that `want` names.
+std::array<Tensor, 4> batch_norm_grads(const BatchNormCall& call, const Tensor& dy, std::array<bool, 4> want) {
+  const Tensor &xs = call.x, &ga = call.gamma, &be = call.beta;
+  const int64_t rows = xs.size(0), c = xs.size(1);
+  const auto f32 = xs.options().dtype(at::kFloat);
+  Tensor sums = at::empty({2, c}, f32);                     // dgamma, dbeta
+  const bool want_res = call.has_residual && want[3];
+  Tensor dx, dres, gw, gb;
+  if (want[0] || want_res) dx = at::empty_like(xs);
+  if (want_res) dres = at::empty_like(xs);
+  // the parameter gradients come out in the parameters' dtype where the kernels hold it
+  const bool want_w = ga.defined() && want[1], want_b = be.defined() && want[2];
+  if (want_w && call.wdtype == ga.scalar_type()) gw = at::empty({c}, ga.options());
+  if (want_b && call.bdtype == be.scalar_type() && (!ga.defined() || be.scalar_type() == ga.scalar_type()))
+    gb = at::empty({c}, be.options());
+  Tensor ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), xs);
+  float* s = (float*)sums.data_ptr();
+  check(ocnn_batch_norm_backward(code_of(xs.scalar_type()), ptr(xs), ptr(dy), rows, (int)c, (const float*)ptr(call.mean),
+                                 (const float*)ptr(call.invstd), ptr(ga), ptr(be), param_code(ga, be), call.relu,
+                                 call.training, ptr(call.y), typed<void>(dx), typed<void>(dres), s, s + c, typed<void>(gw),
+                                 typed<void>(gb), ws.data_ptr(), ws.numel(), hip_stream()));
+  if (want_w && !gw.defined()) gw = sums[0].to(call.wdtype);
+  if (want_b && !gb.defined()) gb = sums[1].to(call.bdtype);
+  return {want[0] ? dx : Tensor(), gw, gb, dres};
+}
+
 struct BatchNormBackward : public Node {
   SavedVariable x, mean, invstd, gamma, beta, y;
-  bool relu = false, training = false, has_residual = false, keeps_y = false;
-  at::ScalarType wdtype = at::kFloat, bdtype = at::kFloat;
+  BatchNormCall call;                         // (its flags; the tensors are the saved ones)
+  bool keeps_y = false;
 
   variable_list apply(variable_list&& grads) override {
     variable_list out(4);
     if (!grads[0].defined()) return out;
-    Tensor dy = grads[0].contiguous(), xs = x.unpack(), mu = mean.unpack(), is = invstd.unpack();
-    Tensor ga = gamma.unpack(), be = beta.unpack(), ys;
-    if (keeps_y) ys = y.unpack(shared_from_this());
+    Tensor dy = grads[0].contiguous();
+    BatchNormCall now = call;
+    now.x = x.unpack();
+    now.mean = mean.unpack();
+    now.invstd = invstd.unpack();
+    now.gamma = gamma.unpack();
+    now.beta = beta.unpack();
+    if (keeps_y) now.y = y.unpack(shared_from_this());
     at::AutoDispatchBelowADInplaceOrView below;
-    const int64_t rows = xs.size(0), c = xs.size(1);
-    const auto f32 = xs.options().dtype(at::kFloat);
-    Tensor sums = at::empty({2, c}, f32);                     // dgamma, dbeta
-    const bool want_res = has_residual && task_should_compute_output(3);
-    Tensor dx, dres, gw, gb;
-    if (task_should_compute_output(0) || want_res) dx = at::empty_like(xs);
-    if (want_res) dres = at::empty_like(xs);
-    // the parameter gradients come out in the parameters' dtype where the kernels hold it
-    const bool want_w = ga.defined() && task_should_compute_output(1), want_b = be.defined() && task_should_compute_output(2);
-    if (want_w && wdtype == ga.scalar_type()) gw = at::empty({c}, ga.options());
-    if (want_b && bdtype == be.scalar_type() && (!ga.defined() || be.scalar_type() == ga.scalar_type()))
-      gb = at::empty({c}, be.options());
-    Tensor ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), xs);
-    float* s = (float*)sums.data_ptr();
-    check(ocnn_batch_norm_backward(code_of(xs.scalar_type()), ptr(xs), ptr(dy), rows, (int)c, (const float*)ptr(mu),
-                                   (const float*)ptr(is), ptr(ga), ptr(be), param_code(ga, be), relu, training, ptr(ys),
-                                   typed<void>(dx), typed<void>(dres), s, s + c, typed<void>(gw), typed<void>(gb),
-                                   ws.data_ptr(), ws.numel(), hip_stream()));
-    if (want_w && !gw.defined()) gw = sums[0].to(wdtype);
-    if (want_b && !gb.defined()) gb = sums[1].to(bdtype);
-    if (task_should_compute_output(0)) out[0] = dx;
-    out[1] = gw;
-    out[2] = gb;
-    out[3] = dres;
+    auto g = batch_norm_grads(now, dy, {task_should_compute_output(0), task_should_compute_output(1),
+                                        task_should_compute_output(2), task_should_compute_output(3)});
+    for (int i = 0; i < 4; ++i) out[i] = g[i];
     return out;
   }
   void release_variables() override {
@@ -380,79 +401,83 @@ bool known_type(const Tensor& t) {
   return t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16;
 }
 
-// batch_stats: statistics of this batch (and, with track, the running ones moved by `factor`);
-// otherwise the running statistics.  count: num_batches_tracked, incremented with the statistics.
-Tensor batch_norm(const Tensor& x_in, const Tensor& weight, const Tensor& bias, const Tensor& running_mean,
-                  const Tensor& running_var, const Tensor& count, bool batch_stats, bool track, double factor, double eps,
-                  bool relu, const Tensor& residual_in) {
-  const variable_list inputs{x_in, weight, bias, residual_in};
-  const bool grad = any_requires_grad(inputs);
-  Tensor x, mean, invstd, gamma, beta, y;
-  {
-    at::AutoDispatchBelowADInplaceOrView below;
-    x = x_in.contiguous();
-    const int64_t rows = x.size(0), c = x.size(1);
-    const int code = code_of(x.scalar_type());
-    void* st = hip_stream();
-    gamma = as_param(weight);
-    beta = as_param(bias);
-    if (gamma.defined() && beta.defined() && beta.scalar_type() != gamma.scalar_type()) beta = beta.to(gamma.scalar_type());
-    y = at::empty_like(x);
-    Tensor residual;
-    if (residual_in.defined()) {
-      residual = residual_in.contiguous();
-      TORCH_CHECK(residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type(),
-                  "batch_norm: the residual does not match the input");
-    }
-    const int pcode = param_code(gamma, beta);
-    if (batch_stats) {
-      Tensor stats = at::empty({3, c}, x.options().dtype(at::kFloat));
-      mean = stats[0];
-      invstd = stats[2];
-      Tensor var = stats[1], ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), x);
-      const bool moves = track && running_mean.defined();
-      const bool in_place = moves && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
-                            running_mean.is_contiguous() && running_var.is_contiguous();
-      check(ocnnx_batch_norm_training(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
-                                      (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
-                                      in_place ? running_var.data_ptr() : nullptr,
-                                      in_place ? code_of(running_mean.scalar_type()) : 0, in_place ? (float)factor : 0.f,
-                                      typed<int64_t>(count), ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(),
-                                      ws.data_ptr(), ws.numel(), st));
-      if (moves && !in_place) {
-        Tensor unbiased = var * ((double)rows / (double)std::max<int64_t>(rows - 1, 1));
-        running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
-        running_var.mul_(1 - factor).add_(unbiased.to(running_var.scalar_type()), factor);
-      }
-    }
-    if (!batch_stats && !grad && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
-        running_mean.is_contiguous() && running_var.is_contiguous()) {
-      check(ocnnx_batch_norm_running(code, ptr(x), rows, (int)c, running_mean.data_ptr(), running_var.data_ptr(),
-                                     code_of(running_mean.scalar_type()), (float)eps, ptr(gamma), ptr(beta), pcode, relu,
-                                     ptr(residual), y.data_ptr(), st));
-      return y;
-    }
-    if (!batch_stats) {                               // (the backward pass reads mean and invstd)
-      mean = running_mean.to(at::kFloat).contiguous();
-      invstd = at::rsqrt(running_var.to(at::kFloat) + eps);
-      check(ocnn_batch_norm_apply(code, ptr(x), rows, (int)c, (const float*)mean.data_ptr(),
-                                  (const float*)invstd.data_ptr(), ptr(gamma), ptr(beta), pcode, relu, ptr(residual),
-                                  y.data_ptr(), st));
-    }
+// The result, and in `call` what the backward pass reads.  batch_stats: statistics of this batch (and,
+// with track, the running ones moved by `factor`); otherwise the running statistics.  count:
+// num_batches_tracked, incremented with the statistics.  backward: a backward pass follows.
+Tensor batch_norm_pass(const Tensor& x_in, const Tensor& weight, const Tensor& bias, const Tensor& running_mean,
+                       const Tensor& running_var, const Tensor& count, bool batch_stats, bool track, double factor, double eps,
+                       bool relu, const Tensor& residual_in, bool backward, BatchNormCall* call) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor x = x_in.contiguous();
+  const int64_t rows = x.size(0), c = x.size(1);
+  const int code = code_of(x.scalar_type());
+  void* st = hip_stream();
+  Tensor gamma = as_param(weight), beta = as_param(bias), mean, invstd;
+  if (gamma.defined() && beta.defined() && beta.scalar_type() != gamma.scalar_type()) beta = beta.to(gamma.scalar_type());
+  Tensor y = at::empty_like(x), residual;
+  if (residual_in.defined()) {
+    residual = residual_in.contiguous();
+    TORCH_CHECK(residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type(),
+                "batch_norm: the residual does not match the input");
   }
+  const int pcode = param_code(gamma, beta);
+  if (batch_stats) {
+    Tensor stats = at::empty({3, c}, x.options().dtype(at::kFloat));
+    mean = stats[0];
+    invstd = stats[2];
+    Tensor var = stats[1], ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), x);
+    const bool moves = track && running_mean.defined();
+    const bool in_place = moves && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
+                          running_mean.is_contiguous() && running_var.is_contiguous();
+    check(ocnnx_batch_norm_training(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
+                                    (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
+                                    in_place ? running_var.data_ptr() : nullptr,
+                                    in_place ? code_of(running_mean.scalar_type()) : 0, in_place ? (float)factor : 0.f,
+                                    typed<int64_t>(count), ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(),
+                                    ws.data_ptr(), ws.numel(), st));
+    if (moves && !in_place) {
+      Tensor unbiased = var * ((double)rows / (double)std::max<int64_t>(rows - 1, 1));
+      running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
+      running_var.mul_(1 - factor).add_(unbiased.to(running_var.scalar_type()), factor);
+    }
+  } else if (!backward && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
+             running_mean.is_contiguous() && running_var.is_contiguous()) {
+    check(ocnnx_batch_norm_running(code, ptr(x), rows, (int)c, running_mean.data_ptr(), running_var.data_ptr(),
+                                   code_of(running_mean.scalar_type()), (float)eps, ptr(gamma), ptr(beta), pcode, relu,
+                                   ptr(residual), y.data_ptr(), st));
+  } else {                                            // (the backward pass reads mean and invstd)
+    mean = running_mean.to(at::kFloat).contiguous();
+    invstd = at::rsqrt(running_var.to(at::kFloat) + eps);
+    check(ocnn_batch_norm_apply(code, ptr(x), rows, (int)c, (const float*)mean.data_ptr(), (const float*)invstd.data_ptr(),
+                                ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(), st));
+  }
+  if (backward) {
+    *call = {x, mean, invstd, gamma, beta, residual_in.defined() && relu ? y : Tensor(), relu, batch_stats,
+             residual_in.defined()};
+    if (weight.defined()) call->wdtype = weight.scalar_type();
+    if (bias.defined()) call->bdtype = bias.scalar_type();
+  }
+  return y;
+}
+
+Tensor batch_norm(const Tensor& x, const Tensor& weight, const Tensor& bias, const Tensor& running_mean,
+                  const Tensor& running_var, const Tensor& count, bool batch_stats, bool track, double factor, double eps,
+                  bool relu, const Tensor& residual) {
+  const variable_list inputs{x, weight, bias, residual};
+  const bool grad = any_requires_grad(inputs);
+  BatchNormCall call;
+  Tensor y = batch_norm_pass(x, weight, bias, running_mean, running_var, count, batch_stats, track, factor, eps, relu, residual,
+                             grad, &call);
   if (grad) {
     auto node = make_node<BatchNormBackward>(inputs);
-    node->relu = relu;
-    node->training = batch_stats;
-    node->has_residual = residual_in.defined();
-    node->keeps_y = node->has_residual && relu;   // with a residual the ReLU's mask is not a function of x alone
-    if (weight.defined()) node->wdtype = weight.scalar_type();
-    if (bias.defined()) node->bdtype = bias.scalar_type();
-    node->x = SavedVariable(x, false);
-    node->mean = SavedVariable(mean, false);
-    node->invstd = SavedVariable(invstd, false);
-    if (gamma.defined()) node->gamma = SavedVariable(gamma, false);
-    if (beta.defined()) node->beta = SavedVariable(beta, false);
+    node->keeps_y = call.y.defined();
+    node->x = SavedVariable(call.x, false);
+    node->mean = SavedVariable(call.mean, false);
+    node->invstd = SavedVariable(call.invstd, false);
+    if (call.gamma.defined()) node->gamma = SavedVariable(call.gamma, false);
+    if (call.beta.defined()) node->beta = SavedVariable(call.beta, false);
+    call.x = call.mean = call.invstd = call.gamma = call.beta = call.y = Tensor();
+    node->call = std::move(call);
     torch::autograd::set_history(y, node);
     if (node->keeps_y) node->y = SavedVariable(y, true);
   }
@@ -708,6 +733,28 @@ PYBIND11_MODULE(ocnn_host, m) {
   m.def("conv", &conv, py::call_guard<py::gil_scoped_release>());
   m.def("conv_bn", &conv_bn, py::call_guard<py::gil_scoped_release>());
   m.def("column_sum", &column_sum, py::call_guard<py::gil_scoped_release>());
+  // (the two passes without an autograd node, for an autograd.Function around them)
+  m.def(
+      "batch_norm_pass",
+      [](const Tensor& x, const OptTensor& w, const OptTensor& b, const OptTensor& rm, const OptTensor& rv,
+         const OptTensor& count, bool batch_stats, bool track, double factor, double eps, bool relu, const OptTensor& res) {
+        BatchNormCall call;
+        Tensor y = batch_norm_pass(x, or_undefined(w), or_undefined(b), or_undefined(rm), or_undefined(rv),
+                                   or_undefined(count), batch_stats, track, factor, eps, relu, or_undefined(res), true, &call);
+        return std::vector<Tensor>{y, call.x, call.mean, call.invstd, call.gamma, call.beta};
+      },
+      py::call_guard<py::gil_scoped_release>());
+  m.def(
+      "batch_norm_grads",
+      [](const Tensor& dy, const Tensor& x, const Tensor& mean, const Tensor& invstd, const OptTensor& gamma,
+         const OptTensor& beta, const OptTensor& y, bool relu, bool training, bool has_residual, at::ScalarType wdtype,
+         at::ScalarType bdtype, std::array<bool, 4> want) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const auto g = batch_norm_grads({x, mean, invstd, or_undefined(gamma), or_undefined(beta), or_undefined(y), relu,
+                                         training, has_residual, wdtype, bdtype}, dy.contiguous(), want);
+        return std::vector<Tensor>(g.begin(), g.end());
+      },
+      py::call_guard<py::gil_scoped_release>());
   m.def(
       "batch_norm",
       [](const Tensor& x, const OptTensor& w, const OptTensor& b, const OptTensor& rm, const OptTensor& rv,

@@ -11,7 +11,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from .nn import OctreeConv, OctreeDeconv
-from .nn.octree_conv import _gather_op, _wgrad_op, conv_wgrad, column_sum
+from .nn.octree_conv import _gather_op, _wgrad_op, call_native, conv_wgrad, column_sum
 from .nn.batchnorm import BatchNormRelu1d
 
 
@@ -39,7 +39,7 @@ def layer_bn(layer, bn, data, *args, residual=None, relu=None):
   """bn(layer(data, *args), residual, relu).  In evaluation without gradients, with the layer and the
   batch norm of this package as they are, one native call: the normalisation then rides on the
   convolution's own pass over its result instead of reading and writing it once more."""
-  if (not torch.is_grad_enabled() and type(bn) is BatchNormRelu1d and not bn.training and
+  if (not torch.is_grad_enabled() and not _lib.recorded() and type(bn) is BatchNormRelu1d and not bn.training and
       bn.running_mean is not None and type(layer) in (OctreeConv, OctreeDeconv, Conv1x1) and not _hooked(layer, bn)):
     native = layer.native_layer(data, *args)
     if native is not None and _lib.lib().ocnn_batch_norm_supported(_lib.DTYPE_CODE[data.dtype], 2, bn.num_features):
@@ -95,6 +95,7 @@ def _identity_table(rows, device):
 _LINEAR = {}
 
 
+@_lib.unrecorded
 def _rows_linear_layer(x, cin, cout):
   """y = x W^T on many rows as the one-slot form of the convolution kernels (weights (out, in) as
   torch.nn.Linear holds them)."""
@@ -161,7 +162,7 @@ class Conv1x1(torch.nn.Module):
     lin = self.linear
     native = self.native_layer(data)
     if native is not None:
-      return _lib.native().conv(native, data, lin.weight, lin.bias)
+      return call_native(native, data, lin.weight, lin.bias)
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 65536 and lin.in_features % 32 == 0 and lin.out_features < 16):
       return _RowsLinearNarrow.apply(data, lin.weight, lin.bias)

@@ -9,6 +9,24 @@ import torch.nn
 from .. import _lib
 
 
+class _BatchNormFunction(torch.autograd.Function):
+  """The module's pass as an autograd.Function, for calls that something records (_lib.recorded)."""
+
+  @staticmethod
+  def forward(ctx, x, weight, bias, residual, running_mean, running_var, counter, use_batch_stats, track, factor, eps, relu):
+    y, *saved = _lib.native().batch_norm_pass(x, weight, bias, running_mean, running_var, counter, use_batch_stats, track,
+                                              factor, eps, relu, residual)
+    ctx.save_for_backward(*saved, y if residual is not None and relu else None)
+    dtypes = [torch.float32 if p is None else p.dtype for p in (weight, bias)]
+    ctx.how = (relu, use_batch_stats, residual is not None, *dtypes)
+    return y
+
+  @staticmethod
+  def backward(ctx, dy):
+    grads = _lib.native().batch_norm_grads(dy, *ctx.saved_tensors, *ctx.how, ctx.needs_input_grad[:4])
+    return (*grads,) + (None,) * 8
+
+
 class BatchNormRelu1d(torch.nn.BatchNorm1d):
   """BatchNorm1d [+ ReLU] in one pass over (rows, C) inputs on the GPU.  Inputs the kernels do
   not take (3-D, channel counts that are not a multiple of 16 bytes, a single row, tensors
@@ -42,9 +60,11 @@ class BatchNormRelu1d(torch.nn.BatchNorm1d):
     use_batch_stats = self.training or (self.running_mean is None and self.running_var is None)
     track = self.training and self.track_running_stats
     running = not use_batch_stats or track
-    return _lib.native().batch_norm(input, self.weight, self.bias, self.running_mean if running else None,
-                                    self.running_var if running else None, counter, use_batch_stats, track,
-                                    factor if track else 0.0, self.eps, relu, residual)
+    stats = (self.running_mean, self.running_var) if running else (None, None)
+    how = (counter, use_batch_stats, track, factor if track else 0.0, self.eps, relu)
+    if _lib.recorded():
+      return _BatchNormFunction.apply(input, self.weight, self.bias, residual, *stats, *how)
+    return _lib.native().batch_norm(input, self.weight, self.bias, *stats, *how, residual)
 
   def extra_repr(self) -> str:
     return super().extra_repr() + ', relu={}'.format(self.fused_relu)

@@ -23,7 +23,7 @@ from ..octree.contract import tables_of
 from ..octree.octree import Octree
 from ..utils import list2str, resize_with_last_val, xavier_uniform_
 from .octree2col import col2octree, octree2col
-from .octree_pad import _depad_raw, _pad_raw, octree_depad, octree_pad
+from .octree_pad import _depad_raw, _pad_raw, _rows, octree_depad, octree_pad
 
 
 # (thresholds of the kernel selection live in the library, csrc/select.hip; these are the ones
@@ -290,6 +290,7 @@ class OctreeConvBase:
   def is_conv_layer(self):
     raise NotImplementedError
 
+  @_lib.unrecorded
   def setup(self, octree, depth: int):
     """Heights of input/output and the table (ocnn/nn/octree_conv.py:51-100)."""
     # (an octree of another class gets its tables from its public members, octree/contract.py)
@@ -361,6 +362,7 @@ class OctreeConvBase:
     return cache[key]
 
   # The three passes as (native pass, table).  None: not one pass; the *_gemm methods put it together.
+  @_lib.unrecorded
   def forward_op(self, dtype, pad_to=None):
     """(fine rows, in_conv) -> (table rows, out_conv); see forward_gemm."""
     if self.dense_children:
@@ -374,6 +376,7 @@ class OctreeConvBase:
     plan = self._plan(dtype, self.fine_h, self.in_conv, self.out_conv)
     return _gather_op(dtype, self.fine_h, rows, K, self.in_conv, self.out_conv, False, False, plan), self.neigh
 
+  @_lib.unrecorded
   def backward_op(self, dtype, coarse_index=None, coarse_rows=0):
     """(table rows, out_conv) -> (fine rows, in_conv); see backward_gemm."""
     rows, K = self.neigh.shape
@@ -394,6 +397,7 @@ class OctreeConvBase:
     return (_gather_op(dtype, rows, self.fine_h, K, self.out_conv, self.in_conv, True, False, plan),
             self._inverse_table())
 
+  @_lib.unrecorded
   def weight_op(self, dtype, out_transposed=False, coarse_index=None, coarse_rows=0):
     """data (fine rows), grad (table rows) -> (K, in_conv, out_conv); see weight_gemm."""
     rows, K = self.neigh.shape
@@ -584,7 +588,7 @@ class OctreeDeconvFunction(Function):
     index = None
     data = data.contiguous()
     if padded:
-      assert tuple(data.shape) == (int(octree.nnum[depth]), in_channels), 'The shape of input data is wrong'
+      assert tuple(data.shape) == (_rows(octree, depth)[0], in_channels), 'The shape of input data is wrong'
       if eng.dense_children:
         index = octree._nempty_index32(depth)                   # the dense kernels read through it
       else:
@@ -613,6 +617,32 @@ class OctreeDeconvFunction(Function):
     grad_w = eng.weight_gemm(grad, data, coarse_index=index) if ctx.needs_input_grad[1] else None
     grad_b = column_sum(grad) if ctx.needs_input_grad[10] else None
     return (grad_out, grad_w) + (None,) * 8 + (grad_b, None)
+
+
+class _NativeLayerFunction(Function):
+  """A layer's native passes as an autograd.Function, for calls that something records (_lib.recorded)."""
+
+  @staticmethod
+  def forward(ctx, data, weights, bias, native):
+    data, weights = data.contiguous(), weights.to(data.dtype).contiguous()
+    ctx.save_for_backward(data, weights)
+    ctx.native = native
+    return native.fwd.run(data, native.fwd_table, weights, bias)
+
+  @staticmethod
+  def backward(ctx, grad):
+    (data, weights), native, grad = ctx.saved_tensors, ctx.native, grad.contiguous()
+    x, g = (grad, data) if native.wgrad_of_grad else (data, grad)
+    return (native.dgrad.run(grad, native.dgrad_table, weights, None) if ctx.needs_input_grad[0] else None,
+            native.wgrad.run(x, g, native.wgrad_table) if ctx.needs_input_grad[1] else None,
+            column_sum(grad) if ctx.needs_input_grad[2] else None, None)
+
+
+def call_native(native, data, weights, bias):
+  """A layer through its native passes (those that the call needs)."""
+  if _lib.recorded():
+    return _NativeLayerFunction.apply(data, weights, bias, native)
+  return _lib.native().conv(native, data, weights, bias)
 
 
 class _Layer:
@@ -644,12 +674,14 @@ class _Layer:
       return eng.forward_op(self.dtype, (eng.octree, self.pad_depth) if self.padded else None)
     return eng.backward_op(self.dtype, *self._coarse(eng.octree))
 
+  @_lib.unrecorded
   def make_dgrad(self, eng):
     made = self._pass(eng, False)
     self.dgrad = made is not None
     if made is not None:
       self.native.dgrad, self.native.dgrad_table = made
 
+  @_lib.unrecorded
   def make_wgrad(self, eng):
     made = eng.weight_op(self.dtype, False, *self._coarse(eng.octree))
     self.wgrad = made is not None
@@ -657,6 +689,7 @@ class _Layer:
       self.native.wgrad, self.native.wgrad_table = made
 
 
+@_lib.unrecorded
 def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
   """The layer's native passes, made at its first call on this octree and kept with it: (layer or
   None where the forward pass is not one native pass, function that makes its engine)."""
@@ -666,6 +699,7 @@ def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_siz
          SPARSE_MIN_ROWS)
   layer = octree._layers.get(key)
 
+  @_lib.unrecorded
   def made_engine():
     eng = engine(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
     eng.setup(octree, depth)
@@ -700,7 +734,7 @@ def _apply(engine, function, data, weights, octree, depth, in_channels, out_chan
           layer.make_wgrad(made_engine())
         ok = layer.wgrad
     if ok:
-      return _lib.native().conv(layer.native, data, weights, bias)
+      return call_native(layer.native, data, weights, bias)
   return function.apply(data, weights, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
                         max_buffer, bias, padded)
 

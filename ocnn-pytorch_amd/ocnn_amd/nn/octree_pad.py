@@ -13,12 +13,19 @@ def _children32(octree, depth):
   return children if children.dtype == torch.int32 and children.is_contiguous() else children.int().contiguous()
 
 
+@_lib.unrecorded
+def _rows(octree, depth):
+  """(all nodes, non-empty nodes) of a layer."""
+  return int(octree.nnum[depth]), int(octree.nnum_nempty[depth])
+
+
 def _pad_raw(data: torch.Tensor, octree, depth: int, val: float = 0.0):
   children = _children32(octree, depth)
   _lib.require_gpu(data, children)
   data = data.contiguous()
-  assert data.shape[0] == int(octree.nnum_nempty[depth]), 'octree_pad: wrong number of rows'
-  n, c = int(octree.nnum[depth]), data.shape[1]
+  n, filled = _rows(octree, depth)
+  assert data.shape[0] == filled, 'octree_pad: wrong number of rows'
+  c = data.shape[1]
   out = torch.empty((n, c), dtype=data.dtype, device=data.device)
   _lib.check(_lib.lib().ocnn_pad(_lib.dtype_code(data), _lib.ptr(data), _lib.ptr(children), n, c,
                                  float(val), _lib.ptr(out), _lib.stream()))
@@ -29,9 +36,10 @@ def _depad_raw(data: torch.Tensor, octree, depth: int):
   children = _children32(octree, depth)
   _lib.require_gpu(data, children)
   data = data.contiguous()
-  assert data.shape[0] == int(octree.nnum[depth]), 'octree_depad: wrong number of rows'
-  n, c = data.shape[0], data.shape[1]
-  out = torch.empty((int(octree.nnum_nempty[depth]), c), dtype=data.dtype, device=data.device)
+  n, filled = _rows(octree, depth)
+  assert data.shape[0] == n, 'octree_depad: wrong number of rows'
+  c = data.shape[1]
+  out = torch.empty((filled, c), dtype=data.dtype, device=data.device)
   _lib.check(_lib.lib().ocnn_depad(_lib.dtype_code(data), _lib.ptr(data), _lib.ptr(children), n, c,
                                    _lib.ptr(out), _lib.stream()))
   return out
