@@ -9,6 +9,7 @@ import importlib.util
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_void_p, POINTER
 
 import torch
+import torch.autograd.forward_ad
 
 from . import build as _build
 
@@ -170,17 +171,22 @@ def native():
 
 
 def recorded():
-  """True where a call has to be an autograd.Function because something looks on: torch.jit.trace records
+  """True where a call has to be an autograd.Function because something looks on.  torch.jit.trace records
   a Function as one Python operation, but of a native call (native().conv, ...) only the torch operations
-  inside, that is an empty tensor."""
-  return torch.jit.is_tracing()
+  inside, that is an empty tensor.  Forward-mode differentiation and the transforms of torch.func are refused
+  by a Function that does not provide for them; a native call would drop the tangents."""
+  return (torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0 or
+          torch._C._are_functorch_transforms_active())
 
 
 def unrecorded(make):
   """For what a layer's first call makes and keeps (tables, plans, passes): no part of a trace, which
-  would hand out values of its own in place of sizes."""
+  would hand out values of its own in place of sizes, and not under a transform of torch.func, which would
+  wrap the tensors that are kept."""
   @functools.wraps(make)
   def call(*args, **kwargs):
+    if torch._C._are_functorch_transforms_active():
+      raise RuntimeError('ocnn_amd layers are autograd.Functions that the transforms of torch.func do not support')
     if not torch.jit.is_tracing():
       return make(*args, **kwargs)
     state = torch._C._get_tracing_state()

@@ -1,10 +1,13 @@
-"""The layers' native nodes under the parts of torch that look on: torch.jit.trace."""
+"""The layers' native nodes under the parts of torch that look on: torch.jit.trace, forward-mode differentiation
+and the transforms of torch.func."""
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 from ocnn_amd import synthetic
-from ocnn_amd.modules import Conv1x1BnRelu, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
+from ocnn_amd.modules import BatchNormRelu1d, Conv1x1, Conv1x1BnRelu, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
+from ocnn_amd.nn import OctreeConv, OctreeDeconv
 from ocnn_amd.octree import Octree, Points
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +72,40 @@ def test_traced_network(dtype, training):
       assert torch.equal(got, want)
     else:
       assert (got.double() - want.double()).abs().max() < 6 * EVAL_TOL[dtype] * want.double().abs().max()
+
+
+def _layers(octree):
+  """Each kind of native node alone: (module, further arguments)."""
+  torch.manual_seed(0)
+  return [(OctreeConv(32, 32, use_bias=True), (octree, DEPTH)), (OctreeDeconv(32, 32), (octree, DEPTH)),
+          (Conv1x1(32, 16), ()), (BatchNormRelu1d(32, relu=True), ()), (OctreeConvBnRelu(32, 32), (octree, DEPTH))]
+
+
+@pytest.mark.parametrize('training', [False, True])
+def test_forward_mode_is_refused(training):
+  """No derivative of the layers in forward mode: a call on a dual tensor is an error, not a value without a
+  tangent; a call without one gives what it gives outside."""
+  octree = _octree()
+  for module, args in _layers(octree):
+    module = module.to('cuda', torch.float16).train(training)
+    x, tangent = _data(octree, torch.float16, 0), _data(octree, torch.float16, 1)
+    with torch.set_grad_enabled(training):
+      want = module(x, *args)
+      with fwAD.dual_level():
+        dual = fwAD.make_dual(x, tangent)
+        with pytest.raises(NotImplementedError):
+          module(dual, *args)
+        got = module(x, *args)
+    assert (got - want).abs().max() <= EVAL_TOL[torch.float16] * want.abs().max()
+
+
+def test_transforms_are_refused():
+  octree = _octree()
+  for module, args in _layers(octree):
+    module = module.to('cuda', torch.float16)
+    x = _data(octree, torch.float16, 0)
+    f = lambda t: module(t, *args).float().sum()
+    with pytest.raises(RuntimeError, match='autograd.Function'):
+      torch.func.grad(f)(x)
+    with pytest.raises(RuntimeError, match='autograd.Function'):
+      torch.func.vmap(lambda t: module(t, *args))(x[None])
