@@ -105,11 +105,12 @@ def _rows_linear_layer(x, cin, cout):
   if layer is None:
     if len(_LINEAR) > 64:
       _LINEAR.clear()
-    layer = _LINEAR[key] = _lib.native().ConvLayer()
+    layer = _lib.native().ConvLayer()
     layer.fwd = _gather_op(x.dtype, rows, rows, 1, cin, cout, True, False, None, True)
     layer.dgrad = _gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True)
     layer.wgrad = _wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin])
     layer.fwd_table = layer.dgrad_table = layer.wgrad_table = _identity_table(rows, x.device)
+    _LINEAR[key] = layer                     # (whole: other threads take it from here)
   return layer
 
 

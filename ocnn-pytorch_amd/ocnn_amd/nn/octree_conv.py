@@ -11,6 +11,7 @@ table is centrally symmetric (stride 1, every kernel but 2x2x2) and through
 the inverse table otherwise, so no atomics are involved anywhere.
 """
 
+import threading
 from typing import List
 
 import torch
@@ -647,21 +648,32 @@ def call_native(native, data, weights, bias):
 
 class _Layer:
   """A layer on an octree in one data type: its native passes and the shape of its input.  (Kept by
-  the octree, and therefore without a reference to it.)"""
+  the octree, and therefore without a reference to it.)
+
+  The backward passes are made when a call first needs them.  Threads share the layer, and a call that
+  runs holds the native object without the interpreter lock: that object is never changed, one with the
+  further pass takes its place."""
 
   def __init__(self, eng, dtype, padded):
     self.dtype, self.padded = dtype, padded    # padded: stride 2 over all nodes, octree_pad / octree_depad folded in
     self.conv = eng.is_conv_layer()
     self.pad_depth = (eng.out_depth if self.conv else eng.in_depth) if padded else None
     self.shape = eng.in_shape if self.conv or not padded else (int(eng.octree.nnum[eng.in_depth]), eng.in_channels)
-    self.native = _lib.native().ConvLayer()
-    self.native.wgrad_of_grad = not self.conv
+    self._lock = threading.Lock()
+    self._made = {'wgrad_of_grad': not self.conv}
+    self.dgrad = self.wgrad = None             # None = not made yet, False = not one pass
     made = self._pass(eng, True)
     self.ok = made is not None                 # the forward pass is one native pass
-    if self.ok:
-      self.native.fwd, self.native.fwd_table = made
-    # the backward passes are made when a call first needs them: None = not yet, False = not one pass
-    self.dgrad = self.wgrad = None
+    self._add('fwd', made)
+
+  def _add(self, name, made):
+    """`made` (a pass and its table, or None) as the pass `name`, visible to other threads at once."""
+    if made is not None:
+      self._made[name], self._made[name + '_table'] = made
+    native = _lib.native().ConvLayer()
+    for field, value in self._made.items():
+      setattr(native, field, value)
+    self.native = native
 
   def _coarse(self, octree):
     """(index, rows) of the padded side: what the passes read the coarse rows through."""
@@ -676,17 +688,19 @@ class _Layer:
 
   @_lib.unrecorded
   def make_dgrad(self, eng):
-    made = self._pass(eng, False)
-    self.dgrad = made is not None
-    if made is not None:
-      self.native.dgrad, self.native.dgrad_table = made
+    with self._lock:
+      if self.dgrad is None:
+        made = self._pass(eng, False)
+        self._add('dgrad', made)
+        self.dgrad = made is not None
 
   @_lib.unrecorded
   def make_wgrad(self, eng):
-    made = eng.weight_op(self.dtype, False, *self._coarse(eng.octree))
-    self.wgrad = made is not None
-    if made is not None:
-      self.native.wgrad, self.native.wgrad_table = made
+    with self._lock:
+      if self.wgrad is None:
+        made = eng.weight_op(self.dtype, False, *self._coarse(eng.octree))
+        self._add('wgrad', made)
+        self.wgrad = made is not None
 
 
 @_lib.unrecorded
@@ -706,7 +720,7 @@ def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_siz
     return eng
 
   if layer is None:
-    layer = octree._layers[key] = _Layer(made_engine(), data.dtype, padded)
+    layer = octree._layers.setdefault(key, _Layer(made_engine(), data.dtype, padded))
   if not layer.ok:
     return None, None
   assert data.shape == layer.shape, \
