@@ -353,6 +353,7 @@ class Octree:
     self._tables_t = {}      # same key -> inverse table
     self._plans = {}         # (key, inverse) -> TilePlan
     self._layers = {}        # the layers' passes on this octree (nn/octree_conv.py)
+    self._built = {}         # depth -> what build_octree made of a layer (see _as_built)
     self._plans_prebuilt = False
 
     self.nnum = torch.zeros(num, dtype=torch.long)
@@ -379,7 +380,7 @@ class Octree:
   lut_kernel = property(lambda self: self._lut(2))
 
   def __getstate__(self):
-    return dict(vars(self), _layers={})        # (native passes are made again when asked for)
+    return dict(vars(self), _layers={}, _built={})        # (native passes are made again when asked for)
 
   # ---- cache bookkeeping ---------------------------------------------------
   def _drop_tables(self, depth, nempty_only=False):
@@ -399,6 +400,7 @@ class Octree:
     self.nempty_indices[depth] = None
     self.nempty_neighs[depth] = None
     self._nempty_indices32[depth] = None
+    self._built.pop(depth, None)
     self._drop_tables(depth, nempty_only=True)
 
   # ---- simple accessors (ocnn/octree/octree.py:108-145) ---------------------
@@ -419,10 +421,23 @@ class Octree:
       self.nempty_masks[depth] = self.children[depth] >= 0
     return self.nempty_masks[depth]
 
-  def _make_nempty_index(self, depth):
-    child = self.children[depth]
+  def _as_built(self, depth, nnum, nnum_nempty, keys=False):
+    """The layer is what build_octree made (and the index of its non-empty nodes from there with it): the octree
+    still holds its tensors, of these counts, and nobody wrote to them.  Children, keys and counts are public."""
+    built = self._built.get(depth)
+    if built is None:
+      return False
+    key, child, versions, index = built
+    return (self.children[depth] is child and child._version == versions[1] and child.shape[0] == nnum and
+            (index is None or index.shape[0] == nnum_nempty) and
+            (not keys or (self.keys[depth] is key and key._version == versions[0])))
+
+  def _make_nempty_index(self, depth, reset=False):
+    child, n = self.children[depth], int(self.nnum_nempty[depth])
+    if not reset and self._as_built(depth, int(self.nnum[depth]), n) and self._built[depth][3] is not None:
+      self._nempty_indices32[depth] = self._built[depth][3]
+      return
     _lib.require_gpu(child)
-    n = int(self.nnum_nempty[depth])
     i32 = torch.empty(n, dtype=torch.int32, device=child.device)
     i64 = torch.empty(n, dtype=torch.long, device=child.device)
     _lib.check(_lib.lib().ocnn_nempty_index(_lib.ptr(child), child.numel(), _lib.ptr(i32),
@@ -432,10 +447,10 @@ class Octree:
 
   def nempty_index(self, depth: int, reset: bool = False):
     if self.nempty_indices[depth] is None or reset:
-      if not reset and self._nempty_indices32[depth] is not None:
+      if reset or self._nempty_indices32[depth] is None:
+        self._make_nempty_index(depth, reset)
+      if self.nempty_indices[depth] is None:
         self.nempty_indices[depth] = self._nempty_indices32[depth].long()
-      else:
-        self._make_nempty_index(depth)
     return self.nempty_indices[depth]
 
   def _nempty_index32(self, depth):
@@ -492,7 +507,11 @@ class Octree:
     self.nempty_masks = [None] * num
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
-    self._nempty_indices32 = tree.index
+    self._nempty_indices32 = [None] * num
+    # (the writes to a tensor made in inference mode are not counted)
+    self._built = {d: (key, child, (key._version, child._version), index)
+                   for d, (key, child, index) in enumerate(zip(tree.keys, tree.children, tree.index))
+                   if not child.is_inference()}
     self._tables, self._tables_t, self._plans, self._layers = {}, {}, {}, {}
     self._plans_prebuilt = False
     return tree.idx
@@ -604,21 +623,32 @@ class Octree:
     depth = self.depth
     nnum = [int(v) for v in self.nnum[:depth + 1].tolist()]
     nempty = [int(v) for v in self.nnum_nempty[:depth + 1].tolist()]
-    if dev.type != 'cuda' or self.full_depth < 1 or \
-        any(c is None for c in self.children[:depth + 1] + self.keys[:depth + 1]) or \
+    if dev.type != 'cuda' or self.full_depth < 1 or any(c is None for c in self.children[:depth + 1]) or \
         min(nnum[1:] + nempty) <= 0 or \
         any(nnum[d] != (self.batch_size << (3 * d) if d <= self.full_depth else 8 * nempty[d - 1])
             for d in range(1, depth + 1)):
       for d in range(1, depth + 1):                       # the layer-by-layer route says what is wrong
         self.construct_neigh(d)
       return
-    index = [self._nempty_index32(d) if self.full_depth <= d < depth else None for d in range(depth + 1)]
     with torch.cuda.device(dev):
-      tables = _lib.native().all_neigh(self.keys[:depth + 1], self.children[:depth + 1], index, nnum, nempty,
-                                       self.full_depth, self.batch_size)
+      if all(self._as_built(d, nnum[d], nempty[d], keys=True) for d in range(depth + 1)):
+        index = [self._built[d][3] if d < depth else None for d in range(depth + 1)]
+        tables = _lib.native().all_neigh(self.keys[:depth + 1], self.children[:depth + 1], index, nnum, nempty,
+                                         self.full_depth, self.batch_size)
+      else:                     # layers from elsewhere: one after the other, from their children alone
+        tables = [torch.empty(n, 27, dtype=torch.int32, device=dev) for n in nnum[1:]]
+        index = [torch.empty(nempty[d], dtype=torch.int32, device=dev) if self.full_depth <= d < depth else None
+                 for d in range(depth + 1)]
+        ptrs = lambda ts: (ctypes.c_void_p * (depth + 1))(*[None if t is None else t.data_ptr() for t in ts])
+        counts = lambda ns: (ctypes.c_int64 * (depth + 1))(*ns)
+        _lib.check(_lib.lib().ocnn_neigh_all(depth, self.full_depth, self.batch_size, counts(nnum), counts(nempty),
+                                             ptrs(self.children[:depth + 1]), ptrs(index), ptrs([None] + tables),
+                                             _lib.stream()))
     for d, table in enumerate(tables, 1):
       self.neighs[d] = table
       self.nempty_neighs[d] = None
+    for d in range(self.full_depth, depth):
+      self._nempty_indices32[d], self.nempty_indices[d] = index[d], None
     self._drop_tables(None)
 
   # ---- search (ocnn/octree/octree.py:448-488) -------------------------------
@@ -878,7 +908,7 @@ class Octree:
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
     self._nempty_indices32 = [None] * num
-    self._tables, self._tables_t, self._plans, self._layers = {}, {}, {}, {}
+    self._tables, self._tables_t, self._plans, self._layers, self._built = {}, {}, {}, {}, {}
     low48 = (1 << 48) - 1
     for d in range(num):
       self.keys[d] = torch.cat([(o.keys[d] & low48) | (i << 48)

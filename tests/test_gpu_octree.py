@@ -295,6 +295,37 @@ def test_larger_synthetic_batch_vs_oracle():
     assert np.array_equal(np_(o._table(7, kern, stride, ne)), w.get_neigh(7, kern, stride, ne))
 
 
+@pytest.mark.parametrize('how', ['children assigned', 'children written', 'keys assigned', 'inference mode'])
+def test_layers_changed_after_the_build(how):
+  """children and keys are public: tables and indices follow what the octree holds when they are made (the
+  tables from the children alone), not what the build left."""
+  depth, at = 6, 4
+  pts, nrm, bid = synthetic.batch_clouds(synthetic.mixed_cloud, 2, 9, n=5000)
+  with torch.inference_mode(how == 'inference mode'):
+    o = Octree(depth, 2, batch_size=2)
+    o.build_octree(Points(pts.to(DEV), nrm.to(DEV), batch_id=bid.to(DEV), batch_size=2))
+    w, _ = R.build_octree(pts.numpy(), nrm.numpy(), None, bid.numpy(), depth, 2, 2)
+    if how == 'keys assigned':
+      o.keys[at] = torch.zeros_like(o.keys[at])
+    else:                                                 # the same number of non-empty nodes, others
+      kept = np.roll(w.children[at] >= 0, 1)
+      w.children[at] = np.where(kept, np.cumsum(kept) - 1, -1).astype(np.int32)
+      new = torch.from_numpy(w.children[at]).to(DEV)
+      if how == 'children assigned':
+        o.children[at] = new
+      else:
+        o.children[at].copy_(new)
+    assert np.array_equal(np_(o.nempty_index(at)), np.nonzero(w.children[at] >= 0)[0])
+    say(how)
+    o.construct_all_neigh()
+    R.construct_all_neigh(w)
+    for d in range(1, depth + 1):
+      assert np.array_equal(np_(o.neighs[d]), w.neighs[d]), d
+      assert np.array_equal(np_(o._nempty_index32(d)), np.nonzero(w.children[d] >= 0)[0]), d
+    for table in (('333', 1, True), ('222', 2, False), ('222', 2, True)):
+      assert np.array_equal(np_(o._table(at, *table)), w.get_neigh(at, *table)), table
+
+
 def test_full_size_invariants():
   say('build+neigh at the benchmark size: 8 x 100k points, depth 8 (properties only)')
   pts, nrm, bid = synthetic.batch_clouds(synthetic.mixed_cloud, 8, 1001, n=100000)
