@@ -531,6 +531,7 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   require_gpu(pts);
   pts = pts.to(at::kFloat).contiguous();
   const int64_t n = pts.size(0);
+  TORCH_CHECK(batch_size == 1 || (batch.has_value() && batch->numel() == n), "build_octree: a batch id for every point");
   bool batch_is_float = false;
   if (batch.has_value()) {
     batch_is_float = batch->is_floating_point();

@@ -477,6 +477,7 @@ class Octree:
                    bbmax: Union[float, torch.Tensor] = 1.0):
     self.device = point_cloud.device
     assert point_cloud.batch_size == self.batch_size, 'Inconsistent batch_size'
+    assert self.batch_size == 1 or point_cloud.batch_id is not None, 'A batch of octrees needs batch_id'
     pts = point_cloud.points
     _lib.require_gpu(pts)
     dev, depth = pts.device, self.depth

@@ -141,6 +141,13 @@ def test_no_cpu_fallback():
     o.construct_neigh(1)
 
 
+def test_batch_without_batch_ids_is_refused():
+  points = ocnn_amd.Points(torch.rand(20, 3))
+  points.batch_size = 2                                  # (set by hand: nothing says which point is whose)
+  with pytest.raises(AssertionError, match='batch_id'):
+    ocnn_amd.Octree(3, 2, batch_size=2).build_octree(points)
+
+
 def test_module_contract():
   from ocnn_amd.nn import OctreeConv, OctreeDeconv, OctreeDWConv
   c = OctreeConv(3, 5, [3], stride=1, nempty=True, use_bias=True)
