@@ -325,6 +325,22 @@ class PlanHistory:
       self._kinds.clear()
 
 
+def _lut_grid(dev):
+  return range_grid(2, 3, dev).unsqueeze(1) + range_grid(-1, 1, dev)
+
+
+def _lut(name, make):
+  """A public lookup table of the reference's class (ocnn/octree/octree.py:85-106), on the device the octree
+  was made on.  An attribute as there, but made when it is first read: nothing here needs them (the kernels
+  compute the first two arithmetically)."""
+  def read(self):
+    if name not in vars(self):
+      vars(self)[name] = make(self._lut_device)
+    return vars(self)[name]
+
+  return property(read, lambda self, value: vars(self).__setitem__(name, value))
+
+
 class Octree:
   """Same constructor, attributes and methods as the reference class
   (ocnn/octree/octree.py:18-106)."""
@@ -362,22 +378,13 @@ class Octree:
     self.batch_nnum = torch.zeros(num, bs, dtype=torch.long)
     self.batch_nnum_nempty = torch.zeros(num, bs, dtype=torch.long)
 
-    self._luts = None
+    for name in ('lut_parent', 'lut_child', 'lut_kernel'):
+      vars(self).pop(name, None)
+    self._lut_device = self.device
 
-  # the reference's public lookup tables (ocnn/octree/octree.py:85-106), made when asked for: the
-  # kernels compute the first two arithmetically
-  def _lut(self, which):
-    if self._luts is None:
-      dev = self.device
-      grid = range_grid(2, 3, dev).unsqueeze(1) + range_grid(-1, 1, dev)
-      self._luts = ((trunc_div(grid, 2) * torch.tensor([9, 3, 1], device=dev)).sum(2),
-                    ((grid % 2) * torch.tensor([4, 2, 1], device=dev)).sum(2),
-                    {k: torch.tensor(v, device=dev) for k, v in LUT_KERNEL.items()})
-    return self._luts[which]
-
-  lut_parent = property(lambda self: self._lut(0))
-  lut_child = property(lambda self: self._lut(1))
-  lut_kernel = property(lambda self: self._lut(2))
+  lut_parent = _lut('lut_parent', lambda dev: (trunc_div(_lut_grid(dev), 2) * torch.tensor([9, 3, 1], device=dev)).sum(2))
+  lut_child = _lut('lut_child', lambda dev: ((_lut_grid(dev) % 2) * torch.tensor([4, 2, 1], device=dev)).sum(2))
+  lut_kernel = _lut('lut_kernel', lambda dev: {k: torch.tensor(v, device=dev) for k, v in LUT_KERNEL.items()})
 
   def __getstate__(self):
     return dict(vars(self), _layers={}, _built={})        # (native passes are made again when asked for)

@@ -2,6 +2,7 @@
 symbol the header declares, the host-evaluable kernel arithmetic agrees with
 the oracle, and the host-side logic (shapes, errors, no CPU fallback)."""
 
+import copy
 import ctypes
 import os
 import re
@@ -139,6 +140,22 @@ def test_no_cpu_fallback():
     ocnn_amd.octree.xyz2key(torch.zeros(3), torch.zeros(3), torch.zeros(3), depth=4)
   with pytest.raises(RuntimeError):
     o.construct_neigh(1)
+
+
+def test_lookup_tables_are_attributes():
+  """lut_parent, lut_child, lut_kernel (ocnn/octree/octree.py:85-106): on the device the octree was made on,
+  whatever is built with it later, and open to assignment."""
+  parent, child = R.neigh_luts()
+  o = ocnn_amd.Octree(3, 2)
+  o.device = torch.device('meta')                        # (what a build on another device sets)
+  assert o.lut_parent.device.type == 'cpu' and np.array_equal(o.lut_parent.numpy(), parent)
+  assert o.lut_child.device.type == 'cpu' and np.array_equal(o.lut_child.numpy(), child)
+  assert o.lut_kernel['222'].tolist() == [13, 14, 16, 17, 22, 23, 25, 26]
+  copied = copy.copy(o)
+  copied.lut_child = o.lut_child + 1
+  assert torch.equal(copied.lut_child, o.lut_child + 1) and copied.lut_parent is o.lut_parent
+  o.reset()
+  assert o.lut_parent.device.type == 'meta'
 
 
 def test_batch_without_batch_ids_is_refused():
