@@ -716,8 +716,13 @@ PYBIND11_MODULE(ocnn_host, m) {
   py::class_<ConvLayer, std::shared_ptr<ConvLayer>>(m, "ConvLayer")
       .def(py::init<>())
 #define FIELD(name) .def_readwrite(#name, &ConvLayer::name)
-      FIELD(fwd) FIELD(dgrad) FIELD(wgrad) FIELD(fwd_table) FIELD(dgrad_table) FIELD(wgrad_table) FIELD(wgrad_of_grad);
+      FIELD(fwd) FIELD(dgrad) FIELD(wgrad) FIELD(fwd_table) FIELD(dgrad_table) FIELD(wgrad_table) FIELD(wgrad_of_grad)
 #undef FIELD
+      .def("with_table", [](const ConvLayer& layer, const Tensor& table) {
+        auto copy = std::make_shared<ConvLayer>(layer);
+        copy->fwd_table = copy->dgrad_table = copy->wgrad_table = table;
+        return copy;
+      });
   py::class_<Tree>(m, "Tree")
 #define FIELD(name) .def_readonly(#name, &Tree::name)
       FIELD(keys) FIELD(children) FIELD(index) FIELD(nnum) FIELD(nnum_nempty) FIELD(idx) FIELD(points) FIELD(normals)

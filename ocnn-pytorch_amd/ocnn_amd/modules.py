@@ -83,16 +83,28 @@ _IDENTITY = {}
 
 
 def _identity_table(rows, device):
-  """(rows, 1) table [0, 1, ..]: row i reads row i."""
-  key = (rows, str(device))
-  if key not in _IDENTITY:
-    if len(_IDENTITY) > 16:
-      _IDENTITY.clear()
-    _IDENTITY[key] = torch.arange(rows, dtype=torch.int32, device=device).view(rows, 1)
-  return _IDENTITY[key]
+  """(rows, 1) table [0, 1, ..]: row i reads row i.  The head of one table per device and stream, as long as
+  the longest asked for (an eighth longer at most): row counts differ with every octree.  Of each stream its
+  own, so that memory given back is not reused before its readers are done; under capture the graph's own."""
+  key = (device, _lib.stream())
+  table = _IDENTITY.get(key)
+  capturing = torch.cuda.is_current_stream_capturing()
+  if table is None or table.shape[0] < rows or capturing:
+    step = max(1024, 1 << max(rows.bit_length() - 3, 0))
+    table = torch.arange(-(-rows // step) * step, dtype=torch.int32, device=device).view(-1, 1)
+    if not capturing:
+      if len(_IDENTITY) > 16:
+        _IDENTITY.clear()
+      _IDENTITY[key] = table
+  return table[:rows]
 
 
 _LINEAR = {}
+
+
+def _reads_table(op):
+  """The pass goes over the one-slot table (the dense kernels do without)."""
+  return (op.padded or op).kernel == _lib.GATHER_PLAIN       # (the same number as WGRAD_PLAIN)
 
 
 @_lib.unrecorded
@@ -100,18 +112,19 @@ def _rows_linear_layer(x, cin, cout):
   """y = x W^T on many rows as the one-slot form of the convolution kernels (weights (out, in) as
   torch.nn.Linear holds them)."""
   rows = x.shape[0]
-  key = (rows, cin, cout, x.dtype, x.device)
-  layer = _LINEAR.get(key)
-  if layer is None:
+  key = (rows, cin, cout, x.dtype)
+  made = _LINEAR.get(key)
+  if made is None:
     if len(_LINEAR) > 64:
       _LINEAR.clear()
     layer = _lib.native().ConvLayer()
     layer.fwd = _gather_op(x.dtype, rows, rows, 1, cin, cout, True, False, None, True)
     layer.dgrad = _gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True)
     layer.wgrad = _wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin])
-    layer.fwd_table = layer.dgrad_table = layer.wgrad_table = _identity_table(rows, x.device)
-    _LINEAR[key] = layer                     # (whole: other threads take it from here)
-  return layer
+    # (whole: other threads take it from here.  Without the table, which would outlive the octree)
+    made = _LINEAR[key] = (layer, any(_reads_table(op) for op in (layer.fwd, layer.dgrad, layer.wgrad)))
+  layer, table = made
+  return layer.with_table(_identity_table(rows, x.device)) if table else layer
 
 
 class _RowsLinearNarrow(torch.autograd.Function):

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from ocnn_amd import synthetic
-from ocnn_amd.modules import Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
+from ocnn_amd.modules import Conv1x1, Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
 from ocnn_amd.octree import Octree, Points
 
 pytestmark = pytest.mark.gpu
@@ -70,3 +70,42 @@ def test_residual_block(dtype, cin, cout):
     block(x, octree, 6)
   handle.remove()
   assert seen == [1]
+
+
+def test_linear_layers_keep_one_table():
+  """A 1x1 layer whose row count differs with every call (a new octree every step): what is kept for it on
+  the GPU does not grow with the calls."""
+  layer = Conv1x1(32, 32).to('cuda', torch.float16)      # (small products: the kernels on the one-slot table)
+  g = torch.Generator(device='cuda').manual_seed(3)
+
+  def step(rows):
+    x = torch.randn(rows, 32, device='cuda', generator=g).half().requires_grad_()
+    layer.zero_grad()
+    layer(x).backward(torch.ones(rows, 32, device='cuda', dtype=torch.float16))
+    want = x.detach().double() @ layer.linear.weight.detach().double().t()
+    assert (layer(x).double() - want).abs().max() < TOL[torch.float16] * want.abs().max()
+
+  step(200000)
+  torch.cuda.synchronize()
+  held = torch.cuda.memory_allocated()
+  for i in range(30):
+    step(100000 + 3001 * i)
+  torch.cuda.synchronize()
+  assert torch.cuda.memory_allocated() <= held + 4096
+
+
+def test_linear_layer_in_a_graph():
+  """Replays of a captured 1x1 layer while larger ones run beside them."""
+  layer = Conv1x1(32, 32).to('cuda', torch.float16).requires_grad_(False)
+  x = torch.randn(5000, 32, device='cuda').half()
+  want = layer(x).clone()
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph):
+    out = layer(x)
+  for rows in (9000, 70000, 600000):
+    out.zero_()
+    layer(torch.randn(rows, 32, device='cuda').half())
+    torch.full((rows,), -1, dtype=torch.int32, device='cuda')      # (over memory that was given back)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
