@@ -31,8 +31,11 @@ class _LayerBn(torch.nn.Module):
 
 
 def _hooked(*modules):
+  """A call of one of the modules runs more than the forward() of its class: hooks, a forward put on the
+  module itself (as libraries that place modules on devices do), a compiled call."""
   return (torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks or
-          any(m._forward_hooks or m._forward_pre_hooks for m in modules))
+          any(m._forward_hooks or m._forward_pre_hooks or 'forward' in vars(m) or m._compiled_call_impl is not None
+              for m in modules))
 
 
 def layer_bn(layer, bn, data, *args, residual=None, relu=None):
