@@ -38,7 +38,7 @@ int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t
 #define OCNNX_GATHER_TILE 8
 int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout, int identity_table,
                         int has_plan, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
-                        double plan_reuse);
+                        double plan_reuse, int plan_overflow);
 
 // ocnn_batch_norm_stats and ocnn_batch_norm_apply after each other: one launch where there are few rows.
 int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows, int channels, float eps, float* mean, float* var,

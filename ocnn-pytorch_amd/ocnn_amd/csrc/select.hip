@@ -1,6 +1,7 @@
 // Which kernel runs a layer: the selection among the gather-GEMM and weight-gradient entry
-// points, as one pair of functions of the C ABI, so that whoever binds the header gets the
-// same choices as the Python layer of this package (which calls these functions too).
+// points.  ocnn_conv_gather_choose and ocnn_conv_wgrad_choose choose among the entry points of the
+// public header, for whoever binds it; this package's own host path calls ocnnx_gather_choose in the
+// place of the first, which knows the kernel of conv_tile.hip in its full range as well.
 //
 // Every *_supported() predicate says whether a kernel takes a shape class; the row ranges that
 // its entry point checks on top (32-bit buffer offsets of the output, of the table, of the
@@ -58,19 +59,42 @@ extern "C" int ocnn_conv_gather_choose(int dtype, int64_t rows_in, int64_t rows_
 }
 
 // The same for this package's own host path, which also has the kernel of conv_tile.hip in its full
-// range: it takes what would run plan-free or multi-pass on a table with a plan (every fp32 layer;
-// 16-bit layers of 32 or 64 output channels that are not square), and the wide layers, which it
-// splits where there are few tiles.
+// range: it takes the wide layers, which it splits where there are few tiles, the multi-pass ones (175
+// layer passes 39.6 ms instead of 58.4, slower in none) and most of what would run plan-free on a table with a
+// plan.  The plan-free kernel stays (us, tile kernel / plan-free)
+//  - for 16-bit layers with little work per row that is staged: on 8 or 9 slots below 4096 channel pairs, on 3
+//    below 16384 and, there, below kTileMinProducts products (too few for all CUs, and the weights
+//    are half of a pass).  64 -> 32 on 4.9 M rows of a 3x1x1 table 369 / 248; 32 -> 64 on those of 2x2x2 502 / 421;
+//    256 -> 256 on three slots of 3826 rows 19 / 14, 128 -> 128 of 100 k rows, 36 % set, 26 / 24, of 235 k rows, 85 %
+//    set, 55 / 65; 128 -> 32 on nine slots 1.17 x faster on the tile kernel in the median, 256 -> 64 1.5 x, 27 slots
+//    1.1 - 2 x from 32 -> 64 on;
+//  - for every data type on 8 or 9 slots of a table of little reuse where rows in tiles too dense for the plan
+//    run apart (plan_overflow): the second launch and the copy of its rows cost 10 - 40 us, which pays from
+//    kTileMinProductsApart on (fp32: three products a pair).  18.8 k rows of 3x3x1 stride 2: 128 -> 128 39 / 19,
+//    fp32 111 / 68; 235 k rows: 106 / 97, fp32 433 / 449 and 64 -> 64 202 / 178.
+// Over 916 bf16 passes (six kernel shapes, strides 1 and 2, all and non-empty nodes, three octrees of 20 k - 1 M
+// points, eleven widths): all plan-free 80.1 ms, all on the tile kernel 74.1, by this rule 70.0, the faster of the
+// two each time 69.3.  Other fp32 layers gain on every table, 1.04 - 9 x: plan-free reads three copies of their rows.
+constexpr double kTileMinProducts = 3.0e9;
+constexpr double kTileMinProductsApart = 1.7e10;
+
 extern "C" int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout,
                                    int identity_table, int has_plan, int plan_max_distinct, int64_t plan_total,
-                                   double plan_occupancy, double plan_reuse) {
+                                   double plan_occupancy, double plan_reuse, int plan_overflow) {
   const int pick = ocnn_conv_gather_choose(dtype, rows_in, rows_out, K, cin, cout, identity_table, has_plan,
                                            plan_max_distinct, plan_total, plan_occupancy, plan_reuse);
-  if (has_plan && rows_ok(rows_out, plan_total) &&
-      (pick == OCNN_GATHER_PLAIN || pick == OCNN_GATHER_PLANNED || pick == OCNN_GATHER_WIDE) &&
-      ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct))
-    return OCNNX_GATHER_TILE;
-  return pick;
+  if (!has_plan || !rows_ok(rows_out, plan_total) ||
+      !ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct))
+    return pick;
+  if (pick == OCNN_GATHER_PLANNED || pick == OCNN_GATHER_WIDE) return OCNNX_GATHER_TILE;
+  if (pick != OCNN_GATHER_PLAIN) return pick;
+  const bool half = dtype != OCNN_F32;
+  const double products = plan_occupancy * (double)rows_out * K * cin * cout * (half ? 1 : 3);
+  if (K < 27) {
+    if (plan_reuse < 2.0 && plan_overflow && products < kTileMinProductsApart) return pick;
+    if (half && (K >= 8 ? cin * cout < 4096 : cin * cout < 16384 || products < kTileMinProducts)) return pick;
+  }
+  return OCNNX_GATHER_TILE;
 }
 
 extern "C" int ocnn_conv_wgrad_choose(int dtype, int64_t rows_x, int64_t rows, int K, int ca, int cb,

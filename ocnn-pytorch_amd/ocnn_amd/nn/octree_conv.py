@@ -114,7 +114,8 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
   L, code = _lib.lib(), _lib.dtype_code_of(dtype)
   op = _lib.native().GatherOp()
   op.rows_in, op.rows, op.K, op.cin, op.cout, op.transposed, op.reverse = rows_in, rows, K, cin, cout, transposed, reverse
-  op.kernel = L.ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan))
+  op.kernel = L.ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan),
+                                    int(plan is not None and plan.overflow_rows is not None))
   if op.kernel == _lib.GATHER_ZERO_PADDED:
     op.padded = _gather_op(dtype, rows_in, rows, K, -(-cin // 32) * 32, -(-cout // 16) * 16, transposed, reverse, plan)
   else:

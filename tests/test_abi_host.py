@@ -297,6 +297,38 @@ def test_kernel_selection_is_consistent_with_the_predicates():
   assert L.ocnn_conv_gather_choose(BF, big, big, 27, 128, 128, 0, 1, 300, big * 2, 0.15, 4.0) != _lib.GATHER_SPARSE
 
 
+def test_selection_of_the_tile_kernel():
+  """ocnnx_gather_choose (host arithmetic only): the tile kernel in the place of the plan-free one, at both sides
+  of each line of its rule; never where its predicate refuses, and otherwise the public choice."""
+  L, (F32, BF) = _lib.lib(), (0, 2)
+  PLAIN, TILE = _lib.GATHER_PLAIN, _lib.GATHER_TILE
+
+  def pick(dtype, rows, K, cin, cout, occ, reuse, apart=0, umax=300):
+    a = (dtype, rows, rows, K, cin, cout, 0, 1, umax, 2 * rows, occ, reuse)
+    got, public = L.ocnnx_gather_choose(*a, apart), L.ocnn_conv_gather_choose(*a)
+    assert got == public or (got == TILE and public in (PLAIN, _lib.GATHER_PLANNED, _lib.GATHER_WIDE) and
+                             L.ocnnx_gather_tile_supported(dtype, rows, K, cin, cout, umax))
+    return got
+
+  for dtype, rows, K, cin, cout, occ, reuse, apart, want in (
+      (BF, 100000, 9, 64, 32, 0.6, 3.0, 0, PLAIN), (BF, 100000, 9, 128, 32, 0.6, 3.0, 0, TILE),      # pairs of channels
+      (BF, 100000, 8, 32, 64, 0.6, 3.0, 0, PLAIN), (BF, 100000, 27, 64, 32, 0.6, 3.0, 0, TILE),
+      (BF, 3826, 3, 256, 256, 0.8, 1.5, 0, PLAIN), (BF, 100000, 3, 256, 256, 0.8, 1.5, 0, TILE),     # products
+      (BF, 3826, 9, 256, 256, 0.3, 1.5, 0, TILE), (BF, 300000, 3, 128, 96, 0.8, 1.5, 0, PLAIN),
+      (BF, 18773, 9, 128, 128, 0.4, 1.7, 0, TILE), (BF, 18773, 9, 128, 128, 0.4, 1.7, 1, PLAIN),     # rows apart
+      (BF, 600000, 9, 256, 256, 0.4, 1.7, 1, TILE), (F32, 18773, 9, 128, 128, 0.4, 1.7, 1, PLAIN),
+      (F32, 235659, 9, 128, 128, 0.2, 1.6, 1, TILE), (F32, 235659, 9, 64, 64, 0.2, 1.6, 1, PLAIN),
+      (F32, 235659, 9, 64, 64, 0.2, 1.6, 0, TILE), (F32, 18773, 9, 128, 128, 0.4, 2.1, 1, TILE),
+      (F32, 1000, 27, 32, 32, 0.1, 1.2, 1, TILE), (F32, 1000, 3, 32, 32, 0.1, 1.2, 0, TILE),
+      (BF, 100000, 27, 256, 256, 0.6, 9.0, 1, TILE), (BF, 100000, 27, 64, 64, 0.6, 9.0, 0, _lib.GATHER_RW)):
+    assert pick(dtype, rows, K, cin, cout, occ, reuse, apart) == want, (dtype, rows, K, cin, cout, occ, reuse, apart)
+  for dtype in (F32, BF):                                # no plan, too many distinct rows, odd channels, offsets
+    assert L.ocnnx_gather_choose(dtype, 1000, 1000, 27, 128, 128, 0, 0, 0, 0, 1.0, 0.0, 0) == PLAIN
+    assert pick(dtype, 9000, 27, 40, 64, 0.6, 3.0) == PLAIN
+    assert pick(dtype, 70_000_000, 27, 128, 128, 0.6, 1.5) == PLAIN
+  assert pick(F32, 9000, 27, 128, 128, 0.6, 3.0, umax=2000) == PLAIN
+
+
 def test_a_stale_library_is_not_loaded(monkeypatch):
   """The built libraries carry the hash of their sources; when a source changes, the loader
   builds again instead of loading the old binary."""
