@@ -572,20 +572,23 @@ extern "C" int ocnnx_tree_fill(const void* workspace, int64_t n, int depth, int 
 // The library's radix sort takes 95 us for 20 000 points (five kernels of 15 us, most of it the chains
 // of its decoupled look-back, and seven fills), four times what its bytes cost.  Here a
 // cloud is a number of spans of kSortSpan points and a pass is counts of the digit by span, then one stable
-// scatter.  Up to kSortInlineSpans spans every workgroup of the scatter reads the counts of all spans
-// itself; more of them are scanned by a launch in between.  Digits have up to 11 bits: a depth-6
-// octree takes two passes, depth 9 with eight clouds three.
+// scatter.  Digits have up to 11 bits: a depth-6 octree takes two passes, depth 9 with eight clouds three.
+// Up to kSortInlineSpans spans every workgroup of the scatter reads the counts of all spans itself; more of
+// them are scanned by a launch in between.  Keys to counted nodes, the launches back to back, itself / scanned:
+// 24 spans 31 / 33 us at depth 5, 33 / 34 at 6, 44 / 40 at 7, 46 / 48 at 9; 64 spans 38 / 34, 40 / 36, 63 / 41, 57 / 51; 128
+// spans 50 / 37, 53 / 39, 95 / 47, 76 / 55.  The line is behind that crossing because a build waits for its sizes, and
+// two launches more in front of the wait cost it 10 - 35 us: build and tables of 45 k points at depth 6 126 / 163 us, 60 k at
+// depth 7 149 / 168, 131 k at depth 6 135 / 141; 100 k at depth 7 159 / 152, 131 k at depth 8 181 / 176.
 constexpr int kSortSpan = 2048;
 constexpr int kSortThreads = 256, kSortItems = kSortSpan / kSortThreads;
 constexpr int kSortMaxBits = 11;
 constexpr int kSortInlineSpans = 64;
 constexpr int64_t kSortMaxPoints = 1 << 22;
-constexpr int64_t kSortAtomicMax = 32768;   // up to here a pass counts the next digit with atomics instead of a launch
 
 struct SortPlan {
   int passes, bits;                          // digits of `bits` bits
   int spans;
-  int64_t key[2], val[2], hist[2], totals, total;   // workspace offsets: ping-pong keys and values, counts [span][digit]
+  int64_t key[2], val[2], hist, totals, total;   // workspace offsets: ping-pong keys and values, counts [span][digit]
 };
 
 static SortPlan sort_plan(int64_t n, int total_bits) {
@@ -596,18 +599,18 @@ static SortPlan sort_plan(int64_t n, int total_bits) {
   int64_t off = 0;
   for (int i = 0; i < 2; ++i) { s.key[i] = off; off += align_up(n * 4, 256); }
   for (int i = 0; i < 2; ++i) { s.val[i] = off; off += align_up(n * 4, 256); }
-  for (int i = 0; i < 2; ++i) { s.hist[i] = off; off += align_up(((int64_t)s.spans << s.bits) * 4, 256); }
+  s.hist = off; off += align_up(((int64_t)s.spans << s.bits) * 4, 256);
   s.totals = off; off += align_up(4ll << s.bits, 256);
   s.total = off;
   return s;
 }
 
-// Normalised points and their sort keys (batch id right above the Morton bits), the counts of the
-// first digit by span, and zeros for the counts of the second.
+// Normalised points and their sort keys (batch id right above the Morton bits) and the counts of the
+// first digit by span.
 __global__ __launch_bounds__(kSortThreads) void tree_keys_kernel(
     const float* __restrict__ pts, int64_t n, float bx, float by, float bz, float factor, const void* __restrict__ batch,
     int batch_is_float, int depth, float* __restrict__ pts_out, uint32_t* __restrict__ key, int bits,
-    uint32_t* __restrict__ hist, uint32_t* __restrict__ hist_next) {
+    uint32_t* __restrict__ hist) {
   __shared__ uint32_t s_hist[1 << kSortMaxBits];
   const int bins = 1 << bits;
   for (int i = threadIdx.x; i < bins; i += kSortThreads) s_hist[i] = 0u;
@@ -632,12 +635,11 @@ __global__ __launch_bounds__(kSortThreads) void tree_keys_kernel(
     atomicAdd(&s_hist[(uint32_t)k & (uint32_t)(bins - 1)], 1u);
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < bins; i += kSortThreads) {
-    hist[(int64_t)blockIdx.x * bins + i] = s_hist[i];
-    hist_next[(int64_t)blockIdx.x * bins + i] = 0u;
-  }
+  for (int i = threadIdx.x; i < bins; i += kSortThreads) hist[(int64_t)blockIdx.x * bins + i] = s_hist[i];
 }
 
+// The counts of a further digit.  (Counting it with atomics in the scatter before instead: 25.2 / 24.7 us with / without
+// for 2 k points at depth 6, 32.7 / 30.8 for 32 k, 42.1 / 40.0 for 131 k.)
 __global__ __launch_bounds__(kSortThreads) void tree_digits_kernel(const uint32_t* __restrict__ key, int64_t n, int shift,
                                                                    int bits, uint32_t* __restrict__ hist) {
   __shared__ uint32_t s_hist[1 << kSortMaxBits];
@@ -680,14 +682,13 @@ __global__ __launch_bounds__(1024) void tree_spans_kernel(uint32_t* __restrict__
 
 // One stable pass.  A wave takes 128 consecutive points, 64 at a time: the lanes with the same digit
 // find each other with one ballot per bit, their rank among the wave's points is kept in registers;
-// the counts of the waves and of the spans before turn it into a place.  hist_next (or null): the
-// counts of the digit above, by the span that is written to.  totals: hist has been scanned.  (Sixteen waves a span and not four:
-// the ballots of a wave are a serial chain, 23 -> 9 us for 20 000 points.)
+// the counts of the waves and of the spans before turn it into a place.  totals: hist has been scanned.
+// (Sixteen waves a span and not four: the ballots of a wave are a serial chain, 23 -> 9 us for 20 000 points.)
 constexpr int kPassThreads = 1024;
 __global__ __launch_bounds__(kPassThreads) void tree_sort_kernel(
     const uint32_t* __restrict__ key, const uint32_t* __restrict__ val, int64_t n, int shift, int bits, int spans,
-    const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals, uint32_t* __restrict__ hist_next,
-    uint32_t* __restrict__ key_out, uint32_t* __restrict__ val_out) {
+    const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals, uint32_t* __restrict__ key_out,
+    uint32_t* __restrict__ val_out) {
   constexpr int kWaves = kPassThreads / 64, kMaxBins = 1 << kSortMaxBits, kPer = kMaxBins / kPassThreads;
   constexpr int kItems = kSortSpan / kPassThreads;
   __shared__ uint16_t s_cnt[kWaves][kMaxBins];               // points of a digit: in the wave, then in the waves before
@@ -777,8 +778,6 @@ __global__ __launch_bounds__(kPassThreads) void tree_sort_kernel(
     const uint32_t to = s_base[d] + s_cnt[wave][d] + rank[it];
     key_out[to] = k[it];
     val_out[to] = v[it];
-    if (hist_next)
-      atomicAdd(&hist_next[(int64_t)(to / kSortSpan) * bins + ((k[it] >> (shift + bits)) & (uint32_t)(bins - 1))], 1u);
   }
 }
 
@@ -815,8 +814,7 @@ extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin
   const SortPlan s = sort_plan(n, tree_key_bits(depth, batch_bits));
   uint32_t* keys[2] = {(uint32_t*)(more + s.key[0]), (uint32_t*)(more + s.key[1])};
   uint32_t* vals[2] = {(uint32_t*)(more + s.val[0]), (uint32_t*)(more + s.val[1])};
-  uint32_t* hist[2] = {(uint32_t*)(more + s.hist[0]), (uint32_t*)(more + s.hist[1])};
-  const bool atomics = n <= kSortAtomicMax && s.passes <= 2;   // (a third pass would need its counts cleared)
+  uint32_t* hist = (uint32_t*)(more + s.hist);
   uint32_t* totals = s.spans > kSortInlineSpans ? (uint32_t*)(more + s.totals) : nullptr;
   BuildLayout L;
   if (build_layout_t<uint32_t, 8>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
@@ -826,17 +824,16 @@ extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin
   uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
   const dim3 grid((unsigned)s.spans), block(kSortThreads);
   hipLaunchKernelGGL(tree_keys_kernel, grid, block, 0, st, pts, n, h_bbmin[0], h_bbmin[1], h_bbmin[2], factor, batch,
-                     batch_is_float, depth, pts_out, keys[0], s.bits, hist[0], hist[1]);
+                     batch_is_float, depth, pts_out, keys[0], s.bits, hist);
   for (int p = 0; p < s.passes; ++p) {
     const bool last = p + 1 == s.passes;
-    if (p > 0 && !atomics)
-      hipLaunchKernelGGL(tree_digits_kernel, grid, block, 0, st, keys[p & 1], n, p * s.bits, s.bits, hist[p & 1]);
+    if (p > 0) hipLaunchKernelGGL(tree_digits_kernel, grid, block, 0, st, keys[p & 1], n, p * s.bits, s.bits, hist);
     if (totals)
-      hipLaunchKernelGGL(tree_spans_kernel, dim3((unsigned)cdiv(1 << s.bits, 16)), dim3(1024), 0, st, hist[p & 1], s.spans,
-                         1 << s.bits, totals);
+      hipLaunchKernelGGL(tree_spans_kernel, dim3((unsigned)cdiv(1 << s.bits, 16)), dim3(1024), 0, st, hist, s.spans, 1 << s.bits,
+                         totals);
     hipLaunchKernelGGL(tree_sort_kernel, grid, dim3(kPassThreads), 0, st, keys[p & 1], p == 0 ? nullptr : vals[p & 1], n, p * s.bits,
-                       s.bits, s.spans, hist[p & 1], totals, atomics && !last ? hist[(p + 1) & 1] : nullptr,
-                       last ? csorted : keys[(p + 1) & 1], last ? (uint32_t*)perm : vals[(p + 1) & 1]);
+                       s.bits, s.spans, hist, totals, last ? csorted : keys[(p + 1) & 1],
+                       last ? (uint32_t*)perm : vals[(p + 1) & 1]);
   }
 #define OCNN_TREE_COUNT(N)                                                                                              \
   hipLaunchKernelGGL((build_count_kernel<uint32_t, N>), dim3((unsigned)L.spans), dim3(kBuildThreads), 0, st, csorted, n, \
