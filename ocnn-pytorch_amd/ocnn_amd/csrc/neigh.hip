@@ -40,9 +40,8 @@ constexpr int kParentsPerBlock = 32;
 
 // The 8 x 27 entries below one parent repeat the same (parent slot, child number) pattern, so
 // the pattern sits in LDS once a workgroup, and a thread writes four entries at a time: they
-// never straddle two parents (216 = 4 * 54).  NT: stores that pass the caches by, for tables that
-// would not stay in them (530 MB: 128 -> 102 us).
-template <bool NT>
+// never straddle two parents (216 = 4 * 54).  The stores pass the caches by: tables of 13 MB 5.4 -> 5.2 us, 113 MB
+// 24.1 -> 22.7, 340 MB 83 -> 67, and their tile plans, the next to read them, take the same time.
 __global__ __launch_bounds__(256) void neigh_from_parent_kernel(
     const int32_t* __restrict__ child_p, const int32_t* __restrict__ neigh_p,
     const int32_t* __restrict__ nempty_p, int64_t n_ne, int64_t* __restrict__ out64,
@@ -95,8 +94,7 @@ __global__ __launch_bounds__(256) void neigh_from_parent_kernel(
     typedef __attribute__((ext_vector_type(4))) int i32x4;
     if (out32) {
       const i32x4 v = {r[0], r[1], r[2], r[3]};
-      if (NT) __builtin_nontemporal_store(v, (i32x4*)(out32 + o));
-      else *(i32x4*)(out32 + o) = v;
+      __builtin_nontemporal_store(v, (i32x4*)(out32 + o));
     }
     if (out64) {
       *reinterpret_cast<longlong2*>(out64 + o) = make_longlong2((int64_t)r[0], (int64_t)r[1]);
@@ -181,8 +179,10 @@ __global__ __launch_bounds__(256) void neigh_walk_kernel(WalkTree t) {
   }
 }
 
-// layers with up to this many parents are found by walking (27 walks of a few dependent loads each); in
-// larger ones the two loads an entry takes from the parents' table are what counts
+// Layers with up to this many parents are found by walking (27 walks of a few dependent loads each); in
+// larger ones the two loads an entry takes from the parents' table are what counts.  All tables, the last layer
+// by walking / by a launch of its own: 1.1 k parents 9.4 / 12.4 us, 3.8 k 10.5 / 13.4, 10.7 k 14.4 / 15.4, 15.0 k
+// 16.7 / 16.0, 16.9 k 16.8 / 16.6, 43 k 31.5 / 25.0.  (A little behind the crossing: the host has a launch less.)
 constexpr int64_t kWalkMaxParents = 16384;
 
 __global__ void nempty_index_kernel(const int32_t* children, int64_t n, int32_t* i32,
@@ -255,15 +255,10 @@ extern "C" int ocnn_neigh_full(int depth, int batch, int64_t* out64, int32_t* ou
   return check_launch("neigh_full");
 }
 
-constexpr int64_t kStreamBytes = 128ll << 20;
-
 static void launch_from_parent(const int32_t* child_p, const int32_t* neigh_p, const int32_t* nempty_p, int64_t n_ne,
                                int64_t* out64, int32_t* out32, hipStream_t st) {
-  const dim3 grid((unsigned)cdiv(n_ne, kParentsPerBlock));
-  if (n_ne * 216 * 4 >= kStreamBytes)
-    hipLaunchKernelGGL(neigh_from_parent_kernel<true>, grid, dim3(256), 0, st, child_p, neigh_p, nempty_p, n_ne, out64, out32);
-  else
-    hipLaunchKernelGGL(neigh_from_parent_kernel<false>, grid, dim3(256), 0, st, child_p, neigh_p, nempty_p, n_ne, out64, out32);
+  hipLaunchKernelGGL(neigh_from_parent_kernel, dim3((unsigned)cdiv(n_ne, kParentsPerBlock)), dim3(256), 0, st, child_p, neigh_p,
+                     nempty_p, n_ne, out64, out32);
 }
 
 extern "C" int ocnn_neigh_from_parent(const int32_t* child_p, const int32_t* neigh_p,
