@@ -9,7 +9,7 @@ import importlib.util
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_void_p, POINTER
 
 import torch
-import torch.autograd.forward_ad
+from torch.autograd import forward_ad as _forward_ad
 
 from . import build as _build
 
@@ -170,13 +170,16 @@ def native():
   return _native
 
 
+# (taken directly: the layers ask at every call)
+_is_tracing, _transforms_active = torch._C._is_tracing, torch._C._are_functorch_transforms_active
+
+
 def recorded():
   """True where a call has to be an autograd.Function because something looks on.  torch.jit.trace records
   a Function as one Python operation, but of a native call (native().conv, ...) only the torch operations
   inside, that is an empty tensor.  Forward-mode differentiation and the transforms of torch.func are refused
   by a Function that does not provide for them; a native call would drop the tangents."""
-  return (torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0 or
-          torch._C._are_functorch_transforms_active())
+  return _is_tracing() or _forward_ad._current_level >= 0 or _transforms_active()
 
 
 def unrecorded(make):
@@ -185,9 +188,9 @@ def unrecorded(make):
   wrap the tensors that are kept."""
   @functools.wraps(make)
   def call(*args, **kwargs):
-    if torch._C._are_functorch_transforms_active():
+    if _transforms_active():
       raise RuntimeError('ocnn_amd layers are autograd.Functions that the transforms of torch.func do not support')
-    if not torch.jit.is_tracing():
+    if not _is_tracing():
       return make(*args, **kwargs)
     state = torch._C._get_tracing_state()
     torch._C._set_tracing_state(None)

@@ -523,6 +523,14 @@ struct Tree {
   std::vector<int64_t> nnum, nnum_nempty;
   Tensor idx, points, perm, seg_start;
   OptTensor normals;
+  std::vector<int64_t> versions;              // of keys and children, by torch's count of the writes to them
+
+  // Layer d is what the build made: `child` (and `key`, unless null) are its tensors and nobody wrote to
+  // them since.  (The writes to a tensor made in inference mode are not counted.)
+  bool as_built(size_t d, const Tensor* key, const Tensor& child) const {
+    return d < children.size() && !child.is_inference() && child.is_same(children[d]) &&
+           child._version() == versions[2 * d + 1] && (!key || (key->is_same(keys[d]) && key->_version() == versions[2 * d]));
+  }
 };
 
 // Build from the points: one sort, one numbering of all layers, one wait for the layers' sizes.
@@ -589,6 +597,8 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
     check(ocnn_leaf_average((const float*)pts_norm.data_ptr(), 3, (const int32_t*)t.perm.data_ptr(),
                             (const int32_t*)t.seg_start.data_ptr(), size[0], 0, (float*)t.points.data_ptr(), st.stream()));
   }
+  for (int d = 0; d <= depth; ++d)
+    for (const Tensor* made : {&t.keys[d], &t.children[d]}) t.versions.push_back(made->is_inference() ? 0 : made->_version());
   return t;
 }
 
@@ -642,12 +652,18 @@ std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, in
   return out;
 }
 
-// The neighbour tables of layers 1 .. depth (entry 0 is left out).
-std::vector<Tensor> all_neigh(const std::vector<Tensor>& keys, const std::vector<Tensor>& children,
-                              const std::vector<OptTensor>& index, const std::vector<int64_t>& nnum,
-                              const std::vector<int64_t>& nnum_nempty, int full_depth, int batch_size) {
-  const int depth = (int)keys.size() - 1;
+// The neighbour tables of layers 1 .. depth (entry 0 is left out) of an octree as `tree` was built; none if
+// a layer is not, any more: keys, children and counts are public and may be assigned.
+std::vector<Tensor> all_neigh(const Tree& tree, const std::vector<OptTensor>& keys_now, const std::vector<Tensor>& children,
+                              const std::vector<int64_t>& nnum, const std::vector<int64_t>& nnum_nempty, int full_depth,
+                              int batch_size) {
+  const int depth = (int)children.size() - 1;
   std::vector<Tensor> out;
+  if (children.size() != tree.children.size() || nnum != tree.nnum || nnum_nempty != tree.nnum_nempty) return out;
+  for (int d = 0; d <= depth; ++d)
+    if (!keys_now[d].has_value() || !tree.as_built(d, &*keys_now[d], children[d])) return out;
+  const std::vector<Tensor>& keys = tree.keys;
+  const std::vector<OptTensor>& index = tree.index;
   std::vector<const int64_t*> k;
   std::vector<const int32_t*> c, i;
   std::vector<int32_t*> o{nullptr};
@@ -718,16 +734,25 @@ PYBIND11_MODULE(ocnn_host, m) {
 #define FIELD(name) .def_readwrite(#name, &ConvLayer::name)
       FIELD(fwd) FIELD(dgrad) FIELD(wgrad) FIELD(fwd_table) FIELD(dgrad_table) FIELD(wgrad_table) FIELD(wgrad_of_grad)
 #undef FIELD
-      .def("with_table", [](const ConvLayer& layer, const Tensor& table) {
+      .def("with_table", [](const ConvLayer& layer, const Tensor& table, int64_t rows) {      // its first rows
+        at::AutoDispatchBelowADInplaceOrView below;
         auto copy = std::make_shared<ConvLayer>(layer);
-        copy->fwd_table = copy->dgrad_table = copy->wgrad_table = table;
+        copy->fwd_table = copy->dgrad_table = copy->wgrad_table = table.narrow(0, 0, rows);
         return copy;
       });
   py::class_<Tree>(m, "Tree")
 #define FIELD(name) .def_readonly(#name, &Tree::name)
       FIELD(keys) FIELD(children) FIELD(index) FIELD(nnum) FIELD(nnum_nempty) FIELD(idx) FIELD(points) FIELD(normals)
-          FIELD(perm) FIELD(seg_start);
+          FIELD(perm) FIELD(seg_start)
 #undef FIELD
+      .def("layers", [](Tree t) {                 // (what an octree keeps of it)
+        t.idx = t.points = t.perm = t.seg_start = Tensor();
+        t.normals.reset();
+        return t;
+      })
+      .def("as_built", [](const Tree& t, int64_t d, const Tensor& child, int64_t nnum_nempty) {
+        return t.as_built(d, nullptr, child) && t.index[d].has_value() && t.index[d]->numel() == nnum_nempty;
+      });
 #define FIELD(name) .def_readonly(#name, &BuiltPlan::name)
   py::class_<BuiltPlan>(m, "BuiltPlan")
       FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(ucount) FIELD(stats);

@@ -86,8 +86,8 @@ _IDENTITY = {}
 
 
 def _identity_table(rows, device):
-  """(rows, 1) table [0, 1, ..]: row i reads row i.  The head of one table per device and stream, as long as
-  the longest asked for (an eighth longer at most): row counts differ with every octree.  Of each stream its
+  """(rows or more, 1) table [0, 1, ..]: row i reads row i.  One per device and stream, as long as the
+  longest asked for (an eighth longer at most): row counts differ with every octree.  Of each stream its
   own, so that memory given back is not reused before its readers are done; under capture the graph's own."""
   key = (device, _lib.stream())
   table = _IDENTITY.get(key)
@@ -99,7 +99,7 @@ def _identity_table(rows, device):
       if len(_IDENTITY) > 16:
         _IDENTITY.clear()
       _IDENTITY[key] = table
-  return table[:rows]
+  return table
 
 
 _LINEAR = {}
@@ -125,9 +125,12 @@ def _rows_linear_layer(x, cin, cout):
     layer.dgrad = _gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True)
     layer.wgrad = _wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin])
     # (whole: other threads take it from here.  Without the table, which would outlive the octree)
-    made = _LINEAR[key] = (layer, any(_reads_table(op) for op in (layer.fwd, layer.dgrad, layer.wgrad)))
-  layer, table = made
-  return layer.with_table(_identity_table(rows, x.device)) if table else layer
+    forward = _reads_table(layer.fwd)
+    made = _LINEAR[key] = (layer, forward, forward or _reads_table(layer.dgrad) or _reads_table(layer.wgrad))
+  layer, forward, training = made
+  if training if torch.is_grad_enabled() else forward:
+    return layer.with_table(_identity_table(rows, x.device), rows)
+  return layer
 
 
 class _RowsLinearNarrow(torch.autograd.Function):
@@ -152,7 +155,7 @@ class _RowsLinearNarrow(torch.autograd.Function):
     if ctx.needs_input_grad[0]:
       gx = grad @ weight.to(grad.dtype)
     if ctx.needs_input_grad[1]:
-      gw = conv_wgrad(x, grad, _identity_table(rows, x.device), True, None, dense=True)
+      gw = conv_wgrad(x, grad, _identity_table(rows, x.device)[:rows], True, None, dense=True)
       gw = gw.view(weight.shape).to(weight.dtype)
     if ctx.has_bias and ctx.needs_input_grad[2]:
       gb = column_sum(grad)

@@ -655,6 +655,7 @@ class _Layer:
   runs holds the native object without the interpreter lock: that object is never changed, one with the
   further pass takes its place."""
 
+  @_lib.unrecorded
   def __init__(self, eng, dtype, padded):
     self.dtype, self.padded = dtype, padded    # padded: stride 2 over all nodes, octree_pad / octree_depad folded in
     self.conv = eng.is_conv_layer()
@@ -704,7 +705,6 @@ class _Layer:
         self.wgrad = made is not None
 
 
-@_lib.unrecorded
 def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
   """The layer's native passes, made at its first call on this octree and kept with it: (layer or
   None where the forward pass is not one native pass, function that makes its engine)."""
@@ -714,7 +714,6 @@ def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_siz
          SPARSE_MIN_ROWS)
   layer = octree._layers.get(key)
 
-  @_lib.unrecorded
   def made_engine():
     eng = engine(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
     eng.setup(octree, depth)

@@ -369,7 +369,7 @@ class Octree:
     self._tables_t = {}      # same key -> inverse table
     self._plans = {}         # (key, inverse) -> TilePlan
     self._layers = {}        # the layers' passes on this octree (nn/octree_conv.py)
-    self._built = {}         # depth -> what build_octree made of a layer (see _as_built)
+    self._built = None       # what build_octree made (a native Tree): says of a layer whether it still is that
     self._plans_prebuilt = False
 
     self.nnum = torch.zeros(num, dtype=torch.long)
@@ -387,7 +387,7 @@ class Octree:
   lut_kernel = _lut('lut_kernel', lambda dev: {k: torch.tensor(v, device=dev) for k, v in LUT_KERNEL.items()})
 
   def __getstate__(self):
-    return dict(vars(self), _layers={}, _built={})        # (native passes are made again when asked for)
+    return dict(vars(self), _layers={}, _built=None)        # (native passes are made again when asked for)
 
   # ---- cache bookkeeping ---------------------------------------------------
   def _drop_tables(self, depth, nempty_only=False):
@@ -407,7 +407,6 @@ class Octree:
     self.nempty_indices[depth] = None
     self.nempty_neighs[depth] = None
     self._nempty_indices32[depth] = None
-    self._built.pop(depth, None)
     self._drop_tables(depth, nempty_only=True)
 
   # ---- simple accessors (ocnn/octree/octree.py:108-145) ---------------------
@@ -428,21 +427,10 @@ class Octree:
       self.nempty_masks[depth] = self.children[depth] >= 0
     return self.nempty_masks[depth]
 
-  def _as_built(self, depth, nnum, nnum_nempty, keys=False):
-    """The layer is what build_octree made (and the index of its non-empty nodes from there with it): the octree
-    still holds its tensors, of these counts, and nobody wrote to them.  Children, keys and counts are public."""
-    built = self._built.get(depth)
-    if built is None:
-      return False
-    key, child, versions, index = built
-    return (self.children[depth] is child and child._version == versions[1] and child.shape[0] == nnum and
-            (index is None or index.shape[0] == nnum_nempty) and
-            (not keys or (self.keys[depth] is key and key._version == versions[0])))
-
   def _make_nempty_index(self, depth, reset=False):
     child, n = self.children[depth], int(self.nnum_nempty[depth])
-    if not reset and self._as_built(depth, int(self.nnum[depth]), n) and self._built[depth][3] is not None:
-      self._nempty_indices32[depth] = self._built[depth][3]
+    if not reset and self._built is not None and child is not None and self._built.as_built(depth, child, n):
+      self._nempty_indices32[depth] = self._built.index[depth]
       return
     _lib.require_gpu(child)
     i32 = torch.empty(n, dtype=torch.int32, device=child.device)
@@ -516,10 +504,7 @@ class Octree:
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
     self._nempty_indices32 = [None] * num
-    # (the writes to a tensor made in inference mode are not counted)
-    self._built = {d: (key, child, (key._version, child._version), index)
-                   for d, (key, child, index) in enumerate(zip(tree.keys, tree.children, tree.index))
-                   if not child.is_inference()}
+    self._built = tree.layers()
     self._tables, self._tables_t, self._plans, self._layers = {}, {}, {}, {}
     self._plans_prebuilt = False
     return tree.idx
@@ -639,10 +624,10 @@ class Octree:
         self.construct_neigh(d)
       return
     with torch.cuda.device(dev):
-      if all(self._as_built(d, nnum[d], nempty[d], keys=True) for d in range(depth + 1)):
-        index = [self._built[d][3] if d < depth else None for d in range(depth + 1)]
-        tables = _lib.native().all_neigh(self.keys[:depth + 1], self.children[:depth + 1], index, nnum, nempty,
-                                         self.full_depth, self.batch_size)
+      tables = [] if self._built is None else _lib.native().all_neigh(
+          self._built, self.keys[:depth + 1], self.children[:depth + 1], nnum, nempty, self.full_depth, self.batch_size)
+      if tables:
+        index = self._built.index
       else:                     # layers from elsewhere: one after the other, from their children alone
         tables = [torch.empty(n, 27, dtype=torch.int32, device=dev) for n in nnum[1:]]
         index = [torch.empty(nempty[d], dtype=torch.int32, device=dev) if self.full_depth <= d < depth else None
@@ -796,6 +781,8 @@ class Octree:
         walk(vars(v))
 
     walk(vars(self))
+    if self._built is not None:
+      walk(self._built.index)
     return self
 
   def _fine_rows(self, depth, nempty):
@@ -916,7 +903,7 @@ class Octree:
     self.nempty_indices = [None] * num
     self.nempty_neighs = [None] * num
     self._nempty_indices32 = [None] * num
-    self._tables, self._tables_t, self._plans, self._layers, self._built = {}, {}, {}, {}, {}
+    self._tables, self._tables_t, self._plans, self._layers, self._built = {}, {}, {}, {}, None
     low48 = (1 << 48) - 1
     for d in range(num):
       self.keys[d] = torch.cat([(o.keys[d] & low48) | (i << 48)
