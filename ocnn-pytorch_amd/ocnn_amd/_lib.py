@@ -4,7 +4,6 @@ There is no CPU fallback: if the library cannot be loaded the package raises.
 """
 
 import ctypes
-import functools
 import importlib.util
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_void_p, POINTER
 
@@ -182,24 +181,20 @@ def recorded():
   return _is_tracing() or _forward_ad._current_level >= 0 or _transforms_active()
 
 
-def unrecorded(make):
-  """For what a layer's first call makes and keeps (tables, plans, passes): no part of a trace, which
-  would hand out values of its own in place of sizes, and not under a transform of torch.func, which would
-  wrap the tensors that are kept."""
-  @functools.wraps(make)
-  def call(*args, **kwargs):
-    if _transforms_active():
-      raise RuntimeError('ocnn_amd layers are autograd.Functions that the transforms of torch.func do not support')
-    if not _is_tracing():
-      return make(*args, **kwargs)
-    state = torch._C._get_tracing_state()
-    torch._C._set_tracing_state(None)
-    try:
-      return make(*args, **kwargs)
-    finally:
-      torch._C._set_tracing_state(state)
-
-  return call
+def unrecorded(make, *args):
+  """make(*args) for what a layer's first call makes and keeps (tables, plans, passes): no part of a trace,
+  which would hand out values of its own in place of sizes, and not under a transform of torch.func, which
+  would wrap the tensors that are kept."""
+  if _transforms_active():
+    raise RuntimeError('ocnn_amd layers are autograd.Functions that the transforms of torch.func do not support')
+  if not _is_tracing():
+    return make(*args)
+  state = torch._C._get_tracing_state()
+  torch._C._set_tracing_state(None)
+  try:
+    return make(*args)
+  finally:
+    torch._C._set_tracing_state(state)
 
 
 class OcnnHipError(RuntimeError):

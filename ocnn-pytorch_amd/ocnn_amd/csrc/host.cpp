@@ -255,7 +255,7 @@ Tensor column_sum(Tensor g) {
 
 // The passes of one layer on one octree, in one data type.  fwd: data -> out; dgrad: grad -> data
 // gradient; wgrad over (data, grad), for a deconvolution over (grad, data).  The backward passes are
-// made when a call first needs them.
+// made when a call first needs them, as a copy with the pass: threads share the object.
 struct ConvLayer {
   std::shared_ptr<GatherOp> fwd, dgrad;
   std::shared_ptr<WgradOp> wgrad;
@@ -730,8 +730,26 @@ PYBIND11_MODULE(ocnn_host, m) {
         return op.run(x, g, or_undefined(table));
       });
   py::class_<ConvLayer, std::shared_ptr<ConvLayer>>(m, "ConvLayer")
-      .def(py::init<>())
-#define FIELD(name) .def_readwrite(#name, &ConvLayer::name)
+      .def(py::init([](std::shared_ptr<GatherOp> fwd, const OptTensor& table, bool wgrad_of_grad) {
+        auto layer = std::make_shared<ConvLayer>();
+        layer->fwd = std::move(fwd);
+        layer->fwd_table = or_undefined(table);
+        layer->wgrad_of_grad = wgrad_of_grad;
+        return layer;
+      }))
+      .def("with_dgrad", [](const ConvLayer& layer, std::shared_ptr<GatherOp> op, const OptTensor& table) {
+        auto copy = std::make_shared<ConvLayer>(layer);
+        copy->dgrad = std::move(op);
+        copy->dgrad_table = or_undefined(table);
+        return copy;
+      })
+      .def("with_wgrad", [](const ConvLayer& layer, std::shared_ptr<WgradOp> op, const OptTensor& table) {
+        auto copy = std::make_shared<ConvLayer>(layer);
+        copy->wgrad = std::move(op);
+        copy->wgrad_table = or_undefined(table);
+        return copy;
+      })
+#define FIELD(name) .def_readonly(#name, &ConvLayer::name)
       FIELD(fwd) FIELD(dgrad) FIELD(wgrad) FIELD(fwd_table) FIELD(dgrad_table) FIELD(wgrad_table) FIELD(wgrad_of_grad)
 #undef FIELD
       .def("with_table", [](const ConvLayer& layer, const Tensor& table, int64_t rows) {      // its first rows

@@ -110,7 +110,6 @@ def _reads_table(op):
   return (op.padded or op).kernel == _lib.GATHER_PLAIN       # (the same number as WGRAD_PLAIN)
 
 
-@_lib.unrecorded
 def _rows_linear_layer(x, cin, cout):
   """y = x W^T on many rows as the one-slot form of the convolution kernels (weights (out, in) as
   torch.nn.Linear holds them)."""
@@ -120,10 +119,9 @@ def _rows_linear_layer(x, cin, cout):
   if made is None:
     if len(_LINEAR) > 64:
       _LINEAR.clear()
-    layer = _lib.native().ConvLayer()
-    layer.fwd = _gather_op(x.dtype, rows, rows, 1, cin, cout, True, False, None, True)
-    layer.dgrad = _gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True)
-    layer.wgrad = _wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin])
+    layer = _lib.native().ConvLayer(_gather_op(x.dtype, rows, rows, 1, cin, cout, True, False, None, True), None, False)
+    layer = layer.with_dgrad(_gather_op(x.dtype, rows, rows, 1, cout, cin, False, False, None, True), None)
+    layer = layer.with_wgrad(_wgrad_op(x.dtype, rows, rows, 1, cin, cout, True, None, True).seen_as([cout, cin]), None)
     # (whole: other threads take it from here.  Without the table, which would outlive the octree)
     forward = _reads_table(layer.fwd)
     made = _LINEAR[key] = (layer, forward, forward or _reads_table(layer.dgrad) or _reads_table(layer.wgrad))
@@ -175,7 +173,7 @@ class Conv1x1(torch.nn.Module):
     lin = self.linear
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 4096 and lin.in_features % 32 == 0 and lin.out_features % 16 == 0):
-      return _rows_linear_layer(data, lin.in_features, lin.out_features)
+      return _lib.unrecorded(_rows_linear_layer, data, lin.in_features, lin.out_features)
     return None
 
   def forward(self, data: torch.Tensor):

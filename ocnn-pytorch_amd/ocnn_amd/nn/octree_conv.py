@@ -292,7 +292,6 @@ class OctreeConvBase:
   def is_conv_layer(self):
     raise NotImplementedError
 
-  @_lib.unrecorded
   def setup(self, octree, depth: int):
     """Heights of input/output and the table (ocnn/nn/octree_conv.py:51-100)."""
     # (an octree of another class gets its tables from its public members, octree/contract.py)
@@ -364,7 +363,6 @@ class OctreeConvBase:
     return cache[key]
 
   # The three passes as (native pass, table).  None: not one pass; the *_gemm methods put it together.
-  @_lib.unrecorded
   def forward_op(self, dtype, pad_to=None):
     """(fine rows, in_conv) -> (table rows, out_conv); see forward_gemm."""
     if self.dense_children:
@@ -378,7 +376,6 @@ class OctreeConvBase:
     plan = self._plan(dtype, self.fine_h, self.in_conv, self.out_conv)
     return _gather_op(dtype, self.fine_h, rows, K, self.in_conv, self.out_conv, False, False, plan), self.neigh
 
-  @_lib.unrecorded
   def backward_op(self, dtype, coarse_index=None, coarse_rows=0):
     """(table rows, out_conv) -> (fine rows, in_conv); see backward_gemm."""
     rows, K = self.neigh.shape
@@ -399,7 +396,6 @@ class OctreeConvBase:
     return (_gather_op(dtype, rows, self.fine_h, K, self.out_conv, self.in_conv, True, False, plan),
             self._inverse_table())
 
-  @_lib.unrecorded
   def weight_op(self, dtype, out_transposed=False, coarse_index=None, coarse_rows=0):
     """data (fine rows), grad (table rows) -> (K, in_conv, out_conv); see weight_gemm."""
     rows, K = self.neigh.shape
@@ -431,7 +427,7 @@ class OctreeConvBase:
   def forward_gemm(self, data, weights, bias=None, pad_to=None):
     """(fine rows, in_conv) -> (table rows, out_conv).  pad_to = (octree, depth): the result
     padded to all nodes of `depth` (octree_pad of the table rows)."""
-    made = self.forward_op(data.dtype, pad_to)
+    made = _lib.unrecorded(self.forward_op, data.dtype, pad_to)
     if made is not None:
       return made[0].run(data, made[1], weights, bias)
     return _pad_raw(self.forward_gemm(data, weights, bias), *pad_to)
@@ -440,7 +436,7 @@ class OctreeConvBase:
     """(table rows, out_conv) -> (fine rows, in_conv).  coarse_index (int32): `grad` holds the
     table's rows at these rows of a larger tensor (all nodes of the depth, not only the
     non-empty ones the table has rows for)."""
-    made = self.backward_op(grad.dtype, coarse_index, grad.shape[0])
+    made = _lib.unrecorded(lambda: self.backward_op(grad.dtype, coarse_index, grad.shape[0]))
     if made is not None:
       return made[0].run(grad, made[1], weights, bias)
     if coarse_index is not None:
@@ -507,7 +503,7 @@ class OctreeConvBase:
   def weight_gemm(self, data, grad, out_transposed=False, coarse_index=None):
     """data: fine rows; grad: table rows -> (K, in_conv, out_conv).  coarse_index: as in
     backward_gemm."""
-    made = self.weight_op(data.dtype, out_transposed, coarse_index, grad.shape[0])
+    made = _lib.unrecorded(lambda: self.weight_op(data.dtype, out_transposed, coarse_index, grad.shape[0]))
     if made is not None:
       return made[0].run(data, grad, made[1])
     if self.dense_children:
@@ -546,7 +542,7 @@ class OctreeConvFunction(Function):
               kernel_size: List[int] = [3, 3, 3], stride: int = 1, nempty: bool = False,
               max_buffer: int = int(2e8), bias=None, padded: bool = False):
     eng = _OctreeConv(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
-    eng.setup(octree, depth)
+    _lib.unrecorded(eng.setup, octree, depth)
     octree = eng.octree
     eng.check_and_init(data)
     data = data.contiguous()
@@ -585,7 +581,7 @@ class OctreeDeconvFunction(Function):
               kernel_size: List[int] = [3, 3, 3], stride: int = 1, nempty: bool = False,
               max_buffer: int = int(2e8), bias=None, padded: bool = False):
     eng = _OctreeDeconv(in_channels, out_channels, kernel_size, stride, nempty, max_buffer)
-    eng.setup(octree, depth)
+    _lib.unrecorded(eng.setup, octree, depth)
     octree = eng.octree
     index = None
     data = data.contiguous()
@@ -655,27 +651,16 @@ class _Layer:
   runs holds the native object without the interpreter lock: that object is never changed, one with the
   further pass takes its place."""
 
-  @_lib.unrecorded
   def __init__(self, eng, dtype, padded):
     self.dtype, self.padded = dtype, padded    # padded: stride 2 over all nodes, octree_pad / octree_depad folded in
     self.conv = eng.is_conv_layer()
     self.pad_depth = (eng.out_depth if self.conv else eng.in_depth) if padded else None
     self.shape = eng.in_shape if self.conv or not padded else (int(eng.octree.nnum[eng.in_depth]), eng.in_channels)
-    self._lock = threading.Lock()
-    self._made = {'wgrad_of_grad': not self.conv}
     self.dgrad = self.wgrad = None             # None = not made yet, False = not one pass
+    self._lock = threading.Lock()
     made = self._pass(eng, True)
     self.ok = made is not None                 # the forward pass is one native pass
-    self._add('fwd', made)
-
-  def _add(self, name, made):
-    """`made` (a pass and its table, or None) as the pass `name`, visible to other threads at once."""
-    if made is not None:
-      self._made[name], self._made[name + '_table'] = made
-    native = _lib.native().ConvLayer()
-    for field, value in self._made.items():
-      setattr(native, field, value)
-    self.native = native
+    self.native = _lib.native().ConvLayer(*made, not self.conv) if self.ok else None
 
   def _coarse(self, octree):
     """(index, rows) of the padded side: what the passes read the coarse rows through."""
@@ -688,20 +673,21 @@ class _Layer:
       return eng.forward_op(self.dtype, (eng.octree, self.pad_depth) if self.padded else None)
     return eng.backward_op(self.dtype, *self._coarse(eng.octree))
 
-  @_lib.unrecorded
-  def make_dgrad(self, eng):
+  def make_dgrad(self, make_engine):
     with self._lock:
       if self.dgrad is None:
-        made = self._pass(eng, False)
-        self._add('dgrad', made)
+        made = self._pass(make_engine(), False)
+        if made is not None:
+          self.native = self.native.with_dgrad(*made)
         self.dgrad = made is not None
 
-  @_lib.unrecorded
-  def make_wgrad(self, eng):
+  def make_wgrad(self, make_engine):
     with self._lock:
       if self.wgrad is None:
+        eng = make_engine()
         made = eng.weight_op(self.dtype, False, *self._coarse(eng.octree))
-        self._add('wgrad', made)
+        if made is not None:
+          self.native = self.native.with_wgrad(*made)
         self.wgrad = made is not None
 
 
@@ -720,7 +706,7 @@ def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_siz
     return eng
 
   if layer is None:
-    layer = octree._layers.setdefault(key, _Layer(made_engine(), data.dtype, padded))
+    layer = octree._layers.setdefault(key, _lib.unrecorded(lambda: _Layer(made_engine(), data.dtype, padded)))
   if not layer.ok:
     return None, None
   assert data.shape == layer.shape, \
@@ -741,11 +727,11 @@ def _apply(engine, function, data, weights, octree, depth, in_channels, out_chan
         ok = False
       if ok and data.requires_grad:
         if layer.dgrad is None:
-          layer.make_dgrad(made_engine())
+          _lib.unrecorded(layer.make_dgrad, made_engine)
         ok = layer.dgrad
       if ok and weights.requires_grad:
         if layer.wgrad is None:
-          layer.make_wgrad(made_engine())
+          _lib.unrecorded(layer.make_wgrad, made_engine)
         ok = layer.wgrad
     if ok:
       return call_native(layer.native, data, weights, bias)

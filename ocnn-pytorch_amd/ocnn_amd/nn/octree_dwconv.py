@@ -107,7 +107,7 @@ class OctreeDWConvFunction(Function):
               kernel_size: List[int] = [3, 3, 3], stride: int = 1, nempty: bool = False,
               max_buffer: int = int(2e8)):
     eng = OctreeDWConvBase(in_channels, kernel_size, stride, nempty, max_buffer)
-    eng.setup(octree, depth)
+    _lib.unrecorded(eng.setup, octree, depth)
     eng.check_and_init(data)
     data = data.contiguous()
     weights = weights.to(data.dtype).contiguous()

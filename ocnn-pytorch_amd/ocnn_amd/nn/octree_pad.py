@@ -13,10 +13,9 @@ def _children32(octree, depth):
   return children if children.dtype == torch.int32 and children.is_contiguous() else children.int().contiguous()
 
 
-@_lib.unrecorded
 def _rows(octree, depth):
   """(all nodes, non-empty nodes) of a layer."""
-  return int(octree.nnum[depth]), int(octree.nnum_nempty[depth])
+  return _lib.unrecorded(lambda: (int(octree.nnum[depth]), int(octree.nnum_nempty[depth])))
 
 
 def _pad_raw(data: torch.Tensor, octree, depth: int, val: float = 0.0):

@@ -36,8 +36,8 @@ def test_passes_made_by_several_threads():
   layer = _Layer(eng, torch.float16, False)
   held = layer.native                                    # what a running call holds, without the interpreter lock
   assert layer.ok and held.fwd is not None and held.dgrad is None
-  threads = [threading.Thread(target=layer.make_dgrad, args=(eng,)) for _ in range(2)]
-  threads += [threading.Thread(target=layer.make_wgrad, args=(eng,))]
+  threads = [threading.Thread(target=layer.make_dgrad, args=(lambda: eng,)) for _ in range(2)]
+  threads += [threading.Thread(target=layer.make_wgrad, args=(lambda: eng,))]
   for t in threads:
     t.start()
   assert eng.entered.wait(10)
