@@ -57,39 +57,20 @@ def parse():
   return ap.parse_args()
 
 
-class KernelTimer:
-  """Brackets every call of one library entry point with events on the stream
-  the kernels are launched on (torch's current stream)."""
-
-  def __init__(self, torch, module, name):
-    self.torch, self.module, self.name = torch, module, name
-    self.orig = getattr(module, name)
-    self.events = []
-    self.enabled = False
-
-    def wrapped(*a, **kw):
-      if not self.enabled:
-        return self.orig(*a, **kw)
-      s = torch.cuda.Event(enable_timing=True)
-      e = torch.cuda.Event(enable_timing=True)
+def pass_ms(torch, passes, rounds):
+  """Mean ms of each kind of pass and how many were timed: `passes` ((kind, call) pairs) one after the other,
+  `rounds` times, events around every call on the stream its kernels are launched on."""
+  spans = {}
+  for _ in range(rounds):
+    for kind, call in passes:
+      s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
       s.record()
-      out = self.orig(*a, **kw)
+      call()
       e.record()
-      self.events.append((s, e))
-      return out
-
-    setattr(module, name, wrapped)
-
-  def mean_ms(self):
-    if not self.events:
-      return None
-    return sum(s.elapsed_time(e) for s, e in self.events) / len(self.events)
-
-  def count(self):
-    return len(self.events)
-
-  def reset(self):
-    self.events = []
+      spans.setdefault(kind, []).append((s, e))
+  torch.cuda.synchronize()
+  mean = {kind: sum(s.elapsed_time(e) for s, e in v) / len(v) for kind, v in spans.items()}
+  return mean, {kind: len(v) for kind, v in spans.items()}
 
 
 def cpu_baseline(torch, table32, rows_in, cin, cout, sample_rows):
@@ -193,8 +174,6 @@ def main():
   x_dev = torch.randn(rows, C, generator=g).to(dev)
   gout_dev = torch.randn(rows, C, generator=g).to(dev)
 
-  t_gather = KernelTimer(torch, conv_mod, 'conv_gather')
-  t_wgrad = KernelTimer(torch, conv_mod, 'conv_wgrad')
   eng = conv_mod._OctreeConv(C, C, [3], 1, nempty)
   eng.setup(octree, depth)
 
@@ -219,17 +198,25 @@ def main():
         x.grad = None
         m.weights.grad = None
         m(x, oct, depth).backward(gout)
+
+    def passes():
+      """The passes that a step runs, each alone (after the first step)."""
+      if only != 'all':
+        return [('wgrad' if only == 'wgrad' else 'gather', step)]
+      layer, xd = m.native_layer(x, oct, depth), x.detach()
+      return [('gather', lambda: layer.fwd.run(xd, layer.fwd_table, w_cast, None)),
+              ('gather', lambda: layer.dgrad.run(gout, layer.dgrad_table, w_cast, None)),
+              ('wgrad', lambda: layer.wgrad.run(xd, gout, layer.wgrad_table))]
+
+    step.passes = passes
     return step
 
   def run_steps(step, steps, warmup):
-    """`warmup` untimed steps, then `steps` timed ones between synchronisations: ms per step,
-    and the mean launch times of the two kernel families (events around every launch)."""
+    """`warmup` untimed steps, then `steps` timed ones between synchronisations: ms per step.  Behind them
+    as many rounds of the step's passes: the mean times of the two kernel families and the number of gathers."""
     for _ in range(warmup):
       step()
     torch.cuda.synchronize()
-    t_gather.reset()
-    t_wgrad.reset()
-    t_gather.enabled = t_wgrad.enabled = True
     marks = [torch.cuda.Event(enable_timing=True) for _ in range(steps + 1)]
     t0 = time.perf_counter()
     marks[0].record()
@@ -238,10 +225,10 @@ def main():
       marks[i + 1].record()
     torch.cuda.synchronize()
     dt_s = time.perf_counter() - t0
-    t_gather.enabled = t_wgrad.enabled = False
     per_step = sorted(marks[i].elapsed_time(marks[i + 1]) for i in range(steps))
     run_steps.median_ms = per_step[len(per_step) // 2] if per_step else float('nan')
-    return dt_s * 1e3 / steps, t_gather.mean_ms(), t_wgrad.mean_ms(), t_gather.count()
+    mean, count = pass_ms(torch, step.passes(), steps)
+    return dt_s * 1e3 / steps, mean.get('gather'), mean.get('wgrad'), count.get('gather', 0)
 
   def timed_steps(dt, steps, warmup, oct=octree, only='all'):
     return run_steps(make_step(dt, oct, only), steps, warmup)
@@ -316,7 +303,8 @@ def main():
       'fraction_of_mfma_peak_whole_step': flops_step / (ms * 1e-3) / 1e12 / PEAK_MFMA_16BIT_TFLOPS,
       'roofline': {
           'kernel': 'conv_gather_rw_kernel (forward and data gradient; mean of both launches, '
-                    'each bracketed with its weight-pack pre-pass)',
+                    'each bracketed with its weight-pack pre-pass; the passes of a step, run K times by '
+                    'themselves right behind the timed steps)',
           'bound': 'mfma',
           'achieved': achieved,
           'peak': PEAK_MFMA_16BIT_TFLOPS,

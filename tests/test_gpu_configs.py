@@ -470,3 +470,20 @@ def test_the_ops_around_the_convolutions_on_more_than_2_31_elements():
     want[v] += xd[ts[v, k]].double() * w[k]
   say('   depth-wise convolution on %d rows: %.1e' % (n_ne, close(out.detach()[rows], want)))
 
+
+
+@pytest.mark.parametrize('dtype', ['bf16', 'fp16'])
+def test_bench_line_has_no_missing_figures(dtype, monkeypatch, capsys):
+  """bench.py on a small octree: one JSON line, every figure of the dominant kernels a number."""
+  import json
+  import bench
+
+  def refuse(text):
+    raise AssertionError(text)
+
+  monkeypatch.setattr(sys, 'argv', ['bench.py', '--points', '3000', '--depth', '6', '--batch', '2', '--steps', '2', '--warmup', '1',
+                                    '--dtype', dtype, '--no-cpu', '--no-extras'])
+  bench.main()
+  line = json.loads([l for l in capsys.readouterr().out.splitlines() if l.startswith('{')][-1], parse_constant=refuse)
+  assert line['value'] > 0 and line['steps'] == 2 and line['n_gpus'] == 1
+  assert line['roofline']['launches'] == 4 and line['roofline']['achieved'] > 0 and line['kernels']['conv_wgrad_ms'] > 0
