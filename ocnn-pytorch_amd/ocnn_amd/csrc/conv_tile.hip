@@ -1,5 +1,6 @@
-// Gather-GEMM on the tile plan of the neighbour table, with the weights streamed from L2: every
-// layer whose weights do not stay in registers (conv_rw.hip) and, in fp32, every planned layer.
+// Gather-GEMM on the tile plan of the neighbour table, with the weights streamed from L2: the
+// layers whose weights do not stay in registers (conv_rw.hip) and, in fp32, the planned layers
+// (which of them: select.hip).
 //
 // A workgroup takes one tile of 128 table rows and 32 .. 256 output channels.  The distinct input
 // rows of the tile are staged in LDS 128 bytes at a time (64 channels of f16 / bf16, 32 of fp32);
