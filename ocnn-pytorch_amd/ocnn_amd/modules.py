@@ -30,12 +30,15 @@ class _LayerBn(torch.nn.Module):
     return layer_bn(getattr(self, self._name), self.bn, data, *args)
 
 
-def _hooked(*modules):
-  """A call of one of the modules runs more than the forward() of its class: hooks, a forward put on the
-  module itself (as libraries that place modules on devices do), a compiled call."""
-  return (torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks or
-          any(m._forward_hooks or m._forward_pre_hooks or 'forward' in vars(m) or m._compiled_call_impl is not None
-              for m in modules))
+_nn = torch.nn.modules.module
+
+
+def _plain(module):
+  """A call of the module runs the forward() of its class and nothing else: no hooks, no forward put on the
+  module itself (as libraries that place modules on devices do), no compiled call."""
+  own = module.__dict__
+  return not (own['_forward_hooks'] or own['_forward_pre_hooks'] or 'forward' in own or
+              own.get('_compiled_call_impl') is not None)
 
 
 def layer_bn(layer, bn, data, *args, residual=None, relu=None):
@@ -43,7 +46,8 @@ def layer_bn(layer, bn, data, *args, residual=None, relu=None):
   batch norm of this package as they are, one native call: the normalisation then rides on the
   convolution's own pass over its result instead of reading and writing it once more."""
   if (not torch.is_grad_enabled() and not _lib.recorded() and type(bn) is BatchNormRelu1d and not bn.training and
-      bn.running_mean is not None and type(layer) in (OctreeConv, OctreeDeconv, Conv1x1) and not _hooked(layer, bn)):
+      bn.running_mean is not None and type(layer) in (OctreeConv, OctreeDeconv, Conv1x1) and _plain(layer) and _plain(bn) and
+      not (_nn._global_forward_hooks or _nn._global_forward_pre_hooks)):
     native = layer.native_layer(data, *args)
     if native is not None and _lib.lib().ocnn_batch_norm_supported(_lib.DTYPE_CODE[data.dtype], 2, bn.num_features):
       linear = layer.linear if type(layer) is Conv1x1 else None
