@@ -389,6 +389,10 @@ class Octree:
   def __getstate__(self):
     return dict(vars(self), _layers={}, _built=None)        # (native passes are made again when asked for)
 
+  def __setstate__(self, state):
+    # (an octree may have been saved before one of these was kept)
+    vars(self).update({'_layers': {}, '_built': None, '_lut_device': state.get('device', 'cpu')}, **state)
+
   # ---- cache bookkeeping ---------------------------------------------------
   def _drop_tables(self, depth, nempty_only=False):
     """Forgets what was derived from the tables of a layer (None: of every layer)."""
@@ -407,6 +411,7 @@ class Octree:
     self.nempty_indices[depth] = None
     self.nempty_neighs[depth] = None
     self._nempty_indices32[depth] = None
+    self._built = None         # (a layer is replaced: the build's tensors of it need not be held)
     self._drop_tables(depth, nempty_only=True)
 
   # ---- simple accessors (ocnn/octree/octree.py:108-145) ---------------------

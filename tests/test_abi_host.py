@@ -158,6 +158,18 @@ def test_lookup_tables_are_attributes():
   assert o.lut_parent.device.type == 'meta'
 
 
+def test_octree_saved_without_the_caches():
+  """An octree saved before the layers' passes and the build's record were kept with it loads and works."""
+  o = ocnn_amd.Octree(3, 2)
+  state = {k: v for k, v in o.__getstate__().items() if k not in ('_layers', '_built', '_lut_device')}
+  state['lut_kernel'] = {'222': torch.arange(8)}         # (it was an attribute of every octree)
+  loaded = ocnn_amd.Octree.__new__(ocnn_amd.Octree)
+  loaded.__setstate__(state)
+  loaded._drop_nempty(2)
+  assert loaded._layers == {} and loaded._built is None
+  assert loaded.lut_kernel['222'].tolist() == list(range(8)) and loaded.lut_parent.device.type == 'cpu'
+
+
 def test_batch_without_batch_ids_is_refused():
   points = ocnn_amd.Points(torch.rand(20, 3))
   points.batch_size = 2                                  # (set by hand: nothing says which point is whose)
