@@ -5,10 +5,12 @@
 // A workgroup takes one tile of 128 table rows and 32 .. 256 output channels.  The distinct input
 // rows of the tile are staged in LDS 128 bytes at a time (64 channels of f16 / bf16, 32 of fp32);
 // the weights stream straight into registers, already in the layout of the MFMA A operand (no LDS
-// round trip).  M = output channels, N = rows, v_mfma_f32_32x32x16.  The four waves split the
-// output channels (WR = 1), or, where a layer has fewer than 96 of them, the rows as well (WR = 2:
-// 64 output channels, WR = 4: 32): a wave owns 32 MB channels x 128 / WR rows.  Two workgroups
-// share a CU: while one waits for its next chunk of channels the other computes.
+// round trip).  M = output channels, N = rows, v_mfma_f32_32x32x16.  A wave owns 64 or 96 output channels of
+// 128 or 64 rows (32 of 128 where a layer has no more): a row read from LDS feeds two or three MFMAs and a weight
+// fetched four or two.  Layers of fewer channels than four such waves split the SLOTS over the waves instead, whose
+// sums are added in LDS at the end.  (Waves of 32 channels x 128 rows side by side read LDS once per MFMA, as fast
+// as its pipe delivers gathered rows: on the non-empty nodes of depth 7, 533 k rows, 128 -> 128 381 us, so 328.)
+// Two workgroups share a CU: while one waits for its next chunk of channels the other computes.
 //
 // fp32: x = hi + lo in bf16 pieces, accumulated in fp32 as hi hi + hi lo + lo hi (about 1e-5
 // relative).  The rows are read as fp32 and split on their way into LDS, so that a row's 128 bytes
@@ -18,9 +20,8 @@
 //
 // Few tiles (the coarse levels of a network, small clouds): 128 rows x 128 channels of 256 -> 256 are
 // 50 us of one workgroup's time however many CUs are idle.  The launch then also splits the
-// reduction, over chunks of input channels first (a chunk's rows are staged by one workgroup
-// either way) and over the slots; each part writes fp32 sums of its own, and a second kernel adds
-// them in the order of the parts.
+// reduction, over chunks of input channels and over the slots; each part writes fp32 sums of its own, and a
+// second kernel adds them in the order of the parts.
 #include <algorithm>
 #include <type_traits>
 
@@ -34,9 +35,10 @@ constexpr int kTgRows = 128;   // rows per tile (the plan's tile size)
 constexpr int kTgCap = 416;    // staged rows; plans with a larger tile use another kernel
 constexpr int kTgRowsAlloc = (kTgCap + 8) / 8 * 8;   // LDS rows 0..kTgCap in whole 8-row groups
 // share of a table's entries that are set up to which the kernel tests for empty (32-row block,
-// slot) units: at 32 - 38 % (the non-empty nodes of depths 7 and 6 of a depth-9 octree) a quarter
-// to a half of the units are empty and the launches are 3 - 14 % faster, at 41 - 50 % 0 - 7 % slower
-constexpr double kTgSkipMaxOccupancy = 0.40;
+// slot) units: non-empty nodes of coarse levels, where a tenth to a half of the units are empty.  With the test / without,
+// f16 and fp32, 64 to 256 channels: 0.83 - 0.93 at 22 % set, 0.84 - 0.95 at 36 %, 0.88 - 1.0 at 38 %, 0.96 - 1.0 at
+// 41 - 44 %, 0.99 - 1.03 at 50 - 58 %, 0.99 - 1.03 over all nodes (70 %)
+constexpr double kTgSkipMaxOccupancy = 0.45;
 
 // (Not in the kernel template: the arguments of the global->LDS load builtin must not be
 // type-dependent expressions.)
@@ -179,29 +181,30 @@ __device__ __forceinline__ void layer_tail(const O* bias, const ocnnx_bn& bn, in
 }
 
 // SKIP: per slot and 32-row block of the tile a wave asks whether any row has an entry there (a
-// ballot over the positions it reads anyway) and leaves the block's MFMAs out otherwise.  The
-// kernel is bound by the power its MFMAs draw (also those on zero rows), and the branches cost
-// 2 - 7 % where nothing is empty: it pays from about a quarter of the (block, slot) units empty -
-// the non-empty nodes of coarse levels -, which the launch decides from the table's occupancy.
+// ballot over the positions it reads anyway) and leaves the block's MFMAs out otherwise.  Blocks are the outer
+// loop of a slot, so that one branch stands around a block's 4 - 18 MFMAs: with the k-steps outside and a branch
+// per MFMA the same tables took 6 - 10 % longer.  The reads are not in the branch (they run a block ahead).
 //
-// blockIdx.z = part of the reduction: chunks c0 .. c1 - 1 of input channels, slots k0 .. k1 - 1.
-template <typename T, bool F32, int MB, int WR, bool SKIP>
-__global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
+// The four waves: WC along the output channels (32 MB each), WR along the rows (RB = 4 / WR blocks of 32 rows
+// each), KS over the slots (each takes every KS-th; their sums are added in LDS at the end).
+template <typename T, bool F32, int MB, int WC, int WR, int KS, bool SKIP>
+__global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_tile_kernel(
     const void* __restrict__ in, uint32_t in_bytes, const uint16_t* __restrict__ loc,
     const int32_t* __restrict__ uptr, const int32_t* __restrict__ urows, const T* __restrict__ wpk,
     const void* __restrict__ bias_, ocnnx_bn bn, void* __restrict__ out_, float* __restrict__ partial,
-    int64_t rows_out, int K, int cin, int cout, int64_t tiles, int64_t tiles_per_xcd, int sc, int sk) {
+    int64_t rows_out, int K, int cin, int cout, int64_t tiles, int64_t tiles_per_xcd, int sc, int sk, int rows_alloc) {
   typedef typename std::conditional<F32, float, T>::type O;
-  constexpr int RB = 4 / WR, WC = 4 / WR, CH = F32 ? 32 : 64;
-  __shared__ __attribute__((aligned(16))) char s_rows[kTgRowsAlloc * 128];
-  __shared__ __attribute__((aligned(16))) uint16_t s_loc[27 * kTgRows];
-  __shared__ int32_t s_u[kTgRowsAlloc];
+  constexpr int RB = 4 / WR, RBK = RB / KS, CH = F32 ? 32 : 64;
+  static_assert(WC * WR * KS == 4 && RB % KS == 0, "four waves");
+  extern __shared__ __attribute__((aligned(16))) char s_rows[];    // rows_alloc rows, positions, the list
+  uint16_t* s_loc = (uint16_t*)(s_rows + rows_alloc * 128);
+  int32_t* s_u = (int32_t*)(s_loc + ((K + sk - 1) / sk) * kTgRows);
 
   const int64_t tile = tiles_per_xcd > 0 ? xcd_tile(blockIdx.x, tiles_per_xcd) : (int64_t)blockIdx.x;
   if (tile >= tiles) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wc = wave % WC, wr = wave / WC;
+  const int wc = wave % WC, wr = wave / WC % WR, ks = wave / (WC * WR);
   const int q = lane >> 5, r32 = lane & 31;
   const int ncc = (cin + CH - 1) / CH;
   const int ncg = cout >> 5;
@@ -212,14 +215,22 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
   const int k0 = K * zk / sk, k1 = K * (zk + 1) / sk;
 
   // ---- the tile's list of distinct rows and its table positions -> LDS ----
-  const int32_t p0 = uptr[tile];
-  const int U = uptr[tile + 1] - p0;
-  for (int i = tid; i < kTgRowsAlloc; i += 256)
-    s_u[i] = (i >= 1 && i <= U) ? urows[p0 + i - 1] : -1;  // LDS row p holds list entry p - 1; row 0 = zeros
+  // (positions first: they don't wait for the list's place)
+  constexpr int LP = 27 * 16 / 256 + 1;
+  u32x4 lv[LP];
   {
     const u32x4* src = (const u32x4*)(loc + (tile * K + k0) * (int64_t)kTgRows);
-    for (int i = tid; i < (k1 - k0) * 16; i += 256) ((u32x4*)s_loc)[i] = src[i];
+#pragma unroll
+    for (int i = 0; i < LP; ++i)
+      if (tid + 256 * i < (k1 - k0) * 16) lv[i] = src[tid + 256 * i];
   }
+  const int32_t p0 = uptr[tile];
+  const int U = uptr[tile + 1] - p0;
+  for (int i = tid; i < rows_alloc; i += 256)
+    s_u[i] = (i >= 1 && i <= U) ? urows[p0 + i - 1] : -1;  // LDS row p holds list entry p - 1; row 0 = zeros
+#pragma unroll
+  for (int i = 0; i < LP; ++i)
+    if (tid + 256 * i < (k1 - k0) * 16) ((u32x4*)s_loc)[tid + 256 * i] = lv[i];
   const int groups = (U + 8) >> 3;                          // 8-row groups of LDS rows 0..U
 
   const __amdgpu_buffer_rsrc_t rs_in = make_rsrc(in, in_bytes);
@@ -240,22 +251,20 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
       for (int r = 0; r < 16; ++r) acc[rb][mb][r] = 0.f;
 
   // ---- operands ----
-  // A: weights of (chunk, slot), step s; one 16-byte load per lane and M tile
+  // A: the weights of a (chunk, slot), four pieces of 16 bytes a lane and M tile
   const int64_t kstride = (int64_t)ncg * 2048;               // elements between consecutive (chunk, slot)
-  const T* wbase = wpk + lane * 8;
   const bool active = cg0 < ncg;                             // (wave-uniform)
-  u32x4 A[4][MB];                                            // ring over the steps
-  auto load_a = [&](int kk, int s, u32x4 (&a)[MB]) {
-    const T* p = wbase + (int64_t)kk * kstride + s * 512;
+  const T* wbase[MB];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) a[mb] = *(const u32x4*)(p + (int64_t)min(cg0 + mb, ncg - 1) * 2048);
-  };
-  // the (chunk, slot) after (cc, k) of this part (after the last one: itself, unused)
-  auto next_kk = [&](int cc, int k) {
-    return k + 1 < k1 ? cc * K + k + 1 : (cc + 1 < c1 ? (cc + 1) * K + k0 : cc * K + k);
+  for (int mb = 0; mb < MB; ++mb) wbase[mb] = wpk + lane * 8 + (int64_t)min(cg0 + mb, ncg - 1) * 2048;
+  auto load_a = [&](int kk, u32x4 (&a)[4][MB]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) a[s][mb] = *(const u32x4*)(wbase[mb] + (int64_t)kk * kstride + s * 512);
   };
   // B: a lane reads 16 bytes (8 input channels, or their high or low pieces) of the neighbour row of
-  // row 32 rb + r32.  pv = byte address of the row in s_rows with the swizzle of step 0 folded in.
+  // row 32 rb + r32.  pv = byte address of the row in s_rows with the swizzle of piece 0 folded in.
   const uint16_t* lcw = s_loc + 32 * RB * wr + r32;
   uint32_t pvc[RB], pvn[RB];
   // (SKIP) which 32-row blocks of the tile have an entry in the slot at all, wave-uniform
@@ -271,70 +280,77 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
       if constexpr (SKIP) nz[rb] = __builtin_amdgcn_ballot_w64(l != 0u) != 0ull;
     }
   };
-  auto read_b = [&](const uint32_t (&pv)[RB], int s, u32x4 (&b)[RB]) {
+  auto read_b = [&](uint32_t pv, u32x4 (&b)[4]) {
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) b[rb] = *(const u32x4*)(s_rows + (pv[rb] ^ ((uint32_t)s << 5)));
+    for (int s = 0; s < 4; ++s) b[s] = *(const u32x4*)(s_rows + (pv ^ ((uint32_t)s << 5)));
   };
-  auto multiply = [&](const u32x4 (&a)[MB], const u32x4 (&b)[RB]) {
-    if (active) {
+  // a block of 32 rows with everything of a slot: behind one branch
+  auto multiply = [&](const u32x4 (&a)[4][MB], const u32x4 (&b)[4], f32x16 (&c)[MB], auto STEPS) {
+    constexpr int S = decltype(STEPS)::value;
+    auto mma = [&](int i, int j) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-        if (!SKIP || nzc[rb]) {
+      for (int mb = 0; mb < MB; ++mb) c[mb] = Mma32<T>::run(a[i][mb], b[j], c[mb]);
+    };
+    if constexpr (F32) {                                     // pieces 0, 1 of a: high, low of k-step 0; 0, 2 of b
+      mma(0, 0), mma(0, 2), mma(1, 0);
+      mma(2, 1), mma(2, 3), mma(3, 1);
+    } else {
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb) acc[rb][mb] = Mma32<T>::run(a[mb], b[rb], acc[rb][mb]);
-        }
-    }
-  };
-  auto advance = [&]() {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      pvc[rb] = pvn[rb];
-      if constexpr (SKIP) nzc[rb] = nzn[rb];
+      for (int s = 0; s < S; ++s) mma(s, s);
     }
   };
 
   // the distinct rows' channels of chunk cc -> LDS
-  // the list entries of this lane's pieces, read once for all chunks (one LDS wait, not one per piece)
   __syncthreads();
-  int32_t ids[kRowPieces];
-#pragma unroll
-  for (int i = 0; i < kRowPieces; ++i) ids[i] = s_u[min(st_p + 32 * i, kTgRowsAlloc - 1)];   // -1: out of range, loads zeros
   auto stage_chunk = [&](int cc) {
     if constexpr (F32) {
       // fp32 rows through registers, split into their bf16 pieces on the way: a lane's four channels
       // 4 (lane % 8) .. are half a 16-byte chunk of either piece
-      f32x4 v[kRowPieces];
-#pragma unroll
-      for (int i = 0; i < kRowPieces; ++i)
+      constexpr int D = 7;                                   // loads in flight
+      f32x4 v[D];
+      auto load = [&](int i, f32x4& x) {
         if (wave + 4 * i < groups)
-          v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rs_in, (uint32_t)ids[i] * pitch + (uint32_t)cc * 128u + (uint32_t)(lane & 7) * 16u, 0, 0));
+          x = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rs_in, (uint32_t)s_u[st_p + 32 * i] * pitch + (uint32_t)cc * 128u + (uint32_t)(lane & 7) * 16u, 0, 0));
+      };
+#pragma unroll
+      for (int i = 0; i < D; ++i) load(i, v[i]);
       __syncthreads();                                       // every wave is done with the chunk before
       const uint32_t half = (uint32_t)(lane & 1) * 8u, ch = (uint32_t)(lane & 7) >> 1;
 #pragma unroll
-      for (int i = 0; i < kRowPieces; ++i)
+      for (int i = 0; i < kRowPieces; ++i) {
         if (wave + 4 * i < groups) {
           typedef __attribute__((ext_vector_type(4))) T t4;
           t4 hi, lo;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            hi[j] = (T)v[i][j];
-            lo[j] = (T)(v[i][j] - (float)hi[j]);
+            hi[j] = (T)v[i % D][j];
+            lo[j] = (T)(v[i % D][j] - (float)hi[j]);
           }
           char* row = s_rows + (st_p + 32 * i) * 128;
           *(t4*)(row + (ch ^ st_x) * 16u + half) = hi;
           *(t4*)(row + ((ch | 4u) ^ st_x) * 16u + half) = lo;
         }
+        if (i + D < kRowPieces) load(i + D, v[i % D]);
+      }
       __syncthreads();
     } else {
       __syncthreads();                                       // every wave is done with the chunk before
+      // (list entries in two halves: registers)
+      constexpr int D = (kRowPieces + 1) / 2;
 #pragma unroll
-      for (int i = 0; i < kRowPieces; ++i) {
-        const int g = wave + 4 * i;
-        if (g < groups) {
-          uint32_t off = (uint32_t)ids[i] * pitch + ((uint32_t)cc * 128u + st_c);
-          if (cc == ncc - 1 && half_oob) off = 0xffffff00u;  // past the row's channels: zeros, not the next row
-          tg_dma16(rs_in, s_rows + g * 1024, off);
+      for (int h = 0; h < kRowPieces; h += D) {
+        int32_t ids[D];
+#pragma unroll
+        for (int i = 0; i < D; ++i) ids[i] = s_u[min(st_p + 32 * (h + i), rows_alloc - 1)];   // -1: out of range, loads zeros
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+          const int g = wave + 4 * (h + i);
+          if (h + i < kRowPieces && g < groups) {
+            uint32_t off = (uint32_t)ids[i] * pitch + ((uint32_t)cc * 128u + st_c);
+            if (cc == ncc - 1 && half_oob) off = 0xffffff00u;  // past the row's channels: zeros, not the next row
+            tg_dma16(rs_in, s_rows + g * 1024, off);
+          }
         }
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -342,87 +358,81 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
     }
   };
 
-  if constexpr (F32) {
-    // weights in pairs (high, low piece of a k-step), fetched one k-step ahead
-    u32x4 Bh[2][RB], Bl[2][RB];
-    auto load_pair = [&](int kk, int j) {
-      load_a(kk, 2 * j, A[2 * j]);
-      load_a(kk, 2 * j + 1, A[2 * j + 1]);
-    };
-    load_pair(c0 * K + k0, 0);
-    for (int cc = c0; cc < c1; ++cc) {
-      stage_chunk(cc);
-      load_pos(k0, pvc, nzc);
-      read_b(pvc, 0, Bh[0]);
-      read_b(pvc, 2, Bl[0]);
-      for (int k = k0; k < k1; ++k) {
-        load_pos(k + 1 < k1 ? k + 1 : k0, pvn, nzn);
-        load_pair(cc * K + k, 1);
-        read_b(pvc, 1, Bh[1]);
-        read_b(pvc, 3, Bl[1]);
-        multiply(A[0], Bh[0]);
-        multiply(A[0], Bl[0]);
-        multiply(A[1], Bh[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        load_pair(next_kk(cc, k), 0);
-        read_b(pvn, 0, Bh[0]);                               // (past the last slot: unused)
-        read_b(pvn, 2, Bl[0]);
-        multiply(A[2], Bh[1]);
-        multiply(A[2], Bl[1]);
-        multiply(A[3], Bh[1]);
-        __builtin_amdgcn_sched_barrier(0);
-        advance();
-      }
+  u32x4 A[4][MB], B[2][4];
+  const int kw = k0 + ks;                                    // this wave's slots: kw, kw + KS, ..
+  auto chunk = [&](int cc, auto STEPS) {
+    if (kw < k1) {                                           // (in flight while the rows come)
+      load_a(cc * K + kw, A);
+      load_pos(kw, pvc, nzc);
     }
-  } else {
-    u32x4 Bb[2][RB];
-    const int nfull = min(c1, cin >> 6);                     // whole 64-channel chunks up to here
-    load_a(c0 * K + k0, 0, A[0]);
-    load_a(c0 * K + k0, 1, A[1]);
-    for (int cc = c0; cc < nfull; ++cc) {
-      stage_chunk(cc);
-      load_pos(k0, pvc, nzc);
-      read_b(pvc, 0, Bb[0]);
-      for (int k = k0; k < k1; ++k) {
-        const int kk = cc * K + k, kn = next_kk(cc, k);
+    stage_chunk(cc);
+    if (kw < k1) {
+      read_b(pvc[0], B[0]);
+      for (int k = kw; k < k1; k += KS) {
+        const int kn = k + KS < k1 ? k + KS : kw;            // (past the last slot: fetched, unused)
+        u32x4 An[4][MB];
+        load_pos(kn, pvn, nzn);
+        load_a(cc * K + kn, An);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          // fetches: positions of the next slot, weights two k-steps ahead, rows one k-step ahead
-          if (s == 0) load_pos(k + 1 < k1 ? k + 1 : k0, pvn, nzn);
-          load_a(s >= 2 ? kn : kk, (s + 2) & 3, A[(s + 2) & 3]);
-          if (s < 3) read_b(pvc, s + 1, Bb[(s + 1) & 1]);
-          else read_b(pvn, 0, Bb[0]);                        // (past the last slot: unused)
-          multiply(A[s], Bb[s & 1]);
+        for (int rb = 0; rb < RB; ++rb) {
+          read_b(rb + 1 < RB ? pvc[rb + 1 < RB ? rb + 1 : 0] : pvn[0], B[(rb + 1) & 1]);
+          if (active && (!SKIP || nzc[rb])) multiply(A, B[rb & 1], acc[rb], STEPS);
           __builtin_amdgcn_sched_barrier(0);
         }
-        advance();
+        if constexpr (RB & 1) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) B[0][s] = B[1][s];
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) A[s][mb] = An[s][mb];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          pvc[rb] = pvn[rb];
+          if constexpr (SKIP) nzc[rb] = nzn[rb];
+        }
       }
     }
-    if (nfull < c1) {
-      // Half a chunk at the end (cin % 64 == 32): two k-steps per slot instead of four.  The
-      // weights of a slot sit in one pair of the ring while the next slot's go into the other,
-      // so the slots are taken two at a time (the chunk before left the first pair filled).
-      const int cc = nfull;
-      stage_chunk(cc);
-      load_pos(k0, pvc, nzc);
-      read_b(pvc, 0, Bb[0]);
-      auto half_slot = [&](int k, auto ring) {
-        constexpr int r = decltype(ring)::value;             // this slot's pair of the ring: 0 or 2
-        const int kn = next_kk(cc, k);
+  };
+  const int nfull = F32 ? c1 : min(c1, cin >> 6);            // whole chunks up to here
+  for (int cc = c0; cc < nfull; ++cc) chunk(cc, std::integral_constant<int, 4>{});
+  if constexpr (!F32)
+    if (nfull < c1) chunk(nfull, std::integral_constant<int, 2>{});   // half a chunk: its first two k-steps
+
+  // ---- KS > 1: the waves' sums of a block are added by one of them, in the order of the waves ----
+  if constexpr (KS > 1) {
+    f32x4* ex = (f32x4*)s_rows;
+    const int pair = wave % (WC * WR);
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          if (s == 0) load_pos(k + 1 < k1 ? k + 1 : k0, pvn, nzn);
-          load_a(kn, s, A[(r ^ 2) + s]);
-          if (s == 0) read_b(pvc, 1, Bb[1]);
-          else read_b(pvn, 0, Bb[0]);                        // (past the last slot: unused)
-          multiply(A[r + s], Bb[s]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        advance();
-      };
-      for (int k = k0; k < k1; k += 2) {
-        half_slot(k, std::integral_constant<int, 0>{});
-        if (k + 1 < k1) half_slot(k + 1, std::integral_constant<int, 2>{});
+    for (int o = 0; o < KS; ++o) {                           // owner of blocks RBK o ..
+      __syncthreads();
+      if (ks != o) {
+        const int from = ks < o ? ks : ks - 1;
+#pragma unroll
+        for (int i = 0; i < RBK; ++i)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              ex[((((from * WC * WR + pair) * RBK + i) * MB + mb) * 4 + r) * 64 + lane] =
+                  f32x4{acc[RBK * o + i][mb][4 * r], acc[RBK * o + i][mb][4 * r + 1], acc[RBK * o + i][mb][4 * r + 2],
+                        acc[RBK * o + i][mb][4 * r + 3]};
+      }
+      __syncthreads();
+      if (ks == o) {
+#pragma unroll
+        for (int f = 0; f < KS - 1; ++f)
+#pragma unroll
+          for (int i = 0; i < RBK; ++i)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const f32x4 v = ex[((((f * WC * WR + pair) * RBK + i) * MB + mb) * 4 + r) * 64 + lane];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[RBK * o + i][mb][4 * r + j] += v[j];
+              }
       }
     }
   }
@@ -433,14 +443,17 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
     if (cg0 + mb >= ncg) continue;
     const int co = 32 * (cg0 + mb) + 16 * q;
     if (partial) {
+      // [part][16-channel group][4-channel quarter][row][4]: the lanes of a store are consecutive rows
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
+        if (KS > 1 && rb / RBK != ks) continue;
         const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
         if (row >= rows_out) continue;
-        float* dst = partial + ((int64_t)blockIdx.z * rows_out + row) * cout + co;
+        float* dst = partial + (((int64_t)blockIdx.z * (cout >> 2) + (co >> 2)) * rows_out + row) * 4;
 #pragma unroll
-        for (int r = 0; r < 16; r += 4)
-          *(f32x4*)(dst + r) = f32x4{acc[rb][mb][r], acc[rb][mb][r + 1], acc[rb][mb][r + 2], acc[rb][mb][r + 3]};
+        for (int r = 0; r < 4; ++r)
+          *(f32x4*)(dst + r * rows_out * 4) =
+              f32x4{acc[rb][mb][4 * r], acc[rb][mb][4 * r + 1], acc[rb][mb][4 * r + 2], acc[rb][mb][4 * r + 3]};
       }
       continue;
     }
@@ -448,6 +461,7 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
     layer_tail<O, 16>((const O*)bias_, bn, co, mul, add);
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
+      if (KS > 1 && rb / RBK != ks) continue;
       const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
       if (row >= rows_out) continue;
       float v[16];
@@ -478,24 +492,29 @@ __global__ __launch_bounds__(256, 2) void conv_gather_tile_kernel(
   }
 }
 
-// out = sum of the parts, in their order, and what follows (layer_tail); four consecutive values a thread
+// out = sum of the parts, in their order, and what follows (layer_tail); four consecutive channels a thread, eight
+// threads a row's 32 channels, so that a wave reads 128 bytes of consecutive rows at a time and writes 64 - 128.
 template <typename O>
-__global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict__ partial, int parts, int64_t n, int cout,
+__global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict__ partial, int parts, int64_t rows, int cout,
                                                          const O* __restrict__ bias, ocnnx_bn bn, O* __restrict__ out) {
-  const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (e >= n) return;
-  f32x4 acc = *(const f32x4*)(partial + e);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t row = t >> 3;
+  const int c4 = (int)blockIdx.y * 8 + (int)(t & 7);         // four channels
+  if (row >= rows) return;
+  const int64_t n = rows * cout, e = row * cout + 4 * c4;
+  const float* src = partial + ((int64_t)c4 * rows + row) * 4;
+  f32x4 acc = *(const f32x4*)src;
   int s = 1;
   for (; s + 4 <= parts; s += 4) {                           // four loads in flight
     f32x4 v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = *(const f32x4*)(partial + (s + u) * n + e);
+    for (int u = 0; u < 4; ++u) v[u] = *(const f32x4*)(src + (s + u) * n);
 #pragma unroll
     for (int u = 0; u < 4; ++u) acc += v[u];
   }
-  for (; s < parts; ++s) acc += *(const f32x4*)(partial + s * n + e);
+  for (; s < parts; ++s) acc += *(const f32x4*)(src + s * n);
   float mul[4], add[4];
-  layer_tail<O, 4>(bias, bn, (int)(e % cout), mul, add);
+  layer_tail<O, 4>(bias, bn, 4 * c4, mul, add);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     acc[i] = acc[i] * mul[i] + add[i];
@@ -510,36 +529,50 @@ __global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict
 }
 
 struct TileLaunch {
-  int mb, wr;                  // shape of a wave (see above)
+  int mb, wc, wr, ks;          // shape of a wave: 32 mb channels x 128 / wr rows, every ks-th slot; wc waves along the channels
   int gy;                      // blocks of output channels
   int sc, sk;                  // parts of the reduction: chunks x slots
 };
 
-// How a launch is cut up.  WR by the output channels (96 or more keep three of the four waves busy
-// along them); 256 channels a workgroup halve the LDS reads per MFMA where there are tiles enough.
-//
-// The reduction is split while the launch stays within the workgroups that run at once: one a CU for
-// short ones, whose time is latency (up to 64 (chunk, slot) units of 16 MFMAs a wave; an fp32 unit
-// counts half as much again), two for longer ones, and rounds of them from 200 units on, where
-// the last, half-empty round costs more than the parts' sums.  A part keeps at least kTgMinUnits units:
-// below that staging the rows is all it does.  Measured (us, 3x3x3, 17 - 22 % occupied, one part -> split): fp16
-// 256 -> 256 on 1 / 30 / 100 tiles 72 -> 18, 72 -> 37, 74 -> 65, 128 -> 128 on 1 / 30 / 64 tiles 38 -> 15, 37 -> 25,
-// 37 -> 31 and no gain from 150 on; fp32 256 -> 256 on 30 / 150 / 300 tiles 170 -> 52, 230 -> 171, 379 -> 310.
-constexpr int kTgMinUnits = 6;
+// What a launch of few tiles takes, in us, cut into sc x sk parts: rounds of the workgroups that run at once
+// (two a CU), each of them its rows' staging and its waves' slots one behind the other, and the parts' sums
+// written and read.  A slot takes the longer of its MFMAs (half as long again with a second workgroup on the CU)
+// and a round trip for the next slot's weights.  The constants are a fit to 670 timed launches (2 - 324 tiles, seven
+// pairs of channels, f16 and fp32, 1 - 32 parts): 7 % off in the mean, and the parts it picks take 1.3 % longer
+// than the best ones; a rule by thresholds on units and workgroups took 6 %.
+static double tile_cost(const TileLaunch& t, bool f32, int64_t tiles, int K, int ncc, int cout, int sc, int sk) {
+  const double kLaunch = 8.8, kParts = 3.8, kPartBytes = 1.8e-7, kChunk = 0.96, kSlot = 0.245, kMfma = 0.0228;
+  const int chunks = (int)cdiv(ncc, sc), slots = chunks * (int)cdiv(cdiv(K, sk), t.ks);
+  const double mfma = kMfma * t.mb * (4 / t.wr) * (f32 ? 6 : 4);
+  auto round = [&](int per_cu) { return chunks * kChunk + slots * std::max(kSlot, mfma * (0.5 + 0.5 * per_cu)); };
+  const int64_t groups = tiles * t.gy * sc * sk, rest = groups % 512;
+  const double us = kLaunch + (double)(groups / 512) * round(2) + (rest == 0 ? 0.0 : round(rest <= 256 ? 1 : 2));
+  return sc * sk == 1 ? us : us + kParts + kPartBytes * sc * sk * (double)tiles * kTgRows * cout * 8;
+}
+
+// How a launch is cut up.  256 channels a workgroup stage a tile's rows once for all of them where there are tiles
+// enough.  From some 600 workgroups on the last, half-empty round costs less than the sums.
+constexpr int kTgPartsGroups = 640;
+constexpr int kTgMaxSlotParts = 6;
 
 static TileLaunch tile_launch(bool f32, int64_t tiles, int K, int cin, int cout) {
-  TileLaunch t{1, 1, 1, 1, 1};
-  t.wr = cout <= 32 ? 4 : (cout <= 64 ? 2 : 1);
-  if (!f32 && cout % 256 == 0 && tiles * (cout / 256) > 256) t.mb = 2;
-  t.gy = (int)cdiv(cout, 128 / t.wr * t.mb);
-  const int64_t blocks = tiles * t.gy;
+  TileLaunch t{1, 1, 1, 4, 1, 1, 1};                         // 32 channels
+  if (cout % 256 == 0 && tiles * (cout / 256) > 256) t.mb = 2, t.wc = 4, t.ks = 1;
+  else if (cout % 96 == 0) t.mb = 3, t.wr = 2, t.ks = 2;
+  else if (cout > 64) t.mb = 2, t.wc = 2, t.ks = 2;
+  else if (cout > 32) t.mb = 2;
+  t.gy = (int)cdiv(cout, 32 * t.mb * t.wc);
   const int ncc = (int)cdiv(cin, f32 ? 32 : 64);
-  const int units = ncc * K * (f32 ? 3 : 2) / 2;
-  const int64_t target = units <= 64 ? 256 : (units < 200 ? 512 : 1200);
-  if (blocks > 0 && blocks * 2 <= target) {
-    const int want = (int)std::min<int64_t>(target / blocks, std::max(1, ncc * K / kTgMinUnits));
-    t.sc = std::max(1, std::min(ncc, want));
-    t.sk = std::max(1, std::min(K, want / t.sc));
+  if (tiles > 0 && tiles * t.gy <= kTgPartsGroups) {
+    double best = 0.95 * tile_cost(t, f32, tiles, K, ncc, cout, 1, 1);   // (parts have to be worth it)
+    for (int sc = 1; sc <= ncc; ++sc) {
+      if (sc > 1 && cdiv(ncc, sc) == cdiv(ncc, sc - 1)) continue;        // (no fewer chunks a part)
+      for (int sk = 1; sk <= std::min(K, kTgMaxSlotParts) && tiles * t.gy * sc * sk <= 2048; ++sk) {
+        if (sk > 1 && cdiv(cdiv(K, sk), t.ks) == cdiv(cdiv(K, sk - 1), t.ks)) continue;   // (no fewer slots a wave)
+        const double us = tile_cost(t, f32, tiles, K, ncc, cout, sc, sk);
+        if (us < best) best = us, t.sc = sc, t.sk = sk;
+      }
+    }
   }
   return t;
 }
@@ -569,7 +602,7 @@ extern "C" int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out
 }
 
 template <typename T, bool F32>
-static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr, const int32_t* urows,
+static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr, const int32_t* urows, int umax,
                     int64_t rows_out, int K, int cin, int cout, const void* w, int w_transposed, int reverse,
                     const void* bias, const ocnnx_bn& bn, void* out, void* ws, int64_t ws_bytes, bool skip, int split_c,
                     int split_k, hipStream_t st) {
@@ -597,23 +630,27 @@ static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const 
   const int64_t per_xcd = parts > 1 ? 0 : cdiv(tiles, 8);
   const dim3 grid((unsigned)(per_xcd > 0 ? per_xcd * 8 : tiles), (unsigned)t.gy, (unsigned)parts);
   const uint32_t in_bytes = (uint32_t)(rows_in * cin * sizeof(O));
-#define OCNN_TILE_LAUNCH(MB_, WR_, SKIP_)                                                                           \
-  hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WR_, SKIP_>), grid, dim3(256), 0, st, in, in_bytes, loc, \
-                     uptr, urows, (const T*)ws, bias, bn, out, partial, rows_out, K, cin, cout, tiles, per_xcd, t.sc, t.sk)
-#define OCNN_TILE_CASE(MB_, WR_)           \
-  if (t.mb == MB_ && t.wr == WR_) {        \
-    if (skip) OCNN_TILE_LAUNCH(MB_, WR_, true); \
-    else OCNN_TILE_LAUNCH(MB_, WR_, false);     \
+  const int rows_alloc = std::max((umax + 8) / 8 * 8, 1);
+  // LDS: rows, positions, list; at the end the waves' sums
+  const int kmax = (K + t.sk - 1) / t.sk;
+  const size_t lds = std::max<size_t>((size_t)rows_alloc * 132 + (size_t)kmax * kTgRows * 2,
+                                      (size_t)(t.ks - 1) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
+#define OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, SKIP_)                                                                 \
+  hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WC_, WR_, KS_, SKIP_>), grid, dim3(256), lds, st, in,    \
+                     in_bytes, loc, uptr, urows, (const T*)ws, bias, bn, out, partial, rows_out, K, cin, cout, tiles, \
+                     per_xcd, t.sc, t.sk, rows_alloc)
+#define OCNN_TILE_CASE(MB_, WC_, WR_, KS_)                                   \
+  if (t.mb == MB_ && t.wc == WC_ && t.wr == WR_ && t.ks == KS_) {            \
+    if (skip) OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, true);                    \
+    else OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, false);                        \
   }
-  OCNN_TILE_CASE(1, 1) OCNN_TILE_CASE(1, 2) OCNN_TILE_CASE(1, 4)
-  if constexpr (!F32) {
-    OCNN_TILE_CASE(2, 1)
-  }
+  OCNN_TILE_CASE(1, 1, 1, 4) OCNN_TILE_CASE(2, 1, 1, 4) OCNN_TILE_CASE(3, 1, 2, 2) OCNN_TILE_CASE(2, 2, 1, 2)
+  OCNN_TILE_CASE(2, 4, 1, 1)
 #undef OCNN_TILE_CASE
 #undef OCNN_TILE_LAUNCH
   if (partial)
-    hipLaunchKernelGGL(tile_parts_kernel<O>, dim3((unsigned)cdiv(rows_out * cout / 4, 256)), dim3(256), 0, st, partial,
-                       parts, rows_out * cout, cout, (const O*)bias, bn, (O*)out);
+    hipLaunchKernelGGL(tile_parts_kernel<O>, dim3((unsigned)cdiv(rows_out * 8, 256), (unsigned)(cout / 32)), dim3(256), 0, st,
+                       partial, parts, rows_out, cout, (const O*)bias, bn, (O*)out);
   return check_launch("conv_gather_tile");
 }
 
@@ -639,12 +676,12 @@ extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, con
   // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
   const bool skip = K != 8 && plan_occupancy >= 0.0 && plan_occupancy <= kTgSkipMaxOccupancy;
   if (dtype == OCNN_F32)
-    return run_tile<bf16, true>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
+    return run_tile<bf16, true>(in, rows_in, loc, uptr, urows, plan_max_distinct, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
                                 bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
   if (dtype == OCNN_F16)
-    return run_tile<f16, false>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
+    return run_tile<f16, false>(in, rows_in, loc, uptr, urows, plan_max_distinct, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
                                 bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
-  return run_tile<bf16, false>(in, rows_in, loc, uptr, urows, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
+  return run_tile<bf16, false>(in, rows_in, loc, uptr, urows, plan_max_distinct, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
                                bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
 }
 

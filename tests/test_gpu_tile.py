@@ -53,6 +53,30 @@ def test_tile_kernel(dtype, cin, cout):
           assert torch.equal(got, again)
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,cout,rows,K,spread', [
+    (64, 256, 257 * 128 + 5, 9, 40),                     # tiles enough for 256 channels a workgroup
+    (96, 64, 300, 3, 2),                                 # fewer slots than waves that share them, few distinct rows
+    (64, 32, 300, 2, 0), (32, 96, 300, 1, 0), (64, 128, 300, 1, 3),
+    (32, 192, 1300, 27, 130)])                           # as many distinct rows as are staged
+def test_tile_kernel_wave_shapes(dtype, cin, cout, rows, K, spread):
+  """Every division of the waves over channels, rows and slots, against 64-bit sums over the table."""
+  print('tile kernel, waves', dtype, cin, cout, 'rows', rows, 'K', K, flush=True)
+  g = torch.Generator().manual_seed(rows + cout)
+  t = (torch.arange(rows)[:, None] + torch.randint(-spread, spread + 1, (rows, K), generator=g)).clamp_(0, rows - 1).int()
+  t[torch.rand(rows, K, generator=g) < 0.5] = -1
+  plan = TilePlan(t.cuda())
+  x = torch.randn(rows, cin, generator=g).to(dtype).cuda()
+  w = (torch.randn(K, cin, cout, generator=g) / (K * cin) ** 0.5).to(dtype).cuda()
+  b = torch.randn(cout, generator=g).to(dtype).cuda()
+  zero = torch.cat([x.double(), torch.zeros(1, cin, dtype=torch.float64, device='cuda')])
+  want = b.double() + sum(zero[t[:, k].long().cuda()] @ w[k].double() for k in range(K))
+  for parts in ((0, 0), (1, 1)):
+    for occupancy in (1.0, 0.3):
+      got = _gather(x, plan, w, cout, False, False, b, parts, occupancy).double()
+      assert (got - want).abs().max() / want.abs().max() < TOL[dtype], (parts, occupancy)
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
 def test_tile_kernel_weights_off_alignment(dtype):
   """Weights that start one element past a 16-byte boundary give the bits of aligned ones."""
