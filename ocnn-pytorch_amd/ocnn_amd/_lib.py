@@ -127,6 +127,8 @@ SIGNATURES = {
 # the library's entry points for this package alone (csrc/host_api.hpp)
 INTERNAL_SIGNATURES = {
     'ocnnx_gather_choose': (_i, [_i, _l, _l, _i, _i, _i, _i, _i, _i, _l, _d, _d, _i]),
+    'ocnnx_conv_gather_workspace_bytes': (_l, [_i, _l, _l, _i, _i, _i]),
+    'ocnnx_conv_gather': (_i, [_i, _p, _l, _p, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _p, _l, _p]),
     'ocnnx_gather_tile_supported': (_i, [_i, _l, _i, _i, _i, _i]),
     'ocnnx_gather_tile_workspace_bytes': (_l, [_i, _l, _i, _i, _i]),
     'ocnnx_gather_tile': (_i, [_i, _p, _l, _p, _p, _p, _i, _l, _d, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _p, _l, _i, _i, _p]),

@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "host_api.hpp"
 #include "reduce.hpp"
 #include "mma.hpp"
 
@@ -19,29 +20,31 @@ namespace ocnn {
 // weight packing: (K, cin, cout) [or (K, cout, cin)] -> A-operand fragments
 // --------------------------------------------------------------------------
 // layout: [cout_tile][unit = k * (cin / CB) + cb][s][t][lane][8]
+// A thread packs the eight values of a lane: eight loads in flight (consecutive when the weights are read transposed) and
+// one store.  A value a thread took 9.0 us for 256 x 256 x 27, this 5.8.
 template <typename T>
-__global__ void pack_weights_kernel(const T* __restrict__ w, T* __restrict__ out, int K, int cin,
-                                    int cout, int CB, int MT, int transposed, int reverse) {
-  int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int64_t total = (int64_t)K * cin * cout;
-  if (e >= total) return;
-  const int KS = CB / 32;
-  const int ncb = cin / CB;
-  int j = (int)(e & 7);
-  int lane = (int)((e >> 3) & 63);
-  int64_t r = e >> 9;
-  int t = (int)(r % MT); r /= MT;
-  int s = (int)(r % KS); r /= KS;
-  int64_t units = (int64_t)K * ncb;
-  int64_t u = r % units;
-  int ct = (int)(r / units);
-  int k = (int)(u / ncb), cb = (int)(u % ncb);
-  int g = lane >> 4, i = lane & 15;
-  int chan = cb * CB + (CB == 64 ? 16 * g + 8 * s + j : 8 * g + j);
-  int co = ct * 16 * MT + (i >> 2) * (4 * MT) + 4 * t + (i & 3);
-  int kk = reverse ? K - 1 - k : k;
-  out[e] = transposed ? w[((int64_t)kk * cout + co) * cin + chan]
-                      : w[((int64_t)kk * cin + chan) * cout + co];
+__global__ __launch_bounds__(256) void pack_weights_kernel(const T* __restrict__ w, T* __restrict__ out, int K, int cin,
+                                                           int cout, int CB, int MT, int transposed, int reverse) {
+  typedef __attribute__((ext_vector_type(8))) T t8;
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e * 8 >= (int64_t)K * cin * cout) return;
+  const uint32_t KS = (uint32_t)CB / 32, ncb = (uint32_t)cin / CB, units = K * ncb;
+  const uint32_t lane = (uint32_t)e & 63;
+  uint32_t r = (uint32_t)(e >> 6);
+  const uint32_t t = r % MT; r /= MT;
+  const uint32_t s = r % KS; r /= KS;
+  const uint32_t u = r % units, ct = r / units;
+  const uint32_t k = u / ncb, cb = u % ncb;
+  const uint32_t g = lane >> 4, i = lane & 15;
+  const uint32_t chan = cb * CB + (CB == 64 ? 16 * g + 8 * s : 8 * g);
+  const uint32_t co = ct * 16 * MT + (i >> 2) * (4 * MT) + 4 * t + (i & 3);
+  const uint32_t kk = reverse ? K - 1 - k : k;
+  const T* src = transposed ? w + ((int64_t)kk * cout + co) * cin + chan : w + ((int64_t)kk * cin + chan) * cout + co;
+  const int64_t step = transposed ? 1 : cout;
+  t8 v;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = src[j * step];
+  *(t8*)(out + e * 8) = v;
 }
 
 // --------------------------------------------------------------------------
@@ -51,11 +54,17 @@ __global__ void pack_weights_kernel(const T* __restrict__ w, T* __restrict__ out
 // Output rows are the N dimension of the MFMA, output channels the M dimension,
 // so that a lane ends up with 4*MT consecutive channels of one row.
 // O is the output (and bias) type: T, or float when the operands are bf16 pieces of fp32 data.
+//
+// A workgroup goes through its (slot, channel chunk) units one behind the other, 0.75 us each however few workgroups
+// there are (a unit is a round trip: rows and weights of the next one, a barrier).  Launches of few workgroups split the
+// units over blockIdx.z: parts with fp32 sums of their own (`partial`, [part][row][cout]), which
+// gather_parts_kernel adds in their order.  256 -> 256 bf16 on 512 rows, 27 slots: 85 us on 32 workgroups, 12 in 18 parts.
+// out_index: row i of the result goes to row out_index[i].
 template <typename T, typename O, int CB, int MT, int NT>
 __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
     const T* __restrict__ in, uint32_t in_bytes, const int32_t* __restrict__ table,
-    const T* __restrict__ wpk, const O* __restrict__ bias, O* __restrict__ out,
-    int64_t rows_out, int K, int cin, int cout, int64_t tiles, int64_t tiles_per_xcd) {
+    const T* __restrict__ wpk, const O* __restrict__ bias, O* __restrict__ out, const int64_t* __restrict__ out_index,
+    float* __restrict__ partial, int64_t rows_out, int K, int cin, int cout, int64_t tiles, int64_t tiles_per_xcd) {
   constexpr int KS = CB / 32;
   constexpr int ROWS = 4 * NT * 16;
   constexpr int UNIT = KS * MT * 512;                 // elements per weight unit
@@ -71,6 +80,7 @@ __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
   const int64_t row0 = tile * ROWS;
   const int ncb = cin / CB;
   const int units = K * ncb;
+  const int u0 = (int)((int64_t)units * blockIdx.z / gridDim.z), u1 = (int)((int64_t)units * (blockIdx.z + 1) / gridDim.z);
 
   // neighbour indices of the tile -> LDS (coalesced), -1 past the end
   {
@@ -88,7 +98,7 @@ __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
 #pragma unroll
   for (int c = 0; c < WL; ++c) {
     int ch = tid + c * 256;
-    if (ch < KS * MT * 64) wreg[c] = *(const u32x4*)(wbase + (int64_t)ch * 8);
+    if (ch < KS * MT * 64) wreg[c] = *(const u32x4*)(wbase + (int64_t)u0 * UNIT + (int64_t)ch * 8);
   }
 #pragma unroll
   for (int c = 0; c < WL; ++c) {
@@ -117,11 +127,11 @@ __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
         b[n][s] = __builtin_amdgcn_raw_buffer_load_b128(rs_in, off + 16 * s, 0, 0);
     }
   };
-  gather(0, bcur);
+  gather(u0, bcur);
 
   int cur = 0;
-  for (int u = 0; u < units; ++u) {
-    const bool more = u + 1 < units;
+  for (int u = u0; u < u1; ++u) {
+    const bool more = u + 1 < u1;
     if (more) {
       const T* wsrc = wbase + (int64_t)(u + 1) * UNIT;
 #pragma unroll
@@ -160,6 +170,17 @@ __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
 
   // epilogue: lane holds channels ct*16*MT + g*4*MT + [0, 4*MT) of row lrow + n*16
   const int co0 = ct * 16 * MT + g * 4 * MT;
+  if (partial) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int64_t row = row0 + lrow + n * 16;
+      if (row >= rows_out) continue;
+      float* dst = partial + ((int64_t)blockIdx.z * rows_out + row) * cout + co0;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) *(f32x4*)(dst + 4 * t) = acc[t][n];
+    }
+    return;
+  }
   float bv[4 * MT];
 #pragma unroll
   for (int c = 0; c < 4 * MT; ++c) bv[c] = bias ? to_f32(bias[co0 + c]) : 0.f;
@@ -167,7 +188,7 @@ __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
   for (int n = 0; n < NT; ++n) {
     int64_t row = row0 + lrow + n * 16;
     if (row >= rows_out) continue;
-    O* dst = out + row * cout + co0;
+    O* dst = out + (out_index ? out_index[row] : row) * cout + co0;
     if constexpr (std::is_same<O, float>::value) {
 #pragma unroll
       for (int t = 0; t < MT; ++t)
@@ -189,6 +210,32 @@ __global__ __launch_bounds__(256) void conv_gather_mfma_kernel(
       }
     }
   }
+}
+
+// out = sum of the parts in their order (+ bias); four consecutive channels a thread
+template <typename O>
+__global__ __launch_bounds__(256) void gather_parts_kernel(const float* __restrict__ partial, int parts, int64_t rows, int cout,
+                                                           const O* __restrict__ bias, const int64_t* __restrict__ out_index,
+                                                           O* __restrict__ out) {
+  const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4, n = rows * cout;
+  if (e >= n) return;
+  f32x4 acc = *(const f32x4*)(partial + e);
+  int s = 1;
+  for (; s + 4 <= parts; s += 4) {                           // four loads in flight
+    f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = *(const f32x4*)(partial + (s + u) * n + e);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc += v[u];
+  }
+  for (; s < parts; ++s) acc += *(const f32x4*)(partial + s * n + e);
+  const int64_t row = e / cout;
+  const int c = (int)(e % cout);
+  typedef __attribute__((ext_vector_type(4))) O o4;
+  o4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = from_f32<O>(acc[i] + (bias ? to_f32(bias[c + i]) : 0.f));
+  *(o4*)(out + (out_index ? out_index[row] : row) * cout + c) = o;
 }
 
 // fp32 data as three bf16 pieces: x = hi + lo (+ 2^-17 |x|), and
@@ -244,8 +291,8 @@ __global__ void split3_weights_kernel(const float* __restrict__ w, int K, int ci
 template <typename T>
 __global__ __launch_bounds__(256) void conv_gather_plain_kernel(
     const T* __restrict__ in, int64_t rows_in, const int32_t* __restrict__ table,
-    const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ out, int64_t rows_out,
-    int K, int cin, int cout, int transposed, int reverse) {
+    const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ out, const int64_t* __restrict__ out_index,
+    int64_t rows_out, int K, int cin, int cout, int transposed, int reverse) {
   constexpr int RB = 16, CCH = 128;       // rows per block, input-channel chunk
   __shared__ float s_x[RB][CCH];
   __shared__ int32_t s_i[RB];
@@ -293,7 +340,7 @@ __global__ __launch_bounds__(256) void conv_gather_plain_kernel(
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
         int co = co_blk + cg + 16 * m;
-        if (co < cout) out[row * cout + co] = from_f32<T>(acc[m] + (bias ? to_f32(bias[co]) : 0.f));
+        if (co < cout) out[(out_index ? out_index[row] : row) * cout + co] = from_f32<T>(acc[m] + (bias ? to_f32(bias[co]) : 0.f));
       }
     }
   }
@@ -474,31 +521,55 @@ static GatherPlan plan_gather(int dtype, int64_t rows_in, int64_t rows_out, int 
   return p;
 }
 
+// Parts of the reduction: up to kGatherGroups workgroups (four a CU), of kGatherUnits units each at least.  us in one
+// part -> in parts, weights' packing and sums included: bf16 256 -> 256 on 8 / 27 slots of 512 rows 30 -> 16, 95 -> 27, of
+// 3000 rows 31 -> 27, 95 -> 46; fp32 128 -> 128 on 27 slots of 512 / 9000 rows 142 -> 32, 149 -> 92; bf16 64 -> 64 on 27
+// slots of 9000 rows 26 -> 22, but of 30000 rows (469 workgroups of 27 units) 29 -> 32, so not there.
+constexpr int kGatherGroups = 1024, kGatherUnits = 6;
+
+static int gather_parts(const GatherPlan& p, int64_t rows_out, int K, int cin, int cout) {
+  if (!p.mfma || rows_out == 0) return 1;
+  const int64_t groups = cdiv(rows_out, 64 * p.NT) * (cout / (16 * p.MT)), units = (int64_t)K * (cin / p.CB);
+  if (groups > kGatherGroups / 4 && units < 9 * kGatherUnits) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kGatherGroups / groups, units / kGatherUnits));
+}
+
+static int64_t gather_parts_bytes(int parts, int64_t rows_out, int cout) {
+  return parts > 1 ? align_up(parts * rows_out * cout * 4, 256) : 0;
+}
+
 template <typename T, typename O, int CB, int MT, int NT>
 static void launch_gather(const GatherPlan&, const void* in, int64_t rows_in, const int32_t* table,
                           int64_t rows_out, int K, int cin, int cout, const void* wpk,
-                          const void* bias, void* out, hipStream_t st) {
+                          const void* bias, void* out, const int64_t* out_index, float* partial, int parts, hipStream_t st) {
   constexpr int ROWS = 64 * NT;
   int64_t tiles = cdiv(rows_out, ROWS);
   int64_t per_xcd = cdiv(tiles, 8);
-  dim3 grid((unsigned)(per_xcd * 8), (unsigned)(cout / (16 * MT)));
+  dim3 grid((unsigned)(per_xcd * 8), (unsigned)(cout / (16 * MT)), (unsigned)parts);
   hipLaunchKernelGGL((conv_gather_mfma_kernel<T, O, CB, MT, NT>), grid, dim3(256), 0, st,
                      (const T*)in, (uint32_t)(rows_in * cin * sizeof(T)), table, (const T*)wpk,
-                     (const O*)bias, (O*)out, rows_out, K, cin, cout, tiles, per_xcd);
+                     (const O*)bias, (O*)out, out_index, partial, rows_out, K, cin, cout, tiles, per_xcd);
+  if (partial)
+    hipLaunchKernelGGL(gather_parts_kernel<O>, dim3((unsigned)cdiv(rows_out * cout / 4, 256)), dim3(256), 0, st, partial,
+                       parts, rows_out, cout, (const O*)bias, out_index, (O*)out);
 }
 
+// room: bytes at `sums` for the parts' sums; without enough of it the launch is one part
 template <typename T, typename O = T>
 static int run_gather_mfma(const GatherPlan& p, const void* in, int64_t rows_in,
                            const int32_t* table, int64_t rows_out, int K, const void* w, int cin,
                            int cout, int w_transposed, int reverse, const void* bias, void* out,
-                           void* ws, hipStream_t st) {
+                           const int64_t* out_index, void* ws, char* sums, int64_t room, hipStream_t st) {
+  int parts = gather_parts(p, rows_out, K, cin, cout);
+  if (gather_parts_bytes(parts, rows_out, cout) > room) parts = 1;
+  float* partial = parts > 1 ? (float*)sums : nullptr;
   int64_t total = (int64_t)K * cin * cout;
-  hipLaunchKernelGGL(pack_weights_kernel<T>, dim3(cdiv(total, 256)), dim3(256), 0, st,
+  hipLaunchKernelGGL(pack_weights_kernel<T>, dim3((unsigned)cdiv(total / 8, 256)), dim3(256), 0, st,
                      (const T*)w, (T*)ws, K, cin, cout, p.CB, p.MT, w_transposed, reverse);
 #define OCNN_GATHER_CASE(cb_, mt_, nt_)                                                        \
   if (p.CB == cb_ && p.MT == mt_ && p.NT == nt_) {                                             \
     launch_gather<T, O, cb_, mt_, nt_>(p, in, rows_in, table, rows_out, K, cin, cout, ws, bias,   \
-                                    out, st);                                                  \
+                                    out, out_index, partial, parts, st);                                                  \
     return check_launch("conv_gather_mfma");                                                   \
   }
   OCNN_GATHER_CASE(64, 4, 4) OCNN_GATHER_CASE(64, 4, 2) OCNN_GATHER_CASE(64, 4, 1)
@@ -516,9 +587,9 @@ template <typename T>
 static int run_gather_plain(const void* in, int64_t rows_in, const int32_t* table,
                             int64_t rows_out, int K, const void* w, int cin, int cout,
                             int w_transposed, int reverse, const void* bias, void* out,
-                            hipStream_t st) {
+                            const int64_t* out_index, hipStream_t st) {
   hipLaunchKernelGGL(conv_gather_plain_kernel<T>, dim3((unsigned)cdiv(rows_out, 16)), dim3(256), 0,
-                     st, (const T*)in, rows_in, table, (const T*)w, (const T*)bias, (T*)out,
+                     st, (const T*)in, rows_in, table, (const T*)w, (const T*)bias, (T*)out, out_index,
                      rows_out, K, cin, cout, w_transposed, reverse);
   return check_launch("conv_gather_plain");
 }
@@ -575,10 +646,23 @@ extern "C" int64_t ocnn_conv_gather_workspace_bytes(int dtype, int64_t rows_in, 
   return base;
 }
 
-extern "C" int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in, const int32_t* table,
-                                int64_t rows_out, int K, const void* w, int cin, int cout,
-                                int w_transposed, int reverse_slots, const void* bias, void* out,
-                                void* workspace, int64_t workspace_bytes, void* stream) {
+// packed weights and pieces, rounded up to where the parts' sums begin
+static int64_t gather_base_bytes(int dtype, int64_t rows_in, int K, int cin, int cout) {
+  return align_up(ocnn_conv_gather_workspace_bytes(dtype, rows_in, K, cin, cout), 256);
+}
+
+extern "C" int64_t ocnnx_conv_gather_workspace_bytes(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout) {
+  const bool f32 = dtype == OCNN_F32;
+  if (f32 && f32_gather_workspace(rows_in, K, cin, cout) == 0) return gather_base_bytes(dtype, rows_in, K, cin, cout);
+  const int c = f32 ? 3 * cin : cin;
+  const GatherPlan p = plan_gather(f32 ? OCNN_BF16 : dtype, rows_in, rows_out, c, cout);
+  return gather_base_bytes(dtype, rows_in, K, cin, cout) + gather_parts_bytes(gather_parts(p, rows_out, K, c, cout), rows_out, cout);
+}
+
+extern "C" int ocnnx_conv_gather(int dtype, const void* in, int64_t rows_in, const int32_t* table,
+                                 int64_t rows_out, int K, const void* w, int cin, int cout,
+                                 int w_transposed, int reverse_slots, const void* bias, void* out, const int64_t* out_index,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
   OCNN_REQUIRE(dtype >= 0 && dtype <= 2, "conv_gather: dtype %d", dtype);
   OCNN_REQUIRE(K >= 1 && K <= 27 && cin >= 1 && cout >= 1, "conv_gather: K=%d cin=%d cout=%d", K,
                cin, cout);
@@ -589,6 +673,8 @@ extern "C" int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in, cons
   OCNN_REQUIRE(rows_in == 0 || in, "conv_gather: in is NULL");
   hipStream_t st = (hipStream_t)stream;
   GatherPlan p = plan_gather(dtype, rows_in, rows_out, cin, cout);
+  const int64_t base = gather_base_bytes(dtype, rows_in, K, cin, cout), room = std::max<int64_t>(0, workspace_bytes - base);
+  char* sums = (char*)workspace + base;
   if (p.mfma) {
     if (workspace_bytes < (int64_t)K * cin * cout * 2) {
       set_error("conv_gather: workspace %lld too small", (long long)workspace_bytes);
@@ -596,9 +682,9 @@ extern "C" int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in, cons
     }
     if (dtype == OCNN_F16)
       return run_gather_mfma<f16>(p, in, rows_in, table, rows_out, K, w, cin, cout, w_transposed,
-                                  reverse_slots, bias, out, workspace, st);
+                                  reverse_slots, bias, out, out_index, workspace, sums, room, st);
     return run_gather_mfma<bf16>(p, in, rows_in, table, rows_out, K, w, cin, cout, w_transposed,
-                                 reverse_slots, bias, out, workspace, st);
+                                 reverse_slots, bias, out, out_index, workspace, sums, room, st);
   }
   if (dtype == OCNN_F32) {
     // bf16 pieces on the MFMA kernel when the shape allows and the caller brought the room
@@ -615,16 +701,24 @@ extern "C" int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in, cons
       hipLaunchKernelGGL(split3_weights_kernel, dim3((unsigned)cdiv((int64_t)K * cin * cout, 256)),
                          dim3(256), 0, st, (const float*)w, K, cin, cout, w_transposed, wsp);
       return run_gather_mfma<bf16, float>(p3, xs, rows_in, table, rows_out, K, wsp, 3 * cin, cout,
-                                          w_transposed, reverse_slots, bias, out, wpk, st);
+                                          w_transposed, reverse_slots, bias, out, out_index, wpk, sums, room, st);
     }
     return run_gather_plain<float>(in, rows_in, table, rows_out, K, w, cin, cout, w_transposed,
-                                   reverse_slots, bias, out, st);
+                                   reverse_slots, bias, out, out_index, st);
   }
   if (dtype == OCNN_F16)
     return run_gather_plain<f16>(in, rows_in, table, rows_out, K, w, cin, cout, w_transposed,
-                                 reverse_slots, bias, out, st);
+                                 reverse_slots, bias, out, out_index, st);
   return run_gather_plain<bf16>(in, rows_in, table, rows_out, K, w, cin, cout, w_transposed,
-                                reverse_slots, bias, out, st);
+                                reverse_slots, bias, out, out_index, st);
+}
+
+extern "C" int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in, const int32_t* table,
+                                int64_t rows_out, int K, const void* w, int cin, int cout,
+                                int w_transposed, int reverse_slots, const void* bias, void* out,
+                                void* workspace, int64_t workspace_bytes, void* stream) {
+  return ocnnx_conv_gather(dtype, in, rows_in, table, rows_out, K, w, cin, cout, w_transposed, reverse_slots, bias, out,
+                           nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int64_t ocnn_conv_wgrad_workspace_bytes(int64_t rows, int K, int ca, int cb) {

@@ -146,17 +146,32 @@ struct GatherOp {
         require_gpu(table);
         TORCH_CHECK(table.scalar_type() == at::kInt && table.is_contiguous() && table.numel() == rows * K,
                     "conv_gather: the table does not match");
-        check(ocnn_conv_gather(code, ptr(data), rows_in, typed<int32_t>(table), rows, K, ptr(W), cin, cout, transposed,
-                               reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        check(ocnnx_conv_gather(code, ptr(data), rows_in, typed<int32_t>(table), rows, K, ptr(W), cin, cout, transposed,
+                                reverse, ptr(bias), out.data_ptr(), nullptr, ws.data_ptr(), ws.numel(), st));
     }
     if (overflow) {
       at::tracer::impl::NoTracerDispatchMode quiet;          // (a trace must not own the plan's tensors)
-      out.index_copy_(0, overflow_rows, overflow->run(data, overflow_table, W, bias));
+      overflow->run_into(out, overflow_rows, data, overflow_table, W, bias);
     }
     return followed(view_cols ? out.view({-1, view_cols}) : out, bn);
   }
 
  private:
+  // this pass with row i of its result written to row index[i] of `out`
+  void run_into(Tensor& out, const Tensor& index, const Tensor& data, const Tensor& table, const Tensor& W,
+                const OptTensor& bias) const {
+    if (kernel != OCNN_GATHER_PLAIN || padded) {
+      out.index_copy_(0, index, run(data, table, W, bias));
+      return;
+    }
+    TORCH_CHECK(index.scalar_type() == at::kLong && index.is_contiguous() && index.numel() == rows &&
+                    table.scalar_type() == at::kInt && table.is_contiguous() && table.numel() == rows * K,
+                "conv_gather: the rows that run apart do not match");
+    Tensor ws = workspace(ws_bytes, data);
+    check(ocnnx_conv_gather(code_of(data.scalar_type()), ptr(data), rows_in, typed<int32_t>(table), rows, K, ptr(W), cin,
+                            cout, transposed, reverse, ptr(bias), out.data_ptr(), typed<int64_t>(index), ws.data_ptr(),
+                            ws.numel(), hip_stream()));
+  }
   static Tensor followed(const Tensor& out, const ocnnx_bn* bn) {
     if (bn && out.size(0))
       check(ocnnx_batch_norm_running(code_of(out.scalar_type()), out.data_ptr(), out.size(0), (int)out.size(1), bn->mean,

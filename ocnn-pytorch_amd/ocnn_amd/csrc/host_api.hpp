@@ -34,6 +34,13 @@ int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t
                       const void* bias, const ocnnx_bn* bn, void* out, void* workspace, int64_t workspace_bytes,
                       int split_c, int split_k, void* stream);
 
+// ocnn_conv_gather with row i of the result at row out_index[i] (null: i), and with the room that lets a launch of few
+// rows split its reduction (with less, but ocnn_conv_gather_workspace_bytes, it runs in one part).
+int64_t ocnnx_conv_gather_workspace_bytes(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout);
+int ocnnx_conv_gather(int dtype, const void* in, int64_t rows_in, const int32_t* table, int64_t rows_out, int K,
+                      const void* w, int cin, int cout, int w_transposed, int reverse_slots, const void* bias, void* out,
+                      const int64_t* out_index, void* workspace, int64_t workspace_bytes, void* stream);
+
 // ocnn_conv_gather_choose with that kernel among the choices.
 #define OCNNX_GATHER_TILE 8
 int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout, int identity_table,

@@ -122,6 +122,8 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
     sparse = op.kernel == _lib.GATHER_SPARSE
     op.ws_bytes = (L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout) if sparse else
                    L.ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout) if op.kernel == _lib.GATHER_TILE else
+                   L.ocnnx_conv_gather_workspace_bytes(code, rows_in, rows, K, cin, cout)
+                   if op.kernel == _lib.GATHER_PLAIN else
                    L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
     if op.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE, _lib.GATHER_SPARSE, _lib.GATHER_PLANNED):
       op.plan = _plan_arrays(plan, sparse)

@@ -1963,3 +1963,31 @@ def test_pad_empty_rows_only(dtype, channels):
       out = out.cuda()
       _lib.check(L.ocnn_pad(code, None, P(children), n, channels, 1.5, P(out[1:]), _lib.stream()))
       assert torch.equal(out.cpu(), want), (n, share)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('rows,K,cin,cout', [(1, 27, 64, 64), (63, 8, 256, 48), (65, 27, 96, 96), (600, 27, 256, 256),
+                                             (600, 27, 20, 24), (9001, 8, 128, 64)])
+def test_plan_free_gather_in_parts_and_through_an_index(dtype, rows, K, cin, cout):
+  """The plan-free gather with and without the room to split its reduction, rows written through an index."""
+  L, P = _lib.lib(), _lib.ptr
+  print('plan-free gather', dtype, rows, K, cin, cout, flush=True)
+  g = torch.Generator().manual_seed(rows + cin)
+  t = torch.randint(-1, 2 * rows, (rows, K), generator=g).int().cuda()
+  x = torch.randn(2 * rows, cin, generator=g).to(dtype).cuda()
+  w = (torch.randn(K, cin, cout, generator=g) / (K * cin) ** 0.5).to(dtype).cuda()
+  b = torch.randn(cout, generator=g).to(dtype).cuda()
+  zero = torch.cat([x.double(), torch.zeros(1, cin, dtype=torch.float64, device='cuda')])
+  want = b.double() + sum(zero[t[:, k].long()] @ w[k].double() for k in range(K))
+  index = torch.randperm(3 * rows, generator=g)[:rows].cuda()
+  code = _lib.dtype_code(x)
+  for size in (L.ocnn_conv_gather_workspace_bytes(code, 2 * rows, K, cin, cout),
+               L.ocnnx_conv_gather_workspace_bytes(code, 2 * rows, rows, K, cin, cout)):
+    ws = torch.empty(size, dtype=torch.uint8, device='cuda')
+    for idx in (None, index):
+      out = torch.full((3 * rows if idx is not None else rows, cout), float('nan'), dtype=dtype, device='cuda')
+      _lib.check(L.ocnnx_conv_gather(code, P(x), 2 * rows, P(t), rows, K, P(w), cin, cout, 0, 0, P(b), P(out), P(idx),
+                                     P(ws), size, _lib.stream()))
+      got = (out if idx is None else out[idx]).double()
+      assert (got - want).abs().max() / want.abs().max() < {torch.float32: 2e-5, torch.float16: 2e-3, torch.bfloat16: 1e-2}[dtype]
+      assert int(out.isnan().sum()) == (0 if idx is None else 2 * rows * cout)
