@@ -25,6 +25,7 @@ SOURCES = {
     'conv_staged.hip': [],
     'conv_rw.hip': [],
     'conv_tile.hip': [],
+    'jobs.hip': [],
     'conv_dense.hip': [],
     'conv_sparse.hip': [],
     'wgrad_sparse.hip': [],

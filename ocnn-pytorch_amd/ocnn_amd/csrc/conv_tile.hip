@@ -23,11 +23,10 @@
 // reduction, over chunks of input channels and over the slots; each part writes fp32 sums of its own, and a
 // second kernel adds them in the order of the parts.
 #include <algorithm>
+#include <new>
 #include <type_traits>
 
-#include "common.hpp"
-#include "host_api.hpp"
-#include "mma.hpp"
+#include "jobs.hpp"
 
 namespace ocnn {
 
@@ -44,140 +43,6 @@ constexpr double kTgSkipMaxOccupancy = 0.45;
 // type-dependent expressions.)
 static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char* dst, uint32_t off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, off, 0, 0, 0);
-}
-
-// Packed weights: [input-channel chunk cc][slot k][32 output channels cg][step s][lane][8].
-// v_mfma_f32_32x32x16 A operand: lane l holds A[l % 32][8 * (l / 32) + j];
-// D: lane l, register r holds D[8 * (r / 4) + 4 * (l / 32) + r % 4][l % 32].
-//   output channel = 32 cg + perm(lane % 32), perm(8a + 4q + b) = 16 q + 4 a + b,
-// so that a lane ends with 16 consecutive output channels per M tile.
-//   16-bit: input channel = 64 cc + 16 s + 8 (lane / 32) + j
-//   fp32:   input channel = 32 cc + 16 (s / 2) + 8 (lane / 32) + j, s % 2 = 0: high piece, 1: low
-// Input channels are padded to whole chunks with zero weights.
-//
-// Bound by latency (a layer's weights are 0.1 - 7 MB): few, wide loads a thread, all in flight together.
-// transposed: a thread packs a lane's eight values, consecutive in memory.  Otherwise they are rows of
-// cout values apart and a thread packs four lanes of consecutive output channels: eight loads of four
-// values, 64 consecutive bytes written.  AL: the weights are 16-byte aligned (a module's are; a view
-// into something else may not be, and is read value by value).  fp32 256 -> 256, 27 slots: 8.9 -> 6 us (eight
-// 4-byte loads a thread before); the 103 launches of an fp32 U-Net step 0.68 -> 0.52 ms.
-template <int N, bool AL, typename I>
-__device__ __forceinline__ void load_run(const I* __restrict__ p, I (&v)[N]) {
-  if constexpr (AL) {
-    constexpr int W = N * sizeof(I) < 16 ? N : 16 / sizeof(I);
-    typedef __attribute__((ext_vector_type(W))) I vec;
-#pragma unroll
-    for (int i = 0; i < N; i += W) {
-      const vec x = *(const vec*)(p + i);
-#pragma unroll
-      for (int j = 0; j < W; ++j) v[i + j] = x[j];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = p[i];
-  }
-}
-
-template <typename I, typename T, bool AL>
-__global__ __launch_bounds__(256) void pack_weights_tile_kernel(const I* __restrict__ w, T* __restrict__ out, int K,
-                                                                int cin, int cout, int transposed, int reverse) {
-  constexpr bool F32 = std::is_same<I, float>::value;
-  constexpr int CH = F32 ? 32 : 64, STEPS = F32 ? 2 : 4;
-  typedef __attribute__((ext_vector_type(8))) T t8;
-  const uint32_t e = blockIdx.x * 256 + threadIdx.x;
-  const uint32_t t = transposed ? e & 63 : e & 15, step = transposed ? e >> 6 : e >> 4;
-  const uint32_t ncc = (uint32_t)(cin + CH - 1) / CH, ncg = (uint32_t)cout >> 5;
-  const uint32_t s = step % STEPS, base = step / STEPS;      // base = (cc K + k) ncg + cg
-  if (base >= ncc * K * ncg) return;
-  const uint32_t cg = base % ncg, k = base / ncg % K, cc = base / ncg / K;
-  const uint32_t kk = reverse ? K - 1 - k : k;
-  T* dst = out + (int64_t)base * 2048;
-  // the eight values of a lane -> its place (both pieces of them)
-  auto put = [&](const I (&v)[8], uint32_t lane) {
-    t8 hi;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) hi[j] = (T)v[j];
-    if constexpr (F32) {
-      t8 lo;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) lo[j] = (T)(v[j] - (float)hi[j]);
-      *(t8*)(dst + (2 * s) * 512 + lane * 8) = hi;
-      *(t8*)(dst + (2 * s + 1) * 512 + lane * 8) = lo;
-    } else {
-      *(t8*)(dst + s * 512 + lane * 8) = hi;
-    }
-  };
-  if (transposed) {
-    const uint32_t m = t & 31, chan = CH * cc + 16 * s + 8 * (t >> 5);
-    const uint32_t co = 32 * cg + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
-    I v[8] = {};
-    if (chan < (uint32_t)cin) load_run<8, AL>(w + ((int64_t)kk * cout + co) * cin + chan, v);
-    put(v, t);
-  } else {
-    const uint32_t m4 = t & 7, chan = CH * cc + 16 * s + 8 * (t >> 3);
-    const uint32_t co = 32 * cg + 16 * (m4 & 1) + 4 * (m4 >> 1);
-    I v[8][4] = {};
-    if (chan < (uint32_t)cin) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) load_run<4, AL>(w + ((int64_t)kk * cin + chan + j) * cout + co, v[j]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      I r[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = v[j][i];
-      put(r, 32 * (t >> 3) + 4 * m4 + i);
-    }
-  }
-}
-
-// N consecutive values of a per-channel array (f32 / f16 / bf16; null: dflt), N a multiple of 4
-template <int N>
-__device__ __forceinline__ void load_channels(const void* p, int dtype, int c0, float dflt, float (&v)[N]) {
-  if (!p) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = dflt;
-  } else if (dtype == OCNN_F32) {
-#pragma unroll
-    for (int i = 0; i < N; i += 4) {
-      const f32x4 q = *(const f32x4*)((const float*)p + c0 + i);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[i + j] = q[j];
-    }
-  } else {
-    unsigned short r[N];
-#pragma unroll
-    for (int i = 0; i < N; i += 4) {
-      const u32x2 q = *(const u32x2*)((const unsigned short*)p + c0 + i);
-      r[i] = (unsigned short)q[0], r[i + 1] = (unsigned short)(q[0] >> 16);
-      r[i + 2] = (unsigned short)q[1], r[i + 3] = (unsigned short)(q[1] >> 16);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-      v[i] = dtype == OCNN_F16 ? to_f32(__builtin_bit_cast(f16, r[i])) : __uint_as_float((uint32_t)r[i] << 16);
-  }
-}
-
-// What is added to N channels of a row's sums and what they are multiplied with: bias alone, or the batch
-// norm behind the layer with its running statistics, ((sum + bias) - mean) * sc + beta = sum * sc + sh.
-template <typename O, int N>
-__device__ __forceinline__ void layer_tail(const O* bias, const ocnnx_bn& bn, int c0, float (&sc)[N], float (&sh)[N]) {
-  load_channels<N>(bias, std::is_same<O, float>::value ? OCNN_F32 : (std::is_same<O, f16>::value ? OCNN_F16 : OCNN_BF16), c0,
-                   0.f, sh);
-#pragma unroll
-  for (int i = 0; i < N; ++i) sc[i] = 1.f;
-  if (bn.mean) {
-    float m[N], be[N], ga[N];
-    load_channels<N>(bn.var, bn.stat_dtype, c0, 1.f, sc);
-    load_channels<N>(bn.mean, bn.stat_dtype, c0, 0.f, m);
-    load_channels<N>(bn.gamma, bn.param_dtype, c0, 1.f, ga);
-    load_channels<N>(bn.beta, bn.param_dtype, c0, 0.f, be);
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      sc[i] = ga[i] / sqrtf(sc[i] + bn.eps);
-      sh[i] = (sh[i] - m[i]) * sc[i] + be[i];
-    }
-  }
 }
 
 // SKIP: per slot and 32-row block of the tile a wave asks whether any row has an entry there (a
@@ -492,42 +357,6 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   }
 }
 
-// out = sum of the parts, in their order, and what follows (layer_tail); four consecutive channels a thread, eight
-// threads a row's 32 channels, so that a wave reads 128 bytes of consecutive rows at a time and writes 64 - 128.
-template <typename O>
-__global__ __launch_bounds__(256) void tile_parts_kernel(const float* __restrict__ partial, int parts, int64_t rows, int cout,
-                                                         const O* __restrict__ bias, ocnnx_bn bn, O* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t row = t >> 3;
-  const int c4 = (int)blockIdx.y * 8 + (int)(t & 7);         // four channels
-  if (row >= rows) return;
-  const int64_t n = rows * cout, e = row * cout + 4 * c4;
-  const float* src = partial + ((int64_t)c4 * rows + row) * 4;
-  f32x4 acc = *(const f32x4*)src;
-  int s = 1;
-  for (; s + 4 <= parts; s += 4) {                           // four loads in flight
-    f32x4 v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = *(const f32x4*)(src + (s + u) * n);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) acc += v[u];
-  }
-  for (; s < parts; ++s) acc += *(const f32x4*)(src + s * n);
-  float mul[4], add[4];
-  layer_tail<O, 4>(bias, bn, 4 * c4, mul, add);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    acc[i] = acc[i] * mul[i] + add[i];
-    if (bn.residual) acc[i] += to_f32(((const O*)bn.residual)[e + i]);
-    if (bn.relu) acc[i] = fmaxf(acc[i], 0.f);
-  }
-  typedef __attribute__((ext_vector_type(4))) O o4;
-  o4 o;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = from_f32<O>(acc[i]);
-  *(o4*)(out + e) = o;
-}
-
 struct TileLaunch {
   int mb, wc, wr, ks;          // shape of a wave: 32 mb channels x 128 / wr rows, every ks-th slot; wc waves along the channels
   int gy;                      // blocks of output channels
@@ -601,57 +430,78 @@ extern "C" int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out
   return tile_packed_bytes(dtype, K, cin, cout) + (parts > 1 ? parts * rows_out * cout * 4 : 0);
 }
 
-template <typename T, bool F32>
-static int run_tile(const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr, const int32_t* urows, int umax,
-                    int64_t rows_out, int K, int cin, int cout, const void* w, int w_transposed, int reverse,
-                    const void* bias, const ocnnx_bn& bn, void* out, void* ws, int64_t ws_bytes, bool skip, int split_c,
-                    int split_k, hipStream_t st) {
-  typedef typename std::conditional<F32, float, T>::type O;
-  const int dtype = F32 ? OCNN_F32 : OCNN_F16;
-  const int64_t steps = cdiv(cin, F32 ? 32 : 64) * (int64_t)K * (cout / 32) * (F32 ? 2 : 4);
-  const dim3 pack_grid((unsigned)cdiv(steps * (w_transposed ? 64 : 16), 256));
-  if ((uintptr_t)w % 16 == 0)
-    hipLaunchKernelGGL((pack_weights_tile_kernel<O, T, true>), pack_grid, dim3(256), 0, st, (const O*)w, (T*)ws, K, cin,
-                       cout, w_transposed, reverse);
-  else
-    hipLaunchKernelGGL((pack_weights_tile_kernel<O, T, false>), pack_grid, dim3(256), 0, st, (const O*)w, (T*)ws, K, cin,
-                       cout, w_transposed, reverse);
-  const int64_t tiles = cdiv(rows_out, kTgRows);
-  TileLaunch t = tile_launch(F32, tiles, K, cin, cout);
-  if (split_c > 0 && split_k > 0) {
-    t.sc = std::min<int>(split_c, (int)cdiv(cin, F32 ? 32 : 64));
-    t.sk = std::min(split_k, K);
+template <typename T, bool F32> struct TilePass : Pass {
+  ocnnx_gather_args a;
+  ocnnx_bn bn;
+  TileLaunch t;
+  bool skip;
+  float* partial;
+  hipStream_t st;
+
+  TilePass(const ocnnx_gather_args& args, hipStream_t stream) : a(args), bn(args.bn ? *args.bn : ocnnx_bn{}), st(stream) {
+    const int dtype = std::is_same<T, f16>::value ? OCNN_F16 : (F32 ? OCNN_F32 : OCNN_BF16);
+    // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
+    skip = a.K != 8 && a.plan_occupancy >= 0.0 && a.plan_occupancy <= kTgSkipMaxOccupancy;
+    t = tile_launch(F32, cdiv(a.rows_out, kTgRows), a.K, a.cin, a.cout);
+    if (a.split_c > 0 && a.split_k > 0) {
+      t.sc = std::min<int>(a.split_c, (int)cdiv(a.cin, F32 ? 32 : 64));
+      t.sk = std::min(a.split_k, a.K);
+    }
+    const int64_t packed = tile_packed_bytes(dtype, a.K, a.cin, a.cout);
+    if (packed + (int64_t)t.sc * t.sk * a.rows_out * a.cout * 4 > a.workspace_bytes) t.sc = t.sk = 1;   // (no room for the parts)
+    partial = t.sc * t.sk > 1 ? (float*)((char*)a.workspace + packed) : nullptr;
+    before.add(pack_tile_job(dtype, a.w, a.workspace, a.K, a.cin, a.cout, a.w_transposed, a.reverse_slots));
+    if (partial) after.add(tile_parts_job(partial, t.sc * t.sk, a.rows_out, a.cout, a.bias, bn, a.out));
   }
-  const int64_t packed = tile_packed_bytes(dtype, K, cin, cout);
-  if (packed + (int64_t)t.sc * t.sk * rows_out * cout * 4 > ws_bytes) t.sc = t.sk = 1;   // (no room for the parts)
-  const int parts = t.sc * t.sk;
-  float* partial = parts > 1 ? (float*)((char*)ws + packed) : nullptr;
-  // few tiles: in launch order, so that they spread over the XCDs
-  const int64_t per_xcd = parts > 1 ? 0 : cdiv(tiles, 8);
-  const dim3 grid((unsigned)(per_xcd > 0 ? per_xcd * 8 : tiles), (unsigned)t.gy, (unsigned)parts);
-  const uint32_t in_bytes = (uint32_t)(rows_in * cin * sizeof(O));
-  const int rows_alloc = std::max((umax + 8) / 8 * 8, 1);
-  // LDS: rows, positions, list; at the end the waves' sums
-  const int kmax = (K + t.sk - 1) / t.sk;
-  const size_t lds = std::max<size_t>((size_t)rows_alloc * 132 + (size_t)kmax * kTgRows * 2,
-                                      (size_t)(t.ks - 1) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
-#define OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, SKIP_)                                                                 \
-  hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WC_, WR_, KS_, SKIP_>), grid, dim3(256), lds, st, in,    \
-                     in_bytes, loc, uptr, urows, (const T*)ws, bias, bn, out, partial, rows_out, K, cin, cout, tiles, \
-                     per_xcd, t.sc, t.sk, rows_alloc)
+
+  int main() override {
+    typedef typename std::conditional<F32, float, T>::type O;
+    const int64_t tiles = cdiv(a.rows_out, kTgRows);
+    // few tiles: in launch order, so that they spread over the XCDs
+    const int64_t per_xcd = partial ? 0 : cdiv(tiles, 8);
+    const dim3 grid((unsigned)(per_xcd > 0 ? per_xcd * 8 : tiles), (unsigned)t.gy, (unsigned)(t.sc * t.sk));
+    const uint32_t in_bytes = (uint32_t)(a.rows_in * a.cin * sizeof(O));
+    const int rows_alloc = (a.plan_max_distinct + 8) / 8 * 8;
+    // LDS: rows, positions, list; at the end the waves' sums
+    const int kmax = (a.K + t.sk - 1) / t.sk;
+    const size_t lds = std::max<size_t>((size_t)rows_alloc * 132 + (size_t)kmax * kTgRows * 2,
+                                        (size_t)(t.ks - 1) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
+#define OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, SKIP_)                                                                      \
+  hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WC_, WR_, KS_, SKIP_>), grid, dim3(256), lds, st, a.in,       \
+                     in_bytes, a.loc, a.uptr, a.urows, (const T*)a.workspace, a.bias, bn, a.out, partial, a.rows_out, a.K, \
+                     a.cin, a.cout, tiles, per_xcd, t.sc, t.sk, rows_alloc)
 #define OCNN_TILE_CASE(MB_, WC_, WR_, KS_)                                   \
   if (t.mb == MB_ && t.wc == WC_ && t.wr == WR_ && t.ks == KS_) {            \
     if (skip) OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, true);                    \
     else OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, false);                        \
   }
-  OCNN_TILE_CASE(1, 1, 1, 4) OCNN_TILE_CASE(2, 1, 1, 4) OCNN_TILE_CASE(3, 1, 2, 2) OCNN_TILE_CASE(2, 2, 1, 2)
-  OCNN_TILE_CASE(2, 4, 1, 1)
+    OCNN_TILE_CASE(1, 1, 1, 4) OCNN_TILE_CASE(2, 1, 1, 4) OCNN_TILE_CASE(3, 1, 2, 2) OCNN_TILE_CASE(2, 2, 1, 2)
+    OCNN_TILE_CASE(2, 4, 1, 1)
 #undef OCNN_TILE_CASE
 #undef OCNN_TILE_LAUNCH
-  if (partial)
-    hipLaunchKernelGGL(tile_parts_kernel<O>, dim3((unsigned)cdiv(rows_out * 8, 256), (unsigned)(cout / 32)), dim3(256), 0, st,
-                       partial, parts, rows_out, cout, (const O*)bias, bn, (O*)out);
-  return check_launch("conv_gather_tile");
+    return check_launch("conv_gather_tile");
+  }
+};
+
+// The pass for these arguments, to be deleted by the caller; none for no rows.
+int ocnn::tile_pass(int dtype, const ocnnx_gather_args& a, hipStream_t st, Pass** pass) {
+  *pass = nullptr;
+  OCNN_REQUIRE(ocnnx_gather_tile_supported(dtype, a.rows_in, a.K, a.cin, a.cout, a.plan_max_distinct),
+               "conv_gather_tile: shape not supported");
+  OCNN_REQUIRE(a.rows_out >= 0 && a.rows_out < (1ll << 31) && a.plan_total >= 0 && a.plan_total < (1ll << 29),
+               "conv_gather_tile: rows out of range");
+  if (a.rows_out == 0) return OCNN_OK;
+  OCNN_REQUIRE_PTRS("conv_gather_tile", a.loc, a.uptr, a.urows, a.w, a.out, a.workspace);
+  OCNN_REQUIRE(a.rows_in == 0 || a.in, "conv_gather_tile: in is NULL");
+  if (a.workspace_bytes < (dtype == OCNN_F32 ? (int64_t)a.K * a.cin * a.cout * 4 : (int64_t)a.K * align_up(a.cin, 64) * a.cout * 2)) {
+    set_error("conv_gather_tile: workspace too small");
+    return OCNN_ERR_WORKSPACE;
+  }
+  if (dtype == OCNN_F32) *pass = new (std::nothrow) TilePass<bf16, true>(a, st);
+  else if (dtype == OCNN_F16) *pass = new (std::nothrow) TilePass<f16, false>(a, st);
+  else *pass = new (std::nothrow) TilePass<bf16, false>(a, st);
+  OCNN_REQUIRE(*pass, "conv_gather_tile: out of host memory");
+  return OCNN_OK;
 }
 
 extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
@@ -659,30 +509,17 @@ extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, con
                                  int64_t rows_out, int K, const void* w, int cin, int cout, int w_transposed,
                                  int reverse_slots, const void* bias, const ocnnx_bn* bn_or_null, void* out,
                                  void* workspace, int64_t workspace_bytes, int split_c, int split_k, void* stream) {
-  OCNN_REQUIRE(ocnnx_gather_tile_supported(dtype, rows_in, K, cin, cout, plan_max_distinct),
-               "conv_gather_tile: shape not supported");
-  OCNN_REQUIRE(rows_out >= 0 && rows_out < (1ll << 31) && plan_total >= 0 && plan_total < (1ll << 29),
-               "conv_gather_tile: rows out of range");
-  if (rows_out == 0) return OCNN_OK;
-  OCNN_REQUIRE_PTRS("conv_gather_tile", loc, uptr, urows, w, out, workspace);
-  OCNN_REQUIRE(rows_in == 0 || in, "conv_gather_tile: in is NULL");
-  if (workspace_bytes < (dtype == OCNN_F32 ? (int64_t)K * cin * cout * 4 : (int64_t)K * align_up(cin, 64) * cout * 2)) {
-    set_error("conv_gather_tile: workspace too small");
-    return OCNN_ERR_WORKSPACE;
+  Pass* pass = nullptr;
+  int rc = tile_pass(dtype, {in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out, K, w, cin,
+                             cout, w_transposed, reverse_slots, bias, bn_or_null, out, workspace, workspace_bytes, split_c,
+                             split_k}, (hipStream_t)stream, &pass);
+  if (pass) {
+    launch_jobs(dtype, pass->before, (hipStream_t)stream);
+    rc = pass->main();
+    if (rc == OCNN_OK) launch_jobs(dtype, pass->after, (hipStream_t)stream);
+    delete pass;
   }
-  hipStream_t st = (hipStream_t)stream;
-  ocnnx_bn bn = {};
-  if (bn_or_null) bn = *bn_or_null;
-  // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
-  const bool skip = K != 8 && plan_occupancy >= 0.0 && plan_occupancy <= kTgSkipMaxOccupancy;
-  if (dtype == OCNN_F32)
-    return run_tile<bf16, true>(in, rows_in, loc, uptr, urows, plan_max_distinct, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
-                                bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
-  if (dtype == OCNN_F16)
-    return run_tile<f16, false>(in, rows_in, loc, uptr, urows, plan_max_distinct, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
-                                bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
-  return run_tile<bf16, false>(in, rows_in, loc, uptr, urows, plan_max_distinct, rows_out, K, cin, cout, w, w_transposed, reverse_slots,
-                               bias, bn, out, workspace, workspace_bytes, skip, split_c, split_k, st);
+  return rc == OCNN_OK ? check_launch("conv_gather_tile") : rc;
 }
 
 // The public entry point: 16-bit wide layers, with whatever room for parts the workspace has.

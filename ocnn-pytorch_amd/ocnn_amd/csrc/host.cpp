@@ -156,7 +156,6 @@ struct GatherOp {
     return followed(view_cols ? out.view({-1, view_cols}) : out, bn);
   }
 
- private:
   // this pass with row i of its result written to row index[i] of `out`
   void run_into(Tensor& out, const Tensor& index, const Tensor& data, const Tensor& table, const Tensor& W,
                 const OptTensor& bias) const {
@@ -172,6 +171,7 @@ struct GatherOp {
                             cout, transposed, reverse, ptr(bias), out.data_ptr(), typed<int64_t>(index), ws.data_ptr(),
                             ws.numel(), hip_stream()));
   }
+ private:
   static Tensor followed(const Tensor& out, const ocnnx_bn* bn) {
     if (bn && out.size(0))
       check(ocnnx_batch_norm_running(code_of(out.scalar_type()), out.data_ptr(), out.size(0), (int)out.size(1), bn->mean,
@@ -258,6 +258,40 @@ struct WgradOp {
   }
 };
 
+// Data, weight and (want_bias) bias gradient of a layer in one call, for the pair of kernels whose small launches can
+// be merged; false where the passes are others.
+bool backward_together(const GatherOp& dgrad, const WgradOp& wgrad, const Tensor& grad, const Tensor& w, const Tensor& x,
+                       const Tensor& g, bool want_bias, variable_list& out) {
+  if (dgrad.kernel != OCNNX_GATHER_TILE || wgrad.kernel != OCNN_WGRAD_PLANNED || dgrad.padded || wgrad.padded) return false;
+  for (const Tensor& t : {grad, w, x, g})
+    if (!t.is_cuda() || !t.is_contiguous() || t.scalar_type() != grad.scalar_type()) return false;
+  if (w.numel() != (int64_t)dgrad.K * dgrad.cin * dgrad.cout) return false;
+  const int code = code_of(grad.scalar_type());
+  Tensor gx = at::empty({dgrad.rows, dgrad.cout}, grad.options());
+  Tensor gw = at::empty({wgrad.K, wgrad.out_transposed ? wgrad.cb : wgrad.ca, wgrad.out_transposed ? wgrad.ca : wgrad.cb},
+                        grad.options());
+  Tensor gb = want_bias ? at::empty({grad.size(1)}, grad.options()) : Tensor();
+  // (each with a workspace of its own: the passes overlap)
+  Tensor ws_d = workspace(dgrad.ws_bytes, grad), ws_w = workspace(wgrad.ws_bytes, grad);
+  Tensor ws_b = want_bias ? workspace(ocnn_colsum_workspace_bytes(grad.size(0), (int)grad.size(1)), grad) : Tensor();
+  const PlanArrays &p = *dgrad.plan, &q = *wgrad.plan;
+  const ocnnx_gather_args da{ptr(grad), dgrad.rows_in, typed<uint16_t>(p.loc), typed<int32_t>(p.uptr), typed<int32_t>(p.urows),
+                             p.umax, p.total, p.occupancy, dgrad.rows, dgrad.K, ptr(w), dgrad.cin, dgrad.cout,
+                             dgrad.transposed, dgrad.reverse, nullptr, nullptr, gx.data_ptr(), ws_d.data_ptr(), ws_d.numel(),
+                             0, 0};
+  const ocnnx_wgrad_args wa{ptr(x), wgrad.rows_x, ptr(g), typed<uint16_t>(q.loc), typed<int32_t>(q.uptr),
+                            typed<int32_t>(q.urows), q.umax, q.total, wgrad.rows, wgrad.K, wgrad.ca, wgrad.cb,
+                            wgrad.out_transposed, gw.data_ptr(), ws_w.data_ptr(), ws_w.numel()};
+  check(ocnnx_conv_backward(code, &da, &wa, ptr(grad), grad.size(0), (int)grad.size(1), gb.defined() ? gb.data_ptr() : nullptr,
+                            gb.defined() ? ws_b.data_ptr() : nullptr, gb.defined() ? ws_b.numel() : 0, hip_stream()));
+  if (dgrad.overflow) dgrad.overflow->run_into(gx, dgrad.overflow_rows, grad, dgrad.overflow_table, w, std::nullopt);
+  if (wgrad.overflow) gw.add_(wgrad.overflow->run(x, g.index_select(0, wgrad.overflow_rows), wgrad.overflow_table));
+  out[0] = dgrad.view_cols ? gx.view({-1, dgrad.view_cols}) : gx;
+  out[1] = wgrad.shape.empty() ? gw : gw.view(wgrad.shape);
+  out[2] = gb;
+  return true;
+}
+
 Tensor column_sum(Tensor g) {
   require_gpu(g);
   g = g.contiguous();
@@ -303,6 +337,10 @@ struct ConvBackward : public Node {
     if (!grads[0].defined()) return out;
     Tensor grad = grads[0].contiguous(), x = data.unpack(), w = weights.unpack();
     at::AutoDispatchBelowADInplaceOrView below;
+    if (task_should_compute_output(0) && task_should_compute_output(1) &&
+        backward_together(*layer->dgrad, *layer->wgrad, grad, w, layer->wgrad_of_grad ? grad : x,
+                          layer->wgrad_of_grad ? x : grad, task_should_compute_output(2), out))
+      return out;
     if (task_should_compute_output(0)) out[0] = layer->dgrad->run(grad, layer->dgrad_table, w, std::nullopt);
     if (task_should_compute_output(1))
       out[1] = layer->wgrad_of_grad ? layer->wgrad->run(grad, x, layer->wgrad_table)

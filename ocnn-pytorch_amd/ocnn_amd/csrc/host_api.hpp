@@ -34,6 +34,43 @@ int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t
                       const void* bias, const ocnnx_bn* bn, void* out, void* workspace, int64_t workspace_bytes,
                       int split_c, int split_k, void* stream);
 
+// The backward pass of a layer whose data gradient is ocnnx_gather_tile's and whose weight gradient is
+// ocnn_conv_wgrad_planned's, with the bias gradient (column sums of grad; null: none): as the calls one
+// behind the other, but the launches around the two kernels merged into one before and one after them.
+typedef struct {
+  const void* in;
+  int64_t rows_in;
+  const uint16_t* loc;
+  const int32_t *uptr, *urows;
+  int plan_max_distinct;
+  int64_t plan_total;
+  double plan_occupancy;
+  int64_t rows_out;
+  int K;
+  const void* w;
+  int cin, cout, w_transposed, reverse_slots;
+  const void* bias;
+  const ocnnx_bn* bn;
+  void *out, *workspace;
+  int64_t workspace_bytes;
+  int split_c, split_k;
+} ocnnx_gather_args;
+typedef struct {
+  const void* x;
+  int64_t rows_x;
+  const void* g;
+  const uint16_t* loc;
+  const int32_t *uptr, *urows;
+  int plan_max_distinct;
+  int64_t plan_total, rows;
+  int K, ca, cb, out_transposed;
+  void *gw, *workspace;
+  int64_t workspace_bytes;
+} ocnnx_wgrad_args;
+int ocnnx_conv_backward(int dtype, const ocnnx_gather_args* dgrad, const ocnnx_wgrad_args* wgrad, const void* grad,
+                        int64_t grad_rows, int grad_channels, void* bias_grad, void* colsum_workspace, int64_t colsum_bytes,
+                        void* stream);
+
 // ocnn_conv_gather with row i of the result at row out_index[i] (null: i), and with the room that lets a launch of few
 // rows split its reduction (with less, but ocnn_conv_gather_workspace_bytes, it runs in one part).
 int64_t ocnnx_conv_gather_workspace_bytes(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout);

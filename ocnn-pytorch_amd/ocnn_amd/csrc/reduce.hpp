@@ -30,13 +30,13 @@ __global__ void wgrad_reduce_kernel(const float* __restrict__ partial, int split
 // With ca > 0 the output is (K, cb, ca): the four sums of a thread (consecutive b) go to
 // four rows of the transposed block.
 template <typename T, int LANES>
-__global__ __launch_bounds__(256) void wgrad_reduce4_kernel(const float* __restrict__ partial, int splits, int64_t per,
-                                                            T* __restrict__ out, int ca, int cb) {
+__device__ __forceinline__ void wgrad_reduce4(const float* __restrict__ partial, int splits, int64_t per,
+                                              T* __restrict__ out, int ca, int cb, uint32_t block, float* s_sums) {
   typedef __attribute__((ext_vector_type(4))) float v4;
   constexpr int COLS = 256 / LANES;
-  __shared__ v4 s_sum[LANES > 1 ? 256 : 1];
+  v4* s_sum = (v4*)s_sums;                                   // 256 of them (LANES > 1)
   const int col = threadIdx.x % COLS, l = threadIdx.x / COLS;
-  const int64_t e = ((int64_t)blockIdx.x * COLS + col) * 4;
+  const int64_t e = ((int64_t)block * COLS + col) * 4;
   v4 acc = v4{0.f, 0.f, 0.f, 0.f};
   if (e < per) {
     int s = l;
@@ -72,15 +72,25 @@ __global__ __launch_bounds__(256) void wgrad_reduce4_kernel(const float* __restr
   }
 }
 
+template <typename T, int LANES>
+__global__ __launch_bounds__(256) void wgrad_reduce4_kernel(const float* __restrict__ partial, int splits, int64_t per,
+                                                            T* __restrict__ out, int ca, int cb) {
+  __shared__ __attribute__((aligned(16))) float s_sums[LANES > 1 ? 1024 : 4];
+  wgrad_reduce4<T, LANES>(partial, splits, per, out, ca, cb, blockIdx.x, s_sums);
+}
+
+// lanes a column: as many as leave the launch a few waves a SIMD
+inline int wgrad_reduce_lanes(int splits, int64_t per) { return splits >= 16 && per / 4 < 65536 ? 8 : 1; }
+
 // fp32 values as two bf16 pieces: x = hi + lo (+ 2^-17 |x|); a product of two such values is
 // hi_a hi_b + hi_a lo_b + lo_a hi_b to about 1e-5 relative.  Two tensors (x, then g) in one launch,
 // eight values a thread (counts are multiples of 8).
-static __global__ __launch_bounds__(256) void split2_kernel(const float* __restrict__ x, int64_t nx, bf16* __restrict__ xh,
-                                                            bf16* __restrict__ xl, const float* __restrict__ g, int64_t ng,
-                                                            bf16* __restrict__ gh, bf16* __restrict__ gl) {
+static __device__ __forceinline__ void split2(const float* __restrict__ x, int64_t nx, bf16* __restrict__ xh,
+                                              bf16* __restrict__ xl, const float* __restrict__ g, int64_t ng,
+                                              bf16* __restrict__ gh, bf16* __restrict__ gl, uint32_t block) {
   typedef __attribute__((ext_vector_type(4))) float v4;
   typedef __attribute__((ext_vector_type(8))) bf16 b8;
-  int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  int64_t e = ((int64_t)block * 256 + threadIdx.x) * 8;
   const float* src = x;
   bf16 *hi = xh, *lo = xl;
   if (e >= nx) {
@@ -100,6 +110,12 @@ static __global__ __launch_bounds__(256) void split2_kernel(const float* __restr
   *(b8*)(lo + e) = l;
 }
 
+static __global__ __launch_bounds__(256) void split2_kernel(const float* __restrict__ x, int64_t nx, bf16* __restrict__ xh,
+                                                            bf16* __restrict__ xl, const float* __restrict__ g, int64_t ng,
+                                                            bf16* __restrict__ gh, bf16* __restrict__ gl) {
+  split2(x, nx, xh, xl, g, ng, gh, gl, blockIdx.x);
+}
+
 inline void launch_split2(const void* x, int64_t nx, bf16* xh, bf16* xl, const void* g, int64_t ng, bf16* gh, bf16* gl,
                           hipStream_t st) {
   if (nx + ng > 0)
@@ -113,10 +129,9 @@ inline void launch_wgrad_reduce(const float* partial, int splits, int K, int ca,
                                 int out_transposed, T* out, hipStream_t st) {
   const int64_t per = (int64_t)K * ca * cb;
   if (cb % 4 == 0 && ((uintptr_t)partial % 16) == 0) {
-    // lanes a column: as many as leave the launch a few waves a SIMD
     const int64_t cols = per / 4;
     const int ot = out_transposed ? ca : 0;
-    if (splits >= 16 && cols < 65536)
+    if (wgrad_reduce_lanes(splits, per) == 8)
       hipLaunchKernelGGL((wgrad_reduce4_kernel<T, 8>), dim3((unsigned)cdiv(cols, 32)), dim3(256), 0, st, partial, splits,
                          per, out, ot, cb);
     else

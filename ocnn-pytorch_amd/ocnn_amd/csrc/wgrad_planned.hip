@@ -14,9 +14,10 @@
 // the gather of the x rows for free.  Per-range sums go to `partial` and are
 // added in range order by a second kernel: no atomics, fixed summation order.
 #include <algorithm>
+#include <new>
 #include <type_traits>
 
-#include "common.hpp"
+#include "jobs.hpp"
 #include "mma.hpp"
 #include "reduce.hpp"
 
@@ -509,40 +510,80 @@ static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
 // T: the type of x, g and gw.  float: x and g go through the kernel as two bf16 pieces each, the three
 // products as workgroups of one launch with sums of their own (a third of the ranges each: a third
 // of the sums to add up, and one launch where a small layer waited for three), one reduction over all of them
-template <typename T>
-static int run_wp(const void* x, int64_t rows_x, const void* g, const uint16_t* loc, const int32_t* uptr,
-                  const int32_t* urows, int64_t plan_total, int64_t rows, int K, int ca, int cb,
-                  int out_transposed, void* gw, void* ws, int64_t ws_bytes, hipStream_t st) {
-  constexpr bool kPieces = std::is_same<T, float>::value;
-  const int n_cu = wp_cu_count();
-  if (n_cu <= 0) {
-    set_error("conv_wgrad_planned: cannot query the device");
-    return OCNN_ERR_HIP;
-  }
-  WpArgs a{x, g, nullptr, nullptr, kPieces ? 3 : 1, rows_x, rows, 0, 0, plan_total, loc, uptr, urows, K, ca, cb, 0, nullptr};
-  const int64_t tiles = cdiv(rows, kWpRows);
-  a.per = wp_tiles_per_range(tiles, K, ca, cb, n_cu, a.products);
-  a.used = (int)cdiv(tiles, a.per);
-  a.set = (int64_t)a.used * K * ca * cb;                     // floats of one set of sums
-  const int64_t xb = kPieces ? align_up(rows_x * ca * 2, 256) : 0, gb = kPieces ? align_up(rows * cb * 2, 256) : 0;
-  if (ws_bytes < 2 * xb + 2 * gb + a.products * a.set * 4) {
-    set_error("conv_wgrad_planned: workspace too small");
-    return OCNN_ERR_WORKSPACE;
-  }
-  a.partial = (float*)((char*)ws + 2 * xb + 2 * gb);
-  if (rows > 0) {
-    if constexpr (kPieces) {
-      bf16 *xh = (bf16*)ws, *xl = (bf16*)((char*)ws + xb);
-      bf16 *gh = (bf16*)((char*)ws + 2 * xb), *gl = (bf16*)((char*)ws + 2 * xb + gb);
-      launch_split2(x, rows_x * ca, xh, xl, g, rows * cb, gh, gl, st);
-      a.x = xh, a.x_lo = xl, a.g = gh, a.g_lo = gl;
-      launch_wp_sums<bf16>(a, st);
-    } else {
-      launch_wp_sums<T>(a, st);
+template <typename T> struct WpPass : Pass {
+  WpArgs a;
+  hipStream_t st;
+  int rc = OCNN_OK, splits = 0, out_transposed = 0;
+  void* gw = nullptr;         // set: the reduction is launched behind the kernel (sums at an odd address)
+
+  WpPass(const ocnnx_wgrad_args& p, hipStream_t stream) : st(stream) {
+    constexpr bool kPieces = std::is_same<T, float>::value;
+    const int n_cu = wp_cu_count();
+    if (n_cu <= 0) {
+      set_error("conv_wgrad_planned: cannot query the device");
+      rc = OCNN_ERR_HIP;
+      return;
     }
+    const int K = p.K, ca = p.ca, cb = p.cb;
+    a = WpArgs{p.x, p.g, nullptr, nullptr, kPieces ? 3 : 1, p.rows_x, p.rows, 0, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0,
+               nullptr};
+    const int64_t tiles = cdiv(p.rows, kWpRows);
+    a.per = wp_tiles_per_range(tiles, K, ca, cb, n_cu, a.products);
+    a.used = (int)cdiv(tiles, a.per);
+    a.set = (int64_t)a.used * K * ca * cb;                   // floats of one set of sums
+    const int64_t nx = p.rows_x * ca, ng = p.rows * cb;
+    const int64_t xb = kPieces ? align_up(nx * 2, 256) : 0, gb = kPieces ? align_up(ng * 2, 256) : 0;
+    if (p.workspace_bytes < 2 * xb + 2 * gb + a.products * a.set * 4) {
+      set_error("conv_wgrad_planned: workspace too small");
+      rc = OCNN_ERR_WORKSPACE;
+      return;
+    }
+    char* ws = (char*)p.workspace;
+    a.partial = (float*)(ws + 2 * xb + 2 * gb);
+    if (kPieces && p.rows > 0) {
+      bf16 *xh = (bf16*)ws, *xl = (bf16*)(ws + xb), *gh = (bf16*)(ws + 2 * xb), *gl = (bf16*)(ws + 2 * xb + gb);
+      Job j{Job::kSplit, (unsigned)cdiv((nx + ng) / 8, 256), {}};
+      j.split = SplitJob{(const float*)p.x, (const float*)p.g, xh, xl, gh, gl, nx, ng};
+      before.add(j);
+      a.x = xh, a.x_lo = xl, a.g = gh, a.g_lo = gl;
+    }
+    const int64_t per = (int64_t)K * ca * cb;
+    splits = p.rows > 0 ? a.products * a.used : 0;
+    if ((uintptr_t)a.partial % 16 != 0) {
+      gw = p.gw, out_transposed = p.out_transposed;
+      return;
+    }
+    const int lanes = wgrad_reduce_lanes(splits, per);
+    Job j{Job::kReduce, (unsigned)cdiv(per / 4, 256 / lanes), {}};
+    j.reduce = ReduceJob{a.partial, p.gw, per, splits, p.out_transposed ? ca : 0, cb, lanes};
+    after.add(j);
   }
-  launch_wgrad_reduce<T>(a.partial, rows > 0 ? a.products * a.used : 0, K, ca, cb, out_transposed, (T*)gw, st);
-  return check_launch("conv_wgrad_planned");
+
+  int main() override {
+    if (a.rows > 0) launch_wp_sums<typename std::conditional<std::is_same<T, float>::value, bf16, T>::type>(a, st);
+    if (gw) launch_wgrad_reduce<T>(a.partial, splits, a.K, a.ca, a.cb, out_transposed, (T*)gw, st);
+    return check_launch("conv_wgrad_planned");
+  }
+};
+
+// The pass for these arguments, to be deleted by the caller.
+int ocnn::wgrad_planned_pass(int dtype, const ocnnx_wgrad_args& p, hipStream_t st, Pass** pass) {
+  *pass = nullptr;
+  OCNN_REQUIRE(ocnn_conv_wgrad_planned_supported(dtype, p.rows_x, p.rows, p.K, p.ca, p.cb, p.plan_max_distinct),
+               "conv_wgrad_planned: shape not supported");
+  OCNN_REQUIRE(p.rows >= 0 && (int64_t)p.rows * p.K * 2 < 0xfff00000ll && p.plan_total >= 0 && p.plan_total < (1ll << 29),
+               "conv_wgrad_planned: rows out of range");
+  OCNN_REQUIRE_PTRS("conv_wgrad_planned", p.gw, p.workspace);
+  OCNN_REQUIRE(p.rows == 0 || (p.g && p.loc && p.uptr && p.urows && (p.rows_x == 0 || p.x)),
+               "conv_wgrad_planned: a required pointer is NULL (of x, g, loc, uptr, urows)");
+  auto made = [&](auto* wp) {
+    OCNN_REQUIRE(wp, "conv_wgrad_planned: out of host memory");
+    *pass = wp;
+    return wp->rc;
+  };
+  if (dtype == OCNN_F32) return made(new (std::nothrow) WpPass<float>(p, st));
+  if (dtype == OCNN_F16) return made(new (std::nothrow) WpPass<f16>(p, st));
+  return made(new (std::nothrow) WpPass<bf16>(p, st));
 }
 
 extern "C" int ocnn_conv_wgrad_planned(int dtype, const void* x, int64_t rows_x, const void* g,
@@ -550,21 +591,14 @@ extern "C" int ocnn_conv_wgrad_planned(int dtype, const void* x, int64_t rows_x,
                                        int plan_max_distinct, int64_t plan_total, int64_t rows, int K,
                                        int ca, int cb, int out_transposed, void* gw, void* workspace,
                                        int64_t workspace_bytes, void* stream) {
-  OCNN_REQUIRE(ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct),
-               "conv_wgrad_planned: shape not supported");
-  OCNN_REQUIRE(rows >= 0 && (int64_t)rows * K * 2 < 0xfff00000ll && plan_total >= 0 &&
-                   plan_total < (1ll << 29),
-               "conv_wgrad_planned: rows out of range");
-  OCNN_REQUIRE_PTRS("conv_wgrad_planned", gw, workspace);
-  OCNN_REQUIRE(rows == 0 || (g && loc && uptr && urows && (rows_x == 0 || x)),
-               "conv_wgrad_planned: a required pointer is NULL (of x, g, loc, uptr, urows)");
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == OCNN_F32)
-    return run_wp<float>(x, rows_x, g, loc, uptr, urows, plan_total, rows, K, ca, cb, out_transposed, gw, workspace,
-                         workspace_bytes, st);
-  if (dtype == OCNN_F16)
-    return run_wp<f16>(x, rows_x, g, loc, uptr, urows, plan_total, rows, K, ca, cb, out_transposed, gw, workspace,
-                       workspace_bytes, st);
-  return run_wp<bf16>(x, rows_x, g, loc, uptr, urows, plan_total, rows, K, ca, cb, out_transposed, gw, workspace,
-                      workspace_bytes, st);
+  Pass* pass = nullptr;
+  int rc = wgrad_planned_pass(dtype, {x, rows_x, g, loc, uptr, urows, plan_max_distinct, plan_total, rows, K, ca, cb,
+                                      out_transposed, gw, workspace, workspace_bytes}, (hipStream_t)stream, &pass);
+  if (rc == OCNN_OK) {
+    launch_jobs(dtype, pass->before, (hipStream_t)stream);
+    rc = pass->main();
+    if (rc == OCNN_OK) launch_jobs(dtype, pass->after, (hipStream_t)stream);
+  }
+  delete pass;
+  return rc == OCNN_OK ? check_launch("conv_wgrad_planned") : rc;
 }
