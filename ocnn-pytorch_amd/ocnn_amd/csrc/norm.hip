@@ -5,6 +5,11 @@
 // costs none) and 16-byte accesses on channels-last rows.  Reductions are two-level with a
 // fixed order (per-workgroup partial sums, then one thread per channel in fp64): no atomics,
 // bit-reproducible.
+//
+// The sums walk the rows from the first to the last, all workgroups side by side, and the elementwise pass that
+// reads the same tensors again walks them back: what was read last is in the memory-side cache (256 MB).  With a range
+// of rows per workgroup in both, 1.1 M x 96 fp16 took 135 + 236 us forward + backward, now 131 + 209; 900 k x 96 with a
+// residual 139 + 238, now 129 + 212; 40 k rows the same.
 #include <algorithm>
 #include <mutex>
 #include <utility>
@@ -68,12 +73,11 @@ __device__ __forceinline__ void bn_store(void* p, int dtype, int c, float v) {
 }
 
 // partial[blk][0][c] = sum_r (x[r][c] - x[0][c]),  partial[blk][1][c] = sum_r (x[r][c] - x[0][c])^2
-// over the rows of the workgroup (shifting by the first row keeps the variance free of
+// over the rows of the workgroup, blocks of 4 rpp of them gridDim.x apart (shifting by the first row keeps the variance free of
 // cancellation when the mean is large against the spread).  Thread: VEC channels of every
 // rpp-th row.
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void bn_stats_kernel(const T* __restrict__ x, int64_t rows, int C,
-                                                       int64_t rows_per_blk, float* __restrict__ partial) {
+__global__ __launch_bounds__(256) void bn_stats_kernel(const T* __restrict__ x, int64_t rows, int C, float* __restrict__ partial) {
   typedef BnVec<T, VEC> V;
   __shared__ float s_a[256 * VEC], s_b[256 * VEC];
   const int lpr = C / VEC, rpp = 256 / lpr;
@@ -83,15 +87,13 @@ __global__ __launch_bounds__(256) void bn_stats_kernel(const T* __restrict__ x, 
   for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
   if (rl < rpp) {
     const V k = *(const V*)(x + cl * VEC);
-    const int64_t r0 = (int64_t)blockIdx.x * rows_per_blk;
-    const int64_t r1 = min(rows, r0 + rows_per_blk);
     // four rows in flight per thread (rows past the end repeat row 0, whose shifted value is 0)
-    for (int64_t r = r0 + rl; r < r1; r += 4 * rpp) {
+    for (int64_t r = (int64_t)blockIdx.x * (4 * rpp) + rl; r < rows; r += (int64_t)gridDim.x * (4 * rpp)) {
       V a[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int64_t ru = r + (int64_t)u * rpp;
-        a[u] = *(const V*)(x + (ru < r1 ? ru * C : 0) + cl * VEC);
+        a[u] = *(const V*)(x + (ru < rows ? ru * C : 0) + cl * VEC);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
@@ -197,13 +199,11 @@ __global__ __launch_bounds__(kBnFinishThreads) void bn_stats_finish_kernel(
 }
 
 // y = (x - mean) * (invstd * gamma) + beta (+ res), then max(., 0) when relu.  A thread keeps the
-// constants of its VEC channels in registers and walks every rpp-th row of the workgroup's
-// range, four rows in flight.  run_mean, run_var (dtype rdtype), when given, take the place of mean
+// constants of its VEC channels in registers and walks the rows back to the first, four rows in flight.  run_mean, run_var (dtype rdtype), when given, take the place of mean
 // and invstd: a module's running statistics as it holds them, the reciprocal formed here (made into
 // mean and invstd by passes of their own they were four of the five launches of a layer in evaluation).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, int64_t rows, int C,
-                                                       int64_t rows_per_blk,
                                                        const float* __restrict__ mean,
                                                        const float* __restrict__ invstd,
                                                        const void* __restrict__ gamma,
@@ -233,14 +233,14 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
 #pragma unroll
     for (int v = 0; v < VEC; ++v) sc[v] *= ga[v];
   }
-  const int64_t r0 = (int64_t)blockIdx.x * rows_per_blk;
-  const int64_t r1 = min(rows, r0 + rows_per_blk);
-  for (int64_t r = r0 + rl; r < r1; r += 4 * rpp) {
+  const int64_t last = (rows + 4 * rpp - 1) / (4 * rpp) - 1;
+  for (int64_t at = last - blockIdx.x; at >= 0; at -= gridDim.x) {
+    const int64_t r = at * (4 * rpp) + rl;
     V a[4], b[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int64_t ru = r + (int64_t)u * rpp;
-      if (ru < r1) {
+      if (ru < rows) {
         a[u] = *(const V*)(x + ru * C + cl * VEC);
         if (res) b[u] = *(const V*)(res + ru * C + cl * VEC);
       }
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int64_t ru = r + (int64_t)u * rpp;
-      if (ru >= r1) continue;
+      if (ru >= rows) continue;
       V o;
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
 // ymask: the forward output, when it is not a function of x alone (a residual was added).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__ x, const T* __restrict__ dy,
-                                                           int64_t rows, int C, int64_t rows_per_blk,
+                                                           int64_t rows, int C,
                                                            const float* __restrict__ mean,
                                                            const float* __restrict__ invstd,
                                                            const void* __restrict__ gamma,
@@ -289,15 +289,13 @@ __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__
       is[v] = invstd[cl * VEC + v];
     }
     bn_params<VEC>(gamma, beta, pdtype, cl * VEC, ga, be);
-    const int64_t r0 = (int64_t)blockIdx.x * rows_per_blk;
-    const int64_t r1 = min(rows, r0 + rows_per_blk);
-    for (int64_t r = r0 + rl; r < r1; r += 4 * rpp) {          // four rows of both tensors in flight
+    for (int64_t r = (int64_t)blockIdx.x * (4 * rpp) + rl; r < rows; r += (int64_t)gridDim.x * (4 * rpp)) {   // four rows of both tensors in flight
       V a[4], g[4], ym[4];
       bool ok[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int64_t ru = r + (int64_t)u * rpp;
-        ok[u] = ru < r1;
+        ok[u] = ru < rows;
         a[u] = *(const V*)(x + (ok[u] ? ru * C : 0) + cl * VEC);
         g[u] = *(const V*)(dy + (ok[u] ? ru * C : 0) + cl * VEC);
         if (ymask) ym[u] = *(const V*)(ymask + (ok[u] ? ru * C : 0) + cl * VEC);
@@ -353,7 +351,7 @@ __global__ __launch_bounds__(kBnFinishThreads) void bn_bwd_finish_kernel(const f
 // (evaluation mode): dx = gamma * invstd * dy'.  Thread layout as in bn_apply_kernel.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__ x, const T* __restrict__ dy,
-                                                           int64_t rows, int C, int64_t rows_per_blk,
+                                                           int64_t rows, int C,
                                                            const float* __restrict__ mean,
                                                            const float* __restrict__ invstd,
                                                            const void* __restrict__ gamma,
@@ -379,14 +377,14 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
   bn_params<VEC>(gamma, beta, pdtype, cl * VEC, sc, be);
 #pragma unroll
   for (int v = 0; v < VEC; ++v) sc[v] *= is[v];
-  const int64_t r0 = (int64_t)blockIdx.x * rows_per_blk;
-  const int64_t r1 = min(rows, r0 + rows_per_blk);
-  for (int64_t r = r0 + rl; r < r1; r += 2 * rpp) {     // (four rows in flight cost more in occupancy than they gain)
+  const int64_t last = (rows + 2 * rpp - 1) / (2 * rpp) - 1;       // (four rows in flight cost more in occupancy than they gain)
+  for (int64_t at = last - blockIdx.x; at >= 0; at -= gridDim.x) {
+    const int64_t r = at * (2 * rpp) + rl;
     V a[2], g[2], ym[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t ru = r + (int64_t)u * rpp;
-      if (ru < r1) {
+      if (ru < rows) {
         a[u] = *(const V*)(x + ru * C + cl * VEC);
         g[u] = *(const V*)(dy + ru * C + cl * VEC);
         if (ymask) ym[u] = *(const V*)(ymask + ru * C + cl * VEC);
@@ -395,7 +393,7 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t ru = r + (int64_t)u * rpp;
-      if (ru >= r1) continue;
+      if (ru >= rows) continue;
       V o, gr;
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
@@ -660,11 +658,10 @@ extern "C" int ocnn_batch_norm_supported(int dtype, int64_t rows, int channels) 
   return rows >= 1;
 }
 
-// rows of a workgroup (a multiple of the rows its threads cover per pass) and their number
-static void bn_blocks(int dtype, int64_t rows, int channels, int max_blocks, int64_t* per, int* nblk) {
+// workgroups: one for every four rows a thread, max_blocks at most
+static int bn_blocks(int dtype, int64_t rows, int channels, int max_blocks) {
   const int rpp = 256 / (channels / bn_vec(dtype));
-  *per = align_up(std::max<int64_t>(cdiv(rows, max_blocks), 4 * rpp), rpp);
-  *nblk = (int)cdiv(rows, *per);
+  return (int)std::min<int64_t>(max_blocks, cdiv(rows, 4 * rpp));
 }
 
 // Workgroups of 256 threads of `kernel` that the device holds at once, kBnApplyBlocks at most:
@@ -700,14 +697,11 @@ extern "C" int ocnn_batch_norm_stats(int dtype, const void* x, int64_t rows, int
   OCNN_REQUIRE_PTRS("batch_norm_stats", x, mean, var, invstd, workspace);
   OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels), "batch_norm_stats: workspace too small");
   hipStream_t st = (hipStream_t)stream;
-  int64_t per;
-  int nblk;
-  bn_blocks(dtype, rows, channels, kBnMaxBlocks, &per, &nblk);
+  const int nblk = bn_blocks(dtype, rows, channels, kBnMaxBlocks);
   float* partial = (float*)workspace;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
-    hipLaunchKernelGGL((bn_stats_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, per,
-                       partial);
+    hipLaunchKernelGGL((bn_stats_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, partial);
     hipLaunchKernelGGL(bn_stats_finish_kernel<T>, dim3((unsigned)cdiv(channels, 4)), dim3(kBnFinishThreads), 0, st,
                        partial, nblk, (const T*)x, rows, channels, eps, mean, var, invstd, running_mean, running_var, running_dtype,
                        factor, (long long*)batches_tracked);
@@ -718,13 +712,10 @@ extern "C" int ocnn_batch_norm_stats(int dtype, const void* x, int64_t rows, int
 static int bn_apply(int dtype, const void* x, int64_t rows, int channels, const float* mean, const float* invstd,
                     const void* gamma, const void* beta, int param_dtype, int relu, const void* residual, void* y,
                     const void* run_mean, const void* run_var, int run_dtype, float eps, hipStream_t st) {
-  int64_t per;
-  int nblk;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
-    bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_apply_kernel<T, VEC>), &per, &nblk);
-    hipLaunchKernelGGL((bn_apply_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, per,
-                       mean, invstd, gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var,
+    const int nblk = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_apply_kernel<T, VEC>));
+    hipLaunchKernelGGL((bn_apply_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var,
                        run_dtype, eps);
   });
   return check_launch("batch_norm_apply");
@@ -786,10 +777,6 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
   OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels),
                "batch_norm_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
-  int64_t per;
-  int nblk;
-  int64_t per_a;
-  int nblk_a;
   if (dx && rows <= kBnSmallRows) {
     OCNN_DISPATCH_DTYPE(dtype, {
       constexpr int VEC = 16 / sizeof(T);
@@ -800,18 +787,18 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
     });
     return check_launch("batch_norm_backward");
   }
-  bn_blocks(dtype, rows, channels, kBnMaxBlocks, &per, &nblk);
+  const int nblk = bn_blocks(dtype, rows, channels, kBnMaxBlocks);
   float* partial = (float*)workspace;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
-    bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_bwd_apply_kernel<T, VEC>), &per_a, &nblk_a);
+    const int nblk_a = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_bwd_apply_kernel<T, VEC>));
     hipLaunchKernelGGL((bn_bwd_stats_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, (const T*)dy, rows,
-                       channels, per, mean, invstd, gamma, beta, param_dtype, relu, (const T*)y, partial);
+                       channels, mean, invstd, gamma, beta, param_dtype, relu, (const T*)y, partial);
     hipLaunchKernelGGL(bn_bwd_finish_kernel, dim3((unsigned)cdiv(channels, 4)), dim3(kBnFinishThreads), 0, st, partial, nblk,
                        channels, dbeta, dgamma, grad_gamma, grad_beta, param_dtype);
     if (dx)
       hipLaunchKernelGGL((bn_bwd_apply_kernel<T, VEC>), dim3(nblk_a), dim3(256), 0, st, (const T*)x, (const T*)dy, rows,
-                         channels, per_a, mean, invstd, gamma, beta, param_dtype, relu, dbeta, dgamma, training,
+                         channels, mean, invstd, gamma, beta, param_dtype, relu, dbeta, dgamma, training,
                          (const T*)y, (T*)d_residual, (T*)dx);
   });
   return check_launch("batch_norm_backward");
