@@ -72,17 +72,19 @@ extern "C" int ocnn_conv_gather_choose(int dtype, int64_t rows_in, int64_t rows_
 //    run apart (plan_overflow): the second launch and the copy of its rows cost 10 - 40 us, which pays from
 //    kTileMinProductsApart on (fp32: three products a pair).  18.8 k rows of 3x3x1 stride 2: 128 -> 128 39 / 19,
 //    fp32 111 / 68; 235 k rows: 106 / 97, fp32 433 / 449 and 64 -> 64 202 / 178.
-// It also takes the place of the pair plan (OCNN_GATHER_SPARSE) but on 27 slots with few entries set, where blocks of rows
-// without an entry are the rule and pairs the better form (us, pair plan / tile kernel, f16, 96 -> 96 and 128 -> 128): 1.13 M
-// rows 7 % set 348 / 423, 529 / 540, inverse stride-2 tables 5 - 9 % set 1.1 - 1.4 x slower on the tile kernel; 822 k rows
-// 14 % set 338 / 379, 609 / 497; 947 k rows 15 % set 397 / 390, 578 / 504; 533 k rows 20 % set 257 / 238, 483 / 352; 593 k
-// rows 25 % set 328 / 282, 585 / 419.  On 8 or 9 slots the tile kernel is faster from 5 % on (1.13 M rows 240 / 228, 369 / 274).
+// It also takes the place of the pair plan (OCNN_GATHER_SPARSE) where the slots or blocks of rows without an entry are
+// many: on 8 or 9 slots, and on 27 slots but in the inverse tables of stride 2 (fewer rows read than written), where a
+// block of fine rows has something in every slot, and below 6 % set, the least that was measured (us, pair plan / tile kernel,
+// f16, 96 -> 96 and 128 -> 128): 1.13 M rows 7 % set 349 / 323, 530 / 457; 822 k rows 14 % set 339 / 339, 611 / 484; 533 k
+// rows 20 % set 257 / 221, 482 / 338; stride 2 947 k rows 7 % set 337 / 291, 479 / 409, 593 k rows 9 % set 318 / 308 for 96;
+// inverse of stride 2 1.13 M rows 6 % set 329 / 332, 505 / 449, 264 k rows 8 % set 91 / 120, 133 / 160, 593 k rows 9 % set
+// 190 / 263, 288 / 386; nine slots of 1.13 M rows 16 % set 311 / 247, 454 / 318, inverse 5 % set 241 / 195, 373 / 242.
 // Over 916 bf16 passes (six kernel shapes, strides 1 and 2, all and non-empty nodes, three octrees of 20 k - 1 M
 // points, eleven widths): all plan-free 80.1 ms, all on the tile kernel 74.1, by this rule 70.0, the faster of the
 // two each time 69.3.  Other fp32 layers gain on every table, 1.04 - 9 x: plan-free reads three copies of their rows.
 constexpr double kTileMinProducts = 3.0e9;
 constexpr double kTileMinProductsApart = 1.7e10;
-constexpr double kTileMinOccupancy = 0.12;        // of 27 slots
+constexpr double kTileMinOccupancy = 0.06, kTileMinOccupancyInverse = 0.12;        // of 27 slots
 
 extern "C" int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout,
                                    int identity_table, int has_plan, int plan_max_distinct, int64_t plan_total,
@@ -94,7 +96,10 @@ extern "C" int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out,
     return pick;
   if (pick == OCNN_GATHER_PLANNED || pick == OCNN_GATHER_WIDE) return OCNNX_GATHER_TILE;
   if (pick == OCNN_GATHER_SPARSE)
-    return (K < 27 ? (int64_t)cin * cout >= 4096 : plan_occupancy > kTileMinOccupancy) ? OCNNX_GATHER_TILE : pick;
+    return (K < 27 ? (int64_t)cin * cout >= 4096
+                   : plan_occupancy > (rows_in < rows_out ? kTileMinOccupancyInverse : kTileMinOccupancy))
+               ? OCNNX_GATHER_TILE
+               : pick;
   if (pick != OCNN_GATHER_PLAIN) return pick;
   const bool half = dtype != OCNN_F32;
   const double products = plan_occupancy * (double)rows_out * K * cin * cout * (half ? 1 : 3);

@@ -344,15 +344,17 @@ def test_selection_of_the_tile_kernel():
 def test_selection_of_the_tile_kernel_over_the_pair_plan():
   """ocnnx_gather_choose where the public choice is the pair plan: both sides of each line of its rule."""
   L, BF, SPARSE, TILE = _lib.lib(), 2, _lib.GATHER_SPARSE, _lib.GATHER_TILE
-  for rows, K, cin, cout, occ, umax, want in (
-      (925113, 27, 96, 96, 0.145, 300, TILE), (925113, 27, 96, 96, 0.121, 300, TILE), (925113, 27, 96, 96, 0.12, 300, SPARSE),
-      (925113, 27, 96, 96, 0.145, 450, SPARSE),                      # more distinct rows than the tile kernel stages
-      (925113, 9, 96, 96, 0.05, 300, TILE), (925113, 9, 64, 64, 0.05, 300, _lib.GATHER_RW),
-      (925113, 9, 32, 96, 0.05, 300, SPARSE), (925113, 9, 64, 96, 0.05, 300, TILE)):    # pairs of channels
-    a = (BF, rows, rows, K, cin, cout, 0, 1, umax, 2 * rows, occ, 4.0)
+  for rows_in, rows, K, cin, cout, occ, umax, want in (
+      (925113, 925113, 27, 96, 96, 0.145, 300, TILE), (925113, 925113, 27, 96, 96, 0.061, 300, TILE),
+      (925113, 925113, 27, 96, 96, 0.06, 300, SPARSE), (990000, 925113, 27, 96, 96, 0.061, 300, TILE),
+      (600000, 925113, 27, 96, 96, 0.12, 300, SPARSE), (600000, 925113, 27, 96, 96, 0.121, 300, TILE),   # inverse of stride 2
+      (925113, 925113, 27, 96, 96, 0.145, 450, SPARSE),              # more distinct rows than the tile kernel stages
+      (925113, 925113, 9, 96, 96, 0.05, 300, TILE), (925113, 925113, 9, 64, 64, 0.05, 300, _lib.GATHER_RW),
+      (925113, 925113, 9, 32, 96, 0.05, 300, SPARSE), (925113, 925113, 9, 64, 96, 0.05, 300, TILE)):   # pairs of channels
+    a = (BF, rows_in, rows, K, cin, cout, 0, 1, umax, 2 * rows, occ, 4.0)
     public = L.ocnn_conv_gather_choose(*a)
     assert public == (want if want == _lib.GATHER_RW else SPARSE), (K, cin, cout, occ, umax, public)
-    assert L.ocnnx_gather_choose(*a, 0) == want, (K, cin, cout, occ, umax)
+    assert L.ocnnx_gather_choose(*a, 0) == want, (rows_in, K, cin, cout, occ, umax)
 
 
 def test_a_stale_library_is_not_loaded(monkeypatch):
