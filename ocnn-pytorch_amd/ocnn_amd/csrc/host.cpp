@@ -746,14 +746,27 @@ Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); 
 
 PYBIND11_MODULE(ocnn_host, m) {
   namespace py = pybind11;
+  // (the constructors take what every plan and pass sets: one call instead of one for each field)
   py::class_<PlanArrays, std::shared_ptr<PlanArrays>>(m, "PlanArrays")
       .def(py::init<>())
+      .def(py::init([](Tensor loc, Tensor uptr, Tensor urows, int umax, int64_t total, double occupancy) {
+        auto p = std::make_shared<PlanArrays>();
+        p->loc = std::move(loc), p->uptr = std::move(uptr), p->urows = std::move(urows);
+        p->umax = umax, p->total = total, p->occupancy = occupancy;
+        return p;
+      }))
 #define FIELD(name) .def_readwrite(#name, &PlanArrays::name)
       FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(umax) FIELD(total) FIELD(occupancy) FIELD(cptr) FIELD(ent) FIELD(lists)
           FIELD(n_blocks) FIELD(max_blocks) FIELD(n_lists) FIELD(lists_host) FIELD(group_bounds) FIELD(list_count);
 #undef FIELD
   py::class_<GatherOp, std::shared_ptr<GatherOp>>(m, "GatherOp")
       .def(py::init<>())
+      .def(py::init([](int64_t rows_in, int64_t rows, int K, int cin, int cout, bool transposed, bool reverse) {
+        auto op = std::make_shared<GatherOp>();
+        op->rows_in = rows_in, op->rows = rows, op->K = K, op->cin = cin, op->cout = cout;
+        op->transposed = transposed, op->reverse = reverse;
+        return op;
+      }))
 #define FIELD(name) .def_readwrite(#name, &GatherOp::name)
       FIELD(kernel) FIELD(K) FIELD(cin) FIELD(cout) FIELD(rows_in) FIELD(rows) FIELD(ws_bytes) FIELD(transposed)
           FIELD(reverse) FIELD(plan) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
@@ -767,6 +780,11 @@ PYBIND11_MODULE(ocnn_host, m) {
       });
   py::class_<WgradOp, std::shared_ptr<WgradOp>>(m, "WgradOp")
       .def(py::init<>())
+      .def(py::init([](int64_t rows_x, int64_t rows, int K, int ca, int cb, bool out_transposed) {
+        auto op = std::make_shared<WgradOp>();
+        op->rows_x = rows_x, op->rows = rows, op->K = K, op->ca = ca, op->cb = cb, op->out_transposed = out_transposed;
+        return op;
+      }))
 #define FIELD(name) .def_readwrite(#name, &WgradOp::name)
       FIELD(kernel) FIELD(K) FIELD(ca) FIELD(cb) FIELD(rows_x) FIELD(rows) FIELD(ws_bytes) FIELD(out_transposed) FIELD(plan)
           FIELD(g_index) FIELD(shape) FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded)

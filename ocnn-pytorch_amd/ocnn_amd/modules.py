@@ -12,7 +12,7 @@ import torch.nn.functional as F
 from . import _lib
 from .nn import OctreeConv, OctreeDeconv
 from .nn.octree_conv import _gather_op, _wgrad_op, call_native, conv_wgrad, column_sum
-from .nn.batchnorm import BatchNormRelu1d
+from .nn.batchnorm import BatchNormRelu1d, kernels_take
 
 
 class _LayerBn(torch.nn.Module):
@@ -46,14 +46,20 @@ def layer_bn(layer, bn, data, *args, residual=None, relu=None):
   batch norm of this package as they are, one native call: the normalisation then rides on the
   convolution's own pass over its result instead of reading and writing it once more."""
   if (not torch.is_grad_enabled() and not _lib.recorded() and type(bn) is BatchNormRelu1d and not bn.training and
-      bn.running_mean is not None and type(layer) in (OctreeConv, OctreeDeconv, Conv1x1) and _plain(layer) and _plain(bn) and
+      type(layer) in (OctreeConv, OctreeDeconv, Conv1x1) and _plain(layer) and _plain(bn) and
       not (_nn._global_forward_hooks or _nn._global_forward_pre_hooks)):
-    native = layer.native_layer(data, *args)
-    if native is not None and _lib.lib().ocnn_batch_norm_supported(_lib.DTYPE_CODE[data.dtype], 2, bn.num_features):
-      linear = layer.linear if type(layer) is Conv1x1 else None
-      return _lib.native().conv_bn(native, data, layer.weights if linear is None else linear.weight,
-                                   layer.bias if linear is None else linear.bias, bn.running_mean, bn.running_var, bn.eps,
-                                   bn.weight, bn.bias, bn.fused_relu if relu is None else relu, residual)
+    # (the tensors out of the modules' own dictionaries: as attributes of a Module each costs a search in Python,
+    # a tenth of the host time of a small network; one that is not where the constructor put it: the general route)
+    stats, affine = bn._buffers, bn._parameters
+    if stats.get('running_mean') is not None and 'running_var' in stats and 'weight' in affine and 'bias' in affine:
+      native = layer.native_layer(data, *args)
+      if native is not None and kernels_take(data.dtype, bn.num_features):
+        own, name = (layer.linear, 'weight') if type(layer) is Conv1x1 else (layer, 'weights')
+        held = own._parameters
+        return _lib.native().conv_bn(native, data, held[name] if name in held else getattr(own, name),
+                                     held['bias'] if 'bias' in held else own.bias, stats['running_mean'],
+                                     stats['running_var'], bn.eps, affine['weight'], affine['bias'],
+                                     bn.fused_relu if relu is None else relu, residual)
   if residual is None and relu is None:
     return bn(layer(data, *args))
   return bn(layer(data, *args), residual=residual, relu=relu)
@@ -225,7 +231,8 @@ class OctreeResBlock2(torch.nn.Module):
     if self.in_channels != self.out_channels:
       data = self.conv1x1(data)
     # relu(bn(conv(out)) + data): the sum and the ReLU ride on the batch norm's pass
-    return layer_bn(self.conv3x3b.conv, self.conv3x3b.bn, out, octree, depth, residual=data, relu=True)
+    last = self.conv3x3b
+    return layer_bn(last.conv, last.bn, out, octree, depth, residual=data, relu=True)
 
 
 class OctreeResBlocks(torch.nn.Module):

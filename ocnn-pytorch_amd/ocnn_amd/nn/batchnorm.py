@@ -3,10 +3,19 @@ kernels (same parameters, buffers and state_dict keys as BatchNorm1d).  What the
 builds from BatchNorm1d + ReLU(inplace) after every convolution
 (ocnn/modules/modules.py:32-99, 120-153)."""
 
+import functools
+
 import torch
 import torch.nn
 
 from .. import _lib
+
+
+@functools.lru_cache(maxsize=256)
+def kernels_take(dtype, channels):
+  """The kernels take rows of these channels in this type, any number of them but none."""
+  code = _lib.DTYPE_CODE.get(dtype, -1)
+  return code >= 0 and bool(_lib.lib().ocnn_batch_norm_supported(code, 1, channels))
 
 
 class _BatchNormFunction(torch.autograd.Function):
@@ -40,9 +49,7 @@ class BatchNormRelu1d(torch.nn.BatchNorm1d):
     """residual: added to the normalised values before the ReLU (the tail of a residual
     block), in the same pass.  relu: overrides the module's setting for this call."""
     relu = self.fused_relu if relu is None else relu
-    code = _lib.DTYPE_CODE.get(input.dtype, -1)
-    if not (input.dim() == 2 and input.is_cuda and code >= 0 and input.shape[0] > 1 and
-            _lib.lib().ocnn_batch_norm_supported(code, input.shape[0], input.shape[1])):
+    if not (input.dim() == 2 and input.is_cuda and input.shape[0] > 1 and kernels_take(input.dtype, input.shape[1])):
       out = super().forward(input)
       if residual is not None:
         out = out + residual

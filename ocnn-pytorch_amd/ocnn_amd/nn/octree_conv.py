@@ -81,9 +81,7 @@ def _plan_arrays(plan, pairs):
   name = '_native_pairs' if pairs else '_native'
   arrays = plan.__dict__.get(name)
   if arrays is None:
-    arrays = _lib.native().PlanArrays()
-    arrays.loc, arrays.uptr, arrays.urows = plan.loc, plan.uptr, plan.urows
-    arrays.umax, arrays.total, arrays.occupancy = plan.umax, plan.total, float(plan.occupancy)
+    arrays = _lib.native().PlanArrays(plan.loc, plan.uptr, plan.urows, plan.umax, plan.total, float(plan.occupancy))
     if pairs:
       pp = plan.pairs()
       arrays.cptr, arrays.ent, arrays.lists = pp.cptr, pp.ent, pp.lists
@@ -112,8 +110,7 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
   if op is not None:
     return op
   L, code = _lib.lib(), _lib.dtype_code_of(dtype)
-  op = _lib.native().GatherOp()
-  op.rows_in, op.rows, op.K, op.cin, op.cout, op.transposed, op.reverse = rows_in, rows, K, cin, cout, transposed, reverse
+  op = _lib.native().GatherOp(rows_in, rows, K, cin, cout, transposed, reverse)
   op.kernel = L.ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan),
                                     int(plan is not None and plan.overflow_rows is not None))
   if op.kernel == _lib.GATHER_ZERO_PADDED:
@@ -189,8 +186,7 @@ def _wgrad_op(dtype, rows_x, rows, K, ca, cb, out_transposed, plan=None, dense=F
   if op is not None:
     return op
   L, code = _lib.lib(), _lib.dtype_code_of(dtype)
-  op = _lib.native().WgradOp()
-  op.rows_x, op.rows, op.K, op.ca, op.cb, op.out_transposed = rows_x, rows, K, ca, cb, out_transposed
+  op = _lib.native().WgradOp(rows_x, rows, K, ca, cb, out_transposed)
   op.kernel = L.ocnn_conv_wgrad_choose(code, rows_x, rows, K, ca, cb, int(dense), *_plan_args(plan)[:4])
   if op.kernel == _lib.WGRAD_ZERO_PADDED:
     op.padded = _wgrad_op(dtype, rows_x, rows, K, -(-ca // 32) * 32, -(-cb // 32) * 32, out_transposed, plan)

@@ -6,6 +6,7 @@ import torch
 
 from ocnn_amd import synthetic
 from ocnn_amd.modules import Conv1x1, Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
+from ocnn_amd.nn import OctreeConv
 from ocnn_amd.octree import Octree, Points
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +78,30 @@ def test_residual_block(dtype, cin, cout):
       block(x, octree, 6)
     del part.forward
   assert seen == [1, 2, 2]
+
+
+@pytest.mark.parametrize('part,names', [('conv', ['weights']), ('conv', ['bias']), ('bn', ['weight', 'bias']),
+                                        ('bn', ['running_mean', 'running_var'])])
+def test_tensors_held_as_plain_attributes(part, names):
+  """Parameters and buffers replaced by plain attributes of the module (as libraries that reparametrise
+  modules leave them) are the ones that are used: the same values, and then others."""
+  octree = _octree()
+  block = _randomise(OctreeConvBnRelu(32, 64, nempty=True), torch.float16)
+  if names == ['bias']:
+    block.conv = OctreeConv(32, 64, nempty=True, use_bias=True).to('cuda', torch.float16).eval()
+    torch.nn.init.uniform_(block.conv.bias)
+  x = torch.randn(int(octree.nnum_nempty[5]), 32, generator=torch.Generator().manual_seed(1)).to('cuda', torch.float16)
+  module = getattr(block, part)
+  with torch.no_grad():
+    want = block(x, octree, 5)
+    held = [getattr(module, n).detach().clone() for n in names]
+    for n, t in zip(names, held):
+      delattr(module, n)
+      setattr(module, n, t)
+    # (one pass or two: six roundings of the result apart, as in the tests above)
+    assert (block(x, octree, 5).double() - want.double()).abs().max() <= TOL[torch.float16] * want.double().abs().max()
+    held[0].mul_(2)
+    assert not torch.equal(block(x, octree, 5), want)
 
 
 def test_linear_layers_keep_one_table():
