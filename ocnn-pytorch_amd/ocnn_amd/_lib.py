@@ -129,6 +129,7 @@ INTERNAL_SIGNATURES = {
     'ocnnx_gather_choose': (_i, [_i, _l, _l, _i, _i, _i, _i, _i, _i, _l, _d, _d, _i]),
     'ocnnx_conv_gather_workspace_bytes': (_l, [_i, _l, _l, _i, _i, _i]),
     'ocnnx_conv_gather': (_i, [_i, _p, _l, _p, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _p, _l, _p]),
+    'ocnnx_dense_rows_supported': (_i, [_i, _l, _i, _i]),
     'ocnnx_gather_tile_supported': (_i, [_i, _l, _i, _i, _i, _i]),
     'ocnnx_gather_tile_workspace_bytes': (_l, [_i, _l, _i, _i, _i]),
     'ocnnx_gather_tile': (_i, [_i, _p, _l, _p, _p, _p, _i, _l, _d, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _p, _l, _i, _i, _p]),
@@ -211,10 +212,10 @@ def check(rc):
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
-# codes of ocnn_conv_gather_choose / ocnn_conv_wgrad_choose (include/ocnn_hip.h); TILE: of
+# codes of ocnn_conv_gather_choose / ocnn_conv_wgrad_choose (include/ocnn_hip.h); TILE, ROWS: of
 # ocnnx_gather_choose only
 (GATHER_PLAIN, GATHER_DENSE_RW, GATHER_DENSE, GATHER_RW, GATHER_SPARSE, GATHER_WIDE, GATHER_PLANNED,
- GATHER_ZERO_PADDED, GATHER_TILE) = range(9)
+ GATHER_ZERO_PADDED, GATHER_TILE, GATHER_ROWS) = range(10)
 WGRAD_PLAIN, WGRAD_DENSE_RW, WGRAD_SPARSE, WGRAD_PLANNED, WGRAD_ZERO_PADDED = range(5)
 
 

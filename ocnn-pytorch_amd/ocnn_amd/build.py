@@ -27,6 +27,7 @@ SOURCES = {
     'conv_tile.hip': [],
     'jobs.hip': [],
     'conv_dense.hip': [],
+    'dense_rows.hip': [],
     'conv_sparse.hip': [],
     'wgrad_sparse.hip': [],
     'dense_rw.hip': [],

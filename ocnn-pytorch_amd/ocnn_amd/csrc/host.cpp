@@ -117,6 +117,11 @@ struct GatherOp {
         check(ocnn_conv_dense(code, ptr(data), rows, ptr(W), cin, cout, transposed, ptr(bias), out.data_ptr(),
                               ws.data_ptr(), ws.numel(), st));
         break;
+      case OCNNX_GATHER_ROWS:
+        TORCH_CHECK(data.numel() == rows * cin, "conv_gather: the rows do not match");
+        check(ocnnx_dense_rows(code, ptr(data), rows, ptr(W), cin, cout, transposed, ptr(bias), bn, out.data_ptr(), st));
+        bn = nullptr;
+        break;
       case OCNN_GATHER_RW:
         check(ocnn_conv_gather_rw(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
                                   typed<int32_t>(p->urows), p->umax, p->total, rows, K, ptr(W), cin, cout, transposed,

@@ -78,8 +78,14 @@ int ocnnx_conv_gather(int dtype, const void* in, int64_t rows_in, const int32_t*
                       const void* w, int cin, int cout, int w_transposed, int reverse_slots, const void* bias, void* out,
                       const int64_t* out_index, void* workspace, int64_t workspace_bytes, void* stream);
 
-// ocnn_conv_gather_choose with that kernel among the choices.
+// Dense rows (row i reads row i) of few channels in f16 / bf16: out = in W (+ bias, + the batch norm behind it).
+int ocnnx_dense_rows_supported(int dtype, int64_t rows, int cin, int cout);
+int ocnnx_dense_rows(int dtype, const void* in, int64_t rows, const void* w, int cin, int cout, int w_transposed,
+                     const void* bias, const ocnnx_bn* bn, void* out, void* stream);
+
+// ocnn_conv_gather_choose with ocnnx_gather_tile and ocnnx_dense_rows among the choices.
 #define OCNNX_GATHER_TILE 8
+#define OCNNX_GATHER_ROWS 9
 int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int cin, int cout, int identity_table,
                         int has_plan, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
                         double plan_reuse, int plan_overflow);

@@ -121,6 +121,7 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
                    L.ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout) if op.kernel == _lib.GATHER_TILE else
                    L.ocnnx_conv_gather_workspace_bytes(code, rows_in, rows, K, cin, cout)
                    if op.kernel == _lib.GATHER_PLAIN else
+                   0 if op.kernel == _lib.GATHER_ROWS else
                    L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
     if op.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE, _lib.GATHER_SPARSE, _lib.GATHER_PLANNED):
       op.plan = _plan_arrays(plan, sparse)

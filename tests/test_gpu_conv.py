@@ -1991,3 +1991,32 @@ def test_plan_free_gather_in_parts_and_through_an_index(dtype, rows, K, cin, cou
       got = (out if idx is None else out[idx]).double()
       assert (got - want).abs().max() / want.abs().max() < {torch.float32: 2e-5, torch.float16: 2e-3, torch.bfloat16: 1e-2}[dtype]
       assert int(out.isnan().sum()) == (0 if idx is None else 2 * rows * cout)
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('rows,cin,cout', [(1, 32, 32), (31, 96, 64), (32, 64, 96), (129, 128, 96), (4133, 192, 64),
+                                           (70001, 32, 256), (2000, 64, 192), (33, 96, 128)])
+def test_dense_rows_of_few_channels(dtype, rows, cin, cout):
+  """The one-slot identity on the kernel for few channels (a block of 32 rows a wave): rows that end inside a block,
+  both orders of the weights, weights and bias away from 16-byte boundaries, against float64."""
+  import importlib
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(rows + cin)
+  x = torch.randn(rows, cin, generator=g).to('cuda', dtype)
+  table = torch.arange(rows, dtype=torch.int32, device='cuda').view(-1, 1)
+  for transposed in (False, True):
+    store = torch.randn(cin * cout + 1, generator=g).to('cuda', dtype)
+    for w in (store[:-1], store[1:]):
+      for bias in (None, torch.randn(cout + 1, generator=g).to('cuda', dtype)[1:]):
+        print(dtype, rows, cin, cout, transposed, w.storage_offset(), bias is None, flush=True)
+        op = OC._gather_op(dtype, rows, rows, 1, cin, cout, transposed, False, None, True)
+        assert op.kernel == _lib.GATHER_ROWS
+        out = op.run(x, table, w.view(1, cout, cin) if transposed else w.view(1, cin, cout), bias).double()
+        m = w.view(cout, cin).t().double() if transposed else w.view(cin, cout).double()
+        want = x.double() @ m
+        scale = x.double().abs() @ m.abs()
+        if bias is not None:
+          want, scale = want + bias.double(), scale + bias.double().abs()
+        # cin + 1 additions in fp32, one rounding to the type
+        bound = (cin + 1) * 2.0 ** -24 * scale + torch.finfo(dtype).eps / 2 * want.abs() * (1 + 2.0 ** -8) + 1e-7
+        assert ((out - want).abs() <= bound).all()
