@@ -184,14 +184,15 @@ __global__ __launch_bounds__(256, 1) void conv_dense_rw_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
     // a lane holds the output channels 8 q .. 8 q + 7 and 16 + 8 q .. of a row per M tile: the
-    // two lanes of a row write 32 contiguous bytes per store
+    // two lanes of a row write 32 contiguous bytes per store, and all that the wave has of the row one store behind
+    // the other (with the rows inside the M tiles, 64 -> 512 on 960 k rows took 261 us, so 243; 128 -> 512 266 and 257)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int cl = 32 * (wave * MB + mb) + 8 * q;               // channel within the workgroup's block
-      const f32x4* b4 = (const f32x4*)(&s_bias[cl]);
-      const f32x4 bv[4] = {b4[0], b4[1], b4[4], b4[5]};
+    for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
+      for (int mb = 0; mb < MB; ++mb) {
+        const int cl = 32 * (wave * MB + mb) + 8 * q;             // channel within the workgroup's block
+        const f32x4* b4 = (const f32x4*)(&s_bias[cl]);
+        const f32x4 bv[4] = {b4[0], b4[1], b4[4], b4[5]};
         const int64_t row = tile * RT + 32 * rb + r32;
         // (with an index, rows past the end have no entry: out of range, dropped like the others)
         const uint32_t orow = scattered ? (uint32_t)oq[U].r[rb] : (uint32_t)row;

@@ -83,7 +83,9 @@ extern "C" int ocnn_conv_gather_choose(int dtype, int64_t rows_in, int64_t rows_
 // points, eleven widths): all plan-free 80.1 ms, all on the tile kernel 74.1, by this rule 70.0, the faster of the
 // two each time 69.3.  Other fp32 layers gain on every table, 1.04 - 9 x: plan-free reads three copies of their rows.
 // Dense rows of few channels run on the kernel of dense_rows.hip at every number of rows: over ten pairs of channels
-// its time is 0.76 of the plan-free kernel's on 1.13 M rows, 0.71 on 300 k, 0.68 on 60 k, 0.63 on 16 k, 0.60 on 4096.
+// its time is 0.76 of the plan-free kernel's on 1.13 M rows, 0.71 on 300 k, 0.68 on 60 k, 0.63 on 16 k, 0.60 on 4096; in
+// the place of the dense kernel 64 -> 128 takes 75 us for 93 on 960 k rows, 64 -> 256 117 / 140, 128 -> 128 94 / 105, all
+// three 17 - 28 / 19 - 29 on 240 k (128 -> 128 25.2 / 24.7) and 5 - 11 / 8 - 11 below.  (With an index of the rows: that one.)
 constexpr double kTileMinProducts = 3.0e9;
 constexpr double kTileMinProductsApart = 1.7e10;
 constexpr double kTileMinOccupancy = 0.06, kTileMinOccupancyInverse = 0.12;        // of 27 slots
@@ -93,7 +95,7 @@ extern "C" int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out,
                                    double plan_occupancy, double plan_reuse, int plan_overflow) {
   const int pick = ocnn_conv_gather_choose(dtype, rows_in, rows_out, K, cin, cout, identity_table, has_plan,
                                            plan_max_distinct, plan_total, plan_occupancy, plan_reuse);
-  if (identity_table && K == 1 && rows_out == rows_in && pick == OCNN_GATHER_PLAIN &&
+  if (identity_table && K == 1 && rows_out == rows_in && (pick == OCNN_GATHER_PLAIN || pick == OCNN_GATHER_DENSE_RW) &&
       ocnnx_dense_rows_supported(dtype, rows_out, cin, cout))
     return OCNNX_GATHER_ROWS;
   if (!has_plan || !rows_ok(rows_out, plan_total) ||

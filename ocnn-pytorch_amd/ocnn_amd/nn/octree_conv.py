@@ -140,10 +140,12 @@ def _indexed_gather_op(dtype, rows, data_rows, cin, cout, transposed, in_index=N
   L = _lib.lib()
   base = _gather_op(dtype, rows, rows, 1, cin, cout, transposed, False, None, True)
   n_out = rows if pad_to is None else int(pad_to[0].nnum[pad_to[1]])
-  if base.kernel != _lib.GATHER_DENSE_RW or \
-      not L.ocnn_conv_dense_rw_supported(_lib.dtype_code_of(dtype), max(data_rows, n_out), cin, cout):
+  code = _lib.dtype_code_of(dtype)
+  if base.kernel not in (_lib.GATHER_DENSE_RW, _lib.GATHER_ROWS) or \
+      not L.ocnn_conv_dense_rw_supported(code, max(data_rows, n_out), cin, cout):
     return None
   op = base.copy()
+  op.kernel, op.ws_bytes = _lib.GATHER_DENSE_RW, L.ocnn_conv_gather_workspace_bytes(code, rows, 1, cin, cout)
   if in_index is not None:
     op.in_index = in_index
   if pad_to is not None:

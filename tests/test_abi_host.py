@@ -358,17 +358,18 @@ def test_selection_of_the_tile_kernel_over_the_pair_plan():
 
 
 def test_selection_of_the_dense_rows_kernel():
-  """ocnnx_gather_choose on the one-slot identity: the kernel for few channels in the place of the plan-free one only."""
+  """ocnnx_gather_choose on the one-slot identity: the kernel for few channels in the place of the plan-free and the dense one."""
   L, (F32, F16, BF), PLAIN, ROWS = _lib.lib(), range(3), _lib.GATHER_PLAIN, _lib.GATHER_ROWS
   for dtype, rows, cin, cout, want in (
       (F16, 1, 128, 96, ROWS), (BF, 10 ** 6, 96, 128, ROWS), (F16, 20000, 64, 192, ROWS), (F16, 20000, 32, 256, ROWS),
       (F32, 20000, 64, 64, PLAIN), (F16, 20000, 192, 96, PLAIN), (F16, 20000, 256, 64, PLAIN), (F16, 20000, 160, 64, PLAIN),
       (F16, 20000, 64, 48, PLAIN), (F16, 1 << 26, 32, 32, PLAIN),        # more bytes than a 32-bit offset reaches
-      (F16, 20000, 128, 128, _lib.GATHER_DENSE_RW), (F16, 20000, 40, 64, _lib.GATHER_ZERO_PADDED)):
+      (F16, 20000, 128, 128, ROWS), (BF, 300, 64, 256, ROWS), (F16, 20000, 256, 128, _lib.GATHER_DENSE_RW),
+      (F16, 20000, 40, 64, _lib.GATHER_ZERO_PADDED)):
     a = (dtype, rows, rows, 1, cin, cout, 1, 0, 0, 0, 1.0, 0.0)
     assert L.ocnnx_gather_choose(*a, 0) == want, (dtype, rows, cin, cout)
     public = L.ocnn_conv_gather_choose(*a)
-    assert public == (PLAIN if want == ROWS else want)
+    assert public == want or (want == ROWS and public in (PLAIN, _lib.GATHER_DENSE_RW))
     assert L.ocnnx_gather_choose(dtype, rows, rows, 1, cin, cout, 0, *a[7:], 0) != ROWS      # a table, not the identity
   assert L.ocnnx_gather_choose(F16, 500, 400, 1, 64, 64, 1, 0, 0, 0, 1.0, 0.0, 0) == PLAIN
 

@@ -1995,7 +1995,7 @@ def test_plan_free_gather_in_parts_and_through_an_index(dtype, rows, K, cin, cou
 
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('rows,cin,cout', [(1, 32, 32), (31, 96, 64), (32, 64, 96), (129, 128, 96), (4133, 192, 64),
-                                           (70001, 32, 256), (2000, 64, 192), (33, 96, 128)])
+                                           (70001, 32, 256), (2000, 64, 192), (33, 96, 128), (5000, 128, 128)])
 def test_dense_rows_of_few_channels(dtype, rows, cin, cout):
   """The one-slot identity on the kernel for few channels (a block of 32 rows a wave): rows that end inside a block,
   both orders of the weights, weights and bias away from 16-byte boundaries, against float64."""
