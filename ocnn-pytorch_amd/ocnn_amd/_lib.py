@@ -129,6 +129,9 @@ INTERNAL_SIGNATURES = {
     'ocnnx_gather_choose': (_i, [_i, _l, _l, _i, _i, _i, _i, _i, _i, _l, _d, _d, _i]),
     'ocnnx_conv_gather_workspace_bytes': (_l, [_i, _l, _l, _i, _i, _i]),
     'ocnnx_conv_gather': (_i, [_i, _p, _l, _p, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _p, _l, _p]),
+    'ocnnx_rows_wgrad_supported': (_i, [_i, _l, _i, _i]),
+    'ocnnx_rows_wgrad_workspace_bytes': (_l, [_l, _i, _i]),
+    'ocnnx_rows_wgrad': (_i, [_i, _p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),
     'ocnnx_dense_rows_supported': (_i, [_i, _l, _i, _i]),
     'ocnnx_gather_tile_supported': (_i, [_i, _l, _i, _i, _i, _i]),
     'ocnnx_gather_tile_workspace_bytes': (_l, [_i, _l, _i, _i, _i]),
@@ -182,6 +185,11 @@ def recorded():
   inside, that is an empty tensor.  Forward-mode differentiation and the transforms of torch.func are refused
   by a Function that does not provide for them; a native call would drop the tangents."""
   return _is_tracing() or _forward_ad._current_level >= 0 or _transforms_active()
+
+
+def only_traced():
+  """What looks on is torch.jit.trace and nothing else."""
+  return _is_tracing() and _forward_ad._current_level < 0 and not _transforms_active()
 
 
 def unrecorded(make, *args):

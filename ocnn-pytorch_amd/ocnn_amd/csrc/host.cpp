@@ -307,6 +307,23 @@ Tensor column_sum(Tensor g) {
   return out;
 }
 
+// g^T x of fp32 rows (ocnnx_rows_wgrad)
+Tensor rows_wgrad(Tensor g, Tensor x) {
+  require_gpu(g);
+  require_gpu(x);
+  TORCH_CHECK(g.dim() == 2 && x.dim() == 2 && g.size(0) == x.size(0) && g.scalar_type() == at::kFloat &&
+                  x.scalar_type() == at::kFloat && g.device() == x.device(),
+              "rows_wgrad: two fp32 matrices of as many rows");
+  g = g.contiguous();
+  x = x.contiguous();
+  const int ca = (int)g.size(1), cb = (int)x.size(1);
+  Tensor out = at::empty({ca, cb}, x.options());
+  Tensor ws = workspace(ocnnx_rows_wgrad_workspace_bytes(x.size(0), ca, cb), x);
+  check(ocnnx_rows_wgrad(OCNN_F32, ptr(g), ptr(x), x.size(0), ca, cb, 0, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                         hip_stream()));
+  return out;
+}
+
 // The passes of one layer on one octree, in one data type.  fwd: data -> out; dgrad: grad -> data
 // gradient; wgrad over (data, grad), for a deconvolution over (grad, data).  The backward passes are
 // made when a call first needs them, as a copy with the pass: threads share the object.
@@ -858,6 +875,13 @@ PYBIND11_MODULE(ocnn_host, m) {
   m.def("conv", &conv, py::call_guard<py::gil_scoped_release>());
   m.def("conv_bn", &conv_bn, py::call_guard<py::gil_scoped_release>());
   m.def("column_sum", &column_sum, py::call_guard<py::gil_scoped_release>());
+  m.def(
+      "rows_wgrad",
+      [](const Tensor& g, const Tensor& x) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return rows_wgrad(g, x);
+      },
+      py::call_guard<py::gil_scoped_release>());
   // (the two passes without an autograd node, for an autograd.Function around them)
   m.def(
       "batch_norm_pass",

@@ -83,6 +83,12 @@ int ocnnx_dense_rows_supported(int dtype, int64_t rows, int cin, int cout);
 int ocnnx_dense_rows(int dtype, const void* in, int64_t rows, const void* w, int cin, int cout, int w_transposed,
                      const void* bias, const ocnnx_bn* bn, void* out, void* stream);
 
+// gw = x^T g of fp32 rows, in fp32 throughout (fixed order); any channel counts up to 1024.
+int ocnnx_rows_wgrad_supported(int dtype, int64_t rows, int ca, int cb);
+int64_t ocnnx_rows_wgrad_workspace_bytes(int64_t rows, int ca, int cb);
+int ocnnx_rows_wgrad(int dtype, const void* x, const void* g, int64_t rows, int ca, int cb, int out_transposed, void* gw,
+                     void* workspace, int64_t workspace_bytes, void* stream);
+
 // ocnn_conv_gather_choose with ocnnx_gather_tile and ocnnx_dense_rows among the choices.
 #define OCNNX_GATHER_TILE 8
 #define OCNNX_GATHER_ROWS 9

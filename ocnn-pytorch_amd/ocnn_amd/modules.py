@@ -170,9 +170,64 @@ class _RowsLinearNarrow(torch.autograd.Function):
     return gx, gw, gb
 
 
+class _RowsWgrad(torch.autograd.Function):
+  """g^T x of fp32 rows, every product and sum in fp32 (ocnnx_rows_wgrad), and differentiable again."""
+
+  @staticmethod
+  def forward(ctx, g, x):
+    ctx.save_for_backward(g, x)
+    return _lib.native().rows_wgrad(g, x)
+
+  @staticmethod
+  def backward(ctx, grad):
+    g, x = ctx.saved_tensors
+    return (x @ grad.t() if ctx.needs_input_grad[0] else None, g @ grad if ctx.needs_input_grad[1] else None)
+
+
+class _RowsLinear32(torch.autograd.Function):
+  """torch.nn.functional.linear on many fp32 rows, with the weight gradient on this package's kernel: a sum over all
+  rows into a small matrix, for which the library runs a handful of workgroups (us, library / kernel, with a norm of
+  the error of 1 - 10e-6 / 0.2 - 1e-6: 31 k rows of 96 -> 64 104 / 16, 192 -> 128 84 / 25, 384 -> 256 112 / 65, 512 -> 512
+  180 / 148; 300 k rows 626 / 62, 634 / 171, 752 / 554, 1585 / 1381; 4096 rows 24 - 33 / 10 - 12, 512 -> 512 28 / 30)."""
+
+  @staticmethod
+  def forward(ctx, x, weight, bias):
+    ctx.save_for_backward(x, weight)
+    return F.linear(x, weight, bias)
+
+  @staticmethod
+  def backward(ctx, grad):
+    x, weight = ctx.saved_tensors
+    needs = ctx.needs_input_grad
+    wgrad = _RowsWgrad.apply if torch.is_grad_enabled() else _lib.native().rows_wgrad
+    return grad @ weight if needs[0] else None, wgrad(grad, x) if needs[1] else None, grad.sum(0) if needs[2] else None
+
+
+def _takes_rows32(data, lin):
+  """The fp32 weight gradient of `lin` on `data` can run on this package's kernel: plain tensors of many rows, no hook
+  that would miss the Linear, no data type chosen by autocast.  A trace keeps the Linear, which can be saved with it,
+  unless the module is in training."""
+  weight, bias = lin.weight, lin.bias
+  if not (torch.is_grad_enabled() and data.dim() == 2 and data.is_cuda and data.dtype == torch.float32 and
+          weight.requires_grad and type(data) is torch.Tensor and type(weight) is torch.nn.Parameter and
+          weight.dtype == torch.float32 and weight.device == data.device and
+          (bias is None or (bias.dtype == torch.float32 and bias.device == data.device))):
+    return False
+  rows, (cout, cin) = int(data.shape[0]), map(int, weight.shape)
+  if not (rows >= 4096 and cin == data.shape[1] and cin % 4 == 0 and max(cin, cout) <= 512 and
+          _lib.lib().ocnnx_rows_wgrad_supported(0, rows, cout, cin)):
+    return False
+  if not (type(lin) is torch.nn.Linear and _plain(lin)) or lin._backward_hooks or lin._backward_pre_hooks or \
+      _nn._global_forward_hooks or _nn._global_forward_pre_hooks or _nn._global_backward_hooks or \
+      _nn._global_backward_pre_hooks or torch.is_autocast_enabled() or torch.compiler.is_compiling():
+    return False
+  return not _lib.recorded() or (lin.training and _lib.only_traced())
+
+
 class Conv1x1(torch.nn.Module):
   """ocnn/modules/modules.py:102-117: a 1x1x1 convolution on (N, C) rows is a Linear (same
-  parameters as torch.nn.Linear; large 16-bit inputs run on this package's GEMM kernels)."""
+  parameters as torch.nn.Linear; large 16-bit inputs run on this package's GEMM kernels, and so does the
+  weight gradient of large fp32 ones)."""
 
   def __init__(self, in_channels: int, out_channels: int, use_bias: bool = False):
     super().__init__()
@@ -194,6 +249,8 @@ class Conv1x1(torch.nn.Module):
     if (data.dim() == 2 and data.is_cuda and data.dtype in (torch.float16, torch.bfloat16) and
         data.shape[0] >= 65536 and lin.in_features % 32 == 0 and lin.out_features < 16):
       return _RowsLinearNarrow.apply(data, lin.weight, lin.bias)
+    if _takes_rows32(data, lin):
+      return _RowsLinear32.apply(data, lin.weight, lin.bias)
     return lin(data)
 
 

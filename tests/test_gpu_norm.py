@@ -390,3 +390,45 @@ def test_batch_norm_few_rows(dtype):
         assert torch.equal(rg.grad.cpu(), d.to(dtype))
       again = bn(x.to(DEV), residual=res.to(DEV) if residual else None, relu=True)
       assert torch.equal(again, y)
+
+
+@pytest.mark.parametrize('rows,cin,cout,bias', [(4096, 32, 13, True), (4099, 96, 64, False), (5000, 64, 1, True),
+                                                (20011, 100, 160, True), (4100, 512, 512, False), (70000, 4, 32, True)])
+def test_conv1x1_fp32_weight_gradient(rows, cin, cout, bias, tmp_path):
+  """modules.Conv1x1 on many fp32 rows: output and gradients of torch.nn.Linear (the weight gradient within the bound
+  of an fp32 sum in any order against float64), the second derivative, and the Linear itself where somebody looks on."""
+  from ocnn_amd import modules
+  g = torch.Generator().manual_seed(rows)
+  m = modules.Conv1x1(cin, cout, use_bias=bias).to(DEV)
+  x = torch.randn(rows, cin, generator=g).to(DEV).requires_grad_()
+  dy = torch.randn(rows, cout, generator=g).to(DEV)
+  y, want = m(x), m.linear(x)
+  assert 'RowsLinear32' in type(y.grad_fn).__name__ and torch.equal(y, want)
+  params = [x] + list(m.parameters())
+  got, ref = torch.autograd.grad(y, params, dy), torch.autograd.grad(want, params, dy)
+  assert torch.equal(got[0], ref[0]) and (not bias or torch.equal(got[2], ref[2]))
+  xd, gd = x.detach().double(), dy.double()
+  assert ((got[1].double() - gd.t() @ xd).abs() <= 2.0 ** -24 * rows ** 0.5 * 8 * (gd.t().abs() @ xd.abs()) / rows ** 0.5).all()
+  again = torch.autograd.grad(m(x), params, dy)
+  assert torch.equal(again[1], got[1])                     # a fixed order
+  # the weight gradient differentiated once more, as the Linear's is
+  v = torch.randn(cout, cin, generator=g).to(DEV)
+  dy.requires_grad_()
+  second = [torch.autograd.grad((torch.autograd.grad(layer(x), m.linear.weight, dy, create_graph=True)[0] * v).sum(), (x, dy))
+            for layer in (m, m.linear)]
+  for a, b in zip(*second):
+    assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+  # the Linear where it would be missed
+  seen = []
+  handle = m.linear.register_forward_hook(lambda *a: seen.append(1))
+  m(x)
+  handle.remove()
+  assert seen == [1]
+  with torch.autocast('cuda', torch.bfloat16):
+    assert m(x).dtype == torch.bfloat16
+  jvp = torch.func.jvp(m, (x.detach(),), (x.detach(),))[1]
+  assert (jvp - x.detach() @ m.linear.weight.t()).abs().max() <= 1e-5 * jvp.abs().max()
+  torch.jit.trace(m.eval(), (x,), check_trace=False).save(str(tmp_path / 'm.pt'))
+  for other in (x[:4095], x.detach().double()):
+    layer = m if other.dtype == torch.float32 else m.double()
+    assert 'RowsLinear' not in type(layer(other).grad_fn).__name__
