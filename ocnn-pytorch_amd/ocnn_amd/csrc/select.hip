@@ -6,6 +6,8 @@
 // Every *_supported() predicate says whether a kernel takes a shape class; the row ranges that
 // its entry point checks on top (32-bit buffer offsets of the output, of the table, of the
 // plan) are repeated here, so a choice is always one that the chosen entry point accepts.
+#include <algorithm>
+
 #include "common.hpp"
 #include "host_api.hpp"
 
@@ -131,11 +133,20 @@ extern "C" int ocnn_conv_wgrad_choose(int dtype, int64_t rows_x, int64_t rows, i
     // (32 x 32 and 64 x 64 have planned kernels of their own that are faster still; with channel
     // counts that are not multiples of 64 on the table-row side the pair-plan kernel, which sums
     // exactly ca x cb and only over the pairs, beats zero-padded 64 x 64 blocks on dense tables too)
+    // (32 channels on one side: the planned kernel, whose 64 x 64 blocks are half empty, beats the pair plan on tables of
+    // fewer than 27 slots and, with whole blocks on the other side, on dense ones of 27; us, f16, pair plan / planned:
+    // nine slots, 1.13 M rows 16 % set, 32 -> 64 290 / 86, 96 -> 32 253 / 166; eight, 947 k rows 15 % set, 112 / 60, 151 / 110;
+    // 27, 1.06 M rows 61 % set, 64 -> 32 228 / 197, 128 -> 32 420 / 406, but 96 -> 32 338 / 384, 32 -> 96 213 / 385)
+    const bool narrow = ca != cb && std::min(ca, cb) == 32;
+    const bool planned = narrow && (K < 27 || (plan_occupancy > kSparseMaxOccupancy && std::max(ca, cb) % 64 == 0));
     if ((plan_occupancy <= kSparseMaxOccupancy || cb % 64 != 0) && rows >= kSparseMinRows &&
-        !(ca == cb && (ca == 32 || ca == 64)) &&
+        !(ca == cb && (ca == 32 || ca == 64)) && !planned &&
         ocnn_conv_wgrad_sparse_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_SPARSE;
-    if (ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
+    // (half-empty blocks against the plan-free kernel, us: f16 32 -> 64 on 1.06 M rows 61 % set 201 / 775, 159 k 38 % set
+    // 44 / 106, 41 k 27 / 31, but 20 k 22 / 19 and 10 k 18 / 16; fp32 696 / 2451, 113 / 330, 42 / 94, 33 / 55, 30 / 47)
+    if (!(narrow && dtype != OCNN_F32 && rows < kSparseMinRows) &&
+        ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_PLANNED;
   }
   return OCNN_WGRAD_PLAIN;

@@ -1,4 +1,4 @@
-// Weight gradient for 32 x 32 channels and for multiples of 64 channels (in 64 x 64 blocks)
+// Weight gradient for 32 x 32 channels and, in 64 x 64 blocks, for all other multiples of 32 channels,
 // on the tile plan of the neighbour table.
 //
 //   dW[k][a][b] = sum over table rows r of  x[table[r][k]][a] * g[r][b]
@@ -390,10 +390,13 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 using namespace ocnn;
 
 
+// 64 x 64 blocks (half of one beyond the channels), but for the 32 x 32 layer
+static bool wp_wide(int ca, int cb) { return ca > 32 || cb > 32; }
+
 // workgroups of one range of tiles (and one product of bf16 pieces): the slot groups, the blocks of channel pairs
 static int wp_range_workgroups(int K, int ca, int cb) {
-  const int groups = (K == 27 && ca >= 64) ? 2 : 1;
-  return groups * (ca >= 64 ? ((ca + 63) / 64) * ((cb + 63) / 64) : 1);
+  const int groups = (K == 27 && wp_wide(ca, cb)) ? 2 : 1;
+  return groups * (wp_wide(ca, cb) ? ((ca + 63) / 64) * ((cb + 63) / 64) : 1);
 }
 
 // ranges of tiles at most: as many as keep a workgroup on every CU (the LDS holds one)
@@ -437,7 +440,7 @@ static int wp_cu_count() {
 extern "C" int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int64_t rows, int K, int ca,
                                                  int cb, int plan_max_distinct) {
   if (dtype != OCNN_F16 && dtype != OCNN_BF16 && dtype != OCNN_F32) return 0;   // (fp32: as bf16 pieces)
-  if (!(ca == 32 && cb == 32) && !(ca >= 64 && cb >= 64 && ca % 32 == 0 && cb % 32 == 0 && ca <= 1024 && cb <= 1024))
+  if (ca < 32 || cb < 32 || ca % 32 != 0 || cb % 32 != 0 || ca > 1024 || cb > 1024)
     return 0;
   if (K != 27 && K != 9 && K != 8 && K != 3) return 0;
   if (plan_max_distinct < 0 || plan_max_distinct > kWpCap) return 0;
@@ -493,7 +496,7 @@ static void launch_wp(const WpArgs& a, hipStream_t st) {
 template <typename T>
 static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
 #define OCNN_WP_LAUNCH(CC, KK, NF, NH, GR) launch_wp<T, CC, KK, NF, NH, GR>(a, st)
-  if (a.ca >= 64) {
+  if (wp_wide(a.ca, a.cb)) {
     if (a.K == 27) OCNN_WP_LAUNCH(64, 27, 3, 1, 2);
     else if (a.K == 9) OCNN_WP_LAUNCH(64, 9, 2, 1, 1);
     else if (a.K == 8) OCNN_WP_LAUNCH(64, 8, 2, 0, 1);

@@ -114,7 +114,15 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
   op.kernel = L.ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan),
                                     int(plan is not None and plan.overflow_rows is not None))
   if op.kernel == _lib.GATHER_ZERO_PADDED:
-    op.padded = _gather_op(dtype, rows_in, rows, K, -(-cin // 32) * 32, -(-cout // 16) * 16, transposed, reverse, plan)
+    # (to 32 channels where a kernel on the plan then takes the layer, to 16 for the plan-free one: 64 -> 4 as 64 -> 32
+    # on the tile kernel / 64 -> 16 plan-free, us, f16 and fp32: 1.28 M rows 68 % set 210 / 379, 453 / 1380; 1.13 M rows 7 %
+    # set 119 / 225, 214 / 728; 41 k rows 17 / 19, 27 / 60)
+    wide = -(-cin // 32) * 32, -(-cout // 32) * 32
+    on_plan = plan is not None and L.ocnnx_gather_choose(
+        code, rows_in, rows, K, *wide, 0, *_plan_args(plan), int(plan.overflow_rows is not None)) in (_lib.GATHER_RW,
+                                                                                                  _lib.GATHER_TILE)
+    op.padded = _gather_op(dtype, rows_in, rows, K, wide[0], wide[1] if on_plan else -(-cout // 16) * 16, transposed, reverse,
+                           plan)
   else:
     sparse = op.kernel == _lib.GATHER_SPARSE
     op.ws_bytes = (L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout) if sparse else

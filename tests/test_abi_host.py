@@ -374,6 +374,19 @@ def test_selection_of_the_dense_rows_kernel():
   assert L.ocnnx_gather_choose(F16, 500, 400, 1, 64, 64, 1, 0, 0, 0, 1.0, 0.0, 0) == PLAIN
 
 
+def test_selection_of_the_weight_gradient_with_32_channels_on_one_side():
+  """ocnn_conv_wgrad_choose: both sides of each line of its rule for layers of 32 channels on one side only."""
+  L, (F32, F16) = _lib.lib(), (0, 1)
+  PLAIN, SPARSE, PLANNED = _lib.WGRAD_PLAIN, _lib.WGRAD_SPARSE, _lib.WGRAD_PLANNED
+  for dtype, rows, K, ca, cb, occ, want in (
+      (F16, 500000, 27, 32, 64, 0.3, SPARSE), (F16, 500000, 27, 32, 64, 0.31, PLANNED), (F16, 500000, 27, 64, 32, 0.31, PLANNED),
+      (F16, 500000, 27, 96, 32, 0.31, SPARSE), (F16, 500000, 27, 32, 96, 0.6, SPARSE), (F16, 500000, 27, 128, 32, 0.6, PLANNED),
+      (F16, 500000, 9, 96, 32, 0.1, PLANNED), (F16, 500000, 8, 32, 64, 0.1, PLANNED),
+      (F16, 32768, 27, 32, 64, 0.6, PLANNED), (F16, 32767, 27, 32, 64, 0.6, PLAIN), (F16, 32767, 27, 64, 64, 0.6, PLANNED),
+      (F32, 100, 27, 32, 64, 0.1, PLANNED), (F32, 500000, 27, 96, 32, 0.6, PLANNED), (F16, 500000, 27, 32, 32, 0.1, PLANNED)):
+    assert L.ocnn_conv_wgrad_choose(dtype, rows, rows, K, ca, cb, 0, 1, 300, 2 * rows, occ) == want, (dtype, rows, K, ca, cb, occ)
+
+
 def test_a_stale_library_is_not_loaded(monkeypatch):
   """The built libraries carry the hash of their sources; when a source changes, the loader
   builds again instead of loading the old binary."""

@@ -2020,3 +2020,79 @@ def test_dense_rows_of_few_channels(dtype, rows, cin, cout):
         # cin + 1 additions in fp32, one rounding to the type
         bound = (cin + 1) * 2.0 ** -24 * scale + torch.finfo(dtype).eps / 2 * want.abs() * (1 + 2.0 ** -8) + 1e-7
         assert ((out - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('K,ca,cb', [(27, 32, 64), (27, 64, 32), (27, 96, 32), (9, 32, 96), (8, 128, 32), (3, 32, 160)])
+def test_planned_wgrad_of_32_channels_on_one_side(dtype, K, ca, cb):
+  """Blocks of 64 x 64 pairs of which half lies beyond the channels: the rows of 32 channels are read past their ends
+  into sums that are not kept.  Non-finite values in the rows behind must not come back, and fp32 is no worse than
+  on the plan-free kernel."""
+  import importlib
+  from ocnn_amd.octree.octree import TilePlan
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(K + ca)
+  for rows, rows_in in [(129, 200), (128 * 40 + 5, 5000)]:
+    table = _local_table(rows, rows_in, K, g)
+    table[table == rows_in - 1] = -1                     # the last row of x belongs to nobody
+    tg = table.to(DEV)
+    plan = TilePlan(tg)
+    x = torch.randn(rows_in, ca, generator=g).to(dtype)
+    x[rows_in - 1] = float('inf')
+    gr = torch.randn(rows, cb, generator=g).to(dtype)
+    finite = x.clone()
+    finite[rows_in - 1] = 0
+    want = torch.from_numpy(C.weight_gemm(f64(finite), f64(gr), table.numpy().astype(np.int64)))
+    for transposed in (False, True):
+      op = OC._wgrad_op(dtype, rows_in, rows, K, ca, cb, transposed, plan).copy()
+      assert op.kernel == (_lib.WGRAD_PLANNED if dtype == torch.float32 else _lib.WGRAD_PLAIN)
+      op.kernel, op.plan = _lib.WGRAD_PLANNED, OC._plan_arrays(plan, False)
+      op.ws_bytes = _lib.lib().ocnn_conv_wgrad_planned_workspace_bytes_for(_lib.DTYPE_CODE[dtype], rows_in, rows, K, ca, cb)
+      say('wgrad 32', dtype, K, ca, cb, rows, transposed)
+      gw = op.run(x.to(DEV), gr.to(DEV), tg)
+      gw = gw.transpose(1, 2) if transposed else gw
+      err = rel_err(gw, want.numpy())
+      assert err < TOL[dtype]
+    if dtype == torch.float32:
+      plain = OC._wgrad_op(dtype, rows_in, rows, K, ca, cb, False)
+      assert plain.kernel == _lib.WGRAD_PLAIN
+      off = lambda t: float((t.double().cpu() - want).norm() / want.norm())
+      assert off(gw) <= 1.2 * off(plain.run(finite.to(DEV), gr.to(DEV), tg))
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('K,cin,cout', [(27, 64, 4), (27, 32, 10), (9, 96, 20), (27, 20, 33), (8, 64, 8)])
+def test_odd_output_channels_on_the_plan(dtype, K, cin, cout):
+  """Layers whose output channels are no multiple of 16, over a table with a plan: zero-padded to what the kernels on
+  the plan take, or to 16 for the plan-free one; both orders of the weights, with a bias, against float64."""
+  import importlib
+  from ocnn_amd.octree.octree import TilePlan
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(K + cin)
+  rows = rows_in = 128 * 130 + 3
+  table = _local_table(rows, rows_in, K, g)
+  tg = table.to(DEV)
+  plan = TilePlan(tg)
+  x = torch.randn(rows_in, cin, generator=g).to(dtype).to(DEV)
+  for transposed in (False, True):
+    w = torch.randn(*((K, cout, cin) if transposed else (K, cin, cout)), generator=g).to(dtype).to(DEV)
+    bias = torch.randn(cout, generator=g).to(dtype).to(DEV)
+    op = OC._gather_op(dtype, rows_in, rows, K, cin, cout, transposed, False, plan)
+    wide = op.padded.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE)
+    say('odd', dtype, K, cin, cout, transposed, op.padded.kernel, op.padded.cout)
+    assert op.kernel == _lib.GATHER_ZERO_PADDED and op.padded.cout % (32 if wide else 16) == 0
+    assert wide or K < 27
+    out = op.run(x, tg, w, bias).double()
+    wk = (w.transpose(1, 2) if transposed else w).double()
+    want, scale = bias.double().expand(rows, cout).clone(), bias.double().abs().expand(rows, cout).clone()
+    for k in range(K):
+      src = tg[:, k].long()
+      xk = torch.where(src[:, None] >= 0, x.double()[src.clamp_min(0)], 0.)
+      want += xk @ wk[k]
+      scale += xk.abs() @ wk[k].abs()
+    # fp32: three products of bf16 pieces, the fourth (2^-16 of its factors) left out
+    bound = (K * cin * 2.0 ** -24 + (2.0 ** -15 if dtype == torch.float32 else 0)) * scale + 1e-7
+    if dtype == torch.float16:
+      bound += 2.0 ** -11 * want.abs() * (1 + 2.0 ** -8)
+    assert ((out - want).abs() <= bound).all()
+
