@@ -138,9 +138,11 @@ extern "C" int ocnn_conv_wgrad_choose(int dtype, int64_t rows_x, int64_t rows, i
     // nine slots, 1.13 M rows 16 % set, 32 -> 64 290 / 86, 96 -> 32 253 / 166; eight, 947 k rows 15 % set, 112 / 60, 151 / 110;
     // 27, 1.06 M rows 61 % set, 64 -> 32 228 / 197, 128 -> 32 420 / 406, but 96 -> 32 338 / 384, 32 -> 96 213 / 385)
     const bool narrow = ca != cb && std::min(ca, cb) == 32;
-    const bool planned = narrow && (K < 27 || (plan_occupancy > kSparseMaxOccupancy && std::max(ca, cb) % 64 == 0));
+    // On eight slots it beats the pairs at every width: 128 -> 64 on 947 k rows 15 % set 242 / 127, 290 k 22 % set 124 / 70.
+    const bool planned = K == 8 || (narrow && (K < 27 || (plan_occupancy > kSparseMaxOccupancy && std::max(ca, cb) % 64 == 0)));
     if ((plan_occupancy <= kSparseMaxOccupancy || cb % 64 != 0) && rows >= kSparseMinRows &&
-        !(ca == cb && (ca == 32 || ca == 64)) && !planned &&
+        !(ca == cb && (ca == 32 || ca == 64)) &&
+        !(planned && ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct)) &&
         ocnn_conv_wgrad_sparse_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_SPARSE;
     // (half-empty blocks against the plan-free kernel, us: f16 32 -> 64 on 1.06 M rows 61 % set 201 / 775, 159 k 38 % set

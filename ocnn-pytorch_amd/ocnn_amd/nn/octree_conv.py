@@ -33,6 +33,7 @@ from .octree_pad import _depad_raw, _pad_raw, _rows, octree_depad, octree_pad
 PAD_MIN_ROWS = 16384
 _OPS = {}                # passes without a plan, by shape (see _gather_op)
 SPARSE_MAX_OCCUPANCY = 0.3
+PAIRS_222_MIN_ROWS = 80000   # coarse rows from which _pairs_of_222() may pick them
 SPARSE_MIN_ROWS = 32768
 
 
@@ -405,6 +406,18 @@ class OctreeConvBase:
     return (_gather_op(dtype, rows, self.fine_h, K, self.out_conv, self.in_conv, True, False, plan),
             self._inverse_table())
 
+  def _pairs_of_222(self, dtype):
+    """The weight gradient of 2x2x2 stride 2 over the pairs of the inverse table: only where the planned kernel does
+    not take the layer, and then with channels that leave the plan-free kernel's 64-channel tiles part empty, on
+    many rows (us, f16, pairs / planned: 64 -> 128 on 290 k rows 121 / 70, 947 k 266 / 123, 96 -> 96 138 / 96, 249 / 234;
+    pairs / plan-free: 64 -> 128 on 96 k rows 86 / 46, 160 k 113 / 66, 96 -> 96 84 / 111, 131 / 141, on 68 k 78 / 59)."""
+    rows, cin, cout = self.neigh.shape[0], self.in_conv, self.out_conv
+    plan = self._plan(dtype, self.fine_h, cin, cout)
+    if plan is not None and _lib.lib().ocnn_conv_wgrad_planned_supported(
+        _lib.DTYPE_CODE.get(dtype, -1), self.fine_h, rows, self.kdim, cin, cout, plan.umax):
+      return False
+    return rows >= PAIRS_222_MIN_ROWS and min(cin, cout) > 64 and cin % 64 != 0 and cout % 64 != 0
+
   def weight_op(self, dtype, out_transposed=False, coarse_index=None, coarse_rows=0):
     """data (fine rows), grad (table rows) -> (K, in_conv, out_conv); see weight_gemm."""
     rows, K = self.neigh.shape
@@ -422,8 +435,8 @@ class OctreeConvBase:
       return None
     # (3x3x3 over all nodes: 20 of the 27 slots of a table row are set, and the plan-free kernel
     # over the table is faster than the pairs of the inverse)
-    if self.stride == 2 and (self.kernel == '222' or (self.kernel == '333' and self.nempty)) and \
-        rows >= SPARSE_MIN_ROWS // 8 and \
+    if self.stride == 2 and rows >= SPARSE_MIN_ROWS // 8 and \
+        ((self.kernel == '333' and self.nempty) or (self.kernel == '222' and self._pairs_of_222(dtype))) and \
         _lib.lib().ocnn_conv_wgrad_sparse_supported(_lib.DTYPE_CODE.get(dtype, -1), rows, self.fine_h, self.kdim,
                                                     self.out_conv, self.in_conv, 0):
       plan_t = self.octree._plan(self.neigh_depth, self.kernel, self.stride, self.nempty, True, self.fine_h)

@@ -382,6 +382,7 @@ def test_selection_of_the_weight_gradient_with_32_channels_on_one_side():
       (F16, 500000, 27, 32, 64, 0.3, SPARSE), (F16, 500000, 27, 32, 64, 0.31, PLANNED), (F16, 500000, 27, 64, 32, 0.31, PLANNED),
       (F16, 500000, 27, 96, 32, 0.31, SPARSE), (F16, 500000, 27, 32, 96, 0.6, SPARSE), (F16, 500000, 27, 128, 32, 0.6, PLANNED),
       (F16, 500000, 9, 96, 32, 0.1, PLANNED), (F16, 500000, 8, 32, 64, 0.1, PLANNED),
+      (F16, 500000, 8, 96, 96, 0.1, PLANNED), (F16, 500000, 9, 96, 96, 0.1, SPARSE), (F16, 500000, 8, 128, 64, 0.2, PLANNED),
       (F16, 32768, 27, 32, 64, 0.6, PLANNED), (F16, 32767, 27, 32, 64, 0.6, PLAIN), (F16, 32767, 27, 64, 64, 0.6, PLANNED),
       (F32, 100, 27, 32, 64, 0.1, PLANNED), (F32, 500000, 27, 96, 32, 0.6, PLANNED), (F16, 500000, 27, 32, 32, 0.1, PLANNED)):
     assert L.ocnn_conv_wgrad_choose(dtype, rows, rows, K, ca, cb, 0, 1, 300, 2 * rows, occ) == want, (dtype, rows, K, ca, cb, occ)

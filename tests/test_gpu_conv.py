@@ -2096,3 +2096,24 @@ def test_odd_output_channels_on_the_plan(dtype, K, cin, cout):
       bound += 2.0 ** -11 * want.abs() * (1 + 2.0 ** -8)
     assert ((out - want).abs() <= bound).all()
 
+
+@pytest.mark.parametrize('kind,cin,cout', [('conv', 96, 96), ('deconv', 96, 96), ('conv', 64, 128), ('deconv', 128, 64)])
+def test_weight_gradient_of_222_stride_2(medium, monkeypatch, kind, cin, cout):
+  """2x2x2 stride 2 over non-empty nodes: the planned kernel where the plan allows, the pairs of the inverse table for
+  96 channels on tiles of too many distinct rows, the plan-free kernel otherwise; whole layers against the oracle."""
+  conv_mod = sys.modules['ocnn_amd.nn.octree_conv']
+  for name, value in (('SPARSE_MIN_ROWS', 0), ('SPARSE_MAX_OCCUPANCY', 1.0), ('PAIRS_222_MIN_ROWS', 0)):
+    monkeypatch.setattr(conv_mod, name, value)
+  made = set()
+  for fine in (5, 6, 7):
+    eng = (conv_mod._OctreeConv if kind == 'conv' else conv_mod._OctreeDeconv)(cin, cout, [2], 2, True)
+    eng.setup(medium.gpu, fine if kind == 'conv' else fine - 1)
+    kernel = eng.weight_op(torch.float16)[0].kernel
+    staged = medium.gpu._plan(fine, '222', 2, True, False, eng.fine_h).umax <= 415
+    say('222 stride 2', kind, cin, cout, fine, kernel, staged)
+    assert (kernel == _lib.WGRAD_PLANNED) == staged
+    assert (kernel == _lib.native().WGRAD_SPARSE_INVERSE) == (not staged and cin == 96)
+    made.add(kernel)
+    errs = run_layer(kind, medium, fine if kind == 'conv' else fine - 1, [2], 2, True, cin, cout, torch.float16)
+    assert max(errs.values()) < TOL[torch.float16], (fine, errs)
+  assert len(made) > 1 or cin != 96
