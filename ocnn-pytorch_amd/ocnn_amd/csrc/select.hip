@@ -133,20 +133,23 @@ extern "C" int ocnn_conv_wgrad_choose(int dtype, int64_t rows_x, int64_t rows, i
     // (32 x 32 and 64 x 64 have planned kernels of their own that are faster still; with channel
     // counts that are not multiples of 64 on the table-row side the pair-plan kernel, which sums
     // exactly ca x cb and only over the pairs, beats zero-padded 64 x 64 blocks on dense tables too)
-    // (32 channels on one side: the planned kernel, whose 64 x 64 blocks are half empty, beats the pair plan on tables of
-    // fewer than 27 slots and, with whole blocks on the other side, on dense ones of 27; us, f16, pair plan / planned:
-    // nine slots, 1.13 M rows 16 % set, 32 -> 64 290 / 86, 96 -> 32 253 / 166; eight, 947 k rows 15 % set, 112 / 60, 151 / 110;
-    // 27, 1.06 M rows 61 % set, 64 -> 32 228 / 197, 128 -> 32 420 / 406, but 96 -> 32 338 / 384, 32 -> 96 213 / 385)
+    // (32 channels on one side, pair plan / planned, us, f16.  Of x, whose 32 x 64 blocks hold the sums of all 27 slots: 32 -> 64
+    // on 1.13 M rows 7 % set 135 / 127, 947 k 15 % 127 / 100, 264 k 22 % 86 / 47; 32 -> 96 154 / 225, 150 / 193, but 95 / 65, 324 k
+    // 70 % 96 / 78, and on many rows sparse and dense 533 k 30 % 101 / 108, 1.06 M 61 % 213 / 216.  Of g, in half-empty 64 x 64
+    // blocks: 1.06 M rows 61 % set, 64 -> 32 228 / 197, 128 -> 32 420 / 406, but 96 -> 32 338 / 384.  Nine slots, 1.13 M rows
+    // 16 % set, 32 -> 64 290 / 63, 96 -> 32 253 / 166.  On eight slots the planned kernel is the faster one at every width: 32 -> 64
+    // on 947 k rows 15 % set 112 / 44, 128 -> 64 242 / 127, on 290 k 22 % set 124 / 70.)
     const bool narrow = ca != cb && std::min(ca, cb) == 32;
-    // On eight slots it beats the pairs at every width: 128 -> 64 on 947 k rows 15 % set 242 / 127, 290 k 22 % set 124 / 70.
-    const bool planned = K == 8 || (narrow && (K < 27 || (plan_occupancy > kSparseMaxOccupancy && std::max(ca, cb) % 64 == 0)));
+    const bool planned = K == 8 || (narrow && K < 27) ||
+                         (narrow && ca == 32 && (cb % 64 == 0 || (plan_occupancy > 0.2 && rows < 400000))) ||
+                         (narrow && cb == 32 && ca % 64 == 0 && plan_occupancy > kSparseMaxOccupancy);
     if ((plan_occupancy <= kSparseMaxOccupancy || cb % 64 != 0) && rows >= kSparseMinRows &&
         !(ca == cb && (ca == 32 || ca == 64)) &&
         !(planned && ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct)) &&
         ocnn_conv_wgrad_sparse_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_SPARSE;
-    // (half-empty blocks against the plan-free kernel, us: f16 32 -> 64 on 1.06 M rows 61 % set 201 / 775, 159 k 38 % set
-    // 44 / 106, 41 k 27 / 31, but 20 k 22 / 19 and 10 k 18 / 16; fp32 696 / 2451, 113 / 330, 42 / 94, 33 / 55, 30 / 47)
+    // (against the plan-free kernel, us: f16 32 -> 64 on 1.06 M rows 61 % set 119 / 775, 64 -> 32 197 / 732, 41 k 26 / 31, but 20 k
+    // 22 / 19 and 10 k 18 / 16; fp32 423 / 2451, 691 / 2307, 39 / 94, 34 / 55, 30 / 47)
     if (!(narrow && dtype != OCNN_F32 && rows < kSparseMinRows) &&
         ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_PLANNED;

@@ -48,9 +48,9 @@ struct WpStage {
   char* sl;
 };
 
-// A workgroup sums a C x C block (C = 64 or 32) of the channel pairs of one range of tiles, one
+// A workgroup sums a CA x CB block (64 x 64, 32 x 64 or 32 x 32) of the channel pairs of one range of tiles, one
 // of them when the layer has more channels (BLK; C = 64).  NFULL slots per wave with all
-// C x channels, NHALF (0/1, C = 64 only) slot shared by two waves (one x-channel half each);
+// CA x channels, NHALF (0/1, CA = 64 only) slot shared by two waves (one x-channel half each);
 // GROUPS workgroups split the K slots.  The workgroups of a range (slot groups, blocks) are neighbours in
 // the numbering, and each XCD takes an eighth of all of them in a row: they stage the same rows, and every
 // XCD has the same number however few ranges there are.
@@ -59,7 +59,11 @@ struct WpStage {
 // of 64-byte rows.  A transposing read of a 16-lane group touches 4 rows x 32 B, a
 // half wave 4 rows x 64 B; at a 64-byte pitch four consecutive positions cover all
 // 64 banks, and the second half is the first plus a constant.
-template <typename T, int C, int KK, int NFULL, int NHALF, int GROUPS, bool BLK>
+//
+// 32 channels of x: blocks of 32 x 64 have as many sums over all 27 slots as 64 x 64 over half of them, so one
+// workgroup stages a range's rows for all slots: 32 -> 64 on 1.06 M rows (61 % set) 119 us, in half-empty 64 x 64 blocks of two
+// slot groups 201; fp32 423 / 696.
+template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool BLK>
 __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
     const uint16_t* __restrict__ loc, uint32_t loc_bytes, const int32_t* __restrict__ uptr,
@@ -71,7 +75,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   const int grp = number % GROUPS;
   number /= GROUPS;
   // a block of a wider layer (channel counts are multiples of 32: the last block may be half)
-  const int nbb = BLK ? (cb + C - 1) / C : 1, nblocks = BLK ? nbb * ((ca + C - 1) / C) : 1;
+  const int nbb = BLK ? (cb + CB - 1) / CB : 1, nblocks = BLK ? nbb * ((ca + CA - 1) / CA) : 1;
   const int block = __builtin_amdgcn_readfirstlane(number % nblocks);
   const int split = __builtin_amdgcn_readfirstlane(number / nblocks);
   // fp32 data as bf16 pieces: hi hi, hi lo, lo hi, each with sums of its own.  (A product's number is a grid
@@ -79,27 +83,27 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   if (blockIdx.y == 1) g = g_lo;
   if (blockIdx.y == 2) x = x_lo;
   partial += blockIdx.y * set;
-  constexpr int H = C / 32;                   // 32-channel halves of a row
-  constexpr int NU = H * NFULL + NHALF;       // 32 x C accumulator units per wave
+  constexpr int HA = CA / 32, HB = CB / 32;   // 32-channel halves of a row of x, of g
+  constexpr int NU = HA * NFULL + NHALF;      // 32 x CB accumulator units per wave
   constexpr int NS = NFULL + NHALF;           // distinct slots per wave
   constexpr int SPG = 4 * NFULL + 2 * NHALF;  // slots per group
   constexpr int NL = 2 * NS;                  // table look-ups per lane and step
-  constexpr int NM = H * NU;                  // MFMAs per step
+  constexpr int NM = HB * NU;                 // MFMAs per step
   constexpr int XH = kWpXHalf * 2, GH = kWpGHalf * 2;   // byte offsets of the second halves
-  // C = 64: MFMAs between the position reads and their use
-  constexpr int PF0 = H == 1 ? 1 : ((NM - NL) < 4 ? (NM - NL) : 4);
+  // CA = 64: MFMAs between the position reads and their use
+  constexpr int PF0 = HA == 1 ? 1 : ((NM - NL) < 4 ? (NM - NL) : 4);
   constexpr int IP = (NL + 4 + PF0 - 1) / PF0;
-  // C = 32: positions and g with the first MFMA, the x reads XP per MFMA from MFMA XS on
+  // CA = 32: positions and g with the first MFMA, the x reads XP per MFMA from MFMA XS on
   constexpr int XS = NM > 2 ? 2 : NM - 1;
   constexpr int XP = (NL + (NM - XS) - 1) / (NM - XS);
-  static_assert((H == 1 || H == 2) && NU <= 7 && PF0 >= 1 && (H == 2 || NHALF == 0), "unit layout");
+  static_assert((HA == 1 || HA == 2) && HB >= HA && HB <= 2 && NU <= 7 && PF0 >= 1 && (HA == 2 || NHALF == 0), "unit layout");
 
   // one array per buffer, so that the compiler can tell the buffer being filled
   // from the one being read
-  __shared__ __attribute__((aligned(16))) T s_x0[H * kWpXHalf];
-  __shared__ __attribute__((aligned(16))) T s_x1[H * kWpXHalf];
-  __shared__ __attribute__((aligned(16))) T s_g0[H * kWpGHalf];
-  __shared__ __attribute__((aligned(16))) T s_g1[H * kWpGHalf];
+  __shared__ __attribute__((aligned(16))) T s_x0[HA * kWpXHalf];
+  __shared__ __attribute__((aligned(16))) T s_x1[HA * kWpXHalf];
+  __shared__ __attribute__((aligned(16))) T s_g0[HB * kWpGHalf];
+  __shared__ __attribute__((aligned(16))) T s_g1[HB * kWpGHalf];
   __shared__ __attribute__((aligned(16))) uint16_t s_loc0[kWpLoc];
   __shared__ __attribute__((aligned(16))) uint16_t s_loc1[kWpLoc];
   // lists of distinct rows, from entry 4 on; entry 3 stays -1 ("the row before the first")
@@ -125,10 +129,10 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   const uint32_t byte0 = 32u * (gq & 1) + 8u * (i16 & 3);
   const uint32_t lbF = (uint32_t)(slotF_rd * kWpRows + 8 * q + rs) * 2u;   // [slot][row] positions, 2 B each
   const uint32_t lbH = (uint32_t)(slotH_rd * kWpRows + 8 * q + rs) * 2u;
-  // C = 32: a wave's slots can end inside its group of NFULL (K = 27: slots 21..27), so
+  // CA = 32: a wave's slots can end inside its group of NFULL (K = 27: slots 21..27), so
   // every slot clamps on its own
-  uint32_t lbS[H == 1 ? NFULL : 1];
-  if constexpr (H == 1) {
+  uint32_t lbS[HA == 1 ? NFULL : 1];
+  if constexpr (HA == 1) {
 #pragma unroll
     for (int sl = 0; sl < NFULL; ++sl)
       lbS[sl] = (uint32_t)(min(slotF + sl, KK - 1) * kWpRows + 8 * q + rs) * 2u;
@@ -150,31 +154,33 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   //   2 pieces   table positions
   //   NX pieces  x rows: 16 distinct rows (ids in su) of one channel half
   //   1 piece    the list of distinct rows of the tile after (waves 0 and 1)
-  // (C = 64: 4 + 2 + 13 + 1, a wave takes one half of every second 16-row group;
-  //  C = 32: 2 + 2 + 7 + 1, a wave takes every fourth group.)
+  // (CA = CB = 64: 4 + 2 + 13 + 1, a wave takes one half of every second 16-row group;
+  //  32: 2 + 2 + 7 + 1, a wave takes every fourth group.)
   // The pieces are branch-free: whatever lies past the end of a list, of the table or of
   // the tile range is an out-of-range offset (loads zeros) or row 0.  A wave has one
   // instruction stream for the MFMAs and everything else, so each instruction saved here
   // is MFMA issue time won.
-  constexpr int NG = 2 * H, GST = 4 / H;                   // g pieces; 16-row groups between a wave's pieces
+  constexpr int NG = 2 * HB, GST = 4 / HA, GSG = 4 / HB;   // g pieces; 16-row groups between a wave's pieces of x, of g
   constexpr int NX = ((kWpCap + 16) / 16 + GST - 1) / GST;
   constexpr int tL = NG, tX = NG + 2, tU = NG + 2 + NX, kPieces = tU + 1;
   static_assert(kPieces <= 20 && (kWpCap + 1) % 16 == 0, "five steps of four pieces stage a tile");
-  constexpr int RSH = 5 + H;                               // log2 of the bytes of a C-channel row
-  // a block of a wider layer: rows of ca (cb) channels, this block's 64 start at xb (gb)
+  constexpr int RSH = 5 + HA, RSG = 5 + HB;                // log2 of the bytes of a CA-channel row, of a CB-channel row
+  // a block of a wider layer: rows of ca (cb) channels, this block's start at xb (gb)
   const int blk_a = __builtin_amdgcn_readfirstlane(block / nbb), blk_b = block - blk_a * nbb;
-  const uint32_t x_pitch = BLK ? (uint32_t)ca * 2u : (1u << RSH), g_pitch = BLK ? (uint32_t)cb * 2u : (1u << RSH);
-  const uint32_t xb = (uint32_t)blk_a << RSH, gb = (uint32_t)blk_b << RSH;
-  const int st_half = H == 2 ? (wave & 1) : 0, st_g16 = H == 2 ? (wave >> 1) : wave;
+  const uint32_t x_pitch = BLK ? (uint32_t)ca * 2u : (1u << RSH), g_pitch = BLK ? (uint32_t)cb * 2u : (1u << RSG);
+  const uint32_t xb = (uint32_t)blk_a << RSH, gb = (uint32_t)blk_b << RSG;
+  const int st_half = HA == 2 ? (wave & 1) : 0, st_g16 = HA == 2 ? (wave >> 1) : wave;
+  const int sg_half = HB == 2 ? (wave & 1) : 0, sg_g16 = HB == 2 ? (wave >> 1) : wave;
   const uint32_t st_xc = (uint32_t)st_half * 64u + (uint32_t)(lane & 3) * 16u;   // byte within a row
   const int st_pos = st_g16 * 16 + (lane >> 2);            // position / row of piece 0; piece j: + 16 GST j
-  const uint32_t st_gc = (BLK ? (uint32_t)st_pos * g_pitch + gb : ((uint32_t)st_pos << RSH)) + st_xc;
-  const uint32_t st_gstep = BLK ? 16u * GST * g_pitch : 4096u;   // 16 GST rows further
+  const uint32_t sg_c = (uint32_t)sg_half * 64u + (uint32_t)(lane & 3) * 16u, sg_pos = (uint32_t)(sg_g16 * 16 + (lane >> 2));
+  const uint32_t st_gc = (BLK ? sg_pos * g_pitch + gb : (sg_pos << RSG)) + sg_c;
+  const uint32_t st_gstep = BLK ? 16u * GSG * g_pitch : 4096u;   // 16 GSG rows further
   auto make_stage = [&](int64_t tile, int U, int32_t list_first, int32_t list_len, const int32_t* su,
                         int32_t* su_out, T* sx, T* sg, uint16_t* sl) {
     WpStage st;
     const int64_t tc = min(tile, tiles - 1);              // past the range: any valid tile
-    st.g_off = BLK ? (uint32_t)(tc * kWpRows) * g_pitch : (uint32_t)(tc * kWpRows) << RSH;
+    st.g_off = BLK ? (uint32_t)(tc * kWpRows) * g_pitch : (uint32_t)(tc * kWpRows) << RSG;
     st.loc_off = (uint32_t)(tc * kWpRows * KK * 2);
     const int e = wave * 256 + lane * 4;                   // the four list entries this lane brings in
     st.list_off = e < list_len ? (uint32_t)(list_first + e) * 4u : 0xffffff00u;
@@ -188,7 +194,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   auto stage_piece = [&](int t, const WpStage& st, int32_t id) {
     if (t < NG) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rs_g, (lds_ptr_t)(st.sg + (st_half * kWpGHalf + (st_g16 + GST * t) * 512) * 2), 16,
+          rs_g, (lds_ptr_t)(st.sg + (sg_half * kWpGHalf + (sg_g16 + GSG * t) * 512) * 2), 16,
           st.g_off + st_gc + (uint32_t)t * st_gstep, 0, 0, 0);
     } else if (t < tX) {
       constexpr int nchunk = (kWpRows * KK * 2 + 1023) >> 10;
@@ -208,11 +214,11 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
     }
   };
 
-  f32x16 acc[NU][H];
+  f32x16 acc[NU][HB];
 #pragma unroll
   for (int u = 0; u < NU; ++u)
 #pragma unroll
-    for (int bh = 0; bh < H; ++bh)
+    for (int bh = 0; bh < HB; ++bh)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[u][bh][r] = 0.f;
 
@@ -223,7 +229,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   auto pf_loc = [&](int j, const char* lcs, int sn) {       // j = 2 * slot + h
     const int sl = j >> 1, h = j & 1;
     uint32_t off;
-    if constexpr (H == 1) off = lbS[sl] + (uint32_t)(sn * 32 + h * 8);
+    if constexpr (HA == 1) off = lbS[sl] + (uint32_t)(sn * 32 + h * 8);
     else off = (sl < NFULL ? lbF + (uint32_t)(sl * kWpRows * 2) : lbH) + (uint32_t)(sn * 32 + h * 8);
     pv[j] = *(const uint16_t*)(lcs + off);
   };
@@ -235,14 +241,14 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
     const int sl = j >> 1, h = j & 1;
     const uint32_t ad = (pv[j] << 6) + byte0;                 // position 0 is the zero row
     if (sl < NFULL) {
-      on.a[H * sl][h] = Mma<T>::read_tr((const T*)(xs + ad));
-      if constexpr (H == 2) on.a[2 * sl + 1][h] = Mma<T>::read_tr((const T*)(xs + ad + (uint32_t)XH));
+      on.a[HA * sl][h] = Mma<T>::read_tr((const T*)(xs + ad));
+      if constexpr (HA == 2) on.a[2 * sl + 1][h] = Mma<T>::read_tr((const T*)(xs + ad + (uint32_t)XH));
     } else {
-      on.a[H * NFULL][h] = Mma<T>::read_tr((const T*)(xs + ad + ahH));
+      on.a[HA * NFULL][h] = Mma<T>::read_tr((const T*)(xs + ad + ahH));
     }
   };
   auto mm = [&](int m, const WpOps& oc) {
-    const int u = m / H, bh = m % H;
+    const int u = m / HB, bh = m % HB;
     const u32x4 av = u32x4{oc.a[u][0][0], oc.a[u][0][1], oc.a[u][1][0], oc.a[u][1][1]};
     const u32x4 bv = u32x4{oc.b[bh][0][0], oc.b[bh][0][1], oc.b[bh][1][0], oc.b[bh][1][1]};
     acc[u][bh] = Mma32<T>::run(av, bv, acc[u][bh]);
@@ -259,7 +265,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
       mm(m, oc);
       // operand fetch of the next step: table positions and g first, then the x reads
       // that depend on the positions, PF0 MFMAs later
-      if constexpr (H == 2) {
+      if constexpr (HA == 2) {
         if (m < PF0) {
 #pragma unroll
           for (int t = m * IP; t < (m + 1) * IP && t < NL + 4; ++t) {
@@ -274,7 +280,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 #pragma unroll
           for (int t = 0; t < NL; ++t) pf_loc(t, lcs, sn);
 #pragma unroll
-          for (int t = 0; t < 2; ++t) pf_g(t, gs, sn, on);
+          for (int t = 0; t < 2 * HB; ++t) pf_g(t, gs, sn, on);
         }
         if (m >= XS) {
 #pragma unroll
@@ -303,7 +309,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 #pragma unroll
     for (int t = 0; t < NL; ++t) pf_loc(t, lcs, 0);
 #pragma unroll
-    for (int t = 0; t < 2 * H; ++t) pf_g(t, gs, 0, on);
+    for (int t = 0; t < 2 * HB; ++t) pf_g(t, gs, 0, on);
 #pragma unroll
     for (int t = 0; t < NL; ++t) pf_x(t, xs, on);
   };
@@ -364,18 +370,18 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   const int b32 = lane & 31;
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int slot = u < H * NFULL ? slotF + u / H : slotH;
-    const int ah = u < H * NFULL ? u % H : (wave & 1);
+    const int slot = u < HA * NFULL ? slotF + u / HA : slotH;
+    const int ah = u < HA * NFULL ? u % HA : (wave & 1);
     if (slot >= KK) continue;
-    const int ldb = BLK ? cb : C;
-    float* dst = BLK ? partial + (((int64_t)split * KK + slot) * ca + blk_a * C) * cb + blk_b * C
-                     : partial + ((int64_t)split * KK + slot) * (C * C);
+    const int ldb = BLK ? cb : CB;
+    float* dst = BLK ? partial + (((int64_t)split * KK + slot) * ca + blk_a * CA) * cb + blk_b * CB
+                     : partial + ((int64_t)split * KK + slot) * (CA * CB);
     // a half block at the end of the channels: what the staging loads brought in beyond a
     // row only reached sums that are not written
-    if (BLK && blk_a * C + 32 * ah >= ca) continue;
+    if (BLK && blk_a * CA + 32 * ah >= ca) continue;
 #pragma unroll
-    for (int bh = 0; bh < H; ++bh) {
-      if (BLK && blk_b * C + 32 * bh >= cb) continue;
+    for (int bh = 0; bh < HB; ++bh) {
+      if (BLK && blk_b * CB + 32 * bh >= cb) continue;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int a = 32 * ah + 8 * (r >> 2) + 4 * q + (r & 3);
@@ -390,13 +396,14 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
 using namespace ocnn;
 
 
-// 64 x 64 blocks (half of one beyond the channels), but for the 32 x 32 layer
-static bool wp_wide(int ca, int cb) { return ca > 32 || cb > 32; }
+// blocks of channel pairs: 64 x 64 (the last of a side half beyond the channels), but for 32 channels of x, whose 32 x 64
+// blocks have room for the sums of all 27 slots in one workgroup, and for the 32 x 32 layer
+static bool wp_wide(int ca) { return ca > 32; }
 
 // workgroups of one range of tiles (and one product of bf16 pieces): the slot groups, the blocks of channel pairs
 static int wp_range_workgroups(int K, int ca, int cb) {
-  const int groups = (K == 27 && wp_wide(ca, cb)) ? 2 : 1;
-  return groups * (wp_wide(ca, cb) ? ((ca + 63) / 64) * ((cb + 63) / 64) : 1);
+  const int groups = (K == 27 && wp_wide(ca)) ? 2 : 1;
+  return groups * ((ca + 63) / 64) * ((cb + 63) / 64);
 }
 
 // ranges of tiles at most: as many as keep a workgroup on every CU (the LDS holds one)
@@ -474,20 +481,20 @@ struct WpArgs {
   float* partial;
 };
 
-template <typename T, int C, int KK, int NFULL, int NHALF, int GROUPS>
+template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS>
 static void launch_wp(const WpArgs& a, hipStream_t st) {
   const int64_t tiles = cdiv(a.rows, kWpRows);
   const uint32_t xb = (uint32_t)(a.rows_x * a.ca * 2), gb = (uint32_t)(a.rows * a.cb * 2);
   const int wgs = a.used * wp_range_workgroups(a.K, a.ca, a.cb);
   const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(a.plan_total * 4);
 #define OCNN_WP_KERNEL(BLK_)                                                                                        \
-  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, C, KK, NFULL, NHALF, GROUPS, BLK_>),                                  \
+  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, CA, CB, KK, NFULL, NHALF, GROUPS, BLK_>),                                  \
                      dim3(8 * (unsigned)cdiv(wgs, 8), a.products), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g,    \
                      gb, a.loc, lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial, (const T*)a.x_lo,     \
                      (const T*)a.g_lo, a.set)
-  if (a.ca == C && a.cb == C)
+  if (a.ca == CA && a.cb == CB)
     OCNN_WP_KERNEL(false);
-  else if constexpr (C == 64)
+  else if constexpr (CB == 64)
     OCNN_WP_KERNEL(true);
 #undef OCNN_WP_KERNEL
 }
@@ -495,17 +502,22 @@ static void launch_wp(const WpArgs& a, hipStream_t st) {
 // per-range sums of x^T g into `partial`
 template <typename T>
 static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
-#define OCNN_WP_LAUNCH(CC, KK, NF, NH, GR) launch_wp<T, CC, KK, NF, NH, GR>(a, st)
-  if (wp_wide(a.ca, a.cb)) {
-    if (a.K == 27) OCNN_WP_LAUNCH(64, 27, 3, 1, 2);
-    else if (a.K == 9) OCNN_WP_LAUNCH(64, 9, 2, 1, 1);
-    else if (a.K == 8) OCNN_WP_LAUNCH(64, 8, 2, 0, 1);
-    else OCNN_WP_LAUNCH(64, 3, 1, 0, 1);
+#define OCNN_WP_LAUNCH(CA, CB, KK, NF, NH, GR) launch_wp<T, CA, CB, KK, NF, NH, GR>(a, st)
+  if (wp_wide(a.ca)) {
+    if (a.K == 27) OCNN_WP_LAUNCH(64, 64, 27, 3, 1, 2);
+    else if (a.K == 9) OCNN_WP_LAUNCH(64, 64, 9, 2, 1, 1);
+    else if (a.K == 8) OCNN_WP_LAUNCH(64, 64, 8, 2, 0, 1);
+    else OCNN_WP_LAUNCH(64, 64, 3, 1, 0, 1);
+  } else if (a.cb > 32) {
+    if (a.K == 27) OCNN_WP_LAUNCH(32, 64, 27, 7, 0, 1);
+    else if (a.K == 9) OCNN_WP_LAUNCH(32, 64, 9, 3, 0, 1);
+    else if (a.K == 8) OCNN_WP_LAUNCH(32, 64, 8, 2, 0, 1);
+    else OCNN_WP_LAUNCH(32, 64, 3, 1, 0, 1);
   } else {
-    if (a.K == 27) OCNN_WP_LAUNCH(32, 27, 7, 0, 1);
-    else if (a.K == 9) OCNN_WP_LAUNCH(32, 9, 3, 0, 1);
-    else if (a.K == 8) OCNN_WP_LAUNCH(32, 8, 2, 0, 1);
-    else OCNN_WP_LAUNCH(32, 3, 1, 0, 1);
+    if (a.K == 27) OCNN_WP_LAUNCH(32, 32, 27, 7, 0, 1);
+    else if (a.K == 9) OCNN_WP_LAUNCH(32, 32, 9, 3, 0, 1);
+    else if (a.K == 8) OCNN_WP_LAUNCH(32, 32, 8, 2, 0, 1);
+    else OCNN_WP_LAUNCH(32, 32, 3, 1, 0, 1);
   }
 #undef OCNN_WP_LAUNCH
 }

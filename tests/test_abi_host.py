@@ -379,7 +379,8 @@ def test_selection_of_the_weight_gradient_with_32_channels_on_one_side():
   L, (F32, F16) = _lib.lib(), (0, 1)
   PLAIN, SPARSE, PLANNED = _lib.WGRAD_PLAIN, _lib.WGRAD_SPARSE, _lib.WGRAD_PLANNED
   for dtype, rows, K, ca, cb, occ, want in (
-      (F16, 500000, 27, 32, 64, 0.3, SPARSE), (F16, 500000, 27, 32, 64, 0.31, PLANNED), (F16, 500000, 27, 64, 32, 0.31, PLANNED),
+      (F16, 500000, 27, 32, 64, 0.05, PLANNED), (F16, 500000, 27, 64, 32, 0.3, SPARSE), (F16, 500000, 27, 64, 32, 0.31, PLANNED),
+      (F16, 399999, 27, 32, 96, 0.2, SPARSE), (F16, 399999, 27, 32, 96, 0.21, PLANNED), (F16, 400000, 27, 32, 96, 0.21, SPARSE),
       (F16, 500000, 27, 96, 32, 0.31, SPARSE), (F16, 500000, 27, 32, 96, 0.6, SPARSE), (F16, 500000, 27, 128, 32, 0.6, PLANNED),
       (F16, 500000, 9, 96, 32, 0.1, PLANNED), (F16, 500000, 8, 32, 64, 0.1, PLANNED),
       (F16, 500000, 8, 96, 96, 0.1, PLANNED), (F16, 500000, 9, 96, 96, 0.1, SPARSE), (F16, 500000, 8, 128, 64, 0.2, PLANNED),
