@@ -184,6 +184,16 @@ class _RowsWgrad(torch.autograd.Function):
     return (x @ grad.t() if ctx.needs_input_grad[0] else None, g @ grad if ctx.needs_input_grad[1] else None)
 
 
+def _rows_wgrad(g, x):
+  """g^T x on the kernel; the library's product for operands that it cannot read: gradients asked for as a batch
+  (is_grads_batched: a tensor without storage), negated views and zeros without memory, subclasses, and wherever a
+  tangent, a transform or a trace rides on them."""
+  if _lib.recorded() or not all(type(t) is torch.Tensor and torch._C._has_storage(t) and not t.is_neg() and
+                                not t._is_zerotensor() for t in (g, x)):
+    return g.t() @ x
+  return _RowsWgrad.apply(g, x) if torch.is_grad_enabled() else _lib.native().rows_wgrad(g, x)
+
+
 class _RowsLinear32(torch.autograd.Function):
   """torch.nn.functional.linear on many fp32 rows, with the weight gradient on this package's kernel: a sum over all
   rows into a small matrix, for which the library runs a handful of workgroups (us, library / kernel, with a norm of
@@ -199,8 +209,8 @@ class _RowsLinear32(torch.autograd.Function):
   def backward(ctx, grad):
     x, weight = ctx.saved_tensors
     needs = ctx.needs_input_grad
-    wgrad = _RowsWgrad.apply if torch.is_grad_enabled() else _lib.native().rows_wgrad
-    return grad @ weight if needs[0] else None, wgrad(grad, x) if needs[1] else None, grad.sum(0) if needs[2] else None
+    return (grad @ weight if needs[0] else None, _rows_wgrad(grad, x) if needs[1] else None,
+            grad.sum(0) if needs[2] else None)
 
 
 def _takes_rows32(data, lin):
