@@ -192,6 +192,12 @@ def only_traced():
   return _is_tracing() and _forward_ad._current_level < 0 and not _transforms_active()
 
 
+def trace_stays_here():
+  """The trace that is being recorded holds an operation in Python already, as which every autograd.Function is
+  recorded: it cannot be saved."""
+  return bool(torch._C._get_tracing_state().graph().findAllNodes('prim::PythonOp'))
+
+
 def unrecorded(make, *args):
   """make(*args) for what a layer's first call makes and keeps (tables, plans, passes): no part of a trace,
   which would hand out values of its own in place of sizes, and not under a transform of torch.func, which

@@ -186,10 +186,11 @@ class _RowsWgrad(torch.autograd.Function):
 
 def _rows_wgrad(g, x):
   """g^T x on the kernel; the library's product for operands that it cannot read: gradients asked for as a batch
-  (is_grads_batched: a tensor without storage), negated views and zeros without memory, subclasses, and wherever a
-  tangent, a transform or a trace rides on them."""
+  (is_grads_batched: a tensor without storage), negated views and zeros without memory, subclasses, more than its 4 GB
+  (of a trace, which is not asked again), and wherever a tangent, a transform or a trace rides on them."""
   if _lib.recorded() or not all(type(t) is torch.Tensor and torch._C._has_storage(t) and not t.is_neg() and
-                                not t._is_zerotensor() for t in (g, x)):
+                                not t._is_zerotensor() for t in (g, x)) or \
+      not _lib.lib().ocnnx_rows_wgrad_supported(0, x.shape[0], g.shape[1], x.shape[1]):
     return g.t() @ x
   return _RowsWgrad.apply(g, x) if torch.is_grad_enabled() else _lib.native().rows_wgrad(g, x)
 
@@ -216,22 +217,23 @@ class _RowsLinear32(torch.autograd.Function):
 def _takes_rows32(data, lin):
   """The fp32 weight gradient of `lin` on `data` can run on this package's kernel: plain tensors of many rows, no hook
   that would miss the Linear, no data type chosen by autocast.  A trace keeps the Linear, which can be saved with it,
-  unless the module is in training."""
+  unless what it holds so far cannot be saved anyway: then training gives the bits that it gives outside."""
   weight, bias = lin.weight, lin.bias
-  if not (torch.is_grad_enabled() and data.dim() == 2 and data.is_cuda and data.dtype == torch.float32 and
-          weight.requires_grad and type(data) is torch.Tensor and type(weight) is torch.nn.Parameter and
-          weight.dtype == torch.float32 and weight.device == data.device and
+  if not (torch.is_grad_enabled() and not torch.compiler.is_compiling() and data.dim() == 2 and data.is_cuda and
+          data.dtype == torch.float32 and type(data) is torch.Tensor and weight.requires_grad and
+          type(weight) is torch.nn.Parameter and weight.dtype == torch.float32 and weight.device == data.device and
           (bias is None or (bias.dtype == torch.float32 and bias.device == data.device))):
     return False
-  rows, (cout, cin) = int(data.shape[0]), map(int, weight.shape)
-  if not (rows >= 4096 and cin == data.shape[1] and cin % 4 == 0 and max(cin, cout) <= 512 and
+  if _lib.recorded() and not (lin.training and _lib.only_traced() and _lib.trace_stays_here()):
+    return False
+  rows, width, cout, cin = _lib.unrecorded(lambda: (*data.shape, *weight.shape))     # (numbers, also in a trace)
+  if not (rows >= 4096 and cin == width and cin % 4 == 0 and max(cin, cout) <= 512 and
           _lib.lib().ocnnx_rows_wgrad_supported(0, rows, cout, cin)):
     return False
-  if not (type(lin) is torch.nn.Linear and _plain(lin)) or lin._backward_hooks or lin._backward_pre_hooks or \
-      _nn._global_forward_hooks or _nn._global_forward_pre_hooks or _nn._global_backward_hooks or \
-      _nn._global_backward_pre_hooks or torch.is_autocast_enabled() or torch.compiler.is_compiling():
-    return False
-  return not _lib.recorded() or (lin.training and _lib.only_traced())
+  return (type(lin) is torch.nn.Linear and _plain(lin) and
+          not (lin._backward_hooks or lin._backward_pre_hooks or _nn._global_forward_hooks or
+               _nn._global_forward_pre_hooks or _nn._global_backward_hooks or _nn._global_backward_pre_hooks or
+               torch.is_autocast_enabled()))
 
 
 class Conv1x1(torch.nn.Module):

@@ -58,3 +58,22 @@ def test_module_with_a_batch_of_gradients():
   x64, many64 = x.detach().double(), many.double()
   bound = 8 * 2.0 ** -24 * (many64.abs().transpose(1, 2) @ x64.abs())
   assert ((got[1].double() - many64.transpose(1, 2).contiguous() @ x64).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('training', [False, True])
+def test_traces_keep_the_linear(training, tmp_path):
+  """A trace of layers whose other operations can be saved can be saved, in training as in evaluation; no decision on
+  the sizes is said to be baked into it."""
+  import warnings
+  from ocnn_amd.modules import Conv1x1
+  net = torch.nn.Sequential(Conv1x1(32, 16), torch.nn.ReLU(), Conv1x1(16, 8, use_bias=True)).to('cuda').train(training)
+  x = torch.randn(5000, 32, device='cuda', generator=torch.Generator('cuda').manual_seed(3)).requires_grad_()
+  with warnings.catch_warnings():
+    warnings.simplefilter('error', torch.jit.TracerWarning)
+    traced = torch.jit.trace(net, (x,), check_trace=False)
+  traced.save(str(tmp_path / 'net.pt'))
+  again = torch.jit.load(str(tmp_path / 'net.pt'))
+  assert torch.equal(again(x[:100]), net(x[:100]))
+  (got,), (want,) = (torch.autograd.grad(m(x).sum(), x) for m in (again, net))
+  assert torch.equal(got, want)
