@@ -204,7 +204,8 @@ int64_t ocnn_conv_workspace_bytes(int K, int cin, int cout);
 /* Workspace of ocnn_conv_gather including, for fp32 with cin % 32 == 0 and cout % 16 == 0,
  * the room to run on the bf16 MFMA kernel as three bf16 pieces ([hi | hi | lo] input channels
  * against [hi; lo; hi] weights, fp32 accumulation and output, about 1e-5 relative).  With
- * only ocnn_conv_workspace_bytes() of room fp32 runs on the plain kernel. */
+ * only ocnn_conv_workspace_bytes() of room fp32 runs on the plain kernel.  Of a larger
+ * workspace nothing beyond these bytes is written, and the sums' order is the same. */
 int64_t ocnn_conv_gather_workspace_bytes(int dtype, int64_t rows_in, int K, int cin, int cout);
 int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in,
                      const int32_t* table, int64_t rows_out, int K,
@@ -331,7 +332,7 @@ int ocnn_conv_gather_rw_static(int dtype, const void* in, int64_t rows_in, const
  * channels at a time, the weights stream from L2 into registers in the MFMA operand
  * layout, the four waves of a workgroup split the output channels.  Same arguments and
  * result as ocnn_conv_gather_rw; plan_max_distinct <= 416; workspace K * cin64 * cout * 2 bytes
- * with cin64 = cin rounded up to a multiple of 64.  plan_occupancy: the share of the table's
+ * with cin64 = cin rounded up to a multiple of 64 (more changes nothing).  plan_occupancy: the share of the table's
  * entries that are set (as for ocnn_conv_gather_choose), negative if unknown: from 40 % down
  * (other than 2x2x2 tables) the kernel tests, per slot and 32-row block of a tile, whether any
  * row has an entry there and leaves the block's products out otherwise: the rows of empty

@@ -713,12 +713,14 @@ extern "C" int ocnnx_conv_gather(int dtype, const void* in, int64_t rows_in, con
                                 reverse_slots, bias, out, out_index, st);
 }
 
+// (a larger workspace is not written beyond what the header asks for, and gives no other order of the sums)
 extern "C" int ocnn_conv_gather(int dtype, const void* in, int64_t rows_in, const int32_t* table,
                                 int64_t rows_out, int K, const void* w, int cin, int cout,
                                 int w_transposed, int reverse_slots, const void* bias, void* out,
                                 void* workspace, int64_t workspace_bytes, void* stream) {
   return ocnnx_conv_gather(dtype, in, rows_in, table, rows_out, K, w, cin, cout, w_transposed, reverse_slots, bias, out,
-                           nullptr, workspace, workspace_bytes, stream);
+                           nullptr, workspace, std::min(workspace_bytes, gather_base_bytes(dtype, rows_in, K, cin, cout)),
+                           stream);
 }
 
 extern "C" int64_t ocnn_conv_wgrad_workspace_bytes(int64_t rows, int K, int ca, int cb) {

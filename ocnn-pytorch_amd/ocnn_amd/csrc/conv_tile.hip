@@ -563,7 +563,8 @@ extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, con
   return rc == OCNN_OK ? check_launch("conv_gather_tile") : rc;
 }
 
-// The public entry point: 16-bit wide layers, with whatever room for parts the workspace has.
+// The public entry point: 16-bit wide layers, in one part: its workspace is that of the packed weights, whatever more
+// the caller has (the order of the sums does not hang on it).
 extern "C" int ocnn_conv_gather_wide_supported(int dtype, int64_t rows_in, int K, int cin, int cout,
                                                int plan_max_distinct) {
   if (dtype != OCNN_F16 && dtype != OCNN_BF16) return 0;
@@ -580,6 +581,6 @@ extern "C" int ocnn_conv_gather_wide(int dtype, const void* in, int64_t rows_in,
   OCNN_REQUIRE(ocnn_conv_gather_wide_supported(dtype, rows_in, K, cin, cout, plan_max_distinct),
                "conv_gather_wide: shape not supported");
   return ocnnx_gather_tile(dtype, in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out,
-                           K, w, cin, cout, w_transposed, reverse_slots, bias, nullptr, out, workspace, workspace_bytes, 0, 0,
-                           stream);
+                           K, w, cin, cout, w_transposed, reverse_slots, bias, nullptr, out, workspace,
+                           std::min(workspace_bytes, tile_packed_bytes(dtype, K, cin, cout)), 0, 0, stream);
 }

@@ -2117,3 +2117,38 @@ def test_weight_gradient_of_222_stride_2(medium, monkeypatch, kind, cin, cout):
     errs = run_layer(kind, medium, fine if kind == 'conv' else fine - 1, [2], 2, True, cin, cout, torch.float16)
     assert max(errs.values()) < TOL[torch.float16], (fine, errs)
   assert len(made) > 1 or cin != 96
+
+
+@pytest.mark.parametrize('entry,dtype', [('gather', torch.float32), ('gather', torch.float16), ('gather', torch.bfloat16),
+                                         ('wide', torch.float16), ('wide', torch.bfloat16)])
+def test_a_larger_workspace_changes_nothing(entry, dtype):
+  """ocnn_conv_gather and ocnn_conv_gather_wide on few rows (where the package's own calls cut the sums into parts): with
+  an arena of any size the same bits as with the published bytes, and nothing written beyond those."""
+  from ocnn_amd.octree.octree import TilePlan
+  L, P, code = _lib.lib(), _lib.ptr, _lib.DTYPE_CODE[dtype]
+  g = torch.Generator().manual_seed(5)
+  rows, K, cin, cout = 300, 27, 256, 128
+  table = _local_table(rows, rows, K, g).to(DEV)
+  plan = TilePlan(table)
+  x = torch.randn(rows, cin, generator=g).to(DEV, dtype)
+  w = (torch.randn(K, cin, cout, generator=g) / 80).to(DEV, dtype)
+  size = L.ocnn_conv_gather_workspace_bytes(code, rows, K, cin, cout) if entry == 'gather' else K * cin * cout * 2
+  assert (L.ocnnx_conv_gather_workspace_bytes(code, rows, rows, K, cin, cout) if entry == 'gather' else
+          L.ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout)) > size
+  got = []
+  for more in (0, 8 << 20):
+    out = torch.empty(rows, cout, dtype=dtype, device=DEV)
+    ws = torch.full((size + more,), 91, dtype=torch.uint8, device=DEV)
+    if entry == 'gather':
+      _lib.check(L.ocnn_conv_gather(code, P(x), rows, P(table), rows, K, P(w), cin, cout, 0, 0, None, P(out), P(ws),
+                                    size + more, _lib.stream()))
+    else:
+      _lib.check(L.ocnn_conv_gather_wide(code, P(x), rows, P(plan.loc), P(plan.uptr), P(plan.urows), plan.umax,
+                                         plan.total, -1.0, rows, K, P(w), cin, cout, 0, 0, None, P(out), P(ws), size + more,
+                                         _lib.stream()))
+    got.append(out)
+    written = int(ws[size:].ne(91).sum())
+    assert written == 0
+  same = torch.equal(got[0], got[1])
+  assert same
+  assert rel_err(got[0], C.forward_gemm(f64(x), f64(w), table.cpu().numpy().astype(np.int64))) < TOL[dtype]
