@@ -199,6 +199,12 @@ int ocnn_table_transpose(const int32_t* table, int64_t rows, int K,
  *                     a centrally symmetric table instead of a transposed one,
  *                     as ocnn/nn/kernels/conv_bwd_implicit_gemm.py:56 does)
  * bias may be NULL.  Rows of `in` are addressed by table values only.
+ * Non-finite values, here and in every other gather-GEMM and weight gradient below: a row
+ * of `in` (of x) reaches the results of the entries that name it and no others.  A weight (a row
+ * of g in a weight gradient) reaches the results with an entry in its slot, and may make NaN of
+ * those without one in its output channel: most kernels multiply a row of zeros there, as the
+ * reference's buffer does (ocnn/nn/octree_conv.py:133-137), and leave out what is empty for a
+ * whole tile or block of rows; the pair-plan kernels multiply the pairs only.
  * workspace: ocnn_conv_workspace_bytes(K, cin, cout) bytes (packed weights). */
 int64_t ocnn_conv_workspace_bytes(int K, int cin, int cout);
 /* Workspace of ocnn_conv_gather including, for fp32 with cin % 32 == 0 and cout % 16 == 0,
@@ -332,11 +338,11 @@ int ocnn_conv_gather_rw_static(int dtype, const void* in, int64_t rows_in, const
  * channels at a time, the weights stream from L2 into registers in the MFMA operand
  * layout, the four waves of a workgroup split the output channels.  Same arguments and
  * result as ocnn_conv_gather_rw; plan_max_distinct <= 416; workspace K * cin64 * cout * 2 bytes
- * with cin64 = cin rounded up to a multiple of 64 (more changes nothing).  plan_occupancy: the share of the table's
- * entries that are set (as for ocnn_conv_gather_choose), negative if unknown: from 40 % down
- * (other than 2x2x2 tables) the kernel tests, per slot and 32-row block of a tile, whether any
- * row has an entry there and leaves the block's products out otherwise: the rows of empty
- * entries are zeros (as in the reference's buffer, ocnn/nn/octree_conv.py:133-137), so the
+ * with cin64 = cin rounded up to a multiple of 64 (more changes nothing).  plan_occupancy: the
+ * share of the table's entries that are set (as for ocnn_conv_gather_choose), negative if
+ * unknown: from 45 % down (other than 2x2x2 tables) the kernel leaves out the slots without
+ * an entry in a tile and, per slot, the products of 32-row blocks without one: with finite
+ * weights they are zeros (as in the reference's buffer, ocnn/nn/octree_conv.py:133-137), so the
  * result is the same. */
 int ocnn_conv_gather_wide_supported(int dtype, int64_t rows_in, int K, int cin, int cout,
                                     int plan_max_distinct);

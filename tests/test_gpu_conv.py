@@ -834,7 +834,7 @@ def test_dense_rows_register_kernels(dtype, cin, cout):
 
 def _gather_wide(x, rows_in, table, plan, w, cout, transposed, reverse, bias, occupancy=-1.0):
   """ocnn_conv_gather_wide through the C ABI (the Python layer picks it only for plans with
-  enough reuse).  occupancy: the share of entries set as the entry point is told it (from 40 %
+  enough reuse).  occupancy: the share of entries set as the entry point is told it (from 45 %
   down it leaves out the products of 32-row blocks without an entry in a slot)."""
   L = _lib.lib()
   rows, K = table.shape
@@ -2152,3 +2152,91 @@ def test_a_larger_workspace_changes_nothing(entry, dtype):
   same = torch.equal(got[0], got[1])
   assert same
   assert rel_err(got[0], C.forward_gemm(f64(x), f64(w), table.cpu().numpy().astype(np.int64))) < TOL[dtype]
+
+
+def _sparse_local_table(rows, K, g):
+  """Most entries empty, a slot empty in whole tiles, another one in whole blocks of 32 rows."""
+  table = _local_table(rows, rows, K, g, empty=0.7)
+  table[(torch.arange(rows) // 128) % 2 == 0, 1] = -1
+  table[(torch.arange(rows) // 32) % 3 == 0, 2] = -1
+  return table
+
+
+def _hits(before, after, must, may):
+  """Non-finite exactly where `must`, at will where `may`, and the bits of before elsewhere."""
+  assert not after[must].isfinite().any() and after[~(must | may)].isfinite().all()
+  assert torch.equal(after[~(must | may)], before[~(must | may)])
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('K,cin,cout', [(27, 96, 96), (27, 128, 256), (27, 64, 64), (27, 32, 32), (8, 128, 64), (9, 64, 128)])
+def test_non_finite_values_of_a_gather(dtype, K, cin, cout):
+  """What an infinite value reaches, with and without a plan.  Of a row: the rows that read it, nothing else.  Of a
+  weight: at most what the dense product over the slots reaches, where an empty entry is a row of zeros (its output
+  channel), and every row with an entry in its slot; rows without one may have NaN there or not."""
+  import importlib
+  from ocnn_amd.octree.octree import TilePlan
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(K + cin)
+  rows = 128 * 9 + 5
+  table = _sparse_local_table(rows, K, g).to(DEV)
+  x = torch.randn(rows, cin, generator=g).to(DEV, dtype)
+  w = (torch.randn(K, cin, cout, generator=g) / 30).to(DEV, dtype)
+  x[x == 0] = 1
+  for plan in (TilePlan(table), None):
+    op = OC._gather_op(dtype, rows, rows, K, cin, cout, False, False, plan)
+    say('non-finite', dtype, K, cin, cout, 'kernel', op.kernel)
+    assert op.kernel == (_lib.GATHER_PLAIN if plan is None else
+                         _lib.GATHER_RW if cin == cout <= 64 and dtype != torch.float32 else _lib.GATHER_TILE)
+    before = op.run(x, table, w, None)
+    assert before.isfinite().all()
+    for row, a in ((0, 0), (rows - 1, cin - 1), (700, 17)):
+      bad = x.clone()
+      bad[row, a] = float('inf')
+      reads = (table == row).any(1)[:, None].expand(rows, cout)
+      _hits(before, op.run(bad, table, w, None), reads, torch.zeros_like(reads))
+    for k, a, b in ((1, 0, 0), (2, cin - 1, cout - 1), (K - 1, 17, 9)):
+      bad = w.clone()
+      bad[k, a, b] = float('inf')
+      column = torch.zeros(rows, cout, dtype=torch.bool, device=DEV)
+      column[:, b] = True
+      _hits(before, op.run(x, table, bad, None), column & (table[:, k] >= 0)[:, None], column)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('K,ca,cb', [(27, 64, 64), (27, 32, 32), (27, 32, 64), (27, 128, 32), (8, 96, 96), (27, 128, 64)])
+def test_non_finite_values_of_a_weight_gradient(dtype, K, ca, cb):
+  """As above.  Of a row of x: the slots it stands in, for its channel.  Of a row of g: at most its channel of every slot,
+  and the slots it has an entry in."""
+  import importlib
+  from ocnn_amd.octree.octree import TilePlan
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(K + ca)
+  rows = 128 * 9 + 5
+  table = _sparse_local_table(rows, K, g).to(DEV)
+  table[700, 1] = -1
+  plan = TilePlan(table)
+  x, gr = (torch.randn(rows, c, generator=g).to(DEV, dtype) for c in (ca, cb))
+  x[x == 0] = 1
+  gr[gr == 0] = 1
+  plain = OC._wgrad_op(dtype, rows, rows, K, ca, cb, False)
+  planned = OC._wgrad_op(dtype, rows, rows, K, ca, cb, False, plan).copy()
+  planned.kernel, planned.plan = _lib.WGRAD_PLANNED, OC._plan_arrays(plan, False)     # (16-bit layers of few rows: plan-free)
+  planned.ws_bytes = _lib.lib().ocnn_conv_wgrad_planned_workspace_bytes_for(_lib.DTYPE_CODE[dtype], rows, rows, K, ca, cb)
+  assert plain.kernel == _lib.WGRAD_PLAIN
+  for op in (planned, plain):
+    say('non-finite weight gradient', dtype, K, ca, cb, 'kernel', op.kernel)
+    before = op.run(x, gr, table)
+    assert before.isfinite().all()
+    for row, a in ((5, 0), (700, ca - 1)):
+      bad = x.clone()
+      bad[row, a] = float('inf')
+      must = torch.zeros(K, ca, cb, dtype=torch.bool, device=DEV)
+      must[:, a] = (table == row).any(0)[:, None]
+      _hits(before, op.run(bad, gr, table), must, torch.zeros_like(must))
+    for row, b in ((700, 0), (rows - 1, cb - 1)):
+      bad = gr.clone()
+      bad[row, b] = float('inf')
+      channel = torch.zeros(K, ca, cb, dtype=torch.bool, device=DEV)
+      channel[:, :, b] = True
+      _hits(before, op.run(x, bad, table), channel & (table[row] >= 0)[:, None, None], channel)
