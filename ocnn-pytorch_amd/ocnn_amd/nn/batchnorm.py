@@ -49,7 +49,7 @@ class BatchNormRelu1d(torch.nn.BatchNorm1d):
     """residual: added to the normalised values before the ReLU (the tail of a residual
     block), in the same pass.  relu: overrides the module's setting for this call."""
     relu = self.fused_relu if relu is None else relu
-    if not (input.dim() == 2 and input.is_cuda and input.shape[0] > 1 and kernels_take(input.dtype, input.shape[1])):
+    if not (input.dim() == 2 and input.is_cuda and input.shape[0] > 1 and kernels_take(input.dtype, int(input.shape[1]))):
       out = super().forward(input)
       if residual is not None:
         out = out + residual

@@ -432,3 +432,15 @@ def test_conv1x1_fp32_weight_gradient(rows, cin, cout, bias, tmp_path):
   for other in (x[:4095], x.detach().double()):
     layer = m if other.dtype == torch.float32 else m.double()
     assert 'RowsLinear' not in type(layer(other).grad_fn).__name__
+
+
+def test_traces_leave_nothing_behind():
+  """Which channels the kernels take is kept by their number, not by what stands for it while a trace records."""
+  from ocnn_amd.nn.batchnorm import kernels_take
+  bn = BatchNormRelu1d(32).to(DEV).eval()
+  x = torch.randn(100, 32, device=DEV)
+  bn(x)
+  held = kernels_take.cache_info().currsize
+  for _ in range(2):
+    traced = torch.jit.trace(bn, (x,), check_trace=False)
+  assert kernels_take.cache_info().currsize == held and torch.equal(traced(x), bn(x))
