@@ -479,8 +479,9 @@ int ocnn_conv_wgrad(int dtype, const void* x, int64_t rows_x, const void* g,
                     int out_transposed, void* gw, void* workspace,
                     int64_t workspace_bytes, void* stream);
 
-/* ocnn_conv_wgrad over a tile plan of the same table, for ca = cb = 32 and, summed in
- * 64 x 64 blocks of channel pairs, for ca, cb other multiples of 32 up to 1024 (same
+/* ocnn_conv_wgrad over a tile plan of the same table, for ca, cb multiples of 32 up to 1024:
+ * ca = cb = 32 in one 32 x 32 block of channel pairs, ca = 32 and more channels of g in 32 x 64
+ * blocks, all others in 64 x 64 blocks, of which the last of a side may be half empty (same
  * reference lines, same result up to the fp32 summation order, which is fixed).
  * Per tile the distinct x rows and the g rows are staged once in LDS; persistent
  * workgroups keep the sums of all K slots in accumulator registers over a range

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void rows_wgrad_f32_kernel(
   const __amdgpu_buffer_rsrc_t rs_g = make_rsrc(g, g_bytes);
   struct Step { float a[4][2], b[4][2]; };
   // (channels past a row's end belong to the next row: they reach only sums that are not written.  Rows past the
-  // end of the range are those of the next one but for the last: its are out of range, zeros)
+  // end of the range are out of the buffer's range: zeros of both operands)
   auto load = [&](int64_t row0) {
     Step s;
 #pragma unroll

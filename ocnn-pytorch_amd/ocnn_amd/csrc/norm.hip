@@ -199,8 +199,8 @@ __global__ __launch_bounds__(kBnFinishThreads) void bn_stats_finish_kernel(
 }
 
 // y = (x - mean) * (invstd * gamma) + beta (+ res), then max(., 0) when relu.  A thread keeps the
-// constants of its VEC channels in registers and walks the rows back to the first, four rows in flight.  run_mean, run_var (dtype rdtype), when given, take the place of mean
-// and invstd: a module's running statistics as it holds them, the reciprocal formed here (made into
+// constants of its VEC channels in registers and walks the rows back to the first, four rows in flight.
+// run_mean, run_var (dtype rdtype), when given, take the place of mean and invstd: a module's running statistics as it holds them, the reciprocal formed here (made into
 // mean and invstd by passes of their own they were four of the five launches of a layer in evaluation).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, int64_t rows, int C,
@@ -289,7 +289,8 @@ __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__
       is[v] = invstd[cl * VEC + v];
     }
     bn_params<VEC>(gamma, beta, pdtype, cl * VEC, ga, be);
-    for (int64_t r = (int64_t)blockIdx.x * (4 * rpp) + rl; r < rows; r += (int64_t)gridDim.x * (4 * rpp)) {   // four rows of both tensors in flight
+    // (four rows of both tensors in flight)
+    for (int64_t r = (int64_t)blockIdx.x * (4 * rpp) + rl; r < rows; r += (int64_t)gridDim.x * (4 * rpp)) {
       V a[4], g[4], ym[4];
       bool ok[4];
 #pragma unroll
@@ -715,8 +716,8 @@ static int bn_apply(int dtype, const void* x, int64_t rows, int channels, const 
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
     const int nblk = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_apply_kernel<T, VEC>));
-    hipLaunchKernelGGL((bn_apply_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var,
-                       run_dtype, eps);
+    hipLaunchKernelGGL((bn_apply_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, mean, invstd,
+                       gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var, run_dtype, eps);
   });
   return check_launch("batch_norm_apply");
 }

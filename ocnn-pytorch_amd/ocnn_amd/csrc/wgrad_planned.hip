@@ -1,5 +1,5 @@
-// Weight gradient for 32 x 32 channels and, in 64 x 64 blocks, for all other multiples of 32 channels,
-// on the tile plan of the neighbour table.
+// Weight gradient on the tile plan of the neighbour table, for multiples of 32 channels: 32 x 32, 32 x 64 blocks
+// where x has 32 channels, 64 x 64 blocks otherwise.
 //
 //   dW[k][a][b] = sum over table rows r of  x[table[r][k]][a] * g[r][b]
 //
