@@ -84,10 +84,11 @@ extern "C" int ocnn_conv_gather_choose(int dtype, int64_t rows_in, int64_t rows_
 // Over 916 bf16 passes (six kernel shapes, strides 1 and 2, all and non-empty nodes, three octrees of 20 k - 1 M
 // points, eleven widths): all plan-free 80.1 ms, all on the tile kernel 74.1, by this rule 70.0, the faster of the
 // two each time 69.3.  Other fp32 layers gain on every table, 1.04 - 9 x: plan-free reads three copies of their rows.
-// Dense rows of few channels run on the kernel of dense_rows.hip at every number of rows: over ten pairs of channels
-// its time is 0.76 of the plan-free kernel's on 1.13 M rows, 0.71 on 300 k, 0.68 on 60 k, 0.63 on 16 k, 0.60 on 4096; in
-// the place of the dense kernel 64 -> 128 takes 75 us for 93 on 960 k rows, 64 -> 256 117 / 140, 128 -> 128 94 / 105, all
-// three 17 - 28 / 19 - 29 on 240 k (128 -> 128 25.2 / 24.7) and 5 - 11 / 8 - 11 below.  (With an index of the rows: that one.)
+// Dense rows of few channels run on the kernel of dense_rows.hip at every number of rows.  Over its 22 pairs of channels
+// (f16) its time is 0.75 of that of the kernel chosen otherwise on 1.13 M rows, 0.68 on 300 k, 0.67 on 60 k, 0.71 on 16 k and
+// on 4096.  Pairs without gain: 192 -> 32 on 1.13 M rows 101 / 105 us, 64 -> 256 on 300 k 34 / 34, and 128 -> 128, whose other
+// kernel is the dense one: 110 / 118 on 1.13 M rows, but 29.8 / 28.8 on 300 k, 11.2 / 11.0 on 60 k, 8.1 / 7.1 on 16 k and
+// 7.8 / 7.2 on 4096.  (With an index of the rows: the dense kernel.)
 constexpr double kTileMinProducts = 3.0e9;
 constexpr double kTileMinProductsApart = 1.7e10;
 constexpr double kTileMinOccupancy = 0.06, kTileMinOccupancyInverse = 0.12;        // of 27 slots

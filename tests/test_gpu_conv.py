@@ -2240,3 +2240,39 @@ def test_non_finite_values_of_a_weight_gradient(dtype, K, ca, cb):
       channel = torch.zeros(K, ca, cb, dtype=torch.bool, device=DEV)
       channel[:, :, b] = True
       _hits(before, op.run(x, bad, table), channel & (table[row] >= 0)[:, None, None], channel)
+
+
+DENSE_ROWS = [(ci, co) for ci in (32, 64, 96, 128, 192) for co in (32, 64, 96, 128, 192, 256) if ci * co <= 16384]
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,cout', DENSE_ROWS)
+def test_dense_rows_with_a_batch_norm_behind(dtype, cin, cout):
+  """Every pair of channels of the kernel for few channels, with what its epilogue carries in evaluation: bias, batch
+  norm, residual and ReLU, all or some of them, against float64; rows that end inside a block and inside a wave's walk."""
+  import importlib
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(cin + cout)
+  rand = lambda *shape: torch.randn(*shape, generator=g).to(DEV, dtype)
+  w = rand(cout, cin) / cin ** 0.5
+  for rows, (bias, gamma, beta, residual, relu) in ((4133, (1, 1, 1, 1, 1)), (33, (0, 1, 1, 0, 1)), (1, (0, 0, 0, 0, 0)),
+                                                    (70001, (1, 0, 1, 1, 0)), (257, (0, 1, 0, 1, 1))):
+    say('dense rows and batch norm', dtype, rows, cin, cout, bias, gamma, beta, residual, relu)
+    op = OC._gather_op(dtype, rows, rows, 1, cin, cout, True, False, None, True)
+    assert op.kernel == _lib.GATHER_ROWS
+    layer = _lib.native().ConvLayer(op, None, False)
+    x, mean, var = rand(rows, cin), rand(cout), rand(cout).abs() + 0.5
+    some = lambda wanted, *shape: rand(*shape) if wanted else None
+    b, ga, be, res = some(bias, cout), some(gamma, cout), some(beta, cout), some(residual, rows, cout)
+    out = _lib.native().conv_bn(layer, x, w, b, mean, var, 1e-3, ga, be, bool(relu), res).double()
+    d = lambda t, default: t.double() if t is not None else torch.full((cout,), float(default), dtype=torch.float64, device=DEV)
+    mul = d(ga, 1) / (var.double() + 1e-3).sqrt()
+    want = (x.double() @ w.double().t() + d(b, 0) - mean.double()) * mul + d(be, 0)
+    scale = (x.double().abs() @ w.double().abs().t() + d(b, 0).abs() + mean.double().abs()) * mul.abs() + d(be, 0).abs()
+    if residual:
+      want, scale = want + res.double(), scale + res.double().abs()
+    if relu:
+      want = want.clamp_min(0)
+    # cin additions and some dozen operations of the epilogue in fp32, one rounding to the type
+    bound = (cin + 16) * 2.0 ** -24 * scale + torch.finfo(dtype).eps / 2 * want.abs() * (1 + 2.0 ** -8) + 1e-7
+    assert ((out - want).abs() <= bound).all()

@@ -4,7 +4,7 @@ gradients are on: every kernel that may take the layer, with and without bias, r
 import pytest
 import torch
 
-from ocnn_amd import synthetic
+from ocnn_amd import _lib, synthetic
 from ocnn_amd.modules import Conv1x1, Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
 from ocnn_amd.nn import OctreeConv
 from ocnn_amd.octree import Octree, Points
@@ -104,16 +104,23 @@ def test_tensors_held_as_plain_attributes(part, names):
     assert not torch.equal(block(x, octree, 5), want)
 
 
-def test_linear_layers_keep_one_table():
+# channels of 1x1 layers with a pass over the one-slot table; whether the forward pass is one (else: dense rows)
+LINEAR = [(32, 32, False), (192, 96, True), (288, 48, True)]
+
+
+@pytest.mark.parametrize('cin,cout,forward', LINEAR)
+def test_linear_layers_keep_one_table(cin, cout, forward):
   """A 1x1 layer whose row count differs with every call (a new octree every step): what is kept for it on
   the GPU does not grow with the calls."""
-  layer = Conv1x1(32, 32).to('cuda', torch.float16)      # (small products: the kernels on the one-slot table)
+  layer = Conv1x1(cin, cout).to('cuda', torch.float16)
   g = torch.Generator(device='cuda').manual_seed(3)
 
   def step(rows):
-    x = torch.randn(rows, 32, device='cuda', generator=g).half().requires_grad_()
+    x = torch.randn(rows, cin, device='cuda', generator=g).half().requires_grad_()
+    native = layer.native_layer(x)
+    assert native.fwd_table.shape[0] == rows and (native.fwd.kernel == _lib.GATHER_PLAIN) == forward
     layer.zero_grad()
-    layer(x).backward(torch.ones(rows, 32, device='cuda', dtype=torch.float16))
+    layer(x).backward(torch.ones(rows, cout, device='cuda', dtype=torch.float16))
     want = x.detach().double() @ layer.linear.weight.detach().double().t()
     assert (layer(x).double() - want).abs().max() < TOL[torch.float16] * want.abs().max()
 
@@ -126,17 +133,20 @@ def test_linear_layers_keep_one_table():
   assert torch.cuda.memory_allocated() <= held + 4096
 
 
-def test_linear_layer_in_a_graph():
-  """Replays of a captured 1x1 layer while larger ones run beside them."""
-  layer = Conv1x1(32, 32).to('cuda', torch.float16).requires_grad_(False)
-  x = torch.randn(5000, 32, device='cuda').half()
+@pytest.mark.parametrize('cin,cout,forward', LINEAR)
+def test_linear_layer_in_a_graph(cin, cout, forward):
+  """Replays of a captured 1x1 layer while larger ones run beside them: the table that the graph reads is its own."""
+  layer = Conv1x1(cin, cout).to('cuda', torch.float16).requires_grad_(False)
+  x = torch.randn(5000, cin, device='cuda').half()
+  with torch.no_grad():
+    assert (layer.native_layer(x).fwd_table is not None) == forward
   want = layer(x).clone()
   graph = torch.cuda.CUDAGraph()
   with torch.cuda.graph(graph):
     out = layer(x)
   for rows in (9000, 70000, 600000):
     out.zero_()
-    layer(torch.randn(rows, 32, device='cuda').half())
+    layer(torch.randn(rows, cin, device='cuda').half())
     torch.full((rows,), -1, dtype=torch.int32, device='cuda')      # (over memory that was given back)
     graph.replay()
     torch.cuda.synchronize()
