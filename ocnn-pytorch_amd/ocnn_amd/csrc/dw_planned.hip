@@ -8,11 +8,12 @@
 // tile, 64 channels of them, ONCE in LDS (asynchronous global->LDS loads) and every
 // neighbour read is an LDS read.  The products run on the 4x4x4 matrix instruction (a
 // depth-wise product is a 4x4 block with a diagonal operand), four times the vector unit's
-// rate, which leaves the kernels bound by LDS reads and by how many bytes a CU keeps in flight.
-// One workgroup of eight waves per CU walks a range of tiles: the rows of the next tile are in
-// flight while a tile is multiplied (a third row buffer, which would keep two tiles in flight
-// and is what the measured time per tile asks for, does not fit the 160 KB of LDS at 416 staged
-// rows).  fp32 accumulation; the weight gradient keeps the sums of all slots in registers over
+// rate, which leaves the kernels bound by a tile's chain inside the CU, mostly LDS: on 587 k rows of
+// 128 channels the gather takes 132 us behind the kernels that write its input, and 90 with all
+// rows from 0.5 MB that the caches hold, 69 of them with the LDS pipe busy; the weight gradient 157,
+// 104 and 89.  The difference is the rows' way from HBM: the rows of the next tile are in flight
+// while one workgroup of eight waves per CU multiplies a tile (a third row buffer, which would keep
+// two tiles in flight, does not fit the 160 KB of LDS at 416 staged rows).  fp32 accumulation; the weight gradient keeps the sums of all slots in registers over
 // its range of tiles, adds lanes and waves in a fixed order and leaves per-range sums to the
 // split reduction (no atomics).  Slot counts 27, 9, 8 and 3 (the kernel shapes the layers use).
 #include <algorithm>
