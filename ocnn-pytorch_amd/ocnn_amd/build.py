@@ -32,6 +32,7 @@ SOURCES = {
     'wgrad_sparse.hip': [],
     'dense_rw.hip': [],
     'dw_planned.hip': [],
+    'dw_siblings.hip': [],
     'wgrad_planned.hip': [],
     'plan.hip': [],
     'misc.hip': [],

@@ -18,6 +18,7 @@ constexpr int kPlanHashQuick = 1024;    // slots of the one-pass build: an octre
 constexpr int kPlanRankMax = 1024;      // up to here the distinct rows are ordered by counting
 constexpr int kPlanThreads = 512;       // threads a tile: the kernel waits on LDS round trips, more waves hide them
 constexpr int kPlanOverflow = 1 << 20;  // count of a tile whose blocks did not fit the quick build's slots
+constexpr int kPlanSiblings = 1 << 20;  // added to the set entries of a tile of sibling groups (3456 entries at most)
 constexpr int kPlanPosWords = (27 * (kPlanRows + 8) + 1) / 2;   // the staged positions, in 32-bit words
 
 template <int HASH>
@@ -40,9 +41,13 @@ __device__ __forceinline__ int plan_hash(int32_t v) {
 // locality: by a bitonic sort) and counting bits: the position of a row is the number of rows
 // in smaller blocks plus the bits below its own in its block's mask.
 //
+// GROUPS: tile_nnz also says (kPlanSiblings) whether the tile is one of sibling groups: 27 slots, whole groups of eight
+// rows, and slot o of sibling s is the same row for every (o, s) of the same o + s, so that the 8 x 27 entries are 64 cells.
+// (Compared in LDS, where the positions are: 766 k rows 100 -> 111 us a plan.)
+//
 // HASH = kPlanHashQuick (mode 2 only): a tile whose blocks do not fit gives up, ucount[tile] =
 // kPlanOverflow; the caller then plans the table in two passes with HASH = kPlanHash.
-template <int HASH>
+template <int HASH, bool GROUPS = false>
 __device__ __forceinline__ void plan_tile(
     const int64_t tile, const int32_t* __restrict__ table, int64_t rows, int K, int mode,
     int32_t* __restrict__ ucount, const int32_t* __restrict__ uptr, int32_t* __restrict__ urows,
@@ -293,6 +298,27 @@ __device__ __forceinline__ void plan_tile(
   u32x4* dst = (u32x4*)(loc + e0);
   for (int i = tid; i < K * (kPlanRows / 8); i += kPlanThreads)
     dst[i] = *(const u32x4*)(s_pos + (i >> 4) * kPitch + (i & 15) * 8);
+  if constexpr (GROUPS) if (K == 27 && rows % 8 == 0) {
+    // along each axis: slot o >= 1 of the siblings on this side is slot o - 1 of those on the other (a group's positions of a slot
+    // are 16 bytes: siblings x = 0 | x = 1 are its halves, y the words of a half, z the halves of a word)
+    bool same = true;
+#pragma unroll 1
+    for (int i = tid; i < 3 * 18 * (kPlanRows / 8); i += kPlanThreads) {
+      const int axis = i / 288, o = (i >> 4) % 18, at = (i & 15) * 8;
+      const int k = axis == 0 ? 9 + o : axis == 1 ? o / 6 * 9 + 3 + o % 6 : o / 2 * 3 + 1 + o % 2;
+      const u32x4 p = *(const u32x4*)(s_pos + k * kPitch + at);
+      const u32x4 q = *(const u32x4*)(s_pos + (k - (axis == 0 ? 9 : axis == 1 ? 3 : 1)) * kPitch + at);
+      if (axis == 0) {
+        same = same && p[0] == q[2] && p[1] == q[3];
+      } else if (axis == 1) {
+        same = same && p[0] == q[1] && p[2] == q[3];
+      } else {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) same = same && (p[w] & 0xffffu) == q[w] >> 16;
+      }
+    }
+    if (__syncthreads_and(same) && tid == 0) tile_nnz[tile] = s_nnz + kPlanSiblings;
+  }
 }
 
 __global__ __launch_bounds__(kPlanThreads) void tile_plan_kernel(
@@ -318,14 +344,16 @@ __device__ __forceinline__ int plan_item_of(const PlanItems& p, int64_t tile) {
   return i;
 }
 
-__global__ __launch_bounds__(kPlanThreads) void tile_plan_build_kernel(PlanItems p, int64_t first, int32_t* __restrict__ ucount,
+// (eight waves a SIMD: four tiles a CU; the comparison of GROUPS costs a few spilled registers for that)
+template <bool GROUPS>
+__global__ __launch_bounds__(kPlanThreads, 8) void tile_plan_build_kernel(PlanItems p, int64_t first, int32_t* __restrict__ ucount,
                                                                        int32_t* __restrict__ lists,
                                                                        int32_t* __restrict__ tile_nnz, int pad) {
   const int64_t tile = first + blockIdx.x;
   const ocnnx_plan_item& it = p.it[plan_item_of(p, tile)];
   const int64_t t0 = it.tile0;
-  plan_tile<kPlanHashQuick>(tile - t0, it.table, it.rows, it.K, 2, ucount + t0, nullptr, lists + t0 * pad, it.loc,
-                            tile_nnz ? tile_nnz + t0 : nullptr, pad);
+  plan_tile<kPlanHashQuick, GROUPS>(tile - t0, it.table, it.rows, it.K, 2, ucount + t0, nullptr, lists + t0 * pad, it.loc,
+                                    tile_nnz ? tile_nnz + t0 : nullptr, pad);
 }
 
 // Pair plan of a table, on top of its tile plan: per tile and LIST the rows that have a
@@ -366,7 +394,7 @@ __global__ void pair_plan_kernel(const uint16_t* __restrict__ loc, int64_t tiles
 // distinct rows are dropped (counted as empty) when they are few: at most a tenth of the
 // tiles.  stats: [tiles over cap, dropped (0 | 1), total, largest count, entries set, tiles the
 // quick one-pass build gave up on (then nothing else here means anything)], the third to fifth
-// without the dropped tiles.
+// without the dropped tiles.  Where every tile is marked as one of sibling groups, the second has 2 added.
 __device__ __forceinline__ void plan_offsets(
     const int32_t* __restrict__ ucount, const int32_t* __restrict__ tile_nnz, int64_t tiles, int cap,
     int32_t* __restrict__ uptr, int64_t* __restrict__ stats, int64_t* __restrict__ host_stats) {
@@ -390,7 +418,7 @@ __device__ __forceinline__ void plan_offsets(
     for (int i = 0; i < 4; ++i) q.v[i] = t + i < tiles ? p[t + i] : 0;
     return q;
   };
-  int big = 0, over = 0;
+  int big = 0, over = 0, plain = 0;
   for (int64_t r = 0; r < rounds; r += 4) {               // four rounds in flight
     Four c4[4];
 #pragma unroll
@@ -423,7 +451,12 @@ __device__ __forceinline__ void plan_offsets(
   for (int64_t r = 0; r < rounds; ++r) {
     const int64_t t = r * 4096 + 4 * tid;
     Four c = cn;
-    const Four z = zn;
+    Four z = zn;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (t + i < tiles && z.v[i] < kPlanSiblings) plain = 1;
+      z.v[i] &= kPlanSiblings - 1;
+    }
     cn = load4(ucount, t + 4096);                         // the next round's, under this round's scan
     zn = load4(tile_nnz, t + 4096);
     int own = 0;
@@ -460,6 +493,7 @@ __device__ __forceinline__ void plan_offsets(
     }
     base += total;
   }
+  const bool siblings = __syncthreads_or(plain) == 0 && tiles > 0;
   const long long wnnz = wave_sum(nnz);
   int wmx = mx;
 #pragma unroll
@@ -477,7 +511,7 @@ __device__ __forceinline__ void plan_offsets(
       max_all = max(max_all, s_wmax[w]);
     }
     uptr[tiles] = (int32_t)base;
-    const int64_t v[6] = {n_big, drop ? 1 : 0, base, max_all, nnz_all, n_over};
+    const int64_t v[6] = {n_big, (drop ? 1 : 0) + (siblings ? 2 : 0), base, max_all, nnz_all, n_over};
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
       stats[i] = v[i];
@@ -509,7 +543,7 @@ __device__ __forceinline__ void plan_compact(
     int cap, int pad, const int32_t* __restrict__ ulist, int32_t* __restrict__ urows, uint16_t* __restrict__ loc, int K) {
   const int lane = threadIdx.x & 63;
   const int U = ucount[tile];
-  if (stats[1] != 0 && U > cap) {
+  if ((stats[1] & 1) != 0 && U > cap) {
     u32x4* p = (u32x4*)(loc + tile * (int64_t)(K * kPlanRows));
     for (int i = lane; i < K * (kPlanRows / 8); i += 64) p[i] = u32x4{0u, 0u, 0u, 0u};
     return;
@@ -620,9 +654,11 @@ extern "C" int ocnnx_plan_build(const ocnnx_plan_item* items, int n, int cap, in
   if (const int rc = plan_items_check(items, n)) return rc;
   hipStream_t st = (hipStream_t)stream;
   plan_groups(items, n, [&](const PlanItems& p, int64_t first, int64_t tiles, int g) {
+    bool groups = false;                                     // (tables that can be of sibling groups)
+    for (int i = 0; i < p.n; ++i) groups = groups || (p.it[i].K == 27 && p.it[i].rows % 8 == 0);
     if (tiles > 0)
-      hipLaunchKernelGGL(tile_plan_build_kernel, dim3((unsigned)tiles), dim3(kPlanThreads), 0, st, p, first, ucount, lists,
-                         tile_nnz, pad);
+      hipLaunchKernelGGL(groups ? tile_plan_build_kernel<true> : tile_plan_build_kernel<false>, dim3((unsigned)tiles),
+                         dim3(kPlanThreads), 0, st, p, first, ucount, lists, tile_nnz, pad);
     hipLaunchKernelGGL(tile_plan_offsets_many_kernel, dim3((unsigned)p.n), dim3(1024), 0, st, p, ucount, tile_nnz, cap,
                        stats + 6 * g, host_stats + 6 * g);
   });
@@ -651,7 +687,7 @@ extern "C" int ocnn_tile_plan_build(const int32_t* table, int64_t rows, int K, i
   PlanItems p;
   p.n = 1;
   p.it[0] = {table, loc, nullptr, nullptr, rows, 0, K};
-  hipLaunchKernelGGL(tile_plan_build_kernel, dim3((unsigned)cdiv(rows, kPlanRows)), dim3(kPlanThreads), 0,
+  hipLaunchKernelGGL(tile_plan_build_kernel<false>, dim3((unsigned)cdiv(rows, kPlanRows)), dim3(kPlanThreads), 0,
                      (hipStream_t)stream, p, (int64_t)0, ucount, ulist, tile_nnz, pad);
   return check_launch("tile_plan");
 }

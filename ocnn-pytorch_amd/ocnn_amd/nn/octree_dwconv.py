@@ -67,6 +67,30 @@ def dw_wgrad(x, g, table, plan=None):
   return gw
 
 
+def dw_backward(x, g, table, w, plan):
+  """(dw_gather(g, w) with mirrored slots, dw_wgrad(x, g)) over a centrally symmetric table from one pass
+  over its tile plan, whose rows of g serve both; None where the kernel does not take the call."""
+  _lib.require_gpu(x, g, table, w)
+  L = _lib.lib()
+  rows, K = table.shape
+  C = x.shape[1]
+  code = _lib.DTYPE_CODE.get(x.dtype, -1)
+  if plan is None or plan.reuse < 2.0 or not L.ocnnx_dwconv_backward_planned_supported(code, rows, K, C, plan.umax):
+    return None
+  x, g, w = x.contiguous(), g.contiguous(), w.contiguous()
+  assert x.shape == g.shape == (rows, C) and w.numel() == K * C and x.dtype == g.dtype == w.dtype
+  dx, gw = torch.empty_like(g), torch.empty((K, 1, C), dtype=x.dtype, device=x.device)
+  ws = _lib.workspace(L.ocnn_dwconv_wgrad_planned_workspace_bytes(K, C), x.device)
+  siblings = plan.siblings and L.ocnnx_dwconv_siblings_supported(code, rows, K, C, plan.umax)
+  _lib.check((L.ocnnx_dwconv_siblings_backward if siblings else L.ocnnx_dwconv_backward_planned)(
+      code, _lib.ptr(x), _lib.ptr(g), _lib.ptr(plan.loc), _lib.ptr(plan.uptr), _lib.ptr(plan.urows), plan.umax,
+      plan.total, rows, K, _lib.ptr(w), C, _lib.ptr(dx), _lib.ptr(gw), _lib.ptr(ws), ws.numel(), _lib.stream()))
+  if plan.overflow_rows is not None:                       # the few tiles too dense for the plan
+    dx.index_copy_(0, plan.overflow_rows, dw_gather(g, rows, plan.overflow_table, w, True))
+    gw += dw_wgrad(g, x.index_select(0, plan.overflow_rows), plan.overflow_table).flip(0)
+  return dx, gw
+
+
 class OctreeDWConvBase(OctreeConvBase):
   """Depth-wise engine (ocnn/nn/octree_dwconv.py:19-118)."""
 
@@ -98,6 +122,12 @@ class OctreeDWConvBase(OctreeConvBase):
   def weight_gemm(self, data, grad, out_transposed=False):
     return dw_wgrad(data, grad, self.neigh, self._dw_plan(data))
 
+  def both_gemms(self, data, grad, weights):
+    """backward_gemm and weight_gemm in one pass, None where there is none."""
+    if not self.symmetric or data.shape != grad.shape or data.dtype != grad.dtype:
+      return None
+    return dw_backward(data, grad, self.neigh, weights, self._dw_plan(data))
+
 
 class OctreeDWConvFunction(Function):
   """Autograd wiring (ocnn/nn/octree_dwconv.py:121-155)."""
@@ -121,6 +151,10 @@ class OctreeDWConvFunction(Function):
     data, weights = ctx.saved_tensors
     eng = ctx.eng
     grad = grad.contiguous()
+    if ctx.needs_input_grad[0] and ctx.needs_input_grad[1]:
+      both = eng.both_gemms(data, grad, weights)
+      if both is not None:
+        return both + (None,) * 7
     grad_out = eng.backward_gemm(grad, weights) if ctx.needs_input_grad[0] else None
     grad_w = eng.weight_gemm(data, grad) if ctx.needs_input_grad[1] else None
     return (grad_out, grad_w) + (None,) * 7

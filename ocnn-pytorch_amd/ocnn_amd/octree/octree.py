@@ -124,6 +124,7 @@ class TilePlan:
   in the middle of a training step wants: every read-back waits for the whole queue of kernels
   before it and leaves the device idle while the host catches up."""
 
+  siblings = False
   CAP = 415      # the smallest limit of the kernels on the plan
   LIST_PAD = 416  # rows a tile's list may have in the one-pass build
 
@@ -162,7 +163,9 @@ class TilePlan:
       # (tiles with more distinct blocks of rows than the one pass holds: no locality)
       ucount, stats = self._count(table, cap)
       self.urows = None
-    _, dropped, self.total, self.umax, self.nnz = stats[:5]
+    _, flags, self.total, self.umax, self.nnz = stats[:5]
+    dropped = flags & 1
+    self.siblings = bool(flags & 2)  # 27 slots over whole groups of siblings (seen by the one-pass build)
     # how often a staged row is used by its tile: near 1 there is nothing to gain from staging
     self.reuse = self.nnz / max(self.total, 1)
     if dropped:

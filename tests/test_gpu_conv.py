@@ -1484,6 +1484,66 @@ def test_dwconv_planned_kernels(dtype, K, ch):
     assert torch.equal(gw, dw_wgrad(x.to(DEV), gr.to(DEV), tg, plan))
 
 
+def _lattice_table(rows, K, g, groups=False):
+  """The centrally symmetric table of `rows` random cells of a lattice in Morton order (groups: whole groups of eight
+  siblings): slot k of a row is the cell at the k-th of the K offsets around it, if there."""
+  if groups:
+    key = torch.randperm(max(rows // 4, 1), generator=g)[:rows // 8].sort().values
+    key = (8 * key[:, None] + torch.arange(8)).view(-1)
+  else:
+    key = torch.randperm(4 * rows, generator=g)[:rows].sort().values
+  bits = int(key.max()).bit_length() // 3 + 1
+  side = 2 ** bits
+  x, y, z = [sum(((key >> (3 * i + j)) & 1) << i for i in range(bits)) for j in (2, 1, 0)]
+  at = torch.full(((side + 2) ** 3,), -1, dtype=torch.int32)
+  pad = ((x + 1) * (side + 2) + y + 1) * (side + 2) + z + 1
+  at[pad] = torch.arange(rows, dtype=torch.int32)
+  offsets = [(i // 9 - 1, i // 3 % 3 - 1, i % 3 - 1) for i in range(27)]
+  offsets = [o for o in offsets if K == 27 or o[0] == 0 and (K == 9 or o[1] == 0)]
+  return torch.stack([at[pad + (a * (side + 2) + b) * (side + 2) + c] for a, b, c in offsets], 1)
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('K,ch,groups', [(27, 64, False), (27, 192, False), (9, 128, False), (3, 64, False), (27, 64, True),
+                                         (27, 192, True), (9, 64, True)])
+def test_dwconv_backward_planned(dtype, K, ch, groups):
+  """Both gradients of a depth-wise layer from one pass over the plan, on any symmetric table and on tables of sibling
+  groups: one tile, whole tiles, a remainder, more tiles than workgroups; against the oracle, and the data gradient
+  to the bit as the gather with mirrored slots gives it: the same products in the same order.
+  A non-finite x or g reaches the sums of the slots with an entry of it, as on the other kernels, and no others."""
+  from ocnn_amd.nn.octree_dwconv import dw_backward, dw_gather
+  from ocnn_amd.octree.octree import TilePlan
+  g = torch.Generator().manual_seed(7 * K + ch)
+  for rows in ((8, 128, 1000, 128 * 300 + 8) if groups else (1, 128, 1000, 128 * 300 + 7)):
+    say('dwconv backward planned', dtype, K, ch, groups, rows)
+    table = _lattice_table(rows, K, g, groups)
+    tg = table.to(DEV)
+    plan = TilePlan(tg)
+    plan.reuse = 10.0
+    assert plan.siblings == (groups and K == 27)
+    t64 = table.numpy().astype(np.int64)
+    x = torch.randn(rows, ch, generator=g).to(dtype)
+    gr = torch.randn(rows, ch, generator=g).to(dtype)
+    w = torch.randn(K, 1, ch, generator=g).to(dtype)
+    dx, gw = dw_backward(x.to(DEV), gr.to(DEV), tg, w.to(DEV), plan)
+    assert rel_err(dx, C.dw_forward(f64(gr), f64(w)[::-1], t64)) < TOL[dtype]
+    assert rel_err(gw, C.dw_weight(f64(x), f64(gr), t64)) < TOL[dtype]
+    assert all(torch.equal(a, b) for a, b in zip((dx, gw), dw_backward(x.to(DEV), gr.to(DEV), tg, w.to(DEV), plan)))
+    assert torch.equal(dx, dw_gather(gr.to(DEV), rows, tg, w.to(DEV), True, None, plan))
+    row, c = rows // 3, 13
+    for value in (float('inf'), float('nan')):
+      for which in (x, gr):
+        bad = which.clone()
+        bad[row, c] = value
+        _, got = dw_backward((bad if which is x else x).to(DEV), (bad if which is gr else gr).to(DEV), tg, w.to(DEV), plan)
+        # slot k of gw multiplies x[table[i][k]] with g[i]
+        named = torch.stack([(table[:, k] == row).any() if which is x else table[row, k] >= 0 for k in range(K)])
+        touched = torch.zeros(K, 1, ch, dtype=torch.bool)
+        touched[named, 0, c] = True
+        assert not bool(torch.isfinite(got.cpu()[touched]).any())
+        assert torch.equal(got.cpu()[~touched], gw.cpu()[~touched])
+
+
 def test_dwconv_planned_non_finite_values_stay_in_their_group_of_four():
   """The planned depth-wise gather multiplies on the 4x4x4 matrix instruction with diag(w) as one
   operand, so 0 x inf of one channel reaches the other three channels of its group of four as
