@@ -125,14 +125,16 @@ int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, int pad, co
 
 // The octree build from the points on: normalised points, keys, sort and node counts (sizes: device,
 // levels + 1, as ocnn_octree_build_scan); then keys, children and the indices of the non-empty nodes of
-// the layers from the deepest full one on (h_index[d], d >= full_depth); then every neighbour table.
+// the layers from the deepest full one on (h_index[d], d >= full_depth) and the leaves' mean points and
+// normals (normals, out_normals: may be null; rows: 32 bytes a point, from the scan to the fill); then every neighbour table.
 int64_t ocnnx_tree_workspace_bytes(int64_t n, int depth, int full_depth, int batch_bits);
 int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch, int batch_is_float,
-                    int depth, int full_depth, int batch_bits, float* pts_out, void* workspace, int64_t workspace_bytes,
-                    int32_t* perm, int64_t* sizes, void* stream);
+                    int depth, int full_depth, int batch_bits, const float* normals, float* rows, void* workspace,
+                    int64_t workspace_bytes, int32_t* perm, int64_t* sizes, void* stream);
 int ocnnx_tree_fill(const void* workspace, int64_t n, int depth, int full_depth, int batch_size, int batch_bits,
                     const int64_t* h_sizes, const int32_t* perm, int64_t* const* h_keys, int32_t* const* h_children,
-                    int32_t* const* h_index, int64_t* inverse, int32_t* seg_start, void* stream);
+                    int32_t* const* h_index, int64_t* inverse, int32_t* seg_start, const float* rows, float* out_pts,
+                    float* out_normals, void* stream);
 int ocnnx_neigh_all(int depth, int full_depth, int batch, const int64_t* h_nnum, const int64_t* h_nnum_nempty,
                     const int64_t* const* h_keys, const int32_t* const* h_children,
                     const int32_t* const* h_nempty_index, int32_t* const* h_neigh, void* stream);

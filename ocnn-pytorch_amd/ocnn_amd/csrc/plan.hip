@@ -515,7 +515,8 @@ __device__ __forceinline__ void plan_offsets(
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
       stats[i] = v[i];
-      if (host_stats) host_stats[i] = v[i];               // (host memory: no copy to wait for on top of the kernel)
+      // (host memory, watched by the host: no copy to wait for on top of the kernel)
+      if (host_stats) __hip_atomic_store(&host_stats[i], v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
 }

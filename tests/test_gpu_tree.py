@@ -44,3 +44,33 @@ def test_build_and_tables(n, depth, full_depth, batch):
   for d in range(1, depth + 1):
     layer.construct_neigh(d)
     assert torch.equal(layer.neighs.get32(d), o.neighs.get32(d)), d
+
+
+@pytest.mark.parametrize('n,depth,batch,same', [(1, 2, 1, False), (255, 2, 1, False), (257, 1, 1, True), (1025, 3, 2, False),
+                                                (20011, 4, 1, False), (65536, 3, 1, False), (65537, 3, 1, False), (70000, 2, 1, True),
+                                                (9000, 11, 2, False)])
+@pytest.mark.parametrize('normals', [True, False])
+def test_leaf_averages_across_spans(n, depth, batch, same, normals):
+  """Leaves of many points, within a span of the scatter and over several (same: all points in one cell), on both sizes of
+  spans and on the library's sort, with and without normals: sums in the order of the points, to the bit of the oracle's."""
+  print('leaves', n, depth, batch, same, normals, flush=True)
+  g = torch.Generator().manual_seed(n)
+  pts = torch.rand(n, 3, generator=g) * (0.01 if same else 1.98) + (0.5 if same else -0.99)
+  nrm = torch.randn(n, 3, generator=g) if normals else None
+  bid = torch.randint(0, batch, (n, 1), generator=g).float()
+  bid[0], bid[-1] = 0, batch - 1
+  o = Octree(depth, 1, batch_size=batch)
+  idx = o.build_octree(Points(pts.cuda(), None if nrm is None else nrm.cuda(), batch_id=bid.cuda() if batch > 1 else None,
+                              batch_size=batch)).cpu().numpy()
+  p = ((pts.numpy() - np.float32(-1)) * np.float32(2 ** depth / 2)).astype(np.float32)
+  leaves = idx.max() + 1
+  sums, count = np.zeros((leaves, 6), np.float32), np.bincount(idx, minlength=leaves).astype(np.float32)
+  rows = np.concatenate([p, np.zeros_like(p) if nrm is None else nrm.numpy()], 1)
+  for i, leaf in enumerate(idx):
+    sums[leaf] += rows[i]
+  assert np.array_equal(o.points[depth].cpu().numpy(), sums[:, :3] / count[:, None])
+  if normals:
+    length = np.maximum(np.sqrt((sums[:, 3:] ** 2).sum(1, keepdims=True)), 1e-12)
+    assert np.abs(o.normals[depth].cpu().numpy() - sums[:, 3:] / length).max() < 1e-6
+  else:
+    assert o.normals[depth] is None
