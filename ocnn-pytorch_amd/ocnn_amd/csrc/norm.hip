@@ -411,26 +411,37 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
   }
 }
 
-// ---- few rows: the whole batch norm in one launch ----
+// ---- few rows: one launch, or two ----
 //
-// At a thousand rows (the coarse levels of a network, small clouds) a pass is launch latency, and a training
-// step's forward and backward pass have three launches each (sums, their sum, the elementwise pass).  Here a workgroup of
-// 1024 threads has 64 bytes of every row (kBnSmallLanes threads) to itself: sums, statistics and the
-// elementwise pass follow each other in the workgroup, the rows come from L2 the second time.  Measured, forward +
-// backward (us, three launches each -> one): fp32 337 x 256 21.5 -> 11.6, 1425 x 256 23.3 -> 17.0, 2048 x 256 23.8 -> 20.0,
-// fp16 337 x 256 28.5 -> 15.6, 2048 x 256 29.6 -> 27.1.  On more rows a workgroup reads too much by itself (with 32 bytes
-// of a row 4096 x 128 22.9 -> 29.5), so that is where the line lies.
-constexpr int kBnSmallThreads = 1024, kBnSmallLanes = 4;
-constexpr int64_t kBnSmallRows = 2048;
+// At some ten thousand rows and below (the coarse levels of a network, small clouds) a pass is launch latency, and a
+// training step's forward and backward pass have three launches each (sums, their sum, the elementwise pass).  Here a
+// workgroup of 1024 threads has 64 or 128 bytes of a row (LANES threads) to itself, of all rows or of a range of them:
+// * one launch: sums, statistics and the elementwise pass follow each other in the workgroup, the rows come from L2 the
+//   second time;
+// * two: the sums of every range, and an elementwise pass whose workgroups add the ranges' sums themselves, while their rows are on
+//   their way: of so few channels that is nothing (of whole rows it was a launch of its own).
+// Forward / backward in us, three launches before, now: fp32 4096 x 128 10.9 / 13.4, 7.8 / 9.1; 20 k x 128 15.4 / 21.7, 9.7 / 17.3;
+// 39 k x 96 17.9 / 25.0, 12.8 / 22.3; fp16 2048 x 256 (one launch before) 12.8 / 20.2, 9.5 / 12.5; 20 k x 96 15.8 / 22.5, 11.1 / 15.4;
+// 60 k x 128 24.4 / 39.5, 17.5 / 31.8.  The lines:
+// * one launch up to 1024 rows: fp32 x 256 800 rows 6.3 / 7.9, two 7.4 / 8.6; 1425 rows 7.7 / 10.1, two 7.2 / 8.8;
+// * the three launches, whose workgroups have whole rows, from 32 MB on forward (fp32 33 k x 256 two 24.4, three 26.4; 66 k x 256
+//   43.9, 41.0) and from 20 MB on backward (60 k x 128 38.8, 38.1; 66 k x 64 24.9, 27.2), where a row's pieces no longer meet in a
+//   cache;
+// * 128 bytes of a row, whole lines, from 4 MB on in fp32 (20 k x 128: 9.7 / 17.3, with 64 bytes 11.0 / 23.7), from 12 MB on in 16
+//   bits, where they are 64 channels (39 k x 96 15.4 / 28.6, with 64 bytes 13.1 / 20.6; 33 k x 256 21.3 / 37.5, 22.4 / 46.2).
+constexpr int kBnSlabThreads = 1024;
+constexpr int64_t kBnSmallRows = 1024, kBnSlabRows = 131072;
+constexpr int64_t kBnSlabForward = 32 << 20, kBnSlabBackward = 20 << 20, kBnWideF32 = 4 << 20, kBnWide16 = 12 << 20;
+constexpr int kBnSlabRanges = 64;         // of the sums, at most (more where the channels are few slabs: a workgroup on every CU)
 
 // sums over the workgroup of the 2 VEC values of each thread, per thread of a row: s_out[kind][channel of the
 // workgroup], in a fixed order: 2 VEC threads' values in fp64, then those sums one after the other.
-template <int VEC>
-__device__ __forceinline__ void bn_small_sums(const float (&s1)[VEC], const float (&s2)[VEC], float* s_f, double* s_d,
-                                              double* s_out) {
-  constexpr int lpr = kBnSmallLanes;
+template <int VEC, int LANES>
+__device__ __forceinline__ void bn_slab_sums(const float (&s1)[VEC], const float (&s2)[VEC], float* s_f, double* s_d,
+                                             double* s_out) {
+  constexpr int lpr = LANES;
   const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
-  constexpr int pitch = kBnSmallThreads / lpr + 1, sums = 2 * lpr * VEC, segments = kBnSmallThreads / sums;
+  constexpr int pitch = kBnSlabThreads / lpr + 1, sums = 2 * lpr * VEC, segments = kBnSlabThreads / sums;
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
     s_f[(cl * VEC + v) * pitch + rl] = s1[v];
@@ -454,189 +465,312 @@ __device__ __forceinline__ void bn_small_sums(const float (&s1)[VEC], const floa
   __syncthreads();
 }
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(kBnSmallThreads) void bn_small_kernel(
-    const T* __restrict__ x, int rows, int C, float eps, float* __restrict__ mean, float* __restrict__ var,
-    float* __restrict__ invstd, void* running_mean, void* running_var, int rdtype, float factor,
-    long long* batches_tracked, const void* __restrict__ gamma, const void* __restrict__ beta, int pdtype, int relu,
-    const T* __restrict__ res, T* __restrict__ y) {
-  typedef BnVec<T, VEC> V;
-  constexpr int lpr = kBnSmallLanes, rpp = kBnSmallThreads / lpr;
-  __shared__ float s_f[2 * VEC * (kBnSmallThreads + lpr)];
-  __shared__ double s_d[kBnSmallThreads], s_sum[2 * lpr * VEC];
-  __shared__ float s_mean[lpr * VEC], s_is[lpr * VEC];
-  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
-  const int c0 = ((int)blockIdx.x * lpr + cl) * VEC;         // first channel of the thread
-  const bool ok = c0 < C;
-  if (batches_tracked != nullptr && blockIdx.x == 0 && tid == 0) *batches_tracked += 1;
-  float s1[VEC], s2[VEC];
-#pragma unroll
-  for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
-  if (ok) {
-    const V k = *(const V*)(x + c0);
-    for (int r = rl; r < rows; r += 4 * rpp) {               // (rows past the end repeat row 0, as in bn_stats_kernel)
-      V a[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) a[u] = *(const V*)(x + (r + u * rpp < rows ? (int64_t)(r + u * rpp) * C : 0) + c0);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          const float d = to_f32(a[u].v[v]) - to_f32(k.v[v]);
-          s1[v] += d;
-          s2[v] += d * d;
-        }
-    }
+// partial[range][kind][channel] of the workgroup's channels added over the ranges, in their order by segments
+template <int VEC, int LANES>
+__device__ __forceinline__ void bn_slab_fold(const double* __restrict__ partial, int ranges, int C, double* s_d, double* s_out) {
+  constexpr int width = LANES * VEC, sums = 2 * width, segments = kBnSlabThreads / sums;
+  const int tid = threadIdx.x, j = tid % sums, seg = tid / sums;
+  const int kind = j / width, c = (int)blockIdx.x * width + j % width;
+  double a = 0.0;
+  if (c < C)
+    for (int i = seg; i < ranges; i += segments) a += partial[((int64_t)i * 2 + kind) * C + c];
+  s_d[tid] = a;
+  __syncthreads();
+  if (tid < sums) {
+    double t = 0.0;
+    for (int i = 0; i < min(ranges, segments); ++i) t += s_d[i * sums + tid];
+    s_out[tid] = t;
   }
-  bn_small_sums<VEC>(s1, s2, s_f, s_d, s_sum);
-  if (tid < lpr * VEC) {
-    const int c = (int)blockIdx.x * lpr * VEC + tid;
-    if (c < C) {
-      const double m = s_sum[tid] / (double)rows;
-      const double va = fmax(s_sum[lpr * VEC + tid] / (double)rows - m * m, 0.0);
-      const float mf = (float)((double)to_f32(x[c]) + m), isf = (float)(1.0 / sqrt(va + (double)eps));
-      s_mean[tid] = mean[c] = mf;
-      s_is[tid] = invstd[c] = isf;
-      var[c] = (float)va;
-      if (running_mean) {
+  __syncthreads();
+}
+
+// sums of the rows r0 .. r1 - 1, shifted by row 0 (whose shifted value, 0, stands in for rows past the end)
+template <typename T, int VEC, int LANES>
+__device__ __forceinline__ void bn_slab_rows(const T* __restrict__ x, int r0, int r1, int C, int c0, float (&s1)[VEC], float (&s2)[VEC]) {
+  typedef BnVec<T, VEC> V;
+  constexpr int rpp = kBnSlabThreads / LANES;
+  const V k = *(const V*)(x + c0);
+  for (int r = r0 + (int)threadIdx.x / LANES; r < r1; r += 4 * rpp) {
+    V a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[u] = *(const V*)(x + (r + u * rpp < r1 ? (int64_t)(r + u * rpp) * C : 0) + c0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        const float d = to_f32(a[u].v[v]) - to_f32(k.v[v]);
+        s1[v] += d;
+        s2[v] += d * d;
+      }
+  }
+}
+
+struct BnStats {                 // where a training pass leaves its statistics
+  float eps;
+  float *mean, *var, *invstd;
+  void *running_mean, *running_var;
+  int rdtype;
+  float factor;
+  long long* batches_tracked;
+};
+
+// mean and 1 / sqrt(var + eps) of the workgroup's channels to LDS; `keep`: also to where they are kept
+template <typename T, int VEC, int LANES>
+__device__ __forceinline__ void bn_slab_finish(const double* s_sum, const T* __restrict__ x, int rows, int C, const BnStats& st,
+                                               bool keep, float* s_mean, float* s_is) {
+  constexpr int width = LANES * VEC;
+  const int tid = threadIdx.x, c = (int)blockIdx.x * width + tid;
+  if (keep && st.batches_tracked != nullptr && blockIdx.x == 0 && tid == 0) *st.batches_tracked += 1;
+  if (tid < width && c < C) {
+    const double m = s_sum[tid] / (double)rows;
+    const double va = fmax(s_sum[width + tid] / (double)rows - m * m, 0.0);
+    const float mf = (float)((double)to_f32(x[c]) + m), isf = (float)(1.0 / sqrt(va + (double)st.eps));
+    s_mean[tid] = mf;
+    s_is[tid] = isf;
+    if (keep) {
+      st.mean[c] = mf;
+      st.invstd[c] = isf;
+      st.var[c] = (float)va;
+      if (st.running_mean) {
         const float unbiased = (float)(va * ((double)rows / (double)max(rows - 1, 1)));
-        bn_store(running_mean, rdtype, c, (1.f - factor) * bn_param(running_mean, rdtype, c, 0.f) + factor * mf);
-        bn_store(running_var, rdtype, c, (1.f - factor) * bn_param(running_var, rdtype, c, 0.f) + factor * unbiased);
+        bn_store(st.running_mean, st.rdtype, c, (1.f - st.factor) * bn_param(st.running_mean, st.rdtype, c, 0.f) + st.factor * mf);
+        bn_store(st.running_var, st.rdtype, c, (1.f - st.factor) * bn_param(st.running_var, st.rdtype, c, 0.f) + st.factor * unbiased);
       }
     }
   }
   __syncthreads();
-  if (!ok) return;
-  float m[VEC], sc[VEC], be[VEC];
-  bn_params<VEC>(gamma, beta, pdtype, c0, sc, be);
-#pragma unroll
-  for (int v = 0; v < VEC; ++v) {
-    m[v] = s_mean[cl * VEC + v];
-    sc[v] = s_is[cl * VEC + v] * sc[v];
-  }
-  for (int r = rl; r < rows; r += 4 * rpp) {
-    V a[4], b[4];
+}
+
+// four rows of a thread from row r on (those below r1), requested and normalised
+template <typename T, int VEC, int LANES> struct BnRows {
+  static constexpr int kPass = kBnSlabThreads / LANES;
+  BnVec<T, VEC> a[4], b[4];
+  __device__ __forceinline__ void load(const T* __restrict__ x, const T* __restrict__ res, int r, int r1, int C, int c0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int64_t at = (int64_t)(r + u * rpp) * C + c0;
-      if (r + u * rpp < rows) {
-        a[u] = *(const V*)(x + at);
-        if (res) b[u] = *(const V*)(res + at);
+      const int64_t at = (int64_t)(r + u * kPass) * C + c0;
+      if (r + u * kPass < r1) {
+        a[u] = *(const BnVec<T, VEC>*)(x + at);
+        if (res) b[u] = *(const BnVec<T, VEC>*)(res + at);
       }
     }
+  }
+  __device__ __forceinline__ void apply(const float (&m)[VEC], const float (&sc)[VEC], const float (&be)[VEC], bool with, int relu,
+                                        T* __restrict__ y, int r, int r1, int C, int c0) const {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      if (r + u * rpp >= rows) continue;
-      V o;
+      if (r + u * kPass >= r1) continue;
+      BnVec<T, VEC> o;
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
         float t = (to_f32(a[u].v[v]) - m[v]) * sc[v] + be[v];
-        if (res) t = to_f32(from_f32<T>(t)) + to_f32(b[u].v[v]);
+        if (with) t = to_f32(from_f32<T>(t)) + to_f32(b[u].v[v]);
         if (relu) t = fmaxf(t, 0.f);
         o.v[v] = from_f32<T>(t);
       }
-      *(V*)(y + (int64_t)(r + u * rpp) * C + c0) = o;
+      *(BnVec<T, VEC>*)(y + (int64_t)(r + u * kPass) * C + c0) = o;
+    }
+  }
+};
+
+// ranges = 1, partial null: the whole batch norm.  SUMS: the sums of range blockIdx.y alone, to partial.  Else: rows of range
+// blockIdx.y (of `per`) with the sums of `ranges` ranges.
+template <typename T, int VEC, int LANES, bool SUMS>
+__global__ __launch_bounds__(kBnSlabThreads) void bn_slab_kernel(
+    const T* __restrict__ x, int rows, int C, int per, double* __restrict__ partial, int ranges, BnStats st,
+    const void* __restrict__ gamma, const void* __restrict__ beta, int pdtype, int relu, const T* __restrict__ res,
+    T* __restrict__ y) {
+  constexpr int lpr = LANES, rpp = kBnSlabThreads / LANES, width = lpr * VEC;
+  __shared__ float s_f[2 * VEC * (kBnSlabThreads + lpr)];
+  __shared__ double s_d[kBnSlabThreads], s_sum[2 * width];
+  __shared__ float s_mean[width], s_is[width];
+  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
+  const int c0 = (int)blockIdx.x * width + cl * VEC;         // first channel of the thread
+  const bool ok = c0 < C;
+  const int r0 = (int)blockIdx.y * per, r1 = min(rows, r0 + per);
+  BnRows<T, VEC, LANES> first;
+  if (!SUMS && partial != nullptr) {
+    if (ok) first.load(x, res, r0 + rl, r1, C, c0);          // (on their way under the sums)
+    bn_slab_fold<VEC, LANES>(partial, ranges, C, s_d, s_sum);
+  } else {
+    float s1[VEC], s2[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
+    if (ok) bn_slab_rows<T, VEC, LANES>(x, r0, r1, C, c0, s1, s2);
+    bn_slab_sums<VEC, LANES>(s1, s2, s_f, s_d, s_sum);
+  }
+  if constexpr (SUMS) {
+    const int c = (int)blockIdx.x * width + tid % width;
+    if (tid < 2 * width && c < C) partial[((int64_t)blockIdx.y * 2 + tid / width) * C + c] = s_sum[tid];
+  } else {
+    bn_slab_finish<T, VEC, LANES>(s_sum, x, rows, C, st, blockIdx.y == 0, s_mean, s_is);
+    if (!ok) return;
+    float m[VEC], sc[VEC], be[VEC];
+    bn_params<VEC>(gamma, beta, pdtype, c0, sc, be);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      m[v] = s_mean[cl * VEC + v];
+      sc[v] = s_is[cl * VEC + v] * sc[v];
+    }
+    for (int r = r0 + rl; r < r1; r += 4 * rpp) {
+      if (partial == nullptr || r != r0 + rl) first.load(x, res, r, r1, C, c0);
+      first.apply(m, sc, be, res != nullptr, relu, y, r, r1, C, c0);
     }
   }
 }
 
-// the gradient, as bn_bwd_stats_kernel, bn_bwd_finish_kernel and bn_bwd_apply_kernel after each other
-template <typename T, int VEC>
-__global__ __launch_bounds__(kBnSmallThreads) void bn_bwd_small_kernel(
-    const T* __restrict__ x, const T* __restrict__ dy, int rows, int C, const float* __restrict__ mean,
-    const float* __restrict__ invstd, const void* __restrict__ gamma, const void* __restrict__ beta, int pdtype, int relu,
-    int training, const T* __restrict__ ymask, float* __restrict__ dbeta, float* __restrict__ dgamma, void* gw, void* gb,
-    T* __restrict__ dres, T* __restrict__ dx) {
-  typedef BnVec<T, VEC> V;
-  constexpr int lpr = kBnSmallLanes, rpp = kBnSmallThreads / lpr;
-  __shared__ float s_f[2 * VEC * (kBnSmallThreads + lpr)];
-  __shared__ double s_d[kBnSmallThreads], s_sum[2 * lpr * VEC];
-  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
-  const int c0 = ((int)blockIdx.x * lpr + cl) * VEC;
-  const bool ok = c0 < C;
-  float s1[VEC], s2[VEC], m[VEC], is[VEC], ga[VEC], be[VEC];
+// two rows of a thread, for the gradient: x, dy and the forward output where it is the mask
+template <typename T, int VEC, int LANES> struct BnBwdRows {
+  static constexpr int kPass = kBnSlabThreads / LANES;
+  BnVec<T, VEC> a[2], g[2], ym[2];
+  __device__ __forceinline__ void load(const T* __restrict__ x, const T* __restrict__ dy, const T* __restrict__ ymask, int r,
+                                       int r1, int C, int c0) {
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
+    for (int u = 0; u < 2; ++u) {
+      const int64_t at = (r + u * kPass < r1 ? (int64_t)(r + u * kPass) * C : 0) + c0;   // (past the end: row 0)
+      a[u] = *(const BnVec<T, VEC>*)(x + at);
+      g[u] = *(const BnVec<T, VEC>*)(dy + at);
+      ym[u] = a[u];                                          // (defined without a mask, too)
+      if (ymask) ym[u] = *(const BnVec<T, VEC>*)(ymask + at);
+    }
+  }
+};
+
+// the gradient, as bn_bwd_stats_kernel, bn_bwd_finish_kernel and bn_bwd_apply_kernel after each other; ranges, partial and
+// SUMS as in bn_slab_kernel
+template <typename T, int VEC, int LANES, bool SUMS>
+__global__ __launch_bounds__(kBnSlabThreads) void bn_bwd_slab_kernel(
+    const T* __restrict__ x, const T* __restrict__ dy, int rows, int C, int per, double* __restrict__ partial, int ranges,
+    const float* __restrict__ mean, const float* __restrict__ invstd, const void* __restrict__ gamma,
+    const void* __restrict__ beta, int pdtype, int relu, int training, const T* __restrict__ ymask, float* __restrict__ dbeta,
+    float* __restrict__ dgamma, void* gw, void* gb, T* __restrict__ dres, T* __restrict__ dx) {
+  typedef BnVec<T, VEC> V;
+  constexpr int lpr = LANES, rpp = kBnSlabThreads / LANES, width = lpr * VEC;
+  __shared__ float s_f[2 * VEC * (kBnSlabThreads + lpr)];
+  __shared__ double s_d[kBnSlabThreads], s_sum[2 * width];
+  const int tid = threadIdx.x, cl = tid % lpr, rl = tid / lpr;
+  const int c0 = (int)blockIdx.x * width + cl * VEC;
+  const bool ok = c0 < C;
+  const int r0 = (int)blockIdx.y * per, r1 = min(rows, r0 + per);
+  float m[VEC], is[VEC], ga[VEC], be[VEC];
+  BnBwdRows<T, VEC, LANES> v2;
   if (ok) {
+    if (!SUMS && partial != nullptr) v2.load(x, dy, ymask, r0 + rl, r1, C, c0);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
       m[v] = mean[c0 + v];
       is[v] = invstd[c0 + v];
     }
     bn_params<VEC>(gamma, beta, pdtype, c0, ga, be);
-    for (int r = rl; r < rows; r += 2 * rpp) {
-      V a[2], g[2], ym[2];
-      bool in[2];
+  }
+  // dy' of a value: dy where the forward output was positive (or without the ReLU)
+  auto passed = [&](int u, int v, float xc, float scale) {
+    const float seen = ymask ? to_f32(v2.ym[u].v[v]) : xc * scale + be[v];
+    const bool on = !relu || seen > 0.f;
+    return on ? to_f32(v2.g[u].v[v]) : 0.f;
+  };
+  if (!SUMS && partial != nullptr) {
+    bn_slab_fold<VEC, LANES>(partial, ranges, C, s_d, s_sum);
+  } else {
+    float s1[VEC], s2[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) s1[v] = s2[v] = 0.f;
+    if (ok)
+      for (int r = r0 + rl; r < r1; r += 2 * rpp) {
+        v2.load(x, dy, ymask, r, r1, C, c0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) {
+            const float xc = to_f32(v2.a[u].v[v]) - m[v];
+            const float xh = xc * is[v];
+            const float d = r + u * rpp < r1 ? passed(u, v, xc, is[v] * ga[v]) : 0.f;
+            s1[v] += d;
+            s2[v] += d * xh;
+          }
+      }
+    bn_slab_sums<VEC, LANES>(s1, s2, s_f, s_d, s_sum);
+  }
+  if constexpr (SUMS) {
+    const int c = (int)blockIdx.x * width + tid % width;
+    if (tid < 2 * width && c < C) partial[((int64_t)blockIdx.y * 2 + tid / width) * C + c] = s_sum[tid];
+  } else {
+    if (tid < width && blockIdx.y == 0) {
+      const int c = (int)blockIdx.x * width + tid;
+      if (c < C) {
+        const float a = (float)s_sum[tid], b = (float)s_sum[width + tid];
+        dbeta[c] = a;
+        dgamma[c] = b;
+        if (gw) bn_store(gw, pdtype, c, b);
+        if (gb) bn_store(gb, pdtype, c, a);
+      }
+    }
+    if (!ok) return;
+    const float inv_n = 1.0f / (float)rows;
+    float db[VEC], dg[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      db[v] = training ? (float)s_sum[cl * VEC + v] * inv_n : 0.f;
+      dg[v] = training ? (float)s_sum[width + cl * VEC + v] * inv_n : 0.f;
+      ga[v] *= is[v];
+    }
+    for (int r = r0 + rl; r < r1; r += 2 * rpp) {
+      if (partial == nullptr || r != r0 + rl) v2.load(x, dy, ymask, r, r1, C, c0);
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        in[u] = r + u * rpp < rows;
-        const int64_t at = (in[u] ? (int64_t)(r + u * rpp) * C : 0) + c0;
-        a[u] = *(const V*)(x + at);
-        g[u] = *(const V*)(dy + at);
-        if (ymask) ym[u] = *(const V*)(ymask + at);
-      }
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
+        if (r + u * rpp >= r1) continue;
+        const int64_t at = (int64_t)(r + u * rpp) * C + c0;
+        V o, gr;
 #pragma unroll
         for (int v = 0; v < VEC; ++v) {
-          const float xc = to_f32(a[u].v[v]) - m[v];
-          const float xh = xc * is[v];
-          float d = in[u] ? to_f32(g[u].v[v]) : 0.f;
-          if (relu && !(ymask ? to_f32(ym[u].v[v]) > 0.f : xc * (is[v] * ga[v]) + be[v] > 0.f)) d = 0.f;
-          s1[v] += d;
-          s2[v] += d * xh;
+          const float xc = to_f32(v2.a[u].v[v]) - m[v];
+          float d = passed(u, v, xc, ga[v]);
+          gr.v[v] = from_f32<T>(d);
+          if (training) d = d - db[v] - (xc * is[v]) * dg[v];
+          o.v[v] = from_f32<T>(d * ga[v]);
         }
-    }
-  }
-  bn_small_sums<VEC>(s1, s2, s_f, s_d, s_sum);
-  if (tid < lpr * VEC) {
-    const int c = (int)blockIdx.x * lpr * VEC + tid;
-    if (c < C) {
-      const float a = (float)s_sum[tid], b = (float)s_sum[lpr * VEC + tid];
-      dbeta[c] = a;
-      dgamma[c] = b;
-      if (gw) bn_store(gw, pdtype, c, b);
-      if (gb) bn_store(gb, pdtype, c, a);
-    }
-  }
-  if (!ok) return;
-  const float inv_n = 1.0f / (float)rows;
-  float db[VEC], dg[VEC];
-#pragma unroll
-  for (int v = 0; v < VEC; ++v) {
-    db[v] = training ? (float)s_sum[cl * VEC + v] * inv_n : 0.f;
-    dg[v] = training ? (float)s_sum[(lpr + cl) * VEC + v] * inv_n : 0.f;
-    ga[v] *= is[v];
-  }
-  for (int r = rl; r < rows; r += 2 * rpp) {
-    V a[2], g[2], ym[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int64_t at = (int64_t)(r + u * rpp) * C + c0;
-      if (r + u * rpp < rows) {
-        a[u] = *(const V*)(x + at);
-        g[u] = *(const V*)(dy + at);
-        if (ymask) ym[u] = *(const V*)(ymask + at);
+        *(V*)(dx + at) = o;
+        if (dres) *(V*)(dres + at) = gr;
       }
     }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (r + u * rpp >= rows) continue;
-      const int64_t at = (int64_t)(r + u * rpp) * C + c0;
-      V o, gr;
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) {
-        const float xc = to_f32(a[u].v[v]) - m[v];
-        float d = to_f32(g[u].v[v]);
-        if (relu && !(ymask ? to_f32(ym[u].v[v]) > 0.f : xc * ga[v] + be[v] > 0.f)) d = 0.f;
-        gr.v[v] = from_f32<T>(d);
-        if (training) d = d - db[v] - (xc * is[v]) * dg[v];
-        o.v[v] = from_f32<T>(d * ga[v]);
-      }
-      *(V*)(dx + at) = o;
-      if (dres) *(V*)(dres + at) = gr;
-    }
   }
+}
+
+// How a pass is launched: LANES and, for two launches, the rows of a workgroup of the sums (a range) and of one of the
+// elementwise pass: whole passes, as few as give every CU a workgroup, `unroll` of them at most.
+struct BnSlabs {
+  int lanes, slabs, sums_per, ranges, per, parts;
+  bool split;                    // two launches
+};
+static BnSlabs bn_slabs(int dtype, int64_t rows, int channels, int unroll) {
+  BnSlabs s;
+  const int vec = dtype == OCNN_F32 ? 4 : 8;
+  s.split = rows > kBnSmallRows;
+  s.lanes = s.split && rows * channels * 16 / vec >= (dtype == OCNN_F32 ? kBnWideF32 : kBnWide16) ? 8 : 4;
+  s.slabs = (int)cdiv(channels, s.lanes * vec);
+  if (!s.split) {
+    s.sums_per = s.per = (int)rows;
+    s.ranges = s.parts = 1;
+    return s;
+  }
+  const int64_t pass = kBnSlabThreads / s.lanes;
+  const int64_t some = std::min<int64_t>(unroll, std::max<int64_t>(1, cdiv(rows * s.slabs, 256 * pass))) * pass;
+  s.sums_per = (int)std::max(some, align_up(cdiv(rows, std::max(kBnSlabRanges, 256 / s.slabs)), pass));
+  s.ranges = (int)cdiv(rows, s.sums_per);
+  s.per = (int)some;
+  s.parts = (int)cdiv(rows, s.per);
+  return s;
+}
+
+// (three launches for more than these)
+static bool bn_slabs_take(int dtype, int64_t rows, int channels, bool backward) {
+  const int64_t limit = backward ? kBnSlabBackward : kBnSlabForward;
+  if (rows <= kBnSmallRows) return true;
+  if (rows > kBnSlabRows || channels < (dtype == OCNN_F32 ? 16 : 32)) return false;
+  // 128 bytes are 64 channels of 16 bits: where they leave half a slab empty, or (backward) are the whole row, no further than
+  // 64 bytes are good for (130 k x 96 forward 31.6, three launches 28.8; 130 k x 64 backward 39.1, 35.6)
+  const bool narrow = dtype != OCNN_F32 && (channels % 64 != 0 || (backward && channels == 64));
+  return rows * channels * (dtype == OCNN_F32 ? 4 : 2) <= (narrow ? std::min(limit, kBnWide16 - 1) : limit);
 }
 
 }  // namespace ocnn
@@ -739,19 +873,25 @@ extern "C" int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows,
                                          void* workspace, int64_t workspace_bytes, void* stream) {
   OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_training: shape not supported");
   OCNN_REQUIRE_PTRS("batch_norm_training", x, mean, var, invstd, y, workspace);
-  if (rows > kBnSmallRows) {
+  OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels), "batch_norm_training: workspace too small");
+  if (!bn_slabs_take(dtype, rows, channels, false)) {
     const int status = ocnn_batch_norm_stats(dtype, x, rows, channels, eps, mean, var, invstd, running_mean, running_var,
                                              running_dtype, factor, batches_tracked, workspace, workspace_bytes, stream);
     if (status != OCNN_OK) return status;
     return bn_apply(dtype, x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, residual, y, nullptr, nullptr,
                     0, 0.f, (hipStream_t)stream);
   }
+  const BnStats keep{eps, mean, var, invstd, running_mean, running_var, running_dtype, factor, (long long*)batches_tracked};
+  const BnSlabs s = bn_slabs(dtype, rows, channels, 4);
+  double* partial = s.split ? (double*)workspace : nullptr;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
-    hipLaunchKernelGGL((bn_small_kernel<T, VEC>), dim3((unsigned)cdiv(channels, kBnSmallLanes * VEC)), dim3(kBnSmallThreads), 0,
-                       (hipStream_t)stream, (const T*)x, (int)rows, channels, eps, mean, var, invstd, running_mean,
-                       running_var, running_dtype, factor, (long long*)batches_tracked, gamma, beta, param_dtype, relu,
-                       (const T*)residual, (T*)y);
+    auto launch = [&](auto kernel, int parts, int per) {
+      hipLaunchKernelGGL(kernel, dim3(s.slabs, parts), dim3(kBnSlabThreads), 0, (hipStream_t)stream, (const T*)x, (int)rows, channels,
+                         per, partial, s.ranges, keep, gamma, beta, param_dtype, relu, (const T*)residual, (T*)y);
+    };
+    if (s.split) launch(s.lanes == 8 ? bn_slab_kernel<T, VEC, 8, true> : bn_slab_kernel<T, VEC, 4, true>, s.ranges, s.sums_per);
+    launch(s.lanes == 8 ? bn_slab_kernel<T, VEC, 8, false> : bn_slab_kernel<T, VEC, 4, false>, s.parts, s.per);
   });
   return check_launch("batch_norm_training");
 }
@@ -778,13 +918,18 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
   OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels),
                "batch_norm_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
-  if (dx && rows <= kBnSmallRows) {
+  if (dx && bn_slabs_take(dtype, rows, channels, true)) {
+    const BnSlabs s = bn_slabs(dtype, rows, channels, 2);
+    double* partial = s.split ? (double*)workspace : nullptr;
     OCNN_DISPATCH_DTYPE(dtype, {
       constexpr int VEC = 16 / sizeof(T);
-      hipLaunchKernelGGL((bn_bwd_small_kernel<T, VEC>), dim3((unsigned)cdiv(channels, kBnSmallLanes * VEC)), dim3(kBnSmallThreads),
-                         0, st, (const T*)x, (const T*)dy, (int)rows, channels, mean, invstd, gamma, beta,
-                         param_dtype, relu, training, (const T*)y, dbeta, dgamma, grad_gamma, grad_beta, (T*)d_residual,
-                         (T*)dx);
+      auto launch = [&](auto kernel, int parts, int per) {
+        hipLaunchKernelGGL(kernel, dim3(s.slabs, parts), dim3(kBnSlabThreads), 0, st, (const T*)x, (const T*)dy, (int)rows, channels,
+                           per, partial, s.ranges, mean, invstd, gamma, beta, param_dtype, relu, training, (const T*)y, dbeta,
+                           dgamma, grad_gamma, grad_beta, (T*)d_residual, (T*)dx);
+      };
+      if (s.split) launch(s.lanes == 8 ? bn_bwd_slab_kernel<T, VEC, 8, true> : bn_bwd_slab_kernel<T, VEC, 4, true>, s.ranges, s.sums_per);
+      launch(s.lanes == 8 ? bn_bwd_slab_kernel<T, VEC, 8, false> : bn_bwd_slab_kernel<T, VEC, 4, false>, s.parts, s.per);
     });
     return check_launch("batch_norm_backward");
   }

@@ -357,9 +357,12 @@ def test_random_batch_norms_vs_torch():
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
 def test_batch_norm_few_rows(dtype):
-  """The one-launch kernels at the edges of their range (up to 2048 rows; channels that fill no whole
-  workgroup) and the passes of their own just above it, against fp64."""
-  for rows, c in [(33, 8), (64, 32), (255, 40), (256, 1024), (1023, 24), (2048, 96), (2049, 96)]:
+  """The kernels for few rows, against fp64: one launch and two at the line between them, channels that fill no whole
+  workgroup, 64 and 128 bytes of a row, the last sizes that two launches take and the first of three."""
+  sizes = [(33, 8), (64, 32), (255, 40), (256, 1024), (1023, 24), (2048, 96), (2049, 96), (1024, 40), (1025, 40), (1025, 8), (2500, 1000),
+           (8192, 128), (8193, 128), (131072, 32), (131073, 32)]
+  sizes += [(70000, 72)] if dtype == torch.float32 else [(65536, 96), (65535, 96), (98304, 64)]
+  for rows, c in sizes:
     say('batch norm, few rows', dtype, rows, c)
     g = torch.Generator().manual_seed(rows)
     x = (torch.randn(rows, c, generator=g) + 3.0).to(dtype)
