@@ -48,23 +48,35 @@ static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char*
 // SKIP: per slot and 32-row block of the tile a wave asks whether any row has an entry there (a
 // ballot over the positions it reads anyway) and leaves the block's MFMAs out otherwise.  Blocks are the outer
 // loop of a slot, so that one branch stands around a block's 4 - 18 MFMAs: with the k-steps outside and a branch
-// per MFMA the same tables took 6 - 10 % longer.  The reads are not in the branch (they run a block ahead).
+// per MFMA the same tables took 6 - 10 % longer.  The rows of a block are read one block ahead, behind a branch of their own.
+//
+// order: the tile's rows in an order that leaves fewer blocks with an entry (plan.hip: tile_order_kernel); position i of
+// a block is row order[i].  It costs the loop nothing (a lane's row is a register either way) and the sums of a row are the
+// same, but which wave adds those of its block.  What bounds the loop on such tables is neither MFMAs nor bytes alone: 96 -> 96 on the
+// 1.13 M rows of depth 9, 7 % set, 334 us: 139 without any slot (rows, results and the chain of loads in front), 280 with a
+// quarter of the MFMAs, 290 with one fetch of weights a chunk.  A turn of the loop therefore waits for as little as can be: two sets
+// of registers in turn in place of copies, the blocks that are live known beforehand (334 -> 320 us), half the weights of
+// half a chunk, and 0.24 instead of 0.39 of the blocks by the order (298).  In us before / now, f16: 947 k rows 15 % set
+// 96 -> 96 329 / 303, 533 k 31 % 128 -> 128 299 / 274, 160 k 38 % 256 -> 256 383 / 349, 40 k 42 % 155 / 144, 822 k 14 % 96 -> 96
+// 333 / 294, nine slots of 1.13 M rows 234 / 215; fp32 132 k 36 % 96 -> 96 153 / 143, 264 k 22 % 64 -> 64 132 / 130, 19 k 128 -> 128
+// 60 / 59.  (Tables above the line below gain where a cloud is flat, 1.28 M rows 68 % set 96 -> 96 620 / 576, and lose elsewhere,
+// 97 k 52 % 256 -> 256 282 / 292: they stay without.)
 //
 // The four waves: WC along the output channels (32 MB each), WR along the rows (RB = 4 / WR blocks of 32 rows
 // each), KS over the slots (each takes every KS-th; their sums are added in LDS at the end).
 template <typename T, bool F32, int MB, int WC, int WR, int KS, bool SKIP>
 __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_tile_kernel(
     const void* __restrict__ in, uint32_t in_bytes, const uint16_t* __restrict__ loc,
-    const int32_t* __restrict__ uptr, const int32_t* __restrict__ urows, const T* __restrict__ wpk,
-    const void* __restrict__ bias_, ocnnx_bn bn, void* __restrict__ out_, float* __restrict__ partial,
+    const int32_t* __restrict__ uptr, const int32_t* __restrict__ urows, const uint8_t* __restrict__ order,
+    const T* __restrict__ wpk, const void* __restrict__ bias_, ocnnx_bn bn, void* __restrict__ out_, float* __restrict__ partial,
     int64_t rows_out, int K, int cin, int cout, int64_t tiles, int64_t tiles_per_xcd, int sc, int sk, int rows_alloc) {
   typedef typename std::conditional<F32, float, T>::type O;
   constexpr int RB = 4 / WR, RBK = RB / KS, CH = F32 ? 32 : 64;
-  static_assert(WC * WR * KS == 4 && RB % KS == 0, "four waves");
+  static_assert(WC * WR * KS == 4 && RB % KS == 0 && RB % 2 == 0, "four waves; blocks in pairs");
   extern __shared__ __attribute__((aligned(16))) char s_rows[];    // rows_alloc rows, positions, the list
   uint16_t* s_loc = (uint16_t*)(s_rows + rows_alloc * 128);
   int32_t* s_u = (int32_t*)(s_loc + ((K + sk - 1) / sk) * kTgRows);
-  uint32_t* s_live = (uint32_t*)(s_u + rows_alloc);                // slots with entries: of rows 0 - 63, 64 - 127 (bits)
+  uint32_t* s_live = (uint32_t*)(s_u + rows_alloc);                // of a slot: its 32-row blocks with an entry (bits)
 
   const int64_t tile = tiles_per_xcd > 0 ? xcd_tile(blockIdx.x, tiles_per_xcd) : (int64_t)blockIdx.x;
   if (tile >= tiles) return;
@@ -118,37 +130,37 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
 
   // ---- operands ----
   // A: the weights of a (chunk, slot), four pieces of 16 bytes a lane and M tile
-  const int64_t kstride = (int64_t)ncg * 2048;               // elements between consecutive (chunk, slot)
+  const uint32_t kstride = (uint32_t)ncg * 4096u;            // bytes between consecutive (chunk, slot)
   const bool active = cg0 < ncg;                             // (wave-uniform)
-  const T* wbase[MB];
+  auto load_a = [&](int kk, u32x4 (&a)[4][MB], auto STEPS) {
+    const char* base = (const char*)wpk + (uint64_t)((uint32_t)kk * kstride);
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) wbase[mb] = wpk + lane * 8 + (int64_t)min(cg0 + mb, ncg - 1) * 2048;
-  auto load_a = [&](int kk, u32x4 (&a)[4][MB]) {
+    for (int mb = 0; mb < MB; ++mb) {
+      const char* tile_of = base + (uint32_t)min(cg0 + mb, ncg - 1) * 4096u;   // (uniform: the lanes differ in a 32-bit offset)
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) a[s][mb] = *(const u32x4*)(wbase[mb] + (int64_t)kk * kstride + s * 512);
-  };
-  // B: a lane reads 16 bytes (8 input channels, or their high or low pieces) of the neighbour row of
-  // row 32 rb + r32.  pv = byte address of the row in s_rows with the swizzle of piece 0 folded in.
-  const uint16_t* lcw = s_loc + 32 * RB * wr + r32;
-  uint32_t pvc[RB], pvn[RB];
-  // (SKIP) which 32-row blocks of the tile have an entry in the slot at all, wave-uniform
-  bool nzc[RB], nzn[RB];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) nzc[rb] = nzn[rb] = true;
-  auto load_pos = [&](int k, uint32_t (&pv)[RB], bool (&nz)[RB]) {
-    const uint16_t* p = lcw + (k - k0) * kTgRows;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const uint32_t l = p[32 * rb];                         // 0 = empty = the zero row
-      pv[rb] = (l << 7) | (((l << 3) & 0x70u) ^ ((uint32_t)q << 4));
-      if constexpr (SKIP) nz[rb] = __builtin_amdgcn_ballot_w64(l != 0u) != 0ull;
+      for (int s = 0; s < decltype(STEPS)::value; ++s) a[s][mb] = *(const u32x4*)(tile_of + (uint32_t)(lane * 16 + s * 1024));
     }
   };
-  auto read_b = [&](uint32_t pv, u32x4 (&b)[4]) {
+  // B: a lane reads 16 bytes (8 input channels, or their high or low pieces) of the neighbour row of
+  // one of the tile's rows, row at[rb] in block rb.  pv = byte address of the row in s_rows with the swizzle of piece 0 folded in.
+  int at[RB];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) b[s] = *(const u32x4*)(s_rows + (pv ^ ((uint32_t)s << 5)));
+  for (int rb = 0; rb < RB; ++rb) {
+    at[rb] = 32 * (RB * wr + rb) + r32;
+    if constexpr (SKIP)
+      if (order) at[rb] = order[tile * kTgRows + at[rb]];
+  }
+  auto load_pos = [&](int k, uint32_t (&pv)[RB]) {
+    const uint16_t* p = s_loc + (k - k0) * kTgRows;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const uint32_t l = p[at[rb]];                          // 0 = empty = the zero row
+      pv[rb] = (l << 7) | (((l << 3) & 0x70u) ^ ((uint32_t)q << 4));
+    }
+  };
+  auto read_b = [&](uint32_t pv, u32x4 (&b)[4], auto STEPS) {
+#pragma unroll
+    for (int s = 0; s < decltype(STEPS)::value; ++s) b[s] = *(const u32x4*)(s_rows + (pv ^ ((uint32_t)s << 5)));
   };
   // a block of 32 rows with everything of a slot: behind one branch
   auto multiply = [&](const u32x4 (&a)[4][MB], const u32x4 (&b)[4], f32x16 (&c)[MB], auto STEPS) {
@@ -230,21 +242,24 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   // (A slot without any costs the weights' way through L1, the busiest unit with 46 - 62 % on such tables, and a turn of the
   // loop.  Indoor scenes, non-empty nodes: 47 % of a tile's slots at depth 9, 1.13 M rows 96 -> 96 423 us, without them 323;
   // 37 % at depth 8, 947 k rows 380 / 327; 30 % at depth 7, 533 k rows 128 -> 128 332 / 317.)
-  uint32_t own = 0;
+  uint32_t own = 0, blocks = 0;                              // blocks, of lane k - k0: its 32-row blocks with an entry (bits)
   bool works = false;
   auto find_live = [&]() {
-    if constexpr (SKIP)
+    if constexpr (SKIP) {
+      const int a = order ? order[tile * kTgRows + lane] : lane, b = order ? order[tile * kTgRows + 64 + lane] : 64 + lane;
       for (int k = wave; k < k1 - k0; k += 4) {
-        const unsigned long long lo = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + lane] != 0);
-        const unsigned long long hi = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + 64 + lane] != 0);
-        if (lane == 0) s_live[k] = (lo ? 1u : 0u) | (hi ? 2u : 0u);
+        const unsigned long long lo = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + a] != 0);
+        const unsigned long long hi = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + b] != 0);
+        if (lane == 0)
+          s_live[k] = ((uint32_t)lo ? 1u : 0u) | (lo >> 32 ? 2u : 0u) | ((uint32_t)hi ? 4u : 0u) | (hi >> 32 ? 8u : 0u);
       }
+    }
   };
   auto deal_slots = [&]() {
     uint32_t live = (1u << (k1 - k0)) - 1u;
     if constexpr (SKIP) {
-      const uint32_t mine = WR == 2 ? 1u << wr : 3u;
-      live = (uint32_t)__builtin_amdgcn_ballot_w64(lane < k1 - k0 && (s_live[min(lane, k1 - k0 - 1)] & mine) != 0u);
+      if (lane < k1 - k0) blocks = (s_live[lane] >> (RB * wr)) & ((1u << RB) - 1u);
+      live = (uint32_t)__builtin_amdgcn_ballot_w64(blocks != 0u);
     }
     // (every KS-th slot whether or not it is live: the same sums as without SKIP, to the bit)
     own = live & ((KS == 4 ? 0x11111111u : (KS == 2 ? 0x55555555u : 0xffffffffu)) << ks);
@@ -252,43 +267,53 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
     if (own == 0u) own = 1u;                                 // (nothing to do: a turn without products)
   };
 
-  u32x4 A[4][MB], B[2][4];
-  auto fetch_slot = [&](int cc, int k, u32x4 (&a)[4][MB], uint32_t (&pv)[RB], bool (&nz)[RB]) {
-    load_pos(k, pv, nz);
-    load_a(cc * K + k, a);
+  // Two slots in hand: the one whose products run, with its weights A, positions and live blocks, and the next one's on
+  // their way.  (Two sets of names, in turn: the copies of one set into the other were 24 - 36 instructions a slot, and the
+  // blocks that have an entry are known from find_live, so that no branch waits for the positions.)
+  u32x4 A[2][4][MB], B[2][4];
+  uint32_t pv[2][RB], nz[2] = {~0u, ~0u};
+  auto fetch_slot = [&](int cc, int k, auto P, auto STEPS) {
+    constexpr int p = decltype(P)::value;
+    load_a(cc * K + k, A[p], STEPS);
+    load_pos(k, pv[p]);
+    if constexpr (SKIP) nz[p] = (uint32_t)__builtin_amdgcn_readlane((int)blocks, k - k0);
   };
-  // A and pvc, nzc hold the first slot's when a chunk begins
+  // set P holds the first slot's when a chunk begins (P = 0)
   auto chunk = [&](int cc, auto STEPS) {
-    read_b(pvc[0], B[0]);
-    {
-      uint32_t rest = own;
-      for (bool more = true; more; more = rest != 0u) {
-        rest &= rest - 1u;
-        // the next slot; behind the last one the first of the next chunk (of this one again behind the last chunk)
-        const int kn = k0 + __builtin_ctz(rest ? rest : own);
-        u32x4 An[4][MB];
-        fetch_slot(rest ? cc : min(cc + 1, c1 - 1), kn, An, pvn, nzn);
+    uint32_t rest = own;
+    auto slot = [&](auto P) {
+      constexpr int p = decltype(P)::value;
+      rest &= rest - 1u;
+      // the next slot; behind the last one the first of the next chunk (of this one again behind the last chunk)
+      const int kn = k0 + __builtin_ctz(rest ? rest : own);
+      fetch_slot(rest ? cc : min(cc + 1, c1 - 1), kn, std::integral_constant<int, 1 - p>{}, STEPS);
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          // (past the last slot: rows of this chunk, unused)
-          read_b(rb + 1 < RB ? pvc[rb + 1 < RB ? rb + 1 : 0] : pvn[0], B[(rb + 1) & 1]);
-          if (works && (!SKIP || nzc[rb])) multiply(A, B[rb & 1], acc[rb], STEPS);
-          __builtin_amdgcn_sched_barrier(0);
+      for (int rb = 0; rb < RB; ++rb) {
+        // the next block's rows (past the last slot: rows of this chunk, unused)
+        if (rb + 1 < RB) {
+          if (!SKIP || (nz[p] & (2u << rb))) read_b(pv[p][rb + 1 < RB ? rb + 1 : 0], B[(rb + 1) & 1], STEPS);
+        } else {
+          if (!SKIP || (nz[1 - p] & 1u)) read_b(pv[1 - p][0], B[0], STEPS);
         }
-        if constexpr (RB & 1) {
-#pragma unroll
-          for (int s = 0; s < 4; ++s) B[0][s] = B[1][s];
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int mb = 0; mb < MB; ++mb) A[s][mb] = An[s][mb];
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          pvc[rb] = pvn[rb];
-          if constexpr (SKIP) nzc[rb] = nzn[rb];
-        }
+        if (works && (!SKIP || (nz[p] & (1u << rb)))) multiply(A[p], B[rb & 1], acc[rb], STEPS);
+        __builtin_amdgcn_sched_barrier(0);
       }
+    };
+    read_b(pv[0][0], B[0], STEPS);
+    for (;;) {
+      slot(std::integral_constant<int, 0>{});
+      if (rest == 0u) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) A[0][s][mb] = A[1][s][mb];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) pv[0][rb] = pv[1][rb];
+        nz[0] = nz[1];
+        break;
+      }
+      slot(std::integral_constant<int, 1>{});
+      if (rest == 0u) break;
     }
   };
   find_live();
@@ -296,7 +321,7 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
     stage_chunk(cc, [&]() {
       if (cc == c0) {                                        // (the first weights come beside the rows)
         deal_slots();
-        fetch_slot(c0, k0 + __builtin_ctz(own), A, pvc, nzc);
+        fetch_slot(c0, k0 + __builtin_ctz(own), std::integral_constant<int, 0>{}, STEPS);
       }
     });
     chunk(cc, STEPS);
@@ -353,7 +378,7 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         if (KS > 1 && rb / RBK != ks) continue;
-        const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
+        const int64_t row = tile * kTgRows + at[rb];
         if (row >= rows_out) continue;
         float* dst = partial + (((int64_t)blockIdx.z * (cout >> 2) + (co >> 2)) * rows_out + row) * 4;
 #pragma unroll
@@ -368,7 +393,7 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       if (KS > 1 && rb / RBK != ks) continue;
-      const int64_t row = tile * kTgRows + 32 * (RB * wr + rb) + r32;
+      const int64_t row = tile * kTgRows + at[rb];
       if (row >= rows_out) continue;
       float v[16];
 #pragma unroll
@@ -465,6 +490,11 @@ extern "C" int ocnnx_gather_tile_supported(int dtype, int64_t rows_in, int K, in
   return 1;
 }
 
+// (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
+extern "C" int ocnnx_gather_tile_ordered(int K, double plan_occupancy) {
+  return K != 8 && plan_occupancy >= 0.0 && plan_occupancy <= kTgSkipMaxOccupancy;
+}
+
 extern "C" int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out, int K, int cin, int cout) {
   const TileLaunch t = tile_launch(dtype == OCNN_F32, cdiv(rows_out, kTgRows), K, cin, cout);
   const int64_t parts = t.sc * t.sk;
@@ -481,8 +511,7 @@ template <typename T, bool F32> struct TilePass : Pass {
 
   TilePass(const ocnnx_gather_args& args, hipStream_t stream) : a(args), bn(args.bn ? *args.bn : ocnnx_bn{}), st(stream) {
     const int dtype = std::is_same<T, f16>::value ? OCNN_F16 : (F32 ? OCNN_F32 : OCNN_BF16);
-    // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
-    skip = a.K != 8 && a.plan_occupancy >= 0.0 && a.plan_occupancy <= kTgSkipMaxOccupancy;
+    skip = ocnnx_gather_tile_ordered(a.K, a.plan_occupancy) != 0;
     t = tile_launch(F32, cdiv(a.rows_out, kTgRows), a.K, a.cin, a.cout);
     if (a.split_c > 0 && a.split_k > 0) {
       t.sc = std::min<int>(a.split_c, (int)cdiv(a.cin, F32 ? 32 : 64));
@@ -509,7 +538,7 @@ template <typename T, bool F32> struct TilePass : Pass {
                                         (size_t)(t.ks - 1) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
 #define OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, SKIP_)                                                                      \
   hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WC_, WR_, KS_, SKIP_>), grid, dim3(256), lds, st, a.in,       \
-                     in_bytes, a.loc, a.uptr, a.urows, (const T*)a.workspace, a.bias, bn, a.out, partial, a.rows_out, a.K, \
+                     in_bytes, a.loc, a.uptr, a.urows, a.order, (const T*)a.workspace, a.bias, bn, a.out, partial, a.rows_out, a.K, \
                      a.cin, a.cout, tiles, per_xcd, t.sc, t.sk, rows_alloc)
 #define OCNN_TILE_CASE(MB_, WC_, WR_, KS_)                                   \
   if (t.mb == MB_ && t.wc == WC_ && t.wr == WR_ && t.ks == KS_) {            \
@@ -545,15 +574,10 @@ int ocnn::tile_pass(int dtype, const ocnnx_gather_args& a, hipStream_t st, Pass*
   return OCNN_OK;
 }
 
-extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
-                                 const int32_t* urows, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
-                                 int64_t rows_out, int K, const void* w, int cin, int cout, int w_transposed,
-                                 int reverse_slots, const void* bias, const ocnnx_bn* bn_or_null, void* out,
-                                 void* workspace, int64_t workspace_bytes, int split_c, int split_k, void* stream) {
+extern "C" int ocnnx_gather_tile_args(int dtype, const ocnnx_gather_args* args, void* stream) {
+  OCNN_REQUIRE_PTRS("conv_gather_tile", args);
   Pass* pass = nullptr;
-  int rc = tile_pass(dtype, {in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out, K, w, cin,
-                             cout, w_transposed, reverse_slots, bias, bn_or_null, out, workspace, workspace_bytes, split_c,
-                             split_k}, (hipStream_t)stream, &pass);
+  int rc = tile_pass(dtype, *args, (hipStream_t)stream, &pass);
   if (pass) {
     launch_jobs(dtype, pass->before, (hipStream_t)stream);
     rc = pass->main();
@@ -561,6 +585,17 @@ extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, con
     delete pass;
   }
   return rc == OCNN_OK ? check_launch("conv_gather_tile") : rc;
+}
+
+extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
+                                 const int32_t* urows, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
+                                 int64_t rows_out, int K, const void* w, int cin, int cout, int w_transposed,
+                                 int reverse_slots, const void* bias, const ocnnx_bn* bn_or_null, void* out,
+                                 void* workspace, int64_t workspace_bytes, int split_c, int split_k, void* stream) {
+  const ocnnx_gather_args args{in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out, K, w,
+                               cin, cout, w_transposed, reverse_slots, bias, bn_or_null, out, workspace, workspace_bytes,
+                               split_c, split_k, nullptr};
+  return ocnnx_gather_tile_args(dtype, &args, stream);
 }
 
 // The public entry point: 16-bit wide layers, in one part: its workspace is that of the packed weights, whatever more

@@ -78,6 +78,7 @@ struct GatherOp {
   int64_t rows_in = 0, rows = 0, ws_bytes = 0;
   bool transposed = false, reverse = false;
   std::shared_ptr<PlanArrays> plan;
+  Tensor order;                               // OCNNX_GATHER_TILE: the tiles' rows in the order the kernel takes them
   // dense one-slot form: rows read / written through an index of the non-empty nodes
   Tensor in_index, out_index, children;
   int64_t rows_all = 0;                       // rows of the padded result
@@ -130,13 +131,12 @@ struct GatherOp {
                                   typed<int32_t>(p->urows), p->umax, p->total, rows, K, ptr(W), cin, cout, transposed,
                                   reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
         break;
-      case OCNNX_GATHER_TILE:
-        check(ocnnx_gather_tile(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
-                                typed<int32_t>(p->urows), p->umax, p->total, p->occupancy, rows, K, ptr(W), cin, cout,
-                                transposed, reverse, ptr(bias), overflow ? nullptr : bn, out.data_ptr(), ws.data_ptr(),
-                                ws.numel(), 0, 0, st));
+      case OCNNX_GATHER_TILE: {
+        const ocnnx_gather_args args = tile_args(ptr(data), ptr(W), ptr(bias), overflow ? nullptr : bn, out, ws);
+        check(ocnnx_gather_tile_args(code, &args, st));
         if (!overflow) bn = nullptr;
         break;
+      }
       case OCNN_GATHER_SPARSE:
         check(ocnn_conv_gather_sparse(code, ptr(data), rows_in, typed<int32_t>(p->uptr), typed<int32_t>(p->urows),
                                       p->umax, p->total, typed<int32_t>(p->cptr), typed<uint32_t>(p->ent), p->n_blocks,
@@ -162,6 +162,14 @@ struct GatherOp {
       overflow->run_into(out, overflow_rows, data, overflow_table, W, bias);
     }
     return followed(view_cols ? out.view({-1, view_cols}) : out, bn);
+  }
+
+  ocnnx_gather_args tile_args(const void* data, const void* W, const void* bias, const ocnnx_bn* bn, const Tensor& out,
+                              const Tensor& ws) const {
+    const PlanArrays& p = *plan;
+    return {data, rows_in, typed<uint16_t>(p.loc), typed<int32_t>(p.uptr), typed<int32_t>(p.urows), p.umax, p.total,
+            p.occupancy, rows, K, W, cin, cout, transposed, reverse, bias, bn, out.data_ptr(), ws.data_ptr(), ws.numel(), 0, 0,
+            order.defined() ? typed<uint8_t>(order) : nullptr};
   }
 
   // this pass with row i of its result written to row index[i] of `out`
@@ -282,11 +290,8 @@ bool backward_together(const GatherOp& dgrad, const WgradOp& wgrad, const Tensor
   // (each with a workspace of its own: the passes overlap)
   Tensor ws_d = workspace(dgrad.ws_bytes, grad), ws_w = workspace(wgrad.ws_bytes, grad);
   Tensor ws_b = want_bias ? workspace(ocnn_colsum_workspace_bytes(grad.size(0), (int)grad.size(1)), grad) : Tensor();
-  const PlanArrays &p = *dgrad.plan, &q = *wgrad.plan;
-  const ocnnx_gather_args da{ptr(grad), dgrad.rows_in, typed<uint16_t>(p.loc), typed<int32_t>(p.uptr), typed<int32_t>(p.urows),
-                             p.umax, p.total, p.occupancy, dgrad.rows, dgrad.K, ptr(w), dgrad.cin, dgrad.cout,
-                             dgrad.transposed, dgrad.reverse, nullptr, nullptr, gx.data_ptr(), ws_d.data_ptr(), ws_d.numel(),
-                             0, 0};
+  const PlanArrays& q = *wgrad.plan;
+  const ocnnx_gather_args da = dgrad.tile_args(ptr(grad), ptr(w), nullptr, nullptr, gx, ws_d);
   const ocnnx_wgrad_args wa{ptr(x), wgrad.rows_x, ptr(g), typed<uint16_t>(q.loc), typed<int32_t>(q.uptr),
                             typed<int32_t>(q.urows), q.umax, q.total, wgrad.rows, wgrad.K, wgrad.ca, wgrad.cb,
                             wgrad.out_transposed, gw.data_ptr(), ws_w.data_ptr(), ws_w.numel()};
@@ -744,6 +749,24 @@ std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, in
   return out;
 }
 
+// The rows of the tiles of several plans in the order of ocnnx_plan_order, by their positions.
+std::vector<Tensor> tile_orders(const std::vector<Tensor>& locs) {
+  std::vector<Tensor> out;
+  std::vector<ocnnx_order_item> items;
+  int64_t tiles = 0;
+  for (const Tensor& loc : locs) {
+    require_gpu(loc);
+    TORCH_CHECK(loc.scalar_type() == at::kShort && loc.dim() == 3 && loc.size(2) == ocnn_tile_plan_rows() &&
+                    loc.is_contiguous() && loc.device() == locs[0].device(),
+                "tile_orders: positions of tile plans of one device");
+    out.push_back(at::empty({loc.size(0), loc.size(2)}, loc.options().dtype(at::kByte)));
+    items.push_back({typed<uint16_t>(loc), typed<uint8_t>(out.back()), loc.size(0), tiles, (int)loc.size(1)});
+    tiles += loc.size(0);
+  }
+  if (!items.empty()) check(ocnnx_plan_order(items.data(), (int)items.size(), hip_stream()));
+  return out;
+}
+
 // The neighbour tables of layers 1 .. depth (entry 0 is left out) of an octree as `tree` was built; none if
 // a layer is not, any more: keys, children and counts are public and may be assigned.
 std::vector<Tensor> all_neigh(const Tree& tree, const std::vector<OptTensor>& keys_now, const std::vector<Tensor>& children,
@@ -808,7 +831,7 @@ PYBIND11_MODULE(ocnn_host, m) {
       }))
 #define FIELD(name) .def_readwrite(#name, &GatherOp::name)
       FIELD(kernel) FIELD(K) FIELD(cin) FIELD(cout) FIELD(rows_in) FIELD(rows) FIELD(ws_bytes) FIELD(transposed)
-          FIELD(reverse) FIELD(plan) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
+          FIELD(reverse) FIELD(plan) FIELD(order) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
               FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded) FIELD(bias_repeat) FIELD(view_cols)
 #undef FIELD
       .def("copy", [](const GatherOp& op) { return std::make_shared<GatherOp>(op); })
@@ -886,6 +909,7 @@ PYBIND11_MODULE(ocnn_host, m) {
       FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(ucount) FIELD(stats);
 #undef FIELD
   m.def("tile_plans", &tile_plans, py::call_guard<py::gil_scoped_release>());
+  m.def("tile_orders", &tile_orders, py::call_guard<py::gil_scoped_release>());
   m.def("build_octree", &build_octree, py::call_guard<py::gil_scoped_release>());
   m.def("all_neigh", &all_neigh, py::call_guard<py::gil_scoped_release>());
   m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;

@@ -54,7 +54,10 @@ typedef struct {
   void *out, *workspace;
   int64_t workspace_bytes;
   int split_c, split_k;
+  const uint8_t* order;       // null, or the tiles' rows in the order of ocnnx_plan_order
 } ocnnx_gather_args;
+int ocnnx_gather_tile_ordered(int K, double plan_occupancy);
+int ocnnx_gather_tile_args(int dtype, const ocnnx_gather_args* args, void* stream);   // ocnnx_gather_tile
 typedef struct {
   const void* x;
   int64_t rows_x;
@@ -122,6 +125,16 @@ int ocnnx_plan_build(const ocnnx_plan_item* items, int n, int cap, int pad, int3
                      int32_t* lists, int64_t* stats, int64_t* host_stats, void* stream);
 int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, int pad, const int32_t* ucount, const int64_t* stats,
                        const int32_t* lists, void* stream);
+
+// The rows of the tiles of n plans (tile0: as above), 128 numbers below 128 a tile, in the order in which ocnnx_gather_tile takes
+// them where it leaves out what is empty (ocnnx_gather_tile_ordered); loc as ocnnx_plan_compact leaves it.
+typedef struct {
+  const uint16_t* loc;
+  uint8_t* order;
+  int64_t tiles, tile0;
+  int K;
+} ocnnx_order_item;
+int ocnnx_plan_order(const ocnnx_order_item* items, int n, void* stream);
 
 // The octree build from the points on: normalised points, keys, sort and node counts (sizes: device,
 // levels + 1, as ocnn_octree_build_scan); then keys, children and the indices of the non-empty nodes of

@@ -576,6 +576,81 @@ __global__ __launch_bounds__(256) void tile_plan_compact_many_kernel(
     plan_compact(tile - t0, ucount + t0, it.uptr, stats + 6 * i, cap, pad, lists + t0 * pad, it.urows, it.loc, it.K);
 }
 
+// The rows of a tile in an order that puts those with entries in the same slots beside each other, for kernels that leave out
+// what is empty for a whole block of them: sorted by the set of their slots, read as a number whose highest bit is the
+// tile's rarest slot.  (Share of (32-row block, slot) units with an entry, in the table's order / in this one, non-empty
+// nodes: depth 9 7 % set 0.39 / 0.24, 14 % 0.68 / 0.48; depth 8 15 % 0.49 / 0.41, 22 % 0.68 / 0.56; depth 7 31 % 0.58 / 0.50,
+// 41 % 0.89 / 0.77.  Other sorting keys and a greedy choice of the blocks gave nothing more.)
+//
+// A wave per tile, a lane two rows; instructions bound it (1100 a wave).
+struct OrderItems {
+  int n;
+  ocnnx_order_item it[kPlanItems];
+};
+
+__global__ __launch_bounds__(256) void tile_order_kernel(OrderItems p, int64_t tiles) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_key[4][kPlanRows];
+  __shared__ uint8_t s_row[4][kPlanRows];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t all = (int64_t)blockIdx.x * 4 + wave;
+  if (all >= tiles) return;
+  int i = 0;
+  while (i + 1 < p.n && all >= p.it[i + 1].tile0) ++i;
+  const ocnnx_order_item& it = p.it[i];
+  const int K = it.K;
+  const int64_t tile = all - it.tile0;
+  const uint32_t* src = (const uint32_t*)(it.loc + tile * K * kPlanRows) + lane;
+  uint32_t set0 = 0, set1 = 0;                               // slots of rows 2 lane, 2 lane + 1
+  int count = 0;                                             // lane k: rows with slot k
+  uint32_t v[27];
+#pragma unroll
+  for (int k = 0; k < 27; ++k) v[k] = k < K ? src[k * (kPlanRows / 2)] : 0u;
+#pragma unroll
+  for (int k = 0; k < 27; ++k) {
+    const bool a = (v[k] & 0xffffu) != 0u, b = (v[k] >> 16) != 0u;
+    set0 |= a ? 1u << k : 0u;
+    set1 |= b ? 1u << k : 0u;
+    const int c = __popcll(__ballot(a)) + __popcll(__ballot(b));
+    if (lane == k) count = c;
+  }
+  int rank = 0;                                              // lane k: slots more frequent than k
+#pragma unroll
+  for (int k = 0; k < 27; ++k) {
+    const int c = __builtin_amdgcn_readlane(count, k);
+    rank += c > count || (c == count && k < lane) ? 1 : 0;
+  }
+  // (25 bits of slots above the 7 of the row, which make the keys distinct: the two most frequent of 27 slots decide nothing)
+  uint32_t key0 = (uint32_t)(2 * lane), key1 = key0 + 1;
+#pragma unroll
+  for (int k = 0; k < 27; ++k) {
+    const int at = __builtin_amdgcn_readlane(rank, k) - 2;
+    if (at >= 0) {
+      key0 |= ((set0 >> k) & 1u) << (at + 7);
+      key1 |= ((set1 >> k) & 1u) << (at + 7);
+    }
+  }
+  typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_;
+  *(u32x2_*)&s_key[wave][2 * lane] = u32x2_{key0, key1};
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  int at0 = 0, at1 = 0;
+#pragma unroll 8
+  for (int j = 0; j < kPlanRows; j += 4) {
+    const u32x4 q = *(const u32x4*)&s_key[wave][j];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      at0 += q[u] < key0 ? 1 : 0;
+      at1 += q[u] < key1 ? 1 : 0;
+    }
+  }
+  s_row[wave][at0] = (uint8_t)(2 * lane);
+  s_row[wave][at1] = (uint8_t)(2 * lane + 1);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  ((uint16_t*)(it.order + tile * kPlanRows))[lane] =
+      (uint16_t)(s_row[wave][2 * lane] | (s_row[wave][2 * lane + 1] << 8));
+}
+
 __global__ void pair_plan_zero_kernel(unsigned long long* __restrict__ slot_count, int K) {
   if ((int)threadIdx.x < K) slot_count[threadIdx.x] = 0;
 }
@@ -677,6 +752,31 @@ extern "C" int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, 
                          first, first + tiles, ucount, stats + 6 * g, cap, pad, lists);
   });
   return check_launch("plan_compact");
+}
+
+extern "C" int ocnnx_plan_order(const ocnnx_order_item* items, int n, void* stream) {
+  OCNN_REQUIRE(n >= 1, "plan_order: bad sizes");
+  OCNN_REQUIRE_PTRS("plan_order", items);
+  int64_t at = 0;
+  for (int i = 0; i < n; ++i) {
+    const ocnnx_order_item& it = items[i];
+    OCNN_REQUIRE(it.K >= 1 && it.K <= 27 && it.tiles >= 0 && it.tiles < (1ll << 24) && it.tile0 == at, "plan_order: bad shape");
+    OCNN_REQUIRE(it.tiles == 0 || (it.loc && it.order), "plan_order: a required pointer is NULL");
+    at += it.tiles;
+  }
+  for (int g = 0; g < n; g += kPlanItems) {
+    OrderItems p;
+    p.n = std::min(kPlanItems, n - g);
+    int64_t tiles = 0;
+    for (int i = 0; i < p.n; ++i) {
+      p.it[i] = items[g + i];
+      p.it[i].tile0 -= items[g].tile0;
+      tiles += p.it[i].tiles;
+    }
+    if (tiles > 0)
+      hipLaunchKernelGGL(tile_order_kernel, dim3((unsigned)cdiv(tiles, 4)), dim3(256), 0, (hipStream_t)stream, p, tiles);
+  }
+  return check_launch("plan_order");
 }
 
 extern "C" int ocnn_tile_plan_build(const int32_t* table, int64_t rows, int K, int pad, int32_t* ucount,

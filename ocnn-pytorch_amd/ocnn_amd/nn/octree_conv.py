@@ -134,6 +134,8 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
                    L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
     if op.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE, _lib.GATHER_SPARSE, _lib.GATHER_PLANNED):
       op.plan = _plan_arrays(plan, sparse)
+      if op.kernel == _lib.GATHER_TILE and L.ocnnx_gather_tile_ordered(K, float(plan.occupancy)):
+        op.order = plan.order()
       if plan.overflow_rows is not None:
         op.overflow_rows, op.overflow_table = plan.overflow_rows, plan.overflow_table
         op.overflow = _gather_op(dtype, rows_in, plan.overflow_table.shape[0], K, cin, cout, transposed, reverse)

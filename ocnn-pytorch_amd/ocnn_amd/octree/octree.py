@@ -125,6 +125,7 @@ class TilePlan:
   before it and leaves the device idle while the host catches up."""
 
   siblings = False
+  _order = None
   CAP = 415      # the smallest limit of the kernels on the plan
   LIST_PAD = 416  # rows a tile's list may have in the one-pass build
 
@@ -157,6 +158,7 @@ class TilePlan:
     self.overflow_rows = self.overflow_table = None
     self._pairs = None
     self._on_pairs = None          # called when the pair plan is first asked for
+    self._order = self._on_order = None
     if built is not None and not built.stats[5]:
       self.uptr, self.urows, self.loc, ucount, stats = built.uptr, built.urows, built.loc, built.ucount, built.stats
     else:
@@ -204,10 +206,10 @@ class TilePlan:
 
   def __getstate__(self):
     """(copies leave out the layers' native passes, which are made again when asked for)"""
-    return {k: v for k, v in vars(self).items() if k not in ('_ops', '_native', '_native_pairs', '_on_pairs')}
+    return {k: v for k, v in vars(self).items() if k not in ('_ops', '_native', '_native_pairs', '_on_pairs', '_on_order')}
 
   def __setstate__(self, state):
-    vars(self).update(state, _on_pairs=None)
+    vars(self).update(state, _on_pairs=None, _on_order=None)
 
   @property
   def occupancy(self):
@@ -222,6 +224,22 @@ class TilePlan:
       if self._on_pairs is not None:
         self._on_pairs()
     return self._pairs
+
+  def order(self):
+    """The rows of each tile in the order in which the tile kernel takes them (ocnnx_plan_order; made on first use)."""
+    if self._order is None:
+      self.order_many([self])
+      if self._on_order is not None:
+        self._on_order()
+    return self._order
+
+  @staticmethod
+  def order_many(plans):
+    """order() of several plans, in one launch."""
+    if plans:
+      with torch.cuda.device(plans[0].loc.device):
+        for plan, order in zip(plans, _lib.native().tile_orders([p.loc for p in plans])):
+          plan._order = order
 
 
 class PairPlan:
@@ -297,7 +315,7 @@ class PairPlan:
 
 
 class PlanHistory:
-  """Which tile plans (and pair plans) octrees of a kind (depth, full_depth) were asked for.
+  """Which tile plans (and pair plans, and orders of the tiles' rows) octrees of a kind (depth, full_depth) were asked for.
   Bounded (the kinds and the plans of a kind seen least recently are dropped) and safe to
   use from several threads."""
 
@@ -307,25 +325,38 @@ class PlanHistory:
   def __init__(self):
     self._lock = threading.Lock()
     self._kinds = {}           # kind -> {plan key: pair plan wanted}, both in order of last use
+    self._ordered = {}         # kind -> keys of the plans whose order was asked for
 
   def requests(self, kind):
     """Snapshot {plan key: pair plan wanted} of a kind."""
     with self._lock:
       return dict(self._kinds.get(kind, {}))
 
-  def note(self, kind, key, pairs=False):
+  def ordered(self, kind):
+    """Keys of the plans of a kind whose order was asked for."""
+    with self._lock:
+      return frozenset(self._ordered.get(kind, ()))
+
+  def note(self, kind, key, pairs=False, order=False):
     with self._lock:
       plans = self._kinds.pop(kind, {})
       plans[key] = plans.pop(key, False) or pairs
+      if order:
+        self._ordered.setdefault(kind, set()).add(key)
       while len(plans) > self.MAX_PLANS:
-        plans.pop(next(iter(plans)))
+        gone = next(iter(plans))
+        plans.pop(gone)
+        self._ordered.get(kind, set()).discard(gone)
       self._kinds[kind] = plans
       while len(self._kinds) > self.MAX_KINDS:
-        self._kinds.pop(next(iter(self._kinds)))
+        gone = next(iter(self._kinds))
+        self._kinds.pop(gone)
+        self._ordered.pop(gone, None)
 
   def clear(self):
     with self._lock:
       self._kinds.clear()
+      self._ordered.clear()
 
 
 def _lut_grid(dev):
@@ -742,6 +773,8 @@ class Octree:
         plan = self._plans[ck]
         if plan._pairs is None:
           plan._on_pairs = lambda: history.note(kind, ck, pairs=True)
+        if plan._order is None:
+          plan._on_order = lambda: history.note(kind, ck, order=True)
     return self._plans[ck]
 
   def prepare(self):
@@ -808,6 +841,9 @@ class Octree:
     plans = TilePlan.build_many(tables)
     for ck, plan in zip(keys, plans):
       self._plans[ck] = plan
+    ordered = self.plan_history.ordered((self.depth, self.full_depth))
+    TilePlan.order_many([plan for ck, plan in zip(keys, plans) if ck in ordered and
+                         _lib.lib().ocnnx_gather_tile_ordered(plan.K, float(plan.occupancy))])
     with_pairs = [plan for ck, plan in zip(keys, plans) if requests[ck]]
     for plan, pp in zip(with_pairs, PairPlan.build_many(with_pairs)):
       plan._pairs = pp

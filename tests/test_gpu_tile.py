@@ -123,3 +123,82 @@ def test_planned_weight_gradient_ranges(dtype, ca, cb):
       if transposed:
         got = got.transpose(1, 2)
       assert (got - want).abs().max() / want.abs().max() < TOL[dtype], (rows, K, transposed)
+
+
+def _row_order(plan):
+  """order() by its definition: in a tile, rows by the set of their slots, the tile's rarest slot first."""
+  loc = plan.loc.cpu().numpy().view(np.uint16)
+  out = np.empty((loc.shape[0], loc.shape[2]), np.uint8)
+  for i, tile in enumerate(loc):
+    there = tile != 0
+    frequent = np.argsort(-there.sum(1), kind='stable')          # (slots as frequent: the lower one first)
+    key = sum(there[k].astype(np.int64) << b for b, k in enumerate(frequent) if b >= 2) if len(tile) > 2 else 0
+    out[i] = np.lexsort((np.arange(128), key + np.zeros(128, np.int64)))
+  return out
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,cout,K', [(96, 96, 27), (32, 64, 27), (160, 128, 9), (64, 256, 27), (128, 128, 3), (32, 32, 27)])
+def test_tile_kernel_row_order(dtype, cin, cout, K):
+  """The order of a tile's rows, and the layers' pass that takes them in it: one row, a remainder, whole tiles, tiles enough
+  for 256 channels a workgroup, rows without an entry, mirrored slots."""
+  from ocnn_amd.nn.octree_conv import _gather_op
+  for rows in (1, 129, 2048, 257 * 128 + 5):
+    print('tile kernel, order', dtype, cin, cout, 'rows', rows, 'K', K, flush=True)
+    g = torch.Generator().manual_seed(rows + cin)
+    t = (torch.arange(rows)[:, None] + torch.randint(-30, 31, (rows, K), generator=g)).clamp_(0, rows - 1).int()
+    t[torch.rand(rows, K, generator=g) < torch.rand(1, K, generator=g) * 0.4 + 0.6] = -1
+    t[torch.rand(rows, generator=g) < 0.1] = -1
+    plan = TilePlan(t.cuda())
+    assert _lib.lib().ocnnx_gather_tile_ordered(K, plan.occupancy)
+    assert np.array_equal(plan.order().cpu().numpy(), _row_order(plan))
+    x = torch.randn(rows, cin, generator=g).to(dtype).cuda()
+    b = torch.randn(cout, generator=g).to(dtype).cuda()
+    zero = torch.cat([x.double(), torch.zeros(1, cin, dtype=torch.float64, device='cuda')])
+    for reverse in (False, True):
+      w = (torch.randn((K, cout, cin) if reverse else (K, cin, cout), generator=g) / (K * cin) ** 0.5).to(dtype).cuda()
+      op = _gather_op(dtype, rows, rows, K, cin, cout, reverse, reverse, plan)
+      if op.kernel != _lib.GATHER_TILE:
+        continue
+      got = op.run(x, t.cuda(), w, b).double()
+      at = lambda k: w[K - 1 - k].T.double() if reverse else w[k].double()
+      want = b.double() + sum(zero[t[:, k].long().cuda()] @ at(k) for k in range(K))
+      assert (got - want).abs().max() / want.abs().max() < TOL[dtype], reverse
+      assert torch.equal(got, op.run(x, t.cuda(), w, b).double())
+
+
+def test_orders_of_several_plans():
+  """Orders made together are those made alone, with plans without rows and more plans than a launch describes."""
+  g = torch.Generator().manual_seed(4)
+  plans = []
+  for i in range(27):
+    rows, K = (0, 1, 130, 1000)[i % 4], (27, 9, 3)[i % 3]
+    t = torch.randint(-20, max(rows, 1), (rows, K), generator=g).clamp_(min=-1).int()
+    plans.append(TilePlan(t.cuda()))
+  alone = [p.order().clone() for p in plans]
+  TilePlan.order_many(plans)
+  for p, a in zip(plans, alone):
+    assert torch.equal(p.order(), a) and np.array_equal(a.cpu().numpy(), _row_order(p))
+
+
+def test_fresh_octree_orders_the_plans_of_its_predecessors():
+  """A layer on the tile kernel asks for its plan's order; the next octree of the kind makes it with the plan."""
+  from ocnn_amd import synthetic
+  from ocnn_amd.nn import OctreeConv
+  from ocnn_amd.octree import Octree, Points
+  from ocnn_amd.octree.octree import PlanHistory
+  history = PlanHistory()
+  layer = OctreeConv(96, 96, [3], 1, nempty=True).cuda().half()
+  for turn in range(2):
+    pts, nrm = synthetic.mixed_cloud(20000, seed=3 + turn)
+    octree = Octree(6, 2)
+    octree.plan_history = history
+    octree.build_octree(Points(pts.cuda(), nrm.cuda()))
+    octree.construct_all_neigh()
+    octree.prepare()
+    key = ((6, '333', 1, True), False)
+    assert (key in octree._plans and octree._plans[key]._order is not None) == (turn == 1)
+    layer(torch.randn(int(octree.nnum_nempty[6]), 96, device='cuda').half(), octree, 6)
+    assert octree._plans[key]._order is not None and history.ordered((6, 2)) == {key}
+  history.clear()
+  assert history.ordered((6, 2)) == frozenset()
