@@ -706,10 +706,12 @@ struct BuiltPlan {
 };
 
 // The one-pass plans of several tables, one wait for the sizes of all of them.
-std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, int pad) {
+// groups[i]: whether table i is one of sibling groups is wanted as well.
+std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, int pad, const std::vector<bool>& groups) {
   const int n = (int)tables.size();
   std::vector<BuiltPlan> out(n);
   if (n == 0) return out;
+  TORCH_CHECK(groups.size() == tables.size(), "tile_plans: one wish a table");
   std::vector<ocnnx_plan_item> items(n);
   const auto i32 = tables[0].options(), i64 = i32.dtype(at::kLong), i16 = i32.dtype(at::kShort);
   const int64_t tile_rows = ocnn_tile_plan_rows();
@@ -723,7 +725,7 @@ std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, in
     out[i].loc = at::empty({own, t.size(1), tile_rows}, i16);
     out[i].uptr = at::empty({own + 1}, i32);
     items[i] = {typed<int32_t>(t), typed<uint16_t>(out[i].loc), typed<int32_t>(out[i].uptr), nullptr, t.size(0), tiles,
-                (int)t.size(1)};
+                (int)t.size(1), groups[i]};
     tiles += own;
   }
   Tensor counts = at::empty({2, std::max<int64_t>(tiles, 1)}, i32), lists = at::empty({std::max<int64_t>(tiles, 1) * pad}, i32);

@@ -119,12 +119,15 @@ typedef struct {
   uint16_t* loc;
   int32_t *uptr, *urows;
   int64_t rows, tile0;
-  int K;
+  int K, groups;              // groups: say whether the table is one of sibling groups (csrc/plan.hip), in the second of the sizes
 } ocnnx_plan_item;
 int ocnnx_plan_build(const ocnnx_plan_item* items, int n, int cap, int pad, int32_t* ucount, int32_t* tile_nnz,
                      int32_t* lists, int64_t* stats, int64_t* host_stats, void* stream);
 int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, int pad, const int32_t* ucount, const int64_t* stats,
                        const int32_t* lists, void* stream);
+
+// The same of one plan, from its positions: tile_marks[tile], zeros before, is nonzero for the tiles of sibling groups.
+int ocnnx_plan_siblings(const uint16_t* loc, int64_t rows, int K, int32_t* tile_marks, void* stream);
 
 // The rows of the tiles of n plans (tile0: as above), 128 numbers below 128 a tile, in the order in which ocnnx_gather_tile takes
 // them where it leaves out what is empty (ocnnx_gather_tile_ordered); loc as ocnnx_plan_compact leaves it.

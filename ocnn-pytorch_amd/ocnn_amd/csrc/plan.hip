@@ -41,13 +41,9 @@ __device__ __forceinline__ int plan_hash(int32_t v) {
 // locality: by a bitonic sort) and counting bits: the position of a row is the number of rows
 // in smaller blocks plus the bits below its own in its block's mask.
 //
-// GROUPS: tile_nnz also says (kPlanSiblings) whether the tile is one of sibling groups: 27 slots, whole groups of eight
-// rows, and slot o of sibling s is the same row for every (o, s) of the same o + s, so that the 8 x 27 entries are 64 cells.
-// (Compared in LDS, where the positions are: 766 k rows 100 -> 111 us a plan.)
-//
 // HASH = kPlanHashQuick (mode 2 only): a tile whose blocks do not fit gives up, ucount[tile] =
 // kPlanOverflow; the caller then plans the table in two passes with HASH = kPlanHash.
-template <int HASH, bool GROUPS = false>
+template <int HASH>
 __device__ __forceinline__ void plan_tile(
     const int64_t tile, const int32_t* __restrict__ table, int64_t rows, int K, int mode,
     int32_t* __restrict__ ucount, const int32_t* __restrict__ uptr, int32_t* __restrict__ urows,
@@ -298,27 +294,6 @@ __device__ __forceinline__ void plan_tile(
   u32x4* dst = (u32x4*)(loc + e0);
   for (int i = tid; i < K * (kPlanRows / 8); i += kPlanThreads)
     dst[i] = *(const u32x4*)(s_pos + (i >> 4) * kPitch + (i & 15) * 8);
-  if constexpr (GROUPS) if (K == 27 && rows % 8 == 0) {
-    // along each axis: slot o >= 1 of the siblings on this side is slot o - 1 of those on the other (a group's positions of a slot
-    // are 16 bytes: siblings x = 0 | x = 1 are its halves, y the words of a half, z the halves of a word)
-    bool same = true;
-#pragma unroll 1
-    for (int i = tid; i < 3 * 18 * (kPlanRows / 8); i += kPlanThreads) {
-      const int axis = i / 288, o = (i >> 4) % 18, at = (i & 15) * 8;
-      const int k = axis == 0 ? 9 + o : axis == 1 ? o / 6 * 9 + 3 + o % 6 : o / 2 * 3 + 1 + o % 2;
-      const u32x4 p = *(const u32x4*)(s_pos + k * kPitch + at);
-      const u32x4 q = *(const u32x4*)(s_pos + (k - (axis == 0 ? 9 : axis == 1 ? 3 : 1)) * kPitch + at);
-      if (axis == 0) {
-        same = same && p[0] == q[2] && p[1] == q[3];
-      } else if (axis == 1) {
-        same = same && p[0] == q[1] && p[2] == q[3];
-      } else {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) same = same && (p[w] & 0xffffu) == q[w] >> 16;
-      }
-    }
-    if (__syncthreads_and(same) && tid == 0) tile_nnz[tile] = s_nnz + kPlanSiblings;
-  }
 }
 
 __global__ __launch_bounds__(kPlanThreads) void tile_plan_kernel(
@@ -344,16 +319,50 @@ __device__ __forceinline__ int plan_item_of(const PlanItems& p, int64_t tile) {
   return i;
 }
 
-// (eight waves a SIMD: four tiles a CU; the comparison of GROUPS costs a few spilled registers for that)
-template <bool GROUPS>
-__global__ __launch_bounds__(kPlanThreads, 8) void tile_plan_build_kernel(PlanItems p, int64_t first, int32_t* __restrict__ ucount,
+__global__ __launch_bounds__(kPlanThreads) void tile_plan_build_kernel(PlanItems p, int64_t first, int32_t* __restrict__ ucount,
                                                                        int32_t* __restrict__ lists,
                                                                        int32_t* __restrict__ tile_nnz, int pad) {
   const int64_t tile = first + blockIdx.x;
   const ocnnx_plan_item& it = p.it[plan_item_of(p, tile)];
   const int64_t t0 = it.tile0;
-  plan_tile<kPlanHashQuick, GROUPS>(tile - t0, it.table, it.rows, it.K, 2, ucount + t0, nullptr, lists + t0 * pad, it.loc,
-                                    tile_nnz ? tile_nnz + t0 : nullptr, pad);
+  plan_tile<kPlanHashQuick>(tile - t0, it.table, it.rows, it.K, 2, ucount + t0, nullptr, lists + t0 * pad, it.loc,
+                            tile_nnz ? tile_nnz + t0 : nullptr, pad);
+}
+
+// Of the tables that want it (groups): marks in tile_nnz (kPlanSiblings) the tiles of sibling groups: 27 slots, whole groups of
+// eight rows, and slot o of sibling s is the same row for every (o, s) of the same o + s, so that the 8 x 27 entries are 64
+// cells.  A wave per tile.  (In the kernel above, where the positions are in LDS, the comparison cost every plan 11 % and a table of
+// 4.9 M rows that no depth-wise layer reads 80 us.)
+__global__ __launch_bounds__(256) void tile_siblings_kernel(PlanItems p, int64_t first, int64_t last, int32_t* __restrict__ tile_nnz) {
+  const int64_t tile = first + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tile >= last) return;
+  const ocnnx_plan_item& it = p.it[plan_item_of(p, tile)];
+  if (!it.groups || it.K != 27 || it.rows % 8 != 0) return;
+  const uint16_t* loc = it.loc + (tile - it.tile0) * (27 * kPlanRows);
+  const int lane = threadIdx.x & 63;
+  // along each axis: slot o >= 1 of the siblings on this side is slot o - 1 of those on the other (a group's positions of a slot
+  // are 16 bytes: siblings x = 0 | x = 1 are its halves, y the words of a half, z the halves of a word)
+  bool same = true;
+#pragma unroll
+  for (int axis = 0; axis < 3; ++axis) {
+    const int back = axis == 0 ? 9 : axis == 1 ? 3 : 1;
+#pragma unroll 3
+    for (int i = lane; i < 18 * (kPlanRows / 8); i += 64) {
+      const int o = i >> 4, at = (i & 15) * 8;
+      const int k = axis == 0 ? 9 + o : axis == 1 ? o / 6 * 9 + 3 + o % 6 : o / 2 * 3 + 1 + o % 2;
+      const u32x4 a = *(const u32x4*)(loc + k * kPlanRows + at);
+      const u32x4 b = *(const u32x4*)(loc + (k - back) * kPlanRows + at);
+      if (axis == 0) {
+        same = same && a[0] == b[2] && a[1] == b[3];
+      } else if (axis == 1) {
+        same = same && a[0] == b[1] && a[2] == b[3];
+      } else {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) same = same && (a[w] & 0xffffu) == b[w] >> 16;
+      }
+    }
+  }
+  if (__ballot(!same) == 0ull && lane == 0) tile_nnz[tile] += kPlanSiblings;
 }
 
 // Pair plan of a table, on top of its tile plan: per tile and LIST the rows that have a
@@ -730,11 +739,13 @@ extern "C" int ocnnx_plan_build(const ocnnx_plan_item* items, int n, int cap, in
   if (const int rc = plan_items_check(items, n)) return rc;
   hipStream_t st = (hipStream_t)stream;
   plan_groups(items, n, [&](const PlanItems& p, int64_t first, int64_t tiles, int g) {
-    bool groups = false;                                     // (tables that can be of sibling groups)
-    for (int i = 0; i < p.n; ++i) groups = groups || (p.it[i].K == 27 && p.it[i].rows % 8 == 0);
+    bool groups = false;
+    for (int i = 0; i < p.n; ++i) groups = groups || p.it[i].groups;
     if (tiles > 0)
-      hipLaunchKernelGGL(groups ? tile_plan_build_kernel<true> : tile_plan_build_kernel<false>, dim3((unsigned)tiles),
-                         dim3(kPlanThreads), 0, st, p, first, ucount, lists, tile_nnz, pad);
+      hipLaunchKernelGGL(tile_plan_build_kernel, dim3((unsigned)tiles), dim3(kPlanThreads), 0, st, p, first, ucount, lists,
+                         tile_nnz, pad);
+    if (tiles > 0 && groups)
+      hipLaunchKernelGGL(tile_siblings_kernel, dim3((unsigned)cdiv(tiles, 4)), dim3(256), 0, st, p, first, first + tiles, tile_nnz);
     hipLaunchKernelGGL(tile_plan_offsets_many_kernel, dim3((unsigned)p.n), dim3(1024), 0, st, p, ucount, tile_nnz, cap,
                        stats + 6 * g, host_stats + 6 * g);
   });
@@ -752,6 +763,19 @@ extern "C" int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, 
                          first, first + tiles, ucount, stats + 6 * g, cap, pad, lists);
   });
   return check_launch("plan_compact");
+}
+
+extern "C" int ocnnx_plan_siblings(const uint16_t* loc, int64_t rows, int K, int32_t* tile_marks, void* stream) {
+  OCNN_REQUIRE(K >= 1 && K <= 27 && rows >= 0 && rows < (1ll << 31), "plan_siblings: bad shape");
+  if (rows == 0) return OCNN_OK;
+  OCNN_REQUIRE_PTRS("plan_siblings", loc, tile_marks);
+  PlanItems p;
+  p.n = 1;
+  p.it[0] = {nullptr, const_cast<uint16_t*>(loc), nullptr, nullptr, rows, 0, K, 1};
+  const int64_t tiles = cdiv(rows, kPlanRows);
+  hipLaunchKernelGGL(tile_siblings_kernel, dim3((unsigned)cdiv(tiles, 4)), dim3(256), 0, (hipStream_t)stream, p, (int64_t)0, tiles,
+                     tile_marks);
+  return check_launch("plan_siblings");
 }
 
 extern "C" int ocnnx_plan_order(const ocnnx_order_item* items, int n, void* stream) {
@@ -787,8 +811,8 @@ extern "C" int ocnn_tile_plan_build(const int32_t* table, int64_t rows, int K, i
   OCNN_REQUIRE(table && ucount && ulist && loc, "tile_plan: a required pointer is NULL");
   PlanItems p;
   p.n = 1;
-  p.it[0] = {table, loc, nullptr, nullptr, rows, 0, K};
-  hipLaunchKernelGGL(tile_plan_build_kernel<false>, dim3((unsigned)cdiv(rows, kPlanRows)), dim3(kPlanThreads), 0,
+  p.it[0] = {table, loc, nullptr, nullptr, rows, 0, K, 0};
+  hipLaunchKernelGGL(tile_plan_build_kernel, dim3((unsigned)cdiv(rows, kPlanRows)), dim3(kPlanThreads), 0,
                      (hipStream_t)stream, p, (int64_t)0, ucount, ulist, tile_nnz, pad);
   return check_launch("tile_plan");
 }

@@ -124,8 +124,7 @@ class TilePlan:
   in the middle of a training step wants: every read-back waits for the whole queue of kernels
   before it and leaves the device idle while the host catches up."""
 
-  siblings = False
-  _order = None
+  _order = _siblings = None
   CAP = 415      # the smallest limit of the kernels on the plan
   LIST_PAD = 416  # rows a tile's list may have in the one-pass build
 
@@ -135,30 +134,31 @@ class TilePlan:
     self._set(table, cap, *self._one_pass([table], cap))
 
   @classmethod
-  def build_many(cls, tables, cap: int = None):
-    """Plans of several tables, in one launch of each kernel and with one wait for their sizes."""
+  def build_many(cls, tables, cap: int = None, groups=None):
+    """Plans of several tables, in one launch of each kernel and with one wait for their sizes.  groups: for which of them
+    `siblings` is going to be asked."""
     plans, tables = [cls.__new__(cls) for _ in tables], [t.contiguous() for t in tables]
     cap = cls.CAP if cap is None else cap
-    for p, t, built in zip(plans, tables, cls._one_pass(tables, cap)):
-      p._set(t, cap, built)
+    for i, (p, t, built) in enumerate(zip(plans, tables, cls._one_pass(tables, cap, groups))):
+      p._set(t, cap, built, groups is not None and groups[i])
     return plans
 
   @classmethod
-  def _one_pass(cls, tables, cap):
+  def _one_pass(cls, tables, cap, groups=None):
     """Counts, positions and lists in one pass over the tables, the lists at fixed places (LIST_PAD
     rows a tile) first.  (A limit above LIST_PAD takes the two passes of count and fill.)"""
     if cap > cls.LIST_PAD or not tables:
       return [None] * len(tables)
     _lib.require_gpu(*tables)
     with torch.cuda.device(tables[0].device):
-      return _lib.native().tile_plans(tables, cap, cls.LIST_PAD)
+      return _lib.native().tile_plans(tables, cap, cls.LIST_PAD, [False] * len(tables) if groups is None else groups)
 
-  def _set(self, table, cap, built):
+  def _set(self, table, cap, built, groups=False):
     self.rows, self.K = table.shape
     self.overflow_rows = self.overflow_table = None
     self._pairs = None
     self._on_pairs = None          # called when the pair plan is first asked for
-    self._order = self._on_order = None
+    self._order = self._on_order = self._siblings = self._on_siblings = None
     if built is not None and not built.stats[5]:
       self.uptr, self.urows, self.loc, ucount, stats = built.uptr, built.urows, built.loc, built.ucount, built.stats
     else:
@@ -167,7 +167,8 @@ class TilePlan:
       self.urows = None
     _, flags, self.total, self.umax, self.nnz = stats[:5]
     dropped = flags & 1
-    self.siblings = bool(flags & 2)  # 27 slots over whole groups of siblings (seen by the one-pass build)
+    if groups and built is not None and not built.stats[5]:
+      self._siblings = bool(flags & 2)
     # how often a staged row is used by its tile: near 1 there is nothing to gain from staging
     self.reuse = self.nnz / max(self.total, 1)
     if dropped:
@@ -206,10 +207,10 @@ class TilePlan:
 
   def __getstate__(self):
     """(copies leave out the layers' native passes, which are made again when asked for)"""
-    return {k: v for k, v in vars(self).items() if k not in ('_ops', '_native', '_native_pairs', '_on_pairs', '_on_order')}
+    return {k: v for k, v in vars(self).items() if k not in ('_ops', '_native', '_native_pairs', '_on_pairs', '_on_order', '_on_siblings')}
 
   def __setstate__(self, state):
-    vars(self).update(state, _on_pairs=None, _on_order=None)
+    vars(self).update(state, _on_pairs=None, _on_order=None, _on_siblings=None)
 
   @property
   def occupancy(self):
@@ -224,6 +225,21 @@ class TilePlan:
       if self._on_pairs is not None:
         self._on_pairs()
     return self._pairs
+
+  @property
+  def siblings(self):
+    """Whether the table is one of 27 slots over whole groups of eight siblings (csrc/plan.hip: tile_siblings_kernel); found
+    with the plan where earlier octrees were asked for it, and otherwise when it is first asked for, with a read-back."""
+    if self._siblings is None:
+      self._siblings = False
+      if self.K == 27 and self.rows % 8 == 0 and self.rows > 0:
+        marks = torch.zeros(self.loc.shape[0], dtype=torch.int32, device=self.loc.device)
+        with torch.cuda.device(marks.device):
+          _lib.check(_lib.lib().ocnnx_plan_siblings(_lib.ptr(self.loc), self.rows, self.K, _lib.ptr(marks), _lib.stream()))
+        self._siblings = bool((marks != 0).all())
+      if self._on_siblings is not None:
+        self._on_siblings()
+    return self._siblings
 
   def order(self):
     """The rows of each tile in the order in which the tile kernel takes them (ocnnx_plan_order; made on first use)."""
@@ -315,7 +331,7 @@ class PairPlan:
 
 
 class PlanHistory:
-  """Which tile plans (and pair plans, and orders of the tiles' rows) octrees of a kind (depth, full_depth) were asked for.
+  """Which tile plans (and pair plans, and what else of a plan) octrees of a kind (depth, full_depth) were asked for.
   Bounded (the kinds and the plans of a kind seen least recently are dropped) and safe to
   use from several threads."""
 
@@ -325,38 +341,38 @@ class PlanHistory:
   def __init__(self):
     self._lock = threading.Lock()
     self._kinds = {}           # kind -> {plan key: pair plan wanted}, both in order of last use
-    self._ordered = {}         # kind -> keys of the plans whose order was asked for
+    self._wished = {}          # kind -> {plan key: names of what was asked for beside it ('order', 'siblings')}
 
   def requests(self, kind):
     """Snapshot {plan key: pair plan wanted} of a kind."""
     with self._lock:
       return dict(self._kinds.get(kind, {}))
 
-  def ordered(self, kind):
-    """Keys of the plans of a kind whose order was asked for."""
+  def wished(self, kind, what):
+    """Keys of the plans of a kind of which `what` was asked for."""
     with self._lock:
-      return frozenset(self._ordered.get(kind, ()))
+      return frozenset(key for key, names in self._wished.get(kind, {}).items() if what in names)
 
-  def note(self, kind, key, pairs=False, order=False):
+  def note(self, kind, key, pairs=False, wish=None):
     with self._lock:
       plans = self._kinds.pop(kind, {})
       plans[key] = plans.pop(key, False) or pairs
-      if order:
-        self._ordered.setdefault(kind, set()).add(key)
+      if wish is not None:
+        self._wished.setdefault(kind, {}).setdefault(key, set()).add(wish)
       while len(plans) > self.MAX_PLANS:
         gone = next(iter(plans))
         plans.pop(gone)
-        self._ordered.get(kind, set()).discard(gone)
+        self._wished.get(kind, {}).pop(gone, None)
       self._kinds[kind] = plans
       while len(self._kinds) > self.MAX_KINDS:
         gone = next(iter(self._kinds))
         self._kinds.pop(gone)
-        self._ordered.pop(gone, None)
+        self._wished.pop(gone, None)
 
   def clear(self):
     with self._lock:
       self._kinds.clear()
-      self._ordered.clear()
+      self._wished.clear()
 
 
 def _lut_grid(dev):
@@ -774,7 +790,9 @@ class Octree:
         if plan._pairs is None:
           plan._on_pairs = lambda: history.note(kind, ck, pairs=True)
         if plan._order is None:
-          plan._on_order = lambda: history.note(kind, ck, order=True)
+          plan._on_order = lambda: history.note(kind, ck, wish='order')
+        if plan._siblings is None:
+          plan._on_siblings = lambda: history.note(kind, ck, wish='siblings')
     return self._plans[ck]
 
   def prepare(self):
@@ -838,10 +856,11 @@ class Octree:
     for (depth, kernel, stride, nempty), inverse in keys:
       tables.append(self._table_t(depth, kernel, stride, nempty, self._fine_rows(depth, nempty)) if inverse
                     else self._table(depth, kernel, stride, nempty))
-    plans = TilePlan.build_many(tables)
+    kind = (self.depth, self.full_depth)
+    ordered, grouped = self.plan_history.wished(kind, 'order'), self.plan_history.wished(kind, 'siblings')
+    plans = TilePlan.build_many(tables, groups=[ck in grouped for ck in keys])
     for ck, plan in zip(keys, plans):
       self._plans[ck] = plan
-    ordered = self.plan_history.ordered((self.depth, self.full_depth))
     TilePlan.order_many([plan for ck, plan in zip(keys, plans) if ck in ordered and
                          _lib.lib().ocnnx_gather_tile_ordered(plan.K, float(plan.occupancy))])
     with_pairs = [plan for ck, plan in zip(keys, plans) if requests[ck]]

@@ -199,6 +199,29 @@ def test_fresh_octree_orders_the_plans_of_its_predecessors():
     key = ((6, '333', 1, True), False)
     assert (key in octree._plans and octree._plans[key]._order is not None) == (turn == 1)
     layer(torch.randn(int(octree.nnum_nempty[6]), 96, device='cuda').half(), octree, 6)
-    assert octree._plans[key]._order is not None and history.ordered((6, 2)) == {key}
+    assert octree._plans[key]._order is not None and history.wished((6, 2), 'order') == {key}
   history.clear()
-  assert history.ordered((6, 2)) == frozenset()
+  assert history.wished((6, 2), 'order') == frozenset()
+
+
+def test_fresh_octree_finds_the_sibling_groups_its_predecessors_were_asked_for():
+  """Whether a table is one of sibling groups: asked of the plan alone, and with the next octree's plan."""
+  from ocnn_amd import synthetic
+  from ocnn_amd.octree import Octree, Points
+  from ocnn_amd.octree.octree import PlanHistory
+  history = PlanHistory()
+  for turn in range(2):
+    pts, nrm = synthetic.mixed_cloud(20000, seed=5 + turn)
+    octree = Octree(6, 2)
+    octree.plan_history = history
+    octree.build_octree(Points(pts.cuda(), nrm.cuda()))
+    octree.construct_all_neigh()
+    octree.prepare()
+    for nempty in (False, True):
+      plan = octree._plan(6, '333', 1, nempty)
+      assert plan._siblings == (None if turn == 0 else not nempty)
+      assert plan.siblings == (not nempty) and TilePlan(octree._table(6, '333', 1, nempty)).siblings == (not nempty)
+  broken = octree._table(6, '333', 1, False).clone()
+  broken[-1, 13] = -1                                      # one entry of the last group
+  assert not TilePlan(broken).siblings and not TilePlan.build_many([broken], groups=[True])[0].siblings
+  assert not TilePlan(torch.empty((0, 27), dtype=torch.int32, device='cuda')).siblings
