@@ -139,6 +139,7 @@ INTERNAL_SIGNATURES = {
     'ocnnx_dense_rows_supported': (_i, [_i, _l, _i, _i]),
     'ocnnx_gather_tile_supported': (_i, [_i, _l, _i, _i, _i, _i]),
     'ocnnx_gather_tile_workspace_bytes': (_l, [_i, _l, _i, _i, _i]),
+    'ocnnx_input_feature': (_i, [_p, _p, _l, _i, ctypes.c_float, _p, _p]),
     'ocnnx_plan_siblings': (_i, [_p, _l, _i, _p, _p]),
     'ocnnx_gather_tile_ordered': (_i, [_i, _d]),
     'ocnnx_gather_tile': (_i, [_i, _p, _l, _p, _p, _p, _i, _l, _d, _l, _i, _p, _i, _i, _i, _i, _p, _p, _p, _p, _l, _i, _i, _p]),

@@ -164,6 +164,16 @@ struct GatherOp {
     return followed(view_cols ? out.view({-1, view_cols}) : out, bn);
   }
 
+  // the kernel for this shape, of a table with these figures of its plan, and the workspace it takes
+  void choose(int code, bool dense, bool has_plan, int umax, int64_t total, double occupancy, double reuse, bool overflows) {
+    kernel = ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, dense, has_plan, umax, total, occupancy, reuse, overflows);
+    ws_bytes = kernel == OCNN_GATHER_ZERO_PADDED || kernel == OCNNX_GATHER_ROWS ? 0
+               : kernel == OCNN_GATHER_SPARSE ? ocnn_conv_gather_sparse_workspace_bytes(cin, cout)
+               : kernel == OCNNX_GATHER_TILE  ? ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout)
+               : kernel == OCNN_GATHER_PLAIN  ? ocnnx_conv_gather_workspace_bytes(code, rows_in, rows, K, cin, cout)
+                                              : ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout);
+  }
+
   ocnnx_gather_args tile_args(const void* data, const void* W, const void* bias, const ocnnx_bn* bn, const Tensor& out,
                               const Tensor& ws) const {
     const PlanArrays& p = *plan;
@@ -217,6 +227,15 @@ struct WgradOp {
   std::vector<int64_t> shape;                 // shape the result is seen with, if not (K, ca, cb)
   Tensor overflow_table, overflow_rows;
   std::shared_ptr<WgradOp> overflow, padded;
+
+  void choose(int code, bool dense, bool has_plan, int umax, int64_t total, double occupancy) {
+    kernel = ocnn_conv_wgrad_choose(code, rows_x, rows, K, ca, cb, dense, has_plan, umax, total, occupancy);
+    ws_bytes = kernel == OCNN_WGRAD_ZERO_PADDED ? 0
+               : kernel == OCNN_WGRAD_DENSE_RW  ? ocnn_conv_dense_wgrad_rw_workspace_bytes(ca, cb)
+               : kernel == OCNN_WGRAD_SPARSE    ? ocnn_conv_wgrad_sparse_workspace_bytes(rows, ca, cb)
+               : kernel == OCNN_WGRAD_PLANNED   ? ocnn_conv_wgrad_planned_workspace_bytes_for(code, rows_x, rows, K, ca, cb)
+                                                : ocnn_conv_wgrad_workspace_bytes_for(code, rows_x, rows, K, ca, cb);
+  }
 
   Tensor run(Tensor x, Tensor g, Tensor table) const {
     require_gpu(x);
@@ -836,6 +855,7 @@ PYBIND11_MODULE(ocnn_host, m) {
           FIELD(reverse) FIELD(plan) FIELD(order) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
               FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded) FIELD(bias_repeat) FIELD(view_cols)
 #undef FIELD
+      .def("choose", &GatherOp::choose)
       .def("copy", [](const GatherOp& op) { return std::make_shared<GatherOp>(op); })
       .def("run", [](const GatherOp& op, const Tensor& data, const OptTensor& table, const Tensor& W, const OptTensor& bias) {
         pybind11::gil_scoped_release free;
@@ -853,6 +873,7 @@ PYBIND11_MODULE(ocnn_host, m) {
       FIELD(kernel) FIELD(K) FIELD(ca) FIELD(cb) FIELD(rows_x) FIELD(rows) FIELD(ws_bytes) FIELD(out_transposed) FIELD(plan)
           FIELD(g_index) FIELD(shape) FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded)
 #undef FIELD
+      .def("choose", &WgradOp::choose)
       .def("copy", [](const WgradOp& op) { return std::make_shared<WgradOp>(op); })
       .def("seen_as", [](const WgradOp& op, std::vector<int64_t> shape) {
         auto copy = std::make_shared<WgradOp>(op);

@@ -129,6 +129,10 @@ int ocnnx_plan_compact(const ocnnx_plan_item* items, int n, int cap, int pad, co
 // The same of one plan, from its positions: tile_marks[tile], zeros before, is nonzero for the tiles of sibling groups.
 int ocnnx_plan_siblings(const uint16_t* loc, int64_t rows, int K, int32_t* tile_marks, void* stream);
 
+// Signals of the leaves side by side, in the order of the bits of `parts`: 1 the normal (3), 2 <offset of the mean point from the
+// voxel's centre, normal> (1), 4 that offset (3), 8 the mean point * scale - 1 (3); points, normals: (n, 3), null where none is read.
+int ocnnx_input_feature(const float* points, const float* normals, int64_t n, int parts, float scale, float* out, void* stream);
+
 // The rows of the tiles of n plans (tile0: as above), 128 numbers below 128 a tile, in the order in which ocnnx_gather_tile takes
 // them where it leaves out what is empty (ocnnx_gather_tile_ordered); loc as ocnnx_plan_compact leaves it.
 typedef struct {

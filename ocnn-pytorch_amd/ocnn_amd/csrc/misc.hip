@@ -350,6 +350,36 @@ static void split_rows(int64_t rows, int64_t cols, int64_t* splits, int64_t* rps
   *splits = cdiv(rows, *rps);
 }
 
+// The input signal of a network from the leaves' mean points and normals (ocnnx_input_feature), a leaf a thread, each step
+// rounded as the torch operations one by one round it.  Five launches of 2 - 6 us in their place on 31 k leaves, where the
+// launches' host side was 96 us of a request's 2200.
+__global__ __launch_bounds__(256) void input_feature_kernel(const float* __restrict__ points, const float* __restrict__ normals,
+                                                            int64_t n, int parts, int channels, float scale,
+                                                            float* __restrict__ out) {
+#pragma clang fp contract(off)
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float p[3] = {0.f, 0.f, 0.f}, v[3] = {0.f, 0.f, 0.f}, offset[3];
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    if (parts & 14) p[e] = points[3 * i + e];
+    if (parts & 3) v[e] = normals[3 * i + e];
+    offset[e] = (p[e] - truncf(p[e])) - 0.5f;
+  }
+  float* dst = out + i * channels;
+  const float along = (offset[0] * v[0] + offset[1] * v[1]) + offset[2] * v[2];
+  if (parts == 3) {                                          // what networks take: 16 bytes a leaf
+    *(f32x4*)dst = f32x4{v[0], v[1], v[2], along};
+    return;
+  }
+  if (parts & 1) { dst[0] = v[0], dst[1] = v[1], dst[2] = v[2]; dst += 3; }
+  if (parts & 2) *dst++ = along;
+  if (parts & 4) { dst[0] = offset[0], dst[1] = offset[1], dst[2] = offset[2]; dst += 3; }
+  if (parts & 8)
+#pragma unroll
+    for (int e = 0; e < 3; ++e) dst[e] = p[e] * scale - 1.f;
+}
+
 }  // namespace ocnn
 
 using namespace ocnn;
@@ -574,4 +604,16 @@ extern "C" int ocnn_colsum(int dtype, const void* g, int64_t rows, int channels,
     launch_jobs<T>(after, st);
   });
   return check_launch("colsum");
+}
+
+extern "C" int ocnnx_input_feature(const float* points, const float* normals, int64_t n, int parts, float scale, float* out,
+                                   void* stream) {
+  OCNN_REQUIRE(n >= 0 && n < (1ll << 31) && parts > 0 && parts < 16, "input_feature: n=%lld parts=%d out of range", (long long)n,
+               parts);
+  if (n == 0) return OCNN_OK;
+  OCNN_REQUIRE(out && ((parts & 14) == 0 || points) && ((parts & 3) == 0 || normals), "input_feature: a required pointer is NULL");
+  const int channels = (parts & 1 ? 3 : 0) + (parts & 2 ? 1 : 0) + (parts & 4 ? 3 : 0) + (parts & 8 ? 3 : 0);
+  hipLaunchKernelGGL(input_feature_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, points, normals, n,
+                     parts, channels, scale, out);
+  return check_launch("input_feature");
 }

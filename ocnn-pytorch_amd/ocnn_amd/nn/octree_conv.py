@@ -112,8 +112,7 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
     return op
   L, code = _lib.lib(), _lib.dtype_code_of(dtype)
   op = _lib.native().GatherOp(rows_in, rows, K, cin, cout, transposed, reverse)
-  op.kernel = L.ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, int(dense), *_plan_args(plan),
-                                    int(plan is not None and plan.overflow_rows is not None))
+  op.choose(code, dense, *_plan_args(plan), plan is not None and plan.overflow_rows is not None)
   if op.kernel == _lib.GATHER_ZERO_PADDED:
     # (to 32 channels where a kernel on the plan then takes the layer, to 16 for the plan-free one: 64 -> 4 as 64 -> 32
     # on the tile kernel / 64 -> 16 plan-free, us, f16 and fp32: 1.28 M rows 68 % set 210 / 379, 453 / 1380; 1.13 M rows 7 %
@@ -125,16 +124,11 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
     op.padded = _gather_op(dtype, rows_in, rows, K, wide[0], wide[1] if on_plan else -(-cout // 16) * 16, transposed, reverse,
                            plan)
   else:
-    sparse = op.kernel == _lib.GATHER_SPARSE
-    op.ws_bytes = (L.ocnn_conv_gather_sparse_workspace_bytes(cin, cout) if sparse else
-                   L.ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout) if op.kernel == _lib.GATHER_TILE else
-                   L.ocnnx_conv_gather_workspace_bytes(code, rows_in, rows, K, cin, cout)
-                   if op.kernel == _lib.GATHER_PLAIN else
-                   0 if op.kernel == _lib.GATHER_ROWS else
-                   L.ocnn_conv_gather_workspace_bytes(code, rows_in, K, cin, cout))
     if op.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE, _lib.GATHER_SPARSE, _lib.GATHER_PLANNED):
-      op.plan = _plan_arrays(plan, sparse)
-      if op.kernel == _lib.GATHER_TILE and L.ocnnx_gather_tile_ordered(K, float(plan.occupancy)):
+      op.plan = _plan_arrays(plan, op.kernel == _lib.GATHER_SPARSE)
+      # (an order made under capture would hold nothing before the graph's first replay)
+      if op.kernel == _lib.GATHER_TILE and L.ocnnx_gather_tile_ordered(K, float(plan.occupancy)) and \
+          (plan._order is not None or not torch.cuda.is_current_stream_capturing()):
         op.order = plan.order()
       if plan.overflow_rows is not None:
         op.overflow_rows, op.overflow_table = plan.overflow_rows, plan.overflow_table
@@ -199,19 +193,10 @@ def _wgrad_op(dtype, rows_x, rows, K, ca, cb, out_transposed, plan=None, dense=F
   op = memo.get(key)
   if op is not None:
     return op
-  L, code = _lib.lib(), _lib.dtype_code_of(dtype)
   op = _lib.native().WgradOp(rows_x, rows, K, ca, cb, out_transposed)
-  op.kernel = L.ocnn_conv_wgrad_choose(code, rows_x, rows, K, ca, cb, int(dense), *_plan_args(plan)[:4])
+  op.choose(_lib.dtype_code_of(dtype), dense, *_plan_args(plan)[:4])
   if op.kernel == _lib.WGRAD_ZERO_PADDED:
     op.padded = _wgrad_op(dtype, rows_x, rows, K, -(-ca // 32) * 32, -(-cb // 32) * 32, out_transposed, plan)
-  elif op.kernel == _lib.WGRAD_DENSE_RW:
-    op.ws_bytes = L.ocnn_conv_dense_wgrad_rw_workspace_bytes(ca, cb)
-  elif op.kernel == _lib.WGRAD_SPARSE:
-    op.ws_bytes = L.ocnn_conv_wgrad_sparse_workspace_bytes(rows, ca, cb)
-  elif op.kernel == _lib.WGRAD_PLANNED:
-    op.ws_bytes = L.ocnn_conv_wgrad_planned_workspace_bytes_for(code, rows_x, rows, K, ca, cb)
-  else:
-    op.ws_bytes = L.ocnn_conv_wgrad_workspace_bytes_for(code, rows_x, rows, K, ca, cb)
   if op.kernel in (_lib.WGRAD_SPARSE, _lib.WGRAD_PLANNED):
     op.plan = _plan_arrays(plan, op.kernel == _lib.WGRAD_SPARSE)
     if plan.overflow_rows is not None:                   # (their share of the sums is added)

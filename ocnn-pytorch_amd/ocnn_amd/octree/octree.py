@@ -231,6 +231,8 @@ class TilePlan:
     """Whether the table is one of 27 slots over whole groups of eight siblings (csrc/plan.hip: tile_siblings_kernel); found
     with the plan where earlier octrees were asked for it, and otherwise when it is first asked for, with a read-back."""
     if self._siblings is None:
+      if torch.cuda.is_current_stream_capturing():         # (no read-back there)
+        return False
       self._siblings = False
       if self.K == 27 and self.rows % 8 == 0 and self.rows > 0:
         marks = torch.zeros(self.loc.shape[0], dtype=torch.int32, device=self.loc.device)
@@ -897,6 +899,18 @@ class Octree:
     from ..nn.octree_pad import octree_pad
     depth, wanted = self.depth, set(feature.upper())
     normals, points = self.normals[depth], self.points[depth]
+    read = ([normals] if wanted & {'N', 'D'} else []) + ([points] if wanted & {'D', 'L', 'P'} else [])
+    if wanted <= set('NDLP') and read and not _lib.recorded() and all(
+        type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.float32 and t.dim() == 2 and t.shape[1] == 3 and
+        t.is_contiguous() and not t.requires_grad and t.shape == read[0].shape and t.device == read[0].device for t in read):
+      # (what the build leaves: one launch in place of five)
+      parts = sum(bit for bit, c in ((1, 'N'), (2, 'D'), (4, 'L'), (8, 'P')) if c in wanted)
+      with torch.cuda.device(read[0].device):
+        out = torch.empty(read[0].shape[0], sum({'N': 3, 'D': 1, 'L': 3, 'P': 3}[c] for c in wanted), device=read[0].device)
+        _lib.check(_lib.lib().ocnnx_input_feature(_lib.ptr(points if len(read) > 1 or not wanted & {'N', 'D'} else None),
+                                                  _lib.ptr(normals if wanted & {'N', 'D'} else None), out.shape[0], parts,
+                                                  2.0 ** (1 - depth), _lib.ptr(out), _lib.stream()))
+      return out if nempty else octree_pad(out, self, depth)
     offset = points.frac() - 0.5 if wanted & {'L', 'D'} else None
     blocks = {
         'N': lambda: normals,

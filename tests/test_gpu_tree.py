@@ -74,3 +74,23 @@ def test_leaf_averages_across_spans(n, depth, batch, same, normals):
     assert np.abs(o.normals[depth].cpu().numpy() - sums[:, 3:] / length).max() < 1e-6
   else:
     assert o.normals[depth] is None
+
+
+@pytest.mark.parametrize('leaves', [0, 1, 255, 257, 70001])
+def test_input_feature_kernel(leaves):
+  """Every set of letters from one launch against the torch operations one by one (taken for signals that need a gradient);
+  the product sums three rounded products, whose order torch chooses: two roundings of a sum of at most 1.5."""
+  g = torch.Generator().manual_seed(leaves)
+  octree = Octree(5, 2)
+  octree.device = torch.device('cuda:0')
+  points = (torch.rand(leaves, 3, generator=g) * 34 - 1).cuda()                # (some outside the box: negative fractions)
+  normals = torch.nn.functional.normalize(torch.randn(leaves, 3, generator=g)).cuda()
+  for bits in range(1, 16):
+    letters = ''.join(c for i, c in enumerate('NDLP') if bits >> i & 1)
+    octree.points[5], octree.normals[5] = points, normals
+    got = octree.get_input_feature(letters, True)
+    octree.points[5], octree.normals[5] = points.clone().requires_grad_(), normals.clone().requires_grad_()
+    want = octree.get_input_feature(letters, True)
+    assert want.requires_grad and got.shape == want.shape and not got.requires_grad
+    if leaves:
+      assert (got - want).abs().max() <= (4e-7 if 'D' in letters else 0.0), letters
