@@ -56,10 +56,11 @@ static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char*
 // 1.13 M rows of depth 9, 7 % set, 334 us: 139 without any slot (rows, results and the chain of loads in front), 280 with a
 // quarter of the MFMAs, 290 with one fetch of weights a chunk.  A turn of the loop therefore waits for as little as can be: two sets
 // of registers in turn in place of copies, the blocks that are live known beforehand (334 -> 320 us), half the weights of
-// half a chunk, and 0.24 instead of 0.39 of the blocks by the order (298).  In us before / now, f16: 947 k rows 15 % set
-// 96 -> 96 329 / 303, 533 k 31 % 128 -> 128 299 / 274, 160 k 38 % 256 -> 256 383 / 349, 40 k 42 % 155 / 144, 822 k 14 % 96 -> 96
-// 333 / 294, nine slots of 1.13 M rows 234 / 215; fp32 132 k 36 % 96 -> 96 153 / 143, 264 k 22 % 64 -> 64 132 / 130, 19 k 128 -> 128
-// 60 / 59.  (Tables above the line below gain where a cloud is flat, 1.28 M rows 68 % set 96 -> 96 620 / 576, and lose elsewhere,
+// half a chunk, 0.24 instead of 0.39 of the blocks by the order (298), and the live blocks of a slot as a byte behind the order in
+// place of 54 reads of LDS and 27 ballots a tile (293).  In us before / now, f16: 947 k rows 15 % set
+// 96 -> 96 329 / 292, 533 k 31 % 128 -> 128 299 / 264, 160 k 38 % 256 -> 256 383 / 341, 40 k 42 % 155 / 143, 822 k 14 % 96 -> 96
+// 333 / 294, 31 k 17 % 26.7 / 21.9, nine slots of 1.13 M rows 234 / 213; fp32 132 k 36 % 96 -> 96 153 / 145, 264 k 22 % 64 -> 64 132 /
+// 124, 19 k 128 -> 128 60 / 59.  (Tables above the line below gain where a cloud is flat, 1.28 M rows 68 % set 96 -> 96 620 / 576, and lose elsewhere,
 // 97 k 52 % 256 -> 256 282 / 292: they stay without.)
 //
 // The four waves: WC along the output channels (32 MB each), WR along the rows (RB = 4 / WR blocks of 32 rows
@@ -96,6 +97,9 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   // (positions first: they don't wait for the list's place)
   constexpr int LP = 27 * 16 / 256 + 1;
   u32x4 lv[LP];
+  uint32_t blocks = 0;                                       // of lane k - k0: the slot's 32-row blocks with an entry (bits)
+  if constexpr (SKIP)
+    if (order && lane < k1 - k0) blocks = order[tile * OCNNX_TILE_ORDER_BYTES + kTgRows + k0 + lane];
   {
     const u32x4* src = (const u32x4*)(loc + (tile * K + k0) * (int64_t)kTgRows);
 #pragma unroll
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   for (int rb = 0; rb < RB; ++rb) {
     at[rb] = 32 * (RB * wr + rb) + r32;
     if constexpr (SKIP)
-      if (order) at[rb] = order[tile * kTgRows + at[rb]];
+      if (order) at[rb] = order[tile * OCNNX_TILE_ORDER_BYTES + at[rb]];
   }
   auto load_pos = [&](int k, uint32_t (&pv)[RB]) {
     const uint16_t* p = s_loc + (k - k0) * kTgRows;
@@ -242,23 +246,23 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   // (A slot without any costs the weights' way through L1, the busiest unit with 46 - 62 % on such tables, and a turn of the
   // loop.  Indoor scenes, non-empty nodes: 47 % of a tile's slots at depth 9, 1.13 M rows 96 -> 96 423 us, without them 323;
   // 37 % at depth 8, 947 k rows 380 / 327; 30 % at depth 7, 533 k rows 128 -> 128 332 / 317.)
-  uint32_t own = 0, blocks = 0;                              // blocks, of lane k - k0: its 32-row blocks with an entry (bits)
+  uint32_t own = 0;
   bool works = false;
   auto find_live = [&]() {
-    if constexpr (SKIP) {
-      const int a = order ? order[tile * kTgRows + lane] : lane, b = order ? order[tile * kTgRows + 64 + lane] : 64 + lane;
-      for (int k = wave; k < k1 - k0; k += 4) {
-        const unsigned long long lo = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + a] != 0);
-        const unsigned long long hi = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + b] != 0);
-        if (lane == 0)
-          s_live[k] = ((uint32_t)lo ? 1u : 0u) | (lo >> 32 ? 2u : 0u) | ((uint32_t)hi ? 4u : 0u) | (hi >> 32 ? 8u : 0u);
-      }
-    }
+    if constexpr (SKIP)
+      if (!order)
+        for (int k = wave; k < k1 - k0; k += 4) {
+          const unsigned long long lo = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + lane] != 0);
+          const unsigned long long hi = __builtin_amdgcn_ballot_w64(s_loc[k * kTgRows + 64 + lane] != 0);
+          if (lane == 0)
+            s_live[k] = ((uint32_t)lo ? 1u : 0u) | (lo >> 32 ? 2u : 0u) | ((uint32_t)hi ? 4u : 0u) | (hi >> 32 ? 8u : 0u);
+        }
   };
   auto deal_slots = [&]() {
     uint32_t live = (1u << (k1 - k0)) - 1u;
     if constexpr (SKIP) {
-      if (lane < k1 - k0) blocks = (s_live[lane] >> (RB * wr)) & ((1u << RB) - 1u);
+      if (!order && lane < k1 - k0) blocks = s_live[lane];
+      blocks = (blocks >> (RB * wr)) & ((1u << RB) - 1u);    // (of this wave's rows)
       live = (uint32_t)__builtin_amdgcn_ballot_w64(blocks != 0u);
     }
     // (every KS-th slot whether or not it is live: the same sums as without SKIP, to the bit)
@@ -334,37 +338,60 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   // ---- KS > 1: the waves' sums of a block are added by one of them, in the order of the waves ----
   if constexpr (KS > 1) {
     f32x4* ex = (f32x4*)s_rows;
-    const int pair = wave % (WC * WR);
+    constexpr int kPart = RBK * MB * 4 * 64;                 // a wave's sums of the blocks of one owner
+    auto put = [&](int o, f32x4* dst) {
 #pragma unroll
-    for (int o = 0; o < KS; ++o) {                           // owner of blocks RBK o ..
+      for (int i = 0; i < RBK; ++i)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            dst[((i * MB + mb) * 4 + r) * 64 + lane] = f32x4{acc[RBK * o + i][mb][4 * r], acc[RBK * o + i][mb][4 * r + 1],
+                                                             acc[RBK * o + i][mb][4 * r + 2], acc[RBK * o + i][mb][4 * r + 3]};
+    };
+    auto take = [&](int o, const f32x4* src) {
+#pragma unroll
+      for (int i = 0; i < RBK; ++i)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const f32x4 v = src[((i * MB + mb) * 4 + r) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[RBK * o + i][mb][4 * r + j] += v[j];
+          }
+    };
+    if constexpr (KS == 2) {
+      // both owners at once
+      f32x4 *mine = ex + wave * kPart, *other = ex + (wave ^ (WC * WR)) * kPart;
       __syncthreads();
-      if (ks != o) {
-        const int from = ks < o ? ks : ks - 1;
-#pragma unroll
-        for (int i = 0; i < RBK; ++i)
-#pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              ex[((((from * WC * WR + pair) * RBK + i) * MB + mb) * 4 + r) * 64 + lane] =
-                  f32x4{acc[RBK * o + i][mb][4 * r], acc[RBK * o + i][mb][4 * r + 1], acc[RBK * o + i][mb][4 * r + 2],
-                        acc[RBK * o + i][mb][4 * r + 3]};
-      }
+      if (ks == 0) put(1, mine);
+      else put(0, mine);
       __syncthreads();
-      if (ks == o) {
-#pragma unroll
-        for (int f = 0; f < KS - 1; ++f)
-#pragma unroll
-          for (int i = 0; i < RBK; ++i)
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const f32x4 v = ex[((((f * WC * WR + pair) * RBK + i) * MB + mb) * 4 + r) * 64 + lane];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[RBK * o + i][mb][4 * r + j] += v[j];
-              }
-      }
+      if (ks == 0) take(0, other);
+      else take(1, other);
+    } else {
+      // halves of the blocks between waves two apart, then single blocks between neighbours: four barriers and
+      // every wave at work, where one owner after the other took eight (f16 32 -> 64 on 264 k rows, 22 % set,
+      // 56.2 us, so 52.9, 64 -> 32 on 132 k rows 28.3 / 25.7, fp32 64 -> 64 129.9 / 128.5)
+      static_assert(KS != 4 || (WC * WR == 1 && RBK == 1), "a block a wave");
+      f32x4 *mine = ex + wave * 2 * kPart, *far = ex + (wave ^ 2) * 2 * kPart, *near = ex + (wave ^ 1) * 2 * kPart;
+      __syncthreads();
+      if (ks < 2) put(2, mine), put(3, mine + kPart);
+      else put(0, mine), put(1, mine + kPart);
+      __syncthreads();
+      if (ks < 2) take(0, far), take(1, far + kPart);
+      else take(2, far), take(3, far + kPart);
+      __syncthreads();
+      if (ks == 0) put(1, mine);
+      else if (ks == 1) put(0, mine);
+      else if (ks == 2) put(3, mine);
+      else put(2, mine);
+      __syncthreads();
+      if (ks == 0) take(0, near);
+      else if (ks == 1) take(1, near);
+      else if (ks == 2) take(2, near);
+      else take(3, near);
     }
   }
 
@@ -535,7 +562,7 @@ template <typename T, bool F32> struct TilePass : Pass {
     // LDS: rows, positions, list; at the end the waves' sums
     const int kmax = (a.K + t.sk - 1) / t.sk;
     const size_t lds = std::max<size_t>((size_t)rows_alloc * 132 + (size_t)kmax * kTgRows * 2 + 128,
-                                        (size_t)(t.ks - 1) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
+                                        (size_t)(t.ks == 4 ? 8 : t.ks == 2 ? 2 : 0) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
 #define OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, SKIP_)                                                                      \
   hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WC_, WR_, KS_, SKIP_>), grid, dim3(256), lds, st, a.in,       \
                      in_bytes, a.loc, a.uptr, a.urows, a.order, (const T*)a.workspace, a.bias, bn, a.out, partial, a.rows_out, a.K, \

@@ -780,7 +780,7 @@ std::vector<Tensor> tile_orders(const std::vector<Tensor>& locs) {
     TORCH_CHECK(loc.scalar_type() == at::kShort && loc.dim() == 3 && loc.size(2) == ocnn_tile_plan_rows() &&
                     loc.is_contiguous() && loc.device() == locs[0].device(),
                 "tile_orders: positions of tile plans of one device");
-    out.push_back(at::empty({loc.size(0), loc.size(2)}, loc.options().dtype(at::kByte)));
+    out.push_back(at::empty({loc.size(0), OCNNX_TILE_ORDER_BYTES}, loc.options().dtype(at::kByte)));
     items.push_back({typed<uint16_t>(loc), typed<uint8_t>(out.back()), loc.size(0), tiles, (int)loc.size(1)});
     tiles += loc.size(0);
   }

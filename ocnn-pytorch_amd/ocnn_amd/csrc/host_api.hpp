@@ -134,7 +134,9 @@ int ocnnx_plan_siblings(const uint16_t* loc, int64_t rows, int K, int32_t* tile_
 int ocnnx_input_feature(const float* points, const float* normals, int64_t n, int parts, float scale, float* out, void* stream);
 
 // The rows of the tiles of n plans (tile0: as above), 128 numbers below 128 a tile, in the order in which ocnnx_gather_tile takes
-// them where it leaves out what is empty (ocnnx_gather_tile_ordered); loc as ocnnx_plan_compact leaves it.
+// them where it leaves out what is empty (ocnnx_gather_tile_ordered), and behind them of each slot which of the tile's four blocks
+// of 32 rows, in that order, have an entry (bits): OCNNX_TILE_ORDER_BYTES a tile.  loc as ocnnx_plan_compact leaves it.
+#define OCNNX_TILE_ORDER_BYTES 160
 typedef struct {
   const uint16_t* loc;
   uint8_t* order;

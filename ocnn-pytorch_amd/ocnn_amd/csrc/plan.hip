@@ -652,12 +652,23 @@ __global__ __launch_bounds__(256) void tile_order_kernel(OrderItems p, int64_t t
       at1 += q[u] < key1 ? 1 : 0;
     }
   }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // (the keys are read: their places hold the sets in order)
+  __builtin_amdgcn_wave_barrier();
   s_row[wave][at0] = (uint8_t)(2 * lane);
   s_row[wave][at1] = (uint8_t)(2 * lane + 1);
+  s_key[wave][at0] = set0;
+  s_key[wave][at1] = set1;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  ((uint16_t*)(it.order + tile * kPlanRows))[lane] =
-      (uint16_t)(s_row[wave][2 * lane] | (s_row[wave][2 * lane + 1] << 8));
+  uint8_t* dst = it.order + tile * OCNNX_TILE_ORDER_BYTES;
+  ((uint16_t*)dst)[lane] = (uint16_t)(s_row[wave][2 * lane] | (s_row[wave][2 * lane + 1] << 8));
+  uint32_t of_block = s_key[wave][2 * lane] | s_key[wave][2 * lane + 1];
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) of_block |= (uint32_t)__shfl_xor((int)of_block, o);
+  uint32_t live = 0;                                         // lane k: the blocks with an entry in slot k
+#pragma unroll
+  for (int b = 0; b < 4; ++b) live |= (((uint32_t)__builtin_amdgcn_readlane((int)of_block, 16 * b) >> (lane & 31)) & 1u) << b;
+  if (lane < OCNNX_TILE_ORDER_BYTES - kPlanRows) dst[kPlanRows + lane] = lane < K ? (uint8_t)live : (uint8_t)0;
 }
 
 __global__ void pair_plan_zero_kernel(unsigned long long* __restrict__ slot_count, int K) {

@@ -244,7 +244,8 @@ class TilePlan:
     return self._siblings
 
   def order(self):
-    """The rows of each tile in the order in which the tile kernel takes them (ocnnx_plan_order; made on first use)."""
+    """The rows of each tile in the order in which the tile kernel takes them, and the live blocks of its slots
+    (ocnnx_plan_order; made on first use)."""
     if self._order is None:
       self.order_many([self])
       if self._on_order is not None:

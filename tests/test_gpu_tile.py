@@ -126,14 +126,20 @@ def test_planned_weight_gradient_ranges(dtype, ca, cb):
 
 
 def _row_order(plan):
-  """order() by its definition: in a tile, rows by the set of their slots, the tile's rarest slot first."""
+  """order() by its definition: in a tile, rows by the set of their slots, the tile's rarest slot first; then of each slot
+  which blocks of 32 rows have an entry."""
   loc = plan.loc.cpu().numpy().view(np.uint16)
-  out = np.empty((loc.shape[0], loc.shape[2]), np.uint8)
+  out = np.zeros((loc.shape[0], 160), np.uint8)
   for i, tile in enumerate(loc):
     there = tile != 0
     frequent = np.argsort(-there.sum(1), kind='stable')          # (slots as frequent: the lower one first)
-    key = sum(there[k].astype(np.int64) << b for b, k in enumerate(frequent) if b >= 2) if len(tile) > 2 else 0
-    out[i] = np.lexsort((np.arange(128), key + np.zeros(128, np.int64)))
+    key = np.zeros(128, np.int64)
+    for b, k in enumerate(frequent):
+      if b >= 2:                                                 # (the two most frequent ones decide nothing)
+        key |= there[k].astype(np.int64) << b
+    out[i, :128] = np.lexsort((np.arange(128), key))
+    blocks = there[:, out[i, :128]].reshape(len(tile), 4, 32).any(2)
+    out[i, 128:128 + len(tile)] = (blocks << np.arange(4)).sum(1)
   return out
 
 
