@@ -127,6 +127,8 @@ class TilePlan:
   _order = _siblings = None
   CAP = 415      # the smallest limit of the kernels on the plan
   LIST_PAD = 416  # rows a tile's list may have in the one-pass build
+  MOST_STAGED = 511  # tiles of more rows are for the multi-pass kernel alone, which takes tables of at least
+  MULTI_PASS_REUSE = 2.0  # this reuse (csrc/select.hip)
 
   def __init__(self, table: torch.Tensor, cap: int = None):
     table = table.contiguous()
@@ -181,7 +183,21 @@ class TilePlan:
       if dropped:
         table = table.clone()
         table[idx] = -1
+      elif built is not None and not built.stats[5] and self.umax > self.MOST_STAGED and self.reuse < self.MULTI_PASS_REUSE:
+        # (2x2x2 tables of coarse levels, three of thirteen in a network: tiles of more rows than any kernel stages, each used
+        # once, so that no layer reads the lists and positions, 7 us each; whoever does gets them then)
+        del self.urows, self.loc
+        self._unfilled = table
+        return
       self._fill(table)
+
+  def __getattr__(self, name):
+    table = vars(self).get('_unfilled')
+    if table is None or name not in ('urows', 'loc'):
+      raise AttributeError(name)
+    with torch.cuda.device(table.device):
+      self._fill(table)
+    return vars(self)[name]
 
   def _count(self, table, cap):
     """First of two passes: distinct rows per tile, their offsets, and the sizes on the host."""

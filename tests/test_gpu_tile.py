@@ -231,3 +231,20 @@ def test_fresh_octree_finds_the_sibling_groups_its_predecessors_were_asked_for()
   broken[-1, 13] = -1                                      # one entry of the last group
   assert not TilePlan(broken).siblings and not TilePlan.build_many([broken], groups=[True])[0].siblings
   assert not TilePlan(torch.empty((0, 27), dtype=torch.int32, device='cuda')).siblings
+
+
+@pytest.mark.parametrize('rows,K,entries', [(500, 8, 512), (500, 8, 700), (300, 8, 100000), (1000, 27, 1000)])
+def test_lists_that_no_kernel_reads_are_made_when_read(rows, K, entries):
+  """Tiles of more rows than any kernel stages, each used about once: lists and positions are those of the two passes."""
+  import copy
+  g = torch.Generator().manual_seed(rows + entries)
+  t = torch.stack([torch.randperm(max(entries, K), generator=g)[:K] for _ in range(rows)]).int().cuda()
+  plan, other, two = TilePlan(t), TilePlan(t), TilePlan(t, cap=4000)
+  assert two.umax == plan.umax
+  left = plan.umax > TilePlan.MOST_STAGED and plan.reuse < TilePlan.MULTI_PASS_REUSE
+  assert ('loc' not in vars(plan)) == left == (K == 8 and entries > 512)
+  other = copy.deepcopy(other)
+  for p in (plan, other):
+    assert torch.equal(p.loc, two.loc) and torch.equal(p.urows[:p.total], two.urows[:two.total]) and torch.equal(p.uptr, two.uptr)
+  with pytest.raises(AttributeError):
+    plan.nothing
