@@ -45,8 +45,7 @@ static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char*
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, off, 0, 0, 0);
 }
 
-// SKIP: per slot and 32-row block of the tile a wave asks whether any row has an entry there (a
-// ballot over the positions it reads anyway) and leaves the block's MFMAs out otherwise.  Blocks are the outer
+// SKIP: a wave leaves out the MFMAs of a slot and 32-row block of the tile where no row has an entry.  Blocks are the outer
 // loop of a slot, so that one branch stands around a block's 4 - 18 MFMAs: with the k-steps outside and a branch
 // per MFMA the same tables took 6 - 10 % longer.  The rows of a block are read one block ahead, behind a branch of their own.
 //

@@ -15,7 +15,7 @@
 // Tried: four waves with one place for rows, two or three workgroups a CU (211 us, the output 158: a wave alone on its SIMD
 // waits for itself); a dword of every row of the tile after next asked for ahead, to have it in L2 (202, 134).
 //
-// Whether a table is of that kind is seen when its plan is made (plan.hip compares the positions); cell (a, b, c), each
+// Whether a table is of that kind is found from its plan's positions (plan.hip: tile_siblings_kernel); cell (a, b, c), each
 // -1 .. 2, is slot (a - sx, b - sy, c - sz) of sibling (sx, sy, sz) for every sibling that it is a neighbour of.
 #include <algorithm>
 #include <type_traits>
