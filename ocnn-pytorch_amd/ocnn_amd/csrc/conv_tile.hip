@@ -10,7 +10,7 @@
 // fetched four or two.  Layers of fewer channels than four such waves split the SLOTS over the waves instead, whose
 // sums are added in LDS at the end.  (Waves of 32 channels x 128 rows side by side read LDS once per MFMA, as fast
 // as its pipe delivers gathered rows: on the non-empty nodes of depth 7, 533 k rows, 128 -> 128 381 us, so 328.)
-// Two workgroups share a CU: while one waits for its next chunk of channels the other computes.
+// Two or three workgroups share a CU: while one waits for its next chunk of channels the others compute.
 //
 // fp32: x = hi + lo in bf16 pieces, accumulated in fp32 as hi hi + hi lo + lo hi (about 1e-5
 // relative).  The rows are read as fp32 and split on their way into LDS, so that a row's 128 bytes
@@ -59,7 +59,7 @@ static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char*
 // place of 54 reads of LDS and 27 ballots a tile (293).  In us before / now, f16: 947 k rows 15 % set
 // 96 -> 96 329 / 292, 533 k 31 % 128 -> 128 299 / 264, 160 k 38 % 256 -> 256 383 / 341, 40 k 42 % 155 / 143, 822 k 14 % 96 -> 96
 // 333 / 294, 31 k 17 % 26.7 / 21.9, nine slots of 1.13 M rows 234 / 213; fp32 132 k 36 % 96 -> 96 153 / 145, 264 k 22 % 64 -> 64 132 /
-// 124, 19 k 128 -> 128 60 / 59.  (Tables above the line below gain where a cloud is flat, 1.28 M rows 68 % set 96 -> 96 620 / 576, and lose elsewhere,
+// 124 (105 with three workgroups a CU: tile_half_waves), 19 k 128 -> 128 60 / 59.  (Tables above the line below gain where a cloud is flat, 1.28 M rows 68 % set 96 -> 96 620 / 576, and lose elsewhere,
 // 97 k 52 % 256 -> 256 282 / 292: they stay without.)
 //
 // The four waves: WC along the output channels (32 MB each), WR along the rows (RB = 4 / WR blocks of 32 rows
@@ -477,11 +477,31 @@ static double tile_cost(const TileLaunch& t, bool f32, int64_t tiles, int K, int
 constexpr int kTgPartsGroups = 640;
 constexpr int kTgMaxSlotParts = 6;
 
-static TileLaunch tile_launch(bool f32, int64_t tiles, int K, int cin, int cout) {
+// Whether the four waves of 64 output channels take 32 channels and half the slots each, three workgroups a CU, in place of
+// 64 channels and a quarter of the slots, two a CU.  Four blocks of sums a wave instead of eight leave registers for the third
+// workgroup, and a tile ends with one round of exchange instead of two; a row read from LDS feeds half the MFMAs.  So it
+// pays where a tile is a chain of waits rather than MFMAs.
+// Where empty units are left out, us before / now: 565 k rows 7 % set f16 32 -> 64 80 / 65, 256 -> 64 233 / 203, fp32 32 -> 64
+// 114 / 89, 64 -> 64 176 / 144, 128 -> 64 276 / 233; 264 k 22 % fp32 64 -> 64 115 / 105; 593 k 25 % f16 128 -> 64 211 / 193; 267 k
+// 31 % fp32 64 -> 64 109 / 102, 256 -> 64 354 / 356; nine slots of 822 k rows 0.79.  The third workgroup has to find LDS (297 k
+// rows, 378 distinct a tile: 0.95 - 1.04), and there have to be tiles for one and a half rounds of three a CU (1035 tiles
+// 0.93 - 1.08, 1130 0.92 - 1.01, 1240 and 1294 0.87 - 0.98, 20 k - 41 k rows 0.91 - 1.08).
+// Elsewhere with one chunk of channels: 0.78 - 0.98 on 656 - 9950 tiles, 61 - 73 % set, 2x2x2 tables; with more chunks 0.97 - 1.03.
+constexpr int kTgThirdRows = 352;                            // staged rows with which three workgroups fit: 53760 bytes each at 27 slots
+constexpr int64_t kTgThirdTiles = 1152;
+
+static bool tile_half_waves(bool f32, int64_t tiles, int cin, bool skip, int max_distinct) {
+  if (skip) return tiles > kTgThirdTiles && max_distinct < kTgThirdRows;
+  return tiles > kTgPartsGroups && cin <= (f32 ? 32 : 64);
+}
+
+// (skip, max_distinct: the shape of the waves, of launches that are not cut up, hangs on them, nothing else)
+static TileLaunch tile_launch(bool f32, int64_t tiles, int K, int cin, int cout, bool skip, int max_distinct) {
   TileLaunch t{1, 1, 1, 4, 1, 1, 1};                         // 32 channels
   if (cout % 256 == 0 && tiles * (cout / 256) > 256) t.mb = 2, t.wc = 4, t.ks = 1;
   else if (cout % 96 == 0) t.mb = 3, t.wr = 2, t.ks = 2;
   else if (cout > 64) t.mb = 2, t.wc = 2, t.ks = 2;
+  else if (cout > 32 && tile_half_waves(f32, tiles, cin, skip, max_distinct)) t.wc = 2, t.ks = 2;
   else if (cout > 32) t.mb = 2;
   t.gy = (int)cdiv(cout, 32 * t.mb * t.wc);
   const int ncc = (int)cdiv(cin, f32 ? 32 : 64);
@@ -523,7 +543,7 @@ extern "C" int ocnnx_gather_tile_ordered(int K, double plan_occupancy) {
 }
 
 extern "C" int64_t ocnnx_gather_tile_workspace_bytes(int dtype, int64_t rows_out, int K, int cin, int cout) {
-  const TileLaunch t = tile_launch(dtype == OCNN_F32, cdiv(rows_out, kTgRows), K, cin, cout);
+  const TileLaunch t = tile_launch(dtype == OCNN_F32, cdiv(rows_out, kTgRows), K, cin, cout, false, 0);
   const int64_t parts = t.sc * t.sk;
   return tile_packed_bytes(dtype, K, cin, cout) + (parts > 1 ? parts * rows_out * cout * 4 : 0);
 }
@@ -539,7 +559,7 @@ template <typename T, bool F32> struct TilePass : Pass {
   TilePass(const ocnnx_gather_args& args, hipStream_t stream) : a(args), bn(args.bn ? *args.bn : ocnnx_bn{}), st(stream) {
     const int dtype = std::is_same<T, f16>::value ? OCNN_F16 : (F32 ? OCNN_F32 : OCNN_BF16);
     skip = ocnnx_gather_tile_ordered(a.K, a.plan_occupancy) != 0;
-    t = tile_launch(F32, cdiv(a.rows_out, kTgRows), a.K, a.cin, a.cout);
+    t = tile_launch(F32, cdiv(a.rows_out, kTgRows), a.K, a.cin, a.cout, skip, a.plan_max_distinct);
     if (a.split_c > 0 && a.split_k > 0) {
       t.sc = std::min<int>(a.split_c, (int)cdiv(a.cin, F32 ? 32 : 64));
       t.sk = std::min(a.split_k, a.K);
@@ -573,7 +593,7 @@ template <typename T, bool F32> struct TilePass : Pass {
     else OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, false);                        \
   }
     OCNN_TILE_CASE(1, 1, 1, 4) OCNN_TILE_CASE(2, 1, 1, 4) OCNN_TILE_CASE(3, 1, 2, 2) OCNN_TILE_CASE(2, 2, 1, 2)
-    OCNN_TILE_CASE(2, 4, 1, 1)
+    OCNN_TILE_CASE(2, 4, 1, 1) OCNN_TILE_CASE(1, 2, 1, 2)
 #undef OCNN_TILE_CASE
 #undef OCNN_TILE_LAUNCH
     return check_launch("conv_gather_tile");

@@ -77,6 +77,31 @@ def test_tile_kernel_wave_shapes(dtype, cin, cout, rows, K, spread):
       assert (got - want).abs().max() / want.abs().max() < TOL[dtype], (parts, occupancy)
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,rows,K,spread,occupancy', [
+    (96, 1152 * 128 + 5, 27, 110, 0.3),                  # the first tile, and the most rows, with three workgroups a CU
+    (96, 1152 * 128, 27, 110, 0.3), (32, 1152 * 128 + 5, 27, 120, 0.3),      # a tile less; more rows
+    (64, 1153 * 128, 3, 4, 0.45), (128, 1200 * 128 + 1, 1, 0, 0.1),          # slots: an odd number, fewer than waves
+    (32, 640 * 128 + 5, 27, 130, 1.0), (32, 640 * 128, 9, 20, 1.0),          # one chunk, nothing left out
+    (64, 641 * 128, 2, 3, 0.6)])
+def test_tile_kernel_waves_of_64_channels(dtype, cin, rows, K, spread, occupancy):
+  """64 output channels on both sides of the lines between their two divisions of the waves, against 64-bit sums."""
+  print('tile kernel, 64 channels', dtype, cin, 'rows', rows, 'K', K, flush=True)
+  g = torch.Generator().manual_seed(rows + cin)
+  t = (torch.arange(rows)[:, None] + torch.randint(-spread, spread + 1, (rows, K), generator=g)).clamp_(0, rows - 1).int()
+  t[torch.rand(rows, K, generator=g) < 0.6] = -1
+  t[(torch.rand(rows // 32 + 1, K, generator=g) < 0.3).repeat_interleave(32, 0)[:rows]] = -1
+  plan = TilePlan(t.cuda())
+  x = torch.randn(rows, cin, generator=g).to(dtype).cuda()
+  w = (torch.randn(K, cin, 64, generator=g) / (K * cin) ** 0.5).to(dtype).cuda()
+  b = torch.randn(64, generator=g).to(dtype).cuda()
+  zero = torch.cat([x.double(), torch.zeros(1, cin, dtype=torch.float64, device='cuda')])
+  want = b.double() + sum(zero[t[:, k].long().cuda()] @ w[k].double() for k in range(K))
+  got = _gather(x, plan, w, 64, False, False, b, (0, 0), occupancy)
+  assert (got.double() - want).abs().max() / want.abs().max() < TOL[dtype]
+  assert torch.equal(got, _gather(x, plan, w, 64, False, False, b, (0, 0), occupancy))
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
 def test_tile_kernel_weights_off_alignment(dtype):
   """Weights that start one element past a 16-byte boundary give the bits of aligned ones."""
