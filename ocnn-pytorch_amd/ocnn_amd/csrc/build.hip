@@ -229,24 +229,49 @@ __global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
   *(int4*)(t.children[d] + j) = c;
 }
 
+struct OpenLeaf {                // a leaf whose points a span does not hold all: its signals' sums so far
+  uint64_t key;
+  int64_t leaf;
+  int count;
+  float sum[6];
+};
+
+// mean point and normal of a leaf from the sums over its points
+__device__ __forceinline__ void leaf_signals(const BuildSignal& sig, int64_t leaf, const float* a, int64_t points) {
+  const float cnt = (float)points;
+#pragma unroll
+  for (int e = 0; e < 3; ++e) sig.out_pts[3 * leaf + e] = a[e] / cnt;
+  if (sig.out_nrm) {
+    const float len = fmaxf(sqrtf(a[3] * a[3] + a[4] * a[4] + a[5] * a[5]), 1e-12f);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) sig.out_nrm[3 * leaf + e] = a[3 + e] / len;
+  }
+}
+
 // Numbers every point's nodes (its span's offsets + the starts before it inside the span, counted
 // with wave ballots) and writes what the point starts: a leaf's entry in its parent's children, a
 // parent's eight keys, and so on up to the deepest full layer.  With signals, also the leaves' mean points and
 // normals: every thread fetches its points' 24 bytes, side by side with everything else, and the thread that starts a
 // leaf adds them from LDS in the order of the points (a launch of its own walked a leaf's points one behind the other,
-// each from memory: 5.6 us of them for 20 k points at depth 6).
+// each from memory: 5.6 us of them for 20 k points at depth 6).  The leaf that goes on in the spans behind is the whole
+// workgroup's: one thread walking on from memory waited for key, point number and signals of every point in turn.  Builds in us,
+// launch of its own / walked on / now: 1 M points of a cube at depth 2 9100 / 5680 / 570, depth 3 1870 / 1290 / 236, depth 4
+// 360 / 280 / 185; of a sphere at depth 5 460 / 427 / 205, depth 6 217 / 220 / 174, 3 M 508 / 600 / 375; 200 k points of one
+// cell 30300 / 51300 / 4760, one chain of additions.
 template <typename K, int N, int SPAN>
 __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     const K* __restrict__ sorted, const uint32_t* __restrict__ offs, const int32_t* __restrict__ perm, int64_t n,
     int key_bits, int depth, int full_depth, BuildTree t, BuildSignal sig, int64_t* __restrict__ inverse,
     int32_t* __restrict__ seg_start) {
   __shared__ uint32_t s_cnt[kBuildThreads / 64][N];
-  __shared__ float s_sig[6][SPAN];
+  __shared__ __attribute__((aligned(16))) float s_sig[6][SPAN];
   __shared__ uint8_t s_new[SPAN];                            // the point starts a leaf (or is none)
+  __shared__ OpenLeaf s_open;
   constexpr int kIt = SPAN / kBuildThreads;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = (int64_t)blockIdx.x * SPAN + wave * (SPAN / 4);
   const int levels = depth - full_depth;
+  if (threadIdx.x == 0) s_open.leaf = -1;
   int lv[kIt], at[kIt];
   uint32_t run[N];
 #pragma unroll
@@ -337,28 +362,60 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     if (!sig.rows) continue;
     float a[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     int j = wave * (SPAN / 4) + it * 64 + lane;
-    int64_t end = q;
+    const int from = j;
     do {
 #pragma unroll
       for (int e = 0; e < 6; ++e) a[e] += s_sig[e][j];
       ++j;
-      ++end;
     } while (j < SPAN && !s_new[j]);
-    if (j == SPAN)                                           // the leaf's points in the spans behind
-      for (; end < n && sorted[end] == (K)c; ++end) {
-        const float* from = (const float*)(sig.rows + 2 * (int64_t)perm[end]);
+    if (j < SPAN) {
+      leaf_signals(sig, leaf, a, j - from);
+    } else {                                                 // (one leaf of the span at most)
+      s_open.key = c;
+      s_open.leaf = leaf;
+      s_open.count = j - from;
 #pragma unroll
-        for (int e = 0; e < 6; ++e) a[e] += from[e];
-      }
-    const float cnt = (float)(end - q);
-#pragma unroll
-    for (int e = 0; e < 3; ++e) sig.out_pts[3 * (int64_t)leaf + e] = a[e] / cnt;
-    if (sig.out_nrm) {
-      const float len = fmaxf(sqrtf(a[3] * a[3] + a[4] * a[4] + a[5] * a[5]), 1e-12f);
-#pragma unroll
-      for (int e = 0; e < 3; ++e) sig.out_nrm[3 * (int64_t)leaf + e] = a[3 + e] / len;
+      for (int e = 0; e < 6; ++e) s_open.sum[e] = a[e];
     }
   }
+  if (!sig.rows) return;
+  // The leaf that reaches the end of the span, whose further points lie in the spans behind: 256 of them at a time to LDS, and
+  // six threads add their signals, in the order of the points
+  __syncthreads();
+  const int64_t leaf = s_open.leaf;
+  if (leaf < 0) return;
+  const K key = (K)s_open.key;
+  int64_t count = s_open.count;
+  float a = threadIdx.x < 6 ? s_open.sum[threadIdx.x] : 0.f;
+  for (int64_t first = ((int64_t)blockIdx.x + 1) * SPAN;; first += kBuildThreads) {
+    const int64_t q = first + threadIdx.x;
+    const bool mine = q < n && sorted[q] == key;             // (the points are sorted: the first so many threads)
+    float4 u = make_float4(0.f, 0.f, 0.f, 0.f), w = u;
+    if (q < n) {                                             // (not behind the comparison)
+      const float4* row = sig.rows + 2 * (int64_t)perm[q];
+      u = row[0];
+      if (sig.out_nrm) w = row[1];
+    }
+    s_sig[0][threadIdx.x] = u.x, s_sig[1][threadIdx.x] = u.y, s_sig[2][threadIdx.x] = u.z;
+    s_sig[3][threadIdx.x] = u.w, s_sig[4][threadIdx.x] = w.x, s_sig[5][threadIdx.x] = w.y;
+    const int more = __syncthreads_count(mine);
+    if (threadIdx.x < 6) {
+#pragma unroll 4
+      for (int j = 0; j < more; j += 4) {
+        const float4 v = *(const float4*)&s_sig[threadIdx.x][j];
+        a += v.x;
+        if (j + 1 < more) a += v.y;
+        if (j + 2 < more) a += v.z;
+        if (j + 3 < more) a += v.w;
+      }
+    }
+    count += more;
+    __syncthreads();
+    if (more < kBuildThreads) break;
+  }
+  if (threadIdx.x < 6) s_open.sum[threadIdx.x] = a;
+  __syncthreads();
+  if (threadIdx.x == 0) leaf_signals(sig, leaf, s_open.sum, count);
 }
 
 using ForceOnesweep = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
