@@ -111,10 +111,12 @@ constexpr int kBuildMaxDepth = 16;
 
 constexpr int kBuildThreads = 256;   // four waves, each on a run of consecutive points
 // Sorted points per workgroup of the counting and the scatter kernel: a thread's points follow each other, so that a cloud
-// too small to fill the chip is cut finer (256 points: 10.2 -> 9.1 us for 20 k points;
-// for 1 M points 6 us more than 1024)
+// too small to fill the chip is cut finer.  The line: counts, offsets and scatter in us, spans of 1024 / 256 points, of a sphere
+// 20 k points depth 6 24.2 / 14.9, 65 k depth 7 25.3 / 18.8, 100 k depth 6 31.4 / 19.9, 131 k depth 7 28.5 / 21.4, 262 k depths 7
+// and 8 31.0 / 26.6, 29.1 / 27.4, 400 k depth 7 36.0 / 36.1, 524 k depths 7 and 8 40.6 / 42.2, 36.4 / 42.4, 1 M depth 9 57.6 /
+// 81.8 (the one workgroup of the offsets has four times the spans to add: 5.2 / 15.7 us of these).
 constexpr int kBuildSpan = 1024, kBuildSmallSpan = 256;
-constexpr int64_t kBuildSmallPoints = 1 << 16;
+constexpr int64_t kBuildSmallPoints = 1 << 18;
 static int build_span(int64_t n) { return n <= kBuildSmallPoints ? kBuildSmallSpan : kBuildSpan; }
 
 // number of layers at which sorted point i starts a node, minus one (-1: same leaf as i - 1)

@@ -76,7 +76,7 @@ def test_leaf_averages_across_spans(n, depth, batch, same, normals):
     assert o.normals[depth] is None
 
 
-@pytest.mark.parametrize('n', [9001, 80001])
+@pytest.mark.parametrize('n', [9001, 262144, 262145])
 @pytest.mark.parametrize('long', [255, 256, 257, 511, 512, 513, 1023, 1025, 4096])
 def test_leaf_that_leaves_its_span(n, long):
   """One leaf of `long` points among leaves of few, wherever it lies in the spans of 256 and 1024 points: its signals are the
