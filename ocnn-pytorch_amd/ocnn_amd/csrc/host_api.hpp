@@ -99,7 +99,7 @@ int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int
                         int has_plan, int plan_max_distinct, int64_t plan_total, double plan_occupancy,
                         double plan_reuse, int plan_overflow);
 
-// ocnn_batch_norm_stats and ocnn_batch_norm_apply after each other: one launch where there are few rows.
+// ocnn_batch_norm_stats and ocnn_batch_norm_apply after each other: one or two launches where there are few rows.  y may be x.
 int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows, int channels, float eps, float* mean, float* var,
                               float* invstd, void* running_mean, void* running_var, int running_dtype, float factor,
                               int64_t* batches_tracked, const void* gamma, const void* beta, int param_dtype, int relu,

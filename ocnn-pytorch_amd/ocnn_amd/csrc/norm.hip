@@ -874,7 +874,8 @@ extern "C" int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows,
   OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_training: shape not supported");
   OCNN_REQUIRE_PTRS("batch_norm_training", x, mean, var, invstd, y, workspace);
   OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels), "batch_norm_training: workspace too small");
-  if (!bn_slabs_take(dtype, rows, channels, false)) {
+  // (in place: not as two launches, of which the second reads row 0, the sums' origin, in every workgroup beside the one that writes it)
+  if (!bn_slabs_take(dtype, rows, channels, false) || (y == x && rows > kBnSmallRows)) {
     const int status = ocnn_batch_norm_stats(dtype, x, rows, channels, eps, mean, var, invstd, running_mean, running_var,
                                              running_dtype, factor, batches_tracked, workspace, workspace_bytes, stream);
     if (status != OCNN_OK) return status;
