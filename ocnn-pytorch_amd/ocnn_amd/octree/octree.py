@@ -189,15 +189,21 @@ class TilePlan:
         del self.urows, self.loc
         self._unfilled = table
         return
-      self._fill(table)
+      self.urows, self.loc = self._lists(table)
 
   def __getattr__(self, name):
-    table = vars(self).get('_unfilled')
-    if table is None or name not in ('urows', 'loc'):
+    state = vars(self)
+    table = state.get('_unfilled') if name in ('urows', 'loc') else None
+    if table is None:
+      if name in state:                                    # (another thread has made them since)
+        return state[name]
       raise AttributeError(name)
     with torch.cuda.device(table.device):
-      self._fill(table)
-    return vars(self)[name]
+      made = dict(zip(('urows', 'loc'), self._lists(table)))
+      if not torch.cuda.is_current_stream_capturing():     # (a graph's tensors hold nothing before its first replay)
+        state.update(made)
+        state.pop('_unfilled', None)
+    return made[name]
 
   def _count(self, table, cap):
     """First of two passes: distinct rows per tile, their offsets, and the sizes on the host."""
@@ -212,14 +218,15 @@ class TilePlan:
     _lib.check(L.ocnn_tile_plan_offsets(P(ucount), P(tile_nnz), tiles, cap, P(self.uptr), P(stats), st))
     return ucount, stats.tolist()
 
-  def _fill(self, table):
+  def _lists(self, table):
     """Second pass: row lists and positions."""
     L, P, dev = _lib.lib(), _lib.ptr, table.device
     tile_rows = L.ocnn_tile_plan_rows()
-    self.urows = torch.empty(max(self.total, 1), dtype=torch.int32, device=dev)
+    urows = torch.empty(max(self.total, 1), dtype=torch.int32, device=dev)
     # uint16 payload, [tile][slot][row in tile]: whole tiles, the tail reads "empty"
-    self.loc = torch.empty((-(-self.rows // tile_rows), self.K, tile_rows), dtype=torch.int16, device=dev)
-    _lib.check(L.ocnn_tile_plan_fill(P(table), self.rows, self.K, P(self.uptr), P(self.urows), P(self.loc), _lib.stream()))
+    loc = torch.empty((-(-self.rows // tile_rows), self.K, tile_rows), dtype=torch.int16, device=dev)
+    _lib.check(L.ocnn_tile_plan_fill(P(table), self.rows, self.K, P(self.uptr), P(urows), P(loc), _lib.stream()))
+    return urows, loc
 
   def __getstate__(self):
     """(copies leave out the layers' native passes, which are made again when asked for)"""

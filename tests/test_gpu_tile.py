@@ -273,3 +273,25 @@ def test_lists_that_no_kernel_reads_are_made_when_read(rows, K, entries):
     assert torch.equal(p.loc, two.loc) and torch.equal(p.urows[:p.total], two.urows[:two.total]) and torch.equal(p.uptr, two.uptr)
   with pytest.raises(AttributeError):
     plan.nothing
+
+
+def test_lists_first_read_under_capture():
+  """A capture records the lists and positions it reads and keeps none of them, which hold nothing before the first replay;
+  a plan that has made them lets go of its table."""
+  g = torch.Generator().manual_seed(8)
+  t = torch.stack([torch.randperm(100000, generator=g)[:8] for _ in range(300)]).int().cuda()
+  plan, want = TilePlan(t), TilePlan(t, cap=4000)
+  assert 'loc' not in vars(plan)
+  graph = torch.cuda.CUDAGraph()
+  torch.cuda.synchronize()
+  with torch.cuda.graph(graph):
+    recorded = plan.loc.clone(), plan.urows.clone()
+  assert 'loc' not in vars(plan) and 'urows' not in vars(plan)
+  assert torch.equal(plan.loc, want.loc) and torch.equal(plan.urows[:plan.total], want.urows[:want.total])
+  assert 'loc' in vars(plan) and '_unfilled' not in vars(plan)
+  for _ in range(3):
+    for r in recorded:
+      r.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(recorded[0], want.loc) and torch.equal(recorded[1][:want.total], want.urows[:want.total])
