@@ -8,6 +8,7 @@
 // made (nn/octree_conv.py); run() allocates the result and a workspace and calls the library.  A
 // ConvLayer holds the up to three passes of a layer on an octree; conv() is its autograd node.
 #include <ATen/ATen.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -19,6 +20,7 @@
 #include <atomic>
 #include <chrono>
 #include <memory>
+#include <mutex>
 #include <optional>
 #include <vector>
 
@@ -57,6 +59,26 @@ Tensor workspace(int64_t bytes, const Tensor& like) {
   return at::empty({std::max<int64_t>(bytes, 256)}, like.options().dtype(at::kByte));
 }
 
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+
+// The rows of the tiles of several plans in the order of ocnnx_plan_order, by their positions.
+std::vector<Tensor> tile_orders(const std::vector<Tensor>& locs) {
+  std::vector<Tensor> out;
+  std::vector<ocnnx_order_item> items;
+  int64_t tiles = 0;
+  for (const Tensor& loc : locs) {
+    require_gpu(loc);
+    TORCH_CHECK(loc.scalar_type() == at::kShort && loc.dim() == 3 && loc.size(2) == ocnn_tile_plan_rows() &&
+                    loc.is_contiguous() && loc.device() == locs[0].device(),
+                "tile_orders: positions of tile plans of one device");
+    out.push_back(at::empty({loc.size(0), OCNNX_TILE_ORDER_BYTES}, loc.options().dtype(at::kByte)));
+    items.push_back({typed<uint16_t>(loc), typed<uint8_t>(out.back()), loc.size(0), tiles, (int)loc.size(1)});
+    tiles += loc.size(0);
+  }
+  if (!items.empty()) check(ocnnx_plan_order(items.data(), (int)items.size(), hip_stream()));
+  return out;
+}
+
 // The arrays and figures of a tile plan and, where a kernel walks pairs, of its pair plan.
 struct PlanArrays {
   Tensor loc, uptr, urows;
@@ -68,7 +90,31 @@ struct PlanArrays {
   int max_blocks = 0, n_lists = 0;
   std::vector<int32_t> lists_host, group_bounds;
   std::vector<int64_t> list_count;
+
+  // The order of the tiles' rows that the passes on this plan share, made by the first that runs without it; null under a
+  // capture that finds none: what a graph makes holds nothing before its first replay, and a pass is right without.
+  const uint8_t* rows_order() {
+    std::lock_guard<std::mutex> lock(order_lock);
+    if (!order.defined() && !capturing()) {
+      at::tracer::impl::NoTracerDispatchMode quiet;
+      order = tile_orders({loc})[0];
+    }
+    return typed<uint8_t>(order);
+  }
+  std::mutex order_lock;
+  Tensor order;
 };
+
+// rows_order() of several plans, in one launch
+void order_many(const std::vector<std::shared_ptr<PlanArrays>>& plans) {
+  std::vector<Tensor> locs;
+  for (const auto& p : plans) locs.push_back(p->loc);
+  const std::vector<Tensor> orders = tile_orders(locs);
+  for (size_t i = 0; i < plans.size(); ++i) {
+    std::lock_guard<std::mutex> lock(plans[i]->order_lock);
+    if (!plans[i]->order.defined()) plans[i]->order = orders[i];
+  }
+}
 
 // codes on top of the library's OCNN_GATHER_* / OCNN_WGRAD_*
 constexpr int kWgradSparseInverse = 5;        // the pair plan of the inverse table, operands exchanged
@@ -78,7 +124,7 @@ struct GatherOp {
   int64_t rows_in = 0, rows = 0, ws_bytes = 0;
   bool transposed = false, reverse = false;
   std::shared_ptr<PlanArrays> plan;
-  Tensor order;                               // OCNNX_GATHER_TILE: the tiles' rows in the order the kernel takes them
+  bool ordered = false;                       // OCNNX_GATHER_TILE: the kernel takes the plan's rows_order()
   // dense one-slot form: rows read / written through an index of the non-empty nodes
   Tensor in_index, out_index, children;
   int64_t rows_all = 0;                       // rows of the padded result
@@ -167,6 +213,7 @@ struct GatherOp {
   // the kernel for this shape, of a table with these figures of its plan, and the workspace it takes
   void choose(int code, bool dense, bool has_plan, int umax, int64_t total, double occupancy, double reuse, bool overflows) {
     kernel = ocnnx_gather_choose(code, rows_in, rows, K, cin, cout, dense, has_plan, umax, total, occupancy, reuse, overflows);
+    ordered = kernel == OCNNX_GATHER_TILE && ocnnx_gather_tile_ordered(K, occupancy);
     ws_bytes = kernel == OCNN_GATHER_ZERO_PADDED || kernel == OCNNX_GATHER_ROWS ? 0
                : kernel == OCNN_GATHER_SPARSE ? ocnn_conv_gather_sparse_workspace_bytes(cin, cout)
                : kernel == OCNNX_GATHER_TILE  ? ocnnx_gather_tile_workspace_bytes(code, rows, K, cin, cout)
@@ -179,7 +226,7 @@ struct GatherOp {
     const PlanArrays& p = *plan;
     return {data, rows_in, typed<uint16_t>(p.loc), typed<int32_t>(p.uptr), typed<int32_t>(p.urows), p.umax, p.total,
             p.occupancy, rows, K, W, cin, cout, transposed, reverse, bias, bn, out.data_ptr(), ws.data_ptr(), ws.numel(), 0, 0,
-            order.defined() ? typed<uint8_t>(order) : nullptr};
+            ordered ? plan->rows_order() : nullptr};
   }
 
   // this pass with row i of its result written to row index[i] of `out`
@@ -770,24 +817,6 @@ std::vector<BuiltPlan> tile_plans(const std::vector<Tensor>& tables, int cap, in
   return out;
 }
 
-// The rows of the tiles of several plans in the order of ocnnx_plan_order, by their positions.
-std::vector<Tensor> tile_orders(const std::vector<Tensor>& locs) {
-  std::vector<Tensor> out;
-  std::vector<ocnnx_order_item> items;
-  int64_t tiles = 0;
-  for (const Tensor& loc : locs) {
-    require_gpu(loc);
-    TORCH_CHECK(loc.scalar_type() == at::kShort && loc.dim() == 3 && loc.size(2) == ocnn_tile_plan_rows() &&
-                    loc.is_contiguous() && loc.device() == locs[0].device(),
-                "tile_orders: positions of tile plans of one device");
-    out.push_back(at::empty({loc.size(0), OCNNX_TILE_ORDER_BYTES}, loc.options().dtype(at::kByte)));
-    items.push_back({typed<uint16_t>(loc), typed<uint8_t>(out.back()), loc.size(0), tiles, (int)loc.size(1)});
-    tiles += loc.size(0);
-  }
-  if (!items.empty()) check(ocnnx_plan_order(items.data(), (int)items.size(), hip_stream()));
-  return out;
-}
-
 // The neighbour tables of layers 1 .. depth (entry 0 is left out) of an octree as `tree` was built; none if
 // a layer is not, any more: keys, children and counts are public and may be assigned.
 std::vector<Tensor> all_neigh(const Tree& tree, const std::vector<OptTensor>& keys_now, const std::vector<Tensor>& children,
@@ -840,8 +869,12 @@ PYBIND11_MODULE(ocnn_host, m) {
       }))
 #define FIELD(name) .def_readwrite(#name, &PlanArrays::name)
       FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(umax) FIELD(total) FIELD(occupancy) FIELD(cptr) FIELD(ent) FIELD(lists)
-          FIELD(n_blocks) FIELD(max_blocks) FIELD(n_lists) FIELD(lists_host) FIELD(group_bounds) FIELD(list_count);
+          FIELD(n_blocks) FIELD(max_blocks) FIELD(n_lists) FIELD(lists_host) FIELD(group_bounds) FIELD(list_count)
 #undef FIELD
+      .def_property_readonly("order", [](PlanArrays& p) {
+        std::lock_guard<std::mutex> lock(p.order_lock);
+        return p.order.defined() ? OptTensor(p.order) : std::nullopt;
+      });
   py::class_<GatherOp, std::shared_ptr<GatherOp>>(m, "GatherOp")
       .def(py::init<>())
       .def(py::init([](int64_t rows_in, int64_t rows, int K, int cin, int cout, bool transposed, bool reverse) {
@@ -852,7 +885,7 @@ PYBIND11_MODULE(ocnn_host, m) {
       }))
 #define FIELD(name) .def_readwrite(#name, &GatherOp::name)
       FIELD(kernel) FIELD(K) FIELD(cin) FIELD(cout) FIELD(rows_in) FIELD(rows) FIELD(ws_bytes) FIELD(transposed)
-          FIELD(reverse) FIELD(plan) FIELD(order) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
+          FIELD(reverse) FIELD(plan) FIELD(ordered) FIELD(in_index) FIELD(out_index) FIELD(children) FIELD(rows_all)
               FIELD(overflow_table) FIELD(overflow_rows) FIELD(overflow) FIELD(padded) FIELD(bias_repeat) FIELD(view_cols)
 #undef FIELD
       .def("choose", &GatherOp::choose)
@@ -932,7 +965,7 @@ PYBIND11_MODULE(ocnn_host, m) {
       FIELD(loc) FIELD(uptr) FIELD(urows) FIELD(ucount) FIELD(stats);
 #undef FIELD
   m.def("tile_plans", &tile_plans, py::call_guard<py::gil_scoped_release>());
-  m.def("tile_orders", &tile_orders, py::call_guard<py::gil_scoped_release>());
+  m.def("order_many", &order_many, py::call_guard<py::gil_scoped_release>());
   m.def("build_octree", &build_octree, py::call_guard<py::gil_scoped_release>());
   m.def("all_neigh", &all_neigh, py::call_guard<py::gil_scoped_release>());
   m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;

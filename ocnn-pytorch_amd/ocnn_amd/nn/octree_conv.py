@@ -126,10 +126,8 @@ def _gather_op(dtype, rows_in, rows, K, cin, cout, transposed, reverse, plan=Non
   else:
     if op.kernel in (_lib.GATHER_RW, _lib.GATHER_TILE, _lib.GATHER_SPARSE, _lib.GATHER_PLANNED):
       op.plan = _plan_arrays(plan, op.kernel == _lib.GATHER_SPARSE)
-      # (an order made under capture would hold nothing before the graph's first replay)
-      if op.kernel == _lib.GATHER_TILE and L.ocnnx_gather_tile_ordered(K, float(plan.occupancy)) and \
-          (plan._order is not None or not torch.cuda.is_current_stream_capturing()):
-        op.order = plan.order()
+      if op.ordered:
+        plan.wish_order()
       if plan.overflow_rows is not None:
         op.overflow_rows, op.overflow_table = plan.overflow_rows, plan.overflow_table
         op.overflow = _gather_op(dtype, rows_in, plan.overflow_table.shape[0], K, cin, cout, transposed, reverse)

@@ -124,7 +124,7 @@ class TilePlan:
   in the middle of a training step wants: every read-back waits for the whole queue of kernels
   before it and leaves the device idle while the host catches up."""
 
-  _order = _siblings = None
+  _siblings = None
   CAP = 415      # the smallest limit of the kernels on the plan
   LIST_PAD = 416  # rows a tile's list may have in the one-pass build
   MOST_STAGED = 511  # tiles of more rows are for the multi-pass kernel alone, which takes tables of at least
@@ -160,7 +160,7 @@ class TilePlan:
     self.overflow_rows = self.overflow_table = None
     self._pairs = None
     self._on_pairs = None          # called when the pair plan is first asked for
-    self._order = self._on_order = self._siblings = self._on_siblings = None
+    self._on_order = self._siblings = self._on_siblings = None
     if built is not None and not built.stats[5]:
       self.uptr, self.urows, self.loc, ucount, stats = built.uptr, built.urows, built.loc, built.ucount, built.stats
     else:
@@ -266,22 +266,34 @@ class TilePlan:
         self._on_siblings()
     return self._siblings
 
+  @property
+  def _order(self):
+    """order() as far as it has been made.  (The native view of the plan holds it: its passes make it when they run without.)"""
+    arrays = vars(self).get('_native')
+    return None if arrays is None else arrays.order
+
   def order(self):
     """The rows of each tile in the order in which the tile kernel takes them, and the live blocks of its slots
     (ocnnx_plan_order; made on first use)."""
-    if self._order is None:
-      self.order_many([self])
-      if self._on_order is not None:
-        self._on_order()
+    self.wish_order()
     return self._order
+
+  def wish_order(self):
+    """order() for a pass on this plan.  Not under capture, where it would hold nothing before the graph's first replay."""
+    if self._order is None and not torch.cuda.is_current_stream_capturing():
+      self.order_many([self])
+    noted, self._on_order = self._on_order, None
+    if noted is not None:
+      noted()
 
   @staticmethod
   def order_many(plans):
     """order() of several plans, in one launch."""
+    from ..nn.octree_conv import _plan_arrays
+    plans = [plan for plan in plans if plan._order is None]
     if plans:
       with torch.cuda.device(plans[0].loc.device):
-        for plan, order in zip(plans, _lib.native().tile_orders([p.loc for p in plans])):
-          plan._order = order
+        _lib.native().order_many([_plan_arrays(plan, False) for plan in plans])
 
 
 class PairPlan:
@@ -864,6 +876,8 @@ class Octree:
           walk(x)
       elif isinstance(v, (TilePlan, PairPlan, _NeighTables)):
         walk(vars(v))
+        if isinstance(v, TilePlan):
+          walk(v._order)
 
     walk(vars(self))
     if self._built is not None:

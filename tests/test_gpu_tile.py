@@ -295,3 +295,33 @@ def test_lists_first_read_under_capture():
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(recorded[0], want.loc) and torch.equal(recorded[1][:want.total], want.urows[:want.total])
+
+
+def test_layer_first_called_under_capture():
+  """A layer whose pass is made while a graph is captured, on a plan that is there already: no order comes out of the capture,
+  the first call after it makes one, and all give the same rows to the bit."""
+  from ocnn_amd import synthetic
+  from ocnn_amd.nn import OctreeConv
+  from ocnn_amd.octree import Octree, Points
+  from ocnn_amd.octree.octree import PlanHistory
+  pts, nrm = synthetic.mixed_cloud(20000, seed=9)
+  octree = Octree(6, 2)
+  octree.plan_history = PlanHistory()
+  octree.build_octree(Points(pts.cuda(), nrm.cuda()))
+  octree.construct_all_neigh()
+  plan = octree._plan(6, '333', 1, True)
+  layer = OctreeConv(96, 96, [3], 1, nempty=True).cuda().half()
+  x = torch.randn(int(octree.nnum_nempty[6]), 96, device='cuda').half()
+  graph = torch.cuda.CUDAGraph()
+  torch.cuda.synchronize()
+  with torch.no_grad():
+    with torch.cuda.graph(graph):
+      recorded = layer(x, octree, 6)
+    assert plan._order is None and octree.plan_history.wished((6, 2), 'order')
+    eager = layer(x, octree, 6)
+    assert np.array_equal(plan._order.cpu().numpy(), _row_order(plan))
+    for turn in range(3):
+      recorded.zero_()
+      graph.replay()
+      torch.cuda.synchronize()
+      assert torch.equal(recorded, eager) and torch.equal(layer(x, octree, 6), eager), turn
