@@ -79,6 +79,43 @@ std::vector<Tensor> tile_orders(const std::vector<Tensor>& locs) {
   return out;
 }
 
+// The end of what the current stream has been given so far, for what is made once and read by later work of any stream.
+class MadeHere {
+ public:
+  MadeHere() : stream_(c10::hip::getCurrentHIPStream().stream()) {
+    TORCH_CHECK(hipEventCreateWithFlags(&event_, hipEventDisableTiming) == hipSuccess &&
+                    hipEventRecord(event_, stream_) == hipSuccess,
+                "cannot record an event");
+  }
+  ~MadeHere() { (void)hipEventDestroy(event_); }
+  MadeHere(const MadeHere&) = delete;
+  MadeHere& operator=(const MadeHere&) = delete;
+
+  // Makes the current stream wait for it, if need be.  False under a capture that it has not come true before: a graph
+  // cannot wait for an event from outside.
+  bool before_current() {
+    if (done_) return true;
+    const bool captures = capturing();
+    const hipStream_t st = c10::hip::getCurrentHIPStream().stream();
+    if (!captures && st == stream_) return true;
+    // (asking is no part of a capture, of this thread or another's)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t status = hipEventQuery(event_);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (status == hipSuccess) return done_ = true;
+    (void)hipGetLastError();
+    if (captures) return false;
+    TORCH_CHECK(hipStreamWaitEvent(st, event_, 0) == hipSuccess, "cannot wait for an event");
+    return true;
+  }
+
+ private:
+  hipStream_t stream_;
+  hipEvent_t event_ = nullptr;
+  std::atomic<bool> done_{false};
+};
+
 // The arrays and figures of a tile plan and, where a kernel walks pairs, of its pair plan.
 struct PlanArrays {
   Tensor loc, uptr, urows;
@@ -91,18 +128,21 @@ struct PlanArrays {
   std::vector<int32_t> lists_host, group_bounds;
   std::vector<int64_t> list_count;
 
-  // The order of the tiles' rows that the passes on this plan share, made by the first that runs without it; null under a
-  // capture that finds none: what a graph makes holds nothing before its first replay, and a pass is right without.
+  // The order of the tiles' rows that the passes on this plan share, made by the first that runs without it and waited for
+  // on other streams; null under a capture that finds none: what a graph makes holds nothing before its first replay, and a
+  // pass is right without.
   const uint8_t* rows_order() {
     std::lock_guard<std::mutex> lock(order_lock);
     if (!order.defined() && !capturing()) {
       at::tracer::impl::NoTracerDispatchMode quiet;
       order = tile_orders({loc})[0];
+      order_made = std::make_shared<MadeHere>();
     }
-    return typed<uint8_t>(order);
+    return order.defined() && order_made->before_current() ? typed<uint8_t>(order) : nullptr;
   }
   std::mutex order_lock;
   Tensor order;
+  std::shared_ptr<MadeHere> order_made;
 };
 
 // rows_order() of several plans, in one launch
@@ -110,9 +150,12 @@ void order_many(const std::vector<std::shared_ptr<PlanArrays>>& plans) {
   std::vector<Tensor> locs;
   for (const auto& p : plans) locs.push_back(p->loc);
   const std::vector<Tensor> orders = tile_orders(locs);
+  const auto made = std::make_shared<MadeHere>();
   for (size_t i = 0; i < plans.size(); ++i) {
     std::lock_guard<std::mutex> lock(plans[i]->order_lock);
-    if (!plans[i]->order.defined()) plans[i]->order = orders[i];
+    if (plans[i]->order.defined()) continue;
+    plans[i]->order = orders[i];
+    plans[i]->order_made = made;
   }
 }
 

@@ -325,3 +325,35 @@ def test_layer_first_called_under_capture():
       graph.replay()
       torch.cuda.synchronize()
       assert torch.equal(recorded, eager) and torch.equal(layer(x, octree, 6), eager), turn
+
+
+@pytest.mark.parametrize('together', [False, True])
+def test_order_made_on_another_stream(together):
+  """A pass waits for an order that is still on its way on the stream it is made on, whoever asked for it."""
+  from ocnn_amd.nn.octree_conv import _gather_op
+  g = torch.Generator().manual_seed(11)
+  rows, K = 6000, 27
+  t = (torch.arange(rows)[:, None] + torch.randint(-30, 31, (rows, K), generator=g)).clamp_(0, rows - 1).int()
+  t[torch.rand(rows, K, generator=g) < 0.8] = -1
+  t = t.cuda()
+  x, w = torch.randn(rows, 96, generator=g).cuda(), (torch.randn(K, 96, 96, generator=g) / 50).cuda()
+  plan, alone = TilePlan(t), TilePlan(t)
+  want = _gather_op(torch.float32, rows, rows, K, 96, 96, False, False, alone).run(x, t, w, None)
+  busy, side = torch.randn(4096, 4096, device='cuda'), torch.cuda.Stream()
+  side.wait_stream(torch.cuda.current_stream())
+  torch.cuda.synchronize()
+  with torch.cuda.stream(side):
+    for _ in range(60):
+      product = busy @ busy
+    if together:
+      TilePlan.order_many([plan])
+    else:
+      plan.order()
+  op = _gather_op(torch.float32, rows, rows, K, 96, 96, False, False, plan)
+  assert op.ordered and op.kernel == _lib.GATHER_TILE
+  got = op.run(x, t, w, None)
+  assert not side.query(), 'the other stream was not busy'
+  torch.cuda.synchronize()
+  assert torch.equal(got, want) and torch.equal(op.run(x, t, w, None), want)
+  assert torch.equal(plan.order(), alone.order())
+  del product
