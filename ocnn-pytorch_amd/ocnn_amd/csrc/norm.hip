@@ -424,14 +424,24 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
 // 39 k x 96 17.9 / 25.0, 12.8 / 22.3; fp16 2048 x 256 (one launch before) 12.8 / 20.2, 9.5 / 12.5; 20 k x 96 15.8 / 22.5, 11.1 / 15.4;
 // 60 k x 128 24.4 / 39.5, 17.5 / 31.8.  The lines:
 // * one launch up to 1024 rows: fp32 x 256 800 rows 6.3 / 7.9, two 7.4 / 8.6; 1425 rows 7.7 / 10.1, two 7.2 / 8.8;
-// * the three launches, whose workgroups have whole rows, from 32 MB on forward (fp32 33 k x 256 two 24.4, three 26.4; 66 k x 256
-//   43.9, 41.0) and from 20 MB on backward (60 k x 128 38.8, 38.1; 66 k x 64 24.9, 27.2), where a row's pieces no longer meet in a
-//   cache;
+// * the three launches, whose workgroups have whole rows, where the elementwise pass is more than a round of workgroups, of
+//   which a CU holds one (registers).  Two / three launches: one round, fp32 130 k x 32 forward 14.2 / 19.4, 60 k x 32 backward
+//   14.1 / 18.0, 60 k x 40 forward 12.6 / 16.1; fp16 64 k x 120 forward 20.2 / 24.1.  What more rounds are worth hangs on the rows:
+//   - of one line of 128 bytes or less, and of channels that leave a workgroup's last part of a row empty, nothing: fp32
+//     160 k x 16 17.9 / 17.6, 27.6 / 22.7, 98 k x 32 backward 23.7 / 22.2, 66 k x 40 17.4 / 16.6, 28.8 / 21.7, 36 k x 104 19.9 /
+//     18.1, 31.9 / 24.5; fp16 131 k x 64 backward 39.9 / 35.3, 150 k x 64 33.3 / 25.6, 24 k x 200 backward 38.0 / 33.4 (less than
+//     a line in two parts backward a little: 84 k x 40 27.3 / 29.4, 90 k x 48 29.7 / 32.9, 84 k x 56 30.8 / 32.3);
+//   - forward two rounds in fp32 (66 k x 64 17.4 / 20.0, 131 k x 64 25.0 / 25.8, 33 k x 256 21.0 / 26.4; the third 87 k x 96 26.3 /
+//     25.3), in 16 bits of whole 512 bytes (66 k x 256 27.8 / 29.5, 33 k x 512 28.9 / 30.8; 74 k x 128 27.0 / 25.0, 60 k x 192
+//     26.6 / 25.5, 40 k x 320 29.2 / 27.1);
+//   - backward two (fp16 66 k x 128 36.3 / 40.0, 82 k 46.4 / 42.9, 30 k x 320 44.7 / 41.6; fp32 60 k x 64 23.1 / 25.4, 74 k 29.7 /
+//     29.3), of more than 256 bytes in fp32 and of whole 512 bytes in 16 bits two and a half (fp32 37 k x 128 26.0 / 29.2,
+//     9.2 k x 512 27.7 / 30.3; fp16 41 k x 256 40.1 / 42.0, 20 k x 512 42.2 / 43.4);
 // * 128 bytes of a row, whole lines, from 4 MB on in fp32 (20 k x 128: 9.7 / 17.3, with 64 bytes 11.0 / 23.7), from 12 MB on in 16
 //   bits, where they are 64 channels (39 k x 96 15.4 / 28.6, with 64 bytes 13.1 / 20.6; 33 k x 256 21.3 / 37.5, 22.4 / 46.2).
 constexpr int kBnSlabThreads = 1024;
-constexpr int64_t kBnSmallRows = 1024, kBnSlabRows = 131072;
-constexpr int64_t kBnSlabForward = 32 << 20, kBnSlabBackward = 20 << 20, kBnWideF32 = 4 << 20, kBnWide16 = 12 << 20;
+constexpr int64_t kBnSmallRows = 1024, kBnRound = 256, kBnWideF32 = 4 << 20, kBnWide16 = 12 << 20;
+constexpr int kBnUnrollForward = 4, kBnUnrollBackward = 2;   // passes over the rows that a workgroup of the elementwise pass takes, at most
 constexpr int kBnSlabRanges = 64;         // of the sums, at most (more where the channels are few slabs: a workgroup on every CU)
 
 // sums over the workgroup of the 2 VEC values of each thread, per thread of a row: s_out[kind][channel of the
@@ -754,7 +764,7 @@ static BnSlabs bn_slabs(int dtype, int64_t rows, int channels, int unroll) {
     return s;
   }
   const int64_t pass = kBnSlabThreads / s.lanes;
-  const int64_t some = std::min<int64_t>(unroll, std::max<int64_t>(1, cdiv(rows * s.slabs, 256 * pass))) * pass;
+  const int64_t some = std::min<int64_t>(unroll, std::max<int64_t>(1, cdiv(rows * s.slabs, kBnRound * pass))) * pass;
   s.sums_per = (int)std::max(some, align_up(cdiv(rows, std::max(kBnSlabRanges, 256 / s.slabs)), pass));
   s.ranges = (int)cdiv(rows, s.sums_per);
   s.per = (int)some;
@@ -762,15 +772,20 @@ static BnSlabs bn_slabs(int dtype, int64_t rows, int channels, int unroll) {
   return s;
 }
 
-// (three launches for more than these)
+// (three launches for rows of more workgroups than these; the lines above)
 static bool bn_slabs_take(int dtype, int64_t rows, int channels, bool backward) {
-  const int64_t limit = backward ? kBnSlabBackward : kBnSlabForward;
   if (rows <= kBnSmallRows) return true;
-  if (rows > kBnSlabRows || channels < (dtype == OCNN_F32 ? 16 : 32)) return false;
-  // 128 bytes are 64 channels of 16 bits: where they leave half a slab empty, or (backward) are the whole row, no further than
-  // 64 bytes are good for (130 k x 96 forward 31.6, three launches 28.8; 130 k x 64 backward 39.1, 35.6)
-  const bool narrow = dtype != OCNN_F32 && (channels % 64 != 0 || (backward && channels == 64));
-  return rows * channels * (dtype == OCNN_F32 ? 4 : 2) <= (narrow ? std::min(limit, kBnWide16 - 1) : limit);
+  if (channels < (dtype == OCNN_F32 ? 16 : 32)) return false;
+  const int unroll = backward ? kBnUnrollBackward : kBnUnrollForward;
+  const BnSlabs s = bn_slabs(dtype, rows, channels, unroll);
+  const int vec = dtype == OCNN_F32 ? 4 : 8, row_bytes = channels * 16 / vec;
+  const bool wide = dtype == OCNN_F32 || row_bytes % 512 == 0;
+  int64_t most = kBnRound;
+  if (channels % (s.lanes * vec) == 0 && row_bytes > 128)
+    most = backward ? (wide && row_bytes > 256 ? 5 * kBnRound / 2 : 2 * kBnRound) : (wide ? 2 * kBnRound : kBnRound);
+  else if (backward && row_bytes < 128 && s.slabs == 2)
+    most = 2 * kBnRound;
+  return rows * s.slabs <= most * unroll * (kBnSlabThreads / s.lanes);
 }
 
 }  // namespace ocnn
@@ -883,7 +898,7 @@ extern "C" int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows,
                     0, 0.f, (hipStream_t)stream);
   }
   const BnStats keep{eps, mean, var, invstd, running_mean, running_var, running_dtype, factor, (long long*)batches_tracked};
-  const BnSlabs s = bn_slabs(dtype, rows, channels, 4);
+  const BnSlabs s = bn_slabs(dtype, rows, channels, kBnUnrollForward);
   double* partial = s.split ? (double*)workspace : nullptr;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
@@ -920,7 +935,7 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
                "batch_norm_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
   if (dx && bn_slabs_take(dtype, rows, channels, true)) {
-    const BnSlabs s = bn_slabs(dtype, rows, channels, 2);
+    const BnSlabs s = bn_slabs(dtype, rows, channels, kBnUnrollBackward);
     double* partial = s.split ? (double*)workspace : nullptr;
     OCNN_DISPATCH_DTYPE(dtype, {
       constexpr int VEC = 16 / sizeof(T);

@@ -361,6 +361,7 @@ def test_batch_norm_few_rows(dtype):
   workgroup, 64 and 128 bytes of a row, the last sizes that two launches take and the first of three."""
   sizes = [(33, 8), (64, 32), (255, 40), (256, 1024), (1023, 24), (2048, 96), (2049, 96), (1024, 40), (1025, 40), (1025, 8), (2500, 1000),
            (8192, 128), (8193, 128), (131072, 32), (131073, 32)]
+  sizes += [(65536, 32), (65537, 40), (60000, 48), (32768, 256), (32769, 256), (40960, 128)]
   sizes += [(70000, 72)] if dtype == torch.float32 else [(65536, 96), (65535, 96), (98304, 64)]
   for rows, c in sizes:
     say('batch norm, few rows', dtype, rows, c)
