@@ -1544,6 +1544,36 @@ def test_dwconv_backward_planned(dtype, K, ch, groups):
         assert torch.equal(got.cpu()[~touched], gw.cpu()[~touched])
 
 
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('K,groups', [(27, False), (27, True), (9, False), (3, True)])
+def test_dwconv_backward_planned_overflow_tiles(dtype, K, groups):
+  """Both gradients from one pass where the densest tiles are left out of the plan and run apart, the weight gradient with its
+  slots mirrored, on any symmetric table and on tables of sibling groups, whose left-out tiles still count as such."""
+  from ocnn_amd.nn.octree_dwconv import dw_backward
+  from ocnn_amd.octree.octree import TilePlan
+  g = torch.Generator().manual_seed(5 * K + groups)
+  rows, ch = 128 * 60 + (8 if groups else 7), 64
+  table = _lattice_table(rows, K, g, groups)
+  counts = sorted(int((t.unique() >= 0).sum()) for t in table.split(128))
+  tg = table.to(DEV)
+  plan = TilePlan(tg, cap=counts[-4] - 1)                  # (at most a tenth of the tiles: they may have as many rows)
+  left_out = sum(c >= counts[-4] for c in counts)
+  assert 4 <= left_out <= 6 and plan.overflow_rows is not None and plan.umax == max(c for c in counts if c < counts[-4])
+  plan.reuse = 10.0
+  assert plan.siblings == (groups and K == 27)
+  t64 = table.numpy().astype(np.int64)
+  x = torch.randn(rows, ch, generator=g).to(dtype)
+  gr = (torch.randn(rows, ch, generator=g) / rows ** 0.5).to(dtype)
+  w = torch.randn(K, 1, ch, generator=g).to(dtype)
+  dx, gw = dw_backward(x.to(DEV), gr.to(DEV), tg, w.to(DEV), plan)
+  assert rel_err(dx, C.dw_forward(f64(gr), f64(w)[::-1], t64)) < TOL[dtype]
+  # (the rows that run apart add a second rounded sum to the first)
+  assert rel_err(gw, C.dw_weight(f64(x), f64(gr), t64)) < 2 * TOL[dtype]
+  apart = plan.overflow_rows.cpu().numpy()
+  assert rel_err(dx.cpu()[apart], C.dw_forward(f64(gr), f64(w)[::-1], t64)[apart]) < TOL[dtype]
+  assert all(torch.equal(a, b) for a, b in zip((dx, gw), dw_backward(x.to(DEV), gr.to(DEV), tg, w.to(DEV), plan)))
+
+
 def test_dwconv_planned_non_finite_values_stay_in_their_group_of_four():
   """The planned depth-wise gather multiplies on the 4x4x4 matrix instruction with diag(w) as one
   operand, so 0 x inf of one channel reaches the other three channels of its group of four as

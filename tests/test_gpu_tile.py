@@ -1,6 +1,8 @@
 """The gather-GEMM of csrc/conv_tile.hip at the edges of its ranges: rows around a tile, every
 division of the waves, halves of a 64-channel chunk, and the reduction in one and several parts."""
 
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -26,6 +28,17 @@ def _gather(x, plan, w, cout, transposed, reverse, b, parts, occupancy):
                                  occupancy, plan.rows, K, P(w), cin, cout, int(transposed), int(reverse), P(b), None, P(out),
                                  P(ws), size, *parts, _lib.stream()))
   return out
+
+
+def _ordered_pass(dtype, plan, rows_in, cin, cout, transposed, reverse):
+  """A layer's pass on the tile kernel with the plan's row order, whichever kernel the layers of its shape take."""
+  from ocnn_amd.nn.octree_conv import _plan_arrays
+  code = _lib.DTYPE_CODE[dtype]
+  op = _lib.native().GatherOp(rows_in, plan.rows, plan.K, cin, cout, transposed, reverse)
+  assert _lib.lib().ocnnx_gather_tile_supported(code, rows_in, plan.K, cin, cout, plan.umax)
+  op.kernel, op.ordered, op.plan = _lib.GATHER_TILE, True, _plan_arrays(plan, False)
+  op.ws_bytes = _lib.lib().ocnnx_gather_tile_workspace_bytes(code, plan.rows, plan.K, cin, cout)
+  return op
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
@@ -85,7 +98,8 @@ def test_tile_kernel_wave_shapes(dtype, cin, cout, rows, K, spread):
     (32, 640 * 128 + 5, 27, 130, 1.0), (32, 640 * 128, 9, 20, 1.0),          # one chunk, nothing left out
     (64, 641 * 128, 2, 3, 0.6)])
 def test_tile_kernel_waves_of_64_channels(dtype, cin, rows, K, spread, occupancy):
-  """64 output channels on both sides of the lines between their two divisions of the waves, against 64-bit sums."""
+  """64 output channels on both sides of the lines between their two divisions of the waves, against 64-bit sums; with the
+  rows in the plan's order, as the layers run where empty blocks are left out, to the bit as without."""
   print('tile kernel, 64 channels', dtype, cin, 'rows', rows, 'K', K, flush=True)
   g = torch.Generator().manual_seed(rows + cin)
   t = (torch.arange(rows)[:, None] + torch.randint(-spread, spread + 1, (rows, K), generator=g)).clamp_(0, rows - 1).int()
@@ -100,6 +114,9 @@ def test_tile_kernel_waves_of_64_channels(dtype, cin, rows, K, spread, occupancy
   got = _gather(x, plan, w, 64, False, False, b, (0, 0), occupancy)
   assert (got.double() - want).abs().max() / want.abs().max() < TOL[dtype]
   assert torch.equal(got, _gather(x, plan, w, 64, False, False, b, (0, 0), occupancy))
+  if _lib.lib().ocnnx_gather_tile_ordered(K, occupancy):
+    assert _lib.lib().ocnnx_gather_tile_ordered(K, plan.occupancy)
+    assert torch.equal(got, _ordered_pass(dtype, plan, rows, cin, 64, False, False).run(x, None, w, b))
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
@@ -171,9 +188,8 @@ def _row_order(plan):
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('cin,cout,K', [(96, 96, 27), (32, 64, 27), (160, 128, 9), (64, 256, 27), (128, 128, 3), (32, 32, 27)])
 def test_tile_kernel_row_order(dtype, cin, cout, K):
-  """The order of a tile's rows, and the layers' pass that takes them in it: one row, a remainder, whole tiles, tiles enough
-  for 256 channels a workgroup, rows without an entry, mirrored slots."""
-  from ocnn_amd.nn.octree_conv import _gather_op
+  """The order of a tile's rows, and the pass that takes them in it: one row, a remainder, whole tiles, tiles enough
+  for 256 channels a workgroup, rows without an entry, mirrored slots; to the bit as in the table's order."""
   for rows in (1, 129, 2048, 257 * 128 + 5):
     print('tile kernel, order', dtype, cin, cout, 'rows', rows, 'K', K, flush=True)
     g = torch.Generator().manual_seed(rows + cin)
@@ -188,10 +204,9 @@ def test_tile_kernel_row_order(dtype, cin, cout, K):
     zero = torch.cat([x.double(), torch.zeros(1, cin, dtype=torch.float64, device='cuda')])
     for reverse in (False, True):
       w = (torch.randn((K, cout, cin) if reverse else (K, cin, cout), generator=g) / (K * cin) ** 0.5).to(dtype).cuda()
-      op = _gather_op(dtype, rows, rows, K, cin, cout, reverse, reverse, plan)
-      if op.kernel != _lib.GATHER_TILE:
-        continue
+      op = _ordered_pass(dtype, plan, rows, cin, cout, reverse, reverse)
       got = op.run(x, t.cuda(), w, b).double()
+      assert torch.equal(got, _gather(x, plan, w, cout, reverse, reverse, b, (0, 0), plan.occupancy).double())
       at = lambda k: w[K - 1 - k].T.double() if reverse else w[k].double()
       want = b.double() + sum(zero[t[:, k].long().cuda()] @ at(k) for k in range(K))
       assert (got - want).abs().max() / want.abs().max() < TOL[dtype], reverse
@@ -210,6 +225,11 @@ def test_orders_of_several_plans():
   TilePlan.order_many(plans)
   for p, a in zip(plans, alone):
     assert torch.equal(p.order(), a) and np.array_equal(a.cpu().numpy(), _row_order(p))
+  others = copy.deepcopy(plans)                            # (copies make theirs again)
+  assert all(p._order is None for p in others)
+  TilePlan.order_many(others)
+  for p, a in zip(others, alone):
+    assert torch.equal(p._order, a)
 
 
 def test_fresh_octree_orders_the_plans_of_its_predecessors():
@@ -261,7 +281,6 @@ def test_fresh_octree_finds_the_sibling_groups_its_predecessors_were_asked_for()
 @pytest.mark.parametrize('rows,K,entries', [(500, 8, 512), (500, 8, 700), (300, 8, 100000), (1000, 27, 1000)])
 def test_lists_that_no_kernel_reads_are_made_when_read(rows, K, entries):
   """Tiles of more rows than any kernel stages, each used about once: lists and positions are those of the two passes."""
-  import copy
   g = torch.Generator().manual_seed(rows + entries)
   t = torch.stack([torch.randperm(max(entries, K), generator=g)[:K] for _ in range(rows)]).int().cuda()
   plan, other, two = TilePlan(t), TilePlan(t), TilePlan(t, cap=4000)
