@@ -50,17 +50,16 @@ static __device__ __forceinline__ void tg_dma16(__amdgpu_buffer_rsrc_t rs, char*
 // per MFMA the same tables took 6 - 10 % longer.  The rows of a block are read one block ahead, behind a branch of their own.
 //
 // order: the tile's rows in an order that leaves fewer blocks with an entry (plan.hip: tile_order_kernel); position i of
-// a block is row order[i].  It costs the loop nothing (a lane's row is a register either way) and the sums of a row are the
-// same, but which wave adds those of its block.  What bounds the loop on such tables is neither MFMAs nor bytes alone: 96 -> 96 on the
-// 1.13 M rows of depth 9, 7 % set, 334 us: 139 without any slot (rows, results and the chain of loads in front), 280 with a
-// quarter of the MFMAs, 290 with one fetch of weights a chunk.  A turn of the loop therefore waits for as little as can be: two sets
-// of registers in turn in place of copies, the blocks that are live known beforehand (334 -> 320 us), half the weights of
-// half a chunk, 0.24 instead of 0.39 of the blocks by the order (298), and the live blocks of a slot as a byte behind the order in
-// place of 54 reads of LDS and 27 ballots a tile (293).  In us before / now, f16: 947 k rows 15 % set
-// 96 -> 96 329 / 292, 533 k 31 % 128 -> 128 299 / 264, 160 k 38 % 256 -> 256 383 / 341, 40 k 42 % 155 / 143, 822 k 14 % 96 -> 96
-// 333 / 294, 31 k 17 % 26.7 / 21.9, nine slots of 1.13 M rows 234 / 213; fp32 132 k 36 % 96 -> 96 153 / 145, 264 k 22 % 64 -> 64 132 /
-// 124 (105 with three workgroups a CU: tile_half_waves), 19 k 128 -> 128 60 / 59.  (Tables above the line below gain where a cloud is flat, 1.28 M rows 68 % set 96 -> 96 620 / 576, and lose elsewhere,
-// 97 k 52 % 256 -> 256 282 / 292: they stay without.)
+// a block is row order[i].  It costs the loop nothing (a lane's row is a register either way), and a row's result is the
+// same to the bit (of finite values): it has the same products in every wave, and the waves' sums meet in the same pairs whichever block the row
+// is in.  Neither MFMAs nor bytes alone bound the loop on such tables (96 -> 96 on 1.13 M rows, 7 % set: 139 us without any slot,
+// 280 with a quarter of the MFMAs, 290 with one fetch of weights a chunk), so a turn of it waits for as little as can be:
+// two sets of registers in turn, the live blocks of a slot known beforehand from a byte behind the order, half the weights
+// of half a chunk.  In us before / now: f16 1.13 M rows 7 % set 96 -> 96 334 / 293, 947 k 15 % 329 / 292, 533 k 31 % 128 -> 128
+// 299 / 264, 160 k 38 % 256 -> 256 383 / 341, 31 k 17 % 96 -> 96 26.7 / 21.9; fp32 132 k 36 % 96 -> 96 153 / 145, 264 k 22 %
+// 64 -> 64 132 / 124 (105 with three workgroups a CU: tile_half_waves).  Up to two thousand rows the order's own fetch shows: 1.8 k
+// rows 28 % set 128 -> 128 20.5 / 21.5, fp32 96 -> 96 22.5 / 23.5, 32 -> 64 13.7 / 13.1.  Above the line of kTgSkipMaxOccupancy
+// it gains where a cloud is flat (1.28 M rows 68 % set 96 -> 96 620 / 576) and loses elsewhere (97 k 52 % 256 -> 256 282 / 292).
 //
 // The four waves: WC along the output channels (32 MB each), WR along the rows (RB = 4 / WR blocks of 32 rows
 // each), KS over the slots (each takes every KS-th; their sums are added in LDS at the end).
@@ -335,7 +334,8 @@ __global__ __launch_bounds__(256, MB * (4 / WR) <= 4 ? 3 : 2) void conv_gather_t
   if constexpr (!F32)
     if (nfull < c1) staged_chunk(nfull, std::integral_constant<int, 2>{});   // half a chunk: its first two k-steps
 
-  // ---- KS > 1: the waves' sums of a block are added by one of them, in the order of the waves ----
+  // ---- KS > 1: the waves' sums of a block are added by one of them: of two waves, or of four as (0 + 2) + (1 + 3), the
+  // same pairs for every block and whichever wave has it ----
   if constexpr (KS > 1) {
     f32x4* ex = (f32x4*)s_rows;
     constexpr int kPart = RBK * MB * 4 * 64;                 // a wave's sums of the blocks of one owner

@@ -198,7 +198,8 @@ __global__ __launch_bounds__(kDpThreads, 1) void dw_siblings_kernel(
 #pragma unroll 1
         for (int it = 0; it < 32; ++it) {                  // sibling it / 4 of group 4 G + it % 4
           const int g = 4 * G + (it & 3), s = it >> 2;
-          const T v = *(const T*)((const char*)s_x + (8 * g + (s ^ (g & 1))) * 128 + ((2 * ch) ^ (((g >> 1) & 1) << 6) ^ (((g >> 2) & 1) << 5)));
+          const int at = (8 * g + (s ^ (g & 1))) * 128 + ((2 * ch) ^ (((g >> 1) & 1) << 6) ^ (((g >> 2) & 1) << 5));
+          const T v = *(const T*)((const char*)s_x + at);
           if ((((__builtin_bit_cast(uint16_t, v) & 0x7fffu) + kOne) & 0x8000u) == 0u) continue;
 #pragma unroll 1
           for (int k = 0; k < kDsK; ++k) {
