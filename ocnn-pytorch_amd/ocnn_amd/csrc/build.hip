@@ -257,9 +257,10 @@ __device__ __forceinline__ void leaf_signals(const BuildSignal& sig, int64_t lea
 // leaf adds them from LDS in the order of the points (a launch of its own walked a leaf's points one behind the other,
 // each from memory: 5.6 us of them for 20 k points at depth 6).  The leaf that goes on in the spans behind is the whole
 // workgroup's: one thread walking on from memory waited for key, point number and signals of every point in turn.  Builds in us,
-// launch of its own / walked on / now: 1 M points of a cube at depth 2 9100 / 5680 / 570, depth 3 1870 / 1290 / 236, depth 4
-// 360 / 280 / 185; of a sphere at depth 5 460 / 427 / 205, depth 6 217 / 220 / 174, 3 M 508 / 600 / 375; 200 k points of one
-// cell 30300 / 51300 / 4760, one chain of additions.
+// launch of its own / walked on / now: 1 M points of a cube at depth 2 9100 / 5680 / 570, depth 3 1870 / 1290 / 240, depth 4
+// 360 / 285 / 187; of a sphere at depth 5 460 / 428 / 207, depth 6 217 / 220 / 174, 3 M 508 / 600 / 372; 200 k points of one
+// cell 30300 / 51400 / 4580, one chain of additions.  (Where the next span starts a leaf, as most do, nothing follows the walk:
+// with the further points asked for in every span a build of 1 M points at depth 9 took 6 us more.)
 template <typename K, int N, int SPAN>
 __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     const K* __restrict__ sorted, const uint32_t* __restrict__ offs, const int32_t* __restrict__ perm, int64_t n,
@@ -273,6 +274,8 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = (int64_t)blockIdx.x * SPAN + wave * (SPAN / 4);
   const int levels = depth - full_depth;
+  const int64_t behind = ((int64_t)blockIdx.x + 1) * SPAN;
+  const bool goes_on = sig.rows && behind < n && sorted[behind] == sorted[behind - 1];   // a leaf does, in the span behind
   if (threadIdx.x == 0) s_open.leaf = -1;
   int lv[kIt], at[kIt];
   uint32_t run[N];
@@ -370,7 +373,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
       for (int e = 0; e < 6; ++e) a[e] += s_sig[e][j];
       ++j;
     } while (j < SPAN && !s_new[j]);
-    if (j < SPAN) {
+    if (j < SPAN || !goes_on) {
       leaf_signals(sig, leaf, a, j - from);
     } else {                                                 // (one leaf of the span at most)
       s_open.key = c;
@@ -380,21 +383,23 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
       for (int e = 0; e < 6; ++e) s_open.sum[e] = a[e];
     }
   }
-  if (!sig.rows) return;
-  // The leaf that reaches the end of the span, whose further points lie in the spans behind: 256 of them at a time to LDS, and
-  // six threads add their signals, in the order of the points
+  if (!goes_on) return;
+  // The leaf whose further points lie in the spans behind: 256 of them at a time to LDS, and six threads add their signals, in
+  // the order of the points
   __syncthreads();
   const int64_t leaf = s_open.leaf;
   if (leaf < 0) return;
   const K key = (K)s_open.key;
   int64_t count = s_open.count;
   float a = threadIdx.x < 6 ? s_open.sum[threadIdx.x] : 0.f;
-  for (int64_t first = ((int64_t)blockIdx.x + 1) * SPAN;; first += kBuildThreads) {
+  for (int64_t first = behind;; first += kBuildThreads) {
     const int64_t q = first + threadIdx.x;
-    const bool mine = q < n && sorted[q] == key;             // (the points are sorted: the first so many threads)
+    const K k = q < n ? sorted[q] : (K)0;
+    const int32_t point = q < n ? perm[q] : 0;               // (beside the key, not behind it)
+    const bool mine = q < n && k == key;                     // (the points are sorted: the first so many threads)
     float4 u = make_float4(0.f, 0.f, 0.f, 0.f), w = u;
-    if (q < n) {                                             // (not behind the comparison)
-      const float4* row = sig.rows + 2 * (int64_t)perm[q];
+    if (mine) {
+      const float4* row = sig.rows + 2 * (int64_t)point;
       u = row[0];
       if (sig.out_nrm) w = row[1];
     }
