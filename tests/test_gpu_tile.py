@@ -344,6 +344,14 @@ def test_layer_first_called_under_capture():
       graph.replay()
       torch.cuda.synchronize()
       assert torch.equal(recorded, eager) and torch.equal(layer(x, octree, 6), eager), turn
+    graph = torch.cuda.CUDAGraph()                         # with an order that another stream has made
+    with torch.cuda.graph(graph):
+      recorded = layer(x, octree, 6)
+    for turn in range(3):
+      recorded.zero_()
+      graph.replay()
+      torch.cuda.synchronize()
+      assert torch.equal(recorded, eager) and torch.equal(layer(x, octree, 6), eager), turn
 
 
 @pytest.mark.parametrize('together', [False, True])
