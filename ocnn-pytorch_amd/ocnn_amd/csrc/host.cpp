@@ -752,8 +752,11 @@ void wait_for(const Tensor& values, const c10::hip::HIPStream& st) {
 Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<float> bbmin, double factor, int depth,
                   int full_depth, int batch_size) {
   require_gpu(pts);
+  for (const OptTensor* t : {&normals, &batch})              // (their pointers go to kernels)
+    TORCH_CHECK(!t->has_value() || (*t)->device() == pts.device(), "build_octree: points, normals and batch ids on one device");
   pts = pts.to(at::kFloat).contiguous();
   const int64_t n = pts.size(0);
+  TORCH_CHECK(!normals.has_value() || normals->numel() == 3 * n, "build_octree: a normal for every point");
   TORCH_CHECK(batch_size == 1 || (batch.has_value() && batch->numel() == n), "build_octree: a batch id for every point");
   bool batch_is_float = false;
   if (batch.has_value()) {

@@ -100,6 +100,25 @@ def test_leaf_that_leaves_its_span(n, long):
     assert np.abs(o.normals[5].cpu().numpy() - sums[:, 3:] / length).max() < 1e-6
 
 
+def test_normals_and_batch_ids_of_another_device_are_refused():
+  """Host memory is not handed to the build's kernels."""
+  g = torch.Generator().manual_seed(2)
+  pts = (torch.rand(500, 3, generator=g) - 0.5).cuda()
+  mixed = Points(pts)
+  mixed.normals = torch.randn(500, 3, generator=g)
+  with pytest.raises(RuntimeError, match='one device'):
+    Octree(4, 2).build_octree(mixed)
+  ids = (torch.arange(500) % 2).float().view(-1, 1)
+  mixed = Points(pts, batch_id=ids.cuda(), batch_size=2)
+  mixed.batch_id = ids
+  with pytest.raises(RuntimeError, match='one device'):
+    Octree(4, 2, batch_size=2).build_octree(mixed)
+  mixed = Points(pts)
+  mixed.normals = torch.randn(499, 3, generator=g).cuda()
+  with pytest.raises(RuntimeError, match='every point'):
+    Octree(4, 2).build_octree(mixed)
+
+
 def test_cloud_in_one_leaf_takes_no_time_a_point():
   """200 000 points of one cell: their sums are one chain of additions, 4.7 ms, but not one of fetches (30 to 51 ms with a
   point fetched at a time; the bound is half of the former)."""
