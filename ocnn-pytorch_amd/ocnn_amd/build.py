@@ -34,6 +34,7 @@ SOURCES = {
     'dw_planned.hip': [],
     'dw_siblings.hip': [],
     'wgrad_planned.hip': [],
+    'wgrad_f32.hip': [],
     'plan.hip': [],
     'misc.hip': [],
     'select.hip': [],

@@ -20,6 +20,7 @@
 #include "jobs.hpp"
 #include "mma.hpp"
 #include "reduce.hpp"
+#include "wgrad_f32.hpp"
 
 namespace ocnn {
 
@@ -68,8 +69,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
     const uint16_t* __restrict__ loc, uint32_t loc_bytes, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ urows, uint32_t urows_bytes, int64_t tiles,
-    int64_t tiles_per_split, int workgroups, int ca, int cb, float* __restrict__ partial,
-    const T* __restrict__ x_lo, const T* __restrict__ g_lo, int64_t set) {
+    int64_t tiles_per_split, int workgroups, int ca, int cb, float* __restrict__ partial) {
   int number = (int)xcd_tile(blockIdx.x, gridDim.x >> 3);
   if (number >= workgroups) return;
   const int grp = number % GROUPS;
@@ -78,11 +78,6 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   const int nbb = BLK ? (cb + CB - 1) / CB : 1, nblocks = BLK ? nbb * ((ca + CA - 1) / CA) : 1;
   const int block = __builtin_amdgcn_readfirstlane(number % nblocks);
   const int split = __builtin_amdgcn_readfirstlane(number / nblocks);
-  // fp32 data as bf16 pieces: hi hi, hi lo, lo hi, each with sums of its own.  (A product's number is a grid
-  // index of its own: out of a division it made the pointers, and every staging load, vectors.)
-  if (blockIdx.y == 1) g = g_lo;
-  if (blockIdx.y == 2) x = x_lo;
-  partial += blockIdx.y * set;
   constexpr int HA = CA / 32, HB = CB / 32;   // 32-channel halves of a row of x, of g
   constexpr int NU = HA * NFULL + NHALF;      // 32 x CB accumulator units per wave
   constexpr int NS = NFULL + NHALF;           // distinct slots per wave
@@ -400,34 +395,32 @@ using namespace ocnn;
 // blocks have room for the sums of all 27 slots in one workgroup, and for the 32 x 32 layer
 static bool wp_wide(int ca) { return ca > 32; }
 
-// workgroups of one range of tiles (and one product of bf16 pieces): the slot groups, the blocks of channel pairs
+// workgroups of one range of tiles: the slot groups, the blocks of channel pairs
 static int wp_range_workgroups(int K, int ca, int cb) {
   const int groups = (K == 27 && wp_wide(ca)) ? 2 : 1;
   return groups * ((ca + 63) / 64) * ((cb + 63) / 64);
 }
 
 // ranges of tiles at most: as many as keep a workgroup on every CU (the LDS holds one)
-static int wp_splits(int K, int ca, int cb, int n_cu, int products) {
-  return std::min(256, std::max(8, n_cu / (wp_range_workgroups(K, ca, cb) * products)));
-}
+static int wp_splits(int range_workgroups, int n_cu) { return std::min(256, std::max(8, n_cu / range_workgroups)); }
 
 // Tiles of a range, for the least time of
 //   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
 //   the first tile, writing the sums) + the sums of all ranges written and read back, in units of one tile's time.
 // Measured (fp16, 64 x 64 blocks of 27 slots): 2.45 us a tile and 8 us besides on 33 - 157 tiles a range; the sums
-// move at about 3.5 TB/s.  Rounds are counted on an XCD's CUs (64 -> 64 in fp32 with 42 ranges is 33
-// workgroups on 32 CUs: 245 us where 40 ranges take 143), the sums where there are few tiles (256 -> 256 in fp32: 21 MB a range).
-constexpr double kWpFixed = 3.3, kWpSumCost = 2.3e-7;        // tiles; tiles a byte of sums
-static int64_t wp_tiles_per_range(int64_t tiles, int K, int ca, int cb, int n_cu, int products) {
-  const int wgs = wp_range_workgroups(K, ca, cb), cu_xcd = std::max(1, n_cu / 8);
-  const double sums = (double)K * ca * cb * 4 * products * kWpSumCost;      // of one range
+// move at about 3.5 TB/s.  Rounds are counted on an XCD's CUs (40 CUs' worth of workgroups on 32 are two rounds), the sums
+// where there are few tiles (256 -> 256: 7 MB a range).
+constexpr double kWpTileUs = 2.45, kWpFixedUs = 8.085, kWpSumUs = 5.635e-7; // us; us a byte of sums
+static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, int n_cu) {
+  const int cu_xcd = std::max(1, n_cu / 8);
   int64_t best = std::max<int64_t>(tiles, 1);
   double least = 1e30;
-  for (int s = 1, most = wp_splits(K, ca, cb, n_cu, products); s <= most; ++s) {
+  for (int s = 1, most = wp_splits(wgs, n_cu); s <= most; ++s) {
     const int64_t per = std::max<int64_t>(1, cdiv(tiles, s));
     const int64_t used = cdiv(tiles, per);
     if (used < s) continue;                                  // (the same ranges as fewer)
-    const double cost = (double)cdiv(cdiv(used * wgs, 8) * products, cu_xcd) * ((double)per + kWpFixed) + (double)used * sums;
+    const double cost = (double)cdiv(cdiv(used * wgs, 8), cu_xcd) * ((double)per * kWpTileUs + kWpFixedUs) +
+                        (double)used * (double)sums_bytes * kWpSumUs;
     if (cost < least) least = cost, best = per;
   }
   return best;
@@ -446,7 +439,7 @@ static int wp_cu_count() {
 
 extern "C" int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int64_t rows, int K, int ca,
                                                  int cb, int plan_max_distinct) {
-  if (dtype != OCNN_F16 && dtype != OCNN_BF16 && dtype != OCNN_F32) return 0;   // (fp32: as bf16 pieces)
+  if (dtype != OCNN_F16 && dtype != OCNN_BF16 && dtype != OCNN_F32) return 0;   // (fp32: wgrad_f32.hip)
   if (ca < 32 || cb < 32 || ca % 32 != 0 || cb % 32 != 0 || ca > 1024 || cb > 1024)
     return 0;
   if (K != 27 && K != 9 && K != 8 && K != 3) return 0;
@@ -458,23 +451,21 @@ extern "C" int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int6
 
 extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes(int K, int ca, int cb) {
   const int n_cu = wp_cu_count();
-  const int64_t splits = n_cu > 0 ? wp_splits(K, ca, cb, n_cu, 1) : 256;
+  const int64_t splits = n_cu > 0 ? wp_splits(wp_range_workgroups(K, ca, cb), n_cu) : 256;
   return align_up(splits * K * ca * cb * 4, 256);
 }
 
-// fp32: three sets of per-range sums (hi_x hi_g, hi_x lo_g, lo_x hi_g) after the bf16 pieces
-// of both tensors
 extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes_for(int dtype, int64_t rows_x, int64_t rows, int K,
                                                                int ca, int cb) {
-  const int64_t sums = ocnn_conv_wgrad_planned_workspace_bytes(K, ca, cb);
-  if (dtype != OCNN_F32 || rows_x < 0 || rows < 0) return sums;
-  return 2 * align_up(rows_x * ca * 2, 256) + 2 * align_up(rows * cb * 2, 256) + 3 * sums;
+  if (dtype != OCNN_F32 || rows_x < 0 || rows < 0) return ocnn_conv_wgrad_planned_workspace_bytes(K, ca, cb);
+  const int n_cu = wp_cu_count();
+  const int64_t tiles = cdiv(rows, kWpRows), run = n_cu > 0 ? wf_split_tiles(tiles, K, ca, cb, n_cu).run : 1;
+  return align_up(cdiv(tiles, run) * K * ca * cb * 4, 256);
 }
 
 struct WpArgs {
-  const void *x, *g, *x_lo, *g_lo;            // x_lo, g_lo: the low bf16 pieces of fp32 data (products = 3)
-  int products;
-  int64_t rows_x, rows, set, per, plan_total;
+  const void *x, *g;
+  int64_t rows_x, rows, per, plan_total;
   const uint16_t* loc;
   const int32_t *uptr, *urows;
   int K, ca, cb, used;                        // used: ranges of tiles
@@ -489,9 +480,8 @@ static void launch_wp(const WpArgs& a, hipStream_t st) {
   const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(a.plan_total * 4);
 #define OCNN_WP_KERNEL(BLK_)                                                                                        \
   hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, CA, CB, KK, NFULL, NHALF, GROUPS, BLK_>),                                  \
-                     dim3(8 * (unsigned)cdiv(wgs, 8), a.products), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g,    \
-                     gb, a.loc, lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial, (const T*)a.x_lo,     \
-                     (const T*)a.g_lo, a.set)
+                     dim3(8 * (unsigned)cdiv(wgs, 8)), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g, gb, a.loc,       \
+                     lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial)
   if (a.ca == CA && a.cb == CB)
     OCNN_WP_KERNEL(false);
   else if constexpr (CB == 64)
@@ -522,17 +512,16 @@ static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
 #undef OCNN_WP_LAUNCH
 }
 
-// T: the type of x, g and gw.  float: x and g go through the kernel as two bf16 pieces each, the three
-// products as workgroups of one launch with sums of their own (a third of the ranges each: a third
-// of the sums to add up, and one launch where a small layer waited for three), one reduction over all of them
+// T: the type of x, g and gw (float: wgrad_f32.hip)
 template <typename T> struct WpPass : Pass {
+  static constexpr bool F32 = std::is_same<T, float>::value;
   WpArgs a;
   hipStream_t st;
+  WfSplit f32;
   int rc = OCNN_OK, splits = 0, out_transposed = 0;
   void* gw = nullptr;         // set: the reduction is launched behind the kernel (sums at an odd address)
 
   WpPass(const ocnnx_wgrad_args& p, hipStream_t stream) : st(stream) {
-    constexpr bool kPieces = std::is_same<T, float>::value;
     const int n_cu = wp_cu_count();
     if (n_cu <= 0) {
       set_error("conv_wgrad_planned: cannot query the device");
@@ -540,30 +529,22 @@ template <typename T> struct WpPass : Pass {
       return;
     }
     const int K = p.K, ca = p.ca, cb = p.cb;
-    a = WpArgs{p.x, p.g, nullptr, nullptr, kPieces ? 3 : 1, p.rows_x, p.rows, 0, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0,
-               nullptr};
-    const int64_t tiles = cdiv(p.rows, kWpRows);
-    a.per = wp_tiles_per_range(tiles, K, ca, cb, n_cu, a.products);
-    a.used = (int)cdiv(tiles, a.per);
-    a.set = (int64_t)a.used * K * ca * cb;                   // floats of one set of sums
-    const int64_t nx = p.rows_x * ca, ng = p.rows * cb;
-    const int64_t xb = kPieces ? align_up(nx * 2, 256) : 0, gb = kPieces ? align_up(ng * 2, 256) : 0;
-    if (p.workspace_bytes < 2 * xb + 2 * gb + a.products * a.set * 4) {
+    a = WpArgs{p.x, p.g, p.rows_x, p.rows, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0, (float*)p.workspace};
+    const int64_t tiles = cdiv(p.rows, kWpRows), sums = (int64_t)K * ca * cb * 4;       // bytes of a range's sums
+    if (F32) {
+      f32 = wf_split_tiles(tiles, K, ca, cb, n_cu);
+      a.used = (int)cdiv(tiles, f32.run);
+    } else {
+      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, n_cu);
+      a.used = (int)cdiv(tiles, a.per);
+    }
+    if (p.workspace_bytes < a.used * sums) {
       set_error("conv_wgrad_planned: workspace too small");
       rc = OCNN_ERR_WORKSPACE;
       return;
     }
-    char* ws = (char*)p.workspace;
-    a.partial = (float*)(ws + 2 * xb + 2 * gb);
-    if (kPieces && p.rows > 0) {
-      bf16 *xh = (bf16*)ws, *xl = (bf16*)(ws + xb), *gh = (bf16*)(ws + 2 * xb), *gl = (bf16*)(ws + 2 * xb + gb);
-      Job j{Job::kSplit, (unsigned)cdiv((nx + ng) / 8, 256), {}};
-      j.split = SplitJob{(const float*)p.x, (const float*)p.g, xh, xl, gh, gl, nx, ng};
-      before.add(j);
-      a.x = xh, a.x_lo = xl, a.g = gh, a.g_lo = gl;
-    }
     const int64_t per = (int64_t)K * ca * cb;
-    splits = p.rows > 0 ? a.products * a.used : 0;
+    splits = p.rows > 0 ? a.used : 0;
     if ((uintptr_t)a.partial % 16 != 0) {
       gw = p.gw, out_transposed = p.out_transposed;
       return;
@@ -575,7 +556,12 @@ template <typename T> struct WpPass : Pass {
   }
 
   int main() override {
-    if (a.rows > 0) launch_wp_sums<typename std::conditional<std::is_same<T, float>::value, bf16, T>::type>(a, st);
+    if (a.rows > 0) {
+      if constexpr (F32)
+        launch_wgrad_f32({(const float*)a.x, (const float*)a.g, a.rows_x, a.rows, a.plan_total, a.loc, a.uptr, a.urows, a.K, a.ca,
+                          a.cb, f32, a.partial}, st);
+      else launch_wp_sums<T>(a, st);
+    }
     if (gw) launch_wgrad_reduce<T>(a.partial, splits, a.K, a.ca, a.cb, out_transposed, (T*)gw, st);
     return check_launch("conv_wgrad_planned");
   }

@@ -697,6 +697,41 @@ def test_planned_weight_gradient_fp32(K, ca, cb):
     assert torch.equal(gwt, gw.transpose(1, 2).contiguous())
 
 
+@pytest.mark.parametrize('K,ca,cb', [(K, ca, cb) for K in (27, 9, 8, 3) for ca, cb in ((32, 32), (32, 64), (64, 96), (96, 32))] +
+                         [(3, 256, 256), (3, 256, 160)])
+def test_planned_weight_gradient_fp32_edges(K, ca, cb):
+  """The fp32 kernel on ragged tiles, ranges of one to several tiles, odd numbers of them, the slots in one and in two
+  parts, ranges of several sets of sums (256 channels), and tiles of exactly as many distinct rows as are staged; a row of x that nobody names is infinite (list ends load
+  row 0).  Element by element against float64: of a product's four pieces lo lo is left out (|lo| <= 2^-9 of the value),
+  and the low pieces are rounded themselves (2^-18 each): 3 x 2^-18 of the sum of the absolute products, and an fp32 sum of
+  them in ranges and by 16-row steps (2^-24 a step)."""
+  from ocnn_amd.octree.octree import TilePlan
+  g = torch.Generator().manual_seed(K * ca + cb)
+  for rows, rows_in, full in [(1, 3, 0), (127, 300, 0), (129, 90, 0), (128 * 3, 128 * 3, 0), (256, 2000, 1), (128 * 131 + 5, 9000, 0),
+                              (128 * 523 + 77, 70000, 0)]:
+    table = _local_table(rows, rows_in - 1, K, g, spread=20) + 1
+    table[table == 0] = -1                               # (rows 1 .. rows_in - 1, and none)
+    if full and K >= 8:
+      table[:, :4] = 1 + (torch.arange(rows)[:, None] % 128 * 4 + torch.arange(4)) % 415 + (torch.arange(rows)[:, None] // 128) * 415
+      table[:, 4:] = -1
+    table = table.to(torch.int32).contiguous()
+    tg = table.to(DEV)
+    plan = TilePlan(tg)
+    assert not (full and K >= 8) or plan.umax == 415
+    say('planned weight gradient, fp32, edges', 'K', K, ca, cb, 'rows', rows, 'rows_in', rows_in)
+    x = torch.randn(rows_in, ca, generator=g)
+    gr = torch.randn(rows, cb, generator=g)
+    dead = x.clone()
+    dead[0] = float('inf')
+    gw = ocnn_amd.nn.conv_wgrad(dead.to(DEV), gr.to(DEV), tg, False, plan).cpu().double()
+    t = table.long()
+    at = lambda m, k: torch.where((t[:, k] >= 0)[:, None], m.double()[t[:, k].clamp(min=0)], 0.0)
+    want = torch.stack([at(x, k).t() @ gr.double() for k in range(K)])
+    size = torch.stack([at(x, k).abs().t() @ gr.double().abs() for k in range(K)])
+    bound = (3 * 2.0 ** -18 + (rows / 16 + 300) * 2.0 ** -24) * size + 1e-30
+    assert bool(((gw - want).abs() <= bound).all()), float(((gw - want).abs() / bound).max())
+
+
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('cin,cout', [(64, 128), (128, 512), (512, 128), (256, 256), (1024, 384), (192, 1024)])
 def test_dense_rows_kernel(dtype, cin, cout):
