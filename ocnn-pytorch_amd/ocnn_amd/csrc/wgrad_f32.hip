@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
 
   constexpr int HB = CB / 32, NS = (KK + 4 * GROUPS - 1) / (4 * GROUPS);
   constexpr int NU = NS * HB, NM = 3 * NU;                   // sums of 32 x 32 a wave; MFMAs a step
-  constexpr int NL = 2 * NS;                                 // look-ups of positions a lane and step
+  constexpr int NL = 2 * NS;                                 // rows of x a lane and step
   constexpr int kSlot = 2 * HB * 512;                        // elements of 16 rows of g: [piece][half][16][32]
   constexpr bool kRing = CB == 64;                           // else two whole buffers of g
   constexpr int kSlots = kRing ? 9 : 16;
@@ -92,13 +92,14 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
   const int64_t t_end = min(tiles, t_begin + tiles_per_split);
   if (t_begin >= t_end) return;
 
-  // lane (i16, gq): rows 8 q + 4 h + i16 / 4 of a 16-row step, channels 16 (gq & 1) + 4 (i16 & 3) ..
+  // lane (i16, gq): places 8 q + 4 h + i16 / 4 of a 16-row step, channels 16 (gq & 1) + 4 (i16 & 3) ..; step 2u + p has row
+  // 32 u + 16 q + 4 (i16 / 4) + 2 p + h there (wgrad_planned.hip)
   const int i16 = lane & 15, gq = lane >> 4, q = lane >> 5, rs = i16 >> 2;
   const uint32_t byte0 = 32u * (gq & 1) + 8u * (i16 & 3);
   const int slot0 = NS * (4 * grp + wave);
   uint32_t lb[NS];                                           // (a wave's slots can end inside its group of NS)
 #pragma unroll
-  for (int sl = 0; sl < NS; ++sl) lb[sl] = (uint32_t)(min(slot0 + sl, KK - 1) * kWfRows + 8 * q + rs) * 2u;
+  for (int sl = 0; sl < NS; ++sl) lb[sl] = (uint32_t)(min(slot0 + sl, KK - 1) * kWfRows + 16 * q + 4 * rs) * 2u;
   uint32_t gad[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) gad[h] = (uint32_t)(8 * q + 4 * h + rs) * 64u + byte0;
@@ -121,11 +122,11 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
     bf16* at = sx + (xp + 32 * j) * 32 + (lane & 7) * 4;
     wf_split(v, at, at + kWfXPiece);
   };
-  // g: CB = 64: load j brings 4 rows of step j, CB = 32: 8 rows of step (wave + 4 j) / 2
-  const int g_row0 = kRing ? 4 * wave + (lane >> 4) : 8 * wave + (lane >> 3);
+  // g: CB = 64: load j brings 4 rows of step j, CB = 32: 8 rows of step wave / 2 + 2 j
+  const int g_row0 = kRing ? 16 * (wave >> 1) + 4 * (lane >> 4) + (wave & 1)
+                           : 16 * (wave & 1) + 4 * ((lane >> 3) & 3) + 2 * (wave >> 1) + (lane >> 5);
   const uint32_t g_pitch = (uint32_t)cb * 4u;
   const uint32_t g_off0 = (uint32_t)g_row0 * g_pitch + (uint32_t)(lane & (kRing ? 15 : 7)) * 16u;
-  const uint32_t g_step = (kRing ? 16u : 32u) * g_pitch;
   const int g_half = kRing ? (lane & 15) >> 3 : 0;
   auto g_rsrc = [&](int64_t tile) {                          // the rows of a tile, this block's channels
     const int64_t tc = min(tile, tiles - 1);
@@ -133,14 +134,14 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
     return make_rsrc(g + tc * kWfRows * cb + blk_b * CB, (uint32_t)n * g_pitch - (uint32_t)blk_b * CB * 4u);
   };
   auto load_g = [&](int j, __amdgpu_buffer_rsrc_t r) -> f32x4 {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, g_off0 + (uint32_t)j * g_step, 0, 0));
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, g_off0 + (uint32_t)(kRing ? 32 * (j >> 1) + 2 * (j & 1) : 32 * j) * g_pitch, 0, 0));
   };
   auto g_place = [&](int buffer, int s) -> bf16* {           // of the 16 rows of step s
     return s_g + (kRing ? (s == 0 ? buffer : s + 1) : 8 * buffer + s) * kSlot;
   };
   auto put_g = [&](int j, f32x4 v, int buffer) {
     bf16* at;
-    if constexpr (kRing) at = g_place(buffer, j) + g_row0 * 32;
+    if constexpr (kRing) at = g_place(buffer, j) + (4 * wave + (lane >> 4)) * 32;
     else at = g_place(buffer, 0) + ((wave + 4 * j) >> 1) * kSlot + (8 * (wave & 1) + (lane >> 3)) * 32;
     at += g_half * 512 + (lane & 7) * 4;
     wf_split(v, at, at + HB * 512);
@@ -165,17 +166,18 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
     u32x2 a[NS][2][2];    // [slot][piece][rows 0-3 / 4-7 of the lane's 8]
     u32x2 b[HB][2][2];
   } ops[2];
-  uint32_t pv[NL];
+  u32x2 pv[NS];          // positions of the lane's two rows in an even step and the one behind it
 
-  auto pf_loc = [&](int j, const uint16_t* sl, int sn) {     // j = 2 slot + h
-    pv[j] = *(const uint16_t*)((const char*)sl + lb[j >> 1] + (uint32_t)(sn * 32 + (j & 1) * 8));
+  auto pf_loc = [&](int slot, const uint16_t* sl, int sn) {  // (sn even)
+    pv[slot] = *(const u32x2*)((const char*)sl + lb[slot] + (uint32_t)(sn * 32));
   };
   auto pf_g = [&](int j, const bf16* place, Ops& on) {       // j = 4 half + 2 piece + h
     const int h = j & 1, p = (j >> 1) & 1, bh = j >> 2;
     on.b[bh][p][h] = Mma<bf16>::read_tr((const bf16*)((const char*)place + gad[h] + (uint32_t)((p * HB + bh) * 1024)));
   };
-  auto pf_x = [&](int j, const bf16* sx, Ops& on) {          // j = 2 slot + h
-    const char* at = (const char*)sx + (pv[j] << 6) + byte0;
+  auto pf_x = [&](int j, const bf16* sx, int sn, Ops& on) {  // j = 2 slot + h
+    const uint32_t two = pv[j >> 1][sn & 1];
+    const char* at = (const char*)sx + ((j & 1 ? two >> 16 : two & 0xffffu) << 6) + byte0;
     on.a[j >> 1][0][j & 1] = Mma<bf16>::read_tr((const bf16*)at);
     on.a[j >> 1][1][j & 1] = Mma<bf16>::read_tr((const bf16*)(at + kWfXPiece * 2));
   };
@@ -194,13 +196,14 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
       mm(m, oc);
       if (m == 0) {
 #pragma unroll
-        for (int t = 0; t < NL; ++t) pf_loc(t, sl, sn);
+        for (int t = 0; t < NS; ++t)
+          if (sn % 2 == 0) pf_loc(t, sl, sn);
 #pragma unroll
         for (int t = 0; t < 4 * HB; ++t) pf_g(t, gp, on);
       }
       if (m >= XS) {
 #pragma unroll
-        for (int t = (m - XS) * XP; t < (m - XS + 1) * XP && t < NL; ++t) pf_x(t, sx, on);
+        for (int t = (m - XS) * XP; t < (m - XS + 1) * XP && t < NL; ++t) pf_x(t, sx, sn, on);
       }
       between(m);
       __builtin_amdgcn_sched_barrier(0);
@@ -231,11 +234,11 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < NL; ++t) pf_loc(t, s_loc0, 0);
+    for (int t = 0; t < NS; ++t) pf_loc(t, s_loc0, 0);
 #pragma unroll
     for (int t = 0; t < 4 * HB; ++t) pf_g(t, g_place(0, 0), ops[0]);
 #pragma unroll
-    for (int t = 0; t < NL; ++t) pf_x(t, s_x0, ops[0]);
+    for (int t = 0; t < NL; ++t) pf_x(t, s_x0, 0, ops[0]);
   }
 
   // One tile out of buffer B; the next tile -> the other buffer meanwhile: x loads in steps 0 - 3, put two steps later; g

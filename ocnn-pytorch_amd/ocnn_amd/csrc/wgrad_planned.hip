@@ -82,12 +82,12 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   constexpr int NU = HA * NFULL + NHALF;      // 32 x CB accumulator units per wave
   constexpr int NS = NFULL + NHALF;           // distinct slots per wave
   constexpr int SPG = 4 * NFULL + 2 * NHALF;  // slots per group
-  constexpr int NL = 2 * NS;                  // table look-ups per lane and step
+  constexpr int NL = 2 * NS;                  // rows of x per lane and step
   constexpr int NM = HB * NU;                 // MFMAs per step
   constexpr int XH = kWpXHalf * 2, GH = kWpGHalf * 2;   // byte offsets of the second halves
   // CA = 64: MFMAs between the position reads and their use
   constexpr int PF0 = HA == 1 ? 1 : ((NM - NL) < 4 ? (NM - NL) : 4);
-  constexpr int IP = (NL + 4 + PF0 - 1) / PF0;
+  constexpr int IP = (NS + 4 + PF0 - 1) / PF0;
   // CA = 32: positions and g with the first MFMA, the x reads XP per MFMA from MFMA XS on
   constexpr int XS = NM > 2 ? 2 : NM - 1;
   constexpr int XP = (NL + (NM - XS) - 1) / (NM - XS);
@@ -118,19 +118,21 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   const int slotH_rd = min(slotH, KK - 1);
   const uint32_t ahH = (uint32_t)(wave & 1) * (uint32_t)XH;        // this wave's half of the shared slot
 
-  // lane (i16, gq): rows 8 q + 4 h + i16 / 4 of a 16-row step, channels 16 (gq & 1) + 4 (i16 & 3) ..
+  // lane (i16, gq): places 8 q + 4 h + i16 / 4 of a 16-row step, channels 16 (gq & 1) + 4 (i16 & 3) ..
+  // Steps 2u and 2u + 1 share 32 rows of the tile: step 2u + p has row 32 u + 16 q + 4 (i16 / 4) + 2 p + h at that place, so
+  // that the positions of a lane's rows in both steps are eight consecutive bytes.  (The g rows are staged in that order.)
   const int i16 = lane & 15, gq = lane >> 4, q = lane >> 5;
   const int rs = i16 >> 2;
   const uint32_t byte0 = 32u * (gq & 1) + 8u * (i16 & 3);
-  const uint32_t lbF = (uint32_t)(slotF_rd * kWpRows + 8 * q + rs) * 2u;   // [slot][row] positions, 2 B each
-  const uint32_t lbH = (uint32_t)(slotH_rd * kWpRows + 8 * q + rs) * 2u;
+  const uint32_t lbF = (uint32_t)(slotF_rd * kWpRows + 16 * q + 4 * rs) * 2u;   // [slot][row] positions, 2 B each
+  const uint32_t lbH = (uint32_t)(slotH_rd * kWpRows + 16 * q + 4 * rs) * 2u;
   // CA = 32: a wave's slots can end inside its group of NFULL (K = 27: slots 21..27), so
   // every slot clamps on its own
   uint32_t lbS[HA == 1 ? NFULL : 1];
   if constexpr (HA == 1) {
 #pragma unroll
     for (int sl = 0; sl < NFULL; ++sl)
-      lbS[sl] = (uint32_t)(min(slotF + sl, KK - 1) * kWpRows + 8 * q + rs) * 2u;
+      lbS[sl] = (uint32_t)(min(slotF + sl, KK - 1) * kWpRows + 16 * q + 4 * rs) * 2u;
   }
   uint32_t gad[2];
 #pragma unroll
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   const int sg_half = HB == 2 ? (wave & 1) : 0, sg_g16 = HB == 2 ? (wave >> 1) : wave;
   const uint32_t st_xc = (uint32_t)st_half * 64u + (uint32_t)(lane & 3) * 16u;   // byte within a row
   const int st_pos = st_g16 * 16 + (lane >> 2);            // position / row of piece 0; piece j: + 16 GST j
-  const uint32_t sg_c = (uint32_t)sg_half * 64u + (uint32_t)(lane & 3) * 16u, sg_pos = (uint32_t)(sg_g16 * 16 + (lane >> 2));
+  const uint32_t sg_c = (uint32_t)sg_half * 64u + (uint32_t)(lane & 3) * 16u, sg_pos = (uint32_t)(32 * (sg_g16 >> 1) + 2 * (sg_g16 & 1) + 16 * (lane >> 5) + 4 * ((lane >> 2) & 3) + ((lane >> 4) & 1));
   const uint32_t st_gc = (BLK ? sg_pos * g_pitch + gb : (sg_pos << RSG)) + sg_c;
   const uint32_t st_gstep = BLK ? 16u * GSG * g_pitch : 4096u;   // 16 GSG rows further
   auto make_stage = [&](int64_t tile, int U, int32_t list_first, int32_t list_len, const int32_t* su,
@@ -218,23 +220,23 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
       for (int r = 0; r < 16; ++r) acc[u][bh][r] = 0.f;
 
   WpOps ops[2];
-  uint32_t pv[NL];       // positions (0 = empty) of the lane's two rows, per slot
+  u32x2 pv[NS];          // positions (0 = empty) of the lane's two rows in an even step and the one behind it, per slot
 
   // ---- the pieces of one step's operand fetch ----
-  auto pf_loc = [&](int j, const char* lcs, int sn) {       // j = 2 * slot + h
-    const int sl = j >> 1, h = j & 1;
+  auto pf_loc = [&](int sl, const char* lcs, int sn) {      // (sn even)
     uint32_t off;
-    if constexpr (HA == 1) off = lbS[sl] + (uint32_t)(sn * 32 + h * 8);
-    else off = (sl < NFULL ? lbF + (uint32_t)(sl * kWpRows * 2) : lbH) + (uint32_t)(sn * 32 + h * 8);
-    pv[j] = *(const uint16_t*)(lcs + off);
+    if constexpr (HA == 1) off = lbS[sl] + (uint32_t)(sn * 32);
+    else off = (sl < NFULL ? lbF + (uint32_t)(sl * kWpRows * 2) : lbH) + (uint32_t)(sn * 32);
+    pv[sl] = *(const u32x2*)(lcs + off);
   };
   auto pf_g = [&](int j, const char* gs, int sn, WpOps& on) {   // j = 2 * bh + h
     const int h = j & 1, bh = j >> 1;
     on.b[bh][h] = Mma<T>::read_tr((const T*)(gs + gad[h] + (uint32_t)(bh * GH + sn * 1024)));
   };
-  auto pf_x = [&](int j, const char* xs, WpOps& on) {            // j = 2 * slot + h
+  auto pf_x = [&](int j, const char* xs, int sn, WpOps& on) {    // j = 2 * slot + h
     const int sl = j >> 1, h = j & 1;
-    const uint32_t ad = (pv[j] << 6) + byte0;                 // position 0 is the zero row
+    const uint32_t two = pv[sl][sn & 1];
+    const uint32_t ad = ((h ? two >> 16 : two & 0xffffu) << 6) + byte0;      // position 0 is the zero row
     if (sl < NFULL) {
       on.a[HA * sl][h] = Mma<T>::read_tr((const T*)(xs + ad));
       if constexpr (HA == 2) on.a[2 * sl + 1][h] = Mma<T>::read_tr((const T*)(xs + ad + (uint32_t)XH));
@@ -263,23 +265,24 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
       if constexpr (HA == 2) {
         if (m < PF0) {
 #pragma unroll
-          for (int t = m * IP; t < (m + 1) * IP && t < NL + 4; ++t) {
-            if (t < NL) pf_loc(t, lcs, sn);
-            else pf_g(t - NL, gs, sn, on);
+          for (int t = m * IP; t < (m + 1) * IP && t < NS + 4; ++t) {
+            if (t >= NS) pf_g(t - NS, gs, sn, on);
+            else if (sn % 2 == 0) pf_loc(t, lcs, sn);
           }
         } else if (m - PF0 < NL) {
-          pf_x(m - PF0, xs, on);
+          pf_x(m - PF0, xs, sn, on);
         }
       } else {
         if (m == 0) {
 #pragma unroll
-          for (int t = 0; t < NL; ++t) pf_loc(t, lcs, sn);
+          for (int t = 0; t < NS; ++t)
+            if (sn % 2 == 0) pf_loc(t, lcs, sn);
 #pragma unroll
           for (int t = 0; t < 2 * HB; ++t) pf_g(t, gs, sn, on);
         }
         if (m >= XS) {
 #pragma unroll
-          for (int t = (m - XS) * XP; t < (m - XS + 1) * XP && t < NL; ++t) pf_x(t, xs, on);
+          for (int t = (m - XS) * XP; t < (m - XS + 1) * XP && t < NL; ++t) pf_x(t, xs, sn, on);
         }
       }
       if (t0 >= 0) {
@@ -302,11 +305,11 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   // operand fetch of a tile's first step when there is no previous step to hide it under
   auto first_fetch = [&](const char* xs, const char* gs, const char* lcs, WpOps& on) {
 #pragma unroll
-    for (int t = 0; t < NL; ++t) pf_loc(t, lcs, 0);
+    for (int t = 0; t < NS; ++t) pf_loc(t, lcs, 0);
 #pragma unroll
     for (int t = 0; t < 2 * HB; ++t) pf_g(t, gs, 0, on);
 #pragma unroll
-    for (int t = 0; t < NL; ++t) pf_x(t, xs, on);
+    for (int t = 0; t < NL; ++t) pf_x(t, xs, 0, on);
   };
 
   // ---- prologue: first list, first tile, second list ----
