@@ -27,7 +27,7 @@ namespace ocnn {
 constexpr int kWpRows = 128;   // rows per tile (the plan's tile size)
 constexpr int kWpCap = 415;    // staged distinct rows per tile: with the zero row, 26 groups of 16
 constexpr int kWpLoc = (kWpRows * 27 * 2 + 1023) / 1024 * 512;   // u16 per buffer, whole KiB
-constexpr int kWpXHalf = (kWpCap + 1) * 32;   // elements of one channel half of the x rows (+ zero row)
+constexpr int kWpCapTwo = 367;   // ... with which two workgroups of 32 x 32 blocks share a CU
 constexpr int kWpGHalf = kWpRows * 32;
 
 struct WpOps {
@@ -61,11 +61,15 @@ struct WpStage {
 // half wave 4 rows x 64 B; at a 64-byte pitch four consecutive positions cover all
 // 64 banks, and the second half is the first plus a constant.
 //
+// CAP: distinct rows of a tile at most.  A wave of the 32 x 32 layer has 212 registers, and with 367 rows two workgroups find
+// room in a CU's LDS, which hides the waits of one behind the other: us, f16, one / two a CU: 7.57 M rows 468 / 425, 4.74 M 295 / 276, 1.13 M
+// (7 % set) 80.7 / 74, 947 k 65 / 59; below 100 k rows the same.
+//
 // 32 channels of x: blocks of 32 x 64 have as many sums over all 27 slots as 64 x 64 over half of them, so one
 // workgroup stages a range's rows for all slots: 32 -> 64 on 1.06 M rows (61 % set) 119 us, in half-empty 64 x 64 blocks of two
 // slot groups 201; fp32 423 / 696.
-template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool BLK>
-__global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
+template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool BLK, int CAP>
+__global__ __launch_bounds__(256, CAP < kWpCap ? 2 : 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
     const uint16_t* __restrict__ loc, uint32_t loc_bytes, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ urows, uint32_t urows_bytes, int64_t tiles,
@@ -84,6 +88,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   constexpr int SPG = 4 * NFULL + 2 * NHALF;  // slots per group
   constexpr int NL = 2 * NS;                  // rows of x per lane and step
   constexpr int NM = HB * NU;                 // MFMAs per step
+  constexpr int kWpXHalf = (CAP + 1) * 32;    // elements of one channel half of the x rows (+ zero row)
   constexpr int XH = kWpXHalf * 2, GH = kWpGHalf * 2;   // byte offsets of the second halves
   // CA = 64: MFMAs between the position reads and their use
   constexpr int PF0 = HA == 1 ? 1 : ((NM - NL) < 4 ? (NM - NL) : 4);
@@ -102,8 +107,9 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   __shared__ __attribute__((aligned(16))) uint16_t s_loc0[kWpLoc];
   __shared__ __attribute__((aligned(16))) uint16_t s_loc1[kWpLoc];
   // lists of distinct rows, from entry 4 on; entry 3 stays -1 ("the row before the first")
-  __shared__ __attribute__((aligned(16))) int32_t s_u0[4 + 512];
-  __shared__ __attribute__((aligned(16))) int32_t s_u1[4 + 512];
+  constexpr int kList = CAP < kWpCap ? 384 : 512;
+  __shared__ __attribute__((aligned(16))) int32_t s_u0[4 + kList];
+  __shared__ __attribute__((aligned(16))) int32_t s_u1[4 + kList];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -158,9 +164,9 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
   // instruction stream for the MFMAs and everything else, so each instruction saved here
   // is MFMA issue time won.
   constexpr int NG = 2 * HB, GST = 4 / HA, GSG = 4 / HB;   // g pieces; 16-row groups between a wave's pieces of x, of g
-  constexpr int NX = ((kWpCap + 16) / 16 + GST - 1) / GST;
+  constexpr int NX = ((CAP + 16) / 16 + GST - 1) / GST;
   constexpr int tL = NG, tX = NG + 2, tU = NG + 2 + NX, kPieces = tU + 1;
-  static_assert(kPieces <= 20 && (kWpCap + 1) % 16 == 0, "five steps of four pieces stage a tile");
+  static_assert(kPieces <= 20 && (CAP + 1) % 16 == 0, "five steps of four pieces stage a tile");
   constexpr int RSH = 5 + HA, RSG = 5 + HB;                // log2 of the bytes of a CA-channel row, of a CB-channel row
   // a block of a wider layer: rows of ca (cb) channels, this block's start at xb (gb)
   const int blk_a = __builtin_amdgcn_readfirstlane(block / nbb), blk_b = block - blk_a * nbb;
@@ -205,7 +211,7 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_planned_kernel(
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rs_x, (lds_ptr_t)(st.sx + (st_half * kWpXHalf + (st_g16 + GST * (t - tX)) * 512) * 2), 16,
           BLK ? (uint32_t)id * x_pitch + (xb + st_xc) : (((uint32_t)id << RSH) | st_xc), 0, 0, 0);
-    } else if (wave < 2) {
+    } else if (wave < kList / 256 || (kList % 256 != 0 && wave * 256 + lane * 4 < kList)) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_u, (lds_ptr_t)(st.su_out + wave * 256), 16, st.list_off, 0,
                                                0, 0);
     }
@@ -405,7 +411,11 @@ static int wp_range_workgroups(int K, int ca, int cb) {
 }
 
 // ranges of tiles at most: as many as keep a workgroup on every CU (the LDS holds one)
-static int wp_splits(int range_workgroups, int n_cu) { return std::min(256, std::max(8, n_cu / range_workgroups)); }
+static int wp_splits(int range_workgroups, int n_cu) { return std::min(512, std::max(8, n_cu / range_workgroups)); }
+
+// workgroups at once: two a CU for 32 x 32 blocks of tiles with few distinct rows
+static int wp_places(int ca, int cb, int n_cu, bool few) { return ca == 32 && cb == 32 && few ? 2 * n_cu : n_cu; }
+
 
 // Tiles of a range, for the least time of
 //   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
@@ -454,7 +464,7 @@ extern "C" int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int6
 
 extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes(int K, int ca, int cb) {
   const int n_cu = wp_cu_count();
-  const int64_t splits = n_cu > 0 ? wp_splits(wp_range_workgroups(K, ca, cb), n_cu) : 256;
+  const int64_t splits = n_cu > 0 ? wp_splits(wp_range_workgroups(K, ca, cb), wp_places(ca, cb, n_cu, true)) : 512;
   return align_up(splits * K * ca * cb * 4, 256);
 }
 
@@ -473,6 +483,7 @@ struct WpArgs {
   const int32_t *uptr, *urows;
   int K, ca, cb, used;                        // used: ranges of tiles
   float* partial;
+  bool two;                                   // two workgroups a CU
 };
 
 template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS>
@@ -481,14 +492,15 @@ static void launch_wp(const WpArgs& a, hipStream_t st) {
   const uint32_t xb = (uint32_t)(a.rows_x * a.ca * 2), gb = (uint32_t)(a.rows * a.cb * 2);
   const int wgs = a.used * wp_range_workgroups(a.K, a.ca, a.cb);
   const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(a.plan_total * 4);
-#define OCNN_WP_KERNEL(BLK_)                                                                                        \
-  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, CA, CB, KK, NFULL, NHALF, GROUPS, BLK_>),                                  \
+#define OCNN_WP_KERNEL(BLK_, CAP_)                                                                                   \
+  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, CA, CB, KK, NFULL, NHALF, GROUPS, BLK_, CAP_>),                           \
                      dim3(8 * (unsigned)cdiv(wgs, 8)), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g, gb, a.loc,       \
                      lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial)
-  if (a.ca == CA && a.cb == CB)
-    OCNN_WP_KERNEL(false);
-  else if constexpr (CB == 64)
-    OCNN_WP_KERNEL(true);
+  if (a.ca == CA && a.cb == CB) {
+    if (CB == 32 && a.two) OCNN_WP_KERNEL(false, CB == 32 ? kWpCapTwo : kWpCap);
+    else OCNN_WP_KERNEL(false, kWpCap);
+  } else if constexpr (CB == 64)
+    OCNN_WP_KERNEL(true, kWpCap);
 #undef OCNN_WP_KERNEL
 }
 
@@ -532,13 +544,13 @@ template <typename T> struct WpPass : Pass {
       return;
     }
     const int K = p.K, ca = p.ca, cb = p.cb;
-    a = WpArgs{p.x, p.g, p.rows_x, p.rows, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0, (float*)p.workspace};
+    a = WpArgs{p.x, p.g, p.rows_x, p.rows, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0, (float*)p.workspace, ca == 32 && cb == 32 && p.plan_max_distinct <= kWpCapTwo};
     const int64_t tiles = cdiv(p.rows, kWpRows), sums = (int64_t)K * ca * cb * 4;       // bytes of a range's sums
     if (F32) {
       f32 = wf_split_tiles(tiles, K, ca, cb, n_cu);
       a.used = (int)cdiv(tiles, f32.run);
     } else {
-      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, n_cu);
+      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, wp_places(ca, cb, n_cu, a.two));
       a.used = (int)cdiv(tiles, a.per);
     }
     if (p.workspace_bytes < a.used * sums) {

@@ -733,6 +733,35 @@ def test_planned_weight_gradient_fp32_edges(K, ca, cb):
 
 
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('distinct', [367, 368])
+def test_planned_weight_gradient_32_two_workgroups_a_cu(dtype, distinct):
+  """32 x 32 blocks over tiles of as many distinct rows as leave room for two workgroups on a CU, and of one more; as many
+  tiles as there are places for workgroups, and one more than twice as many."""
+  from ocnn_amd.octree.octree import TilePlan
+  g = torch.Generator().manual_seed(distinct)
+  for rows in (128 * 5 + 3, 128 * 512, 128 * 1025 + 9):
+    say('planned weight gradient, two workgroups a CU', dtype, distinct, rows)
+    first = torch.arange(rows)[:, None] // 128 * 300
+    table = first + (torch.arange(rows)[:, None] % 128 * 27 + torch.arange(27)) % distinct
+    table[torch.rand(rows, 27, generator=g) < 0.2] = -1
+    whole = rows // 128 * 128
+    table[:whole:128, :14] = first[:whole:128] + torch.arange(14)                # (all of the tile's rows are named)
+    for i in range(14, distinct, 27):
+      at = table[1 + (i - 14) // 27:whole:128]
+      n = min(27, distinct - i)
+      at[:, :n] = first[1 + (i - 14) // 27:whole:128] + i + torch.arange(n)
+    table = table.to(torch.int32).contiguous()
+    rows_in = int(table.max()) + 1
+    plan = TilePlan(table.to(DEV))
+    assert plan.umax == distinct
+    x, gr = torch.randn(rows_in, 32, generator=g).to(dtype), torch.randn(rows, 32, generator=g).to(dtype)
+    want = C.weight_gemm(f64(x), f64(gr), table.numpy().astype(np.int64))
+    gw = ocnn_amd.nn.conv_wgrad(x.to(DEV), gr.to(DEV), table.to(DEV), False, plan)
+    assert rel_err(gw, want) < TOL[dtype]
+    assert torch.equal(gw, ocnn_amd.nn.conv_wgrad(x.to(DEV), gr.to(DEV), table.to(DEV), False, plan))
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('cin,cout', [(64, 128), (128, 512), (512, 128), (256, 256), (1024, 384), (192, 1024)])
 def test_dense_rows_kernel(dtype, cin, cout):
   """out = in W + bias on the kernel for one-slot identity tables (every row-block and
