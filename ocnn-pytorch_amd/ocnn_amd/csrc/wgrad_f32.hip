@@ -374,13 +374,19 @@ WfSplit wf_split_tiles(int64_t tiles, int K, int ca, int cb, int n_cu) {
   double least = 1e30;
   for (int groups = 1; groups <= (K == 27 ? 2 : 1); ++groups) {
     const int wgs = wf_range_workgroups(ca, cb, groups);
-    for (int s = 1, most = std::min(256, std::max(8, n_cu / wgs)); s <= most; ++s) {
+    const int64_t most = std::min(256, std::max(8, n_cu / wgs)), sets_at = wf_run(cb);
+    const double tile_us = wf_tile_us(K, cb, groups);
+    int64_t s = 1;
+    for (bool more = true; more && s <= most;) {             // (the fewest ranges of as many tiles; then of fewer tiles)
       int64_t per = std::max<int64_t>(1, cdiv(tiles, s));
+      more = per > 1;
+      if (more) s = cdiv(tiles, per - 1);
       // (several sets a range: of an even number of tiles each, the buffers take turns)
-      const int64_t sets = cdiv(per, wf_run(cb)), run = sets > 1 ? align_up(cdiv(per, sets), 2) : per;
-      per = run * cdiv(per, run);
-      const double us = (double)cdiv(cdiv(cdiv(tiles, per) * wgs, 8), cu_xcd) * (per * wf_tile_us(K, cb, groups) + kWfFixedUs) +
-                        cdiv(tiles, run) * sums;
+      const int64_t sets = cdiv(per, sets_at), run = sets > 1 ? align_up(cdiv(per, sets), 2) : per;
+      if (sets > 1) per = run * cdiv(per, run);
+      const int64_t used = cdiv(tiles, per);
+      const double us = (double)cdiv(cdiv(used * wgs, 8), cu_xcd) * ((double)per * tile_us + kWfFixedUs) +
+                        (double)(sets > 1 ? cdiv(tiles, run) : used) * sums;
       if (us < least) least = us, best = WfSplit{per, run, groups};
     }
   }

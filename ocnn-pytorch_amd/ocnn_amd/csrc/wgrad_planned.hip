@@ -428,10 +428,12 @@ static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, in
   const int cu_xcd = std::max(1, n_cu / 8);
   int64_t best = std::max<int64_t>(tiles, 1);
   double least = 1e30;
-  for (int s = 1, most = wp_splits(wgs, n_cu); s <= most; ++s) {
-    const int64_t per = std::max<int64_t>(1, cdiv(tiles, s));
-    const int64_t used = cdiv(tiles, per);
-    if (used < s) continue;                                  // (the same ranges as fewer)
+  int64_t s = 1;
+  const int64_t most = wp_splits(wgs, n_cu);
+  for (bool more = true; more && s <= most;) {               // (the fewest ranges of as many tiles; then of fewer tiles)
+    const int64_t per = std::max<int64_t>(1, cdiv(tiles, s)), used = s;
+    more = per > 1;
+    if (more) s = cdiv(tiles, per - 1);
     const double cost = (double)cdiv(cdiv(used * wgs, 8), cu_xcd) * ((double)per * kWpTileUs + kWpFixedUs) +
                         (double)used * (double)sums_bytes * kWpSumUs;
     if (cost < least) least = cost, best = per;
