@@ -137,9 +137,8 @@ __device__ inline uint32_t lanes_below(unsigned long long mask) {
 
 // starts of nodes, by layer, among the points of each workgroup's span: sums[span][N]
 template <typename K, int N, int SPAN>
-__global__ __launch_bounds__(kBuildThreads) void build_count_kernel(const K* __restrict__ sorted, int64_t n,
-                                                                    int key_bits, int levels,
-                                                                    uint32_t* __restrict__ sums) {
+static __device__ __forceinline__ void build_count(const K* __restrict__ sorted, int64_t n, int key_bits, int levels,
+                                                   uint32_t* __restrict__ sums) {
   __shared__ uint32_t s_cnt[kBuildThreads / 64][N];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = (int64_t)blockIdx.x * SPAN + wave * (SPAN / 4);
@@ -163,6 +162,13 @@ __global__ __launch_bounds__(kBuildThreads) void build_count_kernel(const K* __r
     for (int w = 0; w < kBuildThreads / 64; ++w) c += s_cnt[w][threadIdx.x];
     sums[(int64_t)blockIdx.x * N + threadIdx.x] = c;
   }
+}
+
+template <typename K, int N, int SPAN>
+__global__ __launch_bounds__(kBuildThreads) void build_count_kernel(const K* __restrict__ sorted, int64_t n,
+                                                                    int key_bits, int levels,
+                                                                    uint32_t* __restrict__ sums) {
+  build_count<K, N, SPAN>(sorted, n, key_bits, levels, sums);
 }
 
 // offs[span][l] = starts at layer l before the span; sizes[l] = their total.  One workgroup: thread
@@ -207,8 +213,8 @@ struct BuildSignal {
 
 // Full layers, and -1 in the children of every other layer.  Four nodes a thread (the layers below the
 // full ones are whole groups of eight, and so are the full ones from layer 1 on).
-__global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+static __device__ __forceinline__ void build_init(const BuildTree& t, int depth, int full_depth, int64_t thread) {
+  const int64_t i = thread * 4;
   if (i >= t.begin[depth + 1] - t.begin[1] + 4 * ((t.begin[1] + 3) / 4)) return;
   const int64_t root = 4 * ((t.begin[1] + 3) / 4);            // layer 0 (a node per octree) padded to groups of four
   if (i < root) {
@@ -229,6 +235,19 @@ __global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
     if (d < full_depth) c = make_int4((int)j, (int)j + 1, (int)j + 2, (int)j + 3);
   }
   *(int4*)(t.children[d] + j) = c;
+}
+
+__global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
+  build_init(t, depth, full_depth, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// Both in one launch: workgroups behind those of the spans.
+template <typename K, int N, int SPAN>
+__global__ __launch_bounds__(kBuildThreads) void build_count_init_kernel(const K* __restrict__ sorted, int64_t n, int key_bits,
+                                                                         int levels, uint32_t* __restrict__ sums, int spans,
+                                                                         BuildTree t, int depth, int full_depth) {
+  if ((int)blockIdx.x < spans) build_count<K, N, SPAN>(sorted, n, key_bits, levels, sums);
+  else build_init(t, depth, full_depth, (int64_t)(blockIdx.x - spans) * kBuildThreads + threadIdx.x);
 }
 
 struct OpenLeaf {                // a leaf whose points a span does not hold all: its signals' sums so far
@@ -948,37 +967,25 @@ extern "C" int64_t ocnnx_tree_workspace_bytes(int64_t n, int depth, int full_dep
                                                    : align_up(n * 8, 256) + align_up(n * 12, 256));
 }
 
-extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
-                               int batch_is_float, int depth, int full_depth, int batch_bits, const float* normals, float* rows,
-                               void* workspace, int64_t workspace_bytes, int32_t* perm, int64_t* sizes, void* stream) {
-  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
-  OCNN_REQUIRE_PTRS("tree_scan", pts, h_bbmin, rows, workspace, perm, sizes);
-  if (workspace_bytes < ocnnx_tree_workspace_bytes(n, depth, full_depth, batch_bits)) {
-    set_error("tree_scan: workspace too small");
-    return OCNN_ERR_WORKSPACE;
-  }
-  hipStream_t st = (hipStream_t)stream;
-  const int key_bits = 3 * depth, levels = depth - full_depth;
-  const int64_t base = ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits);
-  char* more = (char*)workspace + base;
-  if (!tree_own_sort(n, depth, batch_bits)) {
-    int64_t* key = (int64_t*)more;
-    float* norm = (float*)(more + align_up(n * 8, 256));
-    if (int rc = ocnn_points2key(pts, n, h_bbmin, factor, batch, batch_is_float, depth, norm, key, stream)) return rc;
-    hipLaunchKernelGGL(tree_rows_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, norm, normals, n, (float4*)rows);
-    return ocnn_octree_build_scan(key, n, depth, full_depth, batch_bits, workspace, base, perm, sizes, stream);
-  }
+// where the sorted keys, the spans' counts and their offsets lie in the workspace of this file's own sort
+static int tree_layout(int64_t n, int levels, BuildLayout* L) {
+  if ((levels + 1 > 8 ? build_layout_t<uint32_t, 16>(n, L) : build_layout_t<uint32_t, 8>(n, L)) == OCNN_OK) return OCNN_OK;
+  set_error("tree_scan: rocprim size query failed");
+  return OCNN_ERR_HIP;
+}
+
+static int tree_sort(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch, int batch_is_float,
+                     int depth, int levels, int batch_bits, const float* normals, float* rows, char* workspace, int64_t base,
+                     int32_t* perm, hipStream_t st) {
+  char* more = workspace + base;
   const SortPlan s = sort_plan(n, tree_key_bits(depth, batch_bits));
   uint32_t* keys = (uint32_t*)(more + s.key);
   uint2* pairs[2] = {(uint2*)(more + s.pair[0]), (uint2*)(more + s.pair[1])};
   uint32_t* hist = (uint32_t*)(more + s.hist);
   uint32_t* totals = s.spans > kSortInlineSpans ? (uint32_t*)(more + s.totals) : nullptr;
   BuildLayout L;
-  if (build_layout_t<uint32_t, 8>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
-  if (levels + 1 > 8 && build_layout_t<uint32_t, 16>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
-  uint32_t* csorted = (uint32_t*)((char*)workspace + L.csorted);
-  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
-  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
+  if (int rc = tree_layout(n, levels, &L)) return rc;
+  uint32_t* csorted = (uint32_t*)(workspace + L.csorted);
   const dim3 grid((unsigned)s.spans), block(kSortThreads);
   hipLaunchKernelGGL(tree_keys_kernel, grid, block, 0, st, pts, n, h_bbmin[0], h_bbmin[1], h_bbmin[2], factor, batch,
                      batch_is_float, depth, normals, (float4*)rows, keys, s.bits, hist);
@@ -993,6 +1000,42 @@ extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin
     hipLaunchKernelGGL(pass, grid, dim3(kPassThreads), 0, st, keys, pairs[(p + 1) & 1], n, p * s.bits, s.bits, s.spans, hist, totals,
                        pairs[p & 1], csorted, (uint32_t*)perm);
   }
+  return check_launch("tree_sort");
+}
+
+static int tree_args_ok(int64_t n, int depth, int full_depth, int batch_bits, int64_t workspace_bytes) {
+  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
+  if (workspace_bytes < ocnnx_tree_workspace_bytes(n, depth, full_depth, batch_bits)) {
+    set_error("tree_scan: workspace too small");
+    return OCNN_ERR_WORKSPACE;
+  }
+  return OCNN_OK;
+}
+
+extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
+                               int batch_is_float, int depth, int full_depth, int batch_bits, const float* normals, float* rows,
+                               void* workspace, int64_t workspace_bytes, int32_t* perm, int64_t* sizes, void* stream) {
+  OCNN_REQUIRE_PTRS("tree_scan", pts, h_bbmin, rows, workspace, perm, sizes);
+  if (int rc = tree_args_ok(n, depth, full_depth, batch_bits, workspace_bytes)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  const int key_bits = 3 * depth, levels = depth - full_depth;
+  const int64_t base = ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits);
+  char* more = (char*)workspace + base;
+  if (!tree_own_sort(n, depth, batch_bits)) {
+    int64_t* key = (int64_t*)more;
+    float* norm = (float*)(more + align_up(n * 8, 256));
+    if (int rc = ocnn_points2key(pts, n, h_bbmin, factor, batch, batch_is_float, depth, norm, key, stream)) return rc;
+    hipLaunchKernelGGL(tree_rows_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, norm, normals, n, (float4*)rows);
+    return ocnn_octree_build_scan(key, n, depth, full_depth, batch_bits, workspace, base, perm, sizes, stream);
+  }
+  if (int rc = tree_sort(pts, n, h_bbmin, factor, batch, batch_is_float, depth, levels, batch_bits, normals, rows, (char*)workspace,
+                         base, perm, st))
+    return rc;
+  BuildLayout L;
+  if (int rc = tree_layout(n, levels, &L)) return rc;
+  const uint32_t* csorted = (const uint32_t*)((char*)workspace + L.csorted);
+  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
+  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
 #define OCNN_TREE_COUNT(N)                                                                          \
   launch_build_count<uint32_t, N>(csorted, n, L.spans, key_bits, levels, sums, st);                  \
   hipLaunchKernelGGL(build_offsets_kernel<N>, dim3(1), dim3(1024), 0, st, sums, L.spans, levels, offs, sizes)
@@ -1000,4 +1043,66 @@ extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin
   else { OCNN_TREE_COUNT(16); }
 #undef OCNN_TREE_COUNT
   return check_launch("tree_scan");
+}
+
+// ---- small clouds: the whole build without a wait --------------------------------------------------
+// The sizes of the layers are known when the points are numbered, and what they are written to is allocated then: 20 us between
+// the kernels of a build whose kernels take 45.  A layer has 8 n nodes at most, so a small cloud's arrays can be made for
+// that many while the points are sorted, and shortened when the sizes have come, beside the scatter.  (65536 points: 6 MB a layer, of
+// which a sphere at depth 8 uses half, at depth 9 two thirds.  Every layer: points of batch ids that there are no
+// octrees for have nodes of their own until they are refused.)
+constexpr int64_t kTreeAheadPoints = 1 << 16;
+
+extern "C" int ocnnx_tree_ahead(int64_t n, int depth, int full_depth, int batch_bits) {
+  return n > 0 && n <= kTreeAheadPoints && full_depth < depth && tree_own_sort(n, depth, batch_bits);
+}
+
+extern "C" int ocnnx_tree_sort(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
+                               int batch_is_float, int depth, int full_depth, int batch_bits, const float* normals, float* rows,
+                               void* workspace, int64_t workspace_bytes, int32_t* perm, void* stream) {
+  OCNN_REQUIRE(ocnnx_tree_ahead(n, depth, full_depth, batch_bits), "tree_sort: shape not supported");
+  OCNN_REQUIRE_PTRS("tree_sort", pts, h_bbmin, rows, workspace, perm);
+  if (int rc = tree_args_ok(n, depth, full_depth, batch_bits, workspace_bytes)) return rc;
+  return tree_sort(pts, n, h_bbmin, factor, batch, batch_is_float, depth, depth - full_depth, batch_bits, normals, rows,
+                   (char*)workspace, ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits), perm, (hipStream_t)stream);
+}
+
+extern "C" int ocnnx_tree_number(void* workspace, int64_t n, int depth, int full_depth, int batch_size, int batch_bits,
+                                 const int32_t* perm, int64_t* const* h_keys, int32_t* const* h_children, int32_t* const* h_index,
+                                 int64_t* inverse, int32_t* seg_start, const float* rows, float* out_pts, float* out_normals,
+                                 int64_t* sizes, void* stream) {
+  OCNN_REQUIRE(ocnnx_tree_ahead(n, depth, full_depth, batch_bits), "tree_number: shape not supported");
+  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
+  OCNN_REQUIRE_PTRS("tree_number", workspace, perm, h_keys, h_children, h_index, inverse, seg_start, rows, out_pts, sizes);
+  OCNN_REQUIRE(batch_size >= 1 && batch_size <= (1 << batch_bits) && ((int64_t)batch_size << (3 * full_depth)) < (1ll << 31),
+               "tree_number: batch_size=%d does not fit batch_bits=%d / full_depth=%d", batch_size, batch_bits, full_depth);
+  BuildTree t;
+  t.begin[0] = 0;
+  for (int d = 0; d <= depth; ++d) {
+    OCNN_REQUIRE(h_keys[d] && h_children[d] && (d < full_depth || h_index[d]), "tree_number: depth %d: a missing array", d);
+    t.keys[d] = h_keys[d];
+    t.children[d] = h_children[d];
+    t.index[d] = h_index[d];
+    t.begin[d + 1] = t.begin[d] + (d <= full_depth ? ((int64_t)batch_size << (3 * d)) : 8 * n);
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int key_bits = 3 * depth, levels = depth - full_depth;
+  BuildLayout L;
+  if (int rc = tree_layout(n, levels, &L)) return rc;
+  const uint32_t* csorted = (const uint32_t*)((char*)workspace + L.csorted);
+  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
+  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
+  const int64_t init = cdiv(t.begin[depth + 1] + 4, 4 * kBuildThreads);
+  const BuildSignal sig{(const float4*)rows, out_pts, out_normals};
+#define OCNN_TREE_NUMBER(N)                                                                                                \
+  hipLaunchKernelGGL((build_count_init_kernel<uint32_t, N, kBuildSmallSpan>), dim3((unsigned)(L.spans + init)),              \
+                     dim3(kBuildThreads), 0, st, csorted, n, key_bits, levels, sums, (int)L.spans, t, depth, full_depth);    \
+  hipLaunchKernelGGL(build_offsets_kernel<N>, dim3(1), dim3(1024), 0, st, sums, L.spans, levels, offs, sizes);               \
+  hipLaunchKernelGGL((build_scatter_kernel<uint32_t, N, kBuildSmallSpan>), dim3((unsigned)L.spans), dim3(kBuildThreads), 0,  \
+                     st, csorted, offs, perm, n, key_bits, depth, full_depth, t, sig, inverse, seg_start)
+  static_assert(kTreeAheadPoints <= kBuildSmallPoints, "small spans");
+  if (levels + 1 <= 8) { OCNN_TREE_NUMBER(8); }
+  else { OCNN_TREE_NUMBER(16); }
+#undef OCNN_TREE_NUMBER
+  return check_launch("tree_number");
 }

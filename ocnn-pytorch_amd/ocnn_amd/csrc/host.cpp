@@ -776,9 +776,15 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   Tensor sizes = at::empty({levels + 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
   std::fill_n((int64_t*)sizes.data_ptr(), levels + 1, -1);
   const auto st = c10::hip::getCurrentHIPStream();
-  check(ocnnx_tree_scan((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
-                        full_depth, batch_bits, (const float*)ptr(normals), (float*)rows.data_ptr(), ws.data_ptr(), ws_bytes,
-                        (int32_t*)t.perm.data_ptr(), (int64_t*)sizes.data_ptr(), st.stream()));
+  const bool ahead = ocnnx_tree_ahead(n, depth, full_depth, batch_bits);
+  if (ahead)
+    check(ocnnx_tree_sort((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
+                          full_depth, batch_bits, (const float*)ptr(normals), (float*)rows.data_ptr(), ws.data_ptr(), ws_bytes,
+                          (int32_t*)t.perm.data_ptr(), st.stream()));
+  else
+    check(ocnnx_tree_scan((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
+                          full_depth, batch_bits, (const float*)ptr(normals), (float*)rows.data_ptr(), ws.data_ptr(), ws_bytes,
+                          (int32_t*)t.perm.data_ptr(), (int64_t*)sizes.data_ptr(), st.stream()));
   // what does not wait for the sizes is allocated while the sort runs
   for (int d = 0; d <= full_depth; ++d) {
     t.nnum.push_back((int64_t)batch_size << (3 * d));
@@ -787,16 +793,20 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   }
   t.idx = at::empty({n}, i64);
   t.seg_start = at::empty({n + 1}, i32);
-  wait_for(sizes, st);
-  const std::vector<int64_t> size((int64_t*)sizes.data_ptr(), (int64_t*)sizes.data_ptr() + levels + 1);
-  for (int d = full_depth + 1; d <= depth; ++d) {
-    t.nnum.push_back(8 * size[depth - d + 1]);
-    t.keys.push_back(at::empty({t.nnum[d]}, i64));
-    t.children.push_back(at::empty({t.nnum[d]}, i32));
-  }
+  std::vector<int64_t> size(levels + 1, n);                  // (of a small cloud: room for as many)
+  const auto take_sizes = [&]() {
+    wait_for(sizes, st);
+    size.assign((int64_t*)sizes.data_ptr(), (int64_t*)sizes.data_ptr() + levels + 1);
+  };
+  if (!ahead) take_sizes();
   std::vector<int64_t*> keys;
   std::vector<int32_t*> children, index;
   for (int d = 0; d <= depth; ++d) {
+    if (d > full_depth) {
+      t.nnum.push_back(8 * size[depth - d + 1]);
+      t.keys.push_back(at::empty({t.nnum[d]}, i64));
+      t.children.push_back(at::empty({t.nnum[d]}, i32));
+    }
     t.nnum_nempty.push_back(d < full_depth ? t.nnum[d] : size[depth - d]);
     t.index.push_back(d < full_depth ? OptTensor() : at::empty({t.nnum_nempty[d]}, i32));
     keys.push_back((int64_t*)t.keys[d].data_ptr());
@@ -805,10 +815,33 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   }
   t.points = at::empty({size[0], 3}, pts.options());
   if (normals.has_value()) t.normals = at::empty({size[0], 3}, pts.options());
-  check(ocnnx_tree_fill(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, size.data(),
-                        (const int32_t*)t.perm.data_ptr(), keys.data(), children.data(), index.data(),
-                        (int64_t*)t.idx.data_ptr(), (int32_t*)t.seg_start.data_ptr(), (const float*)rows.data_ptr(),
-                        (float*)t.points.data_ptr(), t.normals.has_value() ? (float*)t.normals->data_ptr() : nullptr, st.stream()));
+  float *out_pts = (float*)t.points.data_ptr(), *out_normals = t.normals.has_value() ? (float*)t.normals->data_ptr() : nullptr;
+  if (ahead) {
+    check(ocnnx_tree_number(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, (const int32_t*)t.perm.data_ptr(),
+                            keys.data(), children.data(), index.data(), (int64_t*)t.idx.data_ptr(),
+                            (int32_t*)t.seg_start.data_ptr(), (const float*)rows.data_ptr(), out_pts, out_normals,
+                            (int64_t*)sizes.data_ptr(), st.stream()));
+    take_sizes();
+    TORCH_CHECK(size[levels] <= (int64_t)batch_size << (3 * full_depth), "octree_build_fill: ", size[levels],
+                " nodes at the deepest full layer of ", batch_size, " octrees");
+    const auto cut = [](const Tensor& made, at::IntArrayRef to) { made.unsafeGetTensorImpl()->set_sizes_contiguous(to); };
+    for (int d = full_depth; d <= depth; ++d) {
+      if (d > full_depth) {
+        t.nnum[d] = 8 * size[depth - d + 1];
+        cut(t.keys[d], {t.nnum[d]});
+        cut(t.children[d], {t.nnum[d]});
+      }
+      t.nnum_nempty[d] = size[depth - d];
+      cut(*t.index[d], {size[depth - d]});
+    }
+    cut(t.points, {size[0], 3});
+    if (t.normals.has_value()) cut(*t.normals, {size[0], 3});
+  } else {
+    check(ocnnx_tree_fill(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, size.data(),
+                          (const int32_t*)t.perm.data_ptr(), keys.data(), children.data(), index.data(),
+                          (int64_t*)t.idx.data_ptr(), (int32_t*)t.seg_start.data_ptr(), (const float*)rows.data_ptr(), out_pts,
+                          out_normals, st.stream()));
+  }
   for (int d = 0; d <= depth; ++d)
     for (const Tensor* made : {&t.keys[d], &t.children[d]}) t.versions.push_back(made->is_inference() ? 0 : made->_version());
   return t;

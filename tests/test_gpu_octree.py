@@ -452,6 +452,54 @@ def test_deep_octrees_vs_oracle(depth, full, batch, n):
       assert np.array_equal(np_(o.nempty_index(d)), np.nonzero(w.children[d] >= 0)[0]), d
 
 
+@pytest.mark.parametrize('n', [1, 255, 257, 65536, 65537])
+@pytest.mark.parametrize('depth,full', [(5, 2), (10, 1)])
+def test_builds_with_and_without_a_wait_for_the_sizes(n, depth, full):
+  """Clouds up to and beyond the size whose layers get their places before their sizes are known (one in which every point is
+  a leaf of its own, as far as there are cells, needs them all), with more layers than eight counters hold: bit exact against the oracle;
+  what the octree holds is contiguous, of the layers' sizes, and can be written to, copied and saved."""
+  import io
+  rng = np.random.default_rng(n + depth)
+  pts = rng.uniform(-1, 0.999999, (n, 3)).astype(np.float32)
+  nrm = rng.standard_normal((n, 3)).astype(np.float32)
+  say('build, sizes ahead or waited for', n, depth, full)
+  o = Octree(depth, full)
+  idx = o.build_octree(Points(torch.from_numpy(pts).to(DEV), torch.from_numpy(nrm).to(DEV)))
+  w, widx = R.build_octree(pts, nrm, None, None, depth, full, 1)
+  assert np.array_equal(o.nnum.numpy(), w.nnum) and np.array_equal(o.nnum_nempty.numpy(), w.nnum_nempty)
+  assert np.array_equal(np_(idx), widx)
+  o.construct_all_neigh()
+  for d in range(depth + 1):
+    for got, want in ((o.keys[d], w.keys[d]), (o.children[d], w.children[d])):
+      assert got.shape == want.shape and got.is_contiguous() and np.array_equal(np_(got), want), d
+    if d >= 1:
+      assert np.array_equal(np_(o.nempty_index(d)), np.nonzero(w.children[d] >= 0)[0]), d
+  assert np.array_equal(np_(o.points[depth]), w.points[depth])
+  assert np.allclose(np_(o.normals[depth]), w.normals[depth], atol=1e-6)
+  file = io.BytesIO()
+  torch.save([o.keys[depth], o.children[depth], o.points[depth]], file)
+  file.seek(0)
+  for got, want in zip(torch.load(file, weights_only=True), (w.keys[depth], w.children[depth], w.points[depth])):
+    assert np.array_equal(np_(got), want)
+  o.children[depth][-1] = -1
+  assert o.children[depth].clone().shape == w.children[depth].shape
+
+
+def test_batch_ids_without_octrees_are_refused():
+  """More nodes at the deepest full layer than the octrees have, of batch ids beyond them: an error, and nothing written
+  outside of the layers (tensors made before and after are as they were)."""
+  before = torch.full((1 << 16,), 7, dtype=torch.int32, device=DEV)
+  grid = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing='ij'), -1).reshape(-1, 3) / 2.0 - 0.9
+  pts = np.tile(grid, (4, 1)).astype(np.float32)
+  bid = torch.arange(4, device=DEV).repeat_interleave(64).view(-1, 1)
+  say('batch ids without octrees')
+  pc = Points(torch.from_numpy(pts).to(DEV), torch.ones(256, 3, device=DEV), batch_id=bid % 2, batch_size=2)
+  pc.batch_id = bid                                    # (the points themselves check what they are made with)
+  with pytest.raises(RuntimeError, match='at the deepest full layer'):
+    Octree(4, 1, batch_size=2).build_octree(pc)
+  assert bool((before == 7).all())
+
+
 def test_octree_without_a_full_layer_below_the_root():
   """full_depth = 0: the build equals the oracle's; the neighbour tables cannot be made (layer 1
   would need the table of layer 0, which does not exist - the reference's construct_neigh(1) fails
