@@ -366,6 +366,8 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
         const int d = depth - l;
         const int64_t kl = m >> (3 * l);
         const int64_t p = (int64_t)s[l + 1 < N ? l + 1 : l] - 1;
+        if constexpr (SPAN == kBuildSmallSpan)                // (points of batch ids beyond batch_size may have no place)
+          if ((p << 3) >= t.begin[d + 1] - t.begin[d]) continue;
         t.children[d][(p << 3) | (kl & 7)] = (int32_t)s[l] - 1;
         if (t.index[d]) t.index[d][s[l] - 1] = (int32_t)((p << 3) | (kl & 7));
         if (l + 1 <= lv[it]) {
@@ -380,7 +382,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
       const int64_t node = (b << (3 * full_depth)) | (m >> (3 * levels));
       if (node < t.begin[full_depth + 1] - t.begin[full_depth]) {    // a batch id beyond batch_size has no node
         t.children[full_depth][node] = (int32_t)top - 1;
-        if (t.index[full_depth]) t.index[full_depth][top - 1] = (int32_t)node;
+        if (t.index[full_depth] && top <= t.begin[full_depth + 1] - t.begin[full_depth]) t.index[full_depth][top - 1] = (int32_t)node;
       }
     }
     if (!sig.rows) continue;
@@ -1047,11 +1049,15 @@ extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin
 
 // ---- small clouds: the whole build without a wait --------------------------------------------------
 // The sizes of the layers are known when the points are numbered, and what they are written to is allocated then: 20 us between
-// the kernels of a build whose kernels take 45.  A layer has 8 n nodes at most, so a small cloud's arrays can be made for
-// that many while the points are sorted, and shortened when the sizes have come, beside the scatter.  (65536 points: 6 MB a layer, of
-// which a sphere at depth 8 uses half, at depth 9 two thirds.  Every layer: points of batch ids that there are no
-// octrees for have nodes of their own until they are refused.)
-constexpr int64_t kTreeAheadPoints = 1 << 16;
+// the kernels of a build whose kernels take 45.  Build and tables, us, waited in the middle / now: 20 k points depth 6 89 / 77,
+// 60 k depth 7 105 / 94, 100 k depth 8 123 / 115, 130 k depth 9 150 / 140, 250 k depth 7 118 / 108, depth 9 157 / 154.  A layer has 8 n nodes at most, and no more than there are cells, so a small
+// cloud's arrays can be made for that many while the points are sorted, and cut when the sizes have come, beside the scatter.  What
+// is not used of them stays theirs: 25 MB a layer from depth 7 on for 262 k points, whose neighbour tables take 100 - 200 MB.
+constexpr int64_t kTreeAheadPoints = 1 << 18;
+
+extern "C" int64_t ocnnx_tree_places(int64_t n, int batch_size, int depth) {
+  return std::min<int64_t>(8 * n, (int64_t)batch_size << (3 * depth));
+}
 
 extern "C" int ocnnx_tree_ahead(int64_t n, int depth, int full_depth, int batch_bits) {
   return n > 0 && n <= kTreeAheadPoints && full_depth < depth && tree_own_sort(n, depth, batch_bits);
@@ -1083,7 +1089,7 @@ extern "C" int ocnnx_tree_number(void* workspace, int64_t n, int depth, int full
     t.keys[d] = h_keys[d];
     t.children[d] = h_children[d];
     t.index[d] = h_index[d];
-    t.begin[d + 1] = t.begin[d] + (d <= full_depth ? ((int64_t)batch_size << (3 * d)) : 8 * n);
+    t.begin[d + 1] = t.begin[d] + (d <= full_depth ? (int64_t)batch_size << (3 * d) : ocnnx_tree_places(n, batch_size, d));
   }
   hipStream_t st = (hipStream_t)stream;
   const int key_bits = 3 * depth, levels = depth - full_depth;

@@ -803,7 +803,7 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   std::vector<int32_t*> children, index;
   for (int d = 0; d <= depth; ++d) {
     if (d > full_depth) {
-      t.nnum.push_back(8 * size[depth - d + 1]);
+      t.nnum.push_back(ahead ? ocnnx_tree_places(n, batch_size, d) : 8 * size[depth - d + 1]);
       t.keys.push_back(at::empty({t.nnum[d]}, i64));
       t.children.push_back(at::empty({t.nnum[d]}, i32));
     }

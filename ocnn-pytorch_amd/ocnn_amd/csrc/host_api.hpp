@@ -158,8 +158,9 @@ int ocnnx_tree_fill(const void* workspace, int64_t n, int depth, int full_depth,
                     int32_t* const* h_index, int64_t* inverse, int32_t* seg_start, const float* rows, float* out_pts,
                     float* out_normals, void* stream);
 // The same in two halves for small clouds (ocnnx_tree_ahead), without the sizes in between: sorted points, then everything else
-// into arrays of 8 n nodes a layer below the full ones and n entries an index; sizes comes back as from the scan.
+// into arrays of ocnnx_tree_places nodes a layer below the full ones and n entries an index; sizes comes back as from the scan.
 int ocnnx_tree_ahead(int64_t n, int depth, int full_depth, int batch_bits);
+int64_t ocnnx_tree_places(int64_t n, int batch_size, int depth);
 int ocnnx_tree_sort(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch, int batch_is_float,
                     int depth, int full_depth, int batch_bits, const float* normals, float* rows, void* workspace,
                     int64_t workspace_bytes, int32_t* perm, void* stream);

@@ -452,11 +452,11 @@ def test_deep_octrees_vs_oracle(depth, full, batch, n):
       assert np.array_equal(np_(o.nempty_index(d)), np.nonzero(w.children[d] >= 0)[0]), d
 
 
-@pytest.mark.parametrize('n', [1, 255, 257, 65536, 65537])
+@pytest.mark.parametrize('n', [1, 255, 257, 40000, 262144, 262145])
 @pytest.mark.parametrize('depth,full', [(5, 2), (10, 1)])
 def test_builds_with_and_without_a_wait_for_the_sizes(n, depth, full):
   """Clouds up to and beyond the size whose layers get their places before their sizes are known (one in which every point is
-  a leaf of its own, as far as there are cells, needs them all), with more layers than eight counters hold: bit exact against the oracle;
+  a leaf of its own, as far as there are cells, needs many), with more layers than eight counters hold: bit exact against the oracle;
   what the octree holds is contiguous, of the layers' sizes, and can be written to, copied and saved."""
   import io
   rng = np.random.default_rng(n + depth)
