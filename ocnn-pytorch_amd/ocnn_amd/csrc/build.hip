@@ -280,12 +280,17 @@ __device__ __forceinline__ void leaf_signals(const BuildSignal& sig, int64_t lea
 // 360 / 285 / 187; of a sphere at depth 5 460 / 428 / 207, depth 6 217 / 220 / 174, 3 M 508 / 600 / 372; 200 k points of one
 // cell 30300 / 51400 / 4580, one chain of additions.  (Where the next span starts a leaf, as most do, nothing follows the walk:
 // with the further points asked for in every span a build of 1 M points at depth 9 took 6 us more.)
-template <typename K, int N, int SPAN>
+//
+// AHEAD (small clouds): offs holds the spans' counts, which every workgroup adds up itself; the first one also leaves their totals
+// in sizes (host memory).  A launch of one workgroup did that in between: build and tables of 20 k points
+// at depth 6 82 / 81 us, waited for by themselves 112 / 85 (seven launches: host.cpp, wait_for), 60 k at depth 7 122 / 108.
+template <typename K, int N, int SPAN, bool AHEAD>
 __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     const K* __restrict__ sorted, const uint32_t* __restrict__ offs, const int32_t* __restrict__ perm, int64_t n,
     int key_bits, int depth, int full_depth, BuildTree t, BuildSignal sig, int64_t* __restrict__ inverse,
-    int32_t* __restrict__ seg_start) {
+    int32_t* __restrict__ seg_start, int64_t* __restrict__ sizes) {
   __shared__ uint32_t s_cnt[kBuildThreads / 64][N];
+  __shared__ uint32_t s_before[AHEAD ? kBuildThreads / N : 1][N];
   __shared__ __attribute__((aligned(16))) float s_sig[6][SPAN];
   __shared__ uint8_t s_new[SPAN];                            // the point starts a leaf (or is none)
   __shared__ OpenLeaf s_open;
@@ -296,6 +301,15 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
   const int64_t behind = ((int64_t)blockIdx.x + 1) * SPAN;
   const bool goes_on = sig.rows && behind < n && sorted[behind] == sorted[behind - 1];   // a leaf does, in the span behind
   if (threadIdx.x == 0) s_open.leaf = -1;
+  if constexpr (AHEAD) {
+    constexpr int kChunks = kBuildThreads / N;
+    const int spans = (int)gridDim.x, l = threadIdx.x % N, c = threadIdx.x / N;
+    const int until = blockIdx.x == 0 ? spans : (int)blockIdx.x;       // (the first span: all of them, for the totals)
+    uint32_t sum = 0u;
+#pragma unroll 8
+    for (int b = c; b < until; b += kChunks) sum += offs[(int64_t)b * N + l];
+    s_before[c][l] = sum;
+  }
   int lv[kIt], at[kIt];
   uint32_t run[N];
 #pragma unroll
@@ -333,9 +347,23 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     s_sig[3][j] = v[it][0].w, s_sig[4][j] = v[it][1].x, s_sig[5][j] = v[it][1].y;
   }
   __syncthreads();
+  if constexpr (AHEAD) {
+    if (threadIdx.x < N) {
+      uint32_t sum = 0u;
+#pragma unroll
+      for (int c = 0; c < kBuildThreads / N; ++c) sum += s_before[c][threadIdx.x];
+      if (blockIdx.x == 0) {
+        if ((int)threadIdx.x <= levels)
+          __hip_atomic_store(&sizes[threadIdx.x], (int64_t)sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        sum = 0u;
+      }
+      s_before[0][threadIdx.x] = sum;
+    }
+    __syncthreads();
+  }
 #pragma unroll
   for (int l = 0; l < N; ++l) {
-    uint32_t r = offs[(int64_t)blockIdx.x * N + l];
+    uint32_t r = AHEAD ? s_before[0][l] : offs[(int64_t)blockIdx.x * N + l];
     for (int w = 0; w < wave; ++w) r += s_cnt[w][l];
     run[l] = r;
   }
@@ -366,7 +394,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
         const int d = depth - l;
         const int64_t kl = m >> (3 * l);
         const int64_t p = (int64_t)s[l + 1 < N ? l + 1 : l] - 1;
-        if constexpr (SPAN == kBuildSmallSpan)                // (points of batch ids beyond batch_size may have no place)
+        if constexpr (AHEAD)                                  // (points of batch ids beyond batch_size may have no place)
           if ((p << 3) >= t.begin[d + 1] - t.begin[d]) continue;
         t.children[d][(p << 3) | (kl & 7)] = (int32_t)s[l] - 1;
         if (t.index[d]) t.index[d][s[l] - 1] = (int32_t)((p << 3) | (kl & 7));
@@ -519,9 +547,10 @@ static int build_fill_t(const char* ws, int64_t n, int key_bits, int depth, int 
   const uint32_t* offs = (const uint32_t*)(ws + L.offs);
   hipLaunchKernelGGL(build_init_kernel, dim3((unsigned)cdiv(t.begin[depth + 1] + 4, 1024)), dim3(256), 0, st, t, depth,
                      full_depth);
-  hipLaunchKernelGGL((build_span(n) == kBuildSpan ? build_scatter_kernel<K, N, kBuildSpan> : build_scatter_kernel<K, N, kBuildSmallSpan>),
+  hipLaunchKernelGGL((build_span(n) == kBuildSpan ? build_scatter_kernel<K, N, kBuildSpan, false>
+                                                  : build_scatter_kernel<K, N, kBuildSmallSpan, false>),
                      dim3((unsigned)L.spans), dim3(kBuildThreads), 0, st, csorted, offs, perm, n, key_bits, depth, full_depth, t,
-                     sig, inverse, seg_start);
+                     sig, inverse, seg_start, (int64_t*)nullptr);
   return check_launch("octree_build_fill");
 }
 
@@ -1097,15 +1126,14 @@ extern "C" int ocnnx_tree_number(void* workspace, int64_t n, int depth, int full
   if (int rc = tree_layout(n, levels, &L)) return rc;
   const uint32_t* csorted = (const uint32_t*)((char*)workspace + L.csorted);
   uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
-  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
   const int64_t init = cdiv(t.begin[depth + 1] + 4, 4 * kBuildThreads);
   const BuildSignal sig{(const float4*)rows, out_pts, out_normals};
 #define OCNN_TREE_NUMBER(N)                                                                                                \
   hipLaunchKernelGGL((build_count_init_kernel<uint32_t, N, kBuildSmallSpan>), dim3((unsigned)(L.spans + init)),              \
                      dim3(kBuildThreads), 0, st, csorted, n, key_bits, levels, sums, (int)L.spans, t, depth, full_depth);    \
-  hipLaunchKernelGGL(build_offsets_kernel<N>, dim3(1), dim3(1024), 0, st, sums, L.spans, levels, offs, sizes);               \
-  hipLaunchKernelGGL((build_scatter_kernel<uint32_t, N, kBuildSmallSpan>), dim3((unsigned)L.spans), dim3(kBuildThreads), 0,  \
-                     st, csorted, offs, perm, n, key_bits, depth, full_depth, t, sig, inverse, seg_start)
+  hipLaunchKernelGGL((build_scatter_kernel<uint32_t, N, kBuildSmallSpan, true>), dim3((unsigned)L.spans),                    \
+                     dim3(kBuildThreads), 0, st, csorted, sums, perm, n, key_bits, depth, full_depth, t, sig, inverse,       \
+                     seg_start, sizes)
   static_assert(kTreeAheadPoints <= kBuildSmallPoints, "small spans");
   if (levels + 1 <= 8) { OCNN_TREE_NUMBER(8); }
   else { OCNN_TREE_NUMBER(16); }

@@ -728,9 +728,10 @@ struct Tree {
 // Waits for values that a kernel launched on `st` stores into pinned memory, n of them, none negative and all -1 until then.
 // They are watched for: a synchronisation comes back several microseconds after the kernel's end, and it would wait for what has
 // been launched behind that kernel.  Build and tables of 20 k points at depth 6, one after the other, 110 - 140 -> 92 - 100 us.  One
-// that is waited for by itself loses (113 -> 126 - 150; the build alone, 65 k points, 89 -> 98): a synchronisation behind eight
-// launches or more, which the one in the middle had kept from adding up, takes 25 us where one behind fewer takes 11.5, and the
-// eighth launch 14 us of the host; in a program that goes on (a network has some hundred launches) that is so either way.
+// that is waited for by itself lost (113 -> 126 - 150): a synchronisation behind eight launches or more, which the one in the
+// middle had kept from adding up, takes 25 us where one behind fewer takes 11.5, and the eighth launch 14 us of the host; in a
+// program that goes on (a network has some hundred launches) that is so either way.  Of small clouds, whose build and tables
+// are seven launches now, it takes 84.
 // Values that take long (a queue in front of them) are waited for, after a millisecond of watching without the interpreter lock.
 void wait_for(const Tensor& values, const c10::hip::HIPStream& st) {
   const volatile int64_t* v = (const volatile int64_t*)values.data_ptr();
