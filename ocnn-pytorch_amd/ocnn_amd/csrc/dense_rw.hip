@@ -291,15 +291,20 @@ __global__ __launch_bounds__(256, 1) void conv_dense_wgrad_rw_kernel(
   const __amdgpu_buffer_rsrc_t rs_xi = make_rsrc(x_index, x_indexed ? (uint32_t)(rows * 4) : 0u);
   const __amdgpu_buffer_rsrc_t rs_gi = make_rsrc(g_index, g_indexed ? (uint32_t)(rows * 4) : 0u);
   struct Idx { int32_t x, g; };
+  // the range's tiles from the last one down
+  auto first_row = [&](int64_t tile) {                             // (past the range: past the rows)
+    const int64_t at = t_begin + t_end - 1 - tile;
+    return (uint32_t)(at < t_begin ? tiles : at) * RT;
+  };
   auto load_index = [&](int64_t tile) {
-    const uint32_t row = (uint32_t)min(tile, tiles) * RT + 8 * wave + rl;
+    const uint32_t row = first_row(tile) + 8 * wave + rl;
     Idx r;
     r.x = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_xi, row * 4u, 0, 0);
     r.g = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_gi, row * 4u, 0, 0);
     return r;
   };
   auto stage = [&](int64_t tile, char* buf, const Idx& ix) {       // every wave issues exactly PW loads
-    const uint32_t row0 = (uint32_t)min(tile, tiles) * RT;        // past the range: past the rows, zeros
+    const uint32_t row0 = first_row(tile);
     const uint32_t row = row0 + 8 * wave + rl;                    // (piece i = wave + 4 j: row group i % 4 = wave)
     const bool live = (int64_t)row < rows;                        // an indexed row past the end must read zeros too
     const uint32_t xrow = x_indexed ? (uint32_t)ix.x : row, grow = g_indexed ? (uint32_t)ix.g : row;

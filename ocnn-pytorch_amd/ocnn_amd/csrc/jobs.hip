@@ -303,8 +303,9 @@ extern "C" int ocnnx_conv_backward(int dtype, const ocnnx_gather_args* dgrad, co
     bool sums = bias_grad == nullptr;
     if (!sums) sums = colsum_jobs(dtype, grad, grad_rows, grad_channels, bias_grad, colsum_workspace, colsum_bytes, before, after);
     launch_jobs(dtype, before, st);
-    if (d) rc = d->main();
-    if (rc == OCNN_OK && w) rc = w->main();
+    // (the data gradient last: what comes next reads it, and the memory-side cache still holds its end)
+    if (w) rc = w->main();
+    if (rc == OCNN_OK && d) rc = d->main();
     if (rc == OCNN_OK) {
       launch_jobs(dtype, after, st);
       rc = check_launch("conv_backward");
