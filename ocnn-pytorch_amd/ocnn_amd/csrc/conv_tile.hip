@@ -537,6 +537,10 @@ extern "C" int ocnnx_gather_tile_supported(int dtype, int64_t rows_in, int K, in
   return 1;
 }
 
+extern "C" int64_t ocnnx_gather_tile_packed_bytes(int dtype, int K, int cin, int cout) {
+  return dtype < 0 || dtype > 2 || K < 1 || cin < 1 || cout < 1 ? 0 : tile_packed_bytes(dtype, K, cin, cout);
+}
+
 // (a 2x2x2 table has an entry in every slot of every 32 rows, whatever its occupancy)
 extern "C" int ocnnx_gather_tile_ordered(int K, double plan_occupancy) {
   return K != 8 && plan_occupancy >= 0.0 && plan_occupancy <= kTgSkipMaxOccupancy;
@@ -567,7 +571,7 @@ template <typename T, bool F32> struct TilePass : Pass {
     const int64_t packed = tile_packed_bytes(dtype, a.K, a.cin, a.cout);
     if (packed + (int64_t)t.sc * t.sk * a.rows_out * a.cout * 4 > a.workspace_bytes) t.sc = t.sk = 1;   // (no room for the parts)
     partial = t.sc * t.sk > 1 ? (float*)((char*)a.workspace + packed) : nullptr;
-    before.add(pack_tile_job(dtype, a.w, a.workspace, a.K, a.cin, a.cout, a.w_transposed, a.reverse_slots));
+    if (!a.packed) before.add(pack_tile_job(dtype, a.w, a.workspace, a.K, a.cin, a.cout, a.w_transposed, a.reverse_slots));
     if (partial) after.add(tile_parts_job(partial, t.sc * t.sk, a.rows_out, a.cout, a.bias, bn, a.out));
   }
 
@@ -585,7 +589,7 @@ template <typename T, bool F32> struct TilePass : Pass {
                                         (size_t)(t.ks == 4 ? 8 : t.ks == 2 ? 2 : 0) * t.wc * t.wr * (4 / t.wr / t.ks) * t.mb * 4096);
 #define OCNN_TILE_LAUNCH(MB_, WC_, WR_, KS_, SKIP_)                                                                      \
   hipLaunchKernelGGL((conv_gather_tile_kernel<T, F32, MB_, WC_, WR_, KS_, SKIP_>), grid, dim3(256), lds, st, a.in,       \
-                     in_bytes, a.loc, a.uptr, a.urows, a.order, (const T*)a.workspace, a.bias, bn, a.out, partial, a.rows_out, a.K, \
+                     in_bytes, a.loc, a.uptr, a.urows, a.order, (const T*)(a.packed ? a.packed : a.workspace), a.bias, bn, a.out, partial, a.rows_out, a.K, \
                      a.cin, a.cout, tiles, per_xcd, t.sc, t.sk, rows_alloc)
 #define OCNN_TILE_CASE(MB_, WC_, WR_, KS_)                                   \
   if (t.mb == MB_ && t.wc == WC_ && t.wr == WR_ && t.ks == KS_) {            \
@@ -641,7 +645,7 @@ extern "C" int ocnnx_gather_tile(int dtype, const void* in, int64_t rows_in, con
                                  void* workspace, int64_t workspace_bytes, int split_c, int split_k, void* stream) {
   const ocnnx_gather_args args{in, rows_in, loc, uptr, urows, plan_max_distinct, plan_total, plan_occupancy, rows_out, K, w,
                                cin, cout, w_transposed, reverse_slots, bias, bn_or_null, out, workspace, workspace_bytes,
-                               split_c, split_k, nullptr};
+                               split_c, split_k, nullptr, nullptr};
   return ocnnx_gather_tile_args(dtype, &args, stream);
 }
 

@@ -178,7 +178,8 @@ struct GatherOp {
 
   // bn: a batch norm with running statistics that follows the layer; in the same pass where the kernel
   // has room for it, in place after it otherwise
-  Tensor run(Tensor data, Tensor table, Tensor W, OptTensor bias, const ocnnx_bn* bn = nullptr) const {
+  // packed: W as ocnnx_pack_tiles leaves it (the kernel of takes_packed())
+  Tensor run(Tensor data, Tensor table, Tensor W, OptTensor bias, const ocnnx_bn* bn = nullptr, const void* packed = nullptr) const {
     require_gpu(data);
     require_gpu(W);
     const int code = code_of(data.scalar_type());
@@ -221,7 +222,8 @@ struct GatherOp {
                                   reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
         break;
       case OCNNX_GATHER_TILE: {
-        const ocnnx_gather_args args = tile_args(ptr(data), ptr(W), ptr(bias), overflow ? nullptr : bn, out, ws);
+        ocnnx_gather_args args = tile_args(ptr(data), ptr(W), ptr(bias), overflow ? nullptr : bn, out, ws);
+        args.packed = packed;
         check(ocnnx_gather_tile_args(code, &args, st));
         if (!overflow) bn = nullptr;
         break;
@@ -269,8 +271,10 @@ struct GatherOp {
     const PlanArrays& p = *plan;
     return {data, rows_in, typed<uint16_t>(p.loc), typed<int32_t>(p.uptr), typed<int32_t>(p.urows), p.umax, p.total,
             p.occupancy, rows, K, W, cin, cout, transposed, reverse, bias, bn, out.data_ptr(), ws.data_ptr(), ws.numel(), 0, 0,
-            ordered ? plan->rows_order() : nullptr};
+            ordered ? plan->rows_order() : nullptr, nullptr};
   }
+
+  bool takes_packed() const { return kernel == OCNNX_GATHER_TILE && !padded; }
 
   // this pass with row i of its result written to row index[i] of `out`
   void run_into(Tensor& out, const Tensor& index, const Tensor& data, const Tensor& table, const Tensor& W,
@@ -679,9 +683,9 @@ Tensor batch_norm(const Tensor& x, const Tensor& weight, const Tensor& bias, con
 
 // A layer and the batch norm (+ residual, + ReLU) behind it, in evaluation and without gradients: the
 // normalisation rides on the convolution's own pass over its result where the kernel takes it.
-Tensor conv_bn(const std::shared_ptr<ConvLayer>& layer, const Tensor& data_in, const Tensor& weights, const OptTensor& bias,
-               const Tensor& running_mean, const Tensor& running_var, double eps, const OptTensor& gamma_in,
-               const OptTensor& beta_in, bool relu, const OptTensor& residual_in) {
+Tensor conv_bn_packed(const std::shared_ptr<ConvLayer>& layer, const Tensor& data_in, const Tensor& weights, const OptTensor& bias,
+                      const Tensor& running_mean, const Tensor& running_var, double eps, const OptTensor& gamma_in,
+                      const OptTensor& beta_in, bool relu, const OptTensor& residual_in, const void* packed) {
   at::AutoDispatchBelowADInplaceOrView below;
   const Tensor data = data_in.contiguous(), w = weights.to(data.scalar_type()).contiguous();
   const int cols = layer->fwd->view_cols ? layer->fwd->view_cols : layer->fwd->cout;
@@ -705,7 +709,58 @@ Tensor conv_bn(const std::shared_ptr<ConvLayer>& layer, const Tensor& data_in, c
   }
   const ocnnx_bn bn{mean.data_ptr(), var.data_ptr(), code_of(mean.scalar_type()), (float)eps,
                     ptr(gamma), ptr(beta), param_code(gamma, beta), relu, ptr(residual)};
-  return layer->fwd->run(data, layer->fwd_table, w, bias, &bn);
+  return layer->fwd->run(data, layer->fwd_table, w, bias, &bn, packed);
+}
+
+Tensor conv_bn(const std::shared_ptr<ConvLayer>& layer, const Tensor& data, const Tensor& weights, const OptTensor& bias,
+               const Tensor& running_mean, const Tensor& running_var, double eps, const OptTensor& gamma, const OptTensor& beta,
+               bool relu, const OptTensor& residual) {
+  return conv_bn_packed(layer, data, weights, bias, running_mean, running_var, eps, gamma, beta, relu, residual, nullptr);
+}
+
+// Residual blocks one behind the other, two such layers each, of which the second adds the block's input (the first block
+// `shortcut` in its place, if it is given).  Their weights are packed in one launch where the kernels read them packed: the
+// segmentation network of 20 blocks on 40 k points takes 1.77 ms so, 1.89 with a call and a packing launch for each layer.
+struct BlockLayer {
+  std::shared_ptr<ConvLayer> layer;
+  Tensor weights, mean, var;
+  OptTensor bias, gamma, beta;
+  double eps;
+  bool relu;
+};
+Tensor res_blocks(const std::vector<std::shared_ptr<BlockLayer>>& layers, Tensor data, const OptTensor& shortcut) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  TORCH_CHECK(layers.size() % 2 == 0, "res_blocks: two layers a block");
+  require_gpu(data);
+  const int code = code_of(data.scalar_type());
+  std::vector<Tensor> w(layers.size()), packed(layers.size());
+  std::vector<ocnnx_pack_item> items;
+  const auto flush = [&]() {
+    if (!items.empty()) check(ocnnx_pack_tiles(code, items.data(), (int)items.size(), hip_stream()));
+    items.clear();
+  };
+  for (size_t i = 0; i < layers.size(); ++i) {
+    const GatherOp& op = *layers[i]->layer->fwd;
+    w[i] = layers[i]->weights.to(data.scalar_type()).contiguous();
+    require_gpu(w[i]);
+    if (!op.takes_packed() || op.rows == 0 || w[i].numel() != (int64_t)op.K * op.cin * op.cout) continue;
+    packed[i] = workspace(ocnnx_gather_tile_packed_bytes(code, op.K, op.cin, op.cout), data);
+    items.push_back({ptr(w[i]), packed[i].data_ptr(), op.K, op.cin, op.cout, op.transposed, op.reverse});
+    if (items.size() == OCNNX_PACK_MOST) flush();
+  }
+  flush();
+  for (size_t i = 0; i < layers.size(); i += 2) {
+    const auto pass = [&](size_t j, const Tensor& x, const OptTensor& residual) {
+      const BlockLayer& l = *layers[j];
+      const GatherOp& op = *l.layer->fwd;
+      TORCH_CHECK(x.dim() == 2 && x.size(0) == op.rows_in && x.size(1) == op.cin, "res_blocks: the layers do not follow each other");
+      return conv_bn_packed(l.layer, x, w[j], l.bias, l.mean, l.var, l.eps, l.gamma, l.beta, l.relu, residual,
+                            packed[j].defined() ? packed[j].data_ptr() : nullptr);
+    };
+    const Tensor inner = pass(i, data, std::nullopt);
+    data = pass(i + 1, inner, i == 0 && shortcut.has_value() ? shortcut : OptTensor(data));
+  }
+  return data;
 }
 
 // ---- octree (octree/octree.py) ----------------------------------------------------------------
@@ -1056,6 +1111,13 @@ PYBIND11_MODULE(ocnn_host, m) {
   m.attr("WGRAD_SPARSE_INVERSE") = kWgradSparseInverse;
   m.def("conv", &conv, py::call_guard<py::gil_scoped_release>());
   m.def("conv_bn", &conv_bn, py::call_guard<py::gil_scoped_release>());
+  py::class_<BlockLayer, std::shared_ptr<BlockLayer>>(m, "BlockLayer")
+      .def(py::init([](std::shared_ptr<ConvLayer> layer, Tensor weights, OptTensor bias, Tensor mean, Tensor var, double eps,
+                       OptTensor gamma, OptTensor beta, bool relu) {
+        return std::make_shared<BlockLayer>(BlockLayer{std::move(layer), std::move(weights), std::move(mean), std::move(var),
+                                                       std::move(bias), std::move(gamma), std::move(beta), eps, relu});
+      }));
+  m.def("res_blocks", &res_blocks, py::call_guard<py::gil_scoped_release>());
   m.def("column_sum", &column_sum, py::call_guard<py::gil_scoped_release>());
   m.def(
       "rows_wgrad",

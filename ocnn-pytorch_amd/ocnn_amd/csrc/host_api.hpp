@@ -55,9 +55,20 @@ typedef struct {
   int64_t workspace_bytes;
   int split_c, split_k;
   const uint8_t* order;       // null, or the tiles' rows in the order of ocnnx_plan_order
+  const void* packed;         // null, or the weights as ocnnx_pack_tiles leaves them (ocnnx_gather_tile_packed_bytes)
 } ocnnx_gather_args;
 int ocnnx_gather_tile_ordered(int K, double plan_occupancy);
 int ocnnx_gather_tile_args(int dtype, const ocnnx_gather_args* args, void* stream);   // ocnnx_gather_tile
+
+// The weights of n layers in the order in which ocnnx_gather_tile reads them, in one launch.
+#define OCNNX_PACK_MOST 12
+typedef struct {
+  const void* w;
+  void* out;
+  int K, cin, cout, transposed, reverse_slots;
+} ocnnx_pack_item;
+int64_t ocnnx_gather_tile_packed_bytes(int dtype, int K, int cin, int cout);
+int ocnnx_pack_tiles(int dtype, const ocnnx_pack_item* items, int n, void* stream);
 typedef struct {
   const void* x;
   int64_t rows_x;

@@ -252,6 +252,24 @@ __global__ __launch_bounds__(256) void job_kernel(Job job) {
   run_job<T, KIND>(job, blockIdx.x, s_sums);
 }
 
+// The weights of several layers.  A launch for one layer is bound by its own start (4.2 us; 40 in a network of 32 - 256
+// channels in 16 bit: 169 us); up to 12 layers fit the arguments: 6 launches of 9.0 us in the same network.
+struct PackJobs {
+  int n;
+  unsigned blocks[OCNNX_PACK_MOST];
+  PackTileJob job[OCNNX_PACK_MOST];
+};
+template <typename T>
+__global__ __launch_bounds__(256) void pack_jobs_kernel(PackJobs jobs) {
+  typedef typename std::conditional<std::is_same<T, float>::value, bf16, T>::type P;
+  uint32_t block = blockIdx.x;
+  int i = 0;
+  while (i + 1 < jobs.n && block >= jobs.blocks[i]) block -= jobs.blocks[i++];
+  const PackTileJob& a = jobs.job[i];
+  if (a.aligned) pack_tile<T, P, true>((const T*)a.w, (P*)a.out, a.K, a.cin, a.cout, a.transposed, a.reverse, block);
+  else pack_tile<T, P, false>((const T*)a.w, (P*)a.out, a.K, a.cin, a.cout, a.transposed, a.reverse, block);
+}
+
 template <typename T> void launch_jobs(const Jobs& jobs, hipStream_t st) {
   unsigned blocks = 0;
   for (int i = 0; i < jobs.n; ++i) blocks += jobs.job[i].blocks;
@@ -283,6 +301,28 @@ Job tile_parts_job(const float* partial, int parts, int64_t rows, int cout, cons
 }  // namespace ocnn
 
 using namespace ocnn;
+
+extern "C" int ocnnx_pack_tiles(int dtype, const ocnnx_pack_item* items, int n, void* stream) {
+  OCNN_REQUIRE(dtype >= 0 && dtype <= 2 && n >= 1 && n <= OCNNX_PACK_MOST, "pack_tiles: dtype=%d n=%d", dtype, n);
+  OCNN_REQUIRE_PTRS("pack_tiles", items);
+  PackJobs jobs;
+  jobs.n = n;
+  unsigned blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    const ocnnx_pack_item& it = items[i];
+    OCNN_REQUIRE(it.w && it.out, "pack_tiles: a required pointer is NULL");
+    OCNN_REQUIRE(ocnnx_gather_tile_supported(dtype, 0, it.K, it.cin, it.cout, 0), "pack_tiles: shape not supported");
+    const Job j = pack_tile_job(dtype, it.w, it.out, it.K, it.cin, it.cout, it.transposed, it.reverse_slots);
+    jobs.blocks[i] = j.blocks;
+    jobs.job[i] = j.pack;
+    blocks += j.blocks;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == OCNN_F32) hipLaunchKernelGGL(pack_jobs_kernel<float>, dim3(blocks), dim3(256), 0, st, jobs);
+  else if (dtype == OCNN_F16) hipLaunchKernelGGL(pack_jobs_kernel<f16>, dim3(blocks), dim3(256), 0, st, jobs);
+  else hipLaunchKernelGGL(pack_jobs_kernel<bf16>, dim3(blocks), dim3(256), 0, st, jobs);
+  return check_launch("pack_tiles");
+}
 
 // Both passes and the bias gradient: what comes before the kernels in one launch, what comes after them in another.
 extern "C" int ocnnx_conv_backward(int dtype, const ocnnx_gather_args* dgrad, const ocnnx_wgrad_args* wgrad, const void* grad,

@@ -11,6 +11,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from .nn import OctreeConv, OctreeDeconv
+from .octree import Octree
 from .nn.octree_conv import _gather_op, _wgrad_op, call_native, conv_wgrad, column_sum
 from .nn.batchnorm import BatchNormRelu1d, kernels_take
 
@@ -63,6 +64,43 @@ def layer_bn(layer, bn, data, *args, residual=None, relu=None):
   if residual is None and relu is None:
     return bn(layer(data, *args))
   return bn(layer(data, *args), residual=residual, relu=relu)
+
+
+def _res_blocks(blocks, data, octree, depth):
+  """Residual blocks one behind the other in evaluation without gradients, every layer and batch norm as this package makes
+  them: one native call, which packs the weights of all of them in one launch.  None: by the modules themselves."""
+  if (torch.is_grad_enabled() or _lib.recorded() or _nn._global_forward_hooks or _nn._global_forward_pre_hooks or
+      not (isinstance(octree, Octree) and data.is_cuda and data.dim() == 2 and data.dtype in _lib.DTYPE_CODE)):
+    return None
+  native, dtype, (rows, width), layers = _lib.native(), data.dtype, data.shape, []
+  for block in blocks:
+    if type(block) is not OctreeResBlock2 or block.in_channels != width:
+      return None
+    parts = block._modules
+    for name, kind, relu in (('conv3x3a', OctreeConvBnRelu, None), ('conv3x3b', OctreeConvBn, True)):
+      part = parts.get(name)
+      if type(part) is not kind or not _plain(part):
+        return None
+      conv, bn = part._modules.get('conv'), part._modules.get('bn')
+      if not (type(conv) is OctreeConv and type(bn) is BatchNormRelu1d and not bn.training and _plain(conv) and _plain(bn)):
+        return None
+      stats, affine, held = bn._buffers, bn._parameters, conv._parameters
+      if not (stats.get('running_mean') is not None and 'running_var' in stats and 'weight' in affine and 'bias' in affine and
+              'weights' in held):
+        return None
+      made = conv.native_of_stride_1(dtype, (rows, width), octree, depth)
+      if made is None or not kernels_take(dtype, bn.num_features):
+        return None
+      width = conv.out_channels
+      layers.append(native.BlockLayer(made, held['weights'], held['bias'] if 'bias' in held else conv.bias, stats['running_mean'],
+                                      stats['running_var'], bn.eps, affine['weight'], affine['bias'],
+                                      bn.fused_relu if relu is None else relu))
+    if block.in_channels != block.out_channels and block is not blocks[0]:
+      return None                                           # (its shortcut is a layer between the blocks)
+    if width != block.out_channels:
+      return None
+  first = blocks[0]
+  return native.res_blocks(layers, data, first.conv1x1(data) if first.in_channels != first.out_channels else None)
 
 
 class OctreeConvBn(_LayerBn):
@@ -296,6 +334,9 @@ class OctreeResBlock2(torch.nn.Module):
     self.relu = torch.nn.ReLU(inplace=True)
 
   def forward(self, data: torch.Tensor, octree, depth: int):
+    out = _res_blocks((self,), data, octree, depth)
+    if out is not None:
+      return out
     out = self.conv3x3a(data, octree, depth)
     if self.in_channels != self.out_channels:
       data = self.conv1x1(data)
@@ -317,7 +358,12 @@ class OctreeResBlocks(torch.nn.Module):
         [resblk(widths[i], widths[i + 1], 1, bottleneck, nempty) for i in range(resblk_num)])
 
   def forward(self, data: torch.Tensor, octree, depth: int):
-    for blk in self.resblks:
+    blocks = tuple(self.resblks)
+    if not torch.is_grad_enabled() and not self.use_checkpoint and blocks and all(_plain(blk) for blk in blocks):
+      out = _res_blocks(blocks, data, octree, depth)
+      if out is not None:
+        return out
+    for blk in blocks:
       if self.use_checkpoint:
         data = torch.utils.checkpoint.checkpoint(blk, data, octree, depth, use_reentrant=False)
       else:

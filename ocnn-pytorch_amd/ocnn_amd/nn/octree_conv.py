@@ -698,13 +698,8 @@ class _Layer:
         self.wgrad = made is not None
 
 
-def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
-  """The layer's native passes, made at its first call on this octree and kept with it: (layer or
-  None where the forward pass is not one native pass, function that makes its engine)."""
-  if not (isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE):
-    return None, None
-  key = (engine, depth, tuple(kernel_size), stride, nempty, in_channels, out_channels, data.dtype, padded,
-         SPARSE_MIN_ROWS)
+def _layer_on(engine, dtype, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
+  key = (engine, depth, tuple(kernel_size), stride, nempty, in_channels, out_channels, dtype, padded, SPARSE_MIN_ROWS)
   layer = octree._layers.get(key)
 
   def made_engine():
@@ -713,7 +708,17 @@ def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_siz
     return eng
 
   if layer is None:
-    layer = octree._layers.setdefault(key, _lib.unrecorded(lambda: _Layer(made_engine(), data.dtype, padded)))
+    layer = octree._layers.setdefault(key, _lib.unrecorded(lambda: _Layer(made_engine(), dtype, padded)))
+  return layer, made_engine
+
+
+def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
+  """The layer's native passes, made at its first call on this octree and kept with it: (layer or
+  None where the forward pass is not one native pass, function that makes its engine)."""
+  if not (isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE):
+    return None, None
+  layer, made_engine = _layer_on(engine, data.dtype, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
+                                 max_buffer, padded)
   if not layer.ok:
     return None, None
   assert data.shape == layer.shape, \
@@ -823,6 +828,14 @@ class OctreeConv(OctreeConvBase, torch.nn.Module):
                          self.out_channels, self.kernel_size, self.stride, self.nempty, self.max_buffer,
                          self.stride == 2 and not self.nempty)
     return None if layer is None else layer.native
+
+  def native_of_stride_1(self, dtype, shape, octree, depth: int):
+    """native_layer for data of this type and shape that is still to be made, of a layer that keeps the rows."""
+    if self.method != 'hip' or self.stride != 1 or not self.is_conv_layer():
+      return None
+    layer, _ = _layer_on(_OctreeConv, dtype, octree, depth, self.in_channels, self.out_channels, self.kernel_size, 1,
+                         self.nempty, self.max_buffer, False)
+    return layer.native if layer.ok and layer.shape == shape else None
 
   def extra_repr(self) -> str:
     return ('in_channels={}, out_channels={}, kernel_size={}, stride={}, '

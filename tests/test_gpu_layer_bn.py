@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from ocnn_amd import _lib, synthetic
-from ocnn_amd.modules import Conv1x1, Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2
+from ocnn_amd.modules import Conv1x1, Conv1x1Bn, OctreeConvBnRelu, OctreeDeconvBnRelu, OctreeResBlock2, OctreeResBlocks
 from ocnn_amd.nn import OctreeConv
 from ocnn_amd.octree import Octree, Points
 
@@ -78,6 +78,30 @@ def test_residual_block(dtype, cin, cout):
       block(x, octree, 6)
     del part.forward
   assert seen == [1, 2, 2]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('cin,cout,blocks,bottleneck,nempty', [(32, 32, 1, 1, True), (64, 32, 7, 1, True), (32, 64, 2, 2, False),
+                                                              (24, 40, 2, 1, True), (256, 256, 6, 1, False)])
+def test_chain_of_blocks(dtype, cin, cout, blocks, bottleneck, nempty):
+  """Blocks in one call give the bits of their layers one by one (which a hook on a part of each asks for): more layers than
+  are packed in one launch, a shortcut of the first, channels that run padded, few rows and many."""
+  octree = _octree(6000, 6)
+  for depth in (3, 6):
+    rows = int((octree.nnum_nempty if nempty else octree.nnum)[depth])
+    print('chain', dtype, cin, cout, blocks, bottleneck, nempty, depth, rows, flush=True)
+    x = torch.randn(rows, cin, generator=torch.Generator().manual_seed(cin)).to('cuda', dtype)
+    chain, seen = _randomise(OctreeResBlocks(cin, cout, blocks, bottleneck, nempty), dtype), []
+    for _ in range(2):
+      with torch.no_grad():
+        one = chain(x, octree, depth)
+        hooks = [block.conv3x3a.register_forward_hook(lambda *a: seen.append(1)) for block in chain.resblks]
+        assert torch.equal(chain(x, octree, depth), one)
+        for hook in hooks:
+          hook.remove()
+        for m in chain.resblks:
+          m.conv3x3b.conv.weights.mul_(0.5)                  # (the weights are read on each call)
+    assert len(seen) == 2 * blocks and _both(chain, x, octree, depth) <= 2 * blocks * TOL[dtype]
 
 
 @pytest.mark.parametrize('part,names', [('conv', ['weights']), ('conv', ['bias']), ('bn', ['weight', 'bias']),
