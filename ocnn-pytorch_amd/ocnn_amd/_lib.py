@@ -133,7 +133,8 @@ INTERNAL_SIGNATURES = {
     'ocnnx_dwconv_backward_planned': (_i, [_i, _p, _p, _p, _p, _p, _i, _l, _l, _i, _p, _i, _p, _p, _p, _l, _p]),
     'ocnnx_dwconv_siblings_supported': (_i, [_i, _l, _i, _i, _i]),
     'ocnnx_dwconv_siblings_backward': (_i, [_i, _p, _p, _p, _p, _p, _i, _l, _l, _i, _p, _i, _p, _p, _p, _l, _p]),
-    'ocnnx_batch_norm_training': (_i, [_i, _p, _l, _i, _f, _p, _p, _p, _p, _p, _i, _f, _p, _p, _p, _i, _i, _p, _p, _p, _l, _p]),
+    'ocnnx_batch_norm_training': (_i, [_i, _p, _l, _i, _f, _p, _p, _p, _p, _p, _i, _f, _p, _p, _p, _i, _i, _p, _p, _p, _p, _l, _p]),
+    'ocnnx_batch_norm_mask_bytes': (_l, [_i, _l, _i]),
     'ocnnx_rows_wgrad_supported': (_i, [_i, _l, _i, _i]),
     'ocnnx_rows_wgrad_workspace_bytes': (_l, [_l, _i, _i]),
     'ocnnx_rows_wgrad': (_i, [_i, _p, _p, _l, _i, _i, _i, _p, _p, _l, _p]),

@@ -538,6 +538,7 @@ struct BatchNormCall {
   Tensor x, mean, invstd, gamma, beta, y;     // (y: only where the ReLU's mask is not a function of x alone)
   bool relu = false, training = false, has_residual = false;
   at::ScalarType wdtype = at::kFloat, bdtype = at::kFloat;
+  Tensor mask;                                // the mask itself, a bit a value, in y's place
 };
 
 // Gradients of x, weight, bias and residual, those of them that `want` names.
@@ -557,9 +558,9 @@ std::array<Tensor, 4> batch_norm_grads(const BatchNormCall& call, const Tensor& 
     gb = at::empty({c}, be.options());
   Tensor ws = workspace(ocnn_batch_norm_workspace_bytes((int)c), xs);
   float* s = (float*)sums.data_ptr();
-  check(ocnn_batch_norm_backward(code_of(xs.scalar_type()), ptr(xs), ptr(dy), rows, (int)c, (const float*)ptr(call.mean),
+  check(ocnnx_batch_norm_backward(code_of(xs.scalar_type()), ptr(xs), ptr(dy), rows, (int)c, (const float*)ptr(call.mean),
                                  (const float*)ptr(call.invstd), ptr(ga), ptr(be), param_code(ga, be), call.relu,
-                                 call.training, ptr(call.y), typed<void>(dx), typed<void>(dres), s, s + c, typed<void>(gw),
+                                 call.training, ptr(call.y), ptr(call.mask), typed<void>(dx), typed<void>(dres), s, s + c, typed<void>(gw),
                                  typed<void>(gb), ws.data_ptr(), ws.numel(), hip_stream()));
   if (want_w && !gw.defined()) gw = sums[0].to(call.wdtype);
   if (want_b && !gb.defined()) gb = sums[1].to(call.bdtype);
@@ -567,9 +568,9 @@ std::array<Tensor, 4> batch_norm_grads(const BatchNormCall& call, const Tensor& 
 }
 
 struct BatchNormBackward : public Node {
-  SavedVariable x, mean, invstd, gamma, beta, y;
+  SavedVariable x, mean, invstd, gamma, beta, y, mask;
   BatchNormCall call;                         // (its flags; the tensors are the saved ones)
-  bool keeps_y = false;
+  bool keeps_y = false, keeps_mask = false;
 
   variable_list apply(variable_list&& grads) override {
     variable_list out(4);
@@ -581,7 +582,8 @@ struct BatchNormBackward : public Node {
     now.invstd = invstd.unpack();
     now.gamma = gamma.unpack();
     now.beta = beta.unpack();
-    if (keeps_y) now.y = y.unpack(shared_from_this());
+    if (keeps_y) now.y = y.unpack(shared_from_this());       // (refuses an output that was changed since, also beside the mask)
+    if (keeps_mask) now.mask = mask.unpack();
     at::AutoDispatchBelowADInplaceOrView below;
     auto g = batch_norm_grads(now, dy, {task_should_compute_output(0), task_should_compute_output(1),
                                         task_should_compute_output(2), task_should_compute_output(3)});
@@ -589,7 +591,7 @@ struct BatchNormBackward : public Node {
     return out;
   }
   void release_variables() override {
-    for (SavedVariable* v : {&x, &mean, &invstd, &gamma, &beta, &y}) v->reset_data();
+    for (SavedVariable* v : {&x, &mean, &invstd, &gamma, &beta, &y, &mask}) v->reset_data();
   }
   std::string name() const override { return "BatchNormReluBackward"; }
 };
@@ -603,7 +605,7 @@ bool known_type(const Tensor& t) {
 // num_batches_tracked, incremented with the statistics.  backward: a backward pass follows.
 Tensor batch_norm_pass(const Tensor& x_in, const Tensor& weight, const Tensor& bias, const Tensor& running_mean,
                        const Tensor& running_var, const Tensor& count, bool batch_stats, bool track, double factor, double eps,
-                       bool relu, const Tensor& residual_in, bool backward, BatchNormCall* call) {
+                       bool relu, const Tensor& residual_in, bool backward, BatchNormCall* call, bool masks) {
   at::AutoDispatchBelowADInplaceOrView below;
   const Tensor x = x_in.contiguous();
   const int64_t rows = x.size(0), c = x.size(1);
@@ -611,7 +613,7 @@ Tensor batch_norm_pass(const Tensor& x_in, const Tensor& weight, const Tensor& b
   void* st = hip_stream();
   Tensor gamma = as_param(weight), beta = as_param(bias), mean, invstd;
   if (gamma.defined() && beta.defined() && beta.scalar_type() != gamma.scalar_type()) beta = beta.to(gamma.scalar_type());
-  Tensor y = at::empty_like(x), residual;
+  Tensor y = at::empty_like(x), residual, mask;
   if (residual_in.defined()) {
     residual = residual_in.contiguous();
     TORCH_CHECK(residual.sizes() == x.sizes() && residual.scalar_type() == x.scalar_type(),
@@ -626,12 +628,14 @@ Tensor batch_norm_pass(const Tensor& x_in, const Tensor& weight, const Tensor& b
     const bool moves = track && running_mean.defined();
     const bool in_place = moves && known_type(running_mean) && running_mean.scalar_type() == running_var.scalar_type() &&
                           running_mean.is_contiguous() && running_var.is_contiguous();
+    if (masks && backward && residual.defined() && relu)
+      if (const int64_t bytes = ocnnx_batch_norm_mask_bytes(code, rows, (int)c)) mask = at::empty({bytes}, x.options().dtype(at::kByte));
     check(ocnnx_batch_norm_training(code, ptr(x), rows, (int)c, (float)eps, (float*)mean.data_ptr(), (float*)var.data_ptr(),
                                     (float*)invstd.data_ptr(), in_place ? running_mean.data_ptr() : nullptr,
                                     in_place ? running_var.data_ptr() : nullptr,
                                     in_place ? code_of(running_mean.scalar_type()) : 0, in_place ? (float)factor : 0.f,
                                     typed<int64_t>(count), ptr(gamma), ptr(beta), pcode, relu, ptr(residual), y.data_ptr(),
-                                    ws.data_ptr(), ws.numel(), st));
+                                    typed<void>(mask), ws.data_ptr(), ws.numel(), st));
     if (moves && !in_place) {
       Tensor unbiased = var * ((double)rows / (double)std::max<int64_t>(rows - 1, 1));
       running_mean.mul_(1 - factor).add_(mean.to(running_mean.scalar_type()), factor);
@@ -651,6 +655,7 @@ Tensor batch_norm_pass(const Tensor& x_in, const Tensor& weight, const Tensor& b
   if (backward) {
     *call = {x, mean, invstd, gamma, beta, residual_in.defined() && relu ? y : Tensor(), relu, batch_stats,
              residual_in.defined()};
+    call->mask = mask;
     if (weight.defined()) call->wdtype = weight.scalar_type();
     if (bias.defined()) call->bdtype = bias.scalar_type();
   }
@@ -664,7 +669,7 @@ Tensor batch_norm(const Tensor& x, const Tensor& weight, const Tensor& bias, con
   const bool grad = any_requires_grad(inputs);
   BatchNormCall call;
   Tensor y = batch_norm_pass(x, weight, bias, running_mean, running_var, count, batch_stats, track, factor, eps, relu, residual,
-                             grad, &call);
+                             grad, &call, true);
   if (grad) {
     auto node = make_node<BatchNormBackward>(inputs);
     node->keeps_y = call.y.defined();
@@ -673,7 +678,9 @@ Tensor batch_norm(const Tensor& x, const Tensor& weight, const Tensor& bias, con
     node->invstd = SavedVariable(call.invstd, false);
     if (call.gamma.defined()) node->gamma = SavedVariable(call.gamma, false);
     if (call.beta.defined()) node->beta = SavedVariable(call.beta, false);
-    call.x = call.mean = call.invstd = call.gamma = call.beta = call.y = Tensor();
+    node->keeps_mask = call.mask.defined();
+    if (node->keeps_mask) node->mask = SavedVariable(call.mask, false);
+    call.mask = call.x = call.mean = call.invstd = call.gamma = call.beta = call.y = Tensor();
     node->call = std::move(call);
     torch::autograd::set_history(y, node);
     if (node->keeps_y) node->y = SavedVariable(y, true);
@@ -1133,7 +1140,8 @@ PYBIND11_MODULE(ocnn_host, m) {
          const OptTensor& count, bool batch_stats, bool track, double factor, double eps, bool relu, const OptTensor& res) {
         BatchNormCall call;
         Tensor y = batch_norm_pass(x, or_undefined(w), or_undefined(b), or_undefined(rm), or_undefined(rv),
-                                   or_undefined(count), batch_stats, track, factor, eps, relu, or_undefined(res), true, &call);
+                                   or_undefined(count), batch_stats, track, factor, eps, relu, or_undefined(res), true, &call,
+                                   false);
         return std::vector<Tensor>{y, call.x, call.mean, call.invstd, call.gamma, call.beta};
       },
       py::call_guard<py::gil_scoped_release>());

@@ -114,7 +114,15 @@ int ocnnx_gather_choose(int dtype, int64_t rows_in, int64_t rows_out, int K, int
 int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows, int channels, float eps, float* mean, float* var,
                               float* invstd, void* running_mean, void* running_var, int running_dtype, float factor,
                               int64_t* batches_tracked, const void* gamma, const void* beta, int param_dtype, int relu,
-                              const void* residual, void* y, void* workspace, int64_t workspace_bytes, void* stream);
+                              const void* residual, void* y, void* mask, void* workspace, int64_t workspace_bytes, void* stream);
+
+// Where both directions run in three launches: the size of what mask (or null) takes above, a bit for each value of y that is
+// positive.  Else 0, and mask is null.  With it ocnn_batch_norm_backward reads neither y nor, for its mask, x.
+int64_t ocnnx_batch_norm_mask_bytes(int dtype, int64_t rows, int channels);
+int ocnnx_batch_norm_backward(int dtype, const void* x, const void* dy, int64_t rows, int channels, const float* mean,
+                              const float* invstd, const void* gamma, const void* beta, int param_dtype, int relu, int training,
+                              const void* y, const void* mask, void* dx, void* d_residual, float* dgamma, float* dbeta,
+                              void* grad_gamma, void* grad_beta, void* workspace, int64_t workspace_bytes, void* stream);
 
 // ocnn_batch_norm_apply with a module's running statistics as it holds them (f32 / f16 / bf16).
 int ocnnx_batch_norm_running(int dtype, const void* x, int64_t rows, int channels, const void* running_mean,

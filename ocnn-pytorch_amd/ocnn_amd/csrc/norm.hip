@@ -2,7 +2,7 @@
 // it in every conv-bn-relu block fused in: training statistics, the normalise (+ ReLU) pass,
 // and the gradient.  Everything here is HBM-bound; the point of the fusion is the number of
 // passes over the tensor (forward 2 reads + 1 write, backward 4 reads + 1 write, the ReLU
-// costs none) and 16-byte accesses on channels-last rows.  Reductions are two-level with a
+// costs none; a residual one more read, and backward a write and two reads of bits) and 16-byte accesses on channels-last rows.  Reductions are two-level with a
 // fixed order (per-workgroup partial sums, then one thread per channel in fp64): no atomics,
 // bit-reproducible.
 //
@@ -12,6 +12,7 @@
 // residual 139 + 238, now 129 + 212; 40 k rows the same.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -210,7 +211,8 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
                                                        const void* __restrict__ beta, int pdtype, int relu,
                                                        const T* __restrict__ res, T* __restrict__ y,
                                                        const void* __restrict__ run_mean,
-                                                       const void* __restrict__ run_var, int rdtype, float eps) {
+                                                       const void* __restrict__ run_var, int rdtype, float eps,
+                                                       uint8_t* __restrict__ mask) {
   typedef BnVec<T, VEC> V;
   const int lpr = C / VEC, rpp = 256 / lpr;
   const int tid = threadIdx.x, rl = tid / lpr, cl = tid - rl * lpr;
@@ -258,21 +260,46 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* __restrict__ x, 
         o.v[v] = from_f32<T>(t);
       }
       *(V*)(y + ru * C + cl * VEC) = o;
+      if (mask) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) bits |= (to_f32(o.v[v]) > 0.f ? 1u : 0u) << v;
+        mask[ru * lpr + cl] = (uint8_t)bits;
+      }
     }
   }
 }
 
+// What the ReLU of the forward pass let through: a function of x alone, or, where a residual was added, its output or a byte
+// of bits for each VEC channels.  The bits are 1/16 of the output, which both passes of the backward pass read otherwise;
+// forward + backward with a residual, us, from the output / from the bits: fp16 1.11 M x 96 508 / 431, 460 k x 128 284 / 239,
+// 200 k x 192 202 / 169, fp32 300 k x 64 171 / 155 (writing them: 1 - 4 of that).  A kernel for each, since the rows of an output
+// that may not be there cost the others registers, a wave a SIMD of the elementwise pass: without residual fp16 1.11 M x 96
+// 361 / 345, 200 k x 192 151 / 143.
+enum BnMask { kBnOfX, kBnOfY, kBnBits };
+template <typename T, int VEC, int MASK> struct BnMasked {
+  typedef typename std::conditional<MASK == kBnBits, uint8_t, BnVec<T, VEC>>::type V;
+  V m;
+  __device__ __forceinline__ void load(const void* __restrict__ mask, int64_t vec) {
+    if constexpr (MASK != kBnOfX) m = ((const V*)mask)[vec];
+  }
+  __device__ __forceinline__ bool passed(int v, float of_x) const {
+    if constexpr (MASK == kBnOfY) return to_f32(m.v[v]) > 0.f;
+    else if constexpr (MASK == kBnBits) return (m >> v) & 1;
+    else return of_x > 0.f;
+  }
+};
+
 // partial[blk][0][c] = sum_r dy'[r][c],  partial[blk][1][c] = sum_r dy'[r][c] * xhat[r][c], with
 // xhat = (x - mean) * invstd and dy' = dy where the forward output was positive (relu) or dy.
-// ymask: the forward output, when it is not a function of x alone (a residual was added).
-template <typename T, int VEC>
+template <typename T, int VEC, int MASK>
 __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__ x, const T* __restrict__ dy,
                                                            int64_t rows, int C,
                                                            const float* __restrict__ mean,
                                                            const float* __restrict__ invstd,
                                                            const void* __restrict__ gamma,
                                                            const void* __restrict__ beta, int pdtype, int relu,
-                                                           const T* __restrict__ ymask,
+                                                           const void* __restrict__ mask,
                                                            float* __restrict__ partial) {
   typedef BnVec<T, VEC> V;
   __shared__ float s_a[256 * VEC], s_b[256 * VEC];
@@ -291,7 +318,8 @@ __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__
     bn_params<VEC>(gamma, beta, pdtype, cl * VEC, ga, be);
     // (four rows of both tensors in flight)
     for (int64_t r = (int64_t)blockIdx.x * (4 * rpp) + rl; r < rows; r += (int64_t)gridDim.x * (4 * rpp)) {
-      V a[4], g[4], ym[4];
+      V a[4], g[4];
+      BnMasked<T, VEC, MASK> pass[4];
       bool ok[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -299,7 +327,7 @@ __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__
         ok[u] = ru < rows;
         a[u] = *(const V*)(x + (ok[u] ? ru * C : 0) + cl * VEC);
         g[u] = *(const V*)(dy + (ok[u] ? ru * C : 0) + cl * VEC);
-        if (ymask) ym[u] = *(const V*)(ymask + (ok[u] ? ru * C : 0) + cl * VEC);
+        pass[u].load(mask, (ok[u] ? ru * lpr : 0) + cl);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
@@ -308,8 +336,7 @@ __global__ __launch_bounds__(256) void bn_bwd_stats_kernel(const T* __restrict__
           const float xc = to_f32(a[u].v[v]) - m[v];
           const float xh = xc * is[v];
           float d = ok[u] ? to_f32(g[u].v[v]) : 0.f;
-          if (relu && !(ymask ? to_f32(ym[u].v[v]) > 0.f
-                              : xc * (is[v] * ga[v]) + be[v] > 0.f)) d = 0.f;       // the forward pass's expression
+          if (relu && !pass[u].passed(v, xc * (is[v] * ga[v]) + be[v])) d = 0.f;       // the forward pass's expression
           s1[v] += d;
           s2[v] += d * xh;
         }
@@ -350,7 +377,7 @@ __global__ __launch_bounds__(kBnFinishThreads) void bn_bwd_finish_kernel(const f
 
 // training: dx = gamma * invstd * (dy' - dbeta / N - xhat * dgamma / N); with fixed statistics
 // (evaluation mode): dx = gamma * invstd * dy'.  Thread layout as in bn_apply_kernel.
-template <typename T, int VEC>
+template <typename T, int VEC, int MASK>
 __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__ x, const T* __restrict__ dy,
                                                            int64_t rows, int C,
                                                            const float* __restrict__ mean,
@@ -359,7 +386,7 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
                                                            const void* __restrict__ beta, int pdtype, int relu,
                                                            const float* __restrict__ dbeta,
                                                            const float* __restrict__ dgamma, int training,
-                                                           const T* __restrict__ ymask, T* __restrict__ dres,
+                                                           const void* __restrict__ mask, T* __restrict__ dres,
                                                            T* __restrict__ dx) {
   typedef BnVec<T, VEC> V;
   const int lpr = C / VEC, rpp = 256 / lpr;
@@ -381,14 +408,15 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
   const int64_t last = (rows + 2 * rpp - 1) / (2 * rpp) - 1;       // (four rows in flight cost more in occupancy than they gain)
   for (int64_t at = last - blockIdx.x; at >= 0; at -= gridDim.x) {
     const int64_t r = at * (2 * rpp) + rl;
-    V a[2], g[2], ym[2];
+    V a[2], g[2];
+    BnMasked<T, VEC, MASK> pass[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t ru = r + (int64_t)u * rpp;
       if (ru < rows) {
         a[u] = *(const V*)(x + ru * C + cl * VEC);
         g[u] = *(const V*)(dy + ru * C + cl * VEC);
-        if (ymask) ym[u] = *(const V*)(ymask + ru * C + cl * VEC);
+        pass[u].load(mask, ru * lpr + cl);
       }
     }
 #pragma unroll
@@ -400,7 +428,7 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
       for (int v = 0; v < VEC; ++v) {
         const float xc = to_f32(a[u].v[v]) - m[v];
         float d = to_f32(g[u].v[v]);
-        if (relu && !(ymask ? to_f32(ym[u].v[v]) > 0.f : xc * sc[v] + be[v] > 0.f)) d = 0.f;
+        if (relu && !pass[u].passed(v, xc * sc[v] + be[v])) d = 0.f;
         gr.v[v] = from_f32<T>(d);                                      // the gradient of the residual
         if (training) d = d - db[v] - (xc * is[v]) * dg[v];
         o.v[v] = from_f32<T>(d * sc[v]);
@@ -861,12 +889,13 @@ extern "C" int ocnn_batch_norm_stats(int dtype, const void* x, int64_t rows, int
 
 static int bn_apply(int dtype, const void* x, int64_t rows, int channels, const float* mean, const float* invstd,
                     const void* gamma, const void* beta, int param_dtype, int relu, const void* residual, void* y,
-                    const void* run_mean, const void* run_var, int run_dtype, float eps, hipStream_t st) {
+                    const void* run_mean, const void* run_var, int run_dtype, float eps, uint8_t* mask, hipStream_t st) {
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
     const int nblk = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_apply_kernel<T, VEC>));
     hipLaunchKernelGGL((bn_apply_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, rows, channels, mean, invstd,
-                       gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var, run_dtype, eps);
+                       gamma, beta, param_dtype, relu, (const T*)residual, (T*)y, run_mean, run_var, run_dtype, eps,
+                       mask);
   });
   return check_launch("batch_norm_apply");
 }
@@ -877,7 +906,14 @@ extern "C" int ocnn_batch_norm_apply(int dtype, const void* x, int64_t rows, int
   OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_apply: shape not supported");
   OCNN_REQUIRE_PTRS("batch_norm_apply", x, mean, invstd, y);
   return bn_apply(dtype, x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, residual, y, nullptr, nullptr, 0,
-                  0.f, (hipStream_t)stream);
+                  0.f, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int64_t ocnnx_batch_norm_mask_bytes(int dtype, int64_t rows, int channels) {
+  if (!ocnn_batch_norm_supported(dtype, rows, channels) || bn_slabs_take(dtype, rows, channels, false) ||
+      bn_slabs_take(dtype, rows, channels, true))
+    return 0;
+  return rows * (channels / bn_vec(dtype));
 }
 
 // Training: statistics of the batch (with the running ones moved) and the normalise pass behind them.
@@ -885,7 +921,7 @@ extern "C" int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows,
                                          float* var, float* invstd, void* running_mean, void* running_var,
                                          int running_dtype, float factor, int64_t* batches_tracked, const void* gamma,
                                          const void* beta, int param_dtype, int relu, const void* residual, void* y,
-                                         void* workspace, int64_t workspace_bytes, void* stream) {
+                                         void* mask, void* workspace, int64_t workspace_bytes, void* stream) {
   OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_training: shape not supported");
   OCNN_REQUIRE_PTRS("batch_norm_training", x, mean, var, invstd, y, workspace);
   OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels), "batch_norm_training: workspace too small");
@@ -895,8 +931,9 @@ extern "C" int ocnnx_batch_norm_training(int dtype, const void* x, int64_t rows,
                                              running_dtype, factor, batches_tracked, workspace, workspace_bytes, stream);
     if (status != OCNN_OK) return status;
     return bn_apply(dtype, x, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, residual, y, nullptr, nullptr,
-                    0, 0.f, (hipStream_t)stream);
+                    0, 0.f, (uint8_t*)mask, (hipStream_t)stream);
   }
+  OCNN_REQUIRE(!mask, "batch_norm_training: no mask of so few rows");
   const BnStats keep{eps, mean, var, invstd, running_mean, running_var, running_dtype, factor, (long long*)batches_tracked};
   const BnSlabs s = bn_slabs(dtype, rows, channels, kBnUnrollForward);
   double* partial = s.split ? (double*)workspace : nullptr;
@@ -919,7 +956,7 @@ extern "C" int ocnnx_batch_norm_running(int dtype, const void* x, int64_t rows, 
   OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_running: shape not supported");
   OCNN_REQUIRE_PTRS("batch_norm_running", x, running_mean, running_var, y);
   return bn_apply(dtype, x, rows, channels, nullptr, nullptr, gamma, beta, param_dtype, relu, residual, y, running_mean,
-                  running_var, running_dtype, eps, (hipStream_t)stream);
+                  running_var, running_dtype, eps, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy, int64_t rows, int channels,
@@ -928,13 +965,23 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
                                         const void* y, void* dx, void* d_residual, float* dgamma, float* dbeta,
                                         void* grad_gamma, void* grad_beta, void* workspace,
                                         int64_t workspace_bytes, void* stream) {
+  return ocnnx_batch_norm_backward(dtype, x, dy, rows, channels, mean, invstd, gamma, beta, param_dtype, relu, training, y,
+                                   nullptr, dx, d_residual, dgamma, dbeta, grad_gamma, grad_beta, workspace, workspace_bytes,
+                                   stream);
+}
+
+extern "C" int ocnnx_batch_norm_backward(int dtype, const void* x, const void* dy, int64_t rows, int channels,
+                                         const float* mean, const float* invstd, const void* gamma, const void* beta,
+                                         int param_dtype, int relu, int training, const void* y, const void* mask, void* dx,
+                                         void* d_residual, float* dgamma, float* dbeta, void* grad_gamma, void* grad_beta,
+                                         void* workspace, int64_t workspace_bytes, void* stream) {
   OCNN_REQUIRE(!d_residual || dx, "batch_norm_backward: d_residual needs dx");
   OCNN_REQUIRE(ocnn_batch_norm_supported(dtype, rows, channels), "batch_norm_backward: shape not supported");
   OCNN_REQUIRE_PTRS("batch_norm_backward", x, dy, mean, invstd, dgamma, dbeta, workspace);
   OCNN_REQUIRE(workspace_bytes >= ocnn_batch_norm_workspace_bytes(channels),
                "batch_norm_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
-  if (dx && bn_slabs_take(dtype, rows, channels, true)) {
+  if (dx && !mask && bn_slabs_take(dtype, rows, channels, true)) {
     const BnSlabs s = bn_slabs(dtype, rows, channels, kBnUnrollBackward);
     double* partial = s.split ? (double*)workspace : nullptr;
     OCNN_DISPATCH_DTYPE(dtype, {
@@ -953,15 +1000,19 @@ extern "C" int ocnn_batch_norm_backward(int dtype, const void* x, const void* dy
   float* partial = (float*)workspace;
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
-    const int nblk_a = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)bn_bwd_apply_kernel<T, VEC>));
-    hipLaunchKernelGGL((bn_bwd_stats_kernel<T, VEC>), dim3(nblk), dim3(256), 0, st, (const T*)x, (const T*)dy, rows,
-                       channels, mean, invstd, gamma, beta, param_dtype, relu, (const T*)y, partial);
-    hipLaunchKernelGGL(bn_bwd_finish_kernel, dim3((unsigned)cdiv(channels, 4)), dim3(kBnFinishThreads), 0, st, partial, nblk,
-                       channels, dbeta, dgamma, grad_gamma, grad_beta, param_dtype);
-    if (dx)
-      hipLaunchKernelGGL((bn_bwd_apply_kernel<T, VEC>), dim3(nblk_a), dim3(256), 0, st, (const T*)x, (const T*)dy, rows,
-                         channels, mean, invstd, gamma, beta, param_dtype, relu, dbeta, dgamma, training,
-                         (const T*)y, (T*)d_residual, (T*)dx);
+    const auto launch = [&](auto sums, auto apply, const void* passed) {
+      const int nblk_a = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)apply));
+      hipLaunchKernelGGL(sums, dim3(nblk), dim3(256), 0, st, (const T*)x, (const T*)dy, rows, channels, mean, invstd, gamma, beta,
+                         param_dtype, relu, passed, partial);
+      hipLaunchKernelGGL(bn_bwd_finish_kernel, dim3((unsigned)cdiv(channels, 4)), dim3(kBnFinishThreads), 0, st, partial, nblk,
+                         channels, dbeta, dgamma, grad_gamma, grad_beta, param_dtype);
+      if (dx)
+        hipLaunchKernelGGL(apply, dim3(nblk_a), dim3(256), 0, st, (const T*)x, (const T*)dy, rows, channels, mean, invstd, gamma,
+                           beta, param_dtype, relu, dbeta, dgamma, training, passed, (T*)d_residual, (T*)dx);
+    };
+    if (mask) launch(bn_bwd_stats_kernel<T, VEC, kBnBits>, bn_bwd_apply_kernel<T, VEC, kBnBits>, mask);
+    else if (y) launch(bn_bwd_stats_kernel<T, VEC, kBnOfY>, bn_bwd_apply_kernel<T, VEC, kBnOfY>, y);
+    else launch(bn_bwd_stats_kernel<T, VEC, kBnOfX>, bn_bwd_apply_kernel<T, VEC, kBnOfX>, nullptr);
   });
   return check_launch("batch_norm_backward");
 }

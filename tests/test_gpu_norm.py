@@ -10,6 +10,7 @@ import pytest
 from conftest import random_cases
 import torch
 
+from ocnn_amd import _lib
 from ocnn_amd.nn import BatchNormRelu1d
 
 pytestmark = pytest.mark.gpu
@@ -135,6 +136,40 @@ def test_batch_norm_residual_relu_vs_torch(dtype, training):
     y3 = bn(x3, residual=r3, relu=True)
     y3.backward(dy.to(DEV))
     assert torch.equal(r3.grad, rg.grad) and torch.equal(y3, y) == (not training or True)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('rows,c', [(300001, 32), (131075, 96), (90000, 264), (263, 32)])
+def test_batch_norm_mask_of_the_residual(dtype, rows, c):
+  """Of many rows the ReLU's mask is kept as bits: the bits of the passes that read the output in their place (and run where
+  something records), also of residuals that are the smallest normal number, infinite or NaN."""
+  from ocnn_amd.nn.batchnorm import _BatchNormFunction
+  say('batch norm mask', dtype, rows, c)
+  size = _lib.lib().ocnnx_batch_norm_mask_bytes(_lib.DTYPE_CODE[dtype], rows, c)
+  assert size == (rows * c // (4 if dtype == torch.float32 else 8) if rows > 1000 else 0)
+  g = torch.Generator(device=DEV).manual_seed(rows + c)
+  rand = lambda: torch.randn(rows, c, generator=g, device=DEV).to(dtype)
+  x, res, dy = rand(), rand(), rand()
+  pick = torch.arange(rows, device=DEV)
+  res[pick % 97 == 3] = float('nan')
+  res[pick % 97 == 50] = float('inf')
+  res[pick % 97 == 51] = -float('inf')
+  res[pick % 89 == 7] = torch.finfo(dtype).tiny
+  outs = []
+  for native in (True, False):
+    xs, rs = x.clone().requires_grad_(), res.clone().requires_grad_()
+    w, b = torch.linspace(-1, 2, c, device=DEV).requires_grad_(), torch.zeros(c, device=DEV).requires_grad_()
+    w.data[3] = 0                                            # (a column of the residual alone)
+    how = (None, True, False, 0.0, 1e-5, True)
+    y = (_lib.native().batch_norm(xs, w, b, None, None, *how, rs) if native
+         else _BatchNormFunction.apply(xs, w, b, rs, None, None, *how))
+    y.backward(dy, retain_graph=True)
+    outs.append([t.view(torch.uint8) for t in (y.detach(), xs.grad, rs.grad, w.grad, b.grad)])
+    with torch.no_grad():
+      y.add_(1)
+    with pytest.raises(RuntimeError, match='modified by an inplace operation'):
+      y.backward(dy)
+  assert all(torch.equal(p, q) for p, q in zip(*outs))
 
 
 def test_batch_norm_fallbacks_and_state_dict():
