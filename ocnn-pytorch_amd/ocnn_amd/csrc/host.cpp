@@ -217,9 +217,10 @@ struct GatherOp {
         bn = nullptr;
         break;
       case OCNN_GATHER_RW:
-        check(ocnn_conv_gather_rw(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
-                                  typed<int32_t>(p->urows), p->umax, p->total, rows, K, ptr(W), cin, cout, transposed,
-                                  reverse, ptr(bias), out.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        check(ocnnx_conv_gather_rw(code, ptr(data), rows_in, typed<uint16_t>(p->loc), typed<int32_t>(p->uptr),
+                                   typed<int32_t>(p->urows), p->umax, p->total, rows, K, ptr(W), cin, cout, transposed,
+                                   reverse, ptr(bias), overflow ? nullptr : bn, out.data_ptr(), ws.data_ptr(), ws.numel(), st));
+        if (!overflow) bn = nullptr;
         break;
       case OCNNX_GATHER_TILE: {
         ocnnx_gather_args args = tile_args(ptr(data), ptr(W), ptr(bias), overflow ? nullptr : bn, out, ws);

@@ -60,6 +60,12 @@ typedef struct {
 int ocnnx_gather_tile_ordered(int K, double plan_occupancy);
 int ocnnx_gather_tile_args(int dtype, const ocnnx_gather_args* args, void* stream);   // ocnnx_gather_tile
 
+// ocnn_conv_gather_rw with the batch norm (or null) behind the layer.
+int ocnnx_conv_gather_rw(int dtype, const void* in, int64_t rows_in, const uint16_t* loc, const int32_t* uptr,
+                         const int32_t* urows, int plan_max_distinct, int64_t plan_total, int64_t rows_out, int K, const void* w,
+                         int cin, int cout, int w_transposed, int reverse_slots, const void* bias, const ocnnx_bn* bn, void* out,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
 // The weights of n layers in the order in which ocnnx_gather_tile reads them, in one launch.
 #define OCNNX_PACK_MOST 12
 typedef struct {

@@ -2430,3 +2430,44 @@ def test_dense_rows_with_a_batch_norm_behind(dtype, cin, cout):
     # cin additions and some dozen operations of the epilogue in fp32, one rounding to the type
     bound = (cin + 16) * 2.0 ** -24 * scale + torch.finfo(dtype).eps / 2 * want.abs() * (1 + 2.0 ** -8) + 1e-7
     assert ((out - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('K', [27, 9, 8, 3])
+@pytest.mark.parametrize('ch', [32, 64])
+def test_register_resident_gathers_with_a_batch_norm_behind(dtype, K, ch):
+  """The kernels with the weights in registers, with what their epilogue carries in evaluation, all or some of it, against
+  float64: fewer rows than a tile, one tile a workgroup, several (whole rounds of the ring of tiles and not)."""
+  import importlib
+  from ocnn_amd.octree.octree import TilePlan
+  OC = importlib.import_module('ocnn_amd.nn.octree_conv')
+  g = torch.Generator().manual_seed(K + ch)
+  rand = lambda *shape: torch.randn(*shape, generator=g).to(DEV, dtype)
+  w = rand(K, ch, ch) / (K * ch) ** 0.5
+  for rows, (bias, gamma, beta, residual, relu) in ((4133, (1, 1, 1, 1, 1)), (33, (0, 1, 1, 0, 1)), (1, (0, 0, 0, 1, 0)),
+                                                    (128 * 300 + 1, (1, 0, 1, 1, 0)), (128 * 1100 + 77, (0, 1, 0, 1, 1))):
+    say('register-resident gather and batch norm', dtype, K, ch, rows, bias, gamma, beta, residual, relu)
+    table = _local_table(rows, rows, K, g).to(DEV)
+    op = OC._gather_op(dtype, rows, rows, K, ch, ch, False, False, TilePlan(table)).copy()
+    op.kernel = _lib.GATHER_RW
+    op.ws_bytes = K * ch * ch * 2
+    layer = _lib.native().ConvLayer(op, table, False)
+    x, mean, var = rand(rows, ch), rand(ch), rand(ch).abs() + 0.5
+    some = lambda wanted, *shape: rand(*shape) if wanted else None
+    b, ga, be, res = some(bias, ch), some(gamma, ch), some(beta, ch), some(residual, rows, ch)
+    out = _lib.native().conv_bn(layer, x, w, b, mean, var, 1e-3, ga, be, bool(relu), res).double()
+    d = lambda t, default: t.double() if t is not None else torch.full((ch,), float(default), dtype=torch.float64, device=DEV)
+    mul = d(ga, 1) / (var.double() + 1e-3).sqrt()
+    want = torch.zeros(rows, ch, dtype=torch.float64, device=DEV)
+    scale = want.clone()
+    for k in range(K):
+      a = x.double()[table[:, k].clamp_min(0).long()] * (table[:, k] >= 0)[:, None]
+      want, scale = want + a @ w[k].double(), scale + a.abs() @ w[k].double().abs()
+    want, scale = (want + d(b, 0) - mean.double()) * mul + d(be, 0), (scale + d(b, 0).abs() + mean.double().abs()) * mul.abs() + d(be, 0).abs()
+    if residual:
+      want, scale = want + res.double(), scale + res.double().abs()
+    if relu:
+      want = want.clamp_min(0)
+    # K ch additions and some dozen operations of the epilogue in fp32, one rounding to the type
+    bound = (K * ch + 16) * 2.0 ** -24 * scale + torch.finfo(dtype).eps / 2 * want.abs() * (1 + 2.0 ** -8) + 1e-7
+    assert ((out - want).abs() <= bound).all()
