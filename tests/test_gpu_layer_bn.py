@@ -81,17 +81,20 @@ def test_residual_block(dtype, cin, cout):
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize('cin,cout,blocks,bottleneck,nempty', [(32, 32, 1, 1, True), (64, 32, 7, 1, True), (32, 64, 2, 2, False),
+@pytest.mark.parametrize('cin,cout,blocks,bottleneck,nempty', [(32, 32, 1, 1, True), (64, 64, 7, 1, True), (64, 32, 7, 1, True), (32, 64, 2, 2, False),
                                                               (24, 40, 2, 1, True), (256, 256, 6, 1, False)])
 def test_chain_of_blocks(dtype, cin, cout, blocks, bottleneck, nempty):
   """Blocks in one call give the bits of their layers one by one (which a hook on a part of each asks for): more layers than
   are packed in one launch, a shortcut of the first, channels that run padded, few rows and many."""
-  octree = _octree(6000, 6)
-  for depth in (3, 6):
+  octree = _octree(30000, 7)
+  for depth in (3, 7):
     rows = int((octree.nnum_nempty if nempty else octree.nnum)[depth])
     print('chain', dtype, cin, cout, blocks, bottleneck, nempty, depth, rows, flush=True)
     x = torch.randn(rows, cin, generator=torch.Generator().manual_seed(cin)).to('cuda', dtype)
     chain, seen = _randomise(OctreeResBlocks(cin, cout, blocks, bottleneck, nempty), dtype), []
+    if depth == 7 and dtype != torch.float32 and bottleneck == 1 and cout in (32, 64):
+      last = chain.resblks[-1].conv3x3b.conv.native_of_stride_1(dtype, (rows, cout), octree, depth)
+      assert last.fwd.kernel == _lib.GATHER_RW
     for _ in range(2):
       with torch.no_grad():
         one = chain(x, octree, depth)
