@@ -1,6 +1,7 @@
 // Jobs that share a launch (jobs.hpp), and the backward pass of a layer with its small launches merged.
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "jobs.hpp"
 
@@ -343,9 +344,12 @@ extern "C" int ocnnx_conv_backward(int dtype, const ocnnx_gather_args* dgrad, co
     bool sums = bias_grad == nullptr;
     if (!sums) sums = colsum_jobs(dtype, grad, grad_rows, grad_channels, bias_grad, colsum_workspace, colsum_bytes, before, after);
     launch_jobs(dtype, before, st);
-    // (the data gradient last: what comes next reads it, and the memory-side cache still holds its end)
-    if (w) rc = w->main();
-    if (rc == OCNN_OK && d) rc = d->main();
+    // The data gradient last: what comes next reads it, and the memory-side cache still holds its end.  First where the launch
+    // behind both finishes it from parts (256 -> 256 on 3 k rows, us a layer: 92.1 with it last, 90.6).
+    Pass* order[2] = {w, d};
+    if (d && d->after.n) std::swap(order[0], order[1]);
+    for (Pass* p : order)
+      if (rc == OCNN_OK && p) rc = p->main();
     if (rc == OCNN_OK) {
       launch_jobs(dtype, after, st);
       rc = check_launch("conv_backward");
