@@ -291,7 +291,9 @@ __global__ __launch_bounds__(256, 1) void conv_dense_wgrad_rw_kernel(
   const __amdgpu_buffer_rsrc_t rs_xi = make_rsrc(x_index, x_indexed ? (uint32_t)(rows * 4) : 0u);
   const __amdgpu_buffer_rsrc_t rs_gi = make_rsrc(g_index, g_indexed ? (uint32_t)(rows * 4) : 0u);
   struct Idx { int32_t x, g; };
-  // the range's tiles from the last one down
+  // The range's tiles from the last one down: x was read, or g written, from the first row up just before, and its last
+  // 256 MB are in the memory-side cache.  Down and up from 64 channels over all nodes of depth 8 (2.3 M rows): 120 us a pass from
+  // the first tile up, 116 so.
   auto first_row = [&](int64_t tile) {                             // (past the range: past the rows)
     const int64_t at = t_begin + t_end - 1 - tile;
     return (uint32_t)(at < t_begin ? tiles : at) * RT;

@@ -2,9 +2,9 @@
 // it in every conv-bn-relu block fused in: training statistics, the normalise (+ ReLU) pass,
 // and the gradient.  Everything here is HBM-bound; the point of the fusion is the number of
 // passes over the tensor (forward 2 reads + 1 write, backward 4 reads + 1 write, the ReLU
-// costs none; a residual one more read, and backward a write and two reads of bits) and 16-byte accesses on channels-last rows.  Reductions are two-level with a
-// fixed order (per-workgroup partial sums, then one thread per channel in fp64): no atomics,
-// bit-reproducible.
+// costs none; a residual one more read, and backward one more write and bits) and 16-byte accesses on
+// channels-last rows.  Reductions are two-level with a fixed order (per-workgroup partial sums,
+// then one thread per channel in fp64): no atomics, bit-reproducible.
 //
 // The sums walk the rows from the first to the last, all workgroups side by side, and the elementwise pass that
 // reads the same tensors again walks them back: what was read last is in the memory-side cache (256 MB).  With a range

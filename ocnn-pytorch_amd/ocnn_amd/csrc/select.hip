@@ -150,7 +150,8 @@ extern "C" int ocnn_conv_wgrad_choose(int dtype, int64_t rows_x, int64_t rows, i
         ocnn_conv_wgrad_sparse_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_SPARSE;
     // (against the plan-free kernel, us: f16 32 -> 64 on 1.06 M rows 61 % set 119 / 775, 64 -> 32 197 / 732, 41 k 26 / 31, but 20 k
-    // 22 / 19 and 10 k 18 / 16; fp32 423 / 2451, 691 / 2307, 39 / 94, 34 / 55, 30 / 47)
+    // 22 / 19 and 10 k 18 / 16; fp32 32 -> 64 on 2.3 M rows 60 % set 660 / 5495, 39 k 32 / 85, 17 k 25 / 52, 4.9 k 19 / 41; 64 -> 32 756 / 5179,
+    // 30 / 80, 22 / 52, 15 / 41)
     if (!(narrow && dtype != OCNN_F32 && rows < kSparseMinRows) &&
         ocnn_conv_wgrad_planned_supported(dtype, rows_x, rows, K, ca, cb, plan_max_distinct))
       return OCNN_WGRAD_PLANNED;

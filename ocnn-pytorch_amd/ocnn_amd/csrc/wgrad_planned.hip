@@ -67,7 +67,7 @@ struct WpStage {
 //
 // 32 channels of x: blocks of 32 x 64 have as many sums over all 27 slots as 64 x 64 over half of them, so one
 // workgroup stages a range's rows for all slots: 32 -> 64 on 1.06 M rows (61 % set) 119 us, in half-empty 64 x 64 blocks of two
-// slot groups 201; fp32 423 / 696.
+// slot groups 201.
 template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool BLK, int CAP>
 __global__ __launch_bounds__(256, CAP < kWpCap ? 2 : 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
