@@ -137,8 +137,9 @@ __device__ inline uint32_t lanes_below(unsigned long long mask) {
 
 // starts of nodes, by layer, among the points of each workgroup's span: sums[span][N]
 template <typename K, int N, int SPAN>
-static __device__ __forceinline__ void build_count(const K* __restrict__ sorted, int64_t n, int key_bits, int levels,
-                                                   uint32_t* __restrict__ sums) {
+__global__ __launch_bounds__(kBuildThreads) void build_count_kernel(const K* __restrict__ sorted, int64_t n,
+                                                                    int key_bits, int levels,
+                                                                    uint32_t* __restrict__ sums) {
   __shared__ uint32_t s_cnt[kBuildThreads / 64][N];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = (int64_t)blockIdx.x * SPAN + wave * (SPAN / 4);
@@ -162,13 +163,6 @@ static __device__ __forceinline__ void build_count(const K* __restrict__ sorted,
     for (int w = 0; w < kBuildThreads / 64; ++w) c += s_cnt[w][threadIdx.x];
     sums[(int64_t)blockIdx.x * N + threadIdx.x] = c;
   }
-}
-
-template <typename K, int N, int SPAN>
-__global__ __launch_bounds__(kBuildThreads) void build_count_kernel(const K* __restrict__ sorted, int64_t n,
-                                                                    int key_bits, int levels,
-                                                                    uint32_t* __restrict__ sums) {
-  build_count<K, N, SPAN>(sorted, n, key_bits, levels, sums);
 }
 
 // offs[span][l] = starts at layer l before the span; sizes[l] = their total.  One workgroup: thread
@@ -213,8 +207,8 @@ struct BuildSignal {
 
 // Full layers, and -1 in the children of every other layer.  Four nodes a thread (the layers below the
 // full ones are whole groups of eight, and so are the full ones from layer 1 on).
-static __device__ __forceinline__ void build_init(const BuildTree& t, int depth, int full_depth, int64_t thread) {
-  const int64_t i = thread * 4;
+__global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= t.begin[depth + 1] - t.begin[1] + 4 * ((t.begin[1] + 3) / 4)) return;
   const int64_t root = 4 * ((t.begin[1] + 3) / 4);            // layer 0 (a node per octree) padded to groups of four
   if (i < root) {
@@ -235,19 +229,6 @@ static __device__ __forceinline__ void build_init(const BuildTree& t, int depth,
     if (d < full_depth) c = make_int4((int)j, (int)j + 1, (int)j + 2, (int)j + 3);
   }
   *(int4*)(t.children[d] + j) = c;
-}
-
-__global__ void build_init_kernel(BuildTree t, int depth, int full_depth) {
-  build_init(t, depth, full_depth, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// Both in one launch: workgroups behind those of the spans.
-template <typename K, int N, int SPAN>
-__global__ __launch_bounds__(kBuildThreads) void build_count_init_kernel(const K* __restrict__ sorted, int64_t n, int key_bits,
-                                                                         int levels, uint32_t* __restrict__ sums, int spans,
-                                                                         BuildTree t, int depth, int full_depth) {
-  if ((int)blockIdx.x < spans) build_count<K, N, SPAN>(sorted, n, key_bits, levels, sums);
-  else build_init(t, depth, full_depth, (int64_t)(blockIdx.x - spans) * kBuildThreads + threadIdx.x);
 }
 
 struct OpenLeaf {                // a leaf whose points a span does not hold all: its signals' sums so far
@@ -280,17 +261,12 @@ __device__ __forceinline__ void leaf_signals(const BuildSignal& sig, int64_t lea
 // 360 / 285 / 187; of a sphere at depth 5 460 / 428 / 207, depth 6 217 / 220 / 174, 3 M 508 / 600 / 372; 200 k points of one
 // cell 30300 / 51400 / 4580, one chain of additions.  (Where the next span starts a leaf, as most do, nothing follows the walk:
 // with the further points asked for in every span a build of 1 M points at depth 9 took 6 us more.)
-//
-// AHEAD (small clouds): offs holds the spans' counts, which every workgroup adds up itself; the first one also leaves their totals
-// in sizes (host memory).  A launch of one workgroup did that in between: build and tables of 20 k points
-// at depth 6 82 / 81 us, waited for by themselves 112 / 85 (seven launches: host.cpp, wait_for), 60 k at depth 7 122 / 108.
-template <typename K, int N, int SPAN, bool AHEAD>
+template <typename K, int N, int SPAN>
 __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     const K* __restrict__ sorted, const uint32_t* __restrict__ offs, const int32_t* __restrict__ perm, int64_t n,
     int key_bits, int depth, int full_depth, BuildTree t, BuildSignal sig, int64_t* __restrict__ inverse,
-    int32_t* __restrict__ seg_start, int64_t* __restrict__ sizes) {
+    int32_t* __restrict__ seg_start) {
   __shared__ uint32_t s_cnt[kBuildThreads / 64][N];
-  __shared__ uint32_t s_before[AHEAD ? kBuildThreads / N : 1][N];
   __shared__ __attribute__((aligned(16))) float s_sig[6][SPAN];
   __shared__ uint8_t s_new[SPAN];                            // the point starts a leaf (or is none)
   __shared__ OpenLeaf s_open;
@@ -301,15 +277,6 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
   const int64_t behind = ((int64_t)blockIdx.x + 1) * SPAN;
   const bool goes_on = sig.rows && behind < n && sorted[behind] == sorted[behind - 1];   // a leaf does, in the span behind
   if (threadIdx.x == 0) s_open.leaf = -1;
-  if constexpr (AHEAD) {
-    constexpr int kChunks = kBuildThreads / N;
-    const int spans = (int)gridDim.x, l = threadIdx.x % N, c = threadIdx.x / N;
-    const int until = blockIdx.x == 0 ? spans : (int)blockIdx.x;       // (the first span: all of them, for the totals)
-    uint32_t sum = 0u;
-#pragma unroll 8
-    for (int b = c; b < until; b += kChunks) sum += offs[(int64_t)b * N + l];
-    s_before[c][l] = sum;
-  }
   int lv[kIt], at[kIt];
   uint32_t run[N];
 #pragma unroll
@@ -347,23 +314,9 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
     s_sig[3][j] = v[it][0].w, s_sig[4][j] = v[it][1].x, s_sig[5][j] = v[it][1].y;
   }
   __syncthreads();
-  if constexpr (AHEAD) {
-    if (threadIdx.x < N) {
-      uint32_t sum = 0u;
-#pragma unroll
-      for (int c = 0; c < kBuildThreads / N; ++c) sum += s_before[c][threadIdx.x];
-      if (blockIdx.x == 0) {
-        if ((int)threadIdx.x <= levels)
-          __hip_atomic_store(&sizes[threadIdx.x], (int64_t)sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        sum = 0u;
-      }
-      s_before[0][threadIdx.x] = sum;
-    }
-    __syncthreads();
-  }
 #pragma unroll
   for (int l = 0; l < N; ++l) {
-    uint32_t r = AHEAD ? s_before[0][l] : offs[(int64_t)blockIdx.x * N + l];
+    uint32_t r = offs[(int64_t)blockIdx.x * N + l];
     for (int w = 0; w < wave; ++w) r += s_cnt[w][l];
     run[l] = r;
   }
@@ -394,8 +347,6 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
         const int d = depth - l;
         const int64_t kl = m >> (3 * l);
         const int64_t p = (int64_t)s[l + 1 < N ? l + 1 : l] - 1;
-        if constexpr (AHEAD)                                  // (points of batch ids beyond batch_size may have no place)
-          if ((p << 3) >= t.begin[d + 1] - t.begin[d]) continue;
         t.children[d][(p << 3) | (kl & 7)] = (int32_t)s[l] - 1;
         if (t.index[d]) t.index[d][s[l] - 1] = (int32_t)((p << 3) | (kl & 7));
         if (l + 1 <= lv[it]) {
@@ -410,7 +361,7 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(
       const int64_t node = (b << (3 * full_depth)) | (m >> (3 * levels));
       if (node < t.begin[full_depth + 1] - t.begin[full_depth]) {    // a batch id beyond batch_size has no node
         t.children[full_depth][node] = (int32_t)top - 1;
-        if (t.index[full_depth] && top <= t.begin[full_depth + 1] - t.begin[full_depth]) t.index[full_depth][top - 1] = (int32_t)node;
+        if (t.index[full_depth]) t.index[full_depth][top - 1] = (int32_t)node;
       }
     }
     if (!sig.rows) continue;
@@ -547,10 +498,9 @@ static int build_fill_t(const char* ws, int64_t n, int key_bits, int depth, int 
   const uint32_t* offs = (const uint32_t*)(ws + L.offs);
   hipLaunchKernelGGL(build_init_kernel, dim3((unsigned)cdiv(t.begin[depth + 1] + 4, 1024)), dim3(256), 0, st, t, depth,
                      full_depth);
-  hipLaunchKernelGGL((build_span(n) == kBuildSpan ? build_scatter_kernel<K, N, kBuildSpan, false>
-                                                  : build_scatter_kernel<K, N, kBuildSmallSpan, false>),
+  hipLaunchKernelGGL((build_span(n) == kBuildSpan ? build_scatter_kernel<K, N, kBuildSpan> : build_scatter_kernel<K, N, kBuildSmallSpan>),
                      dim3((unsigned)L.spans), dim3(kBuildThreads), 0, st, csorted, offs, perm, n, key_bits, depth, full_depth, t,
-                     sig, inverse, seg_start, (int64_t*)nullptr);
+                     sig, inverse, seg_start);
   return check_launch("octree_build_fill");
 }
 
@@ -998,25 +948,37 @@ extern "C" int64_t ocnnx_tree_workspace_bytes(int64_t n, int depth, int full_dep
                                                    : align_up(n * 8, 256) + align_up(n * 12, 256));
 }
 
-// where the sorted keys, the spans' counts and their offsets lie in the workspace of this file's own sort
-static int tree_layout(int64_t n, int levels, BuildLayout* L) {
-  if ((levels + 1 > 8 ? build_layout_t<uint32_t, 16>(n, L) : build_layout_t<uint32_t, 8>(n, L)) == OCNN_OK) return OCNN_OK;
-  set_error("tree_scan: rocprim size query failed");
-  return OCNN_ERR_HIP;
-}
-
-static int tree_sort(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch, int batch_is_float,
-                     int depth, int levels, int batch_bits, const float* normals, float* rows, char* workspace, int64_t base,
-                     int32_t* perm, hipStream_t st) {
-  char* more = workspace + base;
+extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
+                               int batch_is_float, int depth, int full_depth, int batch_bits, const float* normals, float* rows,
+                               void* workspace, int64_t workspace_bytes, int32_t* perm, int64_t* sizes, void* stream) {
+  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
+  OCNN_REQUIRE_PTRS("tree_scan", pts, h_bbmin, rows, workspace, perm, sizes);
+  if (workspace_bytes < ocnnx_tree_workspace_bytes(n, depth, full_depth, batch_bits)) {
+    set_error("tree_scan: workspace too small");
+    return OCNN_ERR_WORKSPACE;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int key_bits = 3 * depth, levels = depth - full_depth;
+  const int64_t base = ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits);
+  char* more = (char*)workspace + base;
+  if (!tree_own_sort(n, depth, batch_bits)) {
+    int64_t* key = (int64_t*)more;
+    float* norm = (float*)(more + align_up(n * 8, 256));
+    if (int rc = ocnn_points2key(pts, n, h_bbmin, factor, batch, batch_is_float, depth, norm, key, stream)) return rc;
+    hipLaunchKernelGGL(tree_rows_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, norm, normals, n, (float4*)rows);
+    return ocnn_octree_build_scan(key, n, depth, full_depth, batch_bits, workspace, base, perm, sizes, stream);
+  }
   const SortPlan s = sort_plan(n, tree_key_bits(depth, batch_bits));
   uint32_t* keys = (uint32_t*)(more + s.key);
   uint2* pairs[2] = {(uint2*)(more + s.pair[0]), (uint2*)(more + s.pair[1])};
   uint32_t* hist = (uint32_t*)(more + s.hist);
   uint32_t* totals = s.spans > kSortInlineSpans ? (uint32_t*)(more + s.totals) : nullptr;
   BuildLayout L;
-  if (int rc = tree_layout(n, levels, &L)) return rc;
-  uint32_t* csorted = (uint32_t*)(workspace + L.csorted);
+  if (build_layout_t<uint32_t, 8>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
+  if (levels + 1 > 8 && build_layout_t<uint32_t, 16>(n, &L) != OCNN_OK) { set_error("tree_scan: rocprim size query failed"); return OCNN_ERR_HIP; }
+  uint32_t* csorted = (uint32_t*)((char*)workspace + L.csorted);
+  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
+  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
   const dim3 grid((unsigned)s.spans), block(kSortThreads);
   hipLaunchKernelGGL(tree_keys_kernel, grid, block, 0, st, pts, n, h_bbmin[0], h_bbmin[1], h_bbmin[2], factor, batch,
                      batch_is_float, depth, normals, (float4*)rows, keys, s.bits, hist);
@@ -1031,42 +993,6 @@ static int tree_sort(const float* pts, int64_t n, const float* h_bbmin, float fa
     hipLaunchKernelGGL(pass, grid, dim3(kPassThreads), 0, st, keys, pairs[(p + 1) & 1], n, p * s.bits, s.bits, s.spans, hist, totals,
                        pairs[p & 1], csorted, (uint32_t*)perm);
   }
-  return check_launch("tree_sort");
-}
-
-static int tree_args_ok(int64_t n, int depth, int full_depth, int batch_bits, int64_t workspace_bytes) {
-  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
-  if (workspace_bytes < ocnnx_tree_workspace_bytes(n, depth, full_depth, batch_bits)) {
-    set_error("tree_scan: workspace too small");
-    return OCNN_ERR_WORKSPACE;
-  }
-  return OCNN_OK;
-}
-
-extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
-                               int batch_is_float, int depth, int full_depth, int batch_bits, const float* normals, float* rows,
-                               void* workspace, int64_t workspace_bytes, int32_t* perm, int64_t* sizes, void* stream) {
-  OCNN_REQUIRE_PTRS("tree_scan", pts, h_bbmin, rows, workspace, perm, sizes);
-  if (int rc = tree_args_ok(n, depth, full_depth, batch_bits, workspace_bytes)) return rc;
-  hipStream_t st = (hipStream_t)stream;
-  const int key_bits = 3 * depth, levels = depth - full_depth;
-  const int64_t base = ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits);
-  char* more = (char*)workspace + base;
-  if (!tree_own_sort(n, depth, batch_bits)) {
-    int64_t* key = (int64_t*)more;
-    float* norm = (float*)(more + align_up(n * 8, 256));
-    if (int rc = ocnn_points2key(pts, n, h_bbmin, factor, batch, batch_is_float, depth, norm, key, stream)) return rc;
-    hipLaunchKernelGGL(tree_rows_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, norm, normals, n, (float4*)rows);
-    return ocnn_octree_build_scan(key, n, depth, full_depth, batch_bits, workspace, base, perm, sizes, stream);
-  }
-  if (int rc = tree_sort(pts, n, h_bbmin, factor, batch, batch_is_float, depth, levels, batch_bits, normals, rows, (char*)workspace,
-                         base, perm, st))
-    return rc;
-  BuildLayout L;
-  if (int rc = tree_layout(n, levels, &L)) return rc;
-  const uint32_t* csorted = (const uint32_t*)((char*)workspace + L.csorted);
-  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
-  uint32_t* offs = (uint32_t*)((char*)workspace + L.offs);
 #define OCNN_TREE_COUNT(N)                                                                          \
   launch_build_count<uint32_t, N>(csorted, n, L.spans, key_bits, levels, sums, st);                  \
   hipLaunchKernelGGL(build_offsets_kernel<N>, dim3(1), dim3(1024), 0, st, sums, L.spans, levels, offs, sizes)
@@ -1074,69 +1000,4 @@ extern "C" int ocnnx_tree_scan(const float* pts, int64_t n, const float* h_bbmin
   else { OCNN_TREE_COUNT(16); }
 #undef OCNN_TREE_COUNT
   return check_launch("tree_scan");
-}
-
-// ---- small clouds: the whole build without a wait --------------------------------------------------
-// The sizes of the layers are known when the points are numbered, and what they are written to is allocated then: 20 us between
-// the kernels of a build whose kernels take 45.  Build and tables, us, waited in the middle / now: 20 k points depth 6 89 / 77,
-// 60 k depth 7 105 / 94, 100 k depth 8 123 / 115, 130 k depth 9 150 / 140, 250 k depth 7 118 / 108, depth 9 157 / 154.  A layer has 8 n nodes at most, and no more than there are cells, so a small
-// cloud's arrays can be made for that many while the points are sorted, and cut when the sizes have come, beside the scatter.  What
-// is not used of them stays theirs: 25 MB a layer from depth 7 on for 262 k points, whose neighbour tables take 100 - 200 MB.
-constexpr int64_t kTreeAheadPoints = 1 << 18;
-
-extern "C" int64_t ocnnx_tree_places(int64_t n, int batch_size, int depth) {
-  return std::min<int64_t>(8 * n, (int64_t)batch_size << (3 * depth));
-}
-
-extern "C" int ocnnx_tree_ahead(int64_t n, int depth, int full_depth, int batch_bits) {
-  return n > 0 && n <= kTreeAheadPoints && full_depth < depth && tree_own_sort(n, depth, batch_bits);
-}
-
-extern "C" int ocnnx_tree_sort(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch,
-                               int batch_is_float, int depth, int full_depth, int batch_bits, const float* normals, float* rows,
-                               void* workspace, int64_t workspace_bytes, int32_t* perm, void* stream) {
-  OCNN_REQUIRE(ocnnx_tree_ahead(n, depth, full_depth, batch_bits), "tree_sort: shape not supported");
-  OCNN_REQUIRE_PTRS("tree_sort", pts, h_bbmin, rows, workspace, perm);
-  if (int rc = tree_args_ok(n, depth, full_depth, batch_bits, workspace_bytes)) return rc;
-  return tree_sort(pts, n, h_bbmin, factor, batch, batch_is_float, depth, depth - full_depth, batch_bits, normals, rows,
-                   (char*)workspace, ocnn_octree_build_workspace_bytes(n, depth, full_depth, batch_bits), perm, (hipStream_t)stream);
-}
-
-extern "C" int ocnnx_tree_number(void* workspace, int64_t n, int depth, int full_depth, int batch_size, int batch_bits,
-                                 const int32_t* perm, int64_t* const* h_keys, int32_t* const* h_children, int32_t* const* h_index,
-                                 int64_t* inverse, int32_t* seg_start, const float* rows, float* out_pts, float* out_normals,
-                                 int64_t* sizes, void* stream) {
-  OCNN_REQUIRE(ocnnx_tree_ahead(n, depth, full_depth, batch_bits), "tree_number: shape not supported");
-  if (int rc = build_args_ok(n, depth, full_depth, batch_bits)) return rc;
-  OCNN_REQUIRE_PTRS("tree_number", workspace, perm, h_keys, h_children, h_index, inverse, seg_start, rows, out_pts, sizes);
-  OCNN_REQUIRE(batch_size >= 1 && batch_size <= (1 << batch_bits) && ((int64_t)batch_size << (3 * full_depth)) < (1ll << 31),
-               "tree_number: batch_size=%d does not fit batch_bits=%d / full_depth=%d", batch_size, batch_bits, full_depth);
-  BuildTree t;
-  t.begin[0] = 0;
-  for (int d = 0; d <= depth; ++d) {
-    OCNN_REQUIRE(h_keys[d] && h_children[d] && (d < full_depth || h_index[d]), "tree_number: depth %d: a missing array", d);
-    t.keys[d] = h_keys[d];
-    t.children[d] = h_children[d];
-    t.index[d] = h_index[d];
-    t.begin[d + 1] = t.begin[d] + (d <= full_depth ? (int64_t)batch_size << (3 * d) : ocnnx_tree_places(n, batch_size, d));
-  }
-  hipStream_t st = (hipStream_t)stream;
-  const int key_bits = 3 * depth, levels = depth - full_depth;
-  BuildLayout L;
-  if (int rc = tree_layout(n, levels, &L)) return rc;
-  const uint32_t* csorted = (const uint32_t*)((char*)workspace + L.csorted);
-  uint32_t* sums = (uint32_t*)((char*)workspace + L.sums);
-  const int64_t init = cdiv(t.begin[depth + 1] + 4, 4 * kBuildThreads);
-  const BuildSignal sig{(const float4*)rows, out_pts, out_normals};
-#define OCNN_TREE_NUMBER(N)                                                                                                \
-  hipLaunchKernelGGL((build_count_init_kernel<uint32_t, N, kBuildSmallSpan>), dim3((unsigned)(L.spans + init)),              \
-                     dim3(kBuildThreads), 0, st, csorted, n, key_bits, levels, sums, (int)L.spans, t, depth, full_depth);    \
-  hipLaunchKernelGGL((build_scatter_kernel<uint32_t, N, kBuildSmallSpan, true>), dim3((unsigned)L.spans),                    \
-                     dim3(kBuildThreads), 0, st, csorted, sums, perm, n, key_bits, depth, full_depth, t, sig, inverse,       \
-                     seg_start, sizes)
-  static_assert(kTreeAheadPoints <= kBuildSmallPoints, "small spans");
-  if (levels + 1 <= 8) { OCNN_TREE_NUMBER(8); }
-  else { OCNN_TREE_NUMBER(16); }
-#undef OCNN_TREE_NUMBER
-  return check_launch("tree_number");
 }

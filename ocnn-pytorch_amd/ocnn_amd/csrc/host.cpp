@@ -792,10 +792,9 @@ struct Tree {
 // Waits for values that a kernel launched on `st` stores into pinned memory, n of them, none negative and all -1 until then.
 // They are watched for: a synchronisation comes back several microseconds after the kernel's end, and it would wait for what has
 // been launched behind that kernel.  Build and tables of 20 k points at depth 6, one after the other, 110 - 140 -> 92 - 100 us.  One
-// that is waited for by itself lost (113 -> 126 - 150): a synchronisation behind eight launches or more, which the one in the
-// middle had kept from adding up, takes 25 us where one behind fewer takes 11.5, and the eighth launch 14 us of the host; in a
-// program that goes on (a network has some hundred launches) that is so either way.  Of small clouds, whose build and tables
-// are seven launches now, it takes 84.
+// that is waited for by itself loses (113 -> 126 - 150; the build alone, 65 k points, 89 -> 98): a synchronisation behind eight
+// launches or more, which the one in the middle had kept from adding up, takes 25 us where one behind fewer takes 11.5, and the
+// eighth launch 14 us of the host; in a program that goes on (a network has some hundred launches) that is so either way.
 // Values that take long (a queue in front of them) are waited for, after a millisecond of watching without the interpreter lock.
 void wait_for(const Tensor& values, const c10::hip::HIPStream& st) {
   const volatile int64_t* v = (const volatile int64_t*)values.data_ptr();
@@ -811,6 +810,18 @@ void wait_for(const Tensor& values, const c10::hip::HIPStream& st) {
   }
   std::atomic_thread_fence(std::memory_order_acquire);
   for (int64_t i = 0; i < n; ++i) TORCH_CHECK(v[i] >= 0, "a kernel left no sizes");
+}
+
+// Memory for a tensor made without elements, on the current device.  The layers of a build get theirs between two kernels, when
+// the sizes are known; the tensors around it are made while the sort runs.  Build and tables, us, with tensors made in between /
+// so: 20 k points at depth 6 87 / 83, 60 k depth 7 106 / 100, 100 k depth 8 120 / 112, 250 k depth 9 154 / 146.
+void room_for(Tensor& made, at::IntArrayRef sizes) {
+  at::TensorImpl* impl = made.unsafeGetTensorImpl();
+  at::StorageImpl* storage = impl->unsafe_storage().unsafeGetStorageImpl();
+  impl->set_sizes_contiguous(sizes);
+  const size_t bytes = (size_t)impl->numel() * made.itemsize();
+  storage->set_data_ptr_noswap(storage->allocator()->allocate(bytes));
+  storage->set_nbytes(bytes);
 }
 
 // Build from the points: one sort, one numbering of all layers, one wait for the layers' sizes.
@@ -841,15 +852,9 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   Tensor sizes = at::empty({levels + 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
   std::fill_n((int64_t*)sizes.data_ptr(), levels + 1, -1);
   const auto st = c10::hip::getCurrentHIPStream();
-  const bool ahead = ocnnx_tree_ahead(n, depth, full_depth, batch_bits);
-  if (ahead)
-    check(ocnnx_tree_sort((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
-                          full_depth, batch_bits, (const float*)ptr(normals), (float*)rows.data_ptr(), ws.data_ptr(), ws_bytes,
-                          (int32_t*)t.perm.data_ptr(), st.stream()));
-  else
-    check(ocnnx_tree_scan((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
-                          full_depth, batch_bits, (const float*)ptr(normals), (float*)rows.data_ptr(), ws.data_ptr(), ws_bytes,
-                          (int32_t*)t.perm.data_ptr(), (int64_t*)sizes.data_ptr(), st.stream()));
+  check(ocnnx_tree_scan((const float*)pts.data_ptr(), n, bbmin.data(), (float)factor, ptr(batch), batch_is_float, depth,
+                        full_depth, batch_bits, (const float*)ptr(normals), (float*)rows.data_ptr(), ws.data_ptr(), ws_bytes,
+                        (int32_t*)t.perm.data_ptr(), (int64_t*)sizes.data_ptr(), st.stream()));
   // what does not wait for the sizes is allocated while the sort runs
   for (int d = 0; d <= full_depth; ++d) {
     t.nnum.push_back((int64_t)batch_size << (3 * d));
@@ -858,55 +863,40 @@ Tree build_octree(Tensor pts, OptTensor normals, OptTensor batch, std::vector<fl
   }
   t.idx = at::empty({n}, i64);
   t.seg_start = at::empty({n + 1}, i32);
-  std::vector<int64_t> size(levels + 1, n);                  // (of a small cloud: room for as many)
-  const auto take_sizes = [&]() {
-    wait_for(sizes, st);
-    size.assign((int64_t*)sizes.data_ptr(), (int64_t*)sizes.data_ptr() + levels + 1);
-  };
-  if (!ahead) take_sizes();
-  std::vector<int64_t*> keys;
-  std::vector<int32_t*> children, index;
+  for (int d = 0; d <= depth; ++d) {                         // (room_for)
+    if (d > full_depth) {
+      t.keys.push_back(at::empty({0}, i64));
+      t.children.push_back(at::empty({0}, i32));
+    }
+    t.index.push_back(d < full_depth ? OptTensor() : at::empty({0}, i32));
+  }
+  t.points = at::empty({0}, pts.options());
+  if (normals.has_value()) t.normals = at::empty({0}, pts.options());
+  std::vector<int64_t*> keys(depth + 1);
+  std::vector<int32_t*> children(depth + 1), index(depth + 1);
+  t.nnum.resize(depth + 1);
+  t.nnum_nempty.resize(depth + 1);
+  wait_for(sizes, st);
+  const std::vector<int64_t> size((int64_t*)sizes.data_ptr(), (int64_t*)sizes.data_ptr() + levels + 1);
+  const c10::DeviceGuard device(pts.device());
   for (int d = 0; d <= depth; ++d) {
     if (d > full_depth) {
-      t.nnum.push_back(ahead ? ocnnx_tree_places(n, batch_size, d) : 8 * size[depth - d + 1]);
-      t.keys.push_back(at::empty({t.nnum[d]}, i64));
-      t.children.push_back(at::empty({t.nnum[d]}, i32));
+      t.nnum[d] = 8 * size[depth - d + 1];
+      room_for(t.keys[d], {t.nnum[d]});
+      room_for(t.children[d], {t.nnum[d]});
     }
-    t.nnum_nempty.push_back(d < full_depth ? t.nnum[d] : size[depth - d]);
-    t.index.push_back(d < full_depth ? OptTensor() : at::empty({t.nnum_nempty[d]}, i32));
-    keys.push_back((int64_t*)t.keys[d].data_ptr());
-    children.push_back((int32_t*)t.children[d].data_ptr());
-    index.push_back(d < full_depth ? nullptr : (int32_t*)t.index[d]->data_ptr());
+    t.nnum_nempty[d] = d < full_depth ? t.nnum[d] : size[depth - d];
+    if (d >= full_depth) room_for(*t.index[d], {t.nnum_nempty[d]});
+    keys[d] = (int64_t*)t.keys[d].data_ptr();
+    children[d] = (int32_t*)t.children[d].data_ptr();
+    index[d] = d < full_depth ? nullptr : (int32_t*)t.index[d]->data_ptr();
   }
-  t.points = at::empty({size[0], 3}, pts.options());
-  if (normals.has_value()) t.normals = at::empty({size[0], 3}, pts.options());
-  float *out_pts = (float*)t.points.data_ptr(), *out_normals = t.normals.has_value() ? (float*)t.normals->data_ptr() : nullptr;
-  if (ahead) {
-    check(ocnnx_tree_number(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, (const int32_t*)t.perm.data_ptr(),
-                            keys.data(), children.data(), index.data(), (int64_t*)t.idx.data_ptr(),
-                            (int32_t*)t.seg_start.data_ptr(), (const float*)rows.data_ptr(), out_pts, out_normals,
-                            (int64_t*)sizes.data_ptr(), st.stream()));
-    take_sizes();
-    TORCH_CHECK(size[levels] <= (int64_t)batch_size << (3 * full_depth), "octree_build_fill: ", size[levels],
-                " nodes at the deepest full layer of ", batch_size, " octrees");
-    const auto cut = [](const Tensor& made, at::IntArrayRef to) { made.unsafeGetTensorImpl()->set_sizes_contiguous(to); };
-    for (int d = full_depth; d <= depth; ++d) {
-      if (d > full_depth) {
-        t.nnum[d] = 8 * size[depth - d + 1];
-        cut(t.keys[d], {t.nnum[d]});
-        cut(t.children[d], {t.nnum[d]});
-      }
-      t.nnum_nempty[d] = size[depth - d];
-      cut(*t.index[d], {size[depth - d]});
-    }
-    cut(t.points, {size[0], 3});
-    if (t.normals.has_value()) cut(*t.normals, {size[0], 3});
-  } else {
-    check(ocnnx_tree_fill(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, size.data(),
-                          (const int32_t*)t.perm.data_ptr(), keys.data(), children.data(), index.data(),
-                          (int64_t*)t.idx.data_ptr(), (int32_t*)t.seg_start.data_ptr(), (const float*)rows.data_ptr(), out_pts,
-                          out_normals, st.stream()));
-  }
+  room_for(t.points, {size[0], 3});
+  if (normals.has_value()) room_for(*t.normals, {size[0], 3});
+  check(ocnnx_tree_fill(ws.data_ptr(), n, depth, full_depth, batch_size, batch_bits, size.data(),
+                        (const int32_t*)t.perm.data_ptr(), keys.data(), children.data(), index.data(),
+                        (int64_t*)t.idx.data_ptr(), (int32_t*)t.seg_start.data_ptr(), (const float*)rows.data_ptr(),
+                        (float*)t.points.data_ptr(), t.normals.has_value() ? (float*)t.normals->data_ptr() : nullptr, st.stream()));
   for (int d = 0; d <= depth; ++d)
     for (const Tensor* made : {&t.keys[d], &t.children[d]}) t.versions.push_back(made->is_inference() ? 0 : made->_version());
   return t;

@@ -182,16 +182,6 @@ int ocnnx_tree_fill(const void* workspace, int64_t n, int depth, int full_depth,
                     const int64_t* h_sizes, const int32_t* perm, int64_t* const* h_keys, int32_t* const* h_children,
                     int32_t* const* h_index, int64_t* inverse, int32_t* seg_start, const float* rows, float* out_pts,
                     float* out_normals, void* stream);
-// The same in two halves for small clouds (ocnnx_tree_ahead), without the sizes in between: sorted points, then everything else
-// into arrays of ocnnx_tree_places nodes a layer below the full ones and n entries an index; sizes comes back as from the scan.
-int ocnnx_tree_ahead(int64_t n, int depth, int full_depth, int batch_bits);
-int64_t ocnnx_tree_places(int64_t n, int batch_size, int depth);
-int ocnnx_tree_sort(const float* pts, int64_t n, const float* h_bbmin, float factor, const void* batch, int batch_is_float,
-                    int depth, int full_depth, int batch_bits, const float* normals, float* rows, void* workspace,
-                    int64_t workspace_bytes, int32_t* perm, void* stream);
-int ocnnx_tree_number(void* workspace, int64_t n, int depth, int full_depth, int batch_size, int batch_bits, const int32_t* perm,
-                      int64_t* const* h_keys, int32_t* const* h_children, int32_t* const* h_index, int64_t* inverse,
-                      int32_t* seg_start, const float* rows, float* out_pts, float* out_normals, int64_t* sizes, void* stream);
 int ocnnx_neigh_all(int depth, int full_depth, int batch, const int64_t* h_nnum, const int64_t* h_nnum_nempty,
                     const int64_t* const* h_keys, const int32_t* const* h_children,
                     const int32_t* const* h_nempty_index, int32_t* const* h_neigh, void* stream);

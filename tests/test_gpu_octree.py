@@ -455,14 +455,14 @@ def test_deep_octrees_vs_oracle(depth, full, batch, n):
 @pytest.mark.parametrize('n', [1, 255, 257, 40000, 262144, 262145])
 @pytest.mark.parametrize('depth,full', [(5, 2), (10, 1)])
 def test_builds_with_and_without_a_wait_for_the_sizes(n, depth, full):
-  """Clouds up to and beyond the size whose layers get their places before their sizes are known (one in which every point is
-  a leaf of its own, as far as there are cells, needs many), with more layers than eight counters hold: bit exact against the oracle;
-  what the octree holds is contiguous, of the layers' sizes, and can be written to, copied and saved."""
+  """Clouds of both spans of points a workgroup, with as many leaves as points where there are cells for them, and with more
+  layers than eight counters hold: bit exact against the oracle; what the octree holds is contiguous, of the layers' sizes, and
+  can be written to, copied and saved."""
   import io
   rng = np.random.default_rng(n + depth)
   pts = rng.uniform(-1, 0.999999, (n, 3)).astype(np.float32)
   nrm = rng.standard_normal((n, 3)).astype(np.float32)
-  say('build, sizes ahead or waited for', n, depth, full)
+  say('build, short and long spans', n, depth, full)
   o = Octree(depth, full)
   idx = o.build_octree(Points(torch.from_numpy(pts).to(DEV), torch.from_numpy(nrm).to(DEV)))
   w, widx = R.build_octree(pts, nrm, None, None, depth, full, 1)
@@ -485,9 +485,38 @@ def test_builds_with_and_without_a_wait_for_the_sizes(n, depth, full):
   assert o.children[depth].clone().shape == w.children[depth].shape
 
 
+@pytest.mark.parametrize('n,depth,full', [(1, 5, 2), (300, 6, 2), (20000, 6, 2), (60000, 9, 2), (262144, 7, 1), (262145, 7, 2)])
+def test_layers_hold_the_memory_of_their_nodes(n, depth, full):
+  """The storages of keys, children, indices and leaf averages end where the tensors end, also of a cloud that fills few of the
+  cells, and so does what torch.save writes; the memory that an octree takes is that of its tensors, to the allocator's grain."""
+  import io
+  g = torch.Generator().manual_seed(n)
+  pts = torch.randn(n, 3, generator=g)
+  nrm = pts / pts.norm(dim=1, keepdim=True)
+  pc = Points((nrm * 0.9).to(DEV), nrm.to(DEV))
+  say('memory of the layers', n, depth, full)
+  Octree(depth, full).build_octree(pc)
+  held = torch.cuda.memory_allocated()
+  o = Octree(depth, full)
+  idx = o.build_octree(pc)
+  held = torch.cuda.memory_allocated() - held
+  made = [*o.keys, *o.children, o.points[depth], o.normals[depth], *(o.nempty_index(d) for d in range(full, depth + 1))]
+  for t in made:
+    assert t.untyped_storage().nbytes() == t.nbytes
+  # (and the point's leaf, order and place: 8 + 4 + 4 bytes; blocks of 512 bytes, from 1 MB on up to 1 MB more)
+  blocks = [t.nbytes for t in made] + [idx.nbytes, 4 * n, 4 * n + 4]
+  assert held <= sum(b + 512 if b < (1 << 20) - 512 else b + (1 << 20) for b in blocks)
+  file = io.BytesIO()
+  torch.save([o.keys[depth], o.children[depth]], file)
+  assert file.tell() <= o.keys[depth].nbytes + o.children[depth].nbytes + 4096
+  o.keys[depth].add_(1)
+  bigger = o.children[depth].clone().resize_(2 * o.children[depth].numel())
+  assert torch.equal(bigger[:o.children[depth].numel()], o.children[depth])
+
+
 def test_batch_ids_without_octrees_are_refused():
-  """More nodes at the deepest full layer than the octrees have, of batch ids beyond them: an error, and nothing written
-  outside of the layers (tensors made before and after are as they were)."""
+  """More nodes at the deepest full layer than the octrees have, of batch ids beyond them: an error, raised when the sizes are
+  known and before a layer is made (a tensor made before is as it was)."""
   before = torch.full((1 << 16,), 7, dtype=torch.int32, device=DEV)
   grid = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing='ij'), -1).reshape(-1, 3) / 2.0 - 0.9
   pts = np.tile(grid, (4, 1)).astype(np.float32)
