@@ -367,10 +367,11 @@ static double wf_tile_us(int K, int cb, int groups) {
 // pieces'.  Blocks of 32 have half the sums to write.
 static int64_t wf_run(int cb) { return wf_block(cb) == 64 ? 24 : 16; }
 
-WfSplit wf_split_tiles(int64_t tiles, int K, int ca, int cb, int n_cu) {
+static WfSplit wf_split_launch(int64_t tiles, int K, int ca, int cb, int n_cu) {
   const int cu_xcd = std::max(1, n_cu / 8);
   const double sums = (double)K * ca * cb * 4 * kWfSumUs;
-  WfSplit best{std::max<int64_t>(tiles, 1), std::max<int64_t>(tiles, 1), 1};
+  tiles = std::max<int64_t>(tiles, 1);
+  WfSplit best{tiles, tiles, 1, tiles, 1};
   double least = 1e30;
   for (int groups = 1; groups <= (K == 27 ? 2 : 1); ++groups) {
     const int wgs = wf_range_workgroups(ca, cb, groups);
@@ -387,10 +388,26 @@ WfSplit wf_split_tiles(int64_t tiles, int K, int ca, int cb, int n_cu) {
       const int64_t used = cdiv(tiles, per);
       const double us = (double)cdiv(cdiv(used * wgs, 8), cu_xcd) * ((double)per * tile_us + kWfFixedUs) +
                         (double)(sets > 1 ? cdiv(tiles, run) : used) * sums;
-      if (us < least) least = us, best = WfSplit{per, run, groups};
+      if (us < least) least = us, best = WfSplit{per, run, groups, tiles, cdiv(tiles, run)};
     }
   }
   return best;
+}
+
+// The sets of sums grow with the rows: 27 slots of 512 x 512 channels 2.4 GB for every 256 k rows.  Beyond this many bytes the tiles
+// are taken in launches of as many as fit, with a reduction into one set behind each.  That costs nothing, the sets of a launch
+// are still in the memory-side cache when they are added: 512 -> 512 on 300 k rows 2.7 GB and 9.71 ms in one launch, 0.76 GB
+// and 9.54 ms in several, 1024 -> 1024 on 60 k 2.3 GB and 7.83 ms, 0.86 and 7.35, nine slots on 100 k 1.2 and 6.88, 0.76 and 6.55.
+// (The sums of a range added to by its workgroup, a read for every further set: the kernel's registers do not hold that beside the
+// accumulators, 64 -> 64 on 252 k rows 139 -> 165 us.)
+constexpr int64_t kWfSumsBytes = 1ll << 30;
+WfSplit wf_split_tiles(int64_t tiles, int K, int ca, int cb, int n_cu) {
+  WfSplit s = wf_split_launch(tiles, K, ca, cb, n_cu);
+  const int64_t room = kWfSumsBytes / ((int64_t)K * ca * cb * 4), most = std::max<int64_t>(1, room - 2);
+  if (s.sets <= std::max<int64_t>(1, room)) return s;
+  for (int64_t n = cdiv(tiles, most * wf_run(cb)); s.sets > most && s.launch > 1; n += cdiv(n, 4))
+    s = wf_split_launch(cdiv(tiles, n), K, ca, cb, n_cu);
+  return s;
 }
 
 template <int CB, int KK, int GROUPS> static void launch_wf(const WfArgs& a, hipStream_t st) {

@@ -474,8 +474,9 @@ extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes_for(int dtype, int64_
                                                                int ca, int cb) {
   if (dtype != OCNN_F32 || rows_x < 0 || rows < 0) return ocnn_conv_wgrad_planned_workspace_bytes(K, ca, cb);
   const int n_cu = wp_cu_count();
-  const int64_t tiles = cdiv(rows, kWpRows), run = n_cu > 0 ? wf_split_tiles(tiles, K, ca, cb, n_cu).run : 1;
-  return align_up(cdiv(tiles, run) * K * ca * cb * 4, 256);
+  const int64_t tiles = cdiv(rows, kWpRows);
+  const int64_t sets = n_cu > 0 ? wf_workspace_sets(wf_split_tiles(tiles, K, ca, cb, n_cu), tiles) : tiles;
+  return align_up(sets * K * ca * cb * 4, 256);
 }
 
 struct WpArgs {
@@ -536,6 +537,7 @@ template <typename T> struct WpPass : Pass {
   hipStream_t st;
   WfSplit f32;
   int rc = OCNN_OK, splits = 0, out_transposed = 0;
+  float* sums_at = nullptr;
   void* gw = nullptr;         // set: the reduction is launched behind the kernel (sums at an odd address)
 
   WpPass(const ocnnx_wgrad_args& p, hipStream_t stream) : st(stream) {
@@ -550,7 +552,7 @@ template <typename T> struct WpPass : Pass {
     const int64_t tiles = cdiv(p.rows, kWpRows), sums = (int64_t)K * ca * cb * 4;       // bytes of a range's sums
     if (F32) {
       f32 = wf_split_tiles(tiles, K, ca, cb, n_cu);
-      a.used = (int)cdiv(tiles, f32.run);
+      a.used = (int)wf_workspace_sets(f32, tiles);
     } else {
       a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, wp_places(ca, cb, n_cu, a.two));
       a.used = (int)cdiv(tiles, a.per);
@@ -562,24 +564,53 @@ template <typename T> struct WpPass : Pass {
     }
     const int64_t per = (int64_t)K * ca * cb;
     splits = p.rows > 0 ? a.used : 0;
+    sums_at = a.partial;
+    if (F32 && p.rows > 0) {                                 // the reduction behind the last launch
+      const WfPart last = part_of((cdiv(tiles, f32.launch) - 1) * f32.launch);
+      splits = (int)last.splits, sums_at = last.sums_at;
+    }
     if ((uintptr_t)a.partial % 16 != 0) {
       gw = p.gw, out_transposed = p.out_transposed;
       return;
     }
     const int lanes = wgrad_reduce_lanes(splits, per);
     Job j{Job::kReduce, (unsigned)cdiv(per / 4, 256 / lanes), {}};
-    j.reduce = ReduceJob{a.partial, p.gw, per, splits, p.out_transposed ? ca : 0, cb, lanes};
+    j.reduce = ReduceJob{sums_at, p.gw, per, splits, p.out_transposed ? ca : 0, cb, lanes};
     after.add(j);
+  }
+
+  // fp32 in several launches: their sets lie at 1 .., and what those before have come to (none before the first) at 0 or behind the
+  // last place for a set, where the reduction of the launch before left it; their own goes to the other of the two.
+  struct WfPart {
+    int64_t first, tiles, splits;               // splits: with the sum of those before
+    float *partial, *sums_at, *sum_to;
+  };
+  WfPart part_of(int64_t first) const {
+    const int64_t tiles = cdiv(a.rows, kWpRows), per = (int64_t)a.K * a.ca * a.cb, n = std::min(f32.launch, tiles - first);
+    if (f32.launch >= tiles) return {0, tiles, f32.sets, a.partial, a.partial, nullptr};
+    const int64_t number = first / f32.launch, sets = cdiv(n, f32.run), end = f32.sets + 1;
+    const bool behind = number % 2 == 0 && number > 0;       // the sum of those before lies behind
+    const int64_t at = behind ? end - sets : 1;
+    return {first, n, sets + (number > 0), a.partial + at * per, a.partial + (number == 0 || behind ? at : 0) * per,
+            a.partial + (number % 2 == 0 ? 0 : end) * per};
   }
 
   int main() override {
     if (a.rows > 0) {
-      if constexpr (F32)
-        launch_wgrad_f32({(const float*)a.x, (const float*)a.g, a.rows_x, a.rows, a.plan_total, a.loc, a.uptr, a.urows, a.K, a.ca,
-                          a.cb, f32, a.partial}, st);
-      else launch_wp_sums<T>(a, st);
+      if constexpr (F32) {
+        const int64_t tiles = cdiv(a.rows, kWpRows);
+        for (int64_t first = 0; first < tiles; first += f32.launch) {
+          const WfPart p = part_of(first);
+          launch_wgrad_f32({(const float*)a.x, (const float*)a.g + first * kWpRows * a.cb, a.rows_x,
+                            std::min(p.tiles * kWpRows, a.rows - first * kWpRows), a.plan_total, a.loc + first * kWpRows * a.K,
+                            a.uptr + first, a.urows, a.K, a.ca, a.cb, f32, p.partial}, st);
+          if (first + p.tiles < tiles) launch_wgrad_reduce<float>(p.sums_at, (int)p.splits, a.K, a.ca, a.cb, 0, p.sum_to, st);
+        }
+      } else {
+        launch_wp_sums<T>(a, st);
+      }
     }
-    if (gw) launch_wgrad_reduce<T>(a.partial, splits, a.K, a.ca, a.cb, out_transposed, (T*)gw, st);
+    if (gw) launch_wgrad_reduce<T>(sums_at, splits, a.K, a.ca, a.cb, out_transposed, (T*)gw, st);
     return check_launch("conv_wgrad_planned");
   }
 };

@@ -732,6 +732,39 @@ def test_planned_weight_gradient_fp32_edges(K, ca, cb):
     assert bool(((gw - want).abs() <= bound).all()), float(((gw - want).abs() / bound).max())
 
 
+@pytest.mark.parametrize('transposed', [False, True])
+@pytest.mark.parametrize('rows', [128 * 100, 128 * 200 + 5, 128 * 330, 128 * 500 + 127])
+def test_planned_weight_gradient_fp32_in_several_launches(rows, transposed):
+  """A wide layer whose sets of sums do not fit their bytes all at once: one launch, two, three and more, the last one whole or
+  not; the bound of the test above."""
+  from ocnn_amd.octree.octree import TilePlan
+  K, c = 27, 1024
+  g = torch.Generator().manual_seed(rows)
+  table = _local_table(rows, 9000, K, g, spread=20).to(torch.int32).contiguous().to(DEV)
+  say('planned weight gradient, fp32, several launches', rows, transposed)
+  plan = TilePlan(table)
+  dev = torch.Generator(DEV).manual_seed(rows)
+  x, gr = torch.randn(9000, c, device=DEV, generator=dev), torch.randn(rows, c, device=DEV, generator=dev)
+  gw = ocnn_amd.nn.conv_wgrad(x, gr, table, transposed, plan)
+  for k in range(K):
+    at = x.double()[table[:, k].clamp_min(0).long()] * (table[:, k] >= 0)[:, None]
+    want, size = at.t() @ gr.double(), at.abs().t() @ gr.double().abs()
+    got = gw[k].t() if transposed else gw[k]
+    bound = (3 * 2.0 ** -18 + (rows / 16 + 300) * 2.0 ** -24) * size + 1e-30
+    assert bool(((got.double() - want).abs() <= bound).all()), k
+
+
+@pytest.mark.parametrize('K', [27, 9, 8, 3])
+@pytest.mark.parametrize('ca,cb', [(32, 32), (64, 96), (256, 256), (512, 512), (1024, 384), (1024, 1024)])
+def test_planned_weight_gradient_fp32_workspace(K, ca, cb):
+  """The workspace stops growing with the rows at 1 GiB; few rows take a few sets of sums."""
+  need = lambda rows: _lib.lib().ocnn_conv_wgrad_planned_workspace_bytes_for(_lib.DTYPE_CODE[torch.float32], rows, rows, K, ca, cb)
+  one = K * ca * cb * 4
+  assert need(0) == one and need(100) == one and need(1000) <= 8 * one
+  for rows in (10000, 100000, 300000, 1000000, 10000000, 70000000):
+    assert one <= need(rows) <= 1 << 30, rows
+
+
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('distinct', [367, 368])
 def test_planned_weight_gradient_32_two_workgroups_a_cu(dtype, distinct):
