@@ -488,8 +488,9 @@ int ocnn_conv_wgrad(int dtype, const void* x, int64_t rows_x, const void* g,
  * of tiles.  plan_max_distinct must be <= 415; ..._supported() tells.
  * fp32 tensors run as two bf16 pieces each (x = hi + lo), split on their way into LDS: the
  * products hi hi, hi lo, lo hi into one fp32 sum, 32 x 64 or 32 x 32 blocks of channel pairs, about
- * 5e-6 relative; a set of sums for 24 (16) tiles at most, 1 GiB of them in several launches:
- * ..._workspace_bytes_for(). */
+ * 5e-6 relative; a set of sums for 24 (16) tiles at most, 1 GiB of them in several launches.  Wide
+ * layers of few slots: split beforehand, into the workspace, three passes of the bf16 kernel into
+ * three sets of sums.  ..._workspace_bytes_for(). */
 int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int64_t rows, int K, int ca,
                                       int cb, int plan_max_distinct);
 int64_t ocnn_conv_wgrad_planned_workspace_bytes(int K, int ca, int cb);   /* f16 / bf16 */

@@ -211,6 +211,9 @@ static __device__ __forceinline__ void run_job(const Job& job, uint32_t block, f
     const PackTileJob& a = job.pack;
     if (a.aligned) pack_tile<T, P, true>((const T*)a.w, (P*)a.out, a.K, a.cin, a.cout, a.transposed, a.reverse, block);
     else pack_tile<T, P, false>((const T*)a.w, (P*)a.out, a.K, a.cin, a.cout, a.transposed, a.reverse, block);
+  } else if constexpr (KIND == Job::kSplit) {
+    const SplitJob& a = job.split;
+    split2(a.x, a.nx, a.xh, a.xl, a.g, a.ng, a.gh, a.gl, block);
   } else if constexpr (KIND == Job::kColsum) {
     const ColsumJob& a = job.colsum;
     colsum_rows<T>((const T*)a.g, a.rows, a.channels, a.rows_per_split, a.partial, block, s_sums);
@@ -228,7 +231,7 @@ static __device__ __forceinline__ void run_job(const Job& job, uint32_t block, f
 }
 
 #define OCNN_JOB_KINDS(DO) \
-  DO(Job::kPackTile) DO(Job::kColsum) DO(Job::kColsumFinish) DO(Job::kTileParts) DO(Job::kReduce)
+  DO(Job::kPackTile) DO(Job::kSplit) DO(Job::kColsum) DO(Job::kColsumFinish) DO(Job::kTileParts) DO(Job::kReduce)
 
 template <typename T> constexpr int kJobSums = 256 * (16 / sizeof(T) + 1);   // floats of LDS that a job may use
 

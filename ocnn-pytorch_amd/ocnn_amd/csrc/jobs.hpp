@@ -1,5 +1,5 @@
-// The small launches around the layers' kernels - weights packed into operand order, column sums, sums of parts and of
-// ranges - as jobs that share a launch.
+// The small launches around the layers' kernels - weights packed into operand order, fp32 operands split into
+// bf16 pieces, column sums, sums of parts and of ranges - as jobs that share a launch.
 //
 // Each of them is 3 - 8 us of latency on a handful of workgroups, and in a chain they add up: the backward
 // pass of a layer had up to seven of them around its two large kernels.  Those that do not depend on each other
@@ -19,6 +19,11 @@ struct PackTileJob {          // conv_tile.hip: weights in the order of its A op
   const void* w;
   void* out;
   int K, cin, cout, transposed, reverse, aligned;
+};
+struct SplitJob {             // reduce.hpp: two fp32 tensors into bf16 pieces
+  const float *x, *g;
+  bf16 *xh, *xl, *gh, *gl;
+  int64_t nx, ng;
 };
 struct ColsumJob {            // column sums of ranges of rows
   const void* g;
@@ -47,10 +52,11 @@ struct ReduceJob {            // reduce.hpp: sums of the ranges of a weight grad
 };
 
 struct Job {
-  enum Kind { kPackTile, kColsum, kColsumFinish, kTileParts, kReduce } kind;
+  enum Kind { kPackTile, kSplit, kColsum, kColsumFinish, kTileParts, kReduce } kind;
   unsigned blocks;            // of 256 threads
   union {
     PackTileJob pack;
+    SplitJob split;
     ColsumJob colsum;
     ColsumFinishJob colsum_finish;
     TilePartsJob parts;

@@ -14,8 +14,8 @@
 // and g staged once for the three products.  Before, the pieces were written by a launch of their own and the three products
 // were workgroups of the 16-bit kernel with sums each, one read per MFMA, every row staged three times.  With the launches
 // around it, us, so / now: 64 -> 64 on 154 k rows 115 / 94, 592 k 376 / 315, 4 k 25.2 / 21.9; 32 -> 32 154 k 54 / 37; 96 -> 96
-// 154 k 338 / 207, 30 k 80 / 51; 128 -> 128 154 k 344 / 284; 256 -> 256 51 k 450 / 380; nine slots 64 -> 64 283 k 113 / 84, but
-// 256 -> 256 194 / 208 (twelve slots' worth of MFMAs for nine); eight slots 64 -> 64 283 k 154 / 112.
+// 154 k 338 / 207, 30 k 80 / 51; 128 -> 128 154 k 344 / 284; 256 -> 256 51 k 450 / 380; nine slots 64 -> 64 283 k 113 / 84, eight
+// 154 / 112.  Wide layers of few slots still go the other way (wp_takes_pieces): nine slots here are twelve slots' worth of MFMAs.
 #include <algorithm>
 #include <type_traits>
 

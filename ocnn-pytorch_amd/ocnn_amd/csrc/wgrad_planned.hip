@@ -68,12 +68,13 @@ struct WpStage {
 // 32 channels of x: blocks of 32 x 64 have as many sums over all 27 slots as 64 x 64 over half of them, so one
 // workgroup stages a range's rows for all slots: 32 -> 64 on 1.06 M rows (61 % set) 119 us, in half-empty 64 x 64 blocks of two
 // slot groups 201.
-template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool BLK, int CAP>
+template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool BLK, int CAP, bool PIECES>
 __global__ __launch_bounds__(256, CAP < kWpCap ? 2 : 1) void conv_wgrad_planned_kernel(
     const T* __restrict__ x, uint32_t x_bytes, const T* __restrict__ g, uint32_t g_bytes,
     const uint16_t* __restrict__ loc, uint32_t loc_bytes, const int32_t* __restrict__ uptr,
     const int32_t* __restrict__ urows, uint32_t urows_bytes, int64_t tiles,
-    int64_t tiles_per_split, int workgroups, int ca, int cb, float* __restrict__ partial) {
+    int64_t tiles_per_split, int workgroups, int ca, int cb, float* __restrict__ partial, const T* __restrict__ x_lo,
+    const T* __restrict__ g_lo, int64_t set) {
   int number = (int)xcd_tile(blockIdx.x, gridDim.x >> 3);
   if (number >= workgroups) return;
   const int grp = number % GROUPS;
@@ -82,6 +83,13 @@ __global__ __launch_bounds__(256, CAP < kWpCap ? 2 : 1) void conv_wgrad_planned_
   const int nbb = BLK ? (cb + CB - 1) / CB : 1, nblocks = BLK ? nbb * ((ca + CA - 1) / CA) : 1;
   const int block = __builtin_amdgcn_readfirstlane(number % nblocks);
   const int split = __builtin_amdgcn_readfirstlane(number / nblocks);
+  // PIECES: fp32 data as bf16 pieces: hi hi, hi lo, lo hi, each with sums of its own.  (A product's number is a grid
+  // index of its own: out of a division it made the pointers, and every staging load, vectors.)
+  if constexpr (PIECES) {
+    if (blockIdx.y == 1) g = g_lo;
+    if (blockIdx.y == 2) x = x_lo;
+    partial += blockIdx.y * set;
+  }
   constexpr int HA = CA / 32, HB = CB / 32;   // 32-channel halves of a row of x, of g
   constexpr int NU = HA * NFULL + NHALF;      // 32 x CB accumulator units per wave
   constexpr int NS = NFULL + NHALF;           // distinct slots per wave
@@ -416,7 +424,6 @@ static int wp_splits(int range_workgroups, int n_cu) { return std::min(512, std:
 // workgroups at once: two a CU for 32 x 32 blocks of tiles with few distinct rows
 static int wp_places(int ca, int cb, int n_cu, bool few) { return ca == 32 && cb == 32 && few ? 2 * n_cu : n_cu; }
 
-
 // Tiles of a range, for the least time of
 //   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
 //   the first tile, writing the sums) + the sums of all ranges written and read back, in units of one tile's time.
@@ -424,21 +431,42 @@ static int wp_places(int ca, int cb, int n_cu, bool few) { return ca == 32 && cb
 // move at about 3.5 TB/s.  Rounds are counted on an XCD's CUs (40 CUs' worth of workgroups on 32 are two rounds), the sums
 // where there are few tiles (256 -> 256: 7 MB a range).
 constexpr double kWpTileUs = 2.45, kWpFixedUs = 8.085, kWpSumUs = 5.635e-7; // us; us a byte of sums
-static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, int n_cu) {
+static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, int n_cu, int products = 1) {
   const int cu_xcd = std::max(1, n_cu / 8);
   int64_t best = std::max<int64_t>(tiles, 1);
   double least = 1e30;
   int64_t s = 1;
-  const int64_t most = wp_splits(wgs, n_cu);
+  const int64_t most = wp_splits(wgs * products, n_cu);
   for (bool more = true; more && s <= most;) {               // (the fewest ranges of as many tiles; then of fewer tiles)
     const int64_t per = std::max<int64_t>(1, cdiv(tiles, s)), used = s;
     more = per > 1;
     if (more) s = cdiv(tiles, per - 1);
-    const double cost = (double)cdiv(cdiv(used * wgs, 8), cu_xcd) * ((double)per * kWpTileUs + kWpFixedUs) +
-                        (double)used * (double)sums_bytes * kWpSumUs;
+    const double cost = (double)cdiv(cdiv(used * wgs, 8) * products, cu_xcd) * ((double)per * kWpTileUs + kWpFixedUs) +
+                        (double)used * (double)(sums_bytes * products) * kWpSumUs;
     if (cost < least) least = cost, best = per;
   }
   return best;
+}
+
+// fp32: whether the operands are split by a launch of their own, and the products are workgroups of the 16-bit kernel on 64 x 64
+// blocks.  With few slots that kernel is ahead where the layer is wide enough to make up for the pieces written and read:
+// wgrad_f32.hip stages every row of x once for 64 channels of g, and issues the MFMAs of twelve slots for nine.  us, wgrad_f32.hip /
+// so: nine slots 256 -> 256 on 4 k rows 32 / 32, 20 k 87 / 84, 100 k 410 / 360; 512 -> 512 on 20 k 323 / 277; 1024 -> 1024 1322 / 956;
+// 224 -> 224 on 40 k 147 / 143, 128 -> 256 99 / 100; eight slots 256 -> 256 on 40 k 138 / 136, 256 -> 384 on 40 k 204 / 190, 512 -> 512 on
+// 20 k 256 / 242; three 256 -> 256 on 40 k 95 / 99, 256 -> 384 145 / 131, 512 -> 512 on 20 k 182 / 166, on 4 k 43 / 48.  (27 slots: wgrad_f32.hip always.)
+static bool wp_takes_pieces(int64_t rows, int K, int ca, int cb) {
+  if (K == 27) return false;
+  const bool nine = K == 9;
+  return ca * cb >= (nine ? 128 : 150) * (ca + cb) && rows * ca * cb >= (nine ? 1ll << 30 : 1ll << 31);
+}
+
+struct WpPieces {                             // ranges of tiles, and where the pieces end in the workspace
+  int64_t per, used, x_bytes, g_bytes;
+};
+static WpPieces wp_pieces(int64_t rows_x, int64_t rows, int K, int ca, int cb, int n_cu) {
+  const int64_t tiles = cdiv(rows, kWpRows);
+  const int64_t per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), (int64_t)K * ca * cb * 4, n_cu, 3);
+  return {per, cdiv(tiles, per), align_up(rows_x * ca * 2, 256), align_up(rows * cb * 2, 256)};
 }
 
 static int wp_cu_count() {
@@ -475,13 +503,17 @@ extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes_for(int dtype, int64_
   if (dtype != OCNN_F32 || rows_x < 0 || rows < 0) return ocnn_conv_wgrad_planned_workspace_bytes(K, ca, cb);
   const int n_cu = wp_cu_count();
   const int64_t tiles = cdiv(rows, kWpRows);
+  if (wp_takes_pieces(rows, K, ca, cb) && n_cu > 0) {
+    const WpPieces p = wp_pieces(rows_x, rows, K, ca, cb, n_cu);
+    return align_up(2 * p.x_bytes + 2 * p.g_bytes + 3 * p.used * K * ca * cb * 4, 256);
+  }
   const int64_t sets = n_cu > 0 ? wf_workspace_sets(wf_split_tiles(tiles, K, ca, cb, n_cu), tiles) : tiles;
   return align_up(sets * K * ca * cb * 4, 256);
 }
 
 struct WpArgs {
-  const void *x, *g;
-  int64_t rows_x, rows, per, plan_total;
+  const void *x, *g, *x_lo, *g_lo;            // x_lo, g_lo: the low bf16 pieces of fp32 data (else null)
+  int64_t rows_x, rows, set, per, plan_total; // set: floats of the sums of one product of pieces
   const uint16_t* loc;
   const int32_t *uptr, *urows;
   int K, ca, cb, used;                        // used: ranges of tiles
@@ -489,16 +521,17 @@ struct WpArgs {
   bool two;                                   // two workgroups a CU
 };
 
-template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS>
+template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool PIECES>
 static void launch_wp(const WpArgs& a, hipStream_t st) {
   const int64_t tiles = cdiv(a.rows, kWpRows);
   const uint32_t xb = (uint32_t)(a.rows_x * a.ca * 2), gb = (uint32_t)(a.rows * a.cb * 2);
   const int wgs = a.used * wp_range_workgroups(a.K, a.ca, a.cb);
   const uint32_t lb = (uint32_t)(tiles * kWpRows * KK * 2), ub = (uint32_t)(a.plan_total * 4);
 #define OCNN_WP_KERNEL(BLK_, CAP_)                                                                                   \
-  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, CA, CB, KK, NFULL, NHALF, GROUPS, BLK_, CAP_>),                           \
-                     dim3(8 * (unsigned)cdiv(wgs, 8)), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g, gb, a.loc,       \
-                     lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial)
+  hipLaunchKernelGGL((conv_wgrad_planned_kernel<T, CA, CB, KK, NFULL, NHALF, GROUPS, BLK_, CAP_, PIECES>),                   \
+                     dim3(8 * (unsigned)cdiv(wgs, 8), PIECES ? 3 : 1), dim3(256), 0, st, (const T*)a.x, xb, (const T*)a.g, \
+                     gb, a.loc, lb, a.uptr, a.urows, ub, tiles, a.per, wgs, a.ca, a.cb, a.partial, (const T*)a.x_lo,       \
+                     (const T*)a.g_lo, a.set)
   if (a.ca == CA && a.cb == CB) {
     if (CB == 32 && a.two) OCNN_WP_KERNEL(false, CB == 32 ? kWpCapTwo : kWpCap);
     else OCNN_WP_KERNEL(false, kWpCap);
@@ -510,7 +543,7 @@ static void launch_wp(const WpArgs& a, hipStream_t st) {
 // per-range sums of x^T g into `partial`
 template <typename T>
 static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
-#define OCNN_WP_LAUNCH(CA, CB, KK, NF, NH, GR) launch_wp<T, CA, CB, KK, NF, NH, GR>(a, st)
+#define OCNN_WP_LAUNCH(CA, CB, KK, NF, NH, GR) launch_wp<T, CA, CB, KK, NF, NH, GR, false>(a, st)
   if (wp_wide(a.ca)) {
     if (a.K == 27) OCNN_WP_LAUNCH(64, 64, 27, 3, 1, 2);
     else if (a.K == 9) OCNN_WP_LAUNCH(64, 64, 9, 2, 1, 1);
@@ -530,7 +563,14 @@ static void launch_wp_sums(const WpArgs& a, hipStream_t st) {
 #undef OCNN_WP_LAUNCH
 }
 
-// T: the type of x, g and gw (float: wgrad_f32.hip)
+// The same of fp32 as three products of bf16 pieces (wp_takes_pieces), sums of their own for each
+static void launch_wp_pieces(const WpArgs& a, hipStream_t st) {
+  if (a.K == 9) launch_wp<bf16, 64, 64, 9, 2, 1, 1, true>(a, st);
+  else if (a.K == 8) launch_wp<bf16, 64, 64, 8, 2, 0, 1, true>(a, st);
+  else launch_wp<bf16, 64, 64, 3, 1, 0, 1, true>(a, st);
+}
+
+// T: the type of x, g and gw (float: wgrad_f32.hip, or as pieces)
 template <typename T> struct WpPass : Pass {
   static constexpr bool F32 = std::is_same<T, float>::value;
   WpArgs a;
@@ -548,24 +588,47 @@ template <typename T> struct WpPass : Pass {
       return;
     }
     const int K = p.K, ca = p.ca, cb = p.cb;
-    a = WpArgs{p.x, p.g, p.rows_x, p.rows, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0, (float*)p.workspace, ca == 32 && cb == 32 && p.plan_max_distinct <= kWpCapTwo};
+    a = WpArgs{p.x, p.g, nullptr, nullptr, p.rows_x, p.rows, 0, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0,
+               (float*)p.workspace, ca == 32 && cb == 32 && p.plan_max_distinct <= kWpCapTwo};
     const int64_t tiles = cdiv(p.rows, kWpRows), sums = (int64_t)K * ca * cb * 4;       // bytes of a range's sums
-    if (F32) {
+    WpPieces pieces{};
+    const bool split = F32 && wp_takes_pieces(p.rows, K, ca, cb);
+    if (split) {
+      pieces = wp_pieces(p.rows_x, p.rows, K, ca, cb, n_cu);
+      a.per = pieces.per;
+      a.used = (int)pieces.used;
+      a.set = pieces.used * K * ca * cb;
+    } else if (F32) {
       f32 = wf_split_tiles(tiles, K, ca, cb, n_cu);
       a.used = (int)wf_workspace_sets(f32, tiles);
     } else {
       a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, wp_places(ca, cb, n_cu, a.two));
       a.used = (int)cdiv(tiles, a.per);
     }
-    if (p.workspace_bytes < a.used * sums) {
+    const int64_t pieces_bytes = 2 * pieces.x_bytes + 2 * pieces.g_bytes;
+    if (p.workspace_bytes < pieces_bytes + (split ? 3 : 1) * a.used * sums) {
       set_error("conv_wgrad_planned: workspace too small");
       rc = OCNN_ERR_WORKSPACE;
       return;
     }
     const int64_t per = (int64_t)K * ca * cb;
     splits = p.rows > 0 ? a.used : 0;
+    if (split) {
+      char* ws = (char*)p.workspace;
+      a.partial = (float*)(ws + pieces_bytes);
+      splits *= 3;
+      if (p.rows > 0) {
+        bf16 *xh = (bf16*)ws, *xl = (bf16*)(ws + pieces.x_bytes), *gh = (bf16*)(ws + 2 * pieces.x_bytes);
+        bf16* gl = (bf16*)(ws + 2 * pieces.x_bytes + pieces.g_bytes);
+        const int64_t nx = p.rows_x * ca, ng = p.rows * cb;
+        Job j{Job::kSplit, (unsigned)cdiv((nx + ng) / 8, 256), {}};
+        j.split = SplitJob{(const float*)p.x, (const float*)p.g, xh, xl, gh, gl, nx, ng};
+        before.add(j);
+        a.x = xh, a.x_lo = xl, a.g = gh, a.g_lo = gl;
+      }
+    }
     sums_at = a.partial;
-    if (F32 && p.rows > 0) {                                 // the reduction behind the last launch
+    if (F32 && !split && p.rows > 0) {                                 // the reduction behind the last launch
       const WfPart last = part_of((cdiv(tiles, f32.launch) - 1) * f32.launch);
       splits = (int)last.splits, sums_at = last.sums_at;
     }
@@ -597,7 +660,9 @@ template <typename T> struct WpPass : Pass {
 
   int main() override {
     if (a.rows > 0) {
-      if constexpr (F32) {
+      if (F32 && a.x_lo) {
+        launch_wp_pieces(a, st);
+      } else if constexpr (F32) {
         const int64_t tiles = cdiv(a.rows, kWpRows);
         for (int64_t first = 0; first < tiles; first += f32.launch) {
           const WfPart p = part_of(first);

@@ -762,7 +762,38 @@ def test_planned_weight_gradient_fp32_workspace(K, ca, cb):
   one = K * ca * cb * 4
   assert need(0) == one and need(100) == one and need(1000) <= 8 * one
   for rows in (10000, 100000, 300000, 1000000, 10000000, 70000000):
-    assert one <= need(rows) <= 1 << 30, rows
+    pieces = _takes_pieces(rows, K, ca, cb) * (4 * rows * (ca + cb) + 4 * 256)         # (two 16-bit values for each of x and g)
+    assert one <= need(rows) <= (1 << 30) + pieces, rows
+
+
+def _takes_pieces(rows, K, ca, cb):
+  """Layers of few slots whose fp32 operands are split by a launch of their own."""
+  return K < 27 and ca * cb >= (128 if K == 9 else 150) * (ca + cb) and rows * ca * cb >= (1 << 30 if K == 9 else 1 << 31)
+
+
+@pytest.mark.parametrize('K,ca,cb,rows', [(9, 256, 256, 16383), (9, 256, 256, 16384), (9, 288, 416, 9000), (8, 320, 288, 23302),
+                                          (8, 320, 288, 23301), (3, 288, 320, 23302), (3, 512, 512, 8197)])
+def test_planned_weight_gradient_fp32_in_pieces(K, ca, cb, rows):
+  """Wide layers of few slots on both sides of the rule that takes them to the 16-bit kernel, with last blocks that are half
+  empty and a last tile that is not full: the bound of the fp32 kernel, and the workspace of the route."""
+  from ocnn_amd.octree.octree import TilePlan
+  g = torch.Generator().manual_seed(rows)
+  table = _local_table(rows, 9000, K, g, spread=20).to(torch.int32).contiguous().to(DEV)
+  say('planned weight gradient, fp32, pieces', K, ca, cb, rows)
+  plan = TilePlan(table)
+  size = _lib.lib().ocnn_conv_wgrad_planned_workspace_bytes_for(_lib.DTYPE_CODE[torch.float32], 9000, rows, K, ca, cb)
+  pieces = 4 * (9000 * ca + rows * cb)
+  assert (size % (4 * K * ca * cb) == 0) != _takes_pieces(rows, K, ca, cb) and (not _takes_pieces(rows, K, ca, cb) or size > pieces)
+  x, gr = torch.randn(9000, ca, generator=g).to(DEV), torch.randn(rows, cb, generator=g).to(DEV)
+  for transposed in (False, True):
+    gw = ocnn_amd.nn.conv_wgrad(x, gr, table, transposed, plan)
+    assert torch.equal(gw, ocnn_amd.nn.conv_wgrad(x, gr, table, transposed, plan))
+    for k in range(K):
+      at = x.double()[table[:, k].clamp_min(0).long()] * (table[:, k] >= 0)[:, None]
+      want, scale = at.t() @ gr.double(), at.abs().t() @ gr.double().abs()
+      got = gw[k].t() if transposed else gw[k]
+      bound = (3 * 2.0 ** -18 + (rows / 16 + 300) * 2.0 ** -24) * scale + 1e-30
+      assert bool(((got.double() - want).abs() <= bound).all()), k
 
 
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
