@@ -1,7 +1,6 @@
 // Jobs that share a launch (jobs.hpp), and the backward pass of a layer with its small launches merged.
 #include <algorithm>
 #include <type_traits>
-#include <utility>
 
 #include "jobs.hpp"
 
@@ -347,10 +346,13 @@ extern "C" int ocnnx_conv_backward(int dtype, const ocnnx_gather_args* dgrad, co
     bool sums = bias_grad == nullptr;
     if (!sums) sums = colsum_jobs(dtype, grad, grad_rows, grad_channels, bias_grad, colsum_workspace, colsum_bytes, before, after);
     launch_jobs(dtype, before, st);
-    // The data gradient last: what comes next reads it, and the memory-side cache still holds its end.  First where the launch
-    // behind both finishes it from parts (256 -> 256 on one cloud's depth 5, us a layer: 92.1 with it last, 90.6).
-    Pass* order[2] = {w, d};
-    if (d && d->after.n) std::swap(order[0], order[1]);
+    // The data gradient last where that pays: what comes next reads it, and the memory-side cache still holds its end.  First where
+    // the launch behind both finishes it from parts, in fp32, and where the gradient is so small that the second kernel finds
+    // all of it in the L2s: the weight gradient gains more from that.  us a layer, forward + backward, first / last: 16 bit, 96 -> 96 on
+    // 3 MB 77.2 / 78.5, 5 MB 82.1 / 82.7, 128 -> 128 on 6 MB 101.3 / 102.0, 192 -> 192 on 9 MB 200.0 / 199.5, 96 -> 96 on 70 MB 506 / 499, 120 MB
+    // 621 / 611; fp32, 64 -> 64 85.7 / 87.1, 539 / 546, 2283 / 2294, 32 -> 32 772 / 780; in parts, 256 -> 256 on one cloud's depth 5 90.6 / 92.1.
+    const bool last = d && d->after.n == 0 && dtype != OCNN_F32 && grad_rows * grad_channels >= (4ll << 20);
+    Pass* order[2] = {last ? w : d, last ? d : w};
     for (Pass* p : order)
       if (rc == OCNN_OK && p) rc = p->main();
     if (rc == OCNN_OK) {

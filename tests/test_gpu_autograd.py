@@ -109,3 +109,20 @@ def test_transforms_are_refused():
       torch.func.grad(f)(x)
     with pytest.raises(RuntimeError, match='autograd.Function'):
       torch.func.vmap(lambda t: module(t, *args))(x[None])
+
+
+@pytest.mark.parametrize('cin,cout,dtype', [(128, 128, torch.float16), (96, 96, torch.float32), (96, 128, torch.bfloat16),
+                                            (4, 96, torch.float16), (64, 64, torch.bfloat16)])
+@pytest.mark.parametrize('n', [3000, 90000])
+def test_gradients_in_either_order(cin, cout, dtype, n):
+  """The passes of a backward pass run in an order that hangs on the gradient's type and size (small and large here) and on
+  padded channels: the same bits as each pass by itself."""
+  octree = _octree(n, 6)
+  layer = OctreeConv(cin, cout, nempty=False).to('cuda', dtype)
+  x = torch.randn(int(octree.nnum[6]), cin, generator=torch.Generator().manual_seed(n)).to('cuda', dtype).requires_grad_()
+  print('gradients in either order', cin, cout, dtype, n, x.shape[0] * cout, flush=True)
+  out = layer(x, octree, 6)
+  g = torch.randn(out.shape, generator=torch.Generator().manual_seed(n + 1)).to('cuda', dtype)
+  both = torch.autograd.grad(out, (x, layer.weights), g, retain_graph=True)
+  alone = [torch.autograd.grad(out, t, g, retain_graph=True)[0] for t in (x, layer.weights)]
+  assert all(torch.equal(a, b) for a, b in zip(both, alone))
