@@ -698,7 +698,12 @@ class _Layer:
         self.wgrad = made is not None
 
 
+_WRONG_SHAPE = 'The shape of input data is wrong: expected {}, got {}.'
+
+
 def _layer_on(engine, dtype, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
+  """The layer's native passes, made at its first call on this octree and kept with it (not `ok` where the forward pass
+  is not one native pass), and a function that makes its engine."""
   key = (engine, depth, tuple(kernel_size), stride, nempty, in_channels, out_channels, dtype, padded, SPARSE_MIN_ROWS)
   layer = octree._layers.get(key)
 
@@ -712,26 +717,15 @@ def _layer_on(engine, dtype, octree, depth, in_channels, out_channels, kernel_si
   return layer, made_engine
 
 
-def _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty, max_buffer, padded):
-  """The layer's native passes, made at its first call on this octree and kept with it: (layer or
-  None where the forward pass is not one native pass, function that makes its engine)."""
-  if not (isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE):
-    return None, None
-  layer, made_engine = _layer_on(engine, data.dtype, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
-                                 max_buffer, padded)
-  if not layer.ok:
-    return None, None
-  assert data.shape == layer.shape, \
-      'The shape of input data is wrong: expected {}, got {}.'.format(layer.shape, tuple(data.shape))
-  return layer, made_engine
-
-
 def _apply(engine, function, data, weights, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
            max_buffer, bias, padded):
   """The layer through the native node where each of its passes is one, through `function` otherwise."""
-  layer, made_engine = _layer_of(engine, data, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
-                                 max_buffer, padded)
-  if layer is not None:
+  layer = None
+  if isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE:
+    layer, made_engine = _layer_on(engine, data.dtype, octree, depth, in_channels, out_channels, kernel_size, stride, nempty,
+                                   max_buffer, padded)
+  if layer is not None and layer.ok:
+    assert data.shape == layer.shape, _WRONG_SHAPE.format(layer.shape, tuple(data.shape))
     ok = True
     if torch.is_grad_enabled():
       # (the rows of a padded gradient are summed over the non-empty nodes only: the other route)
@@ -822,12 +816,15 @@ class OctreeConv(OctreeConvBase, torch.nn.Module):
 
   def native_layer(self, data: torch.Tensor, octree, depth: int):
     """The native passes of this layer on `octree`, or None where it takes another route."""
-    if self.method != 'hip':
+    if self.method != 'hip' or not (isinstance(octree, Octree) and data.is_cuda and data.dtype in _lib.DTYPE_CODE):
       return None
-    layer, _ = _layer_of(_OctreeConv if self.is_conv_layer() else _OctreeDeconv, data, octree, depth, self.in_channels,
-                         self.out_channels, self.kernel_size, self.stride, self.nempty, self.max_buffer,
-                         self.stride == 2 and not self.nempty)
-    return None if layer is None else layer.native
+    layer, _ = _layer_on(_OctreeConv if self.is_conv_layer() else _OctreeDeconv, data.dtype, octree, depth,
+                         self.in_channels, self.out_channels, self.kernel_size, self.stride, self.nempty,
+                         self.max_buffer, self.stride == 2 and not self.nempty)
+    if not layer.ok:
+      return None
+    assert data.shape == layer.shape, _WRONG_SHAPE.format(layer.shape, tuple(data.shape))
+    return layer.native
 
   def native_of_stride_1(self, dtype, shape, octree, depth: int):
     """native_layer for data of this type and shape that is still to be made, of a layer that keeps the rows."""
