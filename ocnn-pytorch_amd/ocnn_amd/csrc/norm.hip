@@ -844,9 +844,15 @@ static int bn_blocks(int dtype, int64_t rows, int channels, int max_blocks) {
   return (int)std::min<int64_t>(max_blocks, cdiv(rows, 4 * rpp));
 }
 
-// Workgroups of 256 threads of `kernel` that the device holds at once, kBnApplyBlocks at most:
+// The backward elementwise pass reads two tensors from where the sums ended, back through the memory-side cache, and writes one or
+// two: of more than four workgroups a CU the streams are more than that takes.  fp32, us, seven (with a residual six) a CU / four:
+// 250 k x 192 98.6 / 95.7 (132.6 / 128.5), 400 k x 128 104.5 / 101.1 (140.4 / 135.1), 700 k x 64 89.4 / 87.3 (121.4 / 116.1).  (16 bit has
+// four by its registers.)
+constexpr int kBnBackwardPerCu = 4;
+
+// Workgroups of 256 threads of `kernel` that the device holds at once, `most` a CU and kBnApplyBlocks at most:
 // an elementwise pass launched with more runs them in rounds, and the last round leaves CUs idle.
-static int bn_resident_blocks(const void* kernel) {
+static int bn_resident_blocks(const void* kernel, int most = 8) {
   static std::mutex mu;
   static std::vector<std::pair<const void*, int>> known;
   std::lock_guard<std::mutex> lock(mu);
@@ -859,7 +865,7 @@ static int bn_resident_blocks(const void* kernel) {
     (void)hipGetLastError();
     per_cu = 2;
   }
-  const int cap = std::min(kBnApplyBlocks, std::max(1, per_cu * n_cu));
+  const int cap = std::min(kBnApplyBlocks, std::max(1, std::min(per_cu, most) * n_cu));
   known.emplace_back(kernel, cap);
   return cap;
 }
@@ -1006,7 +1012,7 @@ extern "C" int ocnnx_batch_norm_backward(int dtype, const void* x, const void* d
   OCNN_DISPATCH_DTYPE(dtype, {
     constexpr int VEC = 16 / sizeof(T);
     const auto launch = [&](auto sums, auto apply, const void* passed) {
-      const int nblk_a = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)apply));
+      const int nblk_a = bn_blocks(dtype, rows, channels, bn_resident_blocks((const void*)apply, kBnBackwardPerCu));
       hipLaunchKernelGGL(sums, dim3(nblk), dim3(256), 0, st, (const T*)x, (const T*)dy, rows, channels, mean, invstd, gamma, beta,
                          param_dtype, relu, passed, partial);
       hipLaunchKernelGGL(bn_bwd_finish_kernel, dim3((unsigned)cdiv(channels, 4)), dim3(kBnFinishThreads), 0, st, partial, nblk,
