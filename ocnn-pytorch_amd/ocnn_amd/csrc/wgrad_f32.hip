@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
     return make_rsrc(g + tc * kWfRows * cb + blk_b * CB, (uint32_t)n * g_pitch - (uint32_t)blk_b * CB * 4u);
   };
   auto load_g = [&](int j, __amdgpu_buffer_rsrc_t r) -> f32x4 {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, g_off0 + (uint32_t)(kRing ? 32 * (j >> 1) + 2 * (j & 1) : 32 * j) * g_pitch, 0, 0));
+    const uint32_t row = (uint32_t)(kRing ? 32 * (j >> 1) + 2 * (j & 1) : 32 * j);
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, g_off0 + row * g_pitch, 0, 0));
   };
   auto g_place = [&](int buffer, int s) -> bf16* {           // of the 16 rows of step s
     return s_g + (kRing ? (s == 0 ? buffer : s + 1) : 8 * buffer + s) * kSlot;
@@ -241,8 +242,13 @@ __global__ __launch_bounds__(256, 1) void conv_wgrad_f32_kernel(
     for (int t = 0; t < NL; ++t) pf_x(t, s_x0, 0, ops[0]);
   }
 
-  // One tile out of buffer B; the next tile -> the other buffer meanwhile: x loads in steps 0 - 3, put two steps later; g
-  // loads in steps 0, 4 and 5, put in step 2 (its first 16 rows) and, behind the barrier, in step 7.
+  // One tile out of buffer B; the next tile -> the other buffer meanwhile: x loads in steps 0 - 3, put two steps later.  g of the next tile:
+  //   CB = 64, one place a step for all tiles, two by turns for step 0: the rows of step 0 are loaded in step 0 and put in step
+  //   2, into the place whose last readers were in step 7 two tiles ago; the others are loaded in steps 4 and 5 and put in
+  //   step 7, behind the barrier that follows step 6, in which this tile's last rows of g are read.
+  //   CB = 32, two whole buffers: loaded in step 4, put in step 6, in front of that barrier: the other buffer's last
+  //   reader was step 6 of the tile before, and two barriers lie between.
+  // Step 7 reads the next tile's first operands: what the barrier in front of it has seen put, in either case.
   auto tile_body = [&](auto BC, int64_t tile) {
     constexpr int B = decltype(BC)::value;
     const bf16* sx = B ? s_x1 : s_x0;

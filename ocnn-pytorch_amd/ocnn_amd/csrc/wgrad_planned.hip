@@ -184,7 +184,8 @@ __global__ __launch_bounds__(256, CAP < kWpCap ? 2 : 1) void conv_wgrad_planned_
   const int sg_half = HB == 2 ? (wave & 1) : 0, sg_g16 = HB == 2 ? (wave >> 1) : wave;
   const uint32_t st_xc = (uint32_t)st_half * 64u + (uint32_t)(lane & 3) * 16u;   // byte within a row
   const int st_pos = st_g16 * 16 + (lane >> 2);            // position / row of piece 0; piece j: + 16 GST j
-  const uint32_t sg_c = (uint32_t)sg_half * 64u + (uint32_t)(lane & 3) * 16u, sg_pos = (uint32_t)(32 * (sg_g16 >> 1) + 2 * (sg_g16 & 1) + 16 * (lane >> 5) + 4 * ((lane >> 2) & 3) + ((lane >> 4) & 1));
+  const uint32_t sg_c = (uint32_t)sg_half * 64u + (uint32_t)(lane & 3) * 16u;
+  const uint32_t sg_pos = (uint32_t)(32 * (sg_g16 >> 1) + 2 * (sg_g16 & 1) + 16 * (lane >> 5) + 4 * ((lane >> 2) & 3) + ((lane >> 4) & 1));
   const uint32_t st_gc = (BLK ? sg_pos * g_pitch + gb : (sg_pos << RSG)) + sg_c;
   const uint32_t st_gstep = BLK ? 16u * GSG * g_pitch : 4096u;   // 16 GSG rows further
   auto make_stage = [&](int64_t tile, int U, int32_t list_first, int32_t list_len, const int32_t* su,
@@ -407,7 +408,6 @@ __global__ __launch_bounds__(256, CAP < kWpCap ? 2 : 1) void conv_wgrad_planned_
 
 using namespace ocnn;
 
-
 // blocks of channel pairs: 64 x 64 (the last of a side half beyond the channels), but for 32 channels of x, whose 32 x 64
 // blocks have room for the sums of all 27 slots in one workgroup, and for the 32 x 32 layer
 static bool wp_wide(int ca) { return ca > 32; }
@@ -418,30 +418,31 @@ static int wp_range_workgroups(int K, int ca, int cb) {
   return groups * ((ca + 63) / 64) * ((cb + 63) / 64);
 }
 
-// ranges of tiles at most: as many as keep a workgroup on every CU (the LDS holds one)
-static int wp_splits(int range_workgroups, int n_cu) { return std::min(512, std::max(8, n_cu / range_workgroups)); }
+// ranges of tiles at most: as many as put a workgroup in every place (wp_places)
+static int wp_splits(int range_workgroups, int places) { return std::min(512, std::max(8, places / range_workgroups)); }
 
-// workgroups at once: two a CU for 32 x 32 blocks of tiles with few distinct rows
+// workgroups at once: one a CU by its LDS, two for 32 x 32 blocks of tiles with few distinct rows
 static int wp_places(int ca, int cb, int n_cu, bool few) { return ca == 32 && cb == 32 && few ? 2 * n_cu : n_cu; }
 
 // Tiles of a range, for the least time of
 //   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
 //   the first tile, writing the sums) + the sums of all ranges written and read back, in units of one tile's time.
 // Measured (fp16, 64 x 64 blocks of 27 slots): 2.45 us a tile and 8 us besides on 33 - 157 tiles a range; the sums
-// move at about 3.5 TB/s.  Rounds are counted on an XCD's CUs (40 CUs' worth of workgroups on 32 are two rounds), the sums
-// where there are few tiles (256 -> 256: 7 MB a range).
+// move at about 3.5 TB/s.  Rounds are counted on an XCD's places (40 workgroups on 32 are two rounds), the sums
+// where there are few tiles (256 -> 256: 7 MB a range).  The other blocks and slot counts and 32 x 32 with two workgroups
+// a CU have no figures of their own.
 constexpr double kWpTileUs = 2.45, kWpFixedUs = 8.085, kWpSumUs = 5.635e-7; // us; us a byte of sums
-static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, int n_cu, int products = 1) {
-  const int cu_xcd = std::max(1, n_cu / 8);
+static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, int places, int products = 1) {
+  const int places_xcd = std::max(1, places / 8);
   int64_t best = std::max<int64_t>(tiles, 1);
   double least = 1e30;
   int64_t s = 1;
-  const int64_t most = wp_splits(wgs * products, n_cu);
+  const int64_t most = wp_splits(wgs * products, places);
   for (bool more = true; more && s <= most;) {               // (the fewest ranges of as many tiles; then of fewer tiles)
     const int64_t per = std::max<int64_t>(1, cdiv(tiles, s)), used = s;
     more = per > 1;
     if (more) s = cdiv(tiles, per - 1);
-    const double cost = (double)cdiv(cdiv(used * wgs, 8) * products, cu_xcd) * ((double)per * kWpTileUs + kWpFixedUs) +
+    const double cost = (double)cdiv(cdiv(used * wgs, 8) * products, places_xcd) * ((double)per * kWpTileUs + kWpFixedUs) +
                         (double)used * (double)(sums_bytes * products) * kWpSumUs;
     if (cost < least) least = cost, best = per;
   }
@@ -452,8 +453,9 @@ static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, in
 // blocks.  With few slots that kernel is ahead where the layer is wide enough to make up for the pieces written and read:
 // wgrad_f32.hip stages every row of x once for 64 channels of g, and issues the MFMAs of twelve slots for nine.  us, wgrad_f32.hip /
 // so: nine slots 256 -> 256 on 4 k rows 32 / 32, 20 k 87 / 84, 100 k 410 / 360; 512 -> 512 on 20 k 323 / 277; 1024 -> 1024 1322 / 956;
-// 224 -> 224 on 40 k 147 / 143, 128 -> 256 99 / 100; eight slots 256 -> 256 on 40 k 138 / 136, 256 -> 384 on 40 k 204 / 190, 512 -> 512 on
-// 20 k 256 / 242; three 256 -> 256 on 40 k 95 / 99, 256 -> 384 145 / 131, 512 -> 512 on 20 k 182 / 166, on 4 k 43 / 48.  (27 slots: wgrad_f32.hip always.)
+// 224 -> 224 on 40 k 147 / 143, 128 -> 256 99 / 100; eight slots 256 -> 256 on 40 k 138 / 136, 256 -> 384 on 40 k 204 / 190,
+// 512 -> 512 on 20 k 256 / 242; three 256 -> 256 on 40 k 95 / 99, 256 -> 384 145 / 131, 512 -> 512 on 20 k 182 / 166, on 4 k 43 / 48.
+// (27 slots: wgrad_f32.hip always.)
 static bool wp_takes_pieces(int64_t rows, int K, int ca, int cb) {
   if (K == 27) return false;
   const bool nine = K == 9;

@@ -516,7 +516,7 @@ def test_layers_hold_the_memory_of_their_nodes(n, depth, full):
 
 def test_batch_ids_without_octrees_are_refused():
   """More nodes at the deepest full layer than the octrees have, of batch ids beyond them: an error, raised when the sizes are
-  known and before a layer is made (a tensor made before is as it was)."""
+  known and before a kernel writes to a layer (a tensor made before the call is as it was)."""
   before = torch.full((1 << 16,), 7, dtype=torch.int32, device=DEV)
   grid = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing='ij'), -1).reshape(-1, 3) / 2.0 - 0.9
   pts = np.tile(grid, (4, 1)).astype(np.float32)
