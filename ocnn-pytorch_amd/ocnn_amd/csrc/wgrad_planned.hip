@@ -453,13 +453,12 @@ static int64_t wp_tiles_per_range(int64_t tiles, int wgs, int64_t sums_bytes, in
 // blocks.  With few slots that kernel is ahead where the layer is wide enough to make up for the pieces written and read:
 // wgrad_f32.hip stages every row of x once for 64 channels of g, and issues the MFMAs of twelve slots for nine.  us, wgrad_f32.hip /
 // so: nine slots 256 -> 256 on 4 k rows 32 / 32, 20 k 87 / 84, 100 k 410 / 360; 512 -> 512 on 20 k 323 / 277; 1024 -> 1024 1322 / 956;
-// 224 -> 224 on 40 k 147 / 143, 128 -> 256 99 / 100; eight slots 256 -> 256 on 40 k 138 / 136, 256 -> 384 on 40 k 204 / 190,
-// 512 -> 512 on 20 k 256 / 242; three 256 -> 256 on 40 k 95 / 99, 256 -> 384 145 / 131, 512 -> 512 on 20 k 182 / 166, on 4 k 43 / 48.
+// 224 -> 224 on 40 k 147 / 143, 128 -> 256 99 / 100; eight slots 256 -> 256 on 40 k 138 / 136, 120 k 396 / 385, 256 -> 384 on 40 k 204 / 190,
+// 512 -> 512 on 20 k 256 / 242; three 256 -> 256 on 40 k 95 / 99, 120 k 284 / 303, 256 -> 384 145 / 131, 512 -> 512 on 20 k 182 / 166, on 4 k 43 / 48.
 // (27 slots: wgrad_f32.hip always.)
 static bool wp_takes_pieces(int64_t rows, int K, int ca, int cb) {
   if (K == 27) return false;
-  const bool nine = K == 9;
-  return ca * cb >= (nine ? 128 : 150) * (ca + cb) && rows * ca * cb >= (nine ? 1ll << 30 : 1ll << 31);
+  return ca * cb >= (K == 3 ? 150 : 128) * (ca + cb) && rows * ca * cb >= (K == 9 ? 1ll << 30 : 1ll << 31);
 }
 
 struct WpPieces {                             // ranges of tiles, and where the pieces end in the workspace

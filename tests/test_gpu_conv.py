@@ -768,11 +768,12 @@ def test_planned_weight_gradient_fp32_workspace(K, ca, cb):
 
 def _takes_pieces(rows, K, ca, cb):
   """Layers of few slots whose fp32 operands are split by a launch of their own."""
-  return K < 27 and ca * cb >= (128 if K == 9 else 150) * (ca + cb) and rows * ca * cb >= (1 << 30 if K == 9 else 1 << 31)
+  return K < 27 and ca * cb >= (150 if K == 3 else 128) * (ca + cb) and rows * ca * cb >= (1 << 30 if K == 9 else 1 << 31)
 
 
 @pytest.mark.parametrize('K,ca,cb,rows', [(9, 256, 256, 16383), (9, 256, 256, 16384), (9, 288, 416, 9000), (8, 320, 288, 23302),
-                                          (8, 320, 288, 23301), (3, 288, 320, 23302), (3, 512, 512, 8197)])
+                                          (8, 320, 288, 23301), (8, 256, 256, 32767), (8, 256, 256, 32768),
+                                          (3, 288, 320, 23302), (3, 512, 512, 8197)])
 def test_planned_weight_gradient_fp32_in_pieces(K, ca, cb, rows):
   """Wide layers of few slots on both sides of the rule that takes them to the 16-bit kernel, with last blocks that are half
   empty and a last tile that is not full: the bound of the fp32 kernel, and the workspace of the route."""
