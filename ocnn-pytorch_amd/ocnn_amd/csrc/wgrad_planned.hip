@@ -418,11 +418,16 @@ static int wp_range_workgroups(int K, int ca, int cb) {
   return groups * ((ca + 63) / 64) * ((cb + 63) / 64);
 }
 
-// ranges of tiles at most: as many as put a workgroup in every place (wp_places)
+// ranges of tiles at most: as many as put a workgroup in every place, one a CU by its LDS or two (wp_two)
 static int wp_splits(int range_workgroups, int places) { return std::min(512, std::max(8, places / range_workgroups)); }
 
-// workgroups at once: one a CU by its LDS, two for 32 x 32 blocks of tiles with few distinct rows
-static int wp_places(int ca, int cb, int n_cu, bool few) { return ca == 32 && cb == 32 && few ? 2 * n_cu : n_cu; }
+// Two workgroups a CU: 32 x 32 blocks of tiles with few distinct rows.  With few slots only where a CU has a dozen tiles: below, the
+// further sets of sums take more than the tiles gain.  us, one a CU / two: nine slots 90 k rows 15.4 / 17.0, 120 k 16.1 / 18.0, 400 k
+// 23.4 / 23.4, 1 M 41.4 / 37.4; eight 120 k 14.8 / 16.5, 400 k 21.1 / 21.2, 1 M 36.8 / 32.5; three 120 k 11.8 / 12.9, 400 k 18.6 / 18.9,
+// 1 M 33.2 / 29.7.
+static bool wp_two(int K, int ca, int cb, int64_t tiles, int max_distinct, int n_cu) {
+  return ca == 32 && cb == 32 && max_distinct <= kWpCapTwo && (K == 27 || tiles >= 12 * n_cu);
+}
 
 // Tiles of a range, for the least time of
 //   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
@@ -495,7 +500,7 @@ extern "C" int ocnn_conv_wgrad_planned_supported(int dtype, int64_t rows_x, int6
 
 extern "C" int64_t ocnn_conv_wgrad_planned_workspace_bytes(int K, int ca, int cb) {
   const int n_cu = wp_cu_count();
-  const int64_t splits = n_cu > 0 ? wp_splits(wp_range_workgroups(K, ca, cb), wp_places(ca, cb, n_cu, true)) : 512;
+  const int64_t splits = n_cu > 0 ? wp_splits(wp_range_workgroups(K, ca, cb), ca == 32 && cb == 32 ? 2 * n_cu : n_cu) : 512;
   return align_up(splits * K * ca * cb * 4, 256);
 }
 
@@ -589,9 +594,9 @@ template <typename T> struct WpPass : Pass {
       return;
     }
     const int K = p.K, ca = p.ca, cb = p.cb;
-    a = WpArgs{p.x, p.g, nullptr, nullptr, p.rows_x, p.rows, 0, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0,
-               (float*)p.workspace, ca == 32 && cb == 32 && p.plan_max_distinct <= kWpCapTwo};
     const int64_t tiles = cdiv(p.rows, kWpRows), sums = (int64_t)K * ca * cb * 4;       // bytes of a range's sums
+    a = WpArgs{p.x, p.g, nullptr, nullptr, p.rows_x, p.rows, 0, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0,
+               (float*)p.workspace, wp_two(K, ca, cb, tiles, p.plan_max_distinct, n_cu)};
     WpPieces pieces{};
     const bool split = F32 && wp_takes_pieces(p.rows, K, ca, cb);
     if (split) {
@@ -603,7 +608,7 @@ template <typename T> struct WpPass : Pass {
       f32 = wf_split_tiles(tiles, K, ca, cb, n_cu);
       a.used = (int)wf_workspace_sets(f32, tiles);
     } else {
-      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, wp_places(ca, cb, n_cu, a.two));
+      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, a.two ? 2 * n_cu : n_cu);
       a.used = (int)cdiv(tiles, a.per);
     }
     const int64_t pieces_bytes = 2 * pieces.x_bytes + 2 * pieces.g_bytes;

@@ -826,6 +826,27 @@ def test_planned_weight_gradient_32_two_workgroups_a_cu(dtype, distinct):
     assert torch.equal(gw, ocnn_amd.nn.conv_wgrad(x.to(DEV), gr.to(DEV), table.to(DEV), False, plan))
 
 
+@pytest.mark.parametrize('K', [9, 8, 3])
+@pytest.mark.parametrize('tiles', [600, 3071, 3072, 4099])
+def test_planned_weight_gradient_32_few_slots(K, tiles):
+  """32 x 32 blocks of few slots, one workgroup a CU up to a dozen tiles each and two beyond: a last tile of one row, from the
+  definition in fp64 (16-bit products are exact in fp32; a sum of that many rounds by 2^-24 of its size a step, the result by 2^-11)."""
+  from ocnn_amd.octree.octree import TilePlan
+  rows = 128 * tiles - 127
+  g = torch.Generator().manual_seed(tiles)
+  table = _local_table(rows, rows, K, g, spread=20).to(torch.int32).contiguous().to(DEV)
+  say('planned weight gradient, 32 x 32, few slots', K, tiles)
+  plan = TilePlan(table)
+  assert plan.umax <= 367
+  x, gr = torch.randn(rows, 32, generator=g).to(DEV, torch.float16), torch.randn(rows, 32, generator=g).to(DEV, torch.float16)
+  gw = ocnn_amd.nn.conv_wgrad(x, gr, table, False, plan)
+  for k in range(K):
+    at = x.double()[table[:, k].clamp_min(0).long()] * (table[:, k] >= 0)[:, None]
+    want, size = at.t() @ gr.double(), at.abs().t() @ gr.double().abs()
+    bound = 2.0 ** -11 * want.abs() + (rows / 16 + 600) * 2.0 ** -24 * size + 1e-30
+    assert bool(((gw[k].double() - want).abs() <= bound).all()), k
+
+
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('cin,cout', [(64, 128), (128, 512), (512, 128), (256, 256), (1024, 384), (192, 1024)])
 def test_dense_rows_kernel(dtype, cin, cout):
