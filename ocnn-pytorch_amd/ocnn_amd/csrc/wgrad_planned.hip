@@ -63,7 +63,8 @@ struct WpStage {
 //
 // CAP: distinct rows of a tile at most.  A wave of the 32 x 32 layer has 212 registers, and with 367 rows two workgroups find
 // room in a CU's LDS, which hides the waits of one behind the other: us, f16, one / two a CU: 7.57 M rows 468 / 425, 4.74 M 295 / 276, 1.13 M
-// (7 % set) 80.7 / 74, 947 k 65 / 59; below 100 k rows the same.
+// (7 % set) 80.7 / 74, 947 k 65 / 59.  Where there are
+// ranges for one a CU only (wp_places) this form is ahead by its smaller buffers: 120 k 23.8 / 22.8, 330 k 35.9 / 34.2.
 //
 // 32 channels of x: blocks of 32 x 64 have as many sums over all 27 slots as 64 x 64 over half of them, so one
 // workgroup stages a range's rows for all slots: 32 -> 64 on 1.06 M rows (61 % set) 119 us, in half-empty 64 x 64 blocks of two
@@ -418,16 +419,14 @@ static int wp_range_workgroups(int K, int ca, int cb) {
   return groups * ((ca + 63) / 64) * ((cb + 63) / 64);
 }
 
-// ranges of tiles at most: as many as put a workgroup in every place, one a CU by its LDS or two (wp_two)
+// ranges of tiles at most: as many as put a workgroup in every place, one a CU by its LDS or two (wp_places)
 static int wp_splits(int range_workgroups, int places) { return std::min(512, std::max(8, places / range_workgroups)); }
 
-// Two workgroups a CU: 32 x 32 blocks of tiles with few distinct rows.  With few slots only where a CU has a dozen tiles: below, the
-// further sets of sums take more than the tiles gain.  us, one a CU / two: nine slots 90 k rows 15.4 / 17.0, 120 k 16.1 / 18.0, 400 k
-// 23.4 / 23.4, 1 M 41.4 / 37.4; eight 120 k 14.8 / 16.5, 400 k 21.1 / 21.2, 1 M 36.8 / 32.5; three 120 k 11.8 / 12.9, 400 k 18.6 / 18.9,
-// 1 M 33.2 / 29.7.
-static bool wp_two(int K, int ca, int cb, int64_t tiles, int max_distinct, int n_cu) {
-  return ca == 32 && cb == 32 && max_distinct <= kWpCapTwo && (K == 27 || tiles >= 12 * n_cu);
-}
+// Workgroups at once: one a CU, and two of 32 x 32 blocks of tiles with few distinct rows (kWpCapTwo) where a CU has 14 tiles: below, the
+// further sets of sums take more than the tiles gain.  us, one a CU / two: 27 slots 250 k rows 30.6 / 32.1, 421 k 40.5 / 41.5, 500 k
+// 45.1 / 44.3, 1.5 M 111.6 / 105.1; nine 120 k 16.1 / 18.0, 400 k 23.4 / 23.4, 1 M 41.4 / 37.4; eight 120 k 14.8 / 16.5, 400 k 21.1 / 21.2,
+// 1 M 36.8 / 32.5; three 120 k 11.8 / 12.9, 400 k 18.6 / 18.9, 1 M 33.2 / 29.7.
+static int wp_places(int64_t tiles, int n_cu, bool two) { return two && tiles >= 14 * n_cu ? 2 * n_cu : n_cu; }
 
 // Tiles of a range, for the least time of
 //   rounds of workgroups x (tiles of a range + what a workgroup costs besides: lists and the staging of
@@ -524,7 +523,7 @@ struct WpArgs {
   const int32_t *uptr, *urows;
   int K, ca, cb, used;                        // used: ranges of tiles
   float* partial;
-  bool two;                                   // two workgroups a CU
+  bool two;                                   // two workgroups fit a CU
 };
 
 template <typename T, int CA, int CB, int KK, int NFULL, int NHALF, int GROUPS, bool PIECES>
@@ -596,7 +595,7 @@ template <typename T> struct WpPass : Pass {
     const int K = p.K, ca = p.ca, cb = p.cb;
     const int64_t tiles = cdiv(p.rows, kWpRows), sums = (int64_t)K * ca * cb * 4;       // bytes of a range's sums
     a = WpArgs{p.x, p.g, nullptr, nullptr, p.rows_x, p.rows, 0, 0, p.plan_total, p.loc, p.uptr, p.urows, K, ca, cb, 0,
-               (float*)p.workspace, wp_two(K, ca, cb, tiles, p.plan_max_distinct, n_cu)};
+               (float*)p.workspace, ca == 32 && cb == 32 && p.plan_max_distinct <= kWpCapTwo};
     WpPieces pieces{};
     const bool split = F32 && wp_takes_pieces(p.rows, K, ca, cb);
     if (split) {
@@ -608,7 +607,7 @@ template <typename T> struct WpPass : Pass {
       f32 = wf_split_tiles(tiles, K, ca, cb, n_cu);
       a.used = (int)wf_workspace_sets(f32, tiles);
     } else {
-      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, a.two ? 2 * n_cu : n_cu);
+      a.per = wp_tiles_per_range(tiles, wp_range_workgroups(K, ca, cb), sums, wp_places(tiles, n_cu, a.two));
       a.used = (int)cdiv(tiles, a.per);
     }
     const int64_t pieces_bytes = 2 * pieces.x_bytes + 2 * pieces.g_bytes;

@@ -826,16 +826,16 @@ def test_planned_weight_gradient_32_two_workgroups_a_cu(dtype, distinct):
     assert torch.equal(gw, ocnn_amd.nn.conv_wgrad(x.to(DEV), gr.to(DEV), table.to(DEV), False, plan))
 
 
-@pytest.mark.parametrize('K', [9, 8, 3])
-@pytest.mark.parametrize('tiles', [600, 3071, 3072, 4099])
-def test_planned_weight_gradient_32_few_slots(K, tiles):
-  """32 x 32 blocks of few slots, one workgroup a CU up to a dozen tiles each and two beyond: a last tile of one row, from the
+@pytest.mark.parametrize('K', [27, 9, 8, 3])
+@pytest.mark.parametrize('tiles', [600, 3583, 3584, 4099])
+def test_planned_weight_gradient_32_places(K, tiles):
+  """32 x 32 blocks, one workgroup a CU up to 14 tiles each and two beyond: a last tile of one row, from the
   definition in fp64 (16-bit products are exact in fp32; a sum of that many rounds by 2^-24 of its size a step, the result by 2^-11)."""
   from ocnn_amd.octree.octree import TilePlan
   rows = 128 * tiles - 127
   g = torch.Generator().manual_seed(tiles)
   table = _local_table(rows, rows, K, g, spread=20).to(torch.int32).contiguous().to(DEV)
-  say('planned weight gradient, 32 x 32, few slots', K, tiles)
+  say('planned weight gradient, 32 x 32, places', K, tiles)
   plan = TilePlan(table)
   assert plan.umax <= 367
   x, gr = torch.randn(rows, 32, generator=g).to(DEV, torch.float16), torch.randn(rows, 32, generator=g).to(DEV, torch.float16)
